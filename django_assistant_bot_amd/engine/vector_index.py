@@ -175,13 +175,18 @@ class VectorIndex:
         self._sorted = None
 
     # ------------------------------------------------------------------ search
+    def _id_rows(self) -> np.ndarray:
+        """int64 [2, items]: the item ids and the row of each."""
+        n = len(self._row_of)
+        return np.stack([np.fromiter(self._row_of.keys(), dtype=np.int64, count=n),
+                         np.fromiter(self._row_of.values(), dtype=np.int64, count=n)])
+
     def rows_of(self, ids) -> np.ndarray:
         """Row index of each live item id (ids that are not in the index are dropped).  Vectorised
         through a sorted (id, row) table rebuilt lazily after upserts / deletes."""
         ids = np.asarray(ids, dtype=np.int64).reshape(-1)
         if self._sorted is None:
-            keys = np.fromiter(self._row_of.keys(), dtype=np.int64, count=len(self._row_of))
-            vals = np.fromiter(self._row_of.values(), dtype=np.int64, count=len(self._row_of))
+            keys, vals = self._id_rows()
             order = np.argsort(keys, kind="stable")
             self._sorted = (keys[order], vals[order])
         keys, vals = self._sorted
@@ -224,13 +229,15 @@ class VectorIndex:
         return self._pack_rows(m)
 
     def _live_ids(self):
-        """(sorted ids of the live rows, their rows) on the device, rebuilt after an update."""
+        """(sorted item ids, the row of each) on the device, rebuilt after an update.  (From the mapping and not the row
+        metadata: an id that one ``add`` names twice has two live rows, and the mapping says which of them is its row.)"""
         table = self._id_table
         if table is None or table[0] != self._version:
             with torch.inference_mode(False):
-                live = (self.row_group[: self.n] >= 0).nonzero().flatten()
-                keys, order = self.row_ids[live].sort()
-                table = self._id_table = (self._version, keys, live[order])
+                host = torch.from_numpy(self._id_rows())
+                ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
+                keys, order = ids.sort()
+                table = self._id_table = (self._version, keys, rows[order])
         return table[1:]
 
     def doc_lt_mask(self, limits, mask=None) -> torch.Tensor:
