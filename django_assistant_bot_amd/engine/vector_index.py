@@ -38,10 +38,10 @@ class VectorIndex:
         self.stats = {"threshold_searches": 0, "threshold_overflows": 0}
         self.vecs = self.row_ids = self.row_docs = self.row_group = None
         self._row_of: dict[int, int] = {}
-        self._sorted = None  # lazily built (sorted ids, rows) for vectorised id -> row lookups
+        self._sorted = None  # lazily built (version, sorted ids, rows) for vectorised id -> row lookups
         # fragment layout (see the module docstring) for bf16 GPU indexes of a 128-multiple width
         self.frag = self.device.type == "cuda" and dtype == torch.bfloat16 and dim % 128 == 0
-        self._version = 0  # bumped by every update: invalidates the cached threshold sample and id table
+        self._version = 0  # bumped at the end of every update: invalidates the cached threshold sample and id tables
         self._sample = None
         self._id_table = None
         self._dead = 0
@@ -109,7 +109,6 @@ class VectorIndex:
         if (grp < 0).any():
             raise ValueError("groups must be >= 0 (negative marks deleted rows)")
         idl = ids.tolist()
-        self._sorted = None
         if len(set(idl)) == n and not (self._row_of.keys() & set(idl)):
             # bulk insert of new ids (ingest): C-speed bookkeeping, contiguous rows
             if self.n + n > self._cap:
@@ -149,7 +148,6 @@ class VectorIndex:
     def remove(self, ids) -> int:
         rows = [self._row_of.pop(int(x)) for x in np.asarray(ids).reshape(-1).tolist() if int(x) in self._row_of]
         if rows:
-            self._sorted = None
             r = torch.as_tensor(rows, dtype=torch.int64, device=self.device)
             self.row_group[r] = -1
             self.row_ids[r] = -1
@@ -168,28 +166,27 @@ class VectorIndex:
         self.row_group[:m] = self.row_group[live]
         self.row_group[m: self.n] = -1
         self.n = m
-        self._version += 1
         self._dead = 0
         ids = self.row_ids[:m].cpu().numpy()
         self._row_of = {int(x): i for i, x in enumerate(ids.tolist())}
-        self._sorted = None
+        self._version += 1
 
     # ------------------------------------------------------------------ search
     def _id_rows(self) -> np.ndarray:
-        """int64 [2, items]: the item ids and the row of each."""
-        n = len(self._row_of)
-        return np.stack([np.fromiter(self._row_of.keys(), dtype=np.int64, count=n),
-                         np.fromiter(self._row_of.values(), dtype=np.int64, count=n)])
+        """int64 [2, items]: the item ids and the row of each (of one moment: an update may run on another thread)."""
+        row_of = self._row_of.copy()
+        return np.stack([np.fromiter(d, dtype=np.int64, count=len(row_of)) for d in (row_of.keys(), row_of.values())])
 
     def rows_of(self, ids) -> np.ndarray:
         """Row index of each live item id (ids that are not in the index are dropped).  Vectorised
         through a sorted (id, row) table rebuilt lazily after upserts / deletes."""
         ids = np.asarray(ids, dtype=np.int64).reshape(-1)
-        if self._sorted is None:
+        table, version = self._sorted, self._version
+        if table is None or table[0] != version:
             keys, vals = self._id_rows()
             order = np.argsort(keys, kind="stable")
-            self._sorted = (keys[order], vals[order])
-        keys, vals = self._sorted
+            table = self._sorted = (version, keys[order], vals[order])
+        _, keys, vals = table
         if not len(keys) or not len(ids):
             return np.zeros(0, dtype=np.int64)
         pos = np.searchsorted(keys, ids)
@@ -231,13 +228,13 @@ class VectorIndex:
     def _live_ids(self):
         """(sorted item ids, the row of each) on the device, rebuilt after an update.  (From the mapping and not the row
         metadata: an id that one ``add`` names twice has two live rows, and the mapping says which of them is its row.)"""
-        table = self._id_table
-        if table is None or table[0] != self._version:
+        table, version = self._id_table, self._version  # (the version first: an update meanwhile makes the table stale)
+        if table is None or table[0] != version:
             with torch.inference_mode(False):
                 host = torch.from_numpy(self._id_rows())
                 ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
                 keys, order = ids.sort()
-                table = self._id_table = (self._version, keys, rows[order])
+                table = self._id_table = (version, keys, rows[order])
         return table[1:]
 
     def doc_lt_mask(self, limits, mask=None) -> torch.Tensor:
@@ -439,6 +436,5 @@ class VectorIndex:
         idx.row_group[:n] = st["group"].to(idx.device)
         idx.n = n
         idx._row_of = {int(x): i for i, x in enumerate(st["ids"].tolist()) if x >= 0}
-        idx._sorted = None
         idx._dead = n - len(idx._row_of)
         return idx

@@ -1,5 +1,6 @@
 """The device tables a ``VectorIndex`` derives from its rows and keeps until the next update."""
 import numpy as np
+import pytest
 import torch
 
 from django_assistant_bot_amd.engine.vector_index import VectorIndex
@@ -31,3 +32,60 @@ def test_id_table_names_the_rows_of_the_mapping():
     while len(idx):
         idx.remove(np.arange(3000))
         assert np.array_equal(_rows_by_table(idx, asked), idx.rows_of(asked))
+
+
+class _Interrupted(VectorIndex):
+    """Runs ``update`` once, after the id -> row mapping was read (as an update on another thread can)."""
+
+    update = None
+
+    def _id_rows(self):
+        got, update, self.update = super()._id_rows(), self.update, None
+        if update is not None:
+            update(self)
+        return got
+
+
+UPDATES = {
+    "add": lambda idx: idx.add([7, 900], torch.randn(2, 128)),
+    "remove": lambda idx: idx.remove([0, 1, 2]),
+    "compact": lambda idx: (idx.remove([3, 4]), idx.compact()),
+}
+
+
+@pytest.mark.parametrize("name", UPDATES)
+@pytest.mark.parametrize("first", ["rows_of", "_live_ids"])
+def test_tables_of_an_older_version_are_rebuilt(name, first):
+    idx = _Interrupted(128, "cpu", capacity=64, dtype=torch.float32)
+    idx.add(np.arange(100), torch.randn(100, 128))
+    asked = np.arange(1000)
+    idx.update = UPDATES[name]
+    idx.rows_of(asked) if first == "rows_of" else idx._live_ids()
+    assert idx.update is None
+    now = np.array(sorted(idx._row_of.items()))
+    assert np.array_equal(idx.rows_of(asked), now[:, 1]) and np.array_equal(_rows_by_table(idx, asked), now[:, 1])
+
+
+class _Replaced(VectorIndex):
+    """Reads its tables just before a compaction replaces the id -> row mapping."""
+
+    @property
+    def _row_of(self):
+        return self._mapping
+
+    @_row_of.setter
+    def _row_of(self, mapping):
+        if hasattr(self, "_mapping"):
+            self.rows_of([5])
+            self._live_ids()
+        self._mapping = mapping
+
+
+def test_compaction_shows_its_version_last():
+    idx = _Replaced(128, "cpu", capacity=64, dtype=torch.float32)
+    idx.add(np.arange(100), torch.randn(100, 128))
+    idx.remove(np.arange(0, 100, 3))
+    idx.compact()
+    now = np.array(sorted(idx._row_of.items()))
+    assert np.array_equal(idx.rows_of(np.arange(100)), now[:, 1])
+    assert np.array_equal(_rows_by_table(idx, np.arange(100)), now[:, 1])
