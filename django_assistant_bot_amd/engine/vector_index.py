@@ -225,17 +225,33 @@ class VectorIndex:
                 m[qi, torch.from_numpy(rows).to(self.device)] = True
         return self._pack_rows(m)
 
+    def _kept(self, slot: str, key, build):
+        """Device tensors derived from the rows, built once and kept in ``slot`` until ``key`` changes.  They are built on
+        the caller's stream and read on any: a reader on another stream waits for the build and holds the memory until
+        its own work is done."""
+        entry = getattr(self, slot)
+        cuda = self.device.type == "cuda"
+        stream = torch.cuda.current_stream(self.device) if cuda else None
+        if entry is None or entry[0] != key:
+            with torch.inference_mode(False):
+                tensors = build()
+            entry = (key, tensors, stream, stream.record_event() if cuda else None)
+            setattr(self, slot, entry)
+        elif stream != entry[2]:
+            stream.wait_event(entry[3])
+            for t in entry[1]:
+                t.record_stream(stream)
+        return entry[1]
+
     def _live_ids(self):
         """(sorted item ids, the row of each) on the device, rebuilt after an update.  (From the mapping and not the row
         metadata: an id that one ``add`` names twice has two live rows, and the mapping says which of them is its row.)"""
-        table, version = self._id_table, self._version  # (the version first: an update meanwhile makes the table stale)
-        if table is None or table[0] != version:
-            with torch.inference_mode(False):
-                host = torch.from_numpy(self._id_rows())
-                ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
-                keys, order = ids.sort()
-                table = self._id_table = (version, keys, rows[order])
-        return table[1:]
+        def build():
+            host = torch.from_numpy(self._id_rows())
+            ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
+            keys, order = ids.sort()
+            return keys, rows[order]
+        return self._kept("_id_table", self._version, build)  # (the version of before the build)
 
     def doc_lt_mask(self, limits, mask=None) -> torch.Tensor:
         """Rows whose document id is < limits[q] (the ingest dedup filter ``document__id__lt``),
@@ -400,18 +416,15 @@ class VectorIndex:
 
     def _sample_rows(self, ns: int):
         """The strided 1/64 row sample (in the index's own layout) and its groups, cached until the next update."""
-        key = (ns, self._version)
-        sample = self._sample
-        if sample is None or sample[0] != key:
+        def build():
             rows = torch.arange(0, ns * self.sample_stride, self.sample_stride, device=self.device)
-            with torch.inference_mode(False):
-                if self.frag:  # whole tiles of 128 rows: the last row again behind the sample
-                    padded = torch.arange(-(-ns // 128) * 128, device=self.device).clamp_(max=ns - 1) * self.sample_stride
-                    data = ops.shuffle_weights(ops.gather_shuffled_rows(self.vecs, padded))
-                else:
-                    data = self.rows_data(rows).contiguous()
-                sample = self._sample = (key, data, self.row_group[rows])
-        return sample[1:]
+            if self.frag:  # whole tiles of 128 rows: the last row again behind the sample
+                padded = torch.arange(-(-ns // 128) * 128, device=self.device).clamp_(max=ns - 1) * self.sample_stride
+                data = ops.shuffle_weights(ops.gather_shuffled_rows(self.vecs, padded))
+            else:
+                data = self.rows_data(rows).contiguous()
+            return data, self.row_group[rows]
+        return self._kept("_sample", (ns, self._version), build)
 
     # ------------------------------------------------------------------ persistence
     def save(self, path: str) -> None:

@@ -89,3 +89,41 @@ def test_compaction_shows_its_version_last():
     now = np.array(sorted(idx._row_of.items()))
     assert np.array_equal(idx.rows_of(np.arange(100)), now[:, 1])
     assert np.array_equal(_rows_by_table(idx, np.arange(100)), now[:, 1])
+
+
+@pytest.mark.gpu
+def test_tables_built_on_one_stream_are_read_on_another():
+    """The id table and the row sample queued behind a long kernel on one stream and used at once on a second, which also
+    outlives the entry: masks and scores as on one stream."""
+    n, dim, k = 70_000, 128, 20
+    g = torch.Generator(device="cuda").manual_seed(0)
+    idx = VectorIndex(dim, "cuda", capacity=n + 10)
+    idx.add(np.random.default_rng(0).permutation(n), torch.randn(n, dim, device="cuda", generator=g))
+    idx.threshold_min_rows = 1
+    q = torch.randn(4, dim, device="cuda", generator=g)
+    allowed = [np.arange(i, n, 7) for i in range(4)]
+    mask, (sample, groups) = idx.allow_mask(allowed), idx._sample_rows(n // 64 // 4 * 4)
+    vals, ids, _ = idx.search(q, k)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(3):
+        idx._version += 1  # (rows as they were: both tables are built anew)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(200_000_000)  # some 0.1 s
+            for t in (*idx._live_ids(), *idx._sample_rows(n // 64 // 4 * 4)):
+                assert t.is_cuda
+        del t
+        with torch.cuda.stream(b):
+            got = idx.allow_mask(allowed)
+            s2, g2 = (t.clone() for t in idx._sample_rows(n // 64 // 4 * 4))
+            idx._id_table = idx._sample = None  # the tables are freed with b's reads in flight
+            junk = [torch.full((n,), -1, device="cuda") for _ in range(8)]
+        torch.cuda.synchronize()
+        assert torch.equal(got, mask) and torch.equal(s2, sample) and torch.equal(g2, groups)
+        with torch.cuda.stream(b):
+            got = idx.search(q, k)
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], vals) and torch.equal(got[1], ids)
+        del junk
+    idx.remove(np.arange(n))
+    assert not idx.allow_mask(allowed).any()  # a table without ids
