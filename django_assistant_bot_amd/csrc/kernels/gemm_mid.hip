@@ -27,7 +27,10 @@
 //     counted wait has retired the stores (no drain); the owner keeps its partial in registers,
 //     waits for each flag (bounded spin), adds the partials with sc1 loads in segment order (no
 //     fence needed: cdna_hip_programming.md section 5 item 2), clears the flags and runs the
-//     epilogue.  Only owners wait, on producers that never wait, so there is no deadlock (and the
+//     epilogue.  A flag holds the
+//     number of the launch that raised it (the workgroups count their ends in the workspace, so a
+//     replayed graph goes on counting): what a launch that gave up left raised, or raised late, means
+//     nothing to the next.  Only owners wait, on producers that never wait, so there is no deadlock (and the
 //     grid is at most one workgroup per CU).  Replaces a last-arriver combine (every segment stored
 //     and drained, then an atomic ticket) that cost 5-9 us per launch on the small projections
 //     (profiles/gemm_mid_r6.md).
@@ -46,7 +49,9 @@ struct GMid {
   bf16* C;
   const bf16* residual;   // GLU epilogues with RES: fp32 bias [gate N / 2 | up N / 2] instead
   float* slabs;  // [tiles_m][gn][2] partial tiles of 128 x 256 fp32 (in accumulator order)
-  int* cnt;      // [tiles_m][gn][2] ready flags of the stored partial tiles, zero at rest
+  int* cnt;      // [tiles_m][gn][2] ready flags of the stored partial tiles (the launch that stored them), zero at rest
+  unsigned* ended;  // workgroups that ended, over all launches on this workspace
+  long spin_limit;
   int M, N, K;
   long lda, ldc, ldr;
   int tiles_m, tiles_n, kt;
@@ -118,7 +123,13 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
 
   // ---- which group / row tile this block is: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that whole
   // groups leave over are joined, XCD after XCD, into further groups
-  const int bid = blockIdx.x;
+  const int bid = blockIdx.x, tid = threadIdx.x;
+  // the launch's number, the same for all of its workgroups: this one has not ended yet, so its launch adds less than
+  // gridDim.x to the count (which may wrap: 2^32 is a multiple of 256 workgroups).  A scalar load: nothing precedes it
+  const int launch = (int)(*p.ended / gridDim.x) + 1;
+  auto count_end = [&]() {
+    if (tid == 0) __hip_atomic_fetch_add(p.ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   const int x = bid & 7, slot = bid >> 3;
   int g = slot / p.tiles_m, mt = slot - g * p.tiles_m, j = x * p.gpx + g;
   if (g >= p.gpx) {
@@ -126,13 +137,13 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
     g = u / p.tiles_m;
     mt = u - g * p.tiles_m;
     j = 8 * p.gpx + g;
-    if (j >= p.gn) return;  // whole workgroup (uniform)
+    if (j >= p.gn) return count_end();  // whole workgroup (uniform)
   }
   const int start = grp_start(j, p.q, p.r);
   const int end = start + p.q + (j < p.r ? 1 : 0);
-  if (end <= start) return;
+  if (end <= start) return count_end();
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = w >> 2, wc = w & 3;
   const int li = lane & 15, gq = lane >> 4;
@@ -248,7 +259,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   auto slab_off = [&](int jj, int side) { return (unsigned)(((mt * p.gn + jj) * 2 + side) * kSlabFloats) * 4u; };
   auto flag_of = [&](int jj, int side) { return p.cnt + (mt * p.gn + jj) * 2 + side; };
   auto raise_flag = [&]() {  // after every wave's stores retired and a barrier
-    if (tid == 0) __hip_atomic_store(p.cnt + pend_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(p.cnt + pend_flag, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     pend_flag = -1;
   };
   while (it < end) {
@@ -344,8 +355,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
           int* fl = flag_of(jj, sd);
           if (tid == 0) {
             long spins = 0;
-            while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-              if (++spins > (1L << 22)) {
+            while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != launch) {
+              if (++spins > p.spin_limit) {
                 ok = false;  // a producer never published (cannot happen in a healthy launch)
                 break;
               }
@@ -470,6 +481,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
 #pragma unroll
       for (int jn = 0; jn < 4; ++jn) acc[i][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  count_end();
 }
 
 namespace {
@@ -508,8 +520,10 @@ int gemm_mid_groups(int M, int N, int K) {
   return us(all) < 0.94f * us(whole) ? all : whole;
 }
 
-// Workspace the launcher needs: partial slabs (bytes) and arrival counters (ints).
-long gemm_mid_slab_bytes() { return (long)cu_count() * 2 * kSlabFloats * 4; }
+// Workspace the launcher needs: partial slabs and behind them a line with the count of ended workgroups (bytes), and
+// ready flags (ints).
+static long slabs_end() { return (long)cu_count() * 2 * kSlabFloats * 4; }
+long gemm_mid_slab_bytes() { return slabs_end() + 128; }
 // ready flags of the partial tiles: two per (row tile, group) <= two per workgroup
 int gemm_mid_counters(int M, int N) {
   (void)M;
@@ -518,14 +532,15 @@ int gemm_mid_counters(int M, int N) {
 }
 
 // epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over
-// 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes() bytes; cnt: >= gemm_mid_counters()
-// ints, zero on first use (the launch leaves them zero).  variant (A/B harness only): 0 default
+// 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes()
+// bytes, the last 128 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).
+// spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
 // (BK 64), 32 / 64 force the K-step, + 1000 = DIAG 1 (split tiles not combined: timing only).
 // BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank
 // conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
 int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const void* residual, long ldr, int M, int N,
              int K, int epilogue, void* slabs, long slab_bytes, int* cnt, int n_cnt, hipStream_t s, int variant,
-             int b_group) {
+             int b_group, long spin_limit) {
   if (!gemm_mid_ok(M, N, K, lda)) return hipErrorInvalidValue;
   if (b_group != 1 && b_group != 8) return hipErrorInvalidValue;
   if (epilogue != MID_NONE && !glu8_epilogue(epilogue)) return hipErrorInvalidValue;
@@ -551,6 +566,8 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.tiles_n = N / 256;
   p.kt = K / bk;
   const int grid = cu_count() & ~7;
+  p.ended = (unsigned*)((char*)slabs + slabs_end());
+  p.spin_limit = spin_limit;
   p.spx = grid / 8;
   p.gpx = p.spx / p.tiles_m;
   p.gn = gemm_mid_groups(M, N, K);

@@ -1,0 +1,81 @@
+"""The ready flags of gemm_mid's divided tiles hold the number of the launch that raised them."""
+import pytest
+import torch
+
+from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.ops import kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# tiles cut between two groups, between many, and between groups joined over the XCDs
+SHAPES = [(300, 512, 4096), (1093, 4096, 1024), (2200, 2560, 1024), (44, 256, 8192)]
+
+
+def _case(M, N, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    A = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+    W = (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).to(torch.bfloat16)
+    return A, ops.shuffle_weights(W), A.float() @ W.float().t()
+
+
+def _close(out, exp):
+    # one rounding to bf16 (2^-8 of the value); the fp32 sums are far below 1e-4
+    return (out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-4
+
+
+def _launch(A, B, out, spin_limit):
+    s = torch.cuda.current_stream().cuda_stream
+    slabs, cnt = kernels._mid_workspace(A.device, s)
+    M, K = A.shape
+    kernels.native().gemm_mid(A.data_ptr(), K, B.data_ptr(), out.data_ptr(), out.stride(0), 0, 0, M, B.shape[0], K, 0,
+                              slabs.data_ptr(), slabs.numel() * 4, cnt.data_ptr(), cnt.numel(), s, spin_limit=spin_limit)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_a_launch_that_gave_up_leaves_nothing_for_the_next(M, N, K):
+    """Owners that look at a flag once and give up write NaN over their tile; the flags raised behind them belong to that
+    launch, and the launches after it take only their own partial tiles."""
+    for seed in range(4):
+        A, B, exp = _case(M, N, K, seed)
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        _launch(A, B, out, 0)
+        assert (_close(out, exp) | out.isnan()).all()
+        for other in range(2):
+            A, B, exp = _case(M, N, K, 100 + 10 * seed + other)
+            assert _close(ops.kernels.gemm_mid(A, B), exp).all()
+
+
+def test_the_count_of_launches_may_wrap():
+    A, B, exp = _case(*SHAPES[1], 0)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ended = kernels._mid_workspace(A.device, s.cuda_stream)[0].view(torch.int32)[-32]
+        s.wait_stream(torch.cuda.default_stream())
+        grid = torch.cuda.get_device_properties(0).multi_processor_count & ~7
+        assert (1 << 32) % grid == 0 and not ended
+        ended.fill_(-2 * grid)
+        for i in range(5):
+            assert _close(ops.kernels.gemm_mid(A, B), exp).all()
+            assert int(ended) == (i - 1) * grid
+
+
+def test_replays_go_on_counting():
+    """A captured launch replayed between eager ones on its workspace."""
+    (M, N, K), s = SHAPES[2], torch.cuda.Stream()
+    cases = [_case(M, N, K, seed) for seed in range(3)]
+    A, B = cases[0][0].clone(), cases[0][1].clone()
+    with torch.cuda.stream(s):
+        s.wait_stream(torch.cuda.default_stream())
+        ops.kernels.gemm_mid(A, B)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            outs = [ops.kernels.gemm_mid(A, B) for _ in range(3)]
+        for i in range(6):
+            a, b, exp = cases[i % 3]
+            A.copy_(a)
+            B.copy_(b)
+            g.replay()
+            a2, b2, exp2 = cases[(i + 1) % 3]
+            eager = ops.kernels.gemm_mid(a2, b2)
+            s.synchronize()
+            assert all(_close(o, exp).all() for o in outs) and _close(eager, exp2).all()
