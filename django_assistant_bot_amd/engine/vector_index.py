@@ -45,6 +45,7 @@ class VectorIndex:
         self._sample = None
         self._id_table = None
         self._dead = 0
+        self._twice = False  # an id may have live rows beside the mapping's one (see ``add``)
         self._grow(max(64, capacity))
 
     # ------------------------------------------------------------------ storage
@@ -126,6 +127,8 @@ class VectorIndex:
                 else:
                     rows[i] = r
             if fresh:
+                # (a new id that one call names twice gets two rows; the mapping keeps the later one)
+                self._twice |= len({idl[i] for i in fresh}) < len(fresh)
                 need = self.n + len(fresh)
                 if need > self._cap:
                     self._grow(max(need, 2 * self._cap))
@@ -243,12 +246,20 @@ class VectorIndex:
                 t.record_stream(stream)
         return entry[1]
 
+    def _live_rows(self):
+        """(item ids, rows) of the live rows, on the device."""
+        live = (self.row_group[: self.n] >= 0).nonzero().flatten()
+        return self.row_ids[live], live
+
     def _live_ids(self):
-        """(sorted item ids, the row of each) on the device, rebuilt after an update.  (From the mapping and not the row
-        metadata: an id that one ``add`` names twice has two live rows, and the mapping says which of them is its row.)"""
+        """(sorted item ids, the row of each) on the device, rebuilt after an update.  From the row metadata (first search of 60k rows:
+        0.36 ms) unless an id may have a second live row: the mapping says which of them is its row (2.25 ms)."""
         def build():
-            host = torch.from_numpy(self._id_rows())
-            ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
+            if self._twice:
+                host = torch.from_numpy(self._id_rows())
+                ids, rows = (host.pin_memory() if self.device.type == "cuda" else host).to(self.device, non_blocking=True)
+            else:
+                ids, rows = self._live_rows()
             keys, order = ids.sort()
             return keys, rows[order]
         return self._kept("_id_table", self._version, build)  # (the version of before the build)
@@ -450,4 +461,5 @@ class VectorIndex:
         idx.n = n
         idx._row_of = {int(x): i for i, x in enumerate(st["ids"].tolist()) if x >= 0}
         idx._dead = n - len(idx._row_of)
+        idx._twice = int((st["group"] >= 0).sum()) != len(idx._row_of)
         return idx

@@ -16,19 +16,25 @@ def _rows_by_table(idx, ids):
     return rows[at[ok]]
 
 
-def test_id_table_names_the_rows_of_the_mapping():
-    """Ids that one ``add`` names twice (the later vector is the item's), updates, removals, a compaction."""
+@pytest.mark.parametrize("twice", [False, True])
+def test_id_table_names_the_rows_of_the_mapping(twice, tmp_path):
+    """Ids that one ``add`` names twice (the later vector is the item's) or once, updates, removals, a compaction, a
+    snapshot."""
     rng = np.random.default_rng(0)
     idx = VectorIndex(128, "cpu", capacity=64, dtype=torch.float32)
     asked = np.arange(-5, 4000)
     for step in range(4):
         ids = rng.integers(0, 3000, 2000)
+        ids = ids if twice else np.unique(ids)
         if step == 2:
             idx.remove(rng.integers(0, 3000, 2500))
         idx.add(ids, torch.from_numpy(rng.standard_normal((len(ids), 128)).astype(np.float32)))
         if step == 3:
             idx.compact()
-        assert np.array_equal(_rows_by_table(idx, asked), idx.rows_of(asked))
+        assert np.array_equal(_rows_by_table(idx, asked), idx.rows_of(asked)) and idx._twice == twice
+    idx.save(str(tmp_path / "rows"))
+    idx = VectorIndex.load(str(tmp_path / "rows"), "cpu")
+    assert np.array_equal(_rows_by_table(idx, asked), idx.rows_of(asked))
     while len(idx):
         idx.remove(np.arange(3000))
         assert np.array_equal(_rows_by_table(idx, asked), idx.rows_of(asked))
@@ -39,11 +45,17 @@ class _Interrupted(VectorIndex):
 
     update = None
 
-    def _id_rows(self):
-        got, update, self.update = super()._id_rows(), self.update, None
+    def _then(self, got):
+        update, self.update = self.update, None
         if update is not None:
             update(self)
         return got
+
+    def _id_rows(self):
+        return self._then(super()._id_rows())
+
+    def _live_rows(self):
+        return self._then(super()._live_rows())
 
 
 UPDATES = {
@@ -54,9 +66,10 @@ UPDATES = {
 
 
 @pytest.mark.parametrize("name", UPDATES)
-@pytest.mark.parametrize("first", ["rows_of", "_live_ids"])
-def test_tables_of_an_older_version_are_rebuilt(name, first):
+@pytest.mark.parametrize("first,twice", [("rows_of", False), ("_live_ids", False), ("_live_ids", True)])
+def test_tables_of_an_older_version_are_rebuilt(name, first, twice):
     idx = _Interrupted(128, "cpu", capacity=64, dtype=torch.float32)
+    idx._twice = twice
     idx.add(np.arange(100), torch.randn(100, 128))
     asked = np.arange(1000)
     idx.update = UPDATES[name]
@@ -83,6 +96,7 @@ class _Replaced(VectorIndex):
 
 def test_compaction_shows_its_version_last():
     idx = _Replaced(128, "cpu", capacity=64, dtype=torch.float32)
+    idx._twice = True
     idx.add(np.arange(100), torch.randn(100, 128))
     idx.remove(np.arange(0, 100, 3))
     idx.compact()
@@ -105,7 +119,7 @@ def test_tables_built_on_one_stream_are_read_on_another():
     mask, (sample, groups) = idx.allow_mask(allowed), idx._sample_rows(n // 64 // 4 * 4)
     vals, ids, _ = idx.search(q, k)
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
-    for _ in range(3):
+    for idx._twice in (False, True, False):  # (from the row metadata, from the mapping)
         idx._version += 1  # (rows as they were: both tables are built anew)
         torch.cuda.synchronize()
         with torch.cuda.stream(a):
