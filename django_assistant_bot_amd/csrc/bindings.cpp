@@ -34,16 +34,21 @@ PYBIND11_MODULE(_native, m) {
   // one-shot all-reduce over IPC peer buffers (parallel/custom_allreduce.py)
   m.def("allreduce_signal_bytes", &dab::allreduce_signal_bytes);
   m.def("custom_allreduce", [](const std::vector<uintptr_t>& bases, int rank, u data, long nbytes, long half_bytes,
-                               long spin_limit, u s) {
-    check(dab::custom_allreduce(bases, rank, VP(data), nbytes, half_bytes, spin_limit, ST(s)), "custom_allreduce");
-  });
+                               long spin_limit, u s, int blocks) {
+    check(dab::custom_allreduce(bases, rank, VP(data), nbytes, half_bytes, spin_limit, ST(s), blocks), "custom_allreduce");
+  }, py::arg("bases"), py::arg("rank"), py::arg("data"), py::arg("nbytes"), py::arg("half_bytes"), py::arg("spin_limit"),
+     py::arg("s"), py::arg("blocks") = dab::kAllReduceBlocks);
+  m.attr("ALLREDUCE_BLOCKS") = dab::kAllReduceBlocks;
   m.def("custom_allreduce_rmsnorm", [](const std::vector<uintptr_t>& bases, int rank, u slabs, int S, long slab_stride,
                                        u x, u res_in, u res_out, u out, u w, int rows, int cols, float eps,
-                                       long half_bytes, long spin_limit, u s) {
+                                       long half_bytes, long spin_limit, u s, int blocks) {
     check(dab::custom_allreduce_rmsnorm(bases, rank, (const float*)slabs, S, slab_stride, CVP(x), CVP(res_in),
-                                        VP(res_out), VP(out), CVP(w), rows, cols, eps, half_bytes, spin_limit, ST(s)),
+                                        VP(res_out), VP(out), CVP(w), rows, cols, eps, half_bytes, spin_limit, ST(s),
+                                        blocks),
           "custom_allreduce_rmsnorm");
-  });
+  }, py::arg("bases"), py::arg("rank"), py::arg("slabs"), py::arg("S"), py::arg("slab_stride"), py::arg("x"),
+     py::arg("res_in"), py::arg("res_out"), py::arg("out"), py::arg("w"), py::arg("rows"), py::arg("cols"), py::arg("eps"),
+     py::arg("half_bytes"), py::arg("spin_limit"), py::arg("s"), py::arg("blocks") = dab::kAllReduceBlocks);
   m.def("allreduce_buffer_alloc", [](long bytes, bool uncached) {
     uintptr_t p = 0;
     check(dab::allreduce_buffer_alloc(bytes, uncached ? 1 : 0, &p), "allreduce_buffer_alloc");

@@ -5,8 +5,8 @@
 // Here every rank reads all W-1 peers directly, one xGMI hop each and all links at once.
 //
 //   * Rank r owns one IPC allocation: a signal area, then two staging halves of `half_bytes`.
-//   * The grid size is fixed (AR_BLOCKS).  Block b owns a contiguous segment of the vector.  Per
-//     call, block b:
+//   * The grid size is fixed for a group (AR_BLOCKS, fewer where its ranks share a device).  Block b
+//     owns a contiguous segment of the vector.  Per call, block b:
 //       1. copies its segment of the local input into staging[e & 1];
 //       2. writes system-scope release flags into every peer's signal area;
 //       3. waits for the W flags addressed to it;
@@ -37,7 +37,7 @@
 namespace dab {
 
 constexpr int AR_MAX_RANKS = 8;
-constexpr int AR_BLOCKS = 64;
+constexpr int AR_BLOCKS = kAllReduceBlocks;
 constexpr int AR_THREADS = 512;
 
 struct ArSignal {
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_kernel(ArParams p) {
   const uint32_t e = e_sh;
   const size_t stage_off = sig_bytes + (size_t)(e & 1) * p.half_bytes;
 
-  const long per = (p.n16 + AR_BLOCKS - 1) / AR_BLOCKS;
+  const long per = (p.n16 + gridDim.x - 1) / gridDim.x;
   const long s0 = min(p.n16, (long)b * per), s1 = min(p.n16, s0 + per);
   u32x4* dst = reinterpret_cast<u32x4*>(p.data);
   auto poison = [&]() {  // bf16 quiet NaN over this block's segment
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_kernel(ArParams p) {
 // One TP decode all-reduce site was three launches: slab_reduce (this rank's fp32 split-K slabs ->
 // bf16 partial) -> allreduce_kernel -> rmsnorm (+ residual).  Here one launch does all three with
 // the same arithmetic, so at W = 1 the result is bitwise that of the sequence:
-//   1. block b sums, for each of its rows (b, b + 64, ...), the S slabs in slab order and rounds to
+//   1. block b sums, for each of its rows (b, b + the grid, ...), the S slabs in slab order and rounds to
 //      bf16 (slab_reduce), into this rank's staging half (or copies a bf16 partial when S == 0);
 //   2. the flag exchange of allreduce_kernel (same signal area, epochs, parity, bounded spins,
 //      sticky error + NaN poisoning);
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(AR_THREADS) void allreduce_kernel(ArParams p) {
 //      all-reduce's output), the residual is added in bf16, and the RMSNorm runs with the thread
 //      mapping and block reduction of rmsnorm_kernel<NT, VPT> (the launcher picks NT / VPT exactly as
 //      rmsnorm's DAB_ROW_DISPATCH does).
-// Every launch runs all AR_BLOCKS blocks (rowless blocks still exchange flags), so every block's
+// Every launch runs all of the group's blocks (rowless blocks still exchange flags), so every block's
 // epoch -- and the staging parity -- stays in step with allreduce_kernel's calls.
 struct ArNormParams {
   char* base[AR_MAX_RANKS];
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(NT) void allreduce_rmsnorm_kernel(ArNormParams p) {
   const int nvec = p.cols >> 3;
   auto poison = [&]() {
     const u32x4 nan4 = {0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
-    for (int row = b; row < p.rows; row += AR_BLOCKS)
+    for (int row = b; row < p.rows; row += gridDim.x)
       for (int i = tid; i < nvec; i += NT) {
         reinterpret_cast<u32x4*>(p.out + (size_t)row * p.cols)[i] = nan4;
         if (p.res_in) reinterpret_cast<u32x4*>(p.res_out + (size_t)row * p.cols)[i] = nan4;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(NT) void allreduce_rmsnorm_kernel(ArNormParams p) {
   }
   // 1. this rank's partial rows -> staging
   u32x4* mine = reinterpret_cast<u32x4*>(p.base[p.rank] + stage_off);
-  for (int row = b; row < p.rows; row += AR_BLOCKS) {
+  for (int row = b; row < p.rows; row += gridDim.x) {
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       const int i = tid + k * NT;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(NT) void allreduce_rmsnorm_kernel(ArNormParams p) {
 #pragma unroll
   for (int r = 0; r < W; ++r) stage[r] = reinterpret_cast<const u32x4*>(p.base[r] + stage_off);
   const u32x4* wr = reinterpret_cast<const u32x4*>(p.w);
-  for (int row = b; row < p.rows; row += AR_BLOCKS) {
+  for (int row = b; row < p.rows; row += gridDim.x) {
     float v[VPT][8];
     float ss = 0.f;
 #pragma unroll
@@ -289,9 +289,9 @@ __global__ __launch_bounds__(NT) void allreduce_rmsnorm_kernel(ArNormParams p) {
 }
 
 template <int W>
-static void launch_ar_norm(const ArNormParams& p, hipStream_t s) {
+static void launch_ar_norm(const ArNormParams& p, int blocks, hipStream_t s) {
   const int nvec = p.cols / 8;
-  const dim3 grid(AR_BLOCKS);
+  const dim3 grid(blocks);
   if (nvec <= 64) hipLaunchKernelGGL((allreduce_rmsnorm_kernel<W, 64, 1>), grid, dim3(64), 0, s, p);
   else if (nvec <= 128) hipLaunchKernelGGL((allreduce_rmsnorm_kernel<W, 128, 1>), grid, dim3(128), 0, s, p);
   else if (nvec <= 256) hipLaunchKernelGGL((allreduce_rmsnorm_kernel<W, 256, 1>), grid, dim3(256), 0, s, p);
@@ -303,9 +303,9 @@ static void launch_ar_norm(const ArNormParams& p, hipStream_t s) {
 int custom_allreduce_rmsnorm(const std::vector<uintptr_t>& bases, int rank, const float* slabs, int S,
                              long slab_stride, const void* x, const void* res_in, void* res_out, void* out,
                              const void* w, int rows, int cols, float eps, long half_bytes, long spin_limit,
-                             hipStream_t s) {
+                             hipStream_t s, int blocks) {
   const int W = (int)bases.size();
-  if (W < 1 || W > AR_MAX_RANKS || rank < 0 || rank >= W) return hipErrorInvalidValue;
+  if (W < 1 || W > AR_MAX_RANKS || rank < 0 || rank >= W || blocks < 1 || blocks > AR_BLOCKS) return hipErrorInvalidValue;
   if (rows <= 0) return 0;
   if (cols % 8 || cols > 16384 || (long)rows * cols * 2 > half_bytes) return hipErrorInvalidValue;
   if ((S > 0 && (!slabs || slab_stride % 4 || slab_stride < (long)rows * cols)) || (S == 0 && !x) || S < 0)
@@ -328,22 +328,22 @@ int custom_allreduce_rmsnorm(const std::vector<uintptr_t>& bases, int rank, cons
   p.cols = cols;
   p.eps = eps;
   switch (W) {
-    case 1: launch_ar_norm<1>(p, s); break;
-    case 2: launch_ar_norm<2>(p, s); break;
-    case 3: launch_ar_norm<3>(p, s); break;
-    case 4: launch_ar_norm<4>(p, s); break;
-    case 5: launch_ar_norm<5>(p, s); break;
-    case 6: launch_ar_norm<6>(p, s); break;
-    case 7: launch_ar_norm<7>(p, s); break;
-    default: launch_ar_norm<8>(p, s); break;
+    case 1: launch_ar_norm<1>(p, blocks, s); break;
+    case 2: launch_ar_norm<2>(p, blocks, s); break;
+    case 3: launch_ar_norm<3>(p, blocks, s); break;
+    case 4: launch_ar_norm<4>(p, blocks, s); break;
+    case 5: launch_ar_norm<5>(p, blocks, s); break;
+    case 6: launch_ar_norm<6>(p, blocks, s); break;
+    case 7: launch_ar_norm<7>(p, blocks, s); break;
+    default: launch_ar_norm<8>(p, blocks, s); break;
   }
   return hipGetLastError();
 }
 
 int custom_allreduce(const std::vector<uintptr_t>& bases, int rank, void* data, long nbytes, long half_bytes,
-                     long spin_limit, hipStream_t s) {
+                     long spin_limit, hipStream_t s, int blocks) {
   const int W = (int)bases.size();
-  if (W < 1 || W > AR_MAX_RANKS || rank < 0 || rank >= W) return hipErrorInvalidValue;
+  if (W < 1 || W > AR_MAX_RANKS || rank < 0 || rank >= W || blocks < 1 || blocks > AR_BLOCKS) return hipErrorInvalidValue;
   if (nbytes % 16 || nbytes > half_bytes || ((uintptr_t)data & 15)) return hipErrorInvalidValue;
   if (nbytes == 0) return 0;
   ArParams p;
@@ -353,7 +353,7 @@ int custom_allreduce(const std::vector<uintptr_t>& bases, int rank, void* data, 
   p.half_bytes = half_bytes;
   p.rank = rank;
   p.spin_limit = spin_limit;
-  const dim3 grid(AR_BLOCKS), block(AR_THREADS);
+  const dim3 grid(blocks), block(AR_THREADS);
   switch (W) {
     case 1: hipLaunchKernelGGL(allreduce_kernel<1>, grid, block, 0, s, p); break;
     case 2: hipLaunchKernelGGL(allreduce_kernel<2>, grid, block, 0, s, p); break;

@@ -35,6 +35,23 @@ class CustomAllReduceError(RuntimeError):
     pass
 
 
+def blocks_for(devices: list, most: int) -> int:
+    """Workgroups of each rank's all-reduce; ``devices``: per rank, (device, its CUs).  Every rank computes the same.
+
+    A workgroup spins on its CU until all peers' have arrived.  Where W ranks share one device, W - 1 of them may spin
+    while the last one's next kernel still has to be placed, and a workgroup of gemm256 takes a CU's whole register file
+    (8 waves of 256 registers): at 8 ranks and 64 workgroups, 448 spinning ones could hold all of the 256 CUs and the rank
+    they wait for never ran.  So the others' workgroups together stay within 7/8 of the CUs, and an eighth of the device is
+    free for the rank behind (gemm_mid, whose workgroups wait for each other, fits beside a spinning one).  8 ranks on 256
+    CUs: 32 workgroups; up to 4, or one rank a device: all 64."""
+    blocks = most
+    for key, cus in devices:
+        others = sum(k == key for k, _ in devices) - 1
+        if others:
+            blocks = min(blocks, cus * 7 // 8 // others)
+    return max(1, blocks)
+
+
 class CustomAllReduce:
     def __init__(self, group=None, device=None, max_bytes: int = 8 << 20, spin_limit: int = 1 << 24,
                  exchange_group=None, uncached: bool = True):
@@ -53,13 +70,15 @@ class CustomAllReduce:
         sig = n.allreduce_signal_bytes()
         with torch.cuda.device(self.device):
             self.base = n.allreduce_buffer_alloc(sig + 2 * self.max_bytes, uncached)
-            handle = n.ipc_get_handle(self.base)
-            handles = [None] * self.world
+            props = torch.cuda.get_device_properties(self.device)
+            key = (str(props.uuid), props.pci_domain_id, props.pci_bus_id, props.pci_device_id)
+            mine = (n.ipc_get_handle(self.base), (key, props.multi_processor_count))
+            ranks = [mine]
             if self.world > 1:
-                dist.all_gather_object(handles, handle, group=exchange_group or group)
-            else:
-                handles = [handle]
-            self.bases = [self.base if r == self.rank else n.ipc_open_handle(handles[r]) for r in range(self.world)]
+                ranks = [None] * self.world
+                dist.all_gather_object(ranks, mine, group=exchange_group or group)
+            self.blocks = blocks_for([device for _, device in ranks], n.ALLREDUCE_BLOCKS)
+            self.bases = [self.base if r == self.rank else n.ipc_open_handle(ranks[r][0]) for r in range(self.world)]
             for b in self.bases:
                 n.ipc_probe(b)  # a bad mapping raises here, never inside the kernel
         self._closed = False
@@ -86,7 +105,7 @@ class CustomAllReduce:
             self.skip_next -= 1
             return x
         self._n.custom_allreduce(self.bases, self.rank, x.data_ptr(), x.numel() * 2, self.max_bytes, self.spin_limit,
-                                 stream(x))
+                                 stream(x), self.blocks)
         return x
 
     def check_error(self) -> None:
@@ -125,7 +144,8 @@ class CustomAllReduce:
             self.bases, self.rank, partial.data_ptr() if slabs else 0, partial.shape[0] if slabs else 0,
             rows * cols if slabs else 0, 0 if slabs else partial.data_ptr(),
             residual.data_ptr() if residual is not None else 0, res_out.data_ptr() if res_out is not None else 0,
-            out.data_ptr(), w.data_ptr(), rows, cols, float(eps), self.max_bytes, self.spin_limit, stream(partial))
+            out.data_ptr(), w.data_ptr(), rows, cols, float(eps), self.max_bytes, self.spin_limit, stream(partial),
+            self.blocks)
         return out, res_out
 
     def enqueue_error_check(self, s: int | None = None) -> None:
