@@ -234,13 +234,15 @@ class VectorIndex:
         its own work is done."""
         entry = getattr(self, slot)
         cuda = self.device.type == "cuda"
-        stream = torch.cuda.current_stream(self.device) if cuda else None
+        handle = torch._C._cuda_getCurrentRawStream(self.vecs.device.index) if cuda else 0  # (a stream object: 3 us)
         if entry is None or entry[0] != key:
             with torch.inference_mode(False):
                 tensors = build()
-            entry = (key, tensors, stream, stream.record_event() if cuda else None)
+            event = torch.cuda.current_stream(self.vecs.device).record_event() if cuda else None
+            entry = (key, tensors, handle, event)
             setattr(self, slot, entry)
-        elif stream != entry[2]:
+        elif handle != entry[2]:
+            stream = torch.cuda.current_stream(self.vecs.device)
             stream.wait_event(entry[3])
             for t in entry[1]:
                 t.record_stream(stream)
