@@ -599,8 +599,8 @@ PYBIND11_MODULE(_native, m) {
   m.def("unit_rows", [](u x, long ldx, u out, int rows, int cols, u s) {
     check(dab::unit_rows((const float*)x, ldx, VP(out), rows, cols, ST(s)), "unit_rows");
   });
-  m.def("rank_value", [](u scores, long ld, int rows, int n, int r, u thr, u cnt, u s) {
-    check(dab::rank_value((const float*)scores, ld, rows, n, r, (float*)thr, (int*)cnt, ST(s)), "rank_value");
+  m.def("rank_value", [](u scores, long ld, int rows, int n, int r, float slack, u thr, u cnt, u s) {
+    check(dab::rank_value((const float*)scores, ld, rows, n, r, slack, (float*)thr, (int*)cnt, ST(s)), "rank_value");
   });
   m.def("rank_hits", [](u cand_val, u cand_idx, u cnt, u thr, int cap, int rows, int k, u row_ids, u row_docs,
                         u out_vals, u out_ids, u out_docs, u status, u s) {

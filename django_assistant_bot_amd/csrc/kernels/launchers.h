@@ -368,7 +368,7 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
 // search.hip
 constexpr int kRankMax = 64;  // largest rank rank_value finds
 int unit_rows(const float* x, long ldx, void* out, int rows, int cols, hipStream_t s);
-int rank_value(const float* scores, long ld, int rows, int n, int r, float* thr, int* cnt, hipStream_t s);
+int rank_value(const float* scores, long ld, int rows, int n, int r, float slack, float* thr, int* cnt, hipStream_t s);
 int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const float* thr, int cap, int rows, int k,
               const int64_t* row_ids, const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs,
               int* status, hipStream_t s);

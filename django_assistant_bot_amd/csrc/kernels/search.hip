@@ -35,7 +35,7 @@ constexpr int RV_MAX = 256;  // maxima ranked: one of every four neighbouring th
 constexpr int RV_CAP = 512;
 constexpr int RV_HELD = 4;
 
-// thr[row] = the r-th largest of the row's n scores (r <= kRankMax; -inf when r > n), cnt[row] = 0.
+// thr[row] = the r-th largest of the row's n scores less `slack` (r <= kRankMax; -inf when r > n), cnt[row] = 0.
 //
 // The r-th largest of 256 maxima over disjoint parts is a lower bound that at least r scores reach, and with the r
 // of a search (7-41 of thousands) only a few more do: those are ranked.  Two looks at the row, the first 16,384 scores
@@ -43,7 +43,7 @@ constexpr int RV_HELD = 4;
 // of one query: 8.6 us, of 128 queries 9.6 (two reads of the row and ranks by LDS loops: 14.5 and 16.5; a radix select's
 // four passes with wave-aggregated histograms: 61 and 91).
 __global__ __launch_bounds__(RV_NT) void rank_value_kernel(const float* __restrict__ scores, long ld, int n, int r,
-                                                           float* __restrict__ thr, int* __restrict__ cnt) {
+                                                           float slack, float* __restrict__ thr, int* __restrict__ cnt) {
   __shared__ uint32_t tmax[RV_MAX];
   __shared__ uint32_t kept[RV_CAP];
   __shared__ uint32_t n_kept, bound;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(RV_NT) void rank_value_kernel(const float* __restri
         above += __popcll(__ballot(in && o > key));
         same += __popcll(__ballot(in && o == key));
       }
-      if (lane == 0 && above < r && r <= above + same) thr[row] = key_float(key);
+      if (lane == 0 && above < r && r <= above + same) thr[row] = key_float(key) - slack;
     }
     return;
   }
@@ -151,13 +151,13 @@ __global__ __launch_bounds__(RV_NT) void rank_value_kernel(const float* __restri
     mask |= 255u << shift;
     __syncthreads();
   }
-  if (tid == 0) thr[row] = key_float(prefix);
+  if (tid == 0) thr[row] = key_float(prefix) - slack;
 }
 
-int rank_value(const float* scores, long ld, int rows, int n, int r, float* thr, int* cnt, hipStream_t s) {
+int rank_value(const float* scores, long ld, int rows, int n, int r, float slack, float* thr, int* cnt, hipStream_t s) {
   if (rows <= 0) return 0;
   if (n <= 0 || r < 1 || r > kRankMax) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rank_value_kernel, dim3(rows), dim3(RV_NT), 0, s, scores, ld, n, r, thr, cnt);
+  hipLaunchKernelGGL(rank_value_kernel, dim3(rows), dim3(RV_NT), 0, s, scores, ld, n, r, slack, thr, cnt);
   return hipGetLastError();
 }
 

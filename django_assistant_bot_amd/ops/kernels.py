@@ -1070,15 +1070,15 @@ def unit_rows(x, dtype=torch.bfloat16):
 RANK_MAX = 64  # largest rank of ``rank_value``
 
 
-def rank_value(scores, r: int):
-    """(r-th largest score of every row of fp32 [rows, n], -inf when r > n; zeroed int32 [rows] for the counts of the
+def rank_value(scores, r: int, slack: float = 0.0):
+    """(r-th largest score of every row of fp32 [rows, n] less ``slack``, -inf when r > n; zeroed int32 [rows] for the counts of the
     scan that takes the value as its threshold)."""
     rows, n = scores.shape
     expect(scores.is_cuda and scores.dtype == torch.float32 and scores.stride(1) == 1, "scores: CUDA fp32 rows")
     expect(n > 0 and 1 <= r <= RANK_MAX, f"rank_value: 1 <= r <= {RANK_MAX}, n > 0")
     thr = torch.empty(rows, dtype=torch.float32, device=scores.device)
     cnt = torch.empty(rows, dtype=torch.int32, device=scores.device)
-    native().rank_value(ptr(scores), scores.stride(0), rows, n, int(r), ptr(thr), ptr(cnt), stream(scores))
+    native().rank_value(ptr(scores), scores.stride(0), rows, n, int(r), float(slack), ptr(thr), ptr(cnt), stream(scores))
     return thr, cnt
 
 
