@@ -33,11 +33,7 @@ class FragmentProjections:
     # Decode batches of 129..256 rows: 64-row tiles, 2 k-groups x 4 row groups (cfg 27; M = 256:
     # qkv 27.4 / o 18.6 / gate_up 98.7 / down 49.2 us against 32.4 / 25.8 / 104 / 55 for two
     # M = 128 passes, profiles/decode_round2.md).
-    # Up to 64 rows: BN 128 where the tiles fill the chip without K-slices, else BN 64 (``STREAM_NARROW``; the figures up to
-    # 32 rows stand at the configurations, at 48 rows (4096, 4096) 11.3 -> 9.6 us, (6144, 4096) 14.3 -> 12.5, gated (16384,
-    # 2048) 19.2 -> 14.2, (2048, 8192) 11.4 -> 9.0).  Above 64 only gate_up below 192 tiles (128 rows of (16384, 2048): 25.4
-    # -> 19.9; qkv 15.5 -> 17.6).  The LM head's 1002 tiles: BN 64 up to 16 rows (162.2 -> 158.7 us), BN 128 above (175 /
-    # 179).
+    # Up to 64 rows (gate_up: 128): BN 64 (``STREAM_NARROW``) where ``_narrow_wins``, else BN 128.
     STREAM_NARROW = {30: 43, 31: 44, 13: 12}
     STREAM_GATE_NARROW = 9
     STREAM_CFG_M16, STREAM_CFG_M32, STREAM_CFG_M64, STREAM_CFG_M128, STREAM_CFG_M256 = 30, 31, 13, 10, 27
@@ -45,7 +41,29 @@ class FragmentProjections:
     STREAM_MAX_M = ops.STREAM_MAX_M
     PREFILL_STREAM_MAX_M = 128  # prefill steps of at most this many tokens stream too (0: off)
 
-    def _stream_cfg(self, name: str, M: int, N: int) -> int:
+    def _narrow_wins(self, name: str, M: int, N: int, K: int) -> bool:
+        """Whether tiles of 64 weight rows beat tiles of 128 (K 0: not known).  They do where each CU still has at most one
+        workgroup, or where they need half the K-slices, so that the workgroups stay as many; but with few K-slices each
+        of them then walks so long a K that the wider tile's smaller share of X counts.
+
+        Time with 64 rows / with 128, M 1 .. 64: as many K-slices, 8-256 workgroups 0.6-1.0, 264-320 of them 1.1-1.4 (gate_up
+        of 22016 x 4096 at 6 rows 30.5 / 37 us, at 100 42 / 57; qkv of 1280 x 8192 8.0 / 9.3); half the K-slices, K / slices up to
+        2048 0.85-1.0; from 3584 on at 33-64 rows 1.0-1.13 (8192 x 28672 at 64 76 / 83 us), from 7168 on at 17-32 rows
+        1.0-1.06, up to 16 rows 0.97-1.03.  An LM head of 1002 tiles up to 16 rows: K 4096 0.98, K 2048 1.0-1.03; above 1.02."""
+        tiles = N // 128
+        if tiles >= 768:
+            return M <= 16 and not 0 < K < 4096
+        if name == "gate_up":
+            S = S2 = 1
+        elif name == "aux":
+            S = S2 = self._aux_splits(K)
+        else:
+            S, S2 = self._stream_splits(N, K), self._stream_splits(N, K, 64)
+        if S2 == S:
+            return 2 * tiles * S <= 256
+        return K // S2 <= (3072 if M > 32 else 6144 if M > 16 else K)
+
+    def _stream_cfg(self, name: str, M: int, N: int, K: int = 0) -> int:
         nat = ops.native()
         if M > 128 and name == "gate_up":
             # decode batches of 129..256: gate_up (+SwiGLU8) on the mid-M GEMM, 67-72 us against 90-96
@@ -65,10 +83,10 @@ class FragmentProjections:
                 cfg = self.STREAM_CFG_M128
         if N % nat.stream_gemm_bn(cfg):
             return -1
-        tiles = N // 128
-        if cfg == self.STREAM_CFG_M128 and name == "gate_up" and tiles < 192:
-            return self.STREAM_GATE_NARROW
-        return cfg if tiles >= 192 and (M > 16 or tiles < 768) else self.STREAM_NARROW.get(cfg, cfg)
+        narrow = self.STREAM_NARROW.get(cfg)
+        if cfg == self.STREAM_CFG_M128 and name == "gate_up":
+            narrow = self.STREAM_GATE_NARROW
+        return cfg if narrow is None or not self._narrow_wins(name, M, N, K) else narrow
 
     @staticmethod
     def _stream_splits(N: int, K: int, bn: int = 128) -> int:
@@ -82,10 +100,14 @@ class FragmentProjections:
                 break
         return best
 
+    @staticmethod
+    def _aux_splits(K: int) -> int:
+        return next((s for s in (16, 8, 4, 2) if K % (128 * s) == 0), 1)
+
     def _stream_choice(self, name: str, M: int, N: int, K: int) -> tuple[int, int]:
         """(stream_gemm cfg, K-slices) of a decode projection; cfg -1 = not streamable.  (The tuning
         harness benchmarks/decode_ab.py overrides this in a subclass.)"""
-        cfg = self._stream_cfg(name, M, N)
+        cfg = self._stream_cfg(name, M, N, K)
         if cfg < 0 or K % 128:
             return -1, 1
         return cfg, self._stream_splits(N, K, ops.native().stream_gemm_bn(cfg))
@@ -157,7 +179,7 @@ class HybridProjections(FragmentProjections):
             return ops.gemm_f32(h, w)
         if dec:
             cfg, _ = self._stream_choice("aux", h.shape[0], w.shape[0], w.shape[1])
-            s = next((s for s in (16, 8, 4, 2) if w.shape[1] % (128 * s) == 0), 1)
+            s = self._aux_splits(w.shape[1])
             if cfg >= 0 and s > 1:
                 return ops.stream_gemm(h, w, splits=s, cfg=cfg, nt=True)
         return ops.gemm_bt(h, w, out_f32=True, shuffled=True) if wide else ops.gemm_narrow(h, w)
