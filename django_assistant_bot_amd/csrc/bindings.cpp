@@ -407,6 +407,7 @@ PYBIND11_MODULE(_native, m) {
     return reinterpret_cast<uintptr_t>(st);
   });
   m.def("destroy_stream", [](u s) { check(hipStreamDestroy(ST(s)), "hipStreamDestroy"); });
+  m.def("decode_partition", &dab::decode_partition_of);
   m.def("paged_decode_attention", [](u q, u kc, u vc, u bt, int max_blocks, int bs, u ctx, u out, u po, u pm, u pl,
                                      u cnt, int batch, int Hq, int Hkv, int D, int part_size, int max_parts,
                                      float scale, u s, u order, u w0, long w0_bytes, u w1, long w1_bytes,

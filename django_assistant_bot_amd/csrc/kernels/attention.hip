@@ -1579,7 +1579,6 @@ struct DecodeParams {
   int* counters;  // [B * Hkv] partition arrivals (zero between launches; the last arriver resets)
   const int* order;  // optional [B] sequence visit order (longest first: see paged_decode_attention)
   int Hq, Hkv, part_size, max_parts;
-  int halve;  // partitions of part_size / 2 may be taken (a multiple of 128)
   float scale_log2;
   // chunk > 0: the new token sees its own chunk's keys only; partitions are counted from the 32-key sub-tile that
   // holds the chunk's first key.  sink (or null): one more score in head h's denominator
@@ -1591,6 +1590,24 @@ struct DecodeParams {
   OutputGate gate;  // EXT, optional (gate.y.p): the finished output times its sigmoid
   L3Warm warm;  // optional: the next projections' weights, warmed into L3 by appended workgroups
 };
+
+constexpr int kCombine = 8;  // partial results requested together by the combine
+
+// Keys of a partition for `items` (sequence, kv head) pairs whose longest context shows `longest` keys.  Few items leave CUs
+// idle while each walks a chain of sub-tiles: partitions of half the size, where the context is combined from several
+// anyway (one partition writes its result directly) and stays within one round of the combine, as long as all of them find a CU at once
+// (192: with more, the halves queue) and the workspace holds them.  us, whole -> halved 512-key partitions, (sequences,
+// key heads, context, head width): (1, 8, 1024, 128) 13.5 -> 10.6, (4, 8, 600, 128) 14.3 -> 11.3, (2, 8, 1150, 64) 11.5 -> 9.5,
+// (6, 8, 1024, 64) 10.2 -> 10.4; not taken: one partition (1, 8, 300, 128) 8.5 -> 9.8, (16, 2, 300, 64) 8.4 -> 10.0; more than a
+// round (1, 1, 8000, 128) 12.1 -> 18.7, (2, 2, 3000, 64) 9.9 -> 11.4; 448 items at (8, 8, 300-1700, 128) 15.8 -> 20.5.
+__host__ __device__ inline int decode_partition(int part_size, int longest, int items, int max_parts) {
+  if (part_size % 256 || part_size > 512 || longest <= part_size) return part_size;
+  const int n = (longest + part_size / 2 - 1) / (part_size / 2);
+  return n <= kCombine && n * items <= 192 && n <= max_parts ? part_size / 2 : part_size;
+}
+int decode_partition_of(int part_size, int longest, int items, int max_parts) {
+  return decode_partition(part_size, longest, items, max_parts);
+}
 
 // DMA (D = 128): each wave streams its 32-key K / V sub-tiles straight into its LDS slot by LDS-DMA
 // (buffer_load ... lds, non-temporal: MI355X_MICROARCH.md rows ldsdma-fill / nt-weights put the
@@ -1655,15 +1672,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
 #pragma unroll
   for (int off = 32; off; off >>= 1) maxc = max(maxc, __shfl_xor(maxc, off));
   maxc = __builtin_amdgcn_readfirstlane(maxc);
-  // Few items leave CUs idle while each walks a chain of sub-tiles: partitions of half the size as long as all of them
-  // find a CU at once (192: with more, the halves queue) and the workspace holds them.  us at (sequences, context, head
-  // width), whole -> halved 512-key partitions: (1, 1150, 128) 13.9 -> 10.8, (1, 4000, 128) 14.6 -> 13.5, (4, 500-1500,
-  // 128) 14.8 -> 13.8, (6, 200-900, 64) 11.8 -> 9.9; 448 items at (8, 300-1700, 128) 15.8 -> 20.5.
-  int part_size = p.part_size;
-  if (p.halve) {
-    const int n = (maxc + part_size / 2 - 1) / (part_size / 2);
-    if (n * BH <= 192 && n <= p.max_parts) part_size /= 2;
-  }
+  const int part_size = decode_partition(p.part_size, maxc, BH, p.max_parts);
   const int live_items = min(p.max_parts, (maxc + part_size - 1) / part_size) * BH;
   for (int item = blockIdx.x; item < live_items; item += attn_blocks) {
     const int part = item / BH;
@@ -1956,7 +1965,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
       __syncthreads();
       if (*last_flag) {
         auto ld = [](const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-        constexpr int NPF = 8;
+        constexpr int NPF = kCombine;
         for (int e = tid; e < G * (D / 4); e += 256) {
           const int qh = e / (D / 4), d = 4 * (e % (D / 4));
           const f32x4 gate = gate4(qh, d);
@@ -2245,7 +2254,6 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   prm.Hkv = Hkv;
   prm.part_size = part_size;
   prm.max_parts = max_parts;
-  prm.halve = batch * Hkv <= 64 && part_size % 256 == 0 && part_size <= 512;
   prm.scale_log2 = scale * 1.4426950408889634f;
   prm.chunk = chunk;
   prm.sink = sink;

@@ -68,6 +68,7 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
 // attention_packed.hip: bidirectional self-attention over packed sequences, heads of 64
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
                    long o_tok, long o_head, const int* cu, int batch, int max_len, int Hq, int Hkv, float scale, hipStream_t s);
+int decode_partition_of(int part_size, int longest, int items, int max_parts);
 int paged_decode_attention(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                            int max_blocks, int block_size, const int* ctx_lens, void* out, float* part_o,
                            float* part_m, float* part_l, int* counters, int batch, int Hq, int Hkv, int D,
