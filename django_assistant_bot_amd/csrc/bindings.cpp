@@ -407,6 +407,13 @@ PYBIND11_MODULE(_native, m) {
     return reinterpret_cast<uintptr_t>(st);
   });
   m.def("destroy_stream", [](u s) { check(hipStreamDestroy(ST(s)), "hipStreamDestroy"); });
+  m.def("flash_packed64", [](u q, long q_tok, long q_head, u k, u v, long kv_tok, long kv_head, u out, long o_tok, long o_head,
+                             u cu, int batch, int max_len, int Hq, int Hkv, float scale, u s) {
+    check(dab::flash_packed64(CVP(q), q_tok, q_head, CVP(k), CVP(v), kv_tok, kv_head, VP(out), o_tok, o_head, (const int*)cu,
+                              batch, max_len, Hq, Hkv, scale, ST(s)),
+          "flash_packed64");
+  });
+  m.def("flash_packed64_wins", &dab::flash_packed64_wins);
   m.def("decode_partition", &dab::decode_partition_of);
   m.def("paged_decode_attention", [](u q, u kc, u vc, u bt, int max_blocks, int bs, u ctx, u out, u po, u pm, u pl,
                                      u cnt, int batch, int Hq, int Hkv, int D, int part_size, int max_parts,

@@ -2173,12 +2173,11 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
       return hipGetLastError();
     }
   }
-  // encoder texts longer than a 64-query block (shorter ones are a chain of one tile, 4-5 us either way); the DAB_ENC_*
-  // switches compare the 16 x 16 forms with each other
-  if (D == 64 && !std::getenv("DAB_ENC_PERSIST") && !std::getenv("DAB_ENC_W5") && !paged && !causal && cu_q == cu_k && max_seqlen_q > 64 && scale > 0.f && kv_stride_tok > 0 &&
-      (q_stride_tok | q_stride_head | kv_stride_tok | kv_stride_head) % 8 == 0 && (o_stride_tok | o_stride_head) % 4 == 0 &&
+  // encoder texts; the DAB_ENC_* switches compare the 16 x 16 forms with each other
+  if (D == 64 && !paged && !causal && cu_q == cu_k && flash_packed64_wins((long)batch * Hq, max_seqlen_q) && scale > 0.f &&
+      kv_stride_tok > 0 && (q_stride_tok | q_stride_head | kv_stride_tok | kv_stride_head) % 8 == 0 && (o_stride_tok | o_stride_head) % 4 == 0 &&
       ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 == 0 && (uintptr_t)out % 8 == 0 &&
-      (long)max_seqlen_q * kv_stride_tok * 2 < (1L << 31))
+      (long)max_seqlen_q * kv_stride_tok * 2 < (1L << 31) && !std::getenv("DAB_ENC_PERSIST") && !std::getenv("DAB_ENC_W5"))
     return flash_packed64(q, q_stride_tok, q_stride_head, k, v, kv_stride_tok, kv_stride_head, out, o_stride_tok, o_stride_head,
                           cu_q, batch, max_seqlen_q, Hq, Hkv, scale, s);
   const bool wide = D == 128 && max_seqlen_q > 64;

@@ -1,5 +1,5 @@
-// Bidirectional attention over packed sequences, heads of 64 (the bge / BERT encoders): the form for texts longer than
-// 64 tokens.  (Reference: HF BertSelfAttention, ai/embedders/transformers.py:18-22.)
+// Bidirectional attention over packed sequences, heads of 64 (the bge / BERT encoders): the form for long texts and for
+// many of them.  (Reference: HF BertSelfAttention, ai/embedders/transformers.py:18-22.)
 //
 // What bounds it: the softmax.  A score costs an exponential (16 cycles a wave) and about three more vector
 // instructions against 8 cycles of MFMA, so everything else has to run beside them.  The 16 x 16 form of attention.hip
@@ -217,6 +217,14 @@ __global__ __launch_bounds__(256, 4) void flash_packed64_kernel(PackedParams p) 
     for (int i = 0; i < 4; ++i)
       *reinterpret_cast<u32x2*>(row + 32 * d + 8 * i) =
           u32x2{pack2bf(o[d][4 * i] * inv, o[d][4 * i + 1] * inv), pack2bf(o[d][4 * i + 2] * inv, o[d][4 * i + 3] * inv)};
+}
+
+// Whether the 32 x 32 form is the faster one for `units` (sequence, head) pairs of up to max_len tokens.  Texts of one
+// 64-query block are a chain of one tile either way.  Up to 256 tokens the 16 x 16 form's workgroups of 64 queries start
+// quicker as long as each of them has a CU.  us, 16 x 16 form / this one, 12 heads: 1 text of 112 tokens 4.8 / 5.2, 8 of
+// 128 5.2 / 5.4, 12 of 128 5.9 / 5.5, 1 of 192 5.9 / 6.0, 6 of 256 8.4 / 7.4, 1 of 512 11.2 / 10.8, 3 of 512 13.6 / 11.1.
+bool flash_packed64_wins(long units, int max_len) {
+  return max_len > 256 || (max_len > 64 && units * ((max_len + 63) / 64) > 256);
 }
 
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
