@@ -419,7 +419,8 @@ __global__ __launch_bounds__(MP_NT) void mean_pool_kernel(float* __restrict__ ou
   float ss = 0.f;
   const bool first = threadIdx.x < nvec;
   if (first) {
-    for (int k = 1; k < G; ++k)
+    const int groups = min(G, end - start);  // (the others have no token)
+    for (int k = 1; k < groups; ++k)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] += part[k * nvec + i][j >> 2][j & 3];
 #pragma unroll
