@@ -1,9 +1,9 @@
 // The sentence encoder's forward as one call: every launch of its layers enqueued from native code.
 //
 // For one question the GPU works about 0.35 ms on 64 launches (0.45 ms on 87 with the LayerNorms apart), and issuing
-// those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a launch costs the runtime's own 1-2 us; the five
-// activation buffers are the caller's, shared by all layers.  (The reference runs one text a call through an eager
-// model: ai/embedders/transformers.py:15-29.)
+// those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a launch costs
+// the runtime's own 1-2 us; the five activation buffers are the caller's, shared by all layers.  (The reference runs
+// one text a call through an eager model: ai/embedders/transformers.py:15-29.)
 #include "common.h"
 #include "launchers.h"
 
@@ -11,19 +11,20 @@ namespace dab {
 
 // Which tile of gemm_small a projection with row-major weights takes, -1: the 128 x 128 / 256 x 256 kernels.
 //
-// The smallest tile that still gives each CU about one workgroup: K split over a workgroup's waves up to 256 tiles of 16 x
-// 16, 32 x 16, 32 x 32, 32 x 64, and 64 x 64 where K is long (K of 384 and more: every other kernel sums K in one order,
-// so that results there do not depend on M); then the barrier-stepped ring with 32 x 64 tiles up to 320, 64 x 64 up to
-// 1200 (512 where K is long: a K-tile's chain is paid K / 64 times and the larger tile has fewer workgroups to queue),
-// 128 x 128 up to 256.  Both sides of each line, us (us of the tile before -> of the tile after it): 192 tiles of 16 x 16
-// at (64, 768, 768) 3.1 / 3.4, 288 at (19, 2304, 768) 3.6 / 3.4; 192 of 32 x 16 at (128, 768, 768) 3.4 / 3.8, 288 at (64,
-// 2304, 768) 5.3 / 4.1; 192 of 32 x 32 at (256, 768, 768) 3.9 / 4.6, 288 at (128, 2304, 768) 5.3 / 4.8; 192 of 32 x 64 at
-// (512, 768, 768) 5.1 / 5.5, with K 3072 11.4 / 14.7, 288 at (256, 2304, 768) 7.9 / 6.4; 224 of 64 x 64 at (870, 1024, 4096)
-// 17.6 / 20.6, 288 at (1500, 768, 3072) 26.5 / 19.6, but with the short K 168 at (870, 768, 768) 7.0 / 6.7; 288 of the
-// ring's 32 x 64 at (256, 2304, 768) 6.4 / 6.8, 384 at (256, 3072, 768) 8.1 / 7.3; 1152 of its 64 x 64 at (2048, 2304, 768)
-// 20.2 / 25.4 (gemm256), 1692 at (3000, 2304, 768) 29.3 / 26.7; with K 3072 288 at (1500, 768, 3072) 19.8 / 36.0, 564 at
-// (3000, 768, 3072) 43.0 / 36.1; 192 of 128 x 128 at (4096, 768, 3072) 37.7 / 64.4 (gemm256), 282 at (6000, 768, 3072) 71.3 /
-// 64.0.
+// The smallest tile that still gives each CU about one workgroup: K split over a workgroup's waves up to 256 tiles of
+// 16 x 16, 32 x 16, 32 x 32, 32 x 64, and 64 x 64 where K is long (K of 384 and more: every other kernel sums K in one
+// order, so that results there do not depend on M); then the barrier-stepped ring with 32 x 64 tiles up to 320, 64 x 64
+// up to 1200 (1000 where M is over 3 N: each XCD streams the rows again for every column block; 512 where K is long: a
+// K-tile's chain is paid K / 64 times and the larger tile has fewer workgroups to queue), 128 x 128 up to 256.  Both
+// sides of each line, us (us of the tile before -> of the tile after it): 192 tiles of 16 x 16 at (64, 768, 768) 3.1 /
+// 3.4, 288 at (19, 2304, 768) 3.6 / 3.4; 192 of 32 x 16 at (128, 768, 768) 3.4 / 3.8, 288 at (64, 2304, 768) 5.3 / 4.1;
+// 192 of 32 x 32 at (256, 768, 768) 3.9 / 4.6, 288 at (128, 2304, 768) 5.3 / 4.8; 192 of 32 x 64 at (512, 768, 768) 5.1
+// / 5.5, with K 3072 11.4 / 14.7, 288 at (256, 2304, 768) 7.9 / 6.4; 224 of 64 x 64 at (870, 1024, 4096) 17.6 / 20.6,
+// 288 at (1500, 768, 3072) 26.5 / 19.6, but with the short K 168 at (870, 768, 768) 7.0 / 6.7; 288 of the ring's 32 x
+// 64 at (256, 2304, 768) 6.4 / 6.8, 384 at (256, 3072, 768) 8.1 / 7.3; 1152 of its 64 x 64 at (2048, 2304, 768) 20.2 /
+// 25.4 (gemm256), 1692 at (3000, 2304, 768) 29.3 / 26.7, 1008 at (5333, 768, 768) 18.0 / 18.4, 1104 at (5866, 768, 768)
+// 20.3 / 18.5, at (4400, 1024, 1024) 23.9 / 22.0; with K 3072 288 at (1500, 768, 3072) 19.8 / 36.0, 564 at (3000, 768,
+// 3072) 43.0 / 36.1; 192 of 128 x 128 at (4096, 768, 3072) 37.7 / 64.4 (gemm256), 282 at (6000, 768, 3072) 71.3 / 64.0.
 int small_tile(int M, int N, int K) {
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (K >= 384) {
@@ -34,7 +35,7 @@ int small_tile(int M, int N, int K) {
     if (K > 1024 && tiles(64, 64) <= 256) return 8;
   }
   if (tiles(32, 64) <= 320) return 2;
-  if (K <= 1024) return tiles(64, 64) <= 1200 ? 3 : -1;
+  if (K <= 1024) return tiles(64, 64) <= (M > 3L * N ? 1000 : 1200) ? 3 : -1;
   if (tiles(64, 64) <= 512) return 4;
   return tiles(128, 128) <= 256 ? 5 : -1;
 }
