@@ -594,6 +594,9 @@ PYBIND11_MODULE(_native, m) {
           "gemm_small");
   });
   m.def("gemm_mid_groups", &dab::gemm_mid_groups);
+  m.def("gemm_mid_us", &dab::gemm_mid_us);
+  m.def("gemm256_wins", &dab::gemm256_wins);
+  m.attr("GEMM256_FILL") = dab::kGemm256Fill;
   m.def("index_scan_takes", [](int M, int K) { return dab::index_scan_takes(M, K) != 0; });
   m.def("index_scan_scores", [](u A, long lda, u Wshuf, int M, int N, int K, u row_group, u q_group, u scores, u s) {
     check(dab::index_scan_scores_shuf(CVP(A), lda, CVP(Wshuf), M, N, K, reinterpret_cast<const int*>(row_group),

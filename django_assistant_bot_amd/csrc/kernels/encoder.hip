@@ -47,8 +47,7 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
   if (tile >= 0 && gemm_small_ok(M, N, K, K, K, N, N) &&
       !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8))
     return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s);
-  const bool wide = M >= 256 && N % 256 == 0 && (long)((M + 255) / 256) * (N / 256) >= 192;
-  if ((M >= 1024 || wide) && gemm256_ok(M, N, K, K, K))
+  if (gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K))
     return gemm256(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, s, 0, 1);
   return gemm_bt(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, 0, nullptr, nullptr, nullptr, 0, s, 0, 1);
 }

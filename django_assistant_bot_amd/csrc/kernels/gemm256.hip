@@ -847,6 +847,12 @@ int gemm256_ok(int M, int N, int K, long lda, long ldb) {
   return 1;
 }
 
+// Shapes that go here instead of to the 128 x 128 kernel: from 1024 rows on, and from 256 rows on where the tiles fill 192
+// CUs (gate_up of Llama-3-8B at M = 384-768: 84-161 us against 105-184, profiles/gemm_mid_r6.md).
+bool gemm256_wins(int M, int N) {
+  return M >= 1024 || (M >= 256 && N % 256 == 0 && (long)((M + 255) / 256) * (N / 256) >= kGemm256Fill);
+}
+
 // b_shuf: B is in the shuffle_weights layout (ldb == K).  Epilogues: 0 none, 1 GELU, 2 SwiGLU over
 // 16-row [gate | up] groups, 4 / 6 SwiGLU / tanh-GELU GLU over 8-row groups (bias: fp32 [gate | up]); bias / residual optional.
 int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,

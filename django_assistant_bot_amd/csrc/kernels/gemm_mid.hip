@@ -502,22 +502,41 @@ int gemm_mid_ok(int M, int N, int K, long lda) {
   return 1;
 }
 
+// Estimated us of a product on `groups` groups: its ends (4 for whole tiles, 8 where every tile is cut into equal parts,
+// 18 otherwise, 1.45 for a part its owner adds, 3.5 for the end of each further tile) and its K-steps (0.45 + 0.0016 a
+// workgroup each).
+struct MidTime {
+  double ends, steps;
+};
+static MidTime mid_time(int M, int N, int K, int groups) {
+  const int tm = (M + 127) / 128, tn = N / 256;
+  const double parts = (double)groups / tn;  // of a tile
+  double ends = tn % groups == 0 ? 4. : groups % tn == 0 ? 8. + 1.45 * parts : 18. + (groups > tn ? 1.45 * (parts - 1.) : 0.);
+  if (tn > groups) ends += 3.5 * (1. / parts - 1.);
+  return {ends, (double)tn * (K / 64) / groups * (0.45 + 0.0016 * (groups * tm))};
+}
+
 // Groups of ceil(M / 128) workgroups: the whole ones of each XCD, and those joined from the slots left over where they
-// gain 6 % by the estimate (us: 0.45 + 0.0016 a workgroup for a K-step; 4 for whole tiles, 8 where every tile is cut
-// into equal parts, 18 otherwise, 1.45 for a part its owner adds, 3.5 for the end of each further tile).  More workgroups are no gain where the whole groups divide the tiles evenly.  us,
-// whole groups -> with the joined ones: gate_up of Llama-3-8B at M 1093 272 -> 238, down 138 -> 128, o 47.7 -> 45.7, down at
-// M 1300 175 -> 156, 2200 338 -> 242, qkv at M 2600 158 -> 120; but qkv at M 1093 (24 tiles, 24 groups) 53.9 -> 63.4, o at
-// M 1700 55.0 -> 60.7.
+// gain 6 % by the estimate.  More workgroups are no gain where the whole groups divide the tiles evenly.  us, whole
+// groups -> with the joined ones: gate_up of Llama-3-8B at M 1093 272 -> 238, down 138 -> 128, o 47.7 -> 45.7, down at M
+// 1300 175 -> 156, 2200 338 -> 242, qkv at M 2600 158 -> 120; but qkv at M 1093 (24 tiles, 24 groups) 53.9 -> 63.4, o at M
+// 1700 55.0 -> 60.7.
 int gemm_mid_groups(int M, int N, int K) {
   const int spx = cu_count() / 8, tm = (M + 127) / 128, tn = N / 256;
   if (M <= 0 || tn <= 0 || tm > spx) return 0;
-  auto us = [&](int g) {
-    const float parts = (float)g / (float)tn;  // of a tile
-    const float fixed = tn % g == 0 ? 4.f : g % tn == 0 ? 8.f + 1.45f * parts : 18.f + (g > tn ? 1.45f * (parts - 1.f) : 0.f);
-    return fixed + (tn > g ? 3.5f * ((float)tn / (float)g - 1.f) : 0.f) + (float)tn * (float)(K / 64) / (float)g * (0.45f + 0.0016f * (float)(g * tm));
-  };
   const int whole = 8 * (spx / tm), all = whole + 8 * (spx % tm) / tm;
-  return us(all) < 0.94f * us(whole) ? all : whole;
+  const MidTime a = mid_time(M, N, K, all), w = mid_time(M, N, K, whole);
+  return a.ends + a.steps < 0.94 * (w.ends + w.steps) ? all : whole;
+}
+
+// Estimated us of the launch, infinite where the kernel does not take M; with few rows the weights' way from memory
+// (4.5 TB/s) is longer than the K-steps.
+double gemm_mid_us(int M, int N, int K) {
+  const int groups = gemm_mid_groups(M, N, K);
+  if (!groups) return M <= 0 || N < 256 ? 0. : __builtin_huge_val();
+  const MidTime t = mid_time(M, N, K, groups);
+  const double weights = (double)(N / 256) * 512 * K / 4.5e6;
+  return t.ends + (t.steps > weights ? t.steps : weights);
 }
 
 // Workspace the launcher needs: partial slabs and behind them a line with the count of ended workgroups (bytes), and

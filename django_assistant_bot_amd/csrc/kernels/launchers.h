@@ -269,6 +269,8 @@ int gemm_grouped(const void* A, long lda, const void* B, void* C, long ldc, int 
 
 // gemm256.hip (large-M prefill / encoder GEMM, 256x256 phased schedule; epilogue 0 none, 1 GELU,
 // 2 SwiGLU on [gate 16 | up 16]-interleaved weight rows; bias / residual optional)
+constexpr int kGemm256Fill = 192;  // 256 x 256 tiles that keep a shape on gemm256 below 1024 rows
+bool gemm256_wins(int M, int N);
 int gemm256_ok(int M, int N, int K, long lda, long ldb);
 int gemm256_candidates(const void* A, long lda, const void* B, long ldb, int M, int N, int K, const int* row_group,
                        const int* q_group, const float* thr, int* cnt, float* cand_val, int* cand_idx, int cap,
@@ -289,6 +291,7 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
 // plane, 128 x 256 tiles, in-launch last-arriver combine; B in the shuffle_weights layout;
 // epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
 int gemm_mid_groups(int M, int N, int K);
+double gemm_mid_us(int M, int N, int K);
 int gemm_mid_ok(int M, int N, int K, long lda);
 long gemm_mid_slab_bytes();
 int gemm_mid_counters(int M, int N);

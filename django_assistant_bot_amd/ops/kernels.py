@@ -391,15 +391,11 @@ def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, part_size=512, wor
 # GEMM
 
 
-GEMM256_MIN_M = 1024  # the phased 256x256 kernel from here on; the 128x128 kernel below
-
-
 # gemm_mid from the first row: at M <= 191 the 128 x 128 kernel re-reads the weights per row tile
 # and leaves most CUs idle -- Llama-3-8B qkv / o / gate_up / down at M = 129-187: 54 / 54 / 72 / 181
 # us against 31 / 29 / 67 / 47 (profiles/small_prefill_r6.md; decode-sized prefill steps of the
 # fragment-layout decoder stream instead, models/llama.py PREFILL_STREAM_MAX_M)
 GEMM_MID_MIN_M = 1
-GEMM_MID_FILL = 192  # gemm256 keeps a shape whose 256 x 256 tiles fill this many of the 256 CUs
 
 
 def _g256_fill(M: int, N: int) -> tuple[int, float]:
@@ -410,7 +406,7 @@ def _g256_fill(M: int, N: int) -> tuple[int, float]:
 
 def use_gemm_mid(M: int, N: int, K: int, lda: int) -> bool:
     """Mid-M shapes on fragment-layout weights go to the stream-K kernel (gemm_mid.hip) where the
-    256 x 256 kernel would leave CUs idle: fewer than GEMM_MID_FILL tiles, or a last wave that
+    256 x 256 kernel would leave CUs idle: fewer than GEMM256_FILL (192) tiles, or a last wave that
     leaves the chip under 70 % busy.  Measured (profiles/gemm_mid_r6.md): Llama-3-8B qkv / o / down
     at M = 384..2048 run 1.2-2.5x faster than the round-5 dispatch, gate_up at M = 640 / 768 (336
     tiles = 1.31 waves) 12 % faster than gemm256; gate_up at 384 / 512 / 1024 / 2048 and qkv at
@@ -418,15 +414,12 @@ def use_gemm_mid(M: int, N: int, K: int, lda: int) -> bool:
     if M < GEMM_MID_MIN_M or N % 256 or not gemm_mid_ok(M, N, K, lda):
         return False
     tiles, fill = _g256_fill(M, N)
-    return tiles < GEMM_MID_FILL or fill < 0.7
+    return tiles < native().GEMM256_FILL or fill < 0.7
 
 
 def use_gemm256(M: int, N: int, K: int, lda: int, ldb: int) -> bool:
-    """Large-M shapes go to the phased 256x256 kernel (gemm256.hip), and so do shapes from M = 256 on
-    whose 256 x 256 tiles fill >= GEMM_MID_FILL CUs (gate_up at M = 384-768: 84-161 us against
-    105-184 on the 128 x 128 kernel, profiles/gemm_mid_r6.md)."""
-    wide = M >= 256 and N % 256 == 0 and -(-M // 256) * (N // 256) >= GEMM_MID_FILL  # e.g. gate_up at M 256-1023
-    return (M >= GEMM256_MIN_M or wide) and bool(native().gemm256_ok(M, N, K, lda, ldb))
+    """Whether the phased 256x256 kernel takes a shape instead of the 128x128 one (``gemm256_wins`` in gemm256.hip)."""
+    return native().gemm256_wins(M, N) and bool(native().gemm256_ok(M, N, K, lda, ldb))
 
 
 def _g256_us(tiles: int, K: int) -> float:
@@ -440,19 +433,8 @@ def _g256_us(tiles: int, K: int) -> float:
 
 def _mid_us(M: int, tiles_n: int, K: int) -> float:
     """Estimated time of gemm_mid: lockstep groups of ceil(M / 128) workgroups share its (weight tile, K-step) plane;
-    tiles that groups share are combined at the end (gemm_mid_groups in gemm_mid.hip has the figures)."""
-    if not M or not tiles_n:
-        return 0.0
-    tm = -(-M // 128)
-    if tm > 32:
-        return float("inf")
-    groups = native().gemm_mid_groups(M, 256 * tiles_n, K)
-    steps = tiles_n * (K // 64) / groups * (0.45 + 0.0016 * groups * tm)
-    weights = tiles_n * 512 * K / 4.5e6  # few rows: the weights' way from memory
-    parts = groups / tiles_n  # of a tile
-    ends = 4 if tiles_n % groups == 0 else 8 + 1.45 * parts if groups % tiles_n == 0 else 18 + 1.45 * max(0.0, parts - 1)
-    ends += 3.5 * max(0.0, 1 / parts - 1)
-    return ends + max(steps, weights)
+    tiles that groups share are combined at the end (``gemm_mid_us`` in gemm_mid.hip)."""
+    return native().gemm_mid_us(M, 256 * tiles_n, K)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -464,7 +446,7 @@ def frag_plan(M: int, N: int, K: int, cols: bool = True):
     where two waves take 157), gemm_mid runs at about half its rate but divides evenly.  So the whole waves go to
     gemm256 and the remaining columns (or rows) to gemm_mid where the estimates (fitted to both kernels at the four
     projections of Llama-3-8B and Llama-3.2-1B, M = 300..5000, mostly within 10 %) gain more than 5 % over one kernel;
-    between one or the other alone the old bounds (GEMM_MID_FILL, 70 % of a wave) decide unless the other's estimate is
+    between one or the other alone the old bounds (GEMM256_FILL, 70 % of a wave) decide unless the other's estimate is
     1.5 % lower.  us, before -> with the plan: gate_up M 513 137 -> 127, 1093 233 -> 213, 700 181 -> 148, qkv 1700 92 -> 77,
     2600 157 -> 118, o 2300 93 -> 72, down 2200 338 -> 236, 4300 533 -> 357."""
     tm, tn = -(-M // 256), N // 256
