@@ -50,7 +50,7 @@ struct GMid {
   const bf16* residual;   // GLU epilogues with RES: fp32 bias [gate N / 2 | up N / 2] instead
   float* slabs;  // [tiles_m][gn][2] partial tiles of 128 x 256 fp32 (in accumulator order)
   int* cnt;      // [tiles_m][gn][2] ready flags of the stored partial tiles (the launch that stored them), zero at rest
-  unsigned* ended;  // workgroups that ended, over all launches on this workspace
+  unsigned* ended;  // [8][32]: workgroups of an XCD label that ended, over all launches on this workspace, a line each
   long spin_limit;
   int M, N, K;
   long lda, ldc, ldr;
@@ -97,7 +97,7 @@ struct MidGeo {
   static constexpr int kDist = kStages - 1;     // stage issued kDist iterations ahead
   static constexpr int kDma = BK == 64 ? 6 : 3;  // LDS-DMA instructions per wave per stage
   static constexpr int kSmem = kStages * kStage;
-  static_assert(kSmem <= 163840, "LDS");
+  static_assert(kSmem + 512 <= 163840, "LDS");
 };
 constexpr int kE = 8;                  // VMEM stores per wave in every epilogue variant
 constexpr int kSlabSt = 16;            // VMEM stores per wave of a published partial tile
@@ -119,29 +119,28 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   using Geo = MidGeo<BK>;
   constexpr int kStage = Geo::kStage, kStages = Geo::kStages, kDist = Geo::kDist, kDma = Geo::kDma;
   constexpr int kA = Geo::kA;
-  __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem];
+  // behind the ring: the count the launch's number comes from
+  __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem + 256];
 
   // ---- which group / row tile this block is: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that whole
   // groups leave over are joined, XCD after XCD, into further groups
   const int bid = blockIdx.x, tid = threadIdx.x;
-  // the launch's number, the same for all of its workgroups: this one has not ended yet, so its launch adds less than
-  // gridDim.x to the count (which may wrap: 2^32 is a multiple of 256 workgroups).  A scalar load: nothing precedes it
-  const int launch = (int)(*p.ended / gridDim.x) + 1;
-  auto count_end = [&]() {
-    if (tid == 0) __hip_atomic_fetch_add(p.ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
   const int x = bid & 7, slot = bid >> 3;
+  unsigned* const ended = p.ended + 32 * x;
+  auto count_out = [&]() {
+    if (tid == 0) __hip_atomic_fetch_add(ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   int g = slot / p.tiles_m, mt = slot - g * p.tiles_m, j = x * p.gpx + g;
   if (g >= p.gpx) {
     const int over = p.spx - p.gpx * p.tiles_m, u = x * over + slot - p.gpx * p.tiles_m;
     g = u / p.tiles_m;
     mt = u - g * p.tiles_m;
     j = 8 * p.gpx + g;
-    if (j >= p.gn) return count_end();  // whole workgroup (uniform)
+    if (j >= p.gn) return count_out();  // whole workgroup (uniform)
   }
   const int start = grp_start(j, p.q, p.r);
   const int end = start + p.q + (j < p.r ? 1 : 0);
-  if (end <= start) return count_end();
+  if (end <= start) return count_out();
 
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -230,6 +229,13 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
       ++s_nt;
     }
   };
+  // The launch's number, the same for all of its workgroups: this one has not ended yet, so its launch has added less
+  // than the label's p.spx workgroups to their count (which may wrap: 2^32 is a multiple of 32).  Wave 0 copies the count
+  // to LDS ahead of the first stage, so that it has landed when that has (a scalar load in front, and one count for all
+  // labels, cost 0.8 to 2 us a launch; the addition behind the prologue instead of at the end 1 to 3 us where a group
+  // takes few K-steps).  The number is read by an asm statement: before an ordinary read hipcc drains the copies in flight.
+  if (w == 0)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(mk_rsrc(ended, 4), (lds_void*)(smem + Geo::kSmem), 4, 0u, 0u, 0, 0);
   // prologue: iterations start .. start + kDist - 1 in flight (buffers 0 ..), the first landed
 #pragma unroll
   for (int d = 0; d < kDist; ++d)
@@ -246,6 +252,12 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
     else wait_vmc<0>();
   }
   mbar();
+  unsigned before;
+  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+               : "=v"(before)
+               : "v"((unsigned)(uintptr_t)(lds_void*)(smem + Geo::kSmem))
+               : "memory");
+  const int launch = (int)((unsigned)__builtin_amdgcn_readfirstlane((int)before) / (unsigned)p.spx) + 1;
 
   int it = start;
   int b = 0;  // ring buffer of iteration `it`
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
 #pragma unroll
       for (int jn = 0; jn < 4; ++jn) acc[i][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  count_end();
+  count_out();
 }
 
 namespace {
@@ -539,10 +551,10 @@ double gemm_mid_us(int M, int N, int K) {
   return t.ends + (t.steps > weights ? t.steps : weights);
 }
 
-// Workspace the launcher needs: partial slabs and behind them a line with the count of ended workgroups (bytes), and
-// ready flags (ints).
+// Workspace the launcher needs: partial slabs and behind them the counts of ended workgroups (bytes), and ready flags
+// (ints).
 static long slabs_end() { return (long)cu_count() * 2 * kSlabFloats * 4; }
-long gemm_mid_slab_bytes() { return slabs_end() + 128; }
+long gemm_mid_slab_bytes() { return slabs_end() + 8 * 128; }
 // ready flags of the partial tiles: two per (row tile, group) <= two per workgroup
 int gemm_mid_counters(int M, int N) {
   (void)M;
@@ -552,7 +564,7 @@ int gemm_mid_counters(int M, int N) {
 
 // epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over
 // 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes()
-// bytes, the last 128 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).
+// bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).
 // spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
 // (BK 64), 32 / 64 force the K-step, + 1000 = DIAG 1 (split tiles not combined: timing only).
 // BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank

@@ -627,13 +627,13 @@ _MID_WS: dict = {}
 def _mid_workspace(device: torch.device, s: int):
     """Partial-tile slabs + ready flags of ``gemm_mid``, one set per (device, stream): two streams
     running the kernel at once must not share them.  The flags are zero at rest (every launch leaves
-    them zero); the slabs' last 128 bytes count the workgroups that ended."""
+    them zero); the slabs' last 1024 bytes count the workgroups that ended."""
     key = (device.index, s)
     ws = _MID_WS.get(key)
     if ws is None:
         nat = native()
         slabs = torch.empty((nat.gemm_mid_slab_bytes() // 4,), dtype=torch.float32, device=device)
-        slabs[-32:].zero_()
+        slabs[-256:].zero_()
         cnt = torch.zeros((1 << 16,), dtype=torch.int32, device=device)
         ws = _MID_WS[key] = (slabs, cnt)
     return ws

@@ -49,14 +49,14 @@ def test_the_count_of_launches_may_wrap():
     A, B, exp = _case(*SHAPES[1], 0)
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
-        ended = kernels._mid_workspace(A.device, s.cuda_stream)[0].view(torch.int32)[-32]
+        ended = kernels._mid_workspace(A.device, s.cuda_stream)[0].view(torch.int32)[-256::32]
         s.wait_stream(torch.cuda.default_stream())
         grid = torch.cuda.get_device_properties(0).multi_processor_count & ~7
-        assert (1 << 32) % grid == 0 and not ended
-        ended.fill_(-2 * grid)
+        assert (1 << 32) % grid == 0 and not ended.any()
+        ended.fill_(-2 * (grid // 8))
         for i in range(5):
             assert _close(ops.kernels.gemm_mid(A, B), exp).all()
-            assert int(ended) == (i - 1) * grid
+            assert (ended == (i - 1) * (grid // 8)).all()
 
 
 def test_replays_go_on_counting():
