@@ -1593,13 +1593,14 @@ struct DecodeParams {
 
 constexpr int kCombine = 8;  // partial results requested together by the combine
 
-// Keys of a partition for `items` (sequence, kv head) pairs whose longest context shows `longest` keys.  Few items leave CUs
-// idle while each walks a chain of sub-tiles: partitions of half the size, where the context is combined from several
-// anyway (one partition writes its result directly) and stays within one round of the combine, as long as all of them find a CU at once
-// (192: with more, the halves queue) and the workspace holds them.  us, whole -> halved 512-key partitions, (sequences,
-// key heads, context, head width): (1, 8, 1024, 128) 13.5 -> 10.6, (4, 8, 600, 128) 14.3 -> 11.3, (2, 8, 1150, 64) 11.5 -> 9.5,
-// (6, 8, 1024, 64) 10.2 -> 10.4; not taken: one partition (1, 8, 300, 128) 8.5 -> 9.8, (16, 2, 300, 64) 8.4 -> 10.0; more than a
-// round (1, 1, 8000, 128) 12.1 -> 18.7, (2, 2, 3000, 64) 9.9 -> 11.4; 448 items at (8, 8, 300-1700, 128) 15.8 -> 20.5.
+// Keys of a partition for `items` (sequence, kv head) pairs whose longest context shows `longest` keys.  Few items
+// leave CUs idle while each walks a chain of sub-tiles: partitions of half the size, where the context is combined from
+// several anyway (one partition writes its result directly) and stays within one round of the combine, as long as all
+// of them find a CU at once (192: with more, the halves queue) and the workspace holds them.  us, whole -> halved
+// 512-key partitions, (sequences, key heads, context, head width): (1, 8, 1024, 128) 13.5 -> 10.6, (4, 8, 600, 128)
+// 14.3 -> 11.3, (2, 8, 1150, 64) 11.5 -> 9.5, (6, 8, 1024, 64) 10.2 -> 10.4; not taken: one partition (1, 8, 300, 128)
+// 8.5 -> 9.8, (16, 2, 300, 64) 8.4 -> 10.0; more than a round (1, 1, 8000, 128) 12.1 -> 18.7, (2, 2, 3000, 64) 9.9 ->
+// 11.4; 448 items at (8, 8, 300-1700, 128) 15.8 -> 20.5.
 __host__ __device__ inline int decode_partition(int part_size, int longest, int items, int max_parts) {
   if (part_size % 256 || part_size > 512 || longest <= part_size) return part_size;
   const int n = (longest + part_size / 2 - 1) / (part_size / 2);

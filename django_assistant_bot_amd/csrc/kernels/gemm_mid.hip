@@ -523,7 +523,9 @@ struct MidTime {
 static MidTime mid_time(int M, int N, int K, int groups) {
   const int tm = (M + 127) / 128, tn = N / 256;
   const double parts = (double)groups / tn;  // of a tile
-  double ends = tn % groups == 0 ? 4. : groups % tn == 0 ? 8. + 1.45 * parts : 18. + (groups > tn ? 1.45 * (parts - 1.) : 0.);
+  double ends = tn % groups == 0   ? 4.
+                : groups % tn == 0 ? 8. + 1.45 * parts
+                                   : 18. + (groups > tn ? 1.45 * (parts - 1.) : 0.);
   if (tn > groups) ends += 3.5 * (1. / parts - 1.);
   return {ends, (double)tn * (K / 64) / groups * (0.45 + 0.0016 * (groups * tm))};
 }
@@ -563,9 +565,9 @@ int gemm_mid_counters(int M, int N) {
 }
 
 // epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over
-// 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes()
-// bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).
-// spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
+// 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs:
+// gemm_mid_slab_bytes() bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the
+// launch leaves them zero).  spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
 // (BK 64), 32 / 64 force the K-step, + 1000 = DIAG 1 (split tiles not combined: timing only).
 // BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank
 // conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.

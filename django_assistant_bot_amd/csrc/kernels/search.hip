@@ -166,7 +166,7 @@ constexpr int RK_BINS = SEL_NT;
 constexpr int RK_FEW = 512;    // entries ranked by counting
 
 // One row's candidates (unordered, cnt[row] of them) -> its k best: score, item id, document id, best first, equal
-// scores in row order; -inf / -1 past the last.  status[row] = 1 where the list cannot be trusted: it overflowed,
+// scores in row order (lists above 4096: in the list's, which its appends leave open); -inf / -1 past the last.  status[row] = 1 where the list cannot be trusted: it overflowed,
 // or it holds fewer than k entries although a threshold cut rows off.
 //
 // A search's lists hold 1-2 thousand entries for some 250 hits.  A histogram of 1024 bins between the list's least and

@@ -254,8 +254,9 @@ class VectorIndex:
         return self.row_ids[live], live
 
     def _live_ids(self):
-        """(sorted item ids, the row of each) on the device, rebuilt after an update.  From the row metadata (first search of 60k rows:
-        0.36 ms) unless an id may have a second live row: the mapping says which of them is its row (2.25 ms)."""
+        """(sorted item ids, the row of each) on the device, rebuilt after an update.  From the row metadata (first search
+        of 60k rows: 0.36 ms) unless an id may have a second live row: the mapping says which of them is its row (2.25
+        ms)."""
         def build():
             if self._twice:
                 host = torch.from_numpy(self._id_rows())
