@@ -71,7 +71,8 @@ class CustomAllReduce:
         with torch.cuda.device(self.device):
             self.base = n.allreduce_buffer_alloc(sig + 2 * self.max_bytes, uncached)
             props = torch.cuda.get_device_properties(self.device)
-            key = (str(props.uuid), props.pci_domain_id, props.pci_bus_id, props.pci_device_id)
+            # (what a torch build does not tell is the same for all ranks: fewer workgroups, never too many)
+            key = tuple(str(getattr(props, a, "")) for a in ("uuid", "pci_domain_id", "pci_bus_id", "pci_device_id"))
             mine = (n.ipc_get_handle(self.base), (key, props.multi_processor_count))
             ranks = [mine]
             if self.world > 1:
