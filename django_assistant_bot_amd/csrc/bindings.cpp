@@ -598,10 +598,18 @@ PYBIND11_MODULE(_native, m) {
   m.def("gemm256_wins", &dab::gemm256_wins);
   m.attr("GEMM256_FILL") = dab::kGemm256Fill;
   m.def("index_scan_takes", [](int M, int K) { return dab::index_scan_takes(M, K) != 0; });
-  m.def("index_scan_scores", [](u A, long lda, u Wshuf, int M, int N, int K, u row_group, u q_group, u scores, u s) {
+  m.def("index_scan_scores", [](u A, long lda, u Wshuf, int M, int N, int K, u row_group, u q_group, u allow, u scores,
+                                u parts, int ldp, u s) {
     check(dab::index_scan_scores_shuf(CVP(A), lda, CVP(Wshuf), M, N, K, reinterpret_cast<const int*>(row_group),
-                                      reinterpret_cast<const int*>(q_group), reinterpret_cast<float*>(scores), ST(s)),
+                                      reinterpret_cast<const int*>(q_group), CVP(allow), reinterpret_cast<float*>(scores),
+                                      VP(parts), ldp, ST(s)),
           "index_scan_scores");
+  });
+  m.def("top_hits", [](u scores, int rows, int n, u parts, int ldp, int k, u row_ids, u row_docs, u out_vals, u out_ids,
+                       u out_docs, u s) {
+    check(dab::top_hits((const float*)scores, rows, n, CVP(parts), ldp, k, (const int64_t*)row_ids, (const int64_t*)row_docs,
+                        (float*)out_vals, (int64_t*)out_ids, (int64_t*)out_docs, ST(s)),
+          "top_hits");
   });
   m.def("gemm_ln", [](u x, u gain, u offset, float eps, u normed, u w, u b, u C, int M, int N, int K, int gelu, int tile, u s) {
     check(dab::gemm_ln(CVP(x), CVP(gain), CVP(offset), eps, VP(normed), CVP(w), CVP(b), VP(C), M, N, K, gelu, tile, ST(s)),

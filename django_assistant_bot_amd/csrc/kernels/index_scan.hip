@@ -43,6 +43,9 @@ struct ScanParams {
   int* cand_idx;
   int cap;
   float* scores;  // SCORES: [M][N]
+  const uint32_t* allow;  // SCORES: [M][ceil(N / 32)] row bitmask or null
+  uint32_t* parts;        // SCORES: [M][ldp] the greatest ordered bits (float_key) of every 16 rows, or null
+  int ldp;
 };
 
 constexpr int kScanKMax = 1024;
@@ -210,8 +213,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void index_scan_kernel(ScanParams 
 // and counters of 32 queries share a cache line (K 256, 1M rows, 128 queries: 238 us against 81 us for one query), and a
 // wave that flushes holds up the others at the barrier.  So the workgroup flushes together (a long list of one wave raises
 // a flag) with one global atomic per query that has hits.
-// SCORES: every score is stored instead, -inf where the group filters drop the row: the row sample of a search.  15,624
-// rows of 768, us (gemm_bt): 1 query 9.5 (14.0), 32: 10.3 (16.5), 128: 20.0 (24.2), 200: 20.5 (25.1).
+// SCORES: every score is stored instead, -inf where the group filters or the row mask drop the row, and on request the
+// greatest of every 16 rows (what the selection of the best k reads first: search.hip).  The filters of a tile travel with
+// its rows, one 4-B copy a lane, and every wave issues the same stores for every tile (masked lanes past the buffer's
+// end), so that the counted wait knows what is younger than the stage it waits for; a load of the filters where they are
+// used, or a wait for the stores, would empty the ring once a tile.  us, rows of 768 (gemm_bt's scores): 4 queries of 60,001
+// rows 17.6 (21.0), 10 of 142,939 41 (51), 42 of 31,098 14.9 (20.8), 1 of 1,000,003 234 (6.6 TB/s).
 // 1M rows of 768, us (floor 236), against queries in LDS / gemm256's candidate epilogue above 96: 1 query 226 (242), 16:
 // 226 (245), 64: 234 (291), 96: 232 (301), 128: 248 (400), 192: 347 (444), 256: 378 (467); of 1024: 1: 300 (315), 128: 333
 // (470); of 256: 1: 81 (83), 128: 124 (257).  20k rows of 768: 1: 21 (23), 128: 27 (36).
@@ -223,8 +230,13 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
   constexpr int H = NCK > 8 ? 2 : 1, HALF = NCK / H;  // stages of a tile, 32-k chunks of a stage
   constexpr int kStage = 2 * HALF * 1024, kDma = kStage / 8192;
   constexpr int NS = NCK <= 16 ? 8 : NCK == 24 ? 6 : 4;
-  constexpr int kQ = 16 * MT * QG, kTail = 64 + 4 * kQ + 8 * kRegList * 10;
+  constexpr int TS = NS / H + 2;  // SCORES: tiles whose filters are held (256 B a wave: 32 row groups, 32 mask words)
+  constexpr int kQ = 16 * MT * QG, kTail = SCORES ? TS * 8 * 256 + 4 * kQ : 64 + 4 * kQ + 8 * kRegList * 10;
   static_assert(RW * RB == 2 && kQ <= 512 && NCK % 8 == 0 && NS * kStage + kTail <= 160 * 1024, "LDS");
+  // entries of a wave's memory queue younger than a stage's rows: those of the NS - 2 stages behind it, and the stores
+  // of the tiles that ended since (SCORES)
+  constexpr int kYoung = (NS - 2) * kDma + (SCORES ? 2 * ((NS - 2) / H) : 0), kStores = SCORES ? 2 * RB * MT : 0;
+  static_assert(kYoung <= 63 && (NS - 2) % H == 0, "vmcnt range");
   typedef __attribute__((address_space(3))) void scan_lds;
   // one array: with two the compiler knows which of them the copies write, and waits for all copies before each read
   __shared__ __attribute__((aligned(16))) char ring[NS * kStage + kTail];
@@ -274,7 +286,12 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
     listed = 0;
     drained();
   };
-  if (tid < 2) flag[tid] = 0;  // read behind the first stage's barrier
+  int* const groups = reinterpret_cast<int*>(ring + NS * kStage + TS * 8 * 256);  // SCORES: of the queries (negative: any)
+  if (SCORES) {
+    if (tid < kQ) groups[tid] = p.row_group && p.q_group ? p.q_group[min(tid, p.M - 1)] : -1;
+  } else if (tid < 2) {
+    flag[tid] = 0;
+  }  // read behind the first stage's barrier
 
   // queries -> registers (rows past the last repeat it; no score reaches their NaN threshold)
   bf16x8 qf[MT][NCK];
@@ -302,8 +319,26 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
     const int d = w + 8 * i;
     dma_off[i] = (unsigned)(((d / HALF) * NCK + d % HALF) * 1024 + lane * 16);
   }
-  // a stage past the last reads an empty range (zeros, no traffic): every step adds kDma copies to the queue
-  auto stage = [&](int buf, int st) {
+  // SCORES: a tile's filters, by lanes 0..31: the rows' groups, and behind them the mask words of the wave's queries
+  const int words = (p.N + 31) / 32;
+  const __amdgpu_buffer_rsrc_t rs_group =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.row_group), (short)0, SCORES && p.row_group ? p.N * 4 : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_allow = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint32_t*>(p.allow), (short)0, SCORES && p.allow ? (int)((unsigned)p.M * (unsigned)words * 4u) : 0, 0x00020000);
+  const uint32_t no_mask = p.allow ? 0u : ~0u;
+  const unsigned allow_off = SCORES ? (unsigned)(q0 + min(lane, 16 * MT - 1)) * (unsigned)words * 4u : 0u;
+  auto filters = [&](int st) {
+    const unsigned tile = st < steps ? blockIdx.x + (unsigned)(st / H) * gridDim.x : 0u;
+    char* dst = ring + NS * kStage + (((unsigned)(st / H) % TS) * 8 + w) * 256;
+    if (lane < 32) {  // (past the end: zeros)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_group, (scan_lds*)dst, 4, 4u * lane, 128u * tile, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_allow, (scan_lds*)(dst + 128), 4, allow_off, 4u * tile, 0, 0);
+    }
+  };
+  // a stage past the last reads an empty range (zeros, no traffic): every step adds the same copies to the queue
+  // (first: it starts a tile)
+  auto stage = [&](int buf, int st, bool first) {
+    if (SCORES && first) filters(st);
     const size_t tile = blockIdx.x + (size_t)(st / H) * gridDim.x;
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(p.W + (st < steps ? tile : 0) * (2 * NCK * 512)), (short)0,
@@ -315,7 +350,12 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (scan_lds*)(dst + i * 8192), 16, (unsigned)dma_off[i], so, 0, 2);
   };
 #pragma unroll
-  for (int st = 0; st < NS - 1; ++st) stage(st, st);
+  for (int st = 0; st < NS - 1; ++st) stage(st, st, st % H == 0);
+  // buffers of the scores and the parts' maxima: a lane without one stores past their end, where it is dropped
+  const __amdgpu_buffer_rsrc_t rs_scores =
+      __builtin_amdgcn_make_buffer_rsrc(p.scores, (short)0, SCORES ? (int)((unsigned)p.M * (unsigned)p.N * 4u) : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_parts =
+      __builtin_amdgcn_make_buffer_rsrc(p.parts, (short)0, p.parts ? (int)((unsigned)p.M * (unsigned)p.ldp * 4u) : 0, 0x00020000);
   int buf = 0;
   for (int st = 0; st < steps; st += H) {
     f32x4 acc[RB][MT];
@@ -325,11 +365,16 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
       for (int t = 0; t < MT; ++t) acc[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int h = 0; h < H; ++h) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"((NS - 2) * kDma) : "memory");
+      // the stores of tile j are younger than stage s where H j + H + NS - 2 >= s: those of the last tiles before this one
+      constexpr int kEnded = (NS - 1) / H, kMost = kYoung + kEnded * kStores;  // (one more tile at the first of two stages)
+      if (SCORES && live && st / H > kEnded)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kMost < 63 ? kMost : 63) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kYoung) : "memory");
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last stage's reads: its buffer is filled next
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      stage(buf == 0 ? NS - 1 : buf - 1, st + h + NS - 1);
+      stage(buf == 0 ? NS - 1 : buf - 1, st + h + NS - 1, (h + NS - 1) % H == 0);
       if (live) {
         const char* src = ring + buf * kStage + rw * (HALF * 1024) + lane * 16;
         constexpr int PF = 4 / RB;  // fragments read ahead
@@ -362,26 +407,43 @@ __global__ __launch_bounds__(512, 2) void index_scan_reg_kernel(ScanParams p) {
     if (!live) continue;
     const int r0 = (blockIdx.x + st / H * gridDim.x) * 32 + 16 * RB * rw;
     if constexpr (SCORES) {
+      const unsigned at = (unsigned)(uintptr_t)(scan_lds*)(ring + NS * kStage + (((unsigned)(st / H) % TS) * 8 + w) * 256);
 #pragma unroll
       for (int a = 0; a < RB; ++a) {
-        const int n = r0 + 16 * a + 4 * g;
-        if (n >= p.N) continue;  // N % 4 == 0 (launcher)
-        int4 rg = {0, 0, 0, 0};
-        if (p.row_group) rg = *reinterpret_cast<const int4*>(p.row_group + n);
-        const int group[4] = {rg.x, rg.y, rg.z, rg.w};
+        const int n = r0 + 16 * a + 4 * g, in = n & 31;  // (N % 4 == 0: four rows are there or none of them)
+        int4 group;  // (read by asm statements: before an ordinary read hipcc may drain the copies in flight)
+        asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(group) : "v"(at + 4u * in) : "memory");
+        const int rg[4] = {group.x, group.y, group.z, group.w};
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
           const int m = q0 + 16 * t + li;
-          if (m >= p.M) continue;
-          const int qgm = p.q_group ? p.q_group[m] : -1;
-          f32x4 v = acc[a][t];
+          uint32_t seen;
+          int q_group;
+          asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(seen), "=&v"(q_group)
+                       : "v"(at + 128u + 4u * (16 * t + li)), "v"((unsigned)(uintptr_t)(scan_lds*)(groups + m)) : "memory");
+          seen = (seen | no_mask) >> in;
+          f32x4 v;  // (without branches: hipcc lost a lane's -inf behind those of && on vector elements)
+          uint32_t best = 0;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (!(group[r] >= 0 && (qgm < 0 || group[r] == qgm))) v[r] = -__builtin_huge_valf();
-          *reinterpret_cast<f32x4*>(p.scores + (size_t)m * p.N + n) = v;
+          for (int r = 0; r < 4; ++r) {
+            const bool pass = (rg[r] >= 0) & ((q_group < 0) | (rg[r] == q_group)) & ((seen >> r & 1u) != 0u) & (n < p.N);
+            const float x = pass ? acc[a][t][r] : -__builtin_huge_valf();
+            best = max(best, float_key(x));
+            v[r] = x;
+          }
+          const bool there = m < p.M && n < p.N;
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs_scores,
+                                                 there ? ((unsigned)m * (unsigned)p.N + (unsigned)n) * 4u : 0xffffff00u, 0, 0);
+          const auto s32 = __builtin_amdgcn_permlane32_swap(best, best, false, false);  // over the 16 rows
+          best = max(s32[0], s32[1]);
+          const auto s16 = __builtin_amdgcn_permlane16_swap(best, best, false, false);
+          best = max(s16[0], s16[1]);
+          __builtin_amdgcn_raw_buffer_store_b32(best, rs_parts,
+                                                there && g == 0 ? ((unsigned)m * (unsigned)p.ldp + (unsigned)(n >> 4)) * 4u : 0xffffff00u,
+                                                0, 0);
         }
       }
-      drained();
       continue;
     }
 #pragma unroll
@@ -499,16 +561,19 @@ int index_scan_candidates_shuf(const void* X, long ldx, const void* W, int M, in
                                int cap, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
   if (cap <= 0) return hipErrorInvalidValue;
-  const ScanParams p = {(const bf16*)X, ldx, (const bf16*)W, K, M, N, K, row_group, q_group, thr, cnt, cand_val, cand_idx, cap, nullptr};
+  const ScanParams p = {(const bf16*)X, ldx, (const bf16*)W, K, M, N, K, row_group, q_group, thr, cnt, cand_val, cand_idx, cap, nullptr, nullptr, nullptr, 0};
   return scan_reg_launch<false>(p, s);
 }
 
-// ... their scores [M][N], N % 4 == 0, -inf where the groups drop a row
+// ... their scores [M][N], N % 4 == 0, -inf where the groups or the row mask drop a row; parts (or null): the greatest
+// ordered bits of every 16 rows, [M][ldp]
 int index_scan_scores_shuf(const void* X, long ldx, const void* W, int M, int N, int K, const int* row_group,
-                           const int* q_group, float* scores, hipStream_t s) {
+                           const int* q_group, const void* allow, float* scores, void* parts, int ldp, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
-  if (N % 4 || ((uintptr_t)scores | (uintptr_t)row_group) % 16) return hipErrorInvalidValue;
-  const ScanParams p = {(const bf16*)X, ldx, (const bf16*)W, K, M, N, K, row_group, q_group, nullptr, nullptr, nullptr, nullptr, 0, scores};
+  if (N % 4 || ((uintptr_t)scores | (uintptr_t)row_group) % 16 || (parts && ldp < (N + 15) / 16)) return hipErrorInvalidValue;
+  if ((long)M * N * 4 > 0xffffff00L || (parts && (long)M * ldp * 4 > 0xffffff00L)) return hipErrorInvalidValue;  // buffer range
+  const ScanParams p = {(const bf16*)X, ldx, (const bf16*)W, K, M, N, K, row_group, q_group, nullptr, nullptr, nullptr, nullptr, 0,
+                        scores, (const uint32_t*)allow, (uint32_t*)parts, ldp};
   return scan_reg_launch<true>(p, s);
 }
 

@@ -319,7 +319,7 @@ int index_scan_candidates_shuf(const void* X, long ldx, const void* W, int M, in
                                const int* q_group, const float* thr, int* cnt, float* cand_val, int* cand_idx,
                                int cap, hipStream_t s);
 int index_scan_scores_shuf(const void* X, long ldx, const void* W, int M, int N, int K, const int* row_group,
-                           const int* q_group, float* scores, hipStream_t s);
+                           const int* q_group, const void* allow, float* scores, void* parts, int ldp, hipStream_t s);
 int stream_score_candidates(const void* X, long ldx, const void* W, long ldw, int M, int N, int K, const int* row_group,
                             const int* q_group, const float* thr, int* cnt, float* cand_val, int* cand_idx, int cap,
                             hipStream_t s);
@@ -377,6 +377,8 @@ int rank_value(const float* scores, long ld, int rows, int n, int r, float slack
 int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const float* thr, int cap, int rows, int k,
               const int64_t* row_ids, const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs,
               int* status, hipStream_t s);
+int top_hits(const float* scores, int rows, int n, const void* parts, int ldp, int k, const int64_t* row_ids,
+             const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs, hipStream_t s);
 int allow_bits(const int64_t* ids, const int64_t* off, const int64_t* keys, const int64_t* rows, int n_keys,
                uint32_t* mask, int words, int queries, int longest, hipStream_t s);
 int doc_lt_bits(const int64_t* docs, const int64_t* limit, int n, uint32_t* mask, int words, int queries, int intersect,

@@ -161,95 +161,25 @@ int rank_value(const float* scores, long ld, int rows, int n, int r, float slack
   return hipGetLastError();
 }
 
-constexpr int RK_SORT = 4096;  // candidates held in LDS
+constexpr int RK_SORT = 4096;  // candidates of a list held in LDS
 constexpr int RK_BINS = SEL_NT;
 constexpr int RK_FEW = 512;    // entries ranked by counting
+constexpr int RK_MANY = 2048;  // entries behind the histogram's cut that are held
 
-// One row's candidates (unordered, cnt[row] of them) -> its k best: score, item id, document id, best first, equal
-// scores in row order (lists above 4096: in the list's, which its appends leave open); -inf / -1 past the last.  status[row] = 1 where the list cannot be trusted: it overflowed,
-// or it holds fewer than k entries although a threshold cut rows off.
-//
-// A search's lists hold 1-2 thousand entries for some 250 hits.  A histogram of 1024 bins between the list's least and
-// greatest score leaves little more than the hits (bins are equal steps of the ordered bits: monotone for any scores),
-// and up to 512 entries are ranked by counting the greater ones: one chain of LDS reads instead of the 66 steps of a
-// bitonic sort of the list.  Where more remain (k above some 400, many near-equal scores) the whole list is sorted: its
-// steps up to stride 64 stay inside the 128 entries of a wave and need no workgroup barrier.  Lists above 4096 are
-// radix-selected.  With the ids and documents in the same launch 7.9 us for 1,300
-// candidates of one query and 9.8 for 128 queries (sorted whole: 22 and 31; radix select of 16,000 and five
-// element-wise launches behind it: 61 and 91).
-__global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restrict__ cand_val,
-                                                           const int* __restrict__ cand_idx,
-                                                           const int* __restrict__ cnt, const float* __restrict__ thr,
-                                                           int cap, int k, const int64_t* __restrict__ row_ids,
-                                                           const int64_t* __restrict__ row_docs,
-                                                           float* __restrict__ out_vals, int64_t* __restrict__ out_ids,
-                                                           int64_t* __restrict__ out_docs, int* __restrict__ status) {
-  __shared__ union {
-    struct {
-      unsigned long long key[RK_SORT];
-      __attribute__((aligned(16))) unsigned long long few[RK_FEW];
-      uint32_t hist[RK_BINS];
-      uint32_t rank[RK_FEW];
-      uint32_t lo[SEL_NT / 64], hi[SEL_NT / 64], total[SEL_NT / 64];
-      uint32_t bin, n;
-    };
-    SelShared sel;
-  } sh;
-  const int row = blockIdx.x, tid = threadIdx.x;
-  const int c = cnt[row];
-  const bool bad = c > cap || (c < k && !(thr[row] == -INFINITY));  // (a NaN threshold passes nothing)
-  if (tid == 0) status[row] = bad;
-  if (bad) return;
-  const float* cv = cand_val + (size_t)row * cap;
-  const int* ci = cand_idx + (size_t)row * cap;
-  out_vals += (size_t)row * k;
-  out_ids += (size_t)row * k;
-  out_docs += (size_t)row * k;
-  auto emit = [&](int i, float v, int r) {
-    out_vals[i] = v;
-    out_ids[i] = row_ids[r];
-    out_docs[i] = row_docs[r];
-  };
-  const int kept = min(k, c);
-  for (int i = kept + tid; i < k; i += SEL_NT) {
-    out_vals[i] = -INFINITY;
-    out_ids[i] = -1;
-    out_docs[i] = -1;
-  }
-  if (c > RK_SORT) {
-    select_topk([&](int i) -> uint32_t { return float_key(cv[i]); }, c, kept, sh.sel);
-    for (int i = tid; i < kept; i += SEL_NT) emit(i, key_float(sh.sel.cand_key[i]), ci[sh.sel.cand_idx[i]]);
-    return;
-  }
-  if (kept == 0) return;
-  const int lane = tid & 63, w = tid >> 6;
-  uint32_t lo = ~0u, hi = 0u;
-  for (int i = tid; i < c; i += SEL_NT) {
-    const uint32_t key = float_key(cv[i]);
-    sh.key[i] = ((unsigned long long)key << 32) | (uint32_t)~ci[i];
-    lo = min(lo, key);
-    hi = max(hi, key);
-  }
-  lo = wave_fold_bits(lo, [](uint32_t x, uint32_t y) { return min(x, y); });
-  hi = wave_fold_bits(hi, [](uint32_t x, uint32_t y) { return max(x, y); });
-  if (lane == 0) {
-    sh.lo[w] = lo;
-    sh.hi[w] = hi;
-  }
-  sh.hist[tid] = 0;
-  if (tid < RK_FEW) sh.rank[tid] = 0;
-  if (tid == 0) sh.n = 0;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < SEL_NT / 64; ++j) {
-    lo = min(lo, sh.lo[j]);
-    hi = max(hi, sh.hi[j]);
-  }
-  const int shift = max(0, 22 - __clz(hi - lo));  // (hi - lo) >> shift < 1024; (__clz(0) = 32)
-  auto bin_of = [&](unsigned long long e) { return ((uint32_t)(e >> 32) - lo) >> shift; };
-  for (int i = tid; i < c; i += SEL_NT) atomicAdd(&sh.hist[bin_of(sh.key[i])], 1u);
-  __syncthreads();
-  // bins from the top: the one in which the count reaches `kept`
+template <int CAP>
+struct RankShared {
+  unsigned long long key[CAP];  // ordered bits of the score, ~row
+  __attribute__((aligned(16))) unsigned long long few[RK_MANY];
+  uint32_t hist[RK_BINS];
+  uint32_t rank[RK_FEW];
+  uint32_t lo[SEL_NT / 64], hi[SEL_NT / 64], total[SEL_NT / 64];
+  uint32_t bin, n;
+};
+
+// The bin in which the count from the top reaches `kept` (of at least that many entries), for all threads.
+template <int CAP>
+__device__ __forceinline__ uint32_t cut_bin(RankShared<CAP>& sh, uint32_t kept) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const uint32_t h = sh.hist[RK_BINS - 1 - tid];
   uint32_t incl = h;
 #pragma unroll
@@ -260,14 +190,70 @@ __global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restri
   if (lane == 63) sh.total[w] = incl;
   __syncthreads();
   for (int j = 0; j < w; ++j) incl += sh.total[j];
-  if (incl - h < (uint32_t)kept && (uint32_t)kept <= incl) sh.bin = RK_BINS - 1 - tid;
+  if (incl - h < kept && kept <= incl) sh.bin = RK_BINS - 1 - tid;
   __syncthreads();
-  const uint32_t least = sh.bin;
+  return sh.bin;
+}
+
+// The block's least and greatest value.
+template <int CAP>
+__device__ __forceinline__ void block_range(RankShared<CAP>& sh, uint32_t& lo, uint32_t& hi) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  lo = wave_fold_bits(lo, [](uint32_t x, uint32_t y) { return min(x, y); });
+  hi = wave_fold_bits(hi, [](uint32_t x, uint32_t y) { return max(x, y); });
+  if (lane == 0) {
+    sh.lo[w] = lo;
+    sh.hi[w] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < SEL_NT / 64; ++j) {
+    lo = min(lo, sh.lo[j]);
+    hi = max(hi, sh.hi[j]);
+  }
+}
+
+// Shift after which steps of (key - lo) fall into RK_BINS bins: monotone for any scores.  (__clz(0) = 32)
+__device__ __forceinline__ int bin_shift(uint32_t lo, uint32_t hi) { return max(0, 22 - __clz(hi - lo)); }
+
+// Bitonic, greatest first; P a power of two, at least 64.  A wave's 64 consecutive pairs lie in its own 128 entries where
+// the stride is 64 or less: no workgroup barrier there.
+__device__ __forceinline__ void sort_desc(unsigned long long* key, int P) {
+  for (int size = 2; size <= P; size <<= 1)
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int p = threadIdx.x; p < P / 2; p += SEL_NT) {
+        const int a = 2 * p - (p & (stride - 1)), b = a + stride;
+        const unsigned long long ka = key[a], kb = key[b];
+        if ((ka > kb) != ((a & size) == 0)) {
+          key[a] = kb;
+          key[b] = ka;
+        }
+      }
+      if (stride > 64 || (stride == 1 && size >= 128))
+        __syncthreads();  // (the next size's first stride is `size`: across waves from size 128 on)
+      else
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // a wave's own LDS operations, in order
+    }
+  __syncthreads();
+}
+
+// sh.key[0 .. c) in any order -> emit(place, entry, id, document) for the `kept` (1 .. c) greatest.  lo, hi: of the entries this thread has
+// written; the caller has cleared hist, rank and n and no barrier is due.
+template <int CAP, typename F>
+__device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uint32_t hi, const int64_t* row_ids,
+                          const int64_t* row_docs, F emit) {
+  const int tid = threadIdx.x;
+  block_range(sh, lo, hi);
+  const int shift = bin_shift(lo, hi);
+  auto bin_of = [&](unsigned long long e) { return ((uint32_t)(e >> 32) - lo) >> shift; };
+  for (int i = tid; i < c; i += SEL_NT) atomicAdd(&sh.hist[bin_of(sh.key[i])], 1u);
+  __syncthreads();
+  const uint32_t least = cut_bin(sh, (uint32_t)kept);
   for (int i = tid; i < c; i += SEL_NT) {
     const unsigned long long e = sh.key[i];
     if (bin_of(e) < least) continue;
     const uint32_t at = atomicAdd(&sh.n, 1u);
-    if (at < RK_FEW) sh.few[at] = e;
+    if (at < RK_MANY) sh.few[at] = e;
   }
   __syncthreads();
   const int m = (int)sh.n;
@@ -293,38 +279,86 @@ __global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restri
       atomicAdd(&sh.rank[e], above);
     }
     __syncthreads();
-    if (own && part == 0) {
-      const int i = (int)sh.rank[e];
-      if (i < kept) {
-        out_vals[i] = key_float((uint32_t)(mine >> 32));
-        out_ids[i] = id;
-        out_docs[i] = doc;
-      }
+    if (own && part == 0 && (int)sh.rank[e] < kept) emit((int)sh.rank[e], mine, id, doc);
+    return;
+  }
+  unsigned long long* list = m <= RK_MANY ? sh.few : sh.key;
+  const int n = m <= RK_MANY ? m : c;
+  int P = 64;
+  while (P < n) P <<= 1;
+  for (int i = n + tid; i < P; i += SEL_NT) list[i] = 0ull;
+  __syncthreads();
+  sort_desc(list, P);
+  for (int i = tid; i < kept; i += SEL_NT) {
+    const uint32_t r = ~(uint32_t)list[i];
+    emit(i, list[i], row_ids[r], row_docs[r]);
+  }
+}
+
+// One row's candidates (unordered, cnt[row] of them) -> its k best: score, item id, document id, best first, equal
+// scores in row order (lists above 4096: in the list's, which its appends leave open); -inf / -1 past the last.  status[row] = 1 where the list cannot be trusted: it overflowed,
+// or it holds fewer than k entries although a threshold cut rows off.
+//
+// A search's lists hold 1-2 thousand entries for some 250 hits.  A histogram of 1024 bins between the list's least and
+// greatest score leaves little more than the hits (bins are equal steps of the ordered bits: monotone for any scores),
+// and up to 512 entries are ranked by counting the greater ones: one chain of LDS reads instead of the 66 steps of a
+// bitonic sort of the list.  Where more remain (k above some 400, many near-equal scores) they are sorted, or the whole
+// list where they are more than 2048.  Lists above 4096 are radix-selected.  With the ids and documents in the same launch 7.9 us for 1,300
+// candidates of one query and 9.8 for 128 queries (sorted whole: 22 and 31; radix select of 16,000 and five
+// element-wise launches behind it: 61 and 91).
+__global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restrict__ cand_val,
+                                                           const int* __restrict__ cand_idx,
+                                                           const int* __restrict__ cnt, const float* __restrict__ thr,
+                                                           int cap, int k, const int64_t* __restrict__ row_ids,
+                                                           const int64_t* __restrict__ row_docs,
+                                                           float* __restrict__ out_vals, int64_t* __restrict__ out_ids,
+                                                           int64_t* __restrict__ out_docs, int* __restrict__ status) {
+  __shared__ union {
+    RankShared<RK_SORT> list;
+    SelShared sel;
+  } sh;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const int c = cnt[row];
+  const bool bad = c > cap || (c < k && !(thr[row] == -INFINITY));  // (a NaN threshold passes nothing)
+  if (tid == 0) status[row] = bad;
+  if (bad) return;
+  const float* cv = cand_val + (size_t)row * cap;
+  const int* ci = cand_idx + (size_t)row * cap;
+  out_vals += (size_t)row * k;
+  out_ids += (size_t)row * k;
+  out_docs += (size_t)row * k;
+  const int kept = min(k, c);
+  for (int i = kept + tid; i < k; i += SEL_NT) {
+    out_vals[i] = -INFINITY;
+    out_ids[i] = -1;
+    out_docs[i] = -1;
+  }
+  if (c > RK_SORT) {
+    select_topk([&](int i) -> uint32_t { return float_key(cv[i]); }, c, kept, sh.sel);
+    for (int i = tid; i < kept; i += SEL_NT) {
+      const int r = ci[sh.sel.cand_idx[i]];
+      out_vals[i] = key_float(sh.sel.cand_key[i]);
+      out_ids[i] = row_ids[r];
+      out_docs[i] = row_docs[r];
     }
     return;
   }
-  int P = 64;
-  while (P < c) P <<= 1;
-  for (int i = c + tid; i < P; i += SEL_NT) sh.key[i] = 0ull;
-  __syncthreads();
-  for (int size = 2; size <= P; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      // pair p = (a, a + stride); a wave's 64 consecutive pairs lie in its own 128 entries when stride <= 64
-      for (int p = tid; p < P / 2; p += SEL_NT) {
-        const int a = 2 * p - (p & (stride - 1)), b = a + stride;
-        const unsigned long long ka = sh.key[a], kb = sh.key[b];
-        if ((ka > kb) != ((a & size) == 0)) {
-          sh.key[a] = kb;
-          sh.key[b] = ka;
-        }
-      }
-      if (stride > 64 || (stride == 1 && size >= 128))
-        __syncthreads();  // (the next size's first stride is `size`: across waves from size 128 on)
-      else
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // a wave's own LDS operations, in order
-    }
-  __syncthreads();
-  for (int i = tid; i < kept; i += SEL_NT) emit(i, key_float((uint32_t)(sh.key[i] >> 32)), (int)~(uint32_t)sh.key[i]);
+  if (kept == 0) return;
+  uint32_t lo = ~0u, hi = 0u;
+  for (int i = tid; i < c; i += SEL_NT) {
+    const uint32_t key = float_key(cv[i]);
+    sh.list.key[i] = ((unsigned long long)key << 32) | (uint32_t)~ci[i];
+    lo = min(lo, key);
+    hi = max(hi, key);
+  }
+  sh.list.hist[tid] = 0;
+  if (tid < RK_FEW) sh.list.rank[tid] = 0;
+  if (tid == 0) sh.list.n = 0;
+  rank_list(sh.list, c, kept, lo, hi, row_ids, row_docs, [&](int i, unsigned long long e, int64_t id, int64_t doc) {
+    out_vals[i] = key_float((uint32_t)(e >> 32));
+    out_ids[i] = id;
+    out_docs[i] = doc;
+  });
 }
 
 int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const float* thr, int cap, int rows, int k,
@@ -334,6 +368,152 @@ int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const 
   if (k < 1 || k > SEL_MAXK || cap < 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(rank_hits_kernel, dim3(rows), dim3(SEL_NT), 0, s, cand_val, cand_idx, cnt, thr, cap, k, row_ids,
                      row_docs, out_vals, out_ids, out_docs, status);
+  return hipGetLastError();
+}
+
+constexpr int TH_CAND = 8192;   // candidates held in LDS, and the scores of a row that need no parts
+constexpr int TH_PARTS = 4096;  // parts looked into
+constexpr int TH_HELD = 16;     // 16-B vectors of part maxima a thread keeps in registers between its two looks
+
+// The k best of every row of scores [n] -> score, item id, document id, best first, equal scores in row order; -inf / -1
+// where fewer rows pass the filters.  One workgroup a row; parts: the greatest ordered bits of every 16 scores.
+//
+// The k-th greatest of maxima over disjoint parts is a bound that at least k scores reach, and where the parts are many
+// times k few more do.  So the scores themselves are read only in the parts that reach it: 64 KB of maxima and some 20 KB
+// of scores for 250 of 262,144, and the rest is the ranking of about 300 candidates.  The bound is the lower end of the
+// bin of a 1024-bin histogram of the threads' maxima in which the count from the top reaches k (parts of up to 1024 threads).
+// Rows of up to 8192 scores are ranked as they are.  Where more than 8192 scores reach the bound (k near the number of
+// parts that pass the filters, many equal scores) the row is radix-selected.
+//
+// us, against a radix select by one workgroup a query (up to 32,768 scores) or selection in chunks and a merge, and the
+// ids' launch: 42 queries of 31,098 rows 9.8 (188), 4 of 60,001 9.5 (34), 10 of 142,939 10.1 (40); 1 of 1,000,003 17.3.
+__global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restrict__ scores, int n,
+                                                          const uint32_t* __restrict__ parts, int ldp, int k,
+                                                          const int64_t* __restrict__ row_ids,
+                                                          const int64_t* __restrict__ row_docs,
+                                                          float* __restrict__ out_vals, int64_t* __restrict__ out_ids,
+                                                          int64_t* __restrict__ out_docs) {
+  __shared__ union {
+    struct {
+      RankShared<TH_CAND> list;
+      uint32_t part[TH_PARTS];
+      uint32_t n_part, n_cand;
+    };
+    SelShared sel;
+  } sh;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const float* s = scores + (size_t)row * n;
+  out_vals += (size_t)row * k;
+  out_ids += (size_t)row * k;
+  out_docs += (size_t)row * k;
+  auto emit = [&](int i, unsigned long long e, int64_t id, int64_t doc) {
+    const float v = key_float((uint32_t)(e >> 32));
+    const bool hit = !isinf(v);
+    out_vals[i] = v;
+    out_ids[i] = hit ? id : -1;
+    out_docs[i] = hit ? doc : -1;
+  };
+  sh.list.hist[tid] = 0;
+  if (tid < RK_FEW) sh.list.rank[tid] = 0;
+  if (tid == 0) {
+    sh.list.n = 0;
+    sh.n_part = 0;
+    sh.n_cand = 0;
+  }
+  uint32_t lo = ~0u, hi = 0u;
+  // a score at or above the bound takes a slot (n % 4 == 0: whole vectors)
+  auto take = [&](int i, uint32_t bound) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(s + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t key = float_key(v[e]);
+      const int at = wave_append(&sh.n_cand, key >= bound && key != kNegInfKey);
+      if (at >= 0 && at < TH_CAND) {
+        sh.list.key[at] = ((unsigned long long)key << 32) | (uint32_t)~(i + e);
+        lo = min(lo, key);
+        hi = max(hi, key);
+      }
+    }
+  };
+  bool over = false;
+  if (n <= TH_CAND) {
+    __syncthreads();
+    for (int i = 4 * tid; i < n; i += 4 * SEL_NT) take(i, 0u);
+  } else {
+    const u32x4* pv = reinterpret_cast<const u32x4*>(parts + (size_t)row * ldp);
+    const int np = (n + 15) / 16, nv = (np + 3) / 4;
+    u32x4 held[TH_HELD];
+    uint32_t m = 0;
+    auto look = [&](int v) {  // past the last part: zeros
+      u32x4 x = pv[min(v, nv - 1)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = 4 * v + e < np ? x[e] : 0u;
+      return x;
+    };
+#pragma unroll
+    for (int j = 0; j < TH_HELD; ++j) held[j] = look(tid + j * SEL_NT);
+#pragma unroll
+    for (int j = 0; j < TH_HELD; ++j) m = max(max(m, max(held[j][0], held[j][1])), max(held[j][2], held[j][3]));
+#pragma unroll 4
+    for (int v = tid + TH_HELD * SEL_NT; v < nv; v += SEL_NT) {
+      const u32x4 x = look(v);
+      m = max(max(m, max(x[0], x[1])), max(x[2], x[3]));
+    }
+    // the bound: of the threads with a score that passed
+    uint32_t mlo = m > kNegInfKey ? m : ~0u, mhi = m;
+    const int live = __syncthreads_count(m > kNegInfKey);
+    block_range(sh.list, mlo, mhi);
+    uint32_t bound = kNegInfKey + 1;
+    if (live >= k) {
+      const int shift = bin_shift(mlo, mhi);
+      if (m > kNegInfKey) atomicAdd(&sh.list.hist[(m - mlo) >> shift], 1u);
+      __syncthreads();
+      bound = mlo + (cut_bin(sh.list, (uint32_t)k) << shift);
+      sh.list.hist[tid] = 0;
+    }
+    auto keep = [&](const u32x4& x, int v) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int at = wave_append(&sh.n_part, x[e] >= bound);
+        if (at >= 0 && at < TH_PARTS) sh.part[at] = 4 * v + e;
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < TH_HELD; ++j)
+      if (__ballot(max(max(held[j][0], held[j][1]), max(held[j][2], held[j][3])) >= bound)) keep(held[j], tid + j * SEL_NT);
+#pragma unroll 4
+    for (int v = tid + TH_HELD * SEL_NT; v < nv; v += SEL_NT) keep(look(v), v);
+    __syncthreads();
+    const int chosen = (int)sh.n_part;
+    over = chosen > TH_PARTS;
+    if (!over)
+      for (int e = tid; e < 4 * chosen; e += SEL_NT) {
+        const int i = 16 * (int)sh.part[e >> 2] + 4 * (e & 3);
+        if (i < n) take(i, bound);
+      }
+  }
+  __syncthreads();
+  const int c = (int)sh.n_cand, kept = min(k, c);
+  if (over || c > TH_CAND) {
+    __syncthreads();  // (the counts are read: the union's other half is written next)
+    select_topk([&](int i) -> uint32_t { return float_key(s[i]); }, n, k, sh.sel);
+    for (int i = tid; i < k; i += SEL_NT) {
+      const int r = sh.sel.cand_idx[i];
+      emit(i, (unsigned long long)sh.sel.cand_key[i] << 32, row_ids[r], row_docs[r]);
+    }
+    return;
+  }
+  for (int i = kept + tid; i < k; i += SEL_NT) emit(i, (unsigned long long)kNegInfKey << 32, -1, -1);
+  if (kept) rank_list(sh.list, c, kept, lo, hi, row_ids, row_docs, emit);
+}
+
+int top_hits(const float* scores, int rows, int n, const void* parts, int ldp, int k, const int64_t* row_ids,
+             const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (n <= 0 || n % 4 || k < 1 || k > n || k > SEL_MAXK || (uintptr_t)scores % 16) return hipErrorInvalidValue;
+  if (n > TH_CAND && (!parts || (uintptr_t)parts % 16 || ldp % 4 || ldp < (n + 15) / 16)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(top_hits_kernel, dim3(rows), dim3(SEL_NT), 0, s, scores, n, (const uint32_t*)parts, ldp, k, row_ids,
+                     row_docs, out_vals, out_ids, out_docs);
   return hipGetLastError();
 }
 

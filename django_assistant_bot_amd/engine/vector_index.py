@@ -273,7 +273,7 @@ class VectorIndex:
         if mask is not None and mask.shape[0] != len(limits):
             return mask & self.doc_lt_mask(limits)
         words = (self.n + 31) // 32
-        lim = torch.as_tensor(np.asarray(limits, dtype=np.int64), device=self.device)
+        lim = self._there(torch.as_tensor(np.asarray(limits, dtype=np.int64)))
         if self.device.type == "cuda" and lim.dim() == 1 and self.n and 0 < len(lim) <= 65535:
             return ops.doc_lt_bits(self.row_docs[: self.n], lim, mask)
         lim = lim[:, None]
@@ -287,18 +287,27 @@ class VectorIndex:
         """fp32 cosine similarities [q, n] (-inf for filtered / deleted rows).  Filters: ``q_groups``
         (per-query row group, e.g. bot + status bit), ``allowed`` (per-query item ids), ``doc_lt``
         (per-query document-id bound); masks are ANDed."""
-        q = ops.unit_rows(torch.as_tensor(queries).to(self.device, torch.float32), self.dtype)
-        qg = None if q_groups is None else torch.as_tensor(q_groups, dtype=torch.int32).to(self.device)
-        allow = None if allowed is None else self.allow_mask(allowed)
-        if doc_lt is not None:
-            allow = self.doc_lt_mask(doc_lt, allow)
-        n = max(self.n, 4)
-        n = (n + 3) // 4 * 4
+        q, qg, allow, n = self._query(queries, q_groups, allowed, doc_lt)
         if self.frag:
             return ops.gemm_bt(q, self.vecs, epilogue=ops.EPI_SCORES, out_f32=True, row_group=self.row_group[:n],
                                q_group=qg, allow=allow, shuffled=True, n=n)
         return ops.gemm_bt(q, self.vecs[:n], epilogue=ops.EPI_SCORES, out_f32=True, row_group=self.row_group[:n],
                            q_group=qg, allow=allow)
+
+    def _there(self, t: torch.Tensor) -> torch.Tensor:
+        """A small host tensor on the index's device, without a wait for the copy (pageable memory is waited for)."""
+        if self.device.type == "cuda" and not t.is_cuda:
+            t = t.pin_memory()
+        return t.to(self.device, non_blocking=True)
+
+    def _query(self, queries, q_groups, allowed, doc_lt):
+        """(unit queries, their groups, row mask, rows in whole fours) on the device."""
+        q = ops.unit_rows(torch.as_tensor(queries).to(self.device, torch.float32), self.dtype)
+        qg = None if q_groups is None else self._there(torch.as_tensor(q_groups, dtype=torch.int32))
+        allow = None if allowed is None else self.allow_mask(allowed)
+        if doc_lt is not None:
+            allow = self.doc_lt_mask(doc_lt, allow)
+        return q, qg, allow, (max(self.n, 4) + 3) // 4 * 4
 
     @torch.inference_mode()
     def search(self, queries, k: int, q_groups=None, allowed=None, doc_lt=None):
@@ -311,14 +320,39 @@ class VectorIndex:
         if self.n == 0 or k <= 0 or nq == 0:
             z = torch.full((nq, max(k, 0)), -1, dtype=torch.int64, device=self.device)
             return torch.full((nq, max(k, 0)), float("-inf"), device=self.device), z, z.clone()
-        if (self.device.type == "cuda" and allowed is None and doc_lt is None and self.n >= self.threshold_min_rows
-                and k <= 1024 and self.threshold_search):
+        plain = allowed is None and doc_lt is None
+        if self._selects(nq, plain):
+            return self._selected_search(queries, k, q_groups, allowed, doc_lt)
+        if self.device.type == "cuda" and plain and self.n >= self.threshold_min_rows and k <= 1024 and self.threshold_search:
             got = self._threshold_search(queries, k, q_groups)
             if got is not None:
                 return got
         s = self.scores(queries, q_groups, allowed, doc_lt)
         vals, rows = ops.topk_rows(s, min(k, s.shape[1], 1024))
         return (vals, *ops.hit_ids(vals, rows, self.row_ids, self.row_docs))
+
+    # From ``threshold_min_rows`` on: rows, and scores in all, up to which a search selects from its scores.  It saves the
+    # sample and its two launches, the ranking's and the host read (some 45 us) and writes 4 B a row and query, and one
+    # workgroup a query looks through its maxima.  Threshold / selection, us, rows of 768: 1M and 1 query 298 / 258, 4: 299 /
+    # 282, 8: 301 / 293, 16: 298 / 303; 600k and 16 213 / 196, 32: 210 / 207; 2M and 1 517 / 514, 4: 517 / 555.  Of 256: 1M
+    # and 16 143 / 129; of 1024: 1M and 8 368 / 369.
+    select_rows, select_scores = 1_500_000, 8_000_000
+
+    def _selects(self, nq: int, plain: bool) -> bool:
+        """Whether the scan writes the scores and their parts' maxima, and ``top_hits`` selects from them."""
+        if not (self.threshold_search and self.frag and ops.scan_scores_ok(nq, (max(self.n, 4) + 3) // 4 * 4, self.dim)):
+            return False
+        return (not plain or self.n < self.threshold_min_rows
+                or self.n <= self.select_rows and nq * self.n <= self.select_scores)
+
+    def _selected_search(self, queries, k: int, q_groups, allowed, doc_lt):
+        """Exact top-k in three launches and without a host read: unit queries, scores with the greatest of every 16 rows,
+        selection.  (The bound below which parts are not looked into is the k-th greatest of those maxima.)"""
+        q, qg, allow, n = self._query(queries, q_groups, allowed, doc_lt)
+        scores, parts = ops.scores_and_parts(q, self.vecs, n, self.row_group[:n], qg, allow)
+        if self.n >= self.threshold_min_rows and allow is None:
+            self.stats["threshold_searches"] += 1
+        return ops.top_hits(scores, parts, min(k, n, 1024), self.row_ids, self.row_docs)
 
     def _sample_rank(self, k: int) -> int:
         """Rank in the row sample whose score is taken as a search's threshold.  The sample holds Binomial(k, 1/stride)
@@ -342,7 +376,7 @@ class VectorIndex:
         It is exact whenever the list holds k rows (or the threshold cut nothing off), which the ranking kernel
         reports per query: one host read at the end, and the rare query that fails it takes ``_safe_search``."""
         q = ops.unit_rows(torch.as_tensor(queries).to(self.device, torch.float32), self.dtype)
-        qg = None if q_groups is None else torch.as_tensor(q_groups, dtype=torch.int32).to(self.device)
+        qg = None if q_groups is None else self._there(torch.as_tensor(q_groups, dtype=torch.int32))
         n4 = (self.n + 3) // 4 * 4
         ns = (self.n // self.sample_stride) // 4 * 4
         if ns < k:  # (``_safe_search`` needs k rows in the sample)

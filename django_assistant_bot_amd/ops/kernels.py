@@ -736,6 +736,17 @@ def score_candidates_shuffled(A, B_shuf, N, thr, cap, row_group=None, q_group=No
 def scores_shuffled(A, B_shuf, N, row_group, q_group=None):
     """fp32 scores [M, N] of A [M, K] against the first N rows of a ``shuffle_weights`` copy (R >= round_up(N, 128)), -inf
     where the groups drop a row: the scan of index_scan.hip where it takes the shape, else ``gemm_bt``'s."""
+    _expect_scores(A, B_shuf, N, row_group, q_group)
+    if not (native().index_scan_takes(*A.shape) and A.stride(-1) == 1 and A.stride(0) % 8 == 0 and row_group.data_ptr() % 16 == 0):
+        return gemm_bt(A, B_shuf, epilogue=EPI_SCORES, out_f32=True, row_group=row_group, q_group=q_group, shuffled=True, n=N)
+    M, K = A.shape
+    out = torch.empty((M, N), dtype=torch.float32, device=A.device)
+    native().index_scan_scores(ptr(A), A.stride(0), ptr(B_shuf), M, int(N), K, ptr(row_group), ptr(q_group), 0, ptr(out), 0, 0,
+                               stream(A))
+    return out
+
+
+def _expect_scores(A, B_shuf, N, row_group, q_group):
     M, K = A.shape
     expect(A.is_cuda and A.dtype == torch.bfloat16 and B_shuf.dtype == torch.bfloat16 and N > 0 and N % 4 == 0, "bf16, N % 4")
     expect(B_shuf.is_contiguous() and B_shuf.shape[1] == K and B_shuf.shape[0] % 16 == 0
@@ -745,11 +756,47 @@ def scores_shuffled(A, B_shuf, N, row_group, q_group=None):
     if q_group is not None:
         _i32(q_group)
         expect(q_group.numel() >= M, "q_group shorter than M")
-    if not (native().index_scan_takes(M, K) and A.stride(-1) == 1 and A.stride(0) % 8 == 0 and row_group.data_ptr() % 16 == 0):
-        return gemm_bt(A, B_shuf, epilogue=EPI_SCORES, out_f32=True, row_group=row_group, q_group=q_group, shuffled=True, n=N)
+
+
+def scan_scores_ok(M: int, N: int, K: int) -> bool:
+    """Shapes ``scores_and_parts`` serves: the scan's, and scores that one buffer can address."""
+    return bool(native().index_scan_takes(M, K)) and 4 * M * N <= 0xffffff00
+
+
+def scores_and_parts(A, B_shuf, N, row_group, q_group=None, allow=None):
+    """(fp32 scores [M, N] as ``scores_shuffled`` gives them, also -inf where the int32 bitmask ``allow`` [M, ceil(N / 32)]
+    has no bit; int32 [M, P] ordered bits of the greatest score of every 16 rows, P = round_up(ceil(N / 16), 4) with the
+    last ones unwritten): what ``top_hits`` selects from."""
+    _expect_scores(A, B_shuf, N, row_group, q_group)
+    M, K = A.shape
+    expect(scan_scores_ok(M, N, K) and A.stride(-1) == 1 and A.stride(0) % 8 == 0 and row_group.data_ptr() % 16 == 0,
+           "scores_and_parts: the scan's shapes, 16-B rows")
+    if allow is not None:
+        _i32(allow)
+        expect(allow.is_contiguous() and allow.shape == (M, (N + 31) // 32), "allow: int32 [M, ceil(N / 32)]")
     out = torch.empty((M, N), dtype=torch.float32, device=A.device)
-    native().index_scan_scores(ptr(A), A.stride(0), ptr(B_shuf), M, int(N), K, ptr(row_group), ptr(q_group), ptr(out), stream(A))
-    return out
+    parts = torch.empty((M, ((N + 15) // 16 + 3) // 4 * 4), dtype=torch.int32, device=A.device)
+    native().index_scan_scores(ptr(A), A.stride(0), ptr(B_shuf), M, int(N), K, ptr(row_group), ptr(q_group), ptr(allow), ptr(out),
+                               ptr(parts), parts.shape[1], stream(A))
+    return out, parts
+
+
+def top_hits(scores, parts, k: int, row_ids, row_docs):
+    """The k best of every row of ``scores_and_parts`` -> (scores fp32 [rows, k] descending, equal ones in row order, item
+    ids, document ids int64; -inf / -1 past the rows that pass the filters), in one launch."""
+    rows, n = scores.shape
+    expect(scores.is_cuda and scores.dtype == torch.float32 and scores.is_contiguous() and n % 4 == 0
+           and 1 <= k <= min(n, 1024), "top_hits: contiguous fp32 [rows, n], n % 4, k <= min(n, 1024)")
+    _i32(parts)
+    expect(parts.is_contiguous() and parts.shape[0] == rows and parts.shape[1] >= (n + 15) // 16 and parts.shape[1] % 4 == 0,
+           "top_hits: the parts of these scores")
+    expect(row_ids.dtype == torch.int64 and row_docs.dtype == torch.int64 and row_ids.is_contiguous()
+           and row_docs.is_contiguous() and min(row_ids.numel(), row_docs.numel()) >= n, "row ids / documents: int64 [>= n]")
+    vals = torch.empty((rows, k), dtype=torch.float32, device=scores.device)
+    ids, docs = (torch.empty((rows, k), dtype=torch.int64, device=scores.device) for _ in range(2))
+    native().top_hits(ptr(scores), rows, n, ptr(parts), parts.shape[1], int(k), ptr(row_ids), ptr(row_docs), ptr(vals),
+                      ptr(ids), ptr(docs), stream(scores))
+    return vals, ids, docs
 
 
 def shuffled_scan_ok(M: int, K: int) -> bool:

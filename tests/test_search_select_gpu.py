@@ -1,0 +1,121 @@
+"""Scores with their parts' maxima (index_scan.hip) and the selection from them (search.hip) against plain torch."""
+import numpy as np
+import pytest
+import torch
+
+from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.engine.vector_index import VectorIndex
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _key(x):
+    """Floats in the kernels' order (-0 below 0), as integers."""
+    bits = x.contiguous().view(torch.int32).long()
+    return torch.where(bits < 0, -(bits & 0x7FFFFFFF) - 1, bits)
+
+
+def _parts(s):
+    n = s.shape[1]
+    pad = torch.full((s.shape[0], -n % 16), float("-inf"), device=s.device)
+    u = _key(torch.cat([s, pad], 1).view(s.shape[0], -1, 16).max(-1)[0]) + (1 << 31)  # unsigned ordered bits
+    p = torch.randint(0, 1 << 30, (s.shape[0], -(-n // 64) * 4), device=s.device, dtype=torch.int32)  # (padding: anything)
+    p[:, : u.shape[1]] = torch.where(u >= 1 << 31, u - (1 << 32), u).to(torch.int32)
+    return p
+
+
+# rows around a wave's 16, a tile's 32, the ring's refill (256 workgroups x 32 rows) and several rounds of it; queries
+# around the 16 of a fragment and the groups' sizes
+@pytest.mark.parametrize("dim,queries", [(256, 1), (256, 65), (256, 256), (512, 17), (768, 1), (768, 64), (768, 129), (1024, 5),
+                                         (1024, 128)])
+@pytest.mark.parametrize("n", [4, 28, 36, 8192, 8228, 70_020])
+def test_scores_and_parts(n, dim, queries):
+    g = torch.Generator(device=DEV).manual_seed(n + dim)
+    q, v = (torch.nn.functional.normalize(torch.randn(m, dim, device=DEV, generator=g), dim=-1).to(torch.bfloat16)
+            for m in (queries, -(-n // 128) * 128))
+    group = (torch.arange(len(v), device=DEV) % 5 - 1).to(torch.int32)
+    qg = (torch.arange(queries, device=DEV) % 6 - 1).clamp(max=3).to(torch.int32)
+    words = (n + 31) // 32
+    allow = torch.randint(-2 ** 31, 2 ** 31, (queries, words), device=DEV, generator=g).to(torch.int32)
+    seen = (allow[:, torch.arange(n, device=DEV) // 32] >> (torch.arange(n, device=DEV) % 32)) & 1 == 1
+    exact = q.double() @ v[:n].double().t()
+    frag = ops.shuffle_weights(v)
+    for gq, mask in ((None, None), (qg, None), (None, allow), (qg, allow)):
+        s, p = ops.scores_and_parts(q, frag, n, group[:n].contiguous(), gq, mask)
+        live = (group[:n] >= 0).expand(queries, -1)
+        if gq is not None:
+            live = live & ((gq[:, None] < 0) | (group[None, :n] == gq[:, None]))
+        if mask is not None:
+            live = live & seen
+        assert torch.equal(torch.isinf(s), ~live)
+        # a sum of dim exact products in fp32, up to 2^-23 of the running sum (unit vectors: below 1) lost a step
+        assert ((s.double() - exact).abs().masked_fill(~live, 0) <= dim * 2.0 ** -23).all()
+        u = (n + 15) // 16
+        assert torch.equal(p[:, :u], _parts(s)[:, :u])
+
+
+@pytest.mark.parametrize("n", [4, 60, 1024, 8192, 8196, 20_004, 70_000, 1_100_000])
+@pytest.mark.parametrize("k", [1, 16, 250, 1024])
+def test_top_hits(n, k):
+    """Scores of any spread, equal ones (in row order where they are few enough to be ranked), rows that few or no scores
+    pass, infinities."""
+    k = min(k, n)
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    s = torch.randn(8, n, device=DEV, generator=g)
+    s[1] = torch.round(s[1] * 3)  # thousands of equal scores
+    s[2] = float("-inf")
+    s[3, torch.rand(n, device=DEV, generator=g) < 0.98] = float("-inf")
+    s[4, 40:] = float("-inf")
+    s[5] = torch.where(s[5] > 0, s[5] * 1e-30, s[5] * 1e30)
+    s[6, : n // 2: 2] = 0.0
+    s[6, 1: n // 2: 2] = -0.0
+    s[7, n // 3] = float("inf")
+    ids, docs = torch.randperm(n + 3, device=DEV, generator=g), torch.arange(n + 3, device=DEV) // 3
+    row_of = torch.empty_like(ids)
+    row_of[ids] = torch.arange(n + 3, device=DEV)
+    vals, got, gdocs = ops.top_hits(s, _parts(s), k, ids, docs)
+    for m in range(len(s)):
+        key = _key(s[m])
+        at = torch.argsort(-key, stable=True)[:k]
+        assert torch.equal(_key(vals[m]), key[at])
+        hit = torch.isfinite(vals[m])
+        assert torch.equal(got[m] >= 0, hit) and torch.equal(gdocs[m] >= 0, hit)
+        rows = row_of[got[m][hit]]
+        assert torch.equal(_key(s[m])[rows], _key(vals[m])[hit]) and rows.unique().numel() == rows.numel()
+        assert torch.equal(gdocs[m][hit], docs[rows])
+        if m not in (1, 6):
+            assert torch.equal(rows, at[hit])
+
+
+@pytest.mark.parametrize("n", [5, 8190, 20_003])
+@pytest.mark.parametrize("flt", ["none", "group", "allowed", "doc_lt", "all"])
+def test_search_by_selection_is_the_full_search(n, flt):
+    """The route of searches that select against the scores of ``gemm_bt`` and ``topk_rows``: removed rows, k above the
+    rows that are left, one query without a hit."""
+    rng = np.random.default_rng(n)
+    ids, docs = rng.permutation(n) + 7, np.arange(n) // 6
+    idx = VectorIndex(768, DEV, capacity=n)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    idx.add(ids, torch.randn(n, 768, device=DEV, generator=g), doc_ids=docs, groups=docs % 3)
+    idx.remove(ids[: n // 4])
+    q = torch.randn(6, 768, device=DEV, generator=g)
+    kw = {}
+    if flt in ("group", "all"):
+        kw["q_groups"] = [0, 1, -1, 2, 1, 9]
+    if flt in ("allowed", "all"):
+        kw["allowed"] = [rng.choice(ids, max(1, n // (2 + i)), replace=False) for i in range(5)] + [np.empty(0, np.int64)]
+    if flt in ("doc_lt", "all"):
+        kw["doc_lt"] = [0, 1, n // 8, n // 6, 10 ** 9, 3]
+    for k in (1, 250, 3000):
+        idx.threshold_search = False
+        ev, ei, ed = idx.search(q, k, **kw)
+        idx.threshold_search = True
+        assert idx._selects(6, not ("allowed" in kw or "doc_lt" in kw))
+        gv, gi, gd = idx.search(q, k, **kw)
+        assert gv.shape == ev.shape and torch.equal(torch.isinf(gv), torch.isinf(ev))
+        hit = ~torch.isinf(gv)
+        assert ((gv - ev)[hit].abs() <= 768 * 2.0 ** -22).all()  # two fp32 sums of 768 products of unit vectors
+        assert torch.equal(gi >= 0, hit) and torch.equal(gd >= 0, hit)
+        same = gi == ei  # (neighbours that close may change places)
+        assert torch.equal(gd[same], ed[same]) and same.float().mean() > 0.97
