@@ -18,8 +18,9 @@
 //     K-tile is fetched from HBM once and served to the group's other workgroups from their XCD's
 //     L2 (groups are formed from blocks that share blockIdx % 8; the slots that whole groups leave over on
 //     the XCDs are joined into further groups, whose weights come from HBM or MALL once for each of their two or
-//     three XCDs).  The iteration space tiles_n x (K / 64) is split evenly over the floor(256 / tiles_m) groups
-//     (stream-K in the N x K plane): every CU gets the same number of MFMAs whatever the tile count;
+//     three XCDs).  The iteration space tiles_n x (K / 64) is split evenly over the groups, floor(256 / tiles_m) or
+//     fewer (gemm_mid_groups; stream-K in the N x K plane): every working CU gets the same number of MFMAs whatever
+//     the tile count;
 //   * a tile whose K range spans several groups is combined in-launch by its OWNER, the group
 //     holding the tile's first K-steps: that segment ends the owner's range, so in time it finishes
 //     last.  The other segments store their fp32 partial (write-through sc1 stores, 1 KB per
@@ -34,6 +35,8 @@
 //     grid is at most one workgroup per CU).  Replaces a last-arriver combine (every segment stored
 //     and drained, then an atomic ticket) that cost 5-9 us per launch on the small projections
 //     (profiles/gemm_mid_r6.md).
+#include <cmath>
+
 #include "common.h"
 #include "launchers.h"
 
@@ -514,43 +517,61 @@ int gemm_mid_ok(int M, int N, int K, long lda) {
   return 1;
 }
 
-// Estimated us of a product on `groups` groups: its ends (4 for whole tiles, 8 where every tile is cut into equal parts,
-// 18 otherwise, 1.45 for a part its owner adds, 3.5 for the end of each further tile) and its K-steps (0.45 + 0.0016 a
-// workgroup each).
-struct MidTime {
-  double ends, steps;
-};
-static MidTime mid_time(int M, int N, int K, int groups) {
-  const int tm = (M + 127) / 128, tn = N / 256;
-  const double parts = (double)groups / tn;  // of a tile
-  double ends = tn % groups == 0   ? 4.
-                : groups % tn == 0 ? 8. + 1.45 * parts
-                                   : 18. + (groups > tn ? 1.45 * (parts - 1.) : 0.);
-  if (tn > groups) ends += 3.5 * (1. / parts - 1.);
-  return {ends, (double)tn * (K / 64) / groups * (0.45 + 0.0016 * (groups * tm))};
+// Estimated us of a product on `groups` groups.  Its K-steps take 0.7 each, from some 120 working workgroups on 0.5 +
+// 0.00165 a workgroup, or the weights' way from memory (4.5 TB/s), whichever is longer; its ends 5.6 for whole tiles, 8.1 and 1.56 a part where every tile is cut into
+// parts of as many K-steps, 10.5 and 1.56 a part otherwise, and 2.5 for each further tile of a group.  (Fitted to 1,480
+// launches of 1-32 row tiles, N 256-28,672, K 256-14,336: half of them within 5 %, nine of ten within 16 %.)
+static double mid_us(int M, int N, int K, int groups) {
+  const int tm = (M + 127) / 128, tn = N / 256, kt = K / 64;
+  const double iters = (double)tn * kt, q = iters / groups;
+  const double step = fmax(0.7, 0.5 + 0.00165 * (groups < iters ? groups : iters) * tm);
+  const double weights = (double)tn * 512 * K / 4.5e6;
+  double ends, steps = q * step;
+  if (tn % groups == 0) {
+    ends = 5.6;
+  } else if (groups % tn == 0 && kt % (groups / tn) == 0) {
+    ends = 8.1 + 1.56 * (groups / tn);
+  } else {
+    ends = 10.5 + 1.56 * (groups > tn ? ceil(kt / (q > 1. ? q : 1.)) : 1.);
+    steps = ceil(q) * step;
+  }
+  if (tn > groups) ends += 2.5 * ((double)tn / groups - 1.);
+  return ends + (steps > weights ? steps : weights);
 }
 
 // Groups of ceil(M / 128) workgroups: the whole ones of each XCD, and those joined from the slots left over where they
-// gain 6 % by the estimate.  More workgroups are no gain where the whole groups divide the tiles evenly.  us, whole
-// groups -> with the joined ones: gate_up of Llama-3-8B at M 1093 272 -> 238, down 138 -> 128, o 47.7 -> 45.7, down at M
-// 1300 175 -> 156, 2200 338 -> 242, qkv at M 2600 158 -> 120; but qkv at M 1093 (24 tiles, 24 groups) 53.9 -> 63.4, o at M
-// 1700 55.0 -> 60.7.
+// gain 3 % by the estimate (or no group has two K-steps).  More workgroups are no gain where the whole groups divide the
+// tiles evenly.  us, whole groups -> with the joined ones: gate_up of Llama-3-8B at M 1093 272 -> 238, down 138 -> 128, down
+// at M 1300 175 -> 156, 2200 338 -> 242, qkv at M 2600 158 -> 120; but qkv at M 1093 (24 tiles, 24 groups) 53.9 -> 63.4, o at
+// M 1700 55.0 -> 60.7.
+// Fewer groups an XCD where that gains 6 % by the estimate: every part of a tile costs its owner a partial tile of 128 KB,
+// and unequal parts an end of their own, so a short K is better cut into few equal parts while much of the chip idles (K
+// below 768 has too few K-steps to choose from).  us, all the groups that fit -> those taken: (130, 2048, 2048) 38.4 on 128
+// groups -> 20.0 on 32, (300, 2048, 2048) 35.3 -> 20.5, (130, 3072, 2048) 31.1 -> 20.3 on 48, (1000, 3072, 2048) 28.6 -> 24.4
+// on 24, (130, 2048, 8192) 45.0 -> 35.5 on 64, (384, 4096, 4096) 35.1 -> 30.1 on 64; over the projections of Llama-3-8B and
+// 1B as planned at M 130-5000 (224 shapes) 0.94-1.96 times as fast, 1.055 in the mean, the worst qkv of 1B at M 1500 31.6 ->
+// 33.6.
 int gemm_mid_groups(int M, int N, int K) {
   const int spx = cu_count() / 8, tm = (M + 127) / 128, tn = N / 256;
-  if (M <= 0 || tn <= 0 || tm > spx) return 0;
+  if (M <= 0 || tn <= 0 || K < 64 || tm > spx) return 0;
   const int whole = 8 * (spx / tm), all = whole + 8 * (spx % tm) / tm;
-  const MidTime a = mid_time(M, N, K, all), w = mid_time(M, N, K, whole);
-  return a.ends + a.steps < 0.94 * (w.ends + w.steps) ? all : whole;
+  int groups = mid_us(M, N, K, all) < 0.97 * mid_us(M, N, K, whole) || (long)tn * (K / 64) <= whole ? all : whole;
+  double least = 0.94 * mid_us(M, N, K, groups);
+  for (int g = 8; K >= 768 && g < whole; g += 8) {
+    const double us = mid_us(M, N, K, g);
+    if (us < least) {
+      least = us;
+      groups = g;
+    }
+  }
+  return groups;
 }
 
-// Estimated us of the launch, infinite where the kernel does not take M; with few rows the weights' way from memory
-// (4.5 TB/s) is longer than the K-steps.
+// Estimated us of the launch, infinite where the kernel does not take M.
 double gemm_mid_us(int M, int N, int K) {
   const int groups = gemm_mid_groups(M, N, K);
   if (!groups) return M <= 0 || N < 256 ? 0. : __builtin_huge_val();
-  const MidTime t = mid_time(M, N, K, groups);
-  const double weights = (double)(N / 256) * 512 * K / 4.5e6;
-  return t.ends + (t.steps > weights ? t.steps : weights);
+  return mid_us(M, N, K, groups);
 }
 
 // Workspace the launcher needs: partial slabs and behind them the counts of ended workgroups (bytes), and ready flags
@@ -602,8 +623,8 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.ended = (unsigned*)((char*)slabs + slabs_end());
   p.spin_limit = spin_limit;
   p.spx = grid / 8;
-  p.gpx = p.spx / p.tiles_m;
   p.gn = gemm_mid_groups(M, N, K);
+  p.gpx = min(p.spx / p.tiles_m, p.gn / 8);  // (with fewer groups the other slots' workgroups end at once)
   const int iters = p.tiles_n * p.kt;
   p.q = iters / p.gn;
   p.r = iters % p.gn;
