@@ -55,6 +55,7 @@ class LlamaModel(FragmentProjections):
     # rows of a vocab-parallel LM head shard are padded to a multiple of this (every stream_gemm
     # tile height and the fragment layout divide it); the pad rows are zero and never sampled
     VOCAB_PAD = 384
+    PREFILL_STREAM_MAX_M = 256
 
     def __init__(self, cfg: DecoderConfig, weights: dict, device, tp_group=None, tp_size: int = 1,
                  interleaved_mlp: bool = False, fragment_layout: bool = True, consume: bool = False,
@@ -241,10 +242,15 @@ class LlamaModel(FragmentProjections):
         # are summed by the consumers (RoPE/KV write, RMSNorm) instead of a separate reduction.  So
         # do short prefill steps (an interactive prompt, the tail of a batch): at T <= 128 the MFMA
         # tiles read every weight for a handful of rows (qkv / o / gate_up / down 54 / 54 / 65 /
-        # 183 us against 16-21 / 15-19 / 42-49 / 27-32 streamed, profiles/small_prefill_r6.md)
+        # 183 us against 16-21 / 15-19 / 42-49 / 27-32 streamed, profiles/small_prefill_r6.md), and up to 256 gemm_mid's
+        # short K is cut into parts whose sums meet in one workgroup (us on gemm_mid / streamed at T 200, Llama-3-8B qkv
+        # 31 / 27, o 30 / 18, down 54 / 46; 1B 20 / 12, 20 / 9, 36 / 19; gate_up stays there).  The slabs of the latter are fp32,
+        # as gemm_mid's partial tiles are.
         small_pf = (not meta.decode and not meta.n_decode and T <= self.PREFILL_STREAM_MAX_M and self.frag
                     and self.tp_size == 1)
         sk = (meta.decode and T <= self.STREAM_MAX_M or small_pf) and x.is_cuda
+        if sk and not meta.decode and T > 128:
+            sk = self.SLABS_F32
         if sk and meta.decode and T <= self.SMALL_FUSED_MAX_M and self.small_norm_fused and self.fold_norms and self.tp_size == 1:
             h = x  # the residual stream itself: no RMSNorm launches (``_layer_small``)
             for li, L in enumerate(self.layers):

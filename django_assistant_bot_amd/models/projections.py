@@ -124,6 +124,7 @@ class FragmentProjections:
     # slab32,slab16; profiles/decode_slab_r6.md).  TP keeps fp32: its fused all-reduce + norm sums
     # fp32 slabs.
     slab_bf16 = True
+    SLABS_F32 = 2  # ``dec``: streamed, with the slabs in 32 bits (longer prefill steps, whose partial sums other kernels keep in 32)
 
     def _proj(self, x, w, dec: bool, allow_slabs: bool = True, name: str = "", epilogue=ops.EPI_NONE):
         """One projection.  Decode-sized batches (``dec``) stream the fragment-layout weights
@@ -145,7 +146,7 @@ class FragmentProjections:
                 if epilogue != ops.EPI_NONE:
                     return ops.stream_gemm(x, w, epilogue=epilogue, nt=True, cfg=cfg, w_group=grp, out=out,
                                            glu_bias=glu_bias)
-                sd = torch.bfloat16 if (self.slab_bf16 and self.tp_size == 1) else torch.float32
+                sd = torch.bfloat16 if (self.slab_bf16 and self.tp_size == 1 and dec != self.SLABS_F32) else torch.float32
                 out = ops.stream_gemm(x, w, splits=s, cfg=cfg, nt=True, slab_dtype=sd, w_group=grp)
                 return ops.slab_reduce(out) if (s > 1 and not allow_slabs) else out
         return ops.gemm_bt(x, w, epilogue=epilogue, shuffled=self.frag, b_group=grp, out=out, glu_bias=glu_bias)
