@@ -593,6 +593,13 @@ PYBIND11_MODULE(_native, m) {
     check(dab::gemm_small(CVP(A), lda, CVP(B), ldb, VP(C), ldc, CVP(bias), CVP(residual), ldr, M, N, K, gelu, tile, ST(s)),
           "gemm_small");
   });
+  m.def("norm_stream_ok", [](int M, int N, int K, int SO, int bn) { return dab::norm_stream_ok(M, N, K, SO, bn) != 0; });
+  m.def("norm_stream", [](u slabs, int S, int slabs_f32, u residual, u gain, u residual_out, float eps, u W, u out, long ldo,
+                          int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn, u s) {
+    check(dab::norm_stream(CVP(slabs), S, slabs_f32, CVP(residual), CVP(gain), VP(residual_out), eps, CVP(W), VP(out), ldo, M,
+                           N, K, SO, out_f32, glu, w_group, bn, ST(s)),
+          "norm_stream");
+  });
   m.def("gemm_mid_groups", &dab::gemm_mid_groups);
   m.def("gemm_mid_us", &dab::gemm_mid_us);
   m.def("gemm256_wins", &dab::gemm256_wins);

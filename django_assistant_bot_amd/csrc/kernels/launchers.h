@@ -290,6 +290,11 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
 // gemm_mid.hip (M = 256..4096: mixed serving steps / single prompts; grouped stream-K over the N x K
 // plane, 128 x 256 tiles, in-launch last-arriver combine; B in the shuffle_weights layout;
 // epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
+// norm_stream.hip: RMSNorm(sum of slabs + residual) . W^T of up to 4 decode rows
+int norm_stream_ok(int M, int N, int K, int SO, int bn);
+int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, const void* gain, void* residual_out, float eps,
+                const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn,
+                hipStream_t s);
 int gemm_mid_groups(int M, int N, int K);
 double gemm_mid_us(int M, int N, int K);
 int gemm_mid_ok(int M, int N, int K, long lda);

@@ -56,6 +56,7 @@ class LlamaModel(FragmentProjections):
     # tile height and the fragment layout divide it); the pad rows are zero and never sampled
     VOCAB_PAD = 384
     PREFILL_STREAM_MAX_M = 256
+    NORM_STREAM_MAX_M = 4  # rows up to which the norms run inside the projections behind them (0: off)
 
     def __init__(self, cfg: DecoderConfig, weights: dict, device, tp_group=None, tp_size: int = 1,
                  interleaved_mlp: bool = False, fragment_layout: bool = True, consume: bool = False,
@@ -345,14 +346,19 @@ class LlamaModel(FragmentProjections):
         # like the separate bf16 add), so the RMSNorms read and write one tensor instead of two each;
         # x is None then: the residual stream already holds the layer input
         fuse = not sk and self.tp_size == 1 and (x if x is not None else residual).is_cuda
-        if x is None:
-            h, _ = ops.rmsnorm(residual, L.attn_norm, cfg.eps)
-        elif residual is None:
-            h, _ = ops.rmsnorm(x, L.attn_norm, cfg.eps)
-            residual = x
+        few = sk and self.tp_size == 1 and T <= self.NORM_STREAM_MAX_M
+        both = self._norm_proj(x, L.attn_norm, cfg.eps, residual, L.qkv_w, "qkv") if few else None
+        if both is not None:
+            qkv, residual = both
         else:
-            h, residual = self._norm(x, L.attn_norm, residual)
-        qkv = self._proj(h, L.qkv_w, sk, name="qkv")
+            if x is None:
+                h, _ = ops.rmsnorm(residual, L.attn_norm, cfg.eps)
+            elif residual is None:
+                h, _ = ops.rmsnorm(x, L.attn_norm, cfg.eps)
+                residual = x
+            else:
+                h, residual = self._norm(x, L.attn_norm, residual)
+            qkv = self._proj(h, L.qkv_w, sk, name="qkv")
         if (not meta.decode and not meta.n_decode and qkv.is_cuda and qkv.dtype == torch.bfloat16 and qkv.dim() == 2
                 and ops.kernels.flash_rope_ok(D, kv.block_size)):
             # prefill: the RoPE/KV-write kernel writes only K / V; the attention rotates Q on load
@@ -377,6 +383,9 @@ class LlamaModel(FragmentProjections):
     def _layer_tail(self, L, a, residual, sk, fuse, slabs_ok, T, D):
         """o projection, MLP norm, gate_up (+SwiGLU), down: -> (next layer input, residual stream)."""
         cfg = self.cfg
+        # SwiGLU in the GEMM epilogue (8-row [gate | up] groups) on the GPU
+        epi = ops.EPI_SWIGLU8 if (self.interleaved_mlp and a.is_cuda) else ops.EPI_NONE
+        both = None
         if fuse:
             residual = ops.gemm_bt(a.view(T, self.hq * D), L.o_w, residual=residual, shuffled=self.frag,
                                    b_group=self.proj_group.get("o", 1))
@@ -387,12 +396,16 @@ class LlamaModel(FragmentProjections):
             h, residual = self._norm(o, L.mlp_norm, residual)
         else:
             o = self._all_reduce(self._proj(a.view(T, self.hq * D), L.o_w, sk, slabs_ok, name="o"))
-            h, residual = ops.rmsnorm(o, L.mlp_norm, cfg.eps, residual=residual)
-        # SwiGLU in the GEMM epilogue (8-row [gate | up] groups) on the GPU
-        epi = ops.EPI_SWIGLU8 if (self.interleaved_mlp and h.is_cuda) else ops.EPI_NONE
-        act = self._proj(h, L.gate_up_w, sk, name="gate_up", epilogue=epi)
-        if h.is_cuda and epi == ops.EPI_NONE:
-            act = ops.silu_mul(act)
+            if sk and slabs_ok and T <= self.NORM_STREAM_MAX_M and epi != ops.EPI_NONE:
+                both = self._norm_proj(o, L.mlp_norm, cfg.eps, residual, L.gate_up_w, "gate_up", epi)
+            if both is None:
+                h, residual = ops.rmsnorm(o, L.mlp_norm, cfg.eps, residual=residual)
+        if both is not None:
+            act, residual = both
+        else:
+            act = self._proj(h, L.gate_up_w, sk, name="gate_up", epilogue=epi)
+            if h.is_cuda and epi == ops.EPI_NONE:
+                act = ops.silu_mul(act)
         if fuse:
             return None, ops.gemm_bt(act, L.down_w, residual=residual, shuffled=self.frag,
                                      b_group=self.proj_group.get("down", 1))

@@ -138,6 +138,21 @@ class FragmentProjections:
             return ops.linear(x, w)
         return self._stream_or_tile(x, w, dec, allow_slabs, name, epilogue, self.proj_group.get(name, 1))
 
+    def _norm_proj(self, x, gain, eps: float, residual, w, name: str, epilogue=ops.EPI_NONE):
+        """RMSNorm(x + residual) and the projection behind it in one launch for a few decode rows (``ops.norm_stream``, TP 1,
+        fragment layout) -> (product, slabs where a consumer sums them; new residual), or None where that is not taken: up to
+        4 rows, projections that split as ``stream_gemm`` does on 64 weight rows a workgroup, gated ones unsplit on 128 (us,
+        4 rows of gated (28672, 4096) / (16384, 2048): 41.8 / 16.3 on 128, 43.7 / 18.5 on 64).  ``residual`` None: the first layer's
+        input is the residual stream."""
+        M, K, N, grp = x.shape[-2], x.shape[-1], w.shape[0], self.proj_group.get(name, 1)
+        gated = epilogue != ops.EPI_NONE
+        bn, s = (128, 1) if gated else (64, self._stream_splits(N, K, 64))
+        if not self.frag or N % bn or not ops.norm_stream_ok(M, N, K, s, bn):
+            return None
+        sd = torch.bfloat16 if self.slab_bf16 else torch.float32
+        y, new = ops.norm_stream(x, gain, eps, residual, w, splits=s, bn=bn, epilogue=epilogue, slab_dtype=sd, w_group=grp)
+        return y, (x if residual is None else new)
+
     def _stream_or_tile(self, x, w, dec: bool, allow_slabs: bool, name: str, epilogue, grp: int, out=None, glu_bias=None):
         """``out`` / ``glu_bias``: of a gated epilogue (a view to write, fp32 [gate | up])."""
         if dec and self.frag:

@@ -918,6 +918,36 @@ def stream_gemm(x, w, splits=1, epilogue=EPI_NONE, residual=None, out=None, nt=F
     return out
 
 
+def norm_stream_ok(M: int, N: int, K: int, splits: int, bn: int) -> bool:
+    """Shapes ``norm_stream`` serves: up to 4 rows, K of 256..4096, slices of up to 32,768 elements."""
+    return bool(native().norm_stream_ok(M, N, K, splits, bn))
+
+
+def norm_stream(x, gain, eps, residual, w, splits=1, bn=64, epilogue=EPI_NONE, slab_dtype=torch.float32, w_group: int = 1):
+    """``stream_gemm(rmsnorm(x, gain, eps, residual)[0], w, ...)`` of a few decode rows in one launch (norm_stream.hip) ->
+    (product, new residual or None).  x: bf16 rows or split-K slabs [S, M, K]; w: a ``shuffle_weights`` copy; ``bn``: weight
+    rows a workgroup, 64 or 128."""
+    slabs = x.dim() == 3
+    S, (M, K), N = x.shape[0] if slabs else 1, x.shape[-2:], w.shape[0]
+    expect(x.is_cuda and x.is_contiguous() and x.dtype in ((torch.float32, torch.bfloat16) if slabs else (torch.bfloat16,)),
+           "norm_stream: contiguous bf16 rows or slabs")
+    expect_bf16_contig(gain, residual, w)
+    same_device(x, gain, residual, w)
+    expect(gain.numel() == K and w.shape[1] == K and norm_stream_ok(M, N, K, splits, bn), "norm_stream: shapes")
+    expect(residual is None or tuple(residual.shape) == (M, K), "residual shape mismatch")
+    expect(epilogue == EPI_NONE or (epilogue == EPI_SWIGLU8 and splits == 1), "norm_stream: slabs, rows or SwiGLU of 8-row groups")
+    expect(N % (16 * w_group) == 0 and slab_dtype in (torch.float32, torch.bfloat16), "whole groups; fp32 or bf16 slabs")
+    new = None if residual is None else torch.empty_like(residual)
+    if splits > 1:
+        out = torch.empty((splits, M, N), dtype=slab_dtype, device=x.device)
+    else:
+        out = torch.empty((M, N // 2 if epilogue else N), dtype=torch.bfloat16, device=x.device)
+    native().norm_stream(ptr(x), S, int(x.dtype == torch.float32), ptr(residual), ptr(gain), ptr(new), float(eps), ptr(w), ptr(out),
+                         out.shape[-1], M, N, K, splits, int(slab_dtype == torch.float32), int(epilogue != EPI_NONE), int(w_group),
+                         int(bn), stream(x))
+    return out, new
+
+
 def slab_reduce(slabs, residual=None, out=None):
     """fp32 / bf16 slabs [S, M, N] -> bf16 [M, N] (fp32 sum rounded to bf16, then + residual)."""
     if not slabs.is_cuda:
