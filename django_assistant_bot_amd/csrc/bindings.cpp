@@ -419,15 +419,20 @@ PYBIND11_MODULE(_native, m) {
                                      u cnt, int batch, int Hq, int Hkv, int D, int part_size, int max_parts,
                                      float scale, u s, u order, u w0, long w0_bytes, u w1, long w1_bytes,
                                      int w_blocks, int chunk, u sink, float out_scale, long o_stride, u slopes,
-                                     const std::tuple<u, int, int, long, long, int, int>& gate) {
+                                     const std::tuple<u, int, int, long, long, int, int>& gate,
+                                     const std::tuple<u, int, int, int, u, u, u>& rope) {
     dab::L3Warm warm{{(const char*)w0, (const char*)w1}, {w0_bytes, w1_bytes}, w_blocks};
     // gate = (projection, column, columns of the output it covers each)
     const dab::OutputGate og{{CVP(std::get<0>(gate)), std::get<1>(gate), std::get<2>(gate), std::get<3>(gate), std::get<4>(gate)},
                              std::get<5>(gate), std::get<6>(gate)};
+    // rope = (slabs, bf16, S, columns, positions, cos / sin table, slots)
+    const dab::TokenRope rp{CVP(std::get<0>(rope)), std::get<1>(rope), std::get<2>(rope), std::get<3>(rope),
+                            (long)batch * std::get<3>(rope), (const int*)std::get<4>(rope), (const float2*)std::get<5>(rope),
+                            (const int64_t*)std::get<6>(rope)};
     check(dab::paged_decode_attention(CVP(q), CVP(kc), CVP(vc), (const int*)bt, max_blocks, bs, (const int*)ctx, VP(out),
                                       (float*)po, (float*)pm, (float*)pl, (int*)cnt, batch, Hq, Hkv, D, part_size,
                                       max_parts, scale, ST(s), (const int*)order, &warm, chunk, (const float*)sink,
-                                      out_scale, o_stride, (const float*)slopes, &og),
+                                      out_scale, o_stride, (const float*)slopes, &og, &rp),
           "paged_decode_attention");
   }, py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("bt"), py::arg("max_blocks"), py::arg("bs"), py::arg("ctx"),
      py::arg("out"), py::arg("po"), py::arg("pm"), py::arg("pl"), py::arg("cnt"), py::arg("batch"), py::arg("Hq"),
@@ -435,7 +440,9 @@ PYBIND11_MODULE(_native, m) {
      py::arg("order") = 0, py::arg("w0") = 0, py::arg("w0_bytes") = 0, py::arg("w1") = 0, py::arg("w1_bytes") = 0,
      py::arg("w_blocks") = 0, py::arg("chunk") = 0, py::arg("sink") = 0, py::arg("out_scale") = 1.f,
      py::arg("o_stride") = 0, py::arg("slopes") = 0,
-     py::arg("gate") = std::make_tuple((u)0, 0, 1, 0L, 0L, 0, 1));
+     py::arg("gate") = std::make_tuple((u)0, 0, 1, 0L, 0L, 0, 1),
+     py::arg("rope") = std::make_tuple((u)0, 0, 0, 0, (u)0, (u)0, (u)0));
+  m.def("decode_rope_ok", [](int batch, int Hkv, int D, int part_size) { return dab::decode_rope_ok(batch, Hkv, D, part_size) != 0; });
   m.def("gemm_bt", [](u A, long lda, u B, long ldb, u C, long ldc, u bias, u residual, long ldr, int M, int N, int K,
                       int epilogue, int out_f32, u row_group, u q_group, u allow, int allow_words, u s, int b_rows,
                       int b_group) {

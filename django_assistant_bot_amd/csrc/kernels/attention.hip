@@ -1588,8 +1588,13 @@ struct DecodeParams {
   float out_scale;
   long o_stride_tok;
   OutputGate gate;  // EXT, optional (gate.y.p): the finished output times its sigmoid
+  TokenRope rope;   // ROPE: the step's own rows, before their rotation, instead of q
   L3Warm warm;  // optional: the next projections' weights, warmed into L3 by appended workgroups
 };
+
+// Small batches at D = 128: two LDS slots a wave (at batch 128 the one-slot kernel's two workgroups per CU are 2.8 % faster per
+// step: 7.44 vs 7.65 ms, profiles/low_load_latency.md), whose block ids one lane each holds
+static bool decode_two_slots(int batch, int Hkv, int part_size) { return batch * Hkv <= 64 && part_size <= 64 * 4 * 32; }
 
 constexpr int kCombine = 8;  // partial results requested together by the combine
 
@@ -1623,7 +1628,13 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 // one workgroup per CU, which small batches never fill anyway.
 //
 // EXT: slopes (may be null) and the output gate; the plain form is free of both.
-template <int D, bool KV_NT, bool DMA = false, int NSLOT = 1, bool EXT = false>
+//
+// ROPE (the slabs' type): q, and the new token's k and v, come straight from the split-K slabs of the qkv projection, as
+// rope_kv_kernel reads them and with its roundings.  Each wave rotates its group's q rows in registers, under the first
+// copies from the cache; the wave that holds the new token's sub-tile rotates its k, writes both rows to the cache and
+// into its LDS image behind the copy (which read what was there before).  The slabs' loads go out ahead of the first copies
+// and are summed under them.  One launch less a layer against the sums in every workgroup: see decode_rope_ok.
+template <int D, bool KV_NT, bool DMA = false, int NSLOT = 1, bool EXT = false, typename ROPE = void>
 __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(DecodeParams p, int total_items) {
   static_assert(NSLOT == 1 || (NSLOT == 2 && DMA), "two slots: DMA staging only");
   // appended workgroups (small batches leave most CUs idle during this latency-bound launch): warm
@@ -1687,7 +1698,102 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     const int k_end = min(ctx, k_begin + part_size);
 
     bf16x8 qf[NKK];
-    {
+    constexpr bool FUSED = !std::is_same_v<ROPE, void>;
+    // FUSED: the wave that holds the new token (the context's last key), and its rotated k / copied v pieces: lane l of the
+    // first D / 16 holds dims 8 l .. + 7 and those D / 2 on of k, the next D / 16 lanes of v
+    const int k_new = ctx - 1, new_sub = (k_new - k_begin) / KT;
+    const bool own_new = FUSED && k_end == ctx && w == (new_sub & 3);
+    const int new_i0 = 8 * (lane % (D / 16));
+    const bool new_k = (lane / (D / 16) & 1) == 0;
+    u32x4 new_lo, new_hi;
+    bool patch = false;
+    // ... in two steps around the first copies from the cache, so that all of them share one round trip: the loads
+    // (positions, slots, the first slabs; then the cosines, behind the position), and the sums and rotations
+    using RT = std::conditional_t<FUSED, ROPE, float>;
+    constexpr int HK = FUSED ? NKK / 2 : 1, HELD = !FUSED ? 1 : sizeof(RT) == 4 && NSLOT == 1 ? 2 : 4;  // chunk pairs of a q row, slabs held between the steps
+    SlabVec8<RT> qa[HK][HELD], qb[HK][HELD], na[HELD], nb[HELD];
+    float2 q_cs[HK][8], n_cs[8];
+    int64_t new_slot = -1;
+    int new_blk = 0;
+    const RT* const slabs = (const RT*)p.rope.slabs;
+    const size_t q_at = (size_t)b * p.rope.ld + (size_t)(hk * G + min(li, G - 1)) * D + 8 * g;
+    const size_t n_at = (size_t)b * p.rope.ld + (size_t)(p.Hq + (new_k ? 0 : p.Hkv) + hk) * D + new_i0;
+    auto fused_load = [&]() __attribute__((always_inline)) {
+      if constexpr (FUSED) {
+        const int pos = p.rope.positions[b];
+        if (own_new) {  // wave-uniform
+          new_slot = p.rope.slots[b];
+          new_blk = p.block_tables[(size_t)b * p.max_blocks + k_new / p.block_size];
+        }
+#pragma unroll
+        for (int u = 0; u < HELD; ++u) {
+          const RT* src = slabs + (size_t)min(u, p.rope.S - 1) * p.rope.slab_stride;
+#pragma unroll
+          for (int kk = 0; kk < HK; ++kk) {
+            qa[kk][u].load(src + q_at + 32 * kk);
+            qb[kk][u].load(src + q_at + 32 * kk + D / 2);
+          }
+          if (own_new) {
+            na[u].load(src + n_at);
+            nb[u].load(src + n_at + D / 2);
+          }
+        }
+#pragma unroll
+        for (int kk = 0; kk < HK; ++kk) rope_cs(p.rope.cos_sin, pos, D / 2, 32 * kk + 8 * g, q_cs[kk]);
+        if (own_new) rope_cs(p.rope.cos_sin, pos, D / 2, new_i0, n_cs);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto fused_finish = [&]() __attribute__((always_inline)) {
+      if constexpr (FUSED) {
+        __builtin_amdgcn_sched_barrier(0);
+        auto sum = [&](const SlabVec8<RT>(&x)[HELD], size_t at, float(&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = 0.f;
+#pragma unroll
+          for (int u = 0; u < HELD; ++u)
+            if (u < p.rope.S) x[u].add_to(v);
+          for (int u = HELD; u < p.rope.S; ++u) {
+            SlabVec8<RT> y;
+            y.load(slabs + (size_t)u * p.rope.slab_stride + at);
+            y.add_to(v);
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = bf2f(f2bf(v[j]));
+        };
+        float x1[8], x2[8];
+#pragma unroll
+        for (int kk = 0; kk < HK; ++kk) {
+          sum(qa[kk], q_at + 32 * kk, x1);
+          sum(qb[kk], q_at + 32 * kk + D / 2, x2);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) rope_rot(x1[j], x2[j], q_cs[kk][j]);
+          qf[kk] = __builtin_bit_cast(bf16x8, pack8(x1));
+          qf[kk + HK] = __builtin_bit_cast(bf16x8, pack8(x2));
+        }
+        if (own_new) {
+          sum(na, n_at, x1);
+          sum(nb, n_at + D / 2, x2);
+          if (new_k)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) rope_rot(x1[j], x2[j], n_cs[j]);
+          new_lo = pack8(x1);
+          new_hi = pack8(x2);
+          if (new_slot >= 0) {
+            // the row the cache's reader finds at the context's end, where the slot is that row (it is, but for padded rows)
+            patch = new_slot == (int64_t)new_blk * p.block_size + k_new % p.block_size;
+            const int64_t sb = new_slot / p.block_size;
+            bf16* dst = const_cast<bf16*>(new_k ? p.k_cache : p.v_cache) +
+                        (((size_t)sb * p.Hkv + hk) * p.block_size + (new_slot - sb * p.block_size)) * D + new_i0;
+            if (lane < D / 8) {
+              *reinterpret_cast<u32x4*>(dst) = new_lo;
+              *reinterpret_cast<u32x4*>(dst + D / 2) = new_hi;
+            }
+          }
+        }
+      }
+    };
+    if constexpr (!FUSED) {
       const bool qv = li < G;
       const bf16* qrow = p.q + ((size_t)b * p.Hq + hk * G + (qv ? li : 0)) * D;
 #pragma unroll
@@ -1727,6 +1833,16 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
       }
     };
 
+    // FUSED: the new token's rows over the LDS image of its sub-tile (whose copy has landed)
+    auto put_new = [&](int k0) {
+      if (FUSED && patch && k0 == k_begin + new_sub * KT && lane < D / 8) {
+        char* img = lane < D / 16 ? ks : vs;
+        const int ch = lane % (D / 16);
+        *reinterpret_cast<u32x4*>(img + swz<D>(k_new - k0, ch)) = new_lo;
+        *reinterpret_cast<u32x4*>(img + swz<D>(k_new - k0, ch + D / 16)) = new_hi;
+      }
+    };
+
     f32x4 o[NTD];
 #pragma unroll
     for (int t = 0; t < NTD; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1734,6 +1850,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     const float slope = EXT && p.slopes ? p.slopes[hk * G + min(li, G - 1)] * 1.4426950408889634f : 0.f;
 
     auto compute = [&](const int k0) {
+      put_new(k0);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes landed
       __builtin_amdgcn_wave_barrier();
       f32x4 s[2];
@@ -1829,7 +1946,11 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
           vs = ks + SUB_BYTES;
           dma(kw + i * 4 * KT, __builtin_amdgcn_readlane(myblk, i));
         };
-        if (n_sub > 0) issue(0);
+        if (n_sub > 0) {
+          fused_load();
+          issue(0);
+          fused_finish();
+        }
         for (int i = 0; i < n_sub; ++i) {
           if (i + 1 < n_sub) {
             issue(i + 1);  // into the slot sub-tile i - 1 was read from (its MFMAs consumed it)
@@ -1842,9 +1963,12 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
           compute(kw + i * 4 * KT);
         }
       } else {
-      int blk = __builtin_amdgcn_readfirstlane(blk_at(kw));
+      int blk = blk_at(kw);
+      if (kw < k_end) fused_load();
+      blk = __builtin_amdgcn_readfirstlane(blk);
       for (int k0 = kw; k0 < k_end; k0 += 4 * KT) {
         dma(k0, blk);
+        if (k0 == kw) fused_finish();
         blk = blk_at(k0 + 4 * KT);  // in flight under this sub-tile's copy and math
         asm volatile("s_waitcnt vmcnt(1)" ::: "memory");  // this sub-tile's 16 pieces landed
         compute(k0);
@@ -1853,8 +1977,10 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
     } else {
+      if (kw < k_end) fused_load();
       load_sub(kA, vA, kw);
       load_sub(kB, vB, kw + 4 * KT);
+      if (kw < k_end) fused_finish();
       for (int k0 = kw; k0 < k_end; k0 += 8 * KT) {
         stage(kA, vA);
         load_sub(kA, vA, k0 + 8 * KT);
@@ -2220,6 +2346,15 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
   return hipGetLastError();
 }
 
+// Whether a decode step rotates and writes its rows inside the attention: while the items find a CU or two at once (every
+// further round of them pays the sums again).  us a step, rope_kv_write apart -> inside: Llama-3-8B (D 128), 1 sequence 3087
+// -> 3064, 4: 3223 -> 3169, 8: 3424 -> 3356 (above 64 items the one-slot form has no registers left for it); Llama-3.2-1B (D
+// 64, 8 key heads), 6: 944 -> 930, 24: 1054 -> 1032, 48: 1106 -> 1099, 100: 1549 -> 1724.
+int decode_rope_ok(int batch, int Hkv, int D, int part_size) {
+  if (batch <= 0 || Hkv <= 0) return 0;
+  return D == 128 ? decode_two_slots(batch, Hkv, part_size) : D == 64 && batch * Hkv <= 384;
+}
+
 // The workgroups of a launch are dispatched in blockIdx order as CU slots free up; at RAG batch sizes
 // every CU runs about two (sequence, kv head) items one after the other, so with sequences of mixed
 // length the launch ends when the unluckiest slot has run two long ones.  ``order`` (optional, a
@@ -2231,11 +2366,15 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
                            float* part_m, float* part_l, int* counters, int batch, int Hq, int Hkv, int D,
                            int part_size, int max_parts, float scale, hipStream_t s, const int* order,
                            const L3Warm* warm, int chunk, const float* sink, float out_scale, long o_stride_tok,
-                           const float* slopes, const OutputGate* gate) {
+                           const float* slopes, const OutputGate* gate, const TokenRope* rope) {
   if (batch <= 0) return 0;
   if (Hq % Hkv || Hq / Hkv > 16 || part_size % 128 || max_parts < 1 || block_size % 32) return hipErrorInvalidValue;
   if (max_parts > 1 && !counters) return hipErrorInvalidValue;
-  if (!q) return hipErrorInvalidValue;
+  const bool fused = rope && rope->slabs;
+  if (!q && !fused) return hipErrorInvalidValue;
+  if (fused && (slopes || (gate && gate->y.p) || chunk || rope->S < 1 || rope->ld % 8 || rope->slab_stride % 8 || !rope->positions ||
+                !rope->cos_sin || !rope->slots || !decode_rope_ok(batch, Hkv, D, part_size)))
+    return hipErrorInvalidValue;
   DecodeParams prm;
   prm.q = (const bf16*)q;
   prm.k_cache = (const bf16*)k_cache;
@@ -2260,6 +2399,7 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   prm.slopes = slopes;
   prm.gate = gate ? *gate : OutputGate{};
   if (prm.gate.y.p && (prm.gate.per < 1 || prm.gate.y.S < 1)) return hipErrorInvalidValue;
+  prm.rope = fused ? *rope : TokenRope{};
   prm.out_scale = out_scale;
   prm.o_stride_tok = o_stride_tok ? o_stride_tok : (long)Hq * D;
   prm.warm = warm ? *warm : L3Warm{{nullptr, nullptr}, {0, 0}, 0};
@@ -2274,17 +2414,23 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   // profiles/decode_round2.md).  D = 128 stages K / V by LDS-DMA (100.7 vs 102.6 us isolated, same
   // section); D = 64 (small test models) keeps the register path.
   if (D == 128) {
-    // small batches: two LDS slots per wave (at batch 128 the one-slot kernel's two workgroups per CU
-    // are 2.8 % faster per step: 7.44 vs 7.65 ms, profiles/low_load_latency.md)
-    const bool two = batch * Hkv <= 64 && part_size <= 64 * 4 * 32;
-    if (two && ext)
+    const bool two = decode_two_slots(batch, Hkv, part_size);
+    if (fused && rope->bf16_slabs)
+      hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2, false, bf16>), grid, dim3(256), 0, s, prm, total_items);
+    else if (fused)
+      hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2, false, float>), grid, dim3(256), 0, s, prm, total_items);
+    else if (two && ext)
       hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2, true>), grid, dim3(256), 0, s, prm, total_items);
     else if (two) hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2>), grid, dim3(256), 0, s, prm, total_items);
     else if (ext)
       hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 1, true>), grid, dim3(256), 0, s, prm, total_items);
     else hipLaunchKernelGGL((paged_decode_kernel<128, true, true>), grid, dim3(256), 0, s, prm, total_items);
   } else if (D == 64) {
-    if (ext)
+    if (fused && rope->bf16_slabs)
+      hipLaunchKernelGGL((paged_decode_kernel<64, true, false, 1, false, bf16>), grid, dim3(256), 0, s, prm, total_items);
+    else if (fused)
+      hipLaunchKernelGGL((paged_decode_kernel<64, true, false, 1, false, float>), grid, dim3(256), 0, s, prm, total_items);
+    else if (ext)
       hipLaunchKernelGGL((paged_decode_kernel<64, true, false, 1, true>), grid, dim3(256), 0, s, prm, total_items);
     else hipLaunchKernelGGL((paged_decode_kernel<64, true>), grid, dim3(256), 0, s, prm, total_items);
   } else {

@@ -70,13 +70,24 @@ bool flash_packed64_wins(long units, int max_len);
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
                    long o_tok, long o_head, const int* cu, int batch, int max_len, int Hq, int Hkv, float scale, hipStream_t s);
 int decode_partition_of(int part_size, int longest, int items, int max_parts);
+// The rows of a decode step before their rotation: split-K slabs [S][batch][ld] of the qkv projection (fp32 or bf16, summed in
+// order and rounded like a GEMM's output), with the token's position and cache slot (< 0: not written)
+struct TokenRope {
+  const void* slabs;
+  int bf16_slabs, S, ld;
+  long slab_stride;
+  const int* positions;
+  const float2* cos_sin;  // [max_pos, D / 2]
+  const int64_t* slots;
+};
+int decode_rope_ok(int batch, int Hkv, int D, int part_size);
 int paged_decode_attention(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                            int max_blocks, int block_size, const int* ctx_lens, void* out, float* part_o,
                            float* part_m, float* part_l, int* counters, int batch, int Hq, int Hkv, int D,
                            int part_size, int max_parts, float scale, hipStream_t s,
                            const int* order = nullptr, const L3Warm* warm = nullptr, int chunk = 0,
                            const float* sink = nullptr, float out_scale = 1.f, long o_stride_tok = 0,
-                           const float* slopes = nullptr, const OutputGate* gate = nullptr);
+                           const float* slopes = nullptr, const OutputGate* gate = nullptr, const TokenRope* rope = nullptr);
 
 // attention_any.hip (any head width, bf16 or fp32, paged)
 int any_attention(const void* q, const void* kc, const void* vc, int f32, const int* bt, int max_blocks, int bs,

@@ -369,6 +369,11 @@ class LlamaModel(FragmentProjections):
             a = ops.flash_attention_paged(q, kv.k[li], kv.v[li], meta.block_tables, meta.cu_q, meta.ctx_lens,
                                           meta.max_q, causal=True, rope=(meta.positions, self.cos_sin))
             return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D)
+        if meta.decode and qkv.is_cuda and qkv.dtype in (torch.float32, torch.bfloat16) and self.rope_in_decode(T, meta):
+            a = ops.paged_decode_rope(qkv, meta.positions, self.cos_sin, kv.k[li], kv.v[li], meta.slots, self.hq,
+                                      meta.block_tables, meta.ctx_lens, meta.part_size, meta.workspace, order=meta.order,
+                                      warm=self._warm(L, T, qkv))
+            return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D)
         q = ops.rope_kv_write(qkv, meta.positions, self.cos_sin, kv.k[li], kv.v[li], meta.slots, self.hq, self.hkv, D)
         if meta.decode:
             a = ops.paged_decode(q, kv.k[li], kv.v[li], meta.block_tables, meta.ctx_lens, meta.part_size,
@@ -413,6 +418,10 @@ class LlamaModel(FragmentProjections):
             return self._tp_partial(self._proj(act, L.down_w, sk, True, name="down"), cfg.hidden), residual
         x = self._all_reduce(self._proj(act, L.down_w, sk, slabs_ok, name="down"))
         return x, residual
+
+    def rope_in_decode(self, T: int, meta: AttnMeta) -> bool:
+        """Whether a decode step rotates its rows and writes them to the cache inside the attention."""
+        return meta.workspace is not None and ops.decode_rope_ok(T, self.hkv, self.cfg.head_dim, meta.part_size)
 
     @staticmethod
     def _mixed_attention(q, kv: KVCache, li: int, meta: AttnMeta) -> torch.Tensor:

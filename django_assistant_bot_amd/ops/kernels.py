@@ -337,8 +337,32 @@ class DecodeWorkspace:
         self.cnt = torch.zeros((max_batch * Hq,), dtype=torch.int32, device=device)
 
 
+def decode_rope_ok(batch: int, Hkv: int, D: int, part_size: int) -> bool:
+    """Decode steps whose rotary embedding and cache write ``paged_decode_rope`` does inside the attention."""
+    return bool(native().decode_rope_ok(batch, Hkv, D, part_size))
+
+
+def paged_decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slots, Hq, block_tables, ctx_lens, part_size=512,
+                      workspace: DecodeWorkspace | None = None, order=None, warm=None):
+    """``rope_kv_write`` and ``paged_decode`` of a decode step in one launch (``decode_rope_ok``): ``qkv`` bf16 rows or split-K
+    slabs, the step's token the last of each context."""
+    slabs = qkv.dim() == 3
+    Hkv, D = k_cache.shape[1], k_cache.shape[3]
+    T, width = qkv.shape[-2:]
+    expect(qkv.is_cuda and qkv.is_contiguous() and qkv.dtype in ((torch.float32, torch.bfloat16) if slabs else (torch.bfloat16,)),
+           "paged_decode_rope: contiguous bf16 rows or slabs")
+    expect(width == (Hq + 2 * Hkv) * D and positions.numel() == T and slots.numel() == T, "qkv width, positions and slots")
+    _i32(positions)
+    expect(slots.dtype == torch.int64 and slots.is_contiguous(), "slots must be contiguous int64")
+    expect(cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[1] == D // 2, "cos_sin: fp32 [pos, D / 2, 2]")
+    expect(workspace is not None and decode_rope_ok(T, Hkv, D, part_size), "paged_decode_rope: a workspace, batch, heads, partition")
+    out = torch.empty((T, Hq, D), dtype=torch.bfloat16, device=qkv.device)
+    rope = (ptr(qkv), int(qkv.dtype == torch.bfloat16), qkv.shape[0] if slabs else 1, width, ptr(positions), ptr(cos_sin), ptr(slots))
+    return paged_decode(out, k_cache, v_cache, block_tables, ctx_lens, part_size, workspace, out=out, order=order, warm=warm, rope=rope)
+
+
 def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, part_size=512, workspace: DecodeWorkspace | None = None,
-                 scale=None, out=None, order=None, warm=None):
+                 scale=None, out=None, order=None, warm=None, rope=None):
     """q [B, Hq, D] (one new token per sequence) over the paged caches.  ``order`` (int32 [B], a
     permutation of the batch) is the order the (sequence, kv head) items are dispatched in: longest
     context first balances the two rounds of workgroups every CU runs at RAG batch sizes.  Any
@@ -381,6 +405,8 @@ def paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, part_size=512, wor
                    "warm range must be a 16-B multiple inside a contiguous device tensor")
             wargs[f"w{i}"], wargs[f"w{i}_bytes"] = ptr(t), int(nb)
         wargs["w_blocks"] = int(blocks)
+    if rope is not None:  # (``paged_decode_rope``: q is only its shape)
+        wargs["rope"] = rope
     native().paged_decode_attention(ptr(q), ptr(k_cache), ptr(v_cache), ptr(block_tables), block_tables.shape[1], bs,
                                     ptr(ctx_lens), ptr(out), ptr(ws_o), ptr(ws_m), ptr(ws_l), ptr(ws_c), B, Hq, Hkv,
                                     D, int(part_size), int(max_parts), float(scale), stream(q), ptr(order), **wargs)
