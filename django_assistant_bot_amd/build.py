@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import subprocess
 import sys
@@ -85,7 +86,8 @@ def build(force: bool = False, jobs: int | None = None, debug: bool = False, ver
     hipcc = _hipcc()
     opt = ["-O0", "-g"] if debug else ["-O3"]
     common = ["-std=c++17", "-fPIC", *opt, f"-I{CSRC}", "-Wno-unused-result", "-Wno-unused-command-line-argument"]
-    py_inc = [f"-I{sysconfig.get_paths()['include']}", f"-I{pybind11.get_include()}"]
+    torch_inc = Path(importlib.util.find_spec("torch").origin).parent / "include"  # ATen/dlpack.h: plain C structs, nothing to link
+    py_inc = [f"-I{sysconfig.get_paths()['include']}", f"-I{pybind11.get_include()}", f"-isystem{torch_inc}"]
     deps = _headers()
     jobs_list: list[tuple[list[str], Path]] = []
     objs: list[Path] = []

@@ -1,6 +1,7 @@
 // pybind11 module `_native`: kernel launchers (raw device pointers + stream handles passed as
 // integers from the python ops layer, which owns shape/dtype validation) and the native host
 // runtime (tokenizer, paged-KV block manager, retrieval post-processing).
+#include <ATen/dlpack.h>
 #include <hip/hip_runtime.h>
 #include <pybind11/numpy.h>
 #include <pybind11/pybind11.h>
@@ -27,6 +28,49 @@ using u = uintptr_t;
 static void check(int err, const char* name) {
   if (err) throw std::runtime_error(std::string("dab kernel '") + name + "' failed: " + hipGetErrorString((hipError_t)err));
 }
+
+#if DLPACK_MAJOR_VERSION == 1 && DLPACK_MINOR_VERSION >= 3
+// Addresses of the tensors of `rows` (tuples of as many tensors as there are `shapes`), through torch's DLPack exchange
+// table (`api`): each contiguous, bf16, of the shape at its place and on the device of `like`.  None where one is not or
+// the table does not describe it: the caller then looks itself.  0.1 us a tensor; four attributes asked for from Python are 0.45-0.8.
+static py::object operand_ptrs(py::capsule api, py::handle tensor_type, py::handle like, py::sequence rows,
+                               const std::vector<std::vector<int64_t>>& shapes) {
+  auto* table = static_cast<DLPackExchangeAPI*>(PyCapsule_GetPointer(api.ptr(), "dlpack_exchange_api"));
+  if (!table) throw py::error_already_set();
+  auto* type = reinterpret_cast<PyTypeObject*>(tensor_type.ptr());
+  auto view = [&](py::handle t, DLTensor& out) {
+    if (!PyObject_TypeCheck(t.ptr(), type)) return false;
+    if (!table->dltensor_from_py_object_no_sync(t.ptr(), &out)) return true;
+    PyErr_Clear();
+    return false;
+  };
+  DLTensor first, d;
+  if (table->header.version.major != DLPACK_MAJOR_VERSION || !table->dltensor_from_py_object_no_sync || !view(like, first))
+    return py::none();
+  const DLDevice dev = first.device;
+  std::vector<u> out;
+  out.reserve(rows.size() * shapes.size());
+  for (py::handle row : rows) {
+    if (!PyTuple_Check(row.ptr()) || (size_t)PyTuple_GET_SIZE(row.ptr()) != shapes.size()) return py::none();
+    for (size_t i = 0; i < shapes.size(); ++i) {
+      const std::vector<int64_t>& shape = shapes[i];
+      if (!view(PyTuple_GET_ITEM(row.ptr(), (Py_ssize_t)i), d) || !d.data || d.device.device_type != dev.device_type ||
+          d.device.device_id != dev.device_id || d.dtype.code != kDLBfloat || d.dtype.bits != 16 || d.dtype.lanes != 1 ||
+          d.ndim != (int)shape.size())
+        return py::none();
+      int64_t run = 1;
+      for (int k = d.ndim - 1; k >= 0; --k) {
+        if (d.shape[k] != shape[k] || (d.strides && d.shape[k] != 1 && d.strides[k] != run)) return py::none();
+        run *= d.shape[k];
+      }
+      out.push_back(reinterpret_cast<u>(d.data) + d.byte_offset);
+    }
+  }
+  return py::cast(out);
+}
+#else
+static py::object operand_ptrs(py::handle, py::handle, py::handle, py::handle, py::handle) { return py::none(); }
+#endif
 
 PYBIND11_MODULE(_native, m) {
   m.doc() = "MI355X (gfx950) kernels and native runtime of django_assistant_bot_amd";
@@ -594,6 +638,7 @@ PYBIND11_MODULE(_native, m) {
                                l.data(), VP(x), VP(y), VP(att), VP(qkv), VP(ffn), ST(s)),
           "encoder_forward");
   });
+  m.def("operand_ptrs", &operand_ptrs);
   m.def("gemm_small_ok", &dab::gemm_small_ok);
   m.def("gemm_small", [](u A, long lda, u B, long ldb, u C, long ldc, u bias, u residual, long ldr, int M, int N, int K,
                          int gelu, int tile, u s) {

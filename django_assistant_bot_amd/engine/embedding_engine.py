@@ -54,13 +54,15 @@ class EmbeddingEngine:
         """Pre-tokenised (flat ids, offsets) -> [n, H] on the engine device, caller order."""
         norm = self.normalize if normalize is None else normalize
         n = len(offsets) - 1
-        lens = np.diff(offsets)
+        offsets = np.asarray(offsets)
+        lens = offsets[1:] - offsets[:-1]
         order = np.argsort(-lens, kind="stable")
         out = torch.empty((n, self.cfg.hidden), dtype=out_dtype, device=self.device)
         pin = self.device.type == "cuda"
         # batch boundaries over the length-sorted order: greedy token budget (vectorised)
         sorted_lens = lens[order]
-        csum = np.concatenate([[0], np.cumsum(sorted_lens)])
+        csum = np.zeros(n + 1, dtype=np.int64)
+        np.cumsum(sorted_lens, dtype=np.int64, out=csum[1:])
         i = 0
         while i < n:
             # last j with csum[j] - csum[i] <= budget (at least one text per batch)
@@ -68,13 +70,13 @@ class EmbeddingEngine:
             j = max(j, i + 1)
             idx = order[i:j]
             seg_lens = sorted_lens[i:j]
-            total = int(seg_lens.sum())
+            total = int(csum[j] - csum[i])
             # one pinned buffer and one copy: ids | positions | output rows | sequence starts
             m = j - i
             host = torch.empty(2 * total + 2 * m + 1, dtype=torch.int32, pin_memory=pin)
-            h_ids, h_pos, h_rows, cu = np.split(host.numpy(), [total, 2 * total, 2 * total + m])
-            cu[0] = 0
-            np.cumsum(seg_lens, out=cu[1:])
+            buf = host.numpy()
+            h_ids, h_pos, h_rows, cu = buf[:total], buf[total:2 * total], buf[2 * total:2 * total + m], buf[2 * total + m:]
+            np.subtract(csum[i:j + 1], csum[i], out=cu, casting="unsafe")
             h_rows[:] = idx
             # gather index of every token of the batch and its position, without per-text slices
             np.subtract(np.arange(total, dtype=np.int32), np.repeat(cu[:-1], seg_lens), out=h_pos)

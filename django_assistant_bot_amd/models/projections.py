@@ -64,24 +64,23 @@ class FragmentProjections:
         return K // S2 <= (3072 if M > 32 else 6144 if M > 16 else K)
 
     def _stream_cfg(self, name: str, M: int, N: int, K: int = 0) -> int:
-        nat = ops.native()
         if M > 128 and name == "gate_up":
             # decode batches of 129..256: gate_up (+SwiGLU8) on the mid-M GEMM, 67-72 us against 90-96
             # on the M <= 256 streaming tiles (profiles/small_prefill_r6.md); qkv / o / down stream
             return -1
         if M > 128:
             cfg = self.STREAM_CFG_M256
-        elif M <= 16 and N % nat.stream_gemm_bn(self.STREAM_CFG_M16) == 0:
+        elif M <= 16 and N % ops.stream_tile(self.STREAM_CFG_M16)[0] == 0:
             cfg = self.STREAM_CFG_M16
-        elif M <= 32 and N % nat.stream_gemm_bn(self.STREAM_CFG_M32) == 0:
+        elif M <= 32 and N % ops.stream_tile(self.STREAM_CFG_M32)[0] == 0:
             cfg = self.STREAM_CFG_M32
         elif M <= 64:
             cfg = self.STREAM_CFG_M64
         else:
             cfg = self.STREAM_WIDE.get(name)
-            if cfg is None or N % nat.stream_gemm_bn(cfg):
+            if cfg is None or N % ops.stream_tile(cfg)[0]:
                 cfg = self.STREAM_CFG_M128
-        if N % nat.stream_gemm_bn(cfg):
+        if N % ops.stream_tile(cfg)[0]:
             return -1
         narrow = self.STREAM_NARROW.get(cfg)
         if cfg == self.STREAM_CFG_M128 and name == "gate_up":
@@ -110,7 +109,7 @@ class FragmentProjections:
         cfg = self._stream_cfg(name, M, N, K)
         if cfg < 0 or K % 128:
             return -1, 1
-        return cfg, self._stream_splits(N, K, ops.native().stream_gemm_bn(cfg))
+        return cfg, self._stream_splits(N, K, ops.stream_tile(cfg)[0])
 
     # Projections held in the grouped fragment layout (shuffle_weights(w, G): the G row blocks of
     # each 16 G-row group adjacent per 32-deep k chunk), so the decode GEMM's waves (one block each)

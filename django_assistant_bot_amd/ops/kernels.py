@@ -18,6 +18,7 @@ from ._lib import expect, expect_bf16_contig, native, ptr, same_device, stream
 EPI_NONE, EPI_GELU, EPI_SWIGLU, EPI_SCORES = ref.EPI_NONE, ref.EPI_GELU, ref.EPI_SWIGLU, ref.EPI_SCORES
 EPI_SWIGLU8, EPI_GEGLU8, EPI_REGLU8 = ref.EPI_SWIGLU8, ref.EPI_GEGLU8, ref.EPI_REGLU8
 GLU8 = (EPI_SWIGLU8, EPI_GEGLU8, EPI_REGLU8)  # gated epilogues over 8-row [gate | up] groups
+_GLU_ALL = (EPI_SWIGLU, *GLU8)
 
 
 def _i32(t: torch.Tensor) -> None:
@@ -151,12 +152,16 @@ def encoder_forward(ids, pos_ids, cu_seqlens, max_seqlen: int, heads: int, eps: 
         if t.dtype != torch.int32 or not t.is_contiguous() or t.device != dev:
             return None
     shapes = ((3 * H, H), (3 * H,), (H, H), (H,), (H,), (H,), (F_, H), (F_,), (H, F_), (H,), (H,), (H,))
-    flat = []
-    for layer in layers:
-        for t, shape in zip(layer, shapes):
-            if t.shape != shape or t.dtype != bf or not t.is_contiguous() or t.device != dev:
-                return None
-            flat.append(t.data_ptr())
+    # twelve tensors a layer are looked at natively (144 of them 65 us -> 13); what that does not take is looked at here
+    api = getattr(torch.Tensor, "__dlpack_c_exchange_api__", None)
+    flat = None if api is None else native().operand_ptrs(api, torch.Tensor, ids, layers, shapes)
+    if flat is None:
+        flat = []
+        for layer in layers:
+            for t, shape in zip(layer, shapes):
+                if t.shape != shape or t.dtype != bf or not t.is_contiguous() or t.device != dev:
+                    return None
+                flat.append(t.data_ptr())
     for t in tables:
         if t.shape[-1] != H or t.dtype != bf or not t.is_contiguous() or t.device != dev:
             return None
@@ -890,6 +895,14 @@ def unshuffle_weights(w: torch.Tensor, group: int = 1) -> torch.Tensor:
     return w.reshape(N // 16, K // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).contiguous().view(N, K)
 
 
+@functools.lru_cache(maxsize=None)
+def stream_tile(cfg: int) -> tuple[int, int, bool]:
+    """(weight rows a workgroup or -1, most rows of x, whether the weights are in fragment layout) of a ``stream_gemm``
+    configuration."""
+    nat = native()
+    return nat.stream_gemm_bn(cfg), nat.stream_gemm_max_m(cfg), bool(nat.stream_gemm_shuffled(cfg))
+
+
 def stream_gemm(x, w, splits=1, epilogue=EPI_NONE, residual=None, out=None, nt=False, cfg=0, norm_eps: float = 0.0,
                 slab_dtype=torch.float32, w_group: int = 1, glu_bias=None):
     """Decode GEMM y = x w^T on the warp-specialised streaming kernel (``stream_gemm.hip``): bf16
@@ -909,23 +922,26 @@ def stream_gemm(x, w, splits=1, epilogue=EPI_NONE, residual=None, out=None, nt=F
     expect(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "bf16 operands required")
     expect(x.stride(-1) == 1 and w.stride(-1) == 1, "operands must be K-contiguous")
     M, K = x.shape
-    N = w.shape[0]
-    bn = native().stream_gemm_bn(cfg)
-    expect(bn > 0 and M <= native().stream_gemm_max_m(cfg), f"stream_gemm cfg {cfg}: bad config or M too large")
-    expect(w.shape[1] == K and N % bn == 0 and K % (splits * STREAM_KS) == 0,
-           f"stream_gemm needs N % {bn} == 0 and K % ({STREAM_KS}*splits) == 0")
-    expect(x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0, "row strides must be multiples of 8")
-    if native().stream_gemm_shuffled(cfg):
+    N, K_w = w.shape[0], w.shape[1]
+    bn, max_m, shuffled = stream_tile(cfg)
+    if bn <= 0 or M > max_m:
+        raise ValueError(f"stream_gemm cfg {cfg}: bad config or M too large")
+    if K_w != K or N % bn or K % (splits * STREAM_KS):
+        raise ValueError(f"stream_gemm needs N % {bn} == 0 and K % ({STREAM_KS}*splits) == 0")
+    ldx, ldw = x.stride(0), w.stride(0)
+    expect(ldx % 8 == 0 and ldw % 8 == 0, "row strides must be multiples of 8")
+    if shuffled:
         expect(w.is_contiguous(), "shuffled-layout configurations take a contiguous shuffle_weights() tensor")
     if splits > 1:
         expect(epilogue == EPI_NONE and residual is None, "split-K writes raw slabs")
         expect(slab_dtype in (torch.float32, torch.bfloat16), "slabs are fp32 or bf16")
         if out is None:
             out = torch.empty((splits, M, N), dtype=slab_dtype, device=x.device)
-        expect(out.dtype == slab_dtype and out.is_contiguous() and tuple(out.shape) == (splits, M, N), "bad slabs")
+        else:
+            expect(out.dtype == slab_dtype and out.is_contiguous() and tuple(out.shape) == (splits, M, N), "bad slabs")
         ldo = N
     else:
-        n_out = N // 2 if epilogue in (EPI_SWIGLU, *GLU8) else N
+        n_out = N // 2 if epilogue in _GLU_ALL else N
         if residual is not None:
             expect(epilogue == EPI_NONE and residual.dtype == torch.bfloat16 and residual.stride(-1) == 1
                    and tuple(residual.shape) == (M, N), "residual must be bf16 [M, N]")
@@ -934,9 +950,10 @@ def stream_gemm(x, w, splits=1, epilogue=EPI_NONE, residual=None, out=None, nt=F
             expect(bn % 32 == 0, f"stream_gemm cfg {cfg}: EPI_SWIGLU needs 32-row tiles (use EPI_SWIGLU8)")
         if out is None:
             out = torch.empty((M, n_out), dtype=torch.bfloat16, device=x.device)
-        expect(out.dtype == torch.bfloat16 and out.stride(-1) == 1 and tuple(out.shape) == (M, n_out), "bad output")
+        else:
+            expect(out.dtype == torch.bfloat16 and out.stride(-1) == 1 and tuple(out.shape) == (M, n_out), "bad output")
         ldo = out.stride(0)
-    native().stream_gemm(ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(out), ldo,
+    native().stream_gemm(x.data_ptr(), ldx, w.data_ptr(), ldw, out.data_ptr(), ldo,
                          ptr(residual if glu_bias is None else glu_bias),
                          residual.stride(0) if residual is not None else 0, M, N, K, splits, int(epilogue), stream(x),
                          int(bool(nt)), int(cfg), float(norm_eps), int(splits > 1 and out.dtype == torch.bfloat16),
