@@ -670,6 +670,9 @@ PYBIND11_MODULE(_native, m) {
                         (float*)out_vals, (int64_t*)out_ids, (int64_t*)out_docs, ST(s)),
           "top_hits");
   });
+  m.def("gemm_attn", [](u qkv, u cu, int batch, int D, float scale, u w, u b, u residual, u y, int T, int H, u s) {
+    check(dab::gemm_attn(CVP(qkv), (const int*)cu, batch, D, scale, CVP(w), CVP(b), CVP(residual), VP(y), T, H, ST(s)), "gemm_attn");
+  });
   m.def("gemm_ln", [](u x, u gain, u offset, float eps, u normed, u w, u b, u C, int M, int N, int K, int gelu, int tile, u s) {
     check(dab::gemm_ln(CVP(x), CVP(gain), CVP(offset), eps, VP(normed), CVP(w), CVP(b), VP(C), M, N, K, gelu, tile, ST(s)),
           "gemm_ln");

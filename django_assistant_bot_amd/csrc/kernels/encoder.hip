@@ -1,9 +1,9 @@
 // The sentence encoder's forward as one call: every launch of its layers enqueued from native code.
 //
-// For one question the GPU works about 0.35 ms on 64 launches (0.45 ms on 87 with the LayerNorms apart), and issuing
-// those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a launch costs
-// the runtime's own 1-2 us; the five activation buffers are the caller's, shared by all layers.  (The reference runs
-// one text a call through an eager model: ai/embedders/transformers.py:15-29.)
+// For one question the GPU works about 0.25 ms on 50 launches (0.45 ms on 87 with the LayerNorms and the attention apart),
+// and issuing those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a
+// launch costs the runtime's own 1-2 us; the five activation buffers are the caller's, shared by all layers.  (The
+// reference runs one text a call through an eager model: ai/embedders/transformers.py:15-29.)
 #include "common.h"
 #include "launchers.h"
 
@@ -52,8 +52,8 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
   return gemm_bt(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, 0, nullptr, nullptr, nullptr, 0, s, 0, 1);
 }
 
-// Packed token ids [T] -> hidden states x [T, H].  `layers`: per layer qkv, o, ln1, i, d, ln2 as (weight, bias) or
-// (gain, offset) pairs.  Buffers: x, y, att [T, H], qkv [T, 3 H], ffn [T, F].
+// Packed token ids [T] -> hidden states x [T, H].  `layers`: per layer qkv, o, ln1, i, d, ln2 as (weight, bias) or (gain,
+// offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att [T, H], qkv [T, 3 H], ffn [T, F].
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,
                     const void* offset, const uintptr_t* layers, void* x_, void* y_, void* att_, void* qkv_, void* ffn_,
@@ -79,10 +79,12 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     const uintptr_t* w = layers + 12 * l;
     auto W = [&](int i) { return (const void*)w[i]; };
     rc = ln ? norm_projection(ln, W(0), W(1), qkv, 3 * H, 0) : projection(x, W(0), W(1), nullptr, qkv, T, 3 * H, H, 0, s);
-    if (!rc)
+    const bool attn_o = gemm_attn_ok(T, H, D, batch) && !(w[2] % 16 || w[3] % 8);
+    if (!rc && attn_o) rc = gemm_attn(qkv, cu, batch, D, scale, W(2), W(3), x, y, T, H, s);
+    if (!rc && !attn_o)
       rc = flash_attention(qkv, 3 * H, D, qkv + H, qkv + 2 * H, 3 * H, D, nullptr, nullptr, nullptr, 0, 0, att, H, D, cu, cu,
                            nullptr, batch, max_len, heads, heads, D, 0, 0, scale, s);
-    if (!rc) rc = projection(att, W(2), W(3), x, y, T, H, H, 0, s);
+    if (!rc && !attn_o) rc = projection(att, W(2), W(3), x, y, T, H, H, 0, s);
     if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1);
     if (!rc) rc = projection(ffn, W(8), W(9), x, y, T, H, F, 0, s);
     ln = w + 10;

@@ -314,6 +314,156 @@ __global__ __launch_bounds__(512) void gemm_ln_kernel(SmallParams p, SmallNorm n
   small_finish<BM, BN, LDN, W, GELU, E>(p, tail, part, m0, n0);
 }
 
+// Attention over a few packed tokens with the output projection behind it: y = attention(qkv) w^T + b + residual, T <= 32
+// KB, heads of D = 32 or 64.  Apart these are two launches that wait for each other, and the first is a dozen workgroups on
+// 256 CUs.  Here a wave of the projection's split-K tile (its K-pieces w and w + 8 are one head of 64 or two of 32)
+// computes the attention of those heads for the tile's 16 rows itself, from qkv out of the L2, and feeds it to its MFMAs
+// from registers: the accumulators of O^T = V^T P^T are the projection's operand once its weights come in the same order of
+// columns (two runs of 4 for one of 8).  Every column block repeats the attention, 12 MFMAs and 8 exponentials a lane
+// and head.  What bounds it is the chain qkv -> scores -> row maximum -> V -> projection, and a CU's reads of qkv: whole
+// lines, through LDS (fragments of 16 rows x 64 B straight into registers: 6.1 us against 4.9 at 19 tokens, H 768).  K
+// and V share their rows in LDS.  One question of 19 tokens, 12 layers of 768: 298 -> 257 us; weights
+// from HBM 305 -> 282.
+// Arithmetic as in flash_kernel (attention.hip) and gemm_small_kernel: scores and sums fp32, P and O rounded to bf16.
+struct SmallAttention {
+  const bf16* qkv;  // [M, 3 K]
+  const int* cu;
+  int batch;
+  float scale_log2;
+};
+
+template <int D, int KB>
+__global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAttention at) {
+  constexpr int W = 8, LDN = 20, KT = 2 * KB, ND = D / 32, HP = 64 / D;  // HP: heads of a 64-wide piece
+  // a wave's rows of 128 B: 16 of Q, 16 of the weights, 32 KB of K and, once the scores are there, of V
+  constexpr int kW = 2048, kKV = 4096, kWave = kKV + KB * 4096;
+  constexpr float kMasked = -__builtin_huge_valf();
+  __shared__ __attribute__((aligned(16))) float part[W][16 * LDN];
+  __shared__ __attribute__((aligned(16))) char rows[W * kWave];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_m = (p.M + 15) / 16, id = small_id();
+  const int m0 = (id % tiles_m) * 16, n0 = (id / tiles_m) * 16;
+  const SmallTail<1> tail = small_tail<16, 16, 64 * W, 1>(p, m0, n0);
+  const int H = p.K, last = p.M - 1, ld = 3 * H;
+  const int query = min(m0 + li, last);
+  char* const ws = rows + w * kWave;
+
+  // whole lines: a load is 8 rows of 128 B
+  const int r8 = lane >> 3, c8 = lane & 7;
+  bf16x8 q[2][2], k[2][4 * KB], v[2][4 * KB], wt[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c0 = 64 * (w + W * i);
+    if (c0 >= H) break;  // wave-uniform
+    const bf16* base = at.qkv + c0 + 8 * c8;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) q[i][t] = *reinterpret_cast<const bf16x8*>(base + (size_t)min(m0 + 8 * t + r8, last) * ld);
+#pragma unroll
+    for (int t = 0; t < 4 * KB; ++t) k[i][t] = *reinterpret_cast<const bf16x8*>(base + H + (size_t)min(8 * t + r8, last) * ld);
+#pragma unroll
+    for (int t = 0; t < 4 * KB; ++t) v[i][t] = *reinterpret_cast<const bf16x8*>(base + 2 * H + (size_t)min(8 * t + r8, last) * ld);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      wt[i][t] = *reinterpret_cast<const bf16x8*>(p.B + (size_t)min(n0 + 8 * t + r8, p.N - 1) * p.ldb + c0 + 8 * c8);
+  }
+  // the query's sequence: the last start at or before it, the first one after it
+  int lo = 0, hi = p.M;
+  for (int b0 = 0; b0 <= at.batch; b0 += 64) {
+    const int starts = at.cu[min(b0 + lane, at.batch)], n = min(64, at.batch + 1 - b0);
+    for (int b = 0; b < n; ++b) {
+      const int c = __builtin_amdgcn_readlane(starts, b);
+      lo = c <= query ? c : lo;
+      hi = c > query ? min(hi, c) : hi;
+    }
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (64 * (w + W * i) >= H) break;
+    // 16-B chunk c of row r at c ^ ((r / 2) & 7); of V, whose reads transpose pairs of chunks, at c ^ (2 (r / 2) & 7)
+    auto put = [&](int at_, int r, int sw, const bf16x8& x) __attribute__((always_inline)) {
+      *reinterpret_cast<bf16x8*>(ws + at_ + r * 128 + 16 * (c8 ^ (sw & 7))) = x;
+    };
+#pragma unroll
+    for (int t = 0; t < 2; ++t) put(0, 8 * t + r8, (8 * t + r8) >> 1, q[i][t]);
+#pragma unroll
+    for (int t = 0; t < 4 * KB; ++t) put(kKV, 8 * t + r8, (8 * t + r8) >> 1, k[i][t]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) put(kW, 8 * t + r8, (8 * t + r8) >> 1, wt[i][t]);
+    const int sw = (li >> 1) & 7;
+    f32x4 s[HP][KT];
+    float mx[HP];
+#pragma unroll
+    for (int hd = 0; hd < HP; ++hd) {
+      mx[hd] = kMasked;
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+        s[hd][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+          const int off = li * 128 + 16 * ((4 * (ND * hd + c) + g) ^ sw);
+          s[hd][t] = mfma16(*reinterpret_cast<const bf16x8*>(ws + kKV + t * 2048 + off), *reinterpret_cast<const bf16x8*>(ws + off), s[hd][t]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = 16 * t + 4 * g + r;
+          s[hd][t][r] = (key >= lo) & (key < hi) ? s[hd][t][r] * at.scale_log2 : kMasked;
+          mx[hd] = fmaxf(mx[hd], s[hd][t][r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4 * KB; ++t) put(kKV, 8 * t + r8, 2 * ((8 * t + r8) >> 1), v[i][t]);
+#pragma unroll
+    for (int hd = 0; hd < HP; ++hd) {
+      mx[hd] = fmaxf(mx[hd], __shfl_xor(mx[hd], 16, 64));
+      mx[hd] = fmaxf(mx[hd], __shfl_xor(mx[hd], 32, 64));
+      float l = 0.f;
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[hd][t][r] = __builtin_amdgcn_exp2f(s[hd][t][r] - mx[hd]);
+          l += s[hd][t][r];
+        }
+      l += __shfl_xor(l, 16, 64);
+      l += __shfl_xor(l, 32, 64);
+      bf16x8 pb[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const f32x4 x = s[hd][2 * kb], y = s[hd][2 * kb + 1];
+        pb[kb] = __builtin_bit_cast(bf16x8, u32x4{pack2bf(x[0], x[1]), pack2bf(x[2], x[3]), pack2bf(y[0], y[1]), pack2bf(y[2], y[3])});
+      }
+      f32x4 o[2 * ND];
+#pragma unroll
+      for (int t = 0; t < 2 * ND; ++t) {
+        o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const int r = 32 * kb + 4 * g + (li >> 2), ch = 2 * (t + 2 * ND * hd) + ((li & 3) >> 1);
+          const char* src = ws + kKV + r * 128 + 16 * (ch ^ ((2 * (r >> 1)) & 7)) + 8 * (li & 1);
+          const bf16x4 a = ds_read_tr16(src), b = ds_read_tr16(src + 16 * 128);
+          o[t] = mfma16(bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, pb[kb], o[t]);
+        }
+      }
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+      for (int c = 0; c < ND; ++c) {  // 32 columns of the head: their slots (g, e) are columns 4 g + (e & 3) + 16 (e >> 2)
+        const u32x4 a = {pack2bf(o[2 * c][0] * inv, o[2 * c][1] * inv), pack2bf(o[2 * c][2] * inv, o[2 * c][3] * inv),
+                         pack2bf(o[2 * c + 1][0] * inv, o[2 * c + 1][1] * inv), pack2bf(o[2 * c + 1][2] * inv, o[2 * c + 1][3] * inv)};
+        const int ch = 4 * (ND * hd + c) + (g >> 1);
+        const char* wrow = ws + kW + li * 128 + 8 * (g & 1);
+        const u32x2 f0 = *reinterpret_cast<const u32x2*>(wrow + 16 * (ch ^ sw)), f1 = *reinterpret_cast<const u32x2*>(wrow + 16 * ((ch + 2) ^ sw));
+        acc = mfma16(__builtin_bit_cast(bf16x8, u32x4{f0[0], f0[1], f1[0], f1[1]}), __builtin_bit_cast(bf16x8, a), acc);
+      }
+    }
+  }
+  *reinterpret_cast<f32x4*>(&part[w][li * LDN + 4 * g]) = acc;
+  __syncthreads();
+  small_finish<16, 16, LDN, W, false, 1>(p, tail, part, m0, n0);
+}
+
 // BM x BN tiles by 2 x 2 waves over a ring of NS K-tiles (64 wide) in LDS, filled by LDS-DMA NS - 1 tiles ahead with
 // counted waits: one barrier a K-tile and no drained queue.  LDS rows of 128 B, 16-B chunk c of row r at
 // c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly).
@@ -495,6 +645,29 @@ int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void
   LN_GEMM(1, 4)
   LN_GEMM(2, 4)
 #undef LN_GEMM
+  return hipGetLastError();
+}
+
+// y = attention(qkv) w^T + b + residual of a few packed tokens (qkv [T, 3 H], cu [batch + 1]): up to 32, and up to 64 where
+// a wave's two pieces are not yet more than the two launches (us a layer, two launches -> one, one text or four of T / 4: H 384
+// at T 6-32 5.6 -> 4.0, 33-64 5.7-5.9 -> 5.0-5.1; H 768 at 6-32 6.5-6.7 -> 4.7-5.0, 33-64 6.8-7.0 -> 6.4-6.7, eight of 8
+// 7.0 -> 7.05; H 1024 at 6-32 7.2-7.5 -> 5.9-6.3, 33-64 7.5-7.7 -> 8.1-8.9).
+int gemm_attn_ok(int T, int H, int D, int batch) {
+  return T > 0 && T <= (H <= 768 ? 64 : 32) && batch > 0 && (D == 32 || D == 64) && H % 64 == 0 && H > 0 && H <= 1024;
+}
+
+int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
+              void* y, int T, int H, hipStream_t s) {
+  if (!gemm_attn_ok(T, H, D, batch)) return hipErrorInvalidValue;
+  if (((uintptr_t)qkv | (uintptr_t)w) % 16 || ((uintptr_t)b | (uintptr_t)residual | (uintptr_t)y) % 8 || (uintptr_t)cu % 4)
+    return hipErrorInvalidValue;
+  const SmallParams p = {nullptr, (const bf16*)w, (bf16*)y, (const bf16*)b, (const bf16*)residual, T, H, H, H, H, H, H};
+  const SmallAttention at = {(const bf16*)qkv, cu, batch, scale * 1.44269504088896340736f};
+  const dim3 grid(((T + 15) / 16) * (H / 16));
+  if (D == 64 && T <= 32) hipLaunchKernelGGL((gemm_attn_kernel<64, 1>), grid, dim3(512), 0, s, p, at);
+  else if (D == 64) hipLaunchKernelGGL((gemm_attn_kernel<64, 2>), grid, dim3(512), 0, s, p, at);
+  else if (T <= 32) hipLaunchKernelGGL((gemm_attn_kernel<32, 1>), grid, dim3(512), 0, s, p, at);
+  else hipLaunchKernelGGL((gemm_attn_kernel<32, 2>), grid, dim3(512), 0, s, p, at);
   return hipGetLastError();
 }
 

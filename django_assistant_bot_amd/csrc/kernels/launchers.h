@@ -380,6 +380,9 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
 
 // gemm_small.hip
 int gemm_small_ok(long M, long N, long K, long lda, long ldb, long ldc, long ldr);
+int gemm_attn_ok(int T, int H, int D, int batch);
+int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
+              void* y, int T, int H, hipStream_t s);
 int gemm_ln_ok(int M, int N, int K, int tile);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
             int M, int N, int K, int gelu, int tile, hipStream_t s);
