@@ -1592,9 +1592,17 @@ struct DecodeParams {
   L3Warm warm;  // optional: the next projections' weights, warmed into L3 by appended workgroups
 };
 
-// Small batches at D = 128: two LDS slots a wave (at batch 128 the one-slot kernel's two workgroups per CU are 2.8 % faster per
-// step: 7.44 vs 7.65 ms, profiles/low_load_latency.md), whose block ids one lane each holds
-static bool decode_two_slots(int batch, int Hkv, int part_size) { return batch * Hkv <= 64 && part_size <= 64 * 4 * 32; }
+// D = 128: two LDS slots a wave, whose block ids one lane each holds, where the items find a CU each (128 KB of LDS), and up
+// to half as many again in whole contexts.  Beyond that the one-slot form's two workgroups a CU.  us a launch, one slot ->
+// two, (sequences, contexts), 8 key heads: (16, 300-1700) 24.3 -> 22.7, (16, 2000-4000) 48.8 -> 39.6, (24, 300-1700) 29.7 ->
+// 27.5, (32, 300-1700) 34.4 -> 32.3, (48, 300-1700) 44.4 -> 41.3, but (32, 900-1500) 34.3 -> 35.8, (64, 300-1700) 52.2 -> 54.0,
+// (128, 900-1500) 102.7 -> 112.2.  With the rotation inside (decode_rope_ok), us a step of Llama-3-8B: 9 sequences 3612 ->
+// 3544, 16 3989 -> 3843, 32 4325 -> 4240, of 900-1500 4231 -> 4210, 48 4699 -> 4686.
+constexpr int kDecodeCus = 256;
+static bool decode_two_slots(int batch, int Hkv, int part_size) {
+  const long items = (long)batch * Hkv;
+  return part_size <= 64 * 4 * 32 && (items <= kDecodeCus || (items <= 3 * kDecodeCus / 2 && part_size >= 2048));
+}
 
 constexpr int kCombine = 8;  // partial results requested together by the combine
 
@@ -1684,9 +1692,25 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
 #pragma unroll
   for (int off = 32; off; off >>= 1) maxc = max(maxc, __shfl_xor(maxc, off));
   maxc = __builtin_amdgcn_readfirstlane(maxc);
-  const int part_size = decode_partition(p.part_size, maxc, BH, p.max_parts);
+  int part_size = decode_partition(p.part_size, maxc, BH, p.max_parts);
+  if constexpr (NSLOT == 2) {
+    // Above 64 items: partitions doubled, up to 2048 keys, until all of them find a CU at once (a second round waits for
+    // the first, and partitions cost a combine).  us a launch, 512 keys -> those taken: (16, 300-1700) 24.0 -> 22.7, (20,
+    // 800-3000) 42 -> 35.9, (24, 300-1700) 29.1 -> 27.5; (9, 200-2000), which stay at 512, 19.5, at 1024 21.8.
+    auto parts_of = [&](int size) {
+      float n = lane < nb ? (float)((seen_keys(ctx_l) + size - 1) / size) : 0.f;
+      for (int i = lane + 64; i < nb; i += 64) n += (float)((seen_keys(p.ctx_lens[i]) + size - 1) / size);
+      return (int)wave_sum_valu(n) * p.Hkv;
+    };
+    if (BH > 64)
+      while (part_size < 2048 && part_size < maxc && maxc <= part_size * p.max_parts && parts_of(part_size) > kDecodeCus)
+        part_size *= 2;
+  }
   const int live_items = min(p.max_parts, (maxc + part_size - 1) / part_size) * BH;
-  for (int item = blockIdx.x; item < live_items; item += attn_blocks) {
+  for (int r0 = 0, back = 0; r0 < live_items; r0 += attn_blocks, back ^= NSLOT - 1) {
+    // two slots: the launch has a workgroup a CU, so every other round goes backwards (the items come longest first)
+    const int item = r0 + (back ? attn_blocks - 1 - (int)blockIdx.x : (int)blockIdx.x);
+    if (item >= live_items) continue;
     const int part = item / BH;
     const int bh = item - part * BH;
     const int hk = bh % p.Hkv;
@@ -2348,8 +2372,8 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
 
 // Whether a decode step rotates and writes its rows inside the attention: while the items find a CU or two at once (every
 // further round of them pays the sums again).  us a step, rope_kv_write apart -> inside: Llama-3-8B (D 128), 1 sequence 3087
-// -> 3064, 4: 3223 -> 3169, 8: 3424 -> 3356 (above 64 items the one-slot form has no registers left for it); Llama-3.2-1B (D
-// 64, 8 key heads), 6: 944 -> 930, 24: 1054 -> 1032, 48: 1106 -> 1099, 100: 1549 -> 1724.
+// -> 3064, 4: 3223 -> 3169, 8: 3424 -> 3356 (the one-slot form has no registers left for it); Llama-3.2-1B (D 64, 8 key
+// heads), 6: 944 -> 930, 24: 1054 -> 1032, 48: 1106 -> 1099, 100: 1549 -> 1724.
 int decode_rope_ok(int batch, int Hkv, int D, int part_size) {
   if (batch <= 0 || Hkv <= 0) return 0;
   return D == 128 ? decode_two_slots(batch, Hkv, part_size) : D == 64 && batch * Hkv <= 384;
@@ -2408,7 +2432,10 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
     return hipErrorInvalidValue;
   const bool ext = slopes || prm.gate.y.p;
   const int total_items = max_parts * Hkv * batch;
-  dim3 grid((total_items < 2048 ? total_items : 2048) + prm.warm.blocks);
+  // A workgroup without an item still waits for the contexts, and with two slots a CU runs one at a time: a workgroup a CU
+  // (us a step of Llama-3-8B with 2048 workgroups -> 256: 4 sequences 3419 -> 3352, 8 3668 -> 3560).
+  const int most = D == 128 && decode_two_slots(batch, Hkv, part_size) ? kDecodeCus : 2048;
+  dim3 grid((total_items < most ? total_items : most) + prm.warm.blocks);
   // K/V are read exactly once per step: non-temporal loads (aux = 2) -- in the Llama-3-8B decode step
   // at batch 128 this took the attention from 127 to 111 us per layer (5.1 -> 5.8 TB/s;
   // profiles/decode_round2.md).  D = 128 stages K / V by LDS-DMA (100.7 vs 102.6 us isolated, same

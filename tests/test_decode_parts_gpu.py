@@ -10,10 +10,13 @@ DEV = "cuda"
 
 
 # halved: up to 192 items and a workspace that holds them (max_parts); 64 and 65 sequences: lengths held in lanes or not;
-# 8 / 9 / 17 partitions: one, two and three rounds of the combine
+# 8 / 9 / 17 partitions: one, two and three rounds of the combine; above 64 items partitions doubled once, twice, up to
+# 2048 keys with items left for a second and third round of 256 workgroups, and not where the workspace then covered more
 @pytest.mark.parametrize("ctx,Hkv,max_parts", [([1], 8, 16), ([256, 257], 8, 16), ([2048], 2, 8), ([2049], 2, 9), ([2048], 2, 7),
                                                ([4200, 3], 1, 32), ([513] * 12, 8, 4), ([513] * 13, 2, 4), ([70] * 63 + [900], 1, 2),
-                                               ([70] * 64 + [1100], 1, 3)])
+                                               ([70] * 64 + [1100], 1, 3), ([1700, 600, 513, 512] * 4, 8, 4),
+                                               ([2000, 1500, 90, 1] * 6, 8, 4), ([5000, 2049, 4100, 7] * 8, 8, 10),
+                                               ([1500] * 16, 8, 2), ([2100] * 70, 3, 5)])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("order", [False, True])
 def test_decode_partitions(ctx, Hkv, max_parts, D, order):

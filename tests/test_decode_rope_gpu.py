@@ -10,7 +10,7 @@ DEV = "cuda"
 
 # contexts at the edges of a sub-tile (32 keys), a block (64), a partition (512, halved for few items) and of the four waves'
 # round; fewer and more slabs than are held; a padded row (no slot), a slot elsewhere than at the context's end
-@pytest.mark.parametrize("D,Hq,Hkv,B", [(128, 32, 8, 1), (128, 32, 8, 8), (128, 12, 3, 9), (128, 5, 1, 40), (64, 32, 8, 6),
+@pytest.mark.parametrize("D,Hq,Hkv,B", [(128, 32, 8, 1), (128, 32, 8, 8), (128, 12, 3, 9), (128, 5, 1, 40), (128, 32, 8, 32), (64, 32, 8, 6),
                                         (64, 32, 8, 48), (64, 2, 2, 130)])
 @pytest.mark.parametrize("S,dtype", [(0, torch.bfloat16), (2, torch.bfloat16), (3, torch.float32), (4, torch.bfloat16),
                                      (8, torch.bfloat16), (4, torch.float32)])
@@ -48,5 +48,5 @@ def test_rope_inside_the_attention(D, Hq, Hkv, B, S, dtype):
 
 
 def test_what_is_refused():
-    assert not ops.decode_rope_ok(9, 8, 128, 512) and not ops.decode_rope_ok(8, 8, 128, 16384)
+    assert not ops.decode_rope_ok(33, 8, 128, 512) and not ops.decode_rope_ok(8, 8, 128, 16384)
     assert not ops.decode_rope_ok(49, 8, 64, 512) and not ops.decode_rope_ok(1, 8, 32, 512)
