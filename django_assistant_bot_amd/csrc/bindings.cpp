@@ -630,16 +630,27 @@ PYBIND11_MODULE(_native, m) {
   m.def("small_tile", &dab::small_tile);
   m.def("encoder_forward", [](u ids, u pos, u cu, int T, int batch, int max_len, int H, int heads, int F, float eps, u word,
                               u pos_table, u type, u gain, u offset, const std::vector<u>& layers, u x, u y, u att, u qkv,
-                              u ffn, u s) {
+                              u ffn, u slabs, u s) {
     if (layers.size() % 12) throw std::invalid_argument("encoder_forward: 12 tensors a layer");
     std::vector<uintptr_t> l(layers.begin(), layers.end());
     check(dab::encoder_forward((const int*)ids, (const int*)pos, (const int*)cu, T, batch, max_len, H, heads, F,
                                (int)(l.size() / 12), eps, CVP(word), CVP(pos_table), CVP(type), CVP(gain), CVP(offset),
-                               l.data(), VP(x), VP(y), VP(att), VP(qkv), VP(ffn), ST(s)),
+                               l.data(), VP(x), VP(y), VP(att), VP(qkv), VP(ffn), VP(slabs), ST(s)),
           "encoder_forward");
   });
   m.def("operand_ptrs", &operand_ptrs);
   m.def("gemm_small_ok", &dab::gemm_small_ok);
+  m.def("slab_slices", [](int M, int N, int K) {
+    int tile;
+    return dab::slab_slices(M, N, K, &tile);
+  });
+  m.def("gemm_slab", [](u A, u B, u slabs, int M, int N, int K, u s) {
+    check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s)), "gemm_slab");
+  });
+  m.def("layernorm_slabs", [](u out, u slabs, int S, u bias, u res, u gamma, u beta, int rows, int cols, float eps, u s) {
+    check(dab::layernorm_slabs(VP(out), CVP(slabs), S, CVP(bias), CVP(res), CVP(gamma), CVP(beta), rows, cols, eps, ST(s)),
+          "layernorm_slabs");
+  });
   m.def("gemm_small", [](u A, long lda, u B, long ldb, u C, long ldc, u bias, u residual, long ldr, int M, int N, int K,
                          int gelu, int tile, u s) {
     check(dab::gemm_small(CVP(A), lda, CVP(B), ldb, VP(C), ldc, CVP(bias), CVP(residual), ldr, M, N, K, gelu, tile, ST(s)),

@@ -53,11 +53,12 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
 }
 
 // Packed token ids [T] -> hidden states x [T, H].  `layers`: per layer qkv, o, ln1, i, d, ln2 as (weight, bias) or (gain,
-// offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att [T, H], qkv [T, 3 H], ffn [T, F].
+// offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att [T, H], qkv [T, 3 H], ffn [T, F], slabs
+// [slices, T, H] fp32 where the down projection is cut into K-slices that the LayerNorm behind it sums (slab_slices), or null.
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,
                     const void* offset, const uintptr_t* layers, void* x_, void* y_, void* att_, void* qkv_, void* ffn_,
-                    hipStream_t s) {
+                    void* slabs, hipStream_t s) {
   if (T <= 0 || batch <= 0 || max_len <= 0) return 0;
   if (H <= 0 || heads <= 0 || H % heads || H % 64 || F % 64 || F <= 0) return hipErrorInvalidValue;
   const int D = H / heads;
@@ -74,6 +75,8 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s);
     return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s);
   };
+  int tile;
+  const int slices = slabs ? slab_slices(T, H, F, &tile) : 0;
   const uintptr_t* ln = nullptr;  // the layer's own norm of y, applied in front of the next projection
   for (int l = 0; l < n_layers && !rc; ++l) {
     const uintptr_t* w = layers + 12 * l;
@@ -86,6 +89,12 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
                            nullptr, batch, max_len, heads, heads, D, 0, 0, scale, s);
     if (!rc && !attn_o) rc = projection(att, W(2), W(3), x, y, T, H, H, 0, s);
     if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1);
+    if (slices && !(w[8] % 16 || (w[9] | w[10] | w[11]) % 4)) {
+      if (!rc) rc = gemm_slab(ffn, W(8), slabs, T, H, F, s);
+      if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s);
+      ln = nullptr;
+      continue;
+    }
     if (!rc) rc = projection(ffn, W(8), W(9), x, y, T, H, F, 0, s);
     ln = w + 10;
   }

@@ -38,6 +38,8 @@ struct SmallParams {
   const bf16* residual;
   int M, N, K;
   int lda, ldb, ldc, ldr;
+  float* slabs;  // SLAB: the slices' fp32 sums [slices][M][N] instead of C
+  int slices;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const bf16* base, int rows, int ld, int K) {
@@ -467,7 +469,7 @@ __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAtte
 // BM x BN tiles by 2 x 2 waves over a ring of NS K-tiles (64 wide) in LDS, filled by LDS-DMA NS - 1 tiles ahead with
 // counted waits: one barrier a K-tile and no drained queue.  LDS rows of 128 B, 16-B chunk c of row r at
 // c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly).
-template <int BM, int BN, int NS, bool GELU>
+template <int BM, int BN, int NS, bool GELU, bool SLAB = false>
 __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
   constexpr int MI = BM / 32, NI = BN / 32;           // 16 x 16 tiles of a wave
   constexpr int PA = BM / 32, PB = BN / 32;           // LDS-DMA instructions of a wave for a K-tile (8 rows each)
@@ -476,7 +478,9 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w >> 1, wn = w & 1;
-  const int tiles_m = (p.M + BM - 1) / BM, id = small_id();
+  // SLAB: the tiles of a K-slice have neighbouring ids, so an XCD reads one or two slices of A and a few columns' weights
+  const int tiles_m = (p.M + BM - 1) / BM, tiles = SLAB ? tiles_m * ((p.N + BN - 1) / BN) : 0, id0 = small_id();
+  const int slice = SLAB ? id0 / tiles : 0, id = id0 - slice * tiles;
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
 
   const __amdgpu_buffer_rsrc_t ra = rows_rsrc(p.A, p.M, p.lda, p.K), rb = rows_rsrc(p.B, p.N, p.ldb, p.K);
@@ -511,10 +515,10 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int nk = p.K / 64;
+  const int k0 = SLAB ? p.K / 64 * slice / p.slices : 0, nk = (SLAB ? p.K / 64 * (slice + 1) / p.slices : p.K / 64) - k0;
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t)
-    if (t < nk) stage(t, t);
+    if (t < nk) stage(t, k0 + t);
   int buf = 0;
   for (int t = 0; t < nk; ++t) {
     const int ahead = min(NS - 2, nk - 1 - t);  // K-tiles after t that may stay in flight
@@ -525,7 +529,7 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last K-tile's reads: its buffer is filled next
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + NS - 1 < nk) stage(buf == 0 ? NS - 1 : buf - 1, t + NS - 1);
+    if (t + NS - 1 < nk) stage(buf == 0 ? NS - 1 : buf - 1, k0 + t + NS - 1);
     const char* sa = smem + buf * kStage + wm * (BM / 2) * 128;
     const char* sb = smem + buf * kStage + kA + wn * (BN / 2) * 128;
     bf16x8 af[MI][2], bfr[NI][2];
@@ -551,6 +555,14 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
   for (int i = 0; i < NI; ++i) {
     const int n = n0 + wn * (BN / 2) + 16 * i + 4 * g;
     if (n >= p.N) continue;
+    if constexpr (SLAB) {
+#pragma unroll
+      for (int j = 0; j < MI; ++j) {
+        const int m = m0 + wm * (BM / 2) + 16 * j + li;
+        if (m < p.M) *reinterpret_cast<f32x4*>(p.slabs + ((size_t)slice * p.M + m) * p.N + n) = acc[i][j];
+      }
+      continue;
+    }
     f32x4 b4 = {0.f, 0.f, 0.f, 0.f};
     if (p.bias) {
       const u32x2 b = *reinterpret_cast<const u32x2*>(p.bias + n);
@@ -618,6 +630,42 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
   }
 #undef PIPE
 #undef SMALL
+  return hipGetLastError();
+}
+
+// K-slices that a long-K projection in front of a LayerNorm (which sums them: layernorm_slabs) is cut into, 0: none, and its
+// tile (64 or 128 wide).  Its tiles alone leave CUs idle or one workgroup each, whose share of the operands from past L2 is
+// what takes the time; in slices they are two workgroups of 64 x 64 a CU, or one of 128 x 128.  Between those numbers, below
+// 139 tiles of 64 x 64 and with a short K the slabs (8 bytes an element and slice there and back) cost more than that.
+// us of product and LayerNorm, one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 ->
+// 15.9, (1100, 768, 3072) 17.7 -> 17.3, (2200, 384, 1536) 14.2 -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200,
+// 768, 3072) 29.4 -> 26.2, (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5
+// -> 13.9, (1500, 384, 1536) 12.0 -> 12.3 in three slices of 512, (4600, 768, 3072) 41.8 -> 48.3, (832, 768, 768) 9.5 -> 10.3.
+// Whole calls of the encoder: bge-base 725 tokens 621 -> 605, 825 641 -> 619, 1057 738 -> 730, 1649 1042 -> 968, 2543 1247 ->
+// 1162; MiniLM 2815 392 -> 370, 5315 524 -> 501; bge-large 555 1560 -> 1493, 1590 2747 -> 2541, 2021 2979 -> 2720, but 765 in
+// two slices of 2048 1757 -> 1788, not taken.
+int slab_slices(int M, int N, int K, int* tile) {
+  if (M <= 0 || K < 1536 || K % 64 || (N != 384 && N != 768 && N != 1024)) return 0;
+  const long t64 = ((M + 63) / 64) * (long)(N / 64), t128 = ((M + 127) / 128) * (long)(N / 128);
+  *tile = 64;
+  if (t64 >= 139 && t64 <= 170 && K >= 3 * 768) return 3;
+  if (t64 >= 192 && t64 <= 224 && K < 4096) return 2;
+  *tile = 128;
+  if (t128 >= 64 && t128 <= 85) return 3;
+  if (t128 >= 96 && t128 <= 128) return 2;
+  return 0;
+}
+
+// slabs [slices][M][N] fp32 = the K-slices' sums of A w^T, as slab_slices says
+int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s) {
+  int tile = 0;
+  const int slices = slab_slices(M, N, K, &tile);
+  if (!slices || !gemm_small_ok(M, N, K, K, K, N, 0)) return hipErrorInvalidValue;
+  if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)slabs) % 16) return hipErrorInvalidValue;
+  const SmallParams p = {(const bf16*)A, (const bf16*)B, nullptr, nullptr, nullptr, M, N, K, K, K, N, 0, (float*)slabs, slices};
+  const dim3 grid(((M + tile - 1) / tile) * (N / tile) * slices);
+  if (tile == 64) hipLaunchKernelGGL((gemm_pipe_kernel<64, 64, 4, false, true>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((gemm_pipe_kernel<128, 128, 4, false, true>), grid, dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -41,6 +41,8 @@ int rmsnorm(void* out, void* res_out, const void* x, const void* res_in, const v
             hipStream_t s);
 int rmsnorm_slabs(void* out, void* res_out, const void* slabs, int S, long slab_stride, const void* res_in,
                   const void* w, int rows, int cols, float eps, hipStream_t s, int slab_bf16 = 0);
+int layernorm_slabs(void* out, const void* slabs, int S, const void* bias, const void* res, const void* gamma,
+                    const void* beta, int rows, int cols, float eps, hipStream_t s);
 int layernorm(void* out, const void* x, const void* res_in, const void* gamma, const void* beta, int rows, int cols,
               float eps, hipStream_t s);
 int bert_embed(void* out, const int* ids, const int* pos_ids, const int* type_ids, const void* word, const void* pos,
@@ -375,7 +377,7 @@ int topk_rows_2stage(const float* scores, long ld, int rows, int n, int k, float
 int small_tile(int M, int N, int K);
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,
-                    const void* offset, const uintptr_t* layers, void* x, void* y, void* att, void* qkv, void* ffn,
+                    const void* offset, const uintptr_t* layers, void* x, void* y, void* att, void* qkv, void* ffn, void* slabs,
                     hipStream_t s);
 
 // gemm_small.hip
@@ -384,6 +386,8 @@ int gemm_attn_ok(int T, int H, int D, int batch);
 int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
               void* y, int T, int H, hipStream_t s);
 int gemm_ln_ok(int M, int N, int K, int tile);
+int slab_slices(int M, int N, int K, int* tile);
+int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
             int M, int N, int K, int gelu, int tile, hipStream_t s);
 int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, const void* residual,

@@ -298,6 +298,67 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(bf16* __restrict__ 
   }
 }
 
+// LayerNorm(sum of S fp32 slabs [S][rows][cols] + bias + residual), rounded once; a row a wave, every load in front of the
+// sums (a launch and one round trip bound it; out may be the residual).  3.5-4 us at 832 rows of 768 in 3 slabs.
+template <int CP, int S>
+__global__ __launch_bounds__(256) void layernorm_slab_kernel(bf16* out, const float* __restrict__ slabs,
+                                                             const bf16* __restrict__ bias, const bf16* res,
+                                                             const bf16* __restrict__ gamma, const bf16* __restrict__ beta,
+                                                             int rows, float eps) {
+  constexpr int cols = 128 * CP;
+  const int lane = threadIdx.x & 63;
+  const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= (size_t)rows) return;  // whole wave
+  f32x2_t sv[S][CP];
+  uint32_t rv[CP], bv[CP], gv[CP], ov[CP];
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+      sv[k][c] = reinterpret_cast<const f32x2_t*>(slabs + ((size_t)k * rows + row) * cols)[c * 64 + lane];
+    rv[c] = reinterpret_cast<const uint32_t*>(res + row * cols)[c * 64 + lane];
+    bv[c] = reinterpret_cast<const uint32_t*>(bias)[c * 64 + lane];
+  }
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+    gv[c] = reinterpret_cast<const uint32_t*>(gamma)[c * 64 + lane];
+    ov[c] = reinterpret_cast<const uint32_t*>(beta)[c * 64 + lane];
+  }
+  float v[CP][2], s = 0.f;
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float a = sv[0][c][j];
+#pragma unroll
+      for (int k = 1; k < S; ++k) a += sv[k][c][j];
+      v[c][j] = a + bf2f((uint16_t)(bv[c] >> (16 * j))) + bf2f((uint16_t)(rv[c] >> (16 * j)));
+      s += v[c][j];
+    }
+  }
+  s = wave_sum_valu(s);
+  const float mean = s / (float)cols;
+  float sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < CP; ++c)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float d = v[c][j] - mean;
+      sq += d * d;
+    }
+  sq = wave_sum_valu(sq);
+  const float inv = rsqrtf(sq / (float)cols + eps);
+  uint32_t* orow = reinterpret_cast<uint32_t*>(out + row * cols);
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+    float o[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      o[j] = (v[c][j] - mean) * inv * bf2f((uint16_t)(gv[c] >> (16 * j))) + bf2f((uint16_t)(ov[c] >> (16 * j)));
+    orow[c * 64 + lane] = pack2bf(o[0], o[1]);
+  }
+}
+
 // BERT embeddings: LN(word[id] + pos[pos_id] + type[type_id]) fused; type ids default to 0.
 template <int NT, int VPT>
 __global__ __launch_bounds__(NT) void bert_embed_kernel(bf16* __restrict__ out, const int* __restrict__ ids,
@@ -535,6 +596,28 @@ int layernorm(void* out, const void* x, const void* res_in, const void* gamma, c
   DAB_ROW_DISPATCH(layernorm_kernel, rows, cols, s, (bf16*)out, (const bf16*)x, (const bf16*)res_in,
                    (const bf16*)gamma, (const bf16*)beta, cols, eps);
   return hipGetLastError();
+}
+
+int layernorm_slabs(void* out, const void* slabs_, int S, const void* bias, const void* res, const void* gamma,
+                    const void* beta, int rows, int cols, float eps, hipStream_t s) {
+  if (rows <= 0) return 0;
+  const float* slabs = (const float*)slabs_;
+  if ((uintptr_t)slabs % 8 || ((uintptr_t)out | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)gamma | (uintptr_t)beta) % 4)
+    return hipErrorInvalidValue;
+  const dim3 grid((rows + 3) / 4);
+#define LN_SLAB(CP, SS)                                                                                               \
+  if (cols == 128 * CP && S == SS) {                                                                                  \
+    hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS>), grid, dim3(256), 0, s, (bf16*)out, slabs, (const bf16*)bias,  \
+                       (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps);                           \
+    return hipGetLastError();                                                                                         \
+  }
+#define LN_SLABS(CP) LN_SLAB(CP, 2) LN_SLAB(CP, 3)
+  LN_SLABS(3)
+  LN_SLABS(6)
+  LN_SLABS(8)
+#undef LN_SLABS
+#undef LN_SLAB
+  return hipErrorInvalidValue;
 }
 
 int bert_embed(void* out, const int* ids, const int* pos_ids, const int* type_ids, const void* word, const void* pos,

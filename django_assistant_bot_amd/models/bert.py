@@ -83,8 +83,7 @@ class BertEncoder:
             h = ops.linear(a.view(T, H), L.o_w, L.o_b, residual=x)
             x = ops.layernorm(h, L.ln1_g, L.ln1_b, cfg.eps)
             f = ops.linear(x, L.i_w, L.i_b, act="gelu")  # bias + GELU(erf) epilogue
-            h = ops.linear(f, L.d_w, L.d_b, residual=x)
-            x = ops.layernorm(h, L.ln2_g, L.ln2_b, cfg.eps)
+            x = ops.linear_layernorm(f, L.d_w, L.d_b, x, L.ln2_g, L.ln2_b, cfg.eps)
         return x
 
     def encode(self, ids, pos_ids, cu_seqlens, max_seqlen, normalize=None, want_bf16=False, out=None, rows=None):

@@ -167,10 +167,30 @@ def encoder_forward(ids, pos_ids, cu_seqlens, max_seqlen: int, heads: int, eps: 
             return None
     x, y, att = (torch.empty((T, H), dtype=bf, device=dev) for _ in range(3))
     qkv, ffn = torch.empty((T, 3 * H), dtype=bf, device=dev), torch.empty((T, F_), dtype=bf, device=dev)
+    slices = native().slab_slices(T, H, F_)
+    slabs = torch.empty((slices, T, H), dtype=torch.float32, device=dev) if slices else None
     native().encoder_forward(ptr(ids), ptr(pos_ids), ptr(cu_seqlens), T, cu_seqlens.numel() - 1, int(max_seqlen), H, heads,
                              F_, float(eps), *(ptr(t) for t in tables), flat, ptr(x), ptr(y), ptr(att), ptr(qkv), ptr(ffn),
-                             stream(ids))
+                             ptr(slabs), stream(ids))
     return x
+
+
+def linear_layernorm(x, w, b, residual, gamma, beta, eps):
+    """LayerNorm(x w^T + b + residual) of contiguous rows: in K-slices that the norm sums in 32 bits where that is the faster
+    (``slab_slices`` in gemm_small.hip), else ``linear`` and ``layernorm``."""
+    (M, K), N = x.shape, w.shape[0]
+    slices = native().slab_slices(M, N, K) if x.is_cuda and w.dim() == 2 else 0
+    operands = (x, w, b, residual, gamma, beta)
+    if (not slices or any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.device != x.device for t in operands)
+            or w.shape[1] != K or residual.shape != (M, N) or any(t.shape != (N,) for t in (b, gamma, beta))
+            or (ptr(x) | ptr(w)) % 16 or (ptr(b) | ptr(residual) | ptr(gamma) | ptr(beta)) % 4):
+        return layernorm(linear(x, w, b, residual=residual), gamma, beta, eps)
+    slabs = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+    out = torch.empty_like(residual)
+    native().gemm_slab(ptr(x), ptr(w), ptr(slabs), M, N, K, stream(x))
+    native().layernorm_slabs(ptr(out), ptr(slabs), slices, ptr(b), ptr(residual), ptr(gamma), ptr(beta), M, N, float(eps),
+                             stream(x))
+    return out
 
 
 # ----------------------------------------------------------------------------------------------
