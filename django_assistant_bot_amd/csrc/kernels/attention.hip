@@ -450,20 +450,26 @@ __device__ __forceinline__ unsigned lds_addr(const char* p) {
 // sched_group_barrier (4 reads ahead, then one MFMA per read) instead of hipcc's own order; same
 // instructions and accumulation order (bit-identical).
 //
+// SPLIT (causal, 8 waves, 128 queries): the two wave groups take the even and the odd key tiles through a ring of two buffers
+// each (128 KB: a workgroup a CU) and the second group's sums join the first's through LDS at the end.  For grids of about a
+// workgroup a CU, where four waves are one a SIMD and walk all tiles in a row, 2 us each (both sides at the launch).
+//
 // BIAS: softmax sink and slopes (FlashParams, either may be null; no window).  The accumulators of S^T start at the key's
 // distance term, the running maximum at the sink, whose own term is then 1.
 template <bool CAUSAL, bool VPIPE = false, int NW = 4, bool STAG = false, bool PAIR = false, bool ONEBAR = false,
-          bool SMS = false, bool SGB = false, bool BIAS = false>
+          bool SMS = false, bool SGB = false, bool BIAS = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(FlashParams p) {
   static_assert(NW == 4 || NW == 8, "4 or 8 waves");
   static_assert(!STAG || NW == 8, "staggered groups: 8 waves");
   static_assert(!PAIR || (NW == 4 && CAUSAL), "paired blocks: 4 waves, causal");
   static_assert(!BIAS || (CAUSAL && !STAG), "sink and slopes: causal, no staggered groups");
-  constexpr int D = 128, KT = 64, QB = 32 * NW;
+  static_assert(!SPLIT || (NW == 8 && CAUSAL && VPIPE && !STAG && !BIAS && !SMS), "keys split: 8 waves, causal");
+  constexpr int QW = SPLIT ? 4 : NW;  // waves that share a tile
+  constexpr int D = 128, KT = 64, QB = 32 * QW;
   constexpr int TILE = KT * D * 2;  // 16 KB
   constexpr int BUF = 2 * TILE;     // K | V
-  constexpr int NBUF = STAG ? 4 : (NW == 8 ? 3 : 2);
-  constexpr int PPW = 16 / NW;      // 1-KB K (and V) pieces per wave per tile
+  constexpr int NBUF = STAG || SPLIT ? 4 : (NW == 8 ? 3 : 2);
+  constexpr int PPW = 16 / QW;      // 1-KB K (and V) pieces per wave per tile
   __shared__ __attribute__((aligned(16))) char smem[NBUF * BUF];
 
   // same XCD-major (query block, head, sequence) walk as flash_fwd_kernel
@@ -472,7 +478,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
   const int lin = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
   const int xcd = lin % 8, q8 = nwg / 8, r8 = nwg % 8;
   int sid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + lin / 8;
-  if (PAIR && p.lpt) {
+  if ((PAIR || SPLIT) && p.lpt) {
     // the (sequence, head) units split evenly over the XCDs (units % 8 == 0, checked by the host);
     // on each XCD, pair group 0 of every unit, then group 1, ...: the mixed-duration workgroups of
     // a ragged pair split no longer alternate, so greedy dispatch cannot strand a long one at the end
@@ -520,7 +526,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
   const int kv_len = p.ctx_k[b];
   const int hk = h / (p.Hq / p.Hkv);
   const int tid = threadIdx.x, lane = tid & 63, lq = lane & 31, hi = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w_all = __builtin_amdgcn_readfirstlane(tid >> 6), w = SPLIT ? w_all & 3 : w_all, part = SPLIT ? w_all >> 2 : 0;
   int my_q, q_pos, w_kmax;
   bool q_valid, w_any;
   auto set_block = [&](const int q0_) DAB_ALWAYS_INLINE {
@@ -602,7 +608,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
     const size_t base = (((size_t)blk * p.Hkv + hk) * p.block_size + (k0 % p.block_size)) * D;
     const auto rk = __builtin_amdgcn_make_buffer_rsrc((void*)(p.k_cache + base), (short)0, nvalid * D * 2, 0x00020000);
     const auto rv = __builtin_amdgcn_make_buffer_rsrc((void*)(p.v_cache + base), (short)0, nvalid * D * 2, 0x00020000);
-    char* kdst = smem + buf * BUF;
+    char* kdst = smem + (2 * part + buf) * BUF;
 #pragma unroll
     for (int j = 0; j < PPW; ++j) {
       const int i = PPW * w + j;
@@ -628,7 +634,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
 
   // Loop-invariant LDS addresses (the tile buffer and the key block go in the instruction offset).
   // K reads of k-step st: row lq (and 32 + lq: +8 KB), logical chunk 2 st + hi at (2 st + hi) ^ f(lq).
-  const unsigned smem0 = lds_addr(smem);
+  const unsigned smem0 = lds_addr(smem) + 2 * part * BUF;
   unsigned kadr[8];
   {
     const int fr = f128(lq);
@@ -932,7 +938,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
             float4, __builtin_amdgcn_raw_buffer_load_b128(cs_rs, cs_row * 512 + ((16 * st + 8 * hi) / 2 + e) * 16, 0, 0));
   };
   load_cs();
-  if (n_tiles > 0) issue(0, 0, blk_of(0));
+  if (part < n_tiles) issue(part, 0, blk_of(part));
   // PAIR: the next block's Q is loaded one block ahead into qfB (raw; RoPE is applied when it
   // becomes the current block's, at the seam).  Loading qf itself at the seam made hipcc wait for the
   // in-flight DMA before every step's MFMAs.
@@ -950,11 +956,47 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_d128_kernel(Fl
   if constexpr (PAIR) {
     if (next_blk(0) >= 0) load_qB(blk_qb(next_blk(0)));
   }
-  if constexpr (NBUF >= 3) {
+  if constexpr (NBUF >= 3 && !SPLIT) {
     if (n_tiles > 1) issue(1, 1, blk_of(1));
   }
   apply_rope();
-  if constexpr (NBUF >= 3) {
+  if constexpr (SPLIT) {
+    // one barrier a step: this wave's pieces of its group's tile, then everyone's, and everyone past the last step's reads
+    for (int t = part, buf = 0; t - part < n_tiles; t += 2, buf ^= 1) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      if (t + 2 < n_tiles) issue(t + 2, buf ^ 1, blk_of(t + 2));
+      const int k0 = t * KT;
+      if (t < n_tiles && w_any && k0 <= w_kmax) compute(k0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int adv = buf ? -BUF : BUF;
+        kadr[i] += adv;
+        vadr[i] += adv;
+      }
+    }
+    // the second group's sums [wave][register][lane], and its running maximum and row sum behind them
+    float* const sums = reinterpret_cast<float*>(smem) + w * 64 * 64 + lane;
+    float* const ml = reinterpret_cast<float*>(smem) + 4 * 64 * 64 + w * 128 + lane;
+    __syncthreads();
+    if (part == 1) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(16 * db + r) * 64] = o[db][r];
+      ml[0] = m_run;
+      ml[64] = l_run;
+    }
+    __syncthreads();
+    if (part == 1) return;
+    const float m1 = ml[0], m = fmaxf(m_run, m1);
+    const float f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+    l_run = l_run * f0 + ml[64] * f1;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * f0 + sums[(16 * db + r) * 64] * f1;
+  } else if constexpr (NBUF >= 3) {
     const bool g1 = STAG && w >= 4;  // wave-uniform
     bf16x8 pp[4];                    // STAG group 1: P of the pending tile (in the previous buffer)
     bool pend = false;
@@ -2268,13 +2310,26 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
       else hipLaunchKernelGGL((flash_q64_kernel<false>), gq, dim3(256), 0, s, prm);
       return hipGetLastError();
     }
+    // up to 384 query blocks of at least four a sequence, or 512 of at least eight: the keys of each split over two wave groups (SPLIT), heaviest blocks
+    // first.  us, one block or pair a workgroup -> split, 32 heads: 400 tokens 16.3 -> 15.5, 700 23.6 -> 19.6, 1093 36.0 ->
+    // 26.4, 1500 56.0 -> 38.1, 2000 66.7 -> 57.1, 2 x 600 26.6 -> 24.5, 3 x 500 27.8 -> 27.4, 2 x 900 40.5 -> 37.0, 2 x
+    // 1000 43.3 -> 40.1; not taken 200 11.6 -> 11.9 (the second group's sums cost 1.7), 4 x 300 18.2 -> 23.1, 4 x 480 28.0 ->
+    // 30.7, 3 x 600 29.7 -> 32.0, 4 x 700 44.1 -> 48.7, 16 x 250 32.9 -> 50.8
+    const long blocks = (long)g32.x * Hq * batch;
+    if (causal && vpipe && !std::getenv("DAB_FLASH_PAIR") && g32.x >= 4 && blocks <= (g32.x >= 8 ? 512 : 384)) {
+      prm.lpt = ((long)Hq * batch) % 8 == 0;
+      hipLaunchKernelGGL((flash_d128_kernel<true, true, 8, false, false, false, false, false, false, true>), g32, dim3(512), 0, s,
+                         prm);
+      return hipGetLastError();
+    }
     // causal: one workgroup per (long, short) query-block pair by default (+8 % on 16 x 1024,
     // bit-identical: profiles/attn_vpipe_r5.md), unless the pairs would leave CUs idle (a single
     // prompt of <= 1k tokens: 1 x 1024 37.2 vs 42.8 us one block per workgroup,
-    // profiles/attn_prefill_shape_r6.md); DAB_FLASH_PAIR=0 / 1 forces either
+    // profiles/attn_prefill_shape_r6.md) or all blocks find a slot at once (512: 4 x 300 20.5 -> 18.2 one block a
+    // workgroup, 4 x 400 28.2 -> 24.7, 3 x 600 32.9 -> 29.7; 3 x 1000 52.3 -> 66.4); DAB_FLASH_PAIR=0 / 1 forces either
     const char* pe = std::getenv("DAB_FLASH_PAIR");
     const long pair_wgs = (long)(((max_seqlen_q + 127) / 128 + 1) / 2) * Hq * batch;
-    const bool pair = pe && pe[0] == '1' ? true : !(pe && pe[0] == '0') && pair_wgs >= 256;
+    const bool pair = pe && pe[0] == '1' ? true : !(pe && pe[0] == '0') && pair_wgs >= 256 && blocks > 512;
     if (causal && vpipe && pair) {
       // G = 2 pairs per workgroup (1 when that leaves < 1024 workgroups), walked heaviest-first
       // (lpt).  Large G made the workgroups few and long: the headline's prefill step (33 prompts of
