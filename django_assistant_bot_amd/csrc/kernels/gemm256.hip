@@ -56,6 +56,7 @@ struct G256 {
   int M, N, K;
   long lda, ldb, ldc, ldr;
   int gm;  // tile rows per group of the grouped tile order
+  int cn;  // tile columns per block of it
   int rows_b;  // SHUF: rows of the B copy (>= N)
   int bgrp;    // SHUF: row blocks per group of the B copy, 1 or 8 (shuffle_weights(w, 8))
   // G_CAND (index threshold search, see gemm.hip EPI_CANDIDATES): filtered scores >= thr[m] are
@@ -118,14 +119,17 @@ static_assert(2 * kBuf + kCandExtra <= 163840, "LDS");
 
 }  // namespace
 
-// grouped tile order: tile id -> (m0, n0), column-major inside groups of GM tile rows
-__device__ __forceinline__ void tile_of(int sid, int tiles_m, int tiles_n, int GM, int& m0, int& n0) {
-  const int per_group = GM * tiles_n;
+// grouped tile order: tile id -> (m0, n0), blocks of CN tile columns one after the other, column-major inside groups of GM
+// tile rows of one
+__device__ __forceinline__ void tile_of(int sid, int tiles_m, int tiles_n, int GM, int CN, int& m0, int& n0) {
+  const int block = sid / (tiles_m * CN), first_n = block * CN;
+  sid -= block * tiles_m * CN;
+  const int per_group = GM * min(CN, tiles_n - first_n);
   const int grp = sid / per_group, first_m = grp * GM;
   const int gsz = min(GM, tiles_m - first_m);
   const int inner = sid - grp * per_group;
   m0 = (first_m + inner % gsz) << 8;
-  n0 = (inner / gsz) << 8;
+  n0 = (first_n + inner / gsz) << 8;
 }
 
 template <int EPI, bool BIAS, bool RES, bool SHUF = false, bool STAMP = false, int SAUX = 0>
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
   int sid = cstart + l;
   if (sid >= cend) return;  // whole workgroup: uniform
   int m0, n0;
-  tile_of(sid, tiles_m, tiles_n, p.gm, m0, n0);
+  tile_of(sid, tiles_m, tiles_n, p.gm, p.cn, m0, n0);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
     const int nsid = sid + nper;
     const bool more = nsid < cend;
     int nm0 = m0, nn0 = n0;
-    if (more) tile_of(nsid, tiles_m, tiles_n, p.gm, nm0, nn0);
+    if (more) tile_of(nsid, tiles_m, tiles_n, p.gm, p.cn, nm0, nn0);
     const __amdgpu_buffer_rsrc_t nA = rsrc_a(nm0), nB = rsrc_b(nn0);
     // G_CAND: a tile whose rows 128-255 are all past M (97-128 queries, or the last row tile of a
     // larger batch) skips their MFMAs (the accumulators stay zero; their thresholds are +inf).
@@ -737,6 +741,7 @@ int gemm256_candidates(const void* A, long lda, const void* B, long ldb, int M, 
   p.lda = lda;
   p.ldb = ldb;
   p.gm = 4;
+  p.cn = (N + 255) / 256;
   p.row_group = row_group;
   p.q_group = q_group;
   p.thr = thr;
@@ -770,6 +775,7 @@ int gemm256_candidates_stamped(const void* A, long lda, const void* B, int M, in
   p.lda = lda;
   p.ldb = K;
   p.gm = 4;
+  p.cn = (N + 255) / 256;
   p.thr = thr;
   p.cnt = cnt;
   p.cand_val = cand_val;
@@ -808,6 +814,7 @@ int gemm256_stamped(const void* A, long lda, const void* B, void* C, const void*
   p.ldr = N;
   p.rows_b = N;
   p.gm = 4;
+  p.cn = (N + 255) / 256;
   p.stamps = (u32x4*)stamps;
   p.stamp_tiles = stamp_tiles;
   int dev = 0, cus = 256;
@@ -880,7 +887,15 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const int tiles = ((M + 255) / 256) * (N / 256);
-  p.gm = 4;  // grouped tile order: 4 tile rows per group
+  // Tile order.  A of half the Infinity Cache (256 MB) and more has left it when the projection starts, since its producer
+  // moved as much again, and with a short K every K-tile is a first touch from HBM.  Blocks of 3 columns, 8 tile rows each,
+  // keep some 11 row panels under way on an XCD instead of 4; the panels' second and third reads find them on the chip.  us
+  // behind a LayerNorm that wrote A, 4 rows x all columns -> this: (108800, 2304, 768) 439 -> 355, (95000, 2304, 768) 345 ->
+  // 295, (80000, 2304, 1024) 368 -> 313, (108800, 3072, 768) 532 -> 473, (108800, 1792, 768) 300 -> 311; below that
+  // (80000, 2304, 768) 235 -> 240.  The GELU epilogue covers it: up of 108800 rows 553 us either way.
+  const bool far_a = K <= 1024 && !b_shuf && !residual && epilogue == G_NONE && (long)M * K * 2 >= (128L << 20);
+  p.gm = far_a ? 8 : 4;
+  p.cn = far_a ? 3 : N / 256;
   // persistent: one workgroup (128 KB of LDS) per CU walks a strided tile list
   const int nwg = tiles > cus ? cus : tiles;
   const bool hb = bias != nullptr, hr = residual != nullptr;
