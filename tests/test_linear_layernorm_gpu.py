@@ -9,8 +9,8 @@ DEV = "cuda"
 
 # ends of the four ranges of the rule (tiles of 64 or 128, two or three slices), whole tiles and one row more or less, K whose
 # slices are not equal
-SIZES = [(705, 768, 3072, 3), (896, 768, 3072, 3), (1024, 768, 3072, 2), (961, 768, 2624, 2), (1152, 768, 3072, 2), (1281, 768, 3072, 3),
-         (1792, 768, 3072, 3), (1921, 768, 3072, 2), (2688, 768, 1536, 2), (2048, 384, 1536, 2), (2689, 384, 1600, 3),
+SIZES = [(705, 768, 3072, 3), (896, 768, 3072, 3), (1024, 768, 3072, 2), (897, 768, 2624, 2), (1344, 768, 3072, 2), (1345, 768, 3072, 3),
+         (1792, 768, 3072, 3), (1921, 768, 3072, 2), (2688, 768, 1536, 2), (1793, 384, 1536, 2), (2689, 384, 1600, 3),
          (5376, 384, 1536, 2), (575, 1024, 4096, 3), (1280, 1024, 4096, 3), (2048, 1024, 4096, 2)]
 
 
