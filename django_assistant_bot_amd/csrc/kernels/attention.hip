@@ -2386,6 +2386,12 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
       (long)max_seqlen_q * kv_stride_tok * 2 < (1L << 31) && !std::getenv("DAB_ENC_PERSIST") && !std::getenv("DAB_ENC_W5"))
     return flash_packed64(q, q_stride_tok, q_stride_head, k, v, kv_stride_tok, kv_stride_head, out, o_stride_tok, o_stride_head,
                           cu_q, batch, max_seqlen_q, Hq, Hkv, scale, s);
+  // causal prompts over the cache: the same form for any length (attention_packed.hip has both sides), where its vectors fit
+  if (D == 64 && paged && causal && scale > 0.f && (q_stride_tok | q_stride_head) % 8 == 0 &&
+      (o_stride_tok | o_stride_head) % 4 == 0 && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0 &&
+      (uintptr_t)out % 8 == 0)
+    return flash_paged64(q, q_stride_tok, q_stride_head, k_cache, v_cache, block_tables, max_blocks, block_size, out, o_stride_tok,
+                         o_stride_head, cu_q, ctx_k, batch, max_seqlen_q, Hq, Hkv, scale, s);
   const bool wide = D == 128 && max_seqlen_q > 64;
   // the 5-waves-per-SIMD encoder variant by default (3 % faster on the embed bench's packed batch,
   // bit-identical: profiles/embed_r5.md); DAB_ENC_W5=0 selects the unbounded-register kernel

@@ -69,6 +69,9 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
                     const OutputGate* gate = nullptr);  // gate: D = 128, paged, with sink or slopes, over all keys
 // attention_packed.hip: bidirectional self-attention over packed sequences, heads of 64
 bool flash_packed64_wins(long units, int max_len);
+int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, const void* v_cache, const int* tables, int max_blocks,
+                  int block_size, void* out, long o_tok, long o_head, const int* cu, const int* ctx, int batch, int max_q, int Hq,
+                  int Hkv, float scale, hipStream_t s);
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
                    long o_tok, long o_head, const int* cu, int batch, int max_len, int Hq, int Hkv, float scale, hipStream_t s);
 int decode_partition_of(int part_size, int longest, int items, int max_parts);
