@@ -887,14 +887,19 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const int tiles = ((M + 255) / 256) * (N / 256);
-  // Tile order.  A of half the Infinity Cache (256 MB) and more has left it when the projection starts, since its producer
+  // Tile order.  Short K: A of half the Infinity Cache (256 MB) and more has left it when the projection starts, since its producer
   // moved as much again, and with a short K every K-tile is a first touch from HBM.  Blocks of 3 columns, 8 tile rows each,
   // keep some 11 row panels under way on an XCD instead of 4; the panels' second and third reads find them on the chip.  us
   // behind a LayerNorm that wrote A, 4 rows x all columns -> this: (108800, 2304, 768) 439 -> 355, (95000, 2304, 768) 345 ->
   // 295, (80000, 2304, 1024) 368 -> 313, (108800, 3072, 768) 532 -> 473, (108800, 1792, 768) 300 -> 311; below that
   // (80000, 2304, 768) 235 -> 240.  The GELU epilogue covers it: up of 108800 rows 553 us either way.
   const bool far_a = K <= 1024 && !b_shuf && !residual && epilogue == G_NONE && (long)M * K * 2 >= (128L << 20);
-  p.gm = far_a ? 8 : 4;
+  // Otherwise groups of 4 tile rows; where there are many columns, even ones of up to 6: the 32 tiles an XCD runs at once are
+  // then 6 row panels and 5-6 column panels, the fewest, and no group of one row is left over that reads 32.  us a step of
+  // Llama-3-8B (gate_up, 102-112 columns), 4 rows -> these: 1093 tokens (4 + 1 -> 5) 16889 -> 16660, 3000 36434 -> 36171, 11,000
+  // 124055 -> 122744, 7900 83166 -> 83659; Llama-3.2-1B (64 columns) 9600 16477 -> 16476.
+  const int tm = (M + 255) / 256, groups = (tm + 5) / 6;
+  p.gm = far_a ? 8 : N / 256 >= 64 ? (tm + groups - 1) / groups : 4;
   p.cn = far_a ? 3 : N / 256;
   // persistent: one workgroup (128 KB of LDS) per CU walks a strided tile list
   const int nwg = tiles > cus ? cus : tiles;

@@ -1,8 +1,10 @@
-"""Projections whose input is larger than half the Infinity Cache walk their tiles in blocks of columns: the same bits."""
+"""The tile orders of the 256 x 256 GEMM (blocks of columns for an input larger than half the Infinity Cache, even groups of rows
+for many columns): every tile once, the same bits."""
 import pytest
 import torch
 
 from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.ops.kernels import gemm256
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -27,3 +29,18 @@ def test_every_tile_once(M, N):
     exp = a[at].double() @ w.double().t() + b.double()
     slack = K * 2.0 ** -23 * (a[at].double().abs() @ w.double().abs().t() + b.double().abs())
     assert ((out[at].double() - exp).abs() <= 2.0 ** -8 * exp.abs() + slack).all()
+
+
+# one group of 1 and of 6 tile rows, 4 + 4, 5 + 5, 5 + 5 + 3; more than 256 workgroups and fewer
+@pytest.mark.parametrize("M", [1, 1281, 1793, 2305, 3100])
+@pytest.mark.parametrize("cols", [64, 67])
+def test_even_groups_of_rows(M, cols):
+    K, N = 128, 256 * cols
+    g = torch.Generator(device=DEV).manual_seed(M + cols)
+    a = torch.empty(M, K, device=DEV, dtype=torch.bfloat16).normal_(generator=g)
+    w = ops.shuffle_weights(torch.empty(N, K, device=DEV, dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g))
+    for epi in (ops.EPI_NONE, ops.EPI_SWIGLU8):
+        out = gemm256(a, w, epilogue=epi, shuffled=True)
+        at = N // 512 * 256  # (halves of the weights' rows: groups of 4 tile rows)
+        parts = [gemm256(a, x, epilogue=epi, shuffled=True) for x in (w[:at], w[at:])]
+        assert torch.isfinite(out.float()).all() and torch.equal(out, torch.cat(parts, 1))
