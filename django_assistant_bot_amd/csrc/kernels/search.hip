@@ -173,10 +173,11 @@ struct RankShared {
   uint32_t hist[RK_BINS];
   uint32_t rank[RK_FEW];
   uint32_t lo[SEL_NT / 64], hi[SEL_NT / 64], total[SEL_NT / 64];
-  uint32_t bin, n;
+  uint32_t bin, in_bin, upto, n;
 };
 
-// The bin in which the count from the top reaches `kept` (of at least that many entries), for all threads.
+// The bin in which the count from the top reaches `kept`, for all threads (the last one where there are fewer entries); in_bin:
+// the entries in it, upto: those and the ones above.
 template <int CAP>
 __device__ __forceinline__ uint32_t cut_bin(RankShared<CAP>& sh, uint32_t kept) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -190,7 +191,11 @@ __device__ __forceinline__ uint32_t cut_bin(RankShared<CAP>& sh, uint32_t kept) 
   if (lane == 63) sh.total[w] = incl;
   __syncthreads();
   for (int j = 0; j < w; ++j) incl += sh.total[j];
-  if (incl - h < kept && kept <= incl) sh.bin = RK_BINS - 1 - tid;
+  if (incl - h < kept && (kept <= incl || tid == RK_BINS - 1)) {
+    sh.bin = RK_BINS - 1 - tid;
+    sh.in_bin = h;
+    sh.upto = incl;
+  }
   __syncthreads();
   return sh.bin;
 }
@@ -215,6 +220,36 @@ __device__ __forceinline__ void block_range(RankShared<CAP>& sh, uint32_t& lo, u
 
 // Shift after which steps of (key - lo) fall into RK_BINS bins: monotone for any scores.  (__clz(0) = 32)
 __device__ __forceinline__ int bin_shift(uint32_t lo, uint32_t hi) { return max(0, 22 - __clz(hi - lo)); }
+
+// A bound in lo .. hi that at least `need` of the entries reach (all of them, where they are fewer) and at most `most` (need <=
+// most).  each(f) hands this thread's entries to f; those of the block differ from each other (ordered bits << 32 | ~place), so
+// the histograms of ever narrower ranges end at the latest with one entry a bin.  Leaves hist cleared.
+template <int CAP, typename F>
+__device__ __forceinline__ unsigned long long bound_of(RankShared<CAP>& sh, unsigned long long lo, unsigned long long hi, uint32_t need,
+                                       uint32_t most, F each) {
+  for (uint32_t above = 0;;) {
+    const int shift = max(0, 54 - __clzll((long long)(hi - lo)));  // (hi - lo) >> shift < RK_BINS
+    sh.hist[threadIdx.x] = 0;
+    __syncthreads();
+    each([&](unsigned long long e) {
+      const int bin = e >= lo && e <= hi ? (int)((e - lo) >> shift) : -1;
+      const unsigned long long in = __ballot(bin >= 0);
+      if (!in) return;
+      // the lanes of one bin by one atomic: 64 on an address are 64 steps (equal scores)
+      const int leader = __ffsll((long long)in) - 1, first = __builtin_amdgcn_readlane(bin, leader);
+      const unsigned long long same = __ballot(bin == first);
+      if (bin >= 0 && (bin != first || (int)(threadIdx.x & 63) == leader))
+        atomicAdd(&sh.hist[bin], bin == first ? (uint32_t)__popcll(same) : 1u);
+    });
+    __syncthreads();
+    const uint32_t bin = cut_bin(sh, need - above);
+    lo += (unsigned long long)bin << shift;
+    sh.hist[threadIdx.x] = 0;
+    if (above + sh.upto <= most || shift == 0) return lo;
+    above += sh.upto - sh.in_bin;
+    hi = min(hi, lo + ((1ull << shift) - 1));
+  }
+}
 
 // Bitonic, greatest first; P a power of two, at least 64.  A wave's 64 consecutive pairs lie in its own 128 entries where
 // the stride is 64 or less: no workgroup barrier there.
@@ -256,7 +291,23 @@ __device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uin
     if (at < RK_MANY) sh.few[at] = e;
   }
   __syncthreads();
-  const int m = (int)sh.n;
+  int m = (int)sh.n;
+  if (m > RK_MANY) {  // (equal scores in one bin): cut among them by their rows
+    const unsigned long long bound =
+        bound_of(sh, (unsigned long long)lo << 32, ((unsigned long long)hi << 32) | ~0u, (uint32_t)kept,
+                 (uint32_t)(kept <= RK_FEW ? RK_FEW : RK_MANY), [&](auto f) __attribute__((always_inline)) {
+                   for (int i = tid; i < c; i += SEL_NT) f(sh.key[i]);
+                 });
+    if (tid == 0) sh.n = 0;
+    __syncthreads();
+    for (int i = tid; i < c; i += SEL_NT) {
+      const unsigned long long e = sh.key[i];
+      const int at = wave_append(&sh.n, e >= bound);
+      if (at >= 0 && at < RK_MANY) sh.few[at] = e;
+    }
+    __syncthreads();
+    m = (int)sh.n;
+  }
   if (m <= RK_FEW) {  // every entry against all m, m / parts of them a thread
     const int E = (m + 63) & ~63, parts = SEL_NT / E, part = tid / E, e = tid - part * E;
     const bool own = part < parts && e < m;
@@ -282,7 +333,7 @@ __device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uin
     if (own && part == 0 && (int)sh.rank[e] < kept) emit((int)sh.rank[e], mine, id, doc);
     return;
   }
-  unsigned long long* list = m <= RK_MANY ? sh.few : sh.key;
+  unsigned long long* list = m <= RK_MANY ? sh.few : sh.key;  // (else: a list that names a row more than once)
   const int n = m <= RK_MANY ? m : c;
   int P = 64;
   while (P < n) P <<= 1;
@@ -302,8 +353,8 @@ __device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uin
 // A search's lists hold 1-2 thousand entries for some 250 hits.  A histogram of 1024 bins between the list's least and
 // greatest score leaves little more than the hits (bins are equal steps of the ordered bits: monotone for any scores),
 // and up to 512 entries are ranked by counting the greater ones: one chain of LDS reads instead of the 66 steps of a
-// bitonic sort of the list.  Where more remain (k above some 400, many near-equal scores) they are sorted, or the whole
-// list where they are more than 2048.  Lists above 4096 are radix-selected.  With the ids and documents in the same launch 7.9 us for 1,300
+// bitonic sort of the list.  Where more remain (k above some 400, many near-equal scores) they are sorted, up to 2048, or
+// cut by score and row to as many first.  Lists above 4096 are radix-selected.  With the ids and documents in the same launch 7.9 us for 1,300
 // candidates of one query and 9.8 for 128 queries (sorted whole: 22 and 31; radix select of 16,000 and five
 // element-wise launches behind it: 61 and 91).
 __global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restrict__ cand_val,
@@ -372,34 +423,36 @@ int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const 
 }
 
 constexpr int TH_CAND = 8192;   // candidates held in LDS, and the scores of a row that need no parts
-constexpr int TH_PARTS = 4096;  // parts looked into
-constexpr int TH_HELD = 16;     // 16-B vectors of part maxima a thread keeps in registers between its two looks
+constexpr int TH_PARTS = 4096;  // parts looked into (4 k at most, or 1024)
+constexpr int TH_HELD = 16;     // 16-B vectors of part maxima a thread keeps in registers between its looks
+constexpr int TH_FEW = 2;       // threads with a score that passes, as a multiple of k, from which their maxima give the bound
 
 // The k best of every row of scores [n] -> score, item id, document id, best first, equal scores in row order; -inf / -1
 // where fewer rows pass the filters.  One workgroup a row; parts: the greatest ordered bits of every 16 scores.
 //
 // The k-th greatest of maxima over disjoint parts is a bound that at least k scores reach, and where the parts are many
 // times k few more do.  So the scores themselves are read only in the parts that reach it: 64 KB of maxima and some 20 KB
-// of scores for 250 of 262,144, and the rest is the ranking of about 300 candidates.  The bound is the lower end of the
-// bin of a 1024-bin histogram of the threads' maxima in which the count from the top reaches k (parts of up to 1024 threads).
-// Rows of up to 8192 scores are ranked as they are.  Where more than 8192 scores reach the bound (k near the number of
-// parts that pass the filters, many equal scores) the row is radix-selected.
+// of scores for 250 of 262,144, and the rest is the ranking of about 300 candidates.  The bound is the lower end of a
+// bin of a 1024-bin histogram: of the threads' maxima, one atomic each, where 2 k threads have a score that passes, else (k
+// above 500, up to 128 k rows, groups that lie together) of the parts' own, (key, place) in as many rounds as leave 2 k or
+// 1024 of them.  Where those hold more than 8192 scores that reach it (k near the number of parts, equal scores) the bound is
+// raised over these scores in the same way.  Rows of up to 8192 scores are ranked as they are.
 //
 // us, against a radix select by one workgroup a query (up to 32,768 scores) or selection in chunks and a merge, and the
 // ids' launch: 42 queries of 31,098 rows 9.8 (188), 4 of 60,001 9.5 (34), 10 of 142,939 10.1 (40); 1 of 1,000,003 17.3.
+// From the parts, against the same: 250 of 12,000 13.8 (54), 500 of 30,000 21 (115), 1000 of 50,000 29 (85), 1024 of 1,000,000
+// 75 (244), 250 of 600,000 with 12,000 that pass together 21 (66); all scores equal, 1000 of 60,000 43 (62).  (A row that the
+// threads' bound alone did not cut was radix-selected whole by its workgroup: 1024 of 1,000,000 some 2,800.)
 __global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restrict__ scores, int n,
                                                           const uint32_t* __restrict__ parts, int ldp, int k,
                                                           const int64_t* __restrict__ row_ids,
                                                           const int64_t* __restrict__ row_docs,
                                                           float* __restrict__ out_vals, int64_t* __restrict__ out_ids,
                                                           int64_t* __restrict__ out_docs) {
-  __shared__ union {
-    struct {
-      RankShared<TH_CAND> list;
-      uint32_t part[TH_PARTS];
-      uint32_t n_part, n_cand;
-    };
-    SelShared sel;
+  __shared__ struct {
+    RankShared<TH_CAND> list;
+    uint32_t part[TH_PARTS];
+    uint32_t n_part, n_cand;
   } sh;
   const int row = blockIdx.x, tid = threadIdx.x;
   const float* s = scores + (size_t)row * n;
@@ -413,6 +466,7 @@ __global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restric
     out_ids[i] = hit ? id : -1;
     out_docs[i] = hit ? doc : -1;
   };
+  auto entry = [](uint32_t key, int at) { return ((unsigned long long)key << 32) | (uint32_t)~at; };
   sh.list.hist[tid] = 0;
   if (tid < RK_FEW) sh.list.rank[tid] = 0;
   if (tid == 0) {
@@ -422,23 +476,23 @@ __global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restric
   }
   uint32_t lo = ~0u, hi = 0u;
   // a score at or above the bound takes a slot (n % 4 == 0: whole vectors)
-  auto take = [&](int i, uint32_t bound) {
+  auto take = [&](int i, unsigned long long bound) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(s + i);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const uint32_t key = float_key(v[e]);
-      const int at = wave_append(&sh.n_cand, key >= bound && key != kNegInfKey);
+      const unsigned long long x = entry(key, i + e);
+      const int at = wave_append(&sh.n_cand, x >= bound && key != kNegInfKey);
       if (at >= 0 && at < TH_CAND) {
-        sh.list.key[at] = ((unsigned long long)key << 32) | (uint32_t)~(i + e);
+        sh.list.key[at] = x;
         lo = min(lo, key);
         hi = max(hi, key);
       }
     }
   };
-  bool over = false;
   if (n <= TH_CAND) {
     __syncthreads();
-    for (int i = 4 * tid; i < n; i += 4 * SEL_NT) take(i, 0u);
+    for (int i = 4 * tid; i < n; i += 4 * SEL_NT) take(i, 0ull);
   } else {
     const u32x4* pv = reinterpret_cast<const u32x4*>(parts + (size_t)row * ldp);
     const int np = (n + 15) / 16, nv = (np + 3) / 4;
@@ -459,50 +513,89 @@ __global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restric
       const u32x4 x = look(v);
       m = max(max(m, max(x[0], x[1])), max(x[2], x[3]));
     }
-    // the bound: of the threads with a score that passed
-    uint32_t mlo = m > kNegInfKey ? m : ~0u, mhi = m;
+    auto each_vector = [&](int from, auto f) __attribute__((always_inline)) {
+#pragma unroll 4
+      for (int v = from + tid; v < nv; v += SEL_NT) f(look(v), v);
+    };
+    auto each_part = [&](auto f) __attribute__((always_inline)) {
+      each_vector(0, [&](const u32x4& x, int v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f(entry(x[e], 4 * v + e));
+      });
+    };
     const int live = __syncthreads_count(m > kNegInfKey);
-    block_range(sh.list, mlo, mhi);
-    uint32_t bound = kNegInfKey + 1;
-    if (live >= k) {
-      const int shift = bin_shift(mlo, mhi);
-      if (m > kNegInfKey) atomicAdd(&sh.list.hist[(m - mlo) >> shift], 1u);
-      __syncthreads();
-      bound = mlo + (cut_bin(sh.list, (uint32_t)k) << shift);
-      sh.list.hist[tid] = 0;
-    }
-    auto keep = [&](const u32x4& x, int v) {
+    unsigned long long top = entry(m, 0), bound = 0;
+    auto keep = [&](const u32x4& x, int v, auto reaches) __attribute__((always_inline)) {
+      if (!__ballot(max(max(x[0], x[1]), max(x[2], x[3])) >= (uint32_t)(bound >> 32))) return;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int at = wave_append(&sh.n_part, x[e] >= bound);
+        const int at = wave_append(&sh.n_part, reaches(x[e], 4 * v + e));
         if (at >= 0 && at < TH_PARTS) sh.part[at] = 4 * v + e;
       }
     };
+    auto by_key = [&](uint32_t key, int) { return key >= (uint32_t)(bound >> 32); };
+    auto by_entry = [&](uint32_t key, int at) { return entry(key, at) >= bound; };
+    if (live >= TH_FEW * k) {
+      uint32_t mlo = m > kNegInfKey ? m : ~0u, mhi = m;
+      block_range(sh.list, mlo, mhi);
+      top = entry(mhi, 0);
+      const int shift = bin_shift(mlo, mhi);
+      if (m > kNegInfKey) atomicAdd(&sh.list.hist[(m - mlo) >> shift], 1u);
+      __syncthreads();
+      bound = (unsigned long long)(mlo + (cut_bin(sh.list, (uint32_t)k) << shift)) << 32;
+      sh.list.hist[tid] = 0;
 #pragma unroll
-    for (int j = 0; j < TH_HELD; ++j)
-      if (__ballot(max(max(held[j][0], held[j][1]), max(held[j][2], held[j][3])) >= bound)) keep(held[j], tid + j * SEL_NT);
-#pragma unroll 4
-    for (int v = tid + TH_HELD * SEL_NT; v < nv; v += SEL_NT) keep(look(v), v);
+      for (int j = 0; j < TH_HELD; ++j) keep(held[j], tid + j * SEL_NT, by_key);
+      each_vector(TH_HELD * SEL_NT, [&](const u32x4& x, int v) __attribute__((always_inline)) { keep(x, v, by_key); });
+    } else if (live) {
+      uint32_t mlo = ~0u, mhi = m;
+      each_vector(0, [&](const u32x4& x, int) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mlo = min(mlo, x[e] > kNegInfKey ? x[e] : ~0u);
+      });
+      block_range(sh.list, mlo, mhi);
+      top = entry(mhi, 0);
+      const unsigned long long least = entry(mlo, np - 1);
+      bound = bound_of(sh.list, least, top, (uint32_t)k, (uint32_t)max(2 * k, 1024), each_part);
+      if (bound == least) bound = (unsigned long long)(kNegInfKey + 1) << 32;  // all parts, perhaps fewer than k
+      each_vector(0, [&](const u32x4& x, int v) __attribute__((always_inline)) { keep(x, v, by_entry); });
+    }
     __syncthreads();
-    const int chosen = (int)sh.n_part;
-    over = chosen > TH_PARTS;
-    if (!over)
+    int chosen = (int)sh.n_part;
+    static_assert(TH_PARTS >= 4 * SEL_MAXK && TH_PARTS >= 1024, "room for the parts");
+    if (chosen > max(4 * k, 1024)) {  // the threads' bound says little
+      bound = bound_of(sh.list, entry((uint32_t)(bound >> 32), np - 1), top, (uint32_t)k, (uint32_t)max(2 * k, 1024), each_part);
+      if (tid == 0) sh.n_part = 0;
+      __syncthreads();
+      each_vector(0, [&](const u32x4& x, int v) __attribute__((always_inline)) { keep(x, v, by_entry); });
+      __syncthreads();
+      chosen = (int)sh.n_part;
+    }
+    auto each_chosen = [&](auto f) __attribute__((always_inline)) {
       for (int e = tid; e < 4 * chosen; e += SEL_NT) {
         const int i = 16 * (int)sh.part[e >> 2] + 4 * (e & 3);
-        if (i < n) take(i, bound);
+        if (i < n) f(i);
       }
+    };
+    bound = bound >> 32 << 32;
+    each_chosen([&](int i) { take(i, bound); });
+    __syncthreads();
+    if (sh.n_cand > TH_CAND) {  // to what rank_list ranks by counting, or sorts alone
+      bound = bound_of(sh.list, entry((uint32_t)(bound >> 32), n - 1), top, (uint32_t)k, (uint32_t)(k <= RK_FEW ? RK_FEW : RK_MANY), [&](auto f) __attribute__((always_inline)) {
+        each_chosen([&](int i) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(s + i);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f(entry(float_key(v[e]), i + e));
+        });
+      });
+      if (tid == 0) sh.n_cand = 0;
+      lo = ~0u, hi = 0u;
+      __syncthreads();
+      each_chosen([&](int i) { take(i, bound); });
+    }
   }
   __syncthreads();
   const int c = (int)sh.n_cand, kept = min(k, c);
-  if (over || c > TH_CAND) {
-    __syncthreads();  // (the counts are read: the union's other half is written next)
-    select_topk([&](int i) -> uint32_t { return float_key(s[i]); }, n, k, sh.sel);
-    for (int i = tid; i < k; i += SEL_NT) {
-      const int r = sh.sel.cand_idx[i];
-      emit(i, (unsigned long long)sh.sel.cand_key[i] << 32, row_ids[r], row_docs[r]);
-    }
-    return;
-  }
   for (int i = kept + tid; i < k; i += SEL_NT) emit(i, (unsigned long long)kNegInfKey << 32, -1, -1);
   if (kept) rank_list(sh.list, c, kept, lo, hi, row_ids, row_docs, emit);
 }

@@ -321,7 +321,7 @@ class VectorIndex:
             z = torch.full((nq, max(k, 0)), -1, dtype=torch.int64, device=self.device)
             return torch.full((nq, max(k, 0)), float("-inf"), device=self.device), z, z.clone()
         plain = allowed is None and doc_lt is None
-        if self._selects(nq, plain):
+        if self._selects(nq, plain, k):
             return self._selected_search(queries, k, q_groups, allowed, doc_lt)
         if self.device.type == "cuda" and plain and self.n >= self.threshold_min_rows and k <= 1024 and self.threshold_search:
             got = self._threshold_search(queries, k, q_groups)
@@ -335,15 +335,18 @@ class VectorIndex:
     # sample and its two launches, the ranking's and the host read (some 45 us) and writes 4 B a row and query, and one
     # workgroup a query looks through its maxima.  Threshold / selection, us, rows of 768: 1M and 1 query 298 / 258, 4: 299 /
     # 282, 8: 301 / 293, 16: 298 / 303; 600k and 16 213 / 196, 32: 210 / 207; 2M and 1 517 / 514, 4: 517 / 555.  Of 256: 1M
-    # and 16 143 / 129; of 1024: 1M and 8 368 / 369.
+    # and 16 143 / 129; of 1024: 1M and 8 368 / 369.  For more than 512 hits a bound takes longer than a threshold's list:
+    # 1000 of 600k and 4 queries 247 / 235, 1M and 1 342 / 337, 4: 339 / 360, 1.4M and 1 432 / 441, 4: 433 / 484.
     select_rows, select_scores = 1_500_000, 8_000_000
 
-    def _selects(self, nq: int, plain: bool) -> bool:
+    def _selects(self, nq: int, plain: bool, k: int = 1) -> bool:
         """Whether the scan writes the scores and their parts' maxima, and ``top_hits`` selects from them."""
         if not (self.threshold_search and self.frag and ops.scan_scores_ok(nq, (max(self.n, 4) + 3) // 4 * 4, self.dim)):
             return False
-        return (not plain or self.n < self.threshold_min_rows
-                or self.n <= self.select_rows and nq * self.n <= self.select_scores)
+        rows, scores = self.select_rows, self.select_scores
+        if k > 512:
+            rows, scores = 2 * rows // 3, 3 * scores // 8
+        return not plain or self.n < self.threshold_min_rows or self.n <= rows and nq * self.n <= scores
 
     def _selected_search(self, queries, k: int, q_groups, allowed, doc_lt):
         """Exact top-k in three launches and without a host read: unit queries, scores with the greatest of every 16 rows,

@@ -119,3 +119,61 @@ def test_search_by_selection_is_the_full_search(n, flt):
         assert torch.equal(gi >= 0, hit) and torch.equal(gd >= 0, hit)
         same = gi == ei  # (neighbours that close may change places)
         assert torch.equal(gd[same], ed[same]) and same.float().mean() > 0.97
+
+
+# n, k, rows that pass: together, one of so many, or values of so few kinds.  Fewer threads (64 rows each) than k see a score;
+# fewer parts (16 rows) than k do; more than 4096 parts or 8192 scores reach the threads' bound; equal scores fill them.
+FEW_THREADS = [(8_196, 250, "all", 1), (12_000, 250, "all", 1), (30_000, 500, "all", 1), (50_000, 1000, "all", 1),
+               (16_384, 1024, "all", 1), (100_000, 1024, "all", 1), (1_000_000, 1024, "all", 1), (1_300_000, 1000, "all", 1),
+               (100_000, 1000, "every", 4), (600_000, 250, "together", 12_000), (1_000_000, 1000, "together", 50_000),
+               (1_100_000, 500, "together", 20_000), (60_000, 1000, "kinds", 1), (60_000, 250, "kinds", 3),
+               (1_100_000, 700, "kinds", 1), (400_000, 1024, "kinds", 400)]
+
+
+def _few_threads(n, k, kind, arg):
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    s = torch.randn(3, n, device=DEV, generator=g) * 0.05
+    if kind == "every":
+        s[:, torch.arange(n, device=DEV) % arg != 1] = float("-inf")
+    elif kind == "together":
+        s[:, : n // 3] = float("-inf")
+        s[:, n // 3 + arg:] = float("-inf")
+    elif kind == "kinds":
+        s = torch.randint(0, arg, (3, n), device=DEV, generator=g).float() - arg // 2
+    return s
+
+
+@pytest.mark.parametrize("n,k,kind,arg", FEW_THREADS)
+def test_top_hits_where_few_threads_see_a_score(n, k, kind, arg):
+    s = _few_threads(n, k, kind, arg)
+    ids, docs = torch.arange(n, device=DEV) + 5, torch.arange(n, device=DEV) // 3
+    vals, got, gdocs = ops.top_hits(s, _parts(s), k, ids, docs)
+    at = torch.argsort(-_key(s), dim=1, stable=True)[:, :k]  # (equal scores in row order)
+    assert torch.equal(vals, s.gather(1, at))
+    assert torch.equal(got, torch.where(torch.isinf(vals), -1, at + 5)) and torch.equal(gdocs, torch.where(torch.isinf(vals), -1, at // 3))
+
+
+@pytest.mark.parametrize("n,k,kind,arg", FEW_THREADS)
+def test_top_hits_costs_no_more_than_the_general_selection(n, k, kind, arg):
+    """One workgroup that goes over a whole row again and again took up to ten times as long as the selection in chunks."""
+    s = _few_threads(n, k, kind, arg)
+    p, ids = _parts(s), torch.arange(n, device=DEV)
+
+    def us(f):
+        for _ in range(3):
+            f()
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        torch.cuda.synchronize()
+        a.record()
+        for _ in range(20):
+            f()
+        b.record()
+        b.synchronize()
+        return 50 * a.elapsed_time(b)
+
+    def general():
+        vals, rows = ops.topk_rows(s, k)
+        ops.hit_ids(vals, rows, ids, ids)
+    new, old = min(us(lambda: ops.top_hits(s, p, k, ids, ids)) for _ in range(3)), min(us(general) for _ in range(3))
+    print(f"{n} {k} {kind} {arg}: {new:.1f} us, general {old:.1f}")
+    assert new <= 1.15 * old
