@@ -75,7 +75,7 @@ def main(rows=1_000_000, dim=768, k=250):
     res["kb_ms"] = med(lambda: loop.run_until_complete(kb.search_documents("q", q, 5, 5)))
     res["service_over_raw"] = round(res["service_ms"] / res["raw_ms"], 3)
     res["kb_over_raw"] = round(res["kb_ms"] / res["raw_ms"], 3)
-    res["threshold_searches"] = idx.stats["threshold_searches"]
+    res["threshold_searches"], res["selected_searches"] = idx.stats["threshold_searches"], idx.stats.get("selected_searches", 0)
     print(json.dumps({k2: (round(v, 3) if isinstance(v, float) else v) for k2, v in res.items()}), flush=True)
 
 

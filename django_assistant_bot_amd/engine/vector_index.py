@@ -353,8 +353,7 @@ class VectorIndex:
         selection.  (The bound below which parts are not looked into is the k-th greatest of those maxima.)"""
         q, qg, allow, n = self._query(queries, q_groups, allowed, doc_lt)
         scores, parts = ops.scores_and_parts(q, self.vecs, n, self.row_group[:n], qg, allow)
-        if self.n >= self.threshold_min_rows and allow is None:
-            self.stats["threshold_searches"] += 1
+        self.stats["selected_searches"] = self.stats.get("selected_searches", 0) + 1
         return ops.top_hits(scores, parts, min(k, n, 1024), self.row_ids, self.row_docs)
 
     def _sample_rank(self, k: int) -> int:

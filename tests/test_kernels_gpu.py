@@ -805,7 +805,7 @@ def test_index_threshold_search_matches_full_scan(groups, nq):
     idx.remove(list(range(0, 5000, 7)))
     q = torch.randn(nq, dim, device=DEV, generator=g)
     qg = [i % 3 if i % 4 else -1 for i in range(nq)] if groups else None
-    idx.threshold_search = True
+    idx.threshold_search, idx.select_rows = True, 0  # (few queries would select from their scores)
     v1, i1, d1 = idx.search(q, 250, q_groups=qg)
     assert idx.stats["threshold_searches"] == 1 and idx.stats["threshold_overflows"] == 0
     idx.threshold_search = False

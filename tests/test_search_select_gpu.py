@@ -113,6 +113,7 @@ def test_search_by_selection_is_the_full_search(n, flt):
         idx.threshold_search = True
         assert idx._selects(6, not ("allowed" in kw or "doc_lt" in kw))
         gv, gi, gd = idx.search(q, k, **kw)
+        assert idx.stats["threshold_searches"] == 0 and idx.stats["selected_searches"] > 0
         assert gv.shape == ev.shape and torch.equal(torch.isinf(gv), torch.isinf(ev))
         hit = ~torch.isinf(gv)
         assert ((gv - ev)[hit].abs() <= 768 * 2.0 ** -22).all()  # two fp32 sums of 768 products of unit vectors

@@ -24,14 +24,14 @@ def test_rows_of_the_sample_are_found(dim, queries, cand_bytes, monkeypatch):
     for k in (1, 3):
         got = []
         for on in (False, True):
-            idx.threshold_search, idx.threshold_min_rows = on, 1
+            idx.threshold_search, idx.threshold_min_rows, idx.select_rows = on, 1, 0
             if on and cand_bytes:
                 cap = 4 * idx._sample_rank(k) * 64 + 4096
                 monkeypatch.setattr(idx, "CAND_BYTES", 8 * cap * cand_bytes, raising=False)
             parts = [idx.search(q[i:i + queries], k) for i in range(0, nq, queries)]
             got.append([torch.cat(t) for t in zip(*parts)])
         (ev, ei, _), (gv, gi, _) = got
-        assert idx.stats["threshold_searches"] > 0
+        assert idx.stats["threshold_searches"] > 0 and not idx.stats.get("selected_searches")
         assert torch.equal(ei[:, 0], 64 * torch.arange(nq, device="cuda")) and torch.equal(gi[:, 0], ei[:, 0])
         # two fp32 sums of dim products of unit vectors; ranks may change places only where scores are that close
         assert ((gv - ev).abs() <= dim * 2.0 ** -22).all() and (gi >= 0).all()
