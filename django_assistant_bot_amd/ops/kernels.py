@@ -788,7 +788,7 @@ def scores_shuffled(A, B_shuf, N, row_group, q_group=None):
     """fp32 scores [M, N] of A [M, K] against the first N rows of a ``shuffle_weights`` copy (R >= round_up(N, 128)), -inf
     where the groups drop a row: the scan of index_scan.hip where it takes the shape, else ``gemm_bt``'s."""
     _expect_scores(A, B_shuf, N, row_group, q_group)
-    if not (native().index_scan_takes(*A.shape) and A.stride(-1) == 1 and A.stride(0) % 8 == 0 and row_group.data_ptr() % 16 == 0):
+    if not (scan_scores_ok(A.shape[0], N, A.shape[1]) and A.stride(-1) == 1 and A.stride(0) % 8 == 0 and row_group.data_ptr() % 16 == 0):
         return gemm_bt(A, B_shuf, epilogue=EPI_SCORES, out_f32=True, row_group=row_group, q_group=q_group, shuffled=True, n=N)
     M, K = A.shape
     out = torch.empty((M, N), dtype=torch.float32, device=A.device)

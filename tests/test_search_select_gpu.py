@@ -178,3 +178,21 @@ def test_top_hits_costs_no_more_than_the_general_selection(n, k, kind, arg):
     new, old = min(us(lambda: ops.top_hits(s, p, k, ids, ids)) for _ in range(3)), min(us(general) for _ in range(3))
     print(f"{n} {k} {kind} {arg}: {new:.1f} us, general {old:.1f}")
     assert new <= 1.15 * old
+
+
+@pytest.mark.parametrize("n", [(1 << 22) - 4, 1 << 22])
+def test_scores_of_more_than_one_buffer(n):
+    """256 queries by 4.2M rows: the scan's stores reach 4 GB, beyond that the scores are ``gemm_bt``'s."""
+    dim, queries = 256, 256
+    g = torch.Generator(device=DEV).manual_seed(n)
+    q = torch.nn.functional.normalize(torch.randn(queries, dim, device=DEV, generator=g), dim=-1).to(torch.bfloat16)
+    v = torch.nn.functional.normalize(torch.randn(1 << 14, dim, device=DEV, generator=g), dim=-1).to(torch.bfloat16)
+    frag = ops.shuffle_weights(v).repeat((1 << 22) // len(v), 1)  # (a row's 16 neighbours are whole blocks of the copy)
+    group = torch.zeros(1 << 22, dtype=torch.int32, device=DEV)
+    group[7::1000] = -1
+    s = ops.scores_shuffled(q, frag, n, group)
+    rows = torch.cat([torch.arange(0, n, 9973, device=DEV), torch.arange(n - 40, n, device=DEV)])
+    exp = q.double() @ v[rows % len(v)].double().t()
+    live = (group[rows] >= 0).expand(queries, -1)
+    assert s.shape == (queries, n) and torch.equal(torch.isinf(s[:, rows]), ~live)
+    assert ((s[:, rows].double() - exp).abs().masked_fill(~live, 0) <= dim * 2.0 ** -23).all()  # an fp32 sum of exact products
