@@ -295,10 +295,13 @@ class VectorIndex:
                            q_group=qg, allow=allow)
 
     def _there(self, t: torch.Tensor) -> torch.Tensor:
-        """A small host tensor on the index's device, without a wait for the copy (pageable memory is waited for)."""
+        """A small host tensor on the index's device, without a wait for the copy from a pinned one of its own (a caller's
+        pinned tensor comes back from ``pin_memory`` as it is, and may be refilled once the search returns)."""
         if self.device.type == "cuda" and not t.is_cuda:
-            t = t.pin_memory()
-        return t.to(self.device, non_blocking=True)
+            own = t.pin_memory()
+            if own.data_ptr() != t.data_ptr():
+                return own.to(self.device, non_blocking=True)
+        return t.to(self.device)
 
     def _query(self, queries, q_groups, allowed, doc_lt):
         """(unit queries, their groups, row mask, rows in whole fours) on the device."""

@@ -196,3 +196,22 @@ def test_scores_of_more_than_one_buffer(n):
     live = (group[rows] >= 0).expand(queries, -1)
     assert s.shape == (queries, n) and torch.equal(torch.isinf(s[:, rows]), ~live)
     assert ((s[:, rows].double() - exp).abs().masked_fill(~live, 0) <= dim * 2.0 ** -23).all()  # an fp32 sum of exact products
+
+
+def test_a_callers_pinned_filters_may_be_refilled():
+    """Groups and document limits in pinned buffers that the caller fills anew once ``search`` returns, while the device
+    is still busy with what was queued before."""
+    n = 20_000
+    idx = VectorIndex(256, DEV, capacity=n)
+    g = torch.Generator(device=DEV).manual_seed(0)
+    idx.add(np.arange(n), torch.randn(n, 256, device=DEV, generator=g), doc_ids=np.arange(n) // 4, groups=np.arange(n) % 2)
+    q = torch.randn(3, 256, device=DEV, generator=g)
+    groups, limits = torch.tensor([0, 1, 0], dtype=torch.int32), torch.tensor([90, 4000, 2500])
+    exp = idx.search(q, 20, q_groups=groups, doc_lt=limits)
+    groups, limits = groups.pin_memory(), limits.pin_memory()
+    torch.cuda._sleep(200_000_000)  # some 0.1 s
+    got = idx.search(q, 20, q_groups=groups, doc_lt=limits)
+    groups.fill_(1)
+    limits.fill_(3)
+    for a, b in zip(got, exp):
+        assert torch.equal(a, b)
