@@ -1687,6 +1687,7 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 template <int D, bool KV_NT, bool DMA = false, int NSLOT = 1, bool EXT = false, typename ROPE = void>
 __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(DecodeParams p, int total_items) {
   static_assert(NSLOT == 1 || (NSLOT == 2 && DMA), "two slots: DMA staging only");
+  static_assert(std::is_same_v<ROPE, void> || !DMA || NSLOT == 2, "rotation under LDS-DMA: two slots (one has no registers left)");
   // appended workgroups (small batches leave most CUs idle during this latency-bound launch): warm
   // the following projections' weights into the Infinity Cache and leave
   const int attn_blocks = gridDim.x - p.warm.blocks;
@@ -2029,12 +2030,9 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
           compute(kw + i * 4 * KT);
         }
       } else {
-      int blk = blk_at(kw);
-      if (kw < k_end) fused_load();
-      blk = __builtin_amdgcn_readfirstlane(blk);
+      int blk = __builtin_amdgcn_readfirstlane(blk_at(kw));
       for (int k0 = kw; k0 < k_end; k0 += 4 * KT) {
         dma(k0, blk);
-        if (k0 == kw) fused_finish();
         blk = blk_at(k0 + 4 * KT);  // in flight under this sub-tile's copy and math
         asm volatile("s_waitcnt vmcnt(1)" ::: "memory");  // this sub-tile's 16 pieces landed
         compute(k0);
