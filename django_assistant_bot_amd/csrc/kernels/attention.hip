@@ -1641,9 +1641,10 @@ struct DecodeParams {
 // (128, 900-1500) 102.7 -> 112.2.  With the rotation inside (decode_rope_ok), us a step of Llama-3-8B: 9 sequences 3612 ->
 // 3544, 16 3989 -> 3843, 32 4325 -> 4240, of 900-1500 4231 -> 4210, 48 4699 -> 4686.
 constexpr int kDecodeCus = 256;
+constexpr int kTwoSlotKeys = 64 * 4 * 32;  // a lane holds one block id, of a wave's sub-tile
 static bool decode_two_slots(int batch, int Hkv, int part_size) {
   const long items = (long)batch * Hkv;
-  return part_size <= 64 * 4 * 32 && (items <= kDecodeCus || (items <= 3 * kDecodeCus / 2 && part_size >= 2048));
+  return part_size <= kTwoSlotKeys && (items <= kDecodeCus || (items <= 3 * kDecodeCus / 2 && part_size >= 2048));
 }
 
 constexpr int kCombine = 8;  // partial results requested together by the combine
@@ -1665,9 +1666,42 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
   return decode_partition(part_size, longest, items, max_parts);
 }
 
+// ... and of up to 256 items with two slots, a workgroup a CU: the smallest, in whole 128 keys up to 4096, of which every
+// one that holds keys finds a CU at once.  A second round waits for the first and pays a start and a combine again; larger
+// partitions leave CUs idle.  Context lengths are known on the device alone, so the workgroups search for it themselves,
+// where not every one has an item of its own to begin with.  parts_of(size): the (sequence, kv head) partitions of that size.
+// us of a layer with its rotation, 8 key heads, (sequences, contexts): apart on one slot with 512 keys / inside, partitions
+// doubled until they fit or are 2048 and walked with their empty ones / these: (9, 2000-4000) 33.5 / 44.6 / 31.2, (9, 4000)
+// 44.0 / 46.6 / 35.6, (12, 200-2000) 25.6 / 32.9 / 20.3, (16, 300-1700) 26.9 / 26.5 / 21.7, (20, 4000) 72.2 / 88.8 / 63.8,
+// (24, 300-1700) 30.3 / 33.7 / 28.9, (24, 100-8000) 96.2 / 114.3 / 82.3, (28, 2000-4000) 79.7 / 81.9 / 72.5, (32, 300-1700)
+// 38.2 / 37.5 / 33.5, (32, 100-8000) 106.5 / 100.3 / 96.9.
+template <typename F>
+__host__ __device__ inline int decode_partition_fit(int part_size, int longest, int items, int max_parts, F parts_of) {
+  if (items > kDecodeCus || longest <= part_size || longest > (long)part_size * max_parts) return part_size;
+  if (parts_of(part_size) <= kDecodeCus) return part_size;
+  int lo = part_size / 128, hi = (longest + 127) / 128;
+  if (hi > 4096 / 128) hi = 4096 / 128;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    if (parts_of(128 * mid) <= kDecodeCus) hi = mid;
+    else lo = mid;
+  }
+  return 128 * (hi > lo ? hi : lo);
+}
+int decode_partition_fit_of(int part_size, const int* contexts, int batch, int Hkv, int max_parts) {
+  int longest = 0;
+  for (int i = 0; i < batch; ++i) longest = std::max(longest, contexts[i]);
+  return decode_partition_fit(decode_partition(part_size, longest, batch * Hkv, max_parts), longest, batch * Hkv, max_parts,
+                              [&](int size) {
+                                int n = 0;
+                                for (int i = 0; i < batch; ++i) n += (contexts[i] + size - 1) / size;
+                                return n * Hkv;
+                              });
+}
+
 // DMA (D = 128): each wave streams its 32-key K / V sub-tiles straight into its LDS slot by LDS-DMA
-// (buffer_load ... lds, non-temporal: MI355X_MICROARCH.md rows ldsdma-fill / nt-weights put the
-// LDS-DMA stream at 6.5-6.8 TB/s chip-wide against 5.7-5.8 for register gathers) instead of through
+// (buffer_load ... lds, non-temporal: such a stream reads 6.5-6.8 TB/s chip-wide against
+// 5.7-5.8 for register gathers) instead of through
 // a register double buffer + ds_write; one slot per wave, the 8 waves of a CU's two workgroups keep
 // ~128 KB in flight.  The next sub-tile's block id is fetched under the current sub-tile's DMA.
 //
@@ -1675,7 +1709,7 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 // flight while sub-tile i computes, and the wave's block ids are fetched once, one per lane, before
 // the first copy.  At batch 1 - 8 a workgroup's waves walk their sub-tiles back to back with the
 // whole GPU otherwise idle: one copy round trip per sub-tile was the critical path.  128 KB of LDS:
-// one workgroup per CU, which small batches never fill anyway.
+// one workgroup per CU (decode_two_slots and decode_partition_fit say how many items that suits).
 //
 // EXT: slopes (may be null) and the output gate; the plain form is free of both.
 //
@@ -1736,28 +1770,64 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
   for (int off = 32; off; off >>= 1) maxc = max(maxc, __shfl_xor(maxc, off));
   maxc = __builtin_amdgcn_readfirstlane(maxc);
   int part_size = decode_partition(p.part_size, maxc, BH, p.max_parts);
-  if constexpr (NSLOT == 2) {
-    // Above 64 items: partitions doubled, up to 2048 keys, until all of them find a CU at once (a second round waits for
-    // the first, and partitions cost a combine).  us a launch, 512 keys -> those taken: (16, 300-1700) 24.0 -> 22.7, (20,
-    // 800-3000) 42 -> 35.9, (24, 300-1700) 29.1 -> 27.5; (9, 200-2000), which stay at 512, 19.5, at 1024 21.8.
-    auto parts_of = [&](int size) {
-      float n = lane < nb ? (float)((seen_keys(ctx_l) + size - 1) / size) : 0.f;
-      for (int i = lane + 64; i < nb; i += 64) n += (float)((seen_keys(p.ctx_lens[i]) + size - 1) / size);
-      return (int)wave_sum_valu(n) * p.Hkv;
-    };
-    if (BH > 64)
-      while (part_size < 2048 && part_size < maxc && maxc <= part_size * p.max_parts && parts_of(part_size) > kDecodeCus)
-        part_size *= 2;
+  int live_items = min(p.max_parts, (maxc + part_size - 1) / part_size) * BH;
+  constexpr int WORDS = kDecodeCus / 64;  // of up to 256 sequences, four a lane
+  int ends[WORDS];     // two slots: partitions of the sequences up to 64 j + lane
+  bool dense = false;  // items with keys alone
+  if (NSLOT == 2 && live_items > attn_blocks && BH <= kDecodeCus && maxc <= (long)part_size * p.max_parts) {
+    // some workgroups have a second item, or one past its sequence's end and the next
+    int keys[WORDS];
+#pragma unroll
+    for (int j = 0; j < WORDS; ++j)
+      keys[j] = j && nb <= 64 * j ? 0 : lane + 64 * j < nb ? seen_keys(j ? p.ctx_lens[lane + 64 * j] : ctx_l) : 0;
+    auto parts_of = [&](int j, int size) { return (int)((unsigned)(keys[j] + size - 1) / (unsigned)size); };
+    part_size = decode_partition_fit(part_size, maxc, BH, p.max_parts, [&](int size) {
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < WORDS; ++j)
+        if (!j || nb > 64 * j) n += parts_of(j, size);
+      // (a scalar: as the lanes' sum alone it would make every loop and address behind it the lanes' own, 1.5 us a launch)
+      return __builtin_amdgcn_readfirstlane((int)wave_sum_valu((float)n)) * p.Hkv;
+    });
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < WORDS; ++j) {
+      if (j && nb <= 64 * j) continue;
+      ends[j] = parts_of(j, part_size);
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(ends[j], off, 64);
+        if (lane >= off) ends[j] += t;
+      }
+      ends[j] += n;
+      n = __builtin_amdgcn_readlane(ends[j], 63);
+    }
+    dense = n * p.Hkv <= attn_blocks;
+    live_items = dense ? n * p.Hkv : (maxc + part_size - 1) / part_size * BH;
   }
-  const int live_items = min(p.max_parts, (maxc + part_size - 1) / part_size) * BH;
   for (int r0 = 0, back = 0; r0 < live_items; r0 += attn_blocks, back ^= NSLOT - 1) {
-    // two slots: the launch has a workgroup a CU, so every other round goes backwards (the items come longest first)
+    // two slots: the launch has a workgroup a CU, so where there is another round it goes backwards (the items come longest first)
     const int item = r0 + (back ? attn_blocks - 1 - (int)blockIdx.x : (int)blockIdx.x);
     if (item >= live_items) continue;
-    const int part = item / BH;
+    int part = item / BH;
     const int bh = item - part * BH;
-    const int hk = bh % p.Hkv;
-    const int b = held ? __builtin_amdgcn_readlane(ord_l, bh / p.Hkv) : p.order ? p.order[bh / p.Hkv] : bh / p.Hkv;
+    int hk = bh % p.Hkv;
+    int b = held ? __builtin_amdgcn_readlane(ord_l, bh / p.Hkv) : p.order ? p.order[bh / p.Hkv] : bh / p.Hkv;
+    if constexpr (NSLOT == 2) {
+      if (dense) {
+        const int at = item / p.Hkv;
+        hk = item - at * p.Hkv;
+        b = 0;
+        part = at;
+#pragma unroll
+        for (int j = 0; j < WORDS; ++j) {
+          if (j && nb <= 64 * j) continue;
+          const int before = __popcll(__ballot(ends[j] <= at));  // (behind the last sequence: all of them, never)
+          if (before) part = at - __builtin_amdgcn_readlane(ends[j], before - 1);
+          b += before;
+        }
+      }
+    }
     const int ctx = held ? __builtin_amdgcn_readlane(ctx_l, b) : p.ctx_lens[b];
     const int k_lo = first_key(ctx - 1, 0, p.chunk), k_org = k_lo & ~(KT - 1);
     const int k_begin = k_org + part * part_size;

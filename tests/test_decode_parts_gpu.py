@@ -20,6 +20,20 @@ DEV = "cuda"
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("order", [False, True])
 def test_decode_partitions(ctx, Hkv, max_parts, D, order):
+    _check(ctx, Hkv, max_parts, D, order)
+
+
+# two slots: partitions of as many keys as give every one a workgroup, and those alone walked: sequences without and with a
+# second and third one in any place, none (a padded row), words of 64 sequences, contexts beyond the largest partition
+@pytest.mark.parametrize("ctx,Hkv,max_parts", [([200, 2000, 10, 1100] * 3, 8, 4), ([4000, 100] * 5 + [4000], 8, 8), ([300] * 31 + [5000], 8, 10),
+                                               ([600, 0, 1300, 513] * 16, 4, 4), ([900, 20, 30] * 66, 1, 4), ([30] * 255 + [2500], 1, 6),
+                                               ([9000, 700] * 5, 8, 20), ([3000, 9000, 5000] * 10, 8, 18)])
+@pytest.mark.parametrize("order", [False, True])
+def test_partitions_that_find_a_workgroup_each(ctx, Hkv, max_parts, order):
+    _check(ctx, Hkv, max_parts, 128, order)
+
+
+def _check(ctx, Hkv, max_parts, D, order):
     g = torch.Generator(device=DEV).manual_seed(len(ctx) + Hkv)
     B, Hq, bs = len(ctx), 4 * Hkv, 64
     need = [-(-c // bs) for c in ctx]
@@ -35,6 +49,8 @@ def test_decode_partitions(ctx, Hkv, max_parts, D, order):
     for _ in range(2):  # the arrival counters are zero again after a launch
         out = ops.paged_decode(q, kc, vc, bt.to(DEV), ctxt, 512, ws, order=by_len)
         for b, n in enumerate(ctx):
+            if n == 0:
+                continue
             n = min(n, 512 * max_parts)  # what the workspace's partitions cover
             k, v = (ref.gather_paged(c, bt[b].to(DEV), n).double().repeat_interleave(4, 1).transpose(0, 1) for c in (kc, vc))
             s = torch.matmul(k, q[b].double().unsqueeze(-1)).squeeze(-1) * D ** -0.5
