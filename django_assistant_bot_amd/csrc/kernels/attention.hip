@@ -1634,17 +1634,19 @@ struct DecodeParams {
   L3Warm warm;  // optional: the next projections' weights, warmed into L3 by appended workgroups
 };
 
-// D = 128: two LDS slots a wave, whose block ids one lane each holds, where the items find a CU each (128 KB of LDS), and up
-// to half as many again in whole contexts.  Beyond that the one-slot form's two workgroups a CU.  us a launch, one slot ->
-// two, (sequences, contexts), 8 key heads: (16, 300-1700) 24.3 -> 22.7, (16, 2000-4000) 48.8 -> 39.6, (24, 300-1700) 29.7 ->
-// 27.5, (32, 300-1700) 34.4 -> 32.3, (48, 300-1700) 44.4 -> 41.3, but (32, 900-1500) 34.3 -> 35.8, (64, 300-1700) 52.2 -> 54.0,
-// (128, 900-1500) 102.7 -> 112.2.  With the rotation inside (decode_rope_ok), us a step of Llama-3-8B: 9 sequences 3612 ->
-// 3544, 16 3989 -> 3843, 32 4325 -> 4240, of 900-1500 4231 -> 4210, 48 4699 -> 4686.
-constexpr int kDecodeCus = 256;
+// D = 128: two LDS slots a wave, whose block ids one lane each holds, where the items find a CU each (128 KB of LDS).  Beyond
+// that the one-slot form's two workgroups a CU, but for up to half as many items again in whole contexts with the rotation
+// inside (decode_rope_ok): a launch less, and contexts that differ leave the short ones to the second round.
+// us a launch, one slot with 512 keys -> two, (sequences, contexts), 8 key heads: (2, 900-1500) 11.9 -> 12.1, (8, 2000-4000)
+// 31.4 -> 25.6, (16, 300-1700) 24.3 -> 21.5, (24, 300-1700) 27.4 -> 28.7, (32, 900-1500) 35.7 -> 33.6; with slopes or a gate (16,
+// 300-1700) 26.6 -> 23.1, (32, 300-1700) 44.2 -> 35.9; 0.96 in the mean of 120 shapes of 16-256 items.  Above 256, with the rotation
+// apart on one slot / inside on two: (40, 300-1700) 43.2 / 34.5, (48, 300-1700) 47.8 / 40.8, (48, 900-1500) 52.9 / 52.6, (40, 1000)
+// 43.4 / 44.8, (40, 100-300) 17.2 / 18.6; without it (40, 100-300) 14.1 / 15.0, (48, 100-300) 15.5 / 16.8, not taken.
+constexpr int kDecodeCus = 256;  // (of the whole card; with fewer CUs the workgroups queue)
 constexpr int kTwoSlotKeys = 64 * 4 * 32;  // a lane holds one block id, of a wave's sub-tile
-static bool decode_two_slots(int batch, int Hkv, int part_size) {
+static bool decode_two_slots(int batch, int Hkv, int part_size, bool rotated) {
   const long items = (long)batch * Hkv;
-  return part_size <= kTwoSlotKeys && (items <= kDecodeCus || (items <= 3 * kDecodeCus / 2 && part_size >= 2048));
+  return part_size <= kTwoSlotKeys && (items <= kDecodeCus || (rotated && items <= 3 * kDecodeCus / 2 && part_size >= 2048));
 }
 
 constexpr int kCombine = 8;  // partial results requested together by the combine
@@ -1805,6 +1807,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     dense = n * p.Hkv <= attn_blocks;
     live_items = dense ? n * p.Hkv : (maxc + part_size - 1) / part_size * BH;
   }
+  if ((int)blockIdx.x >= live_items) return;  // (ahead of what the loop keeps in registers: most of 2048 workgroups, 1 us)
   for (int r0 = 0, back = 0; r0 < live_items; r0 += attn_blocks, back ^= NSLOT - 1) {
     // two slots: the launch has a workgroup a CU, so where there is another round it goes backwards (the items come longest first)
     const int item = r0 + (back ? attn_blocks - 1 - (int)blockIdx.x : (int)blockIdx.x);
@@ -2505,7 +2508,7 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
 // heads), 6: 944 -> 930, 24: 1054 -> 1032, 48: 1106 -> 1099, 100: 1549 -> 1724.
 int decode_rope_ok(int batch, int Hkv, int D, int part_size) {
   if (batch <= 0 || Hkv <= 0) return 0;
-  return D == 128 ? decode_two_slots(batch, Hkv, part_size) : D == 64 && batch * Hkv <= 384;
+  return D == 128 ? decode_two_slots(batch, Hkv, part_size, true) : D == 64 && batch * Hkv <= 384;
 }
 
 // The workgroups of a launch are dispatched in blockIdx order as CU slots free up; at RAG batch sizes
@@ -2563,14 +2566,14 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   const int total_items = max_parts * Hkv * batch;
   // A workgroup without an item still waits for the contexts, and with two slots a CU runs one at a time: a workgroup a CU
   // (us a step of Llama-3-8B with 2048 workgroups -> 256: 4 sequences 3419 -> 3352, 8 3668 -> 3560).
-  const int most = D == 128 && decode_two_slots(batch, Hkv, part_size) ? kDecodeCus : 2048;
+  const bool two = D == 128 && decode_two_slots(batch, Hkv, part_size, fused);
+  const int most = two ? kDecodeCus : 2048;
   dim3 grid((total_items < most ? total_items : most) + prm.warm.blocks);
   // K/V are read exactly once per step: non-temporal loads (aux = 2) -- in the Llama-3-8B decode step
   // at batch 128 this took the attention from 127 to 111 us per layer (5.1 -> 5.8 TB/s;
   // profiles/decode_round2.md).  D = 128 stages K / V by LDS-DMA (100.7 vs 102.6 us isolated, same
   // section); D = 64 (small test models) keeps the register path.
   if (D == 128) {
-    const bool two = decode_two_slots(batch, Hkv, part_size);
     if (fused && rope->bf16_slabs)
       hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2, false, bf16>), grid, dim3(256), 0, s, prm, total_items);
     else if (fused)

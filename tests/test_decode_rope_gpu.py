@@ -47,6 +47,26 @@ def test_rope_inside_the_attention(D, Hq, Hkv, B, S, dtype):
     assert not ws.cnt.any()
 
 
+def test_rotation_on_two_slots_above_a_workgroup_a_cu():
+    """320 items in whole contexts: the rotation inside takes two slots and two rounds, the two launches one slot."""
+    B, Hq, Hkv, D, bs, part = 40, 16, 8, 128, 64, 2048
+    g = torch.Generator(device=DEV).manual_seed(0)
+    ctx = torch.randint(1, 2048, (B,), device=DEV, generator=g, dtype=torch.int32)
+    ctx[:4] = torch.tensor([2048, 1, 128, 2047])
+    tables = torch.randperm(B * 32, device=DEV, generator=g).view(B, 32).to(torch.int32)
+    k1, v1 = (torch.randn(B * 32, Hkv, bs, D, device=DEV, generator=g).to(torch.bfloat16) for _ in range(2))
+    k2, v2, pos = k1.clone(), v1.clone(), ctx - 1
+    slots = tables[torch.arange(B, device=DEV), (pos // bs).long()].long() * bs + pos % bs
+    qkv = torch.randn(4, B, (Hq + 2 * Hkv) * D, device=DEV, generator=g).to(torch.bfloat16)
+    cs = torch.rand(2048, D // 2, 2, device=DEV, generator=g)
+    ws = ops.DecodeWorkspace(B, Hq, D, 4, DEV)
+    for order in (None, torch.argsort(ctx, descending=True).to(torch.int32)):
+        q = ops.rope_kv_write(qkv, pos, cs, k1, v1, slots, Hq, Hkv, D)
+        exp = ops.paged_decode(q, k1, v1, tables, ctx, part, ws, order=order)
+        got = ops.paged_decode_rope(qkv, pos, cs, k2, v2, slots, Hq, tables, ctx, part, ws, order=order)
+        assert torch.equal(got, exp) and torch.equal(k1, k2) and torch.equal(v1, v2)
+
+
 def test_what_is_refused():
     assert not ops.decode_rope_ok(33, 8, 128, 512) and not ops.decode_rope_ok(8, 8, 128, 16384)
     assert not ops.decode_rope_ok(49, 8, 64, 512) and not ops.decode_rope_ok(1, 8, 32, 512)
