@@ -459,8 +459,8 @@ PYBIND11_MODULE(_native, m) {
   });
   m.def("flash_packed64_wins", &dab::flash_packed64_wins);
   m.def("decode_partition", &dab::decode_partition_of);
-  m.def("decode_partition_fit", [](int part_size, const std::vector<int>& contexts, int Hkv, int max_parts) {
-    return dab::decode_partition_fit_of(part_size, contexts.data(), (int)contexts.size(), Hkv, max_parts);
+  m.def("decode_partition_fit", [](int part_size, const std::vector<int>& contexts, int Hkv, int max_parts, int slots) {
+    return dab::decode_partition_fit_of(part_size, contexts.data(), (int)contexts.size(), Hkv, max_parts, slots);
   });
   m.def("paged_decode_attention", [](u q, u kc, u vc, u bt, int max_blocks, int bs, u ctx, u out, u po, u pm, u pl,
                                      u cnt, int batch, int Hq, int Hkv, int D, int part_size, int max_parts,

@@ -1669,7 +1669,7 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 }
 
 // ... and of up to 256 items with two slots, a workgroup a CU: the smallest, in whole 128 keys up to 4096, of which every
-// one that holds keys finds a CU at once.  A second round waits for the first and pays a start and a combine again; larger
+// one that holds keys finds a CU at once (a slot, generally).  A second round waits for the first and pays a start and a combine again; larger
 // partitions leave CUs idle.  Context lengths are known on the device alone, so the workgroups search for it themselves,
 // where not every one has an item of its own to begin with.  parts_of(size): the (sequence, kv head) partitions of that size.
 // us of a layer with its rotation, 8 key heads, (sequences, contexts): apart on one slot with 512 keys / inside, partitions
@@ -1677,23 +1677,27 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 // 44.0 / 46.6 / 35.6, (12, 200-2000) 25.6 / 32.9 / 20.3, (16, 300-1700) 26.9 / 26.5 / 21.7, (20, 4000) 72.2 / 88.8 / 63.8,
 // (24, 300-1700) 30.3 / 33.7 / 28.9, (24, 100-8000) 96.2 / 114.3 / 82.3, (28, 2000-4000) 79.7 / 81.9 / 72.5, (32, 300-1700)
 // 38.2 / 37.5 / 33.5, (32, 100-8000) 106.5 / 100.3 / 96.9.
+// Heads of 64 with the rotation inside: two workgroups a CU (a third, which they have without it, lacks the registers), so the
+// 512 keys that fit three did not fit two.  Apart / inside with 512 keys / these: (9, 4000) 26.4 / 29.9 / 25.8, (9, 100-8000)
+// 27.8 / 33.7 / 27.0, (12, 4000) 29.5 / 34.6 / 31.0, (16, 2000-4000) 32.7 / 35.2 / 30.5, (16, 100-8000) 43.1 / 48.3 / 35.6.
+constexpr int kRopeSlots = 2 * kDecodeCus;
 template <typename F>
-__host__ __device__ inline int decode_partition_fit(int part_size, int longest, int items, int max_parts, F parts_of) {
+__host__ __device__ inline int decode_partition_fit(int part_size, int longest, int items, int max_parts, int slots, F parts_of) {
   if (items > kDecodeCus || longest <= part_size || longest > (long)part_size * max_parts) return part_size;
-  if (parts_of(part_size) <= kDecodeCus) return part_size;
+  if (parts_of(part_size) <= slots) return part_size;
   int lo = part_size / 128, hi = (longest + 127) / 128;
   if (hi > 4096 / 128) hi = 4096 / 128;
   while (hi - lo > 1) {
     const int mid = (lo + hi) / 2;
-    if (parts_of(128 * mid) <= kDecodeCus) hi = mid;
+    if (parts_of(128 * mid) <= slots) hi = mid;
     else lo = mid;
   }
   return 128 * (hi > lo ? hi : lo);
 }
-int decode_partition_fit_of(int part_size, const int* contexts, int batch, int Hkv, int max_parts) {
+int decode_partition_fit_of(int part_size, const int* contexts, int batch, int Hkv, int max_parts, int slots) {
   int longest = 0;
   for (int i = 0; i < batch; ++i) longest = std::max(longest, contexts[i]);
-  return decode_partition_fit(decode_partition(part_size, longest, batch * Hkv, max_parts), longest, batch * Hkv, max_parts,
+  return decode_partition_fit(decode_partition(part_size, longest, batch * Hkv, max_parts), longest, batch * Hkv, max_parts, slots,
                               [&](int size) {
                                 int n = 0;
                                 for (int i = 0; i < batch; ++i) n += (contexts[i] + size - 1) / size;
@@ -1776,14 +1780,15 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
   constexpr int WORDS = kDecodeCus / 64;  // of up to 256 sequences, four a lane
   int ends[WORDS];     // two slots: partitions of the sequences up to 64 j + lane
   bool dense = false;  // items with keys alone
-  if (NSLOT == 2 && live_items > attn_blocks && BH <= kDecodeCus && maxc <= (long)part_size * p.max_parts) {
+  constexpr bool FUSED = !std::is_same_v<ROPE, void>;
+  if ((NSLOT == 2 || FUSED) && live_items > attn_blocks && BH <= kDecodeCus && maxc <= (long)part_size * p.max_parts) {
     // some workgroups have a second item, or one past its sequence's end and the next
     int keys[WORDS];
 #pragma unroll
     for (int j = 0; j < WORDS; ++j)
       keys[j] = j && nb <= 64 * j ? 0 : lane + 64 * j < nb ? seen_keys(j ? p.ctx_lens[lane + 64 * j] : ctx_l) : 0;
     auto parts_of = [&](int j, int size) { return (int)((unsigned)(keys[j] + size - 1) / (unsigned)size); };
-    part_size = decode_partition_fit(part_size, maxc, BH, p.max_parts, [&](int size) {
+    part_size = decode_partition_fit(part_size, maxc, BH, p.max_parts, attn_blocks, [&](int size) {
       int n = 0;
 #pragma unroll
       for (int j = 0; j < WORDS; ++j)
@@ -1816,7 +1821,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     const int bh = item - part * BH;
     int hk = bh % p.Hkv;
     int b = held ? __builtin_amdgcn_readlane(ord_l, bh / p.Hkv) : p.order ? p.order[bh / p.Hkv] : bh / p.Hkv;
-    if constexpr (NSLOT == 2) {
+    if constexpr (NSLOT == 2 || FUSED) {
       if (dense) {
         const int at = item / p.Hkv;
         hk = item - at * p.Hkv;
@@ -1838,7 +1843,6 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     const int k_end = min(ctx, k_begin + part_size);
 
     bf16x8 qf[NKK];
-    constexpr bool FUSED = !std::is_same_v<ROPE, void>;
     // FUSED: the wave that holds the new token (the context's last key), and its rotated k / copied v pieces: lane l of the
     // first D / 16 holds dims 8 l .. + 7 and those D / 2 on of k, the next D / 16 lanes of v
     const int k_new = ctx - 1, new_sub = (k_new - k_begin) / KT;
@@ -2502,10 +2506,9 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
   return hipGetLastError();
 }
 
-// Whether a decode step rotates and writes its rows inside the attention: while the items find a CU or two at once (every
-// further round of them pays the sums again).  us a step, rope_kv_write apart -> inside: Llama-3-8B (D 128), 1 sequence 3087
-// -> 3064, 4: 3223 -> 3169, 8: 3424 -> 3356 (the one-slot form has no registers left for it); Llama-3.2-1B (D 64, 8 key
-// heads), 6: 944 -> 930, 24: 1054 -> 1032, 48: 1106 -> 1099, 100: 1549 -> 1724.
+// Whether a decode step can rotate and write its rows inside the attention: while the items find a CU or two at once (every
+// further round of them pays the sums again, and the one-slot form for D = 128 has no registers left for it).  us a step,
+// rope_kv_write apart -> inside: Llama-3-8B (D 128), 1 sequence 3087 -> 3064, 4: 3223 -> 3169, 8: 3424 -> 3356.
 int decode_rope_ok(int batch, int Hkv, int D, int part_size) {
   if (batch <= 0 || Hkv <= 0) return 0;
   return D == 128 ? decode_two_slots(batch, Hkv, part_size, true) : D == 64 && batch * Hkv <= 384;
@@ -2567,7 +2570,7 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   // A workgroup without an item still waits for the contexts, and with two slots a CU runs one at a time: a workgroup a CU
   // (us a step of Llama-3-8B with 2048 workgroups -> 256: 4 sequences 3419 -> 3352, 8 3668 -> 3560).
   const bool two = D == 128 && decode_two_slots(batch, Hkv, part_size, fused);
-  const int most = two ? kDecodeCus : 2048;
+  const int most = two ? kDecodeCus : fused && batch * Hkv <= kDecodeCus ? kRopeSlots : 2048;
   dim3 grid((total_items < most ? total_items : most) + prm.warm.blocks);
   // K/V are read exactly once per step: non-temporal loads (aux = 2) -- in the Llama-3-8B decode step
   // at batch 128 this took the attention from 127 to 111 us per layer (5.1 -> 5.8 TB/s;

@@ -75,7 +75,7 @@ int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, c
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
                    long o_tok, long o_head, const int* cu, int batch, int max_len, int Hq, int Hkv, float scale, hipStream_t s);
 int decode_partition_of(int part_size, int longest, int items, int max_parts);
-int decode_partition_fit_of(int part_size, const int* contexts, int batch, int Hkv, int max_parts);
+int decode_partition_fit_of(int part_size, const int* contexts, int batch, int Hkv, int max_parts, int slots);
 // The rows of a decode step before their rotation: split-K slabs [S][batch][ld] of the qkv projection (fp32 or bf16, summed in
 // order and rounded like a GEMM's output), with the token's position and cache slot (< 0: not written)
 struct TokenRope {

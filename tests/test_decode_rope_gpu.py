@@ -67,6 +67,31 @@ def test_rotation_on_two_slots_above_a_workgroup_a_cu():
         assert torch.equal(got, exp) and torch.equal(k1, k2) and torch.equal(v1, v2)
 
 
+def test_rotation_in_longer_partitions_of_heads_of_64():
+    """16 sequences whose partitions of 512 keys are more than two workgroups a CU: longer ones, against the two launches,
+    which keep 512 (their sums meet in another order)."""
+    B, Hq, Hkv, D, bs, part, n = 16, 32, 8, 64, 64, 512, 64
+    g = torch.Generator(device=DEV).manual_seed(1)
+    ctx = torch.randint(2000, n * bs, (B,), device=DEV, generator=g, dtype=torch.int32)
+    ctx[:3] = torch.tensor([n * bs, 1, 3])
+    tables = torch.randperm(B * n, device=DEV, generator=g).view(B, n).to(torch.int32)
+    k1, v1 = (torch.randn(B * n, Hkv, bs, D, device=DEV, generator=g).to(torch.bfloat16) for _ in range(2))
+    k2, v2, pos = k1.clone(), v1.clone(), ctx - 1
+    slots = tables[torch.arange(B, device=DEV), (pos // bs).long()].long() * bs + pos % bs
+    qkv = torch.randn(4, B, (Hq + 2 * Hkv) * D, device=DEV, generator=g).to(torch.bfloat16)
+    cs = torch.rand(n * bs, D // 2, 2, device=DEV, generator=g)
+    ws = ops.DecodeWorkspace(B, Hq, D, n * bs // 512, DEV)
+    for order in (None, torch.argsort(ctx, descending=True).to(torch.int32)):
+        q = ops.rope_kv_write(qkv, pos, cs, k1, v1, slots, Hq, Hkv, D)
+        exp = ops.paged_decode(q, k1, v1, tables, ctx, part, ws, order=order).float()
+        got = ops.paged_decode_rope(qkv, pos, cs, k2, v2, slots, Hq, tables, ctx, part, ws, order=order).float()
+        assert torch.equal(k1, k2) and torch.equal(v1, v2)
+        # both round the probabilities and the result to bf16, with other maxima: 2^-8 of sum |p v| (at most max |v|), twice
+        assert ((got - exp).abs() <= 2 * 2.0 ** -8 * (exp.abs() + v1.abs().max().float())).all()
+        assert (got - exp).norm() <= 2.0 ** -7 * exp.norm()
+    assert not ws.cnt.any()
+
+
 def test_what_is_refused():
     assert not ops.decode_rope_ok(33, 8, 128, 512) and not ops.decode_rope_ok(8, 8, 128, 16384)
     assert not ops.decode_rope_ok(49, 8, 64, 512) and not ops.decode_rope_ok(1, 8, 32, 512)
