@@ -9,7 +9,7 @@ DEV = "cuda"
 
 # ends of the four ranges of the rule (tiles of 64 or 128, two or three slices), whole tiles and one row more or less, K whose
 # slices are not equal
-SIZES = [(705, 768, 3072, 3), (896, 768, 3072, 3), (1024, 768, 3072, 2), (897, 768, 2624, 2), (1344, 768, 3072, 2), (1345, 768, 3072, 3),
+SIZES = [(705, 768, 3072, 3), (896, 768, 3072, 3), (1024, 768, 2048, 2), (897, 768, 2624, 2), (960, 768, 3072, 2), (1344, 768, 1536, 2), (1345, 768, 3072, 3),
          (1792, 768, 3072, 3), (1921, 768, 3072, 2), (2688, 768, 1536, 2), (1793, 384, 1536, 2), (2689, 384, 1600, 3),
          (5376, 384, 1536, 2), (575, 1024, 4096, 3), (1280, 1024, 4096, 3), (2048, 1024, 4096, 2)]
 
@@ -30,7 +30,7 @@ def test_slices_against_64_bits(M, N, K, slices):
 
 
 def test_other_sizes_and_operands_take_two_launches():
-    for M, N, K in ((704, 768, 3072), (900, 768, 768), (900, 512, 3072), (0, 768, 3072), (3100, 768, 3072), (900, 768, 1535), (769, 1024, 4096)):
+    for M, N, K in ((704, 768, 3072), (961, 768, 3072), (1344, 768, 3072), (1000, 768, 2112), (900, 768, 768), (900, 512, 3072), (0, 768, 3072), (3100, 768, 3072), (900, 768, 1535), (769, 1024, 4096)):
         assert ops.native().slab_slices(M, N, K) == 0
     g = torch.Generator(device=DEV).manual_seed(0)
     r = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
