@@ -296,8 +296,9 @@ class VectorIndex:
 
     def _there(self, t: torch.Tensor) -> torch.Tensor:
         """A small host tensor on the index's device, without a wait for the copy from a pinned one of its own (a caller's
-        pinned tensor comes back from ``pin_memory`` as it is, and may be refilled once the search returns)."""
-        if self.device.type == "cuda" and not t.is_cuda:
+        pinned tensor comes back from ``pin_memory`` as it is, and may be refilled once the search returns).  A stream capture
+        refuses the copy that is waited for; it would record the other, whose buffer a replay finds in other hands."""
+        if self.device.type == "cuda" and not t.is_cuda and not torch.cuda.is_current_stream_capturing():
             own = t.pin_memory()
             if own.data_ptr() != t.data_ptr():
                 return own.to(self.device, non_blocking=True)

@@ -215,3 +215,16 @@ def test_a_callers_pinned_filters_may_be_refilled():
     limits.fill_(3)
     for a, b in zip(got, exp):
         assert torch.equal(a, b)
+
+
+def test_a_capture_does_not_record_a_copy_of_filters(monkeypatch):
+    """While a stream is captured the filters take the copy that is waited for (which the capture refuses): a recorded copy
+    from a pinned buffer of the search's own would read whatever that memory holds at the replay."""
+    idx = VectorIndex(256, DEV, capacity=64)
+    pinned = []
+    pin = torch.Tensor.pin_memory
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t, *a: pinned.append(t) or pin(t, *a))
+    group = torch.tensor([1, 2], dtype=torch.int32)
+    assert torch.equal(idx._there(group).cpu(), group) and len(pinned) == 1
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert torch.equal(idx._there(group).cpu(), group) and len(pinned) == 1
