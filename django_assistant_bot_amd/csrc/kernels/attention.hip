@@ -1669,8 +1669,8 @@ int decode_partition_of(int part_size, int longest, int items, int max_parts) {
 }
 
 // ... and of up to 256 items with two slots, a workgroup a CU: the smallest, in whole 128 keys up to 4096, of which every
-// one that holds keys finds a CU at once (a slot, generally).  A second round waits for the first and pays a start and a combine again; larger
-// partitions leave CUs idle.  Context lengths are known on the device alone, so the workgroups search for it themselves,
+// one that holds keys finds a CU at once (a slot, generally).  A second round waits for the first and pays a start and a
+// combine again; larger partitions leave CUs idle.  Context lengths are known on the device alone, so the workgroups search for it themselves,
 // where not every one has an item of its own to begin with.  parts_of(size): the (sequence, kv head) partitions of that size.
 // us of a layer with its rotation, 8 key heads, (sequences, contexts): apart on one slot with 512 keys / inside, partitions
 // doubled until they fit or are 2048 and walked with their empty ones / these: (9, 2000-4000) 33.5 / 44.6 / 31.2, (9, 4000)
@@ -1854,7 +1854,8 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
     // ... in two steps around the first copies from the cache, so that all of them share one round trip: the loads
     // (positions, slots, the first slabs; then the cosines, behind the position), and the sums and rotations
     using RT = std::conditional_t<FUSED, ROPE, float>;
-    constexpr int HK = FUSED ? NKK / 2 : 1, HELD = !FUSED ? 1 : sizeof(RT) == 4 && NSLOT == 1 ? 2 : 4;  // chunk pairs of a q row, slabs held between the steps
+    constexpr int HK = FUSED ? NKK / 2 : 1;  // chunk pairs of a q row
+    constexpr int HELD = !FUSED ? 1 : sizeof(RT) == 4 && NSLOT == 1 ? 2 : 4;  // slabs held between the steps
     SlabVec8<RT> qa[HK][HELD], qb[HK][HELD], na[HELD], nb[HELD];
     float2 q_cs[HK][8], n_cs[8];
     int64_t new_slot = -1;
@@ -2385,8 +2386,8 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
       else hipLaunchKernelGGL((flash_q64_kernel<false>), gq, dim3(256), 0, s, prm);
       return hipGetLastError();
     }
-    // up to 384 query blocks of at least four a sequence, or 512 of at least eight: the keys of each split over two wave groups (SPLIT), heaviest blocks
-    // first.  us, one block or pair a workgroup -> split, 32 heads: 400 tokens 16.3 -> 15.5, 700 23.6 -> 19.6, 1093 36.0 ->
+    // up to 384 query blocks of at least four a sequence, or 512 of at least eight: the keys of each split over two wave
+    // groups (SPLIT), heaviest blocks first.  us, one block or pair a workgroup -> split, 32 heads: 400 tokens 16.3 -> 15.5, 700 23.6 -> 19.6, 1093 36.0 ->
     // 26.4, 1500 56.0 -> 38.1, 2000 66.7 -> 57.1, 2 x 600 26.6 -> 24.5, 3 x 500 27.8 -> 27.4, 2 x 900 40.5 -> 37.0, 2 x
     // 1000 43.3 -> 40.1; not taken 200 11.6 -> 11.9 (the second group's sums cost 1.7), 4 x 300 18.2 -> 23.1, 4 x 480 28.0 ->
     // 30.7, 3 x 600 29.7 -> 32.0, 4 x 700 44.1 -> 48.7, 16 x 250 32.9 -> 50.8
@@ -2575,7 +2576,7 @@ int paged_decode_attention(const void* q, const void* k_cache, const void* v_cac
   // K/V are read exactly once per step: non-temporal loads (aux = 2) -- in the Llama-3-8B decode step
   // at batch 128 this took the attention from 127 to 111 us per layer (5.1 -> 5.8 TB/s;
   // profiles/decode_round2.md).  D = 128 stages K / V by LDS-DMA (100.7 vs 102.6 us isolated, same
-  // section); D = 64 (small test models) keeps the register path.
+  // section); D = 64 (Llama-3.2-1B) keeps the register path.
   if (D == 128) {
     if (fused && rope->bf16_slabs)
       hipLaunchKernelGGL((paged_decode_kernel<128, true, true, 2, false, bf16>), grid, dim3(256), 0, s, prm, total_items);

@@ -269,8 +269,8 @@ int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const 
 }
 
 // Causal attention of packed queries [T, Hq, 64] over a paged cache.
-int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, const void* v_cache, const int* tables, int max_blocks,
-                  int block_size, void* out, long o_tok, long o_head, const int* cu, const int* ctx, int batch, int max_q, int Hq,
+int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, const void* v_cache, const int* tables,
+                  int max_blocks, int block_size, void* out, long o_tok, long o_head, const int* cu, const int* ctx, int batch, int max_q, int Hq,
                   int Hkv, float scale, hipStream_t s) {
   if (batch <= 0 || max_q <= 0) return 0;
   if (Hkv <= 0 || Hq % Hkv || !(scale > 0.f) || block_size <= 0 || block_size % 64 ||

@@ -1,7 +1,7 @@
 // The sentence encoder's forward as one call: every launch of its layers enqueued from native code.
 //
-// For one question the GPU works about 0.25 ms on 50 launches (0.45 ms on 87 with the LayerNorms and the attention apart),
-// and issuing those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a
+// For one question the GPU works 0.26 ms on 52 launches (0.45 ms on 87 with the LayerNorms and the attention apart), and
+// issuing those from Python took 1.06 ms (11.6 us a launch: wrapper, checks, a tensor for each result).  Here a
 // launch costs the runtime's own 1-2 us; the five activation buffers are the caller's, shared by all layers.  (The
 // reference runs one text a call through an eager model: ai/embedders/transformers.py:15-29.)
 #include "common.h"
@@ -53,8 +53,8 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
 }
 
 // Packed token ids [T] -> hidden states x [T, H].  `layers`: per layer qkv, o, ln1, i, d, ln2 as (weight, bias) or (gain,
-// offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att [T, H], qkv [T, 3 H], ffn [T, F], slabs
-// [slices, T, H] fp32 where the down projection is cut into K-slices that the LayerNorm behind it sums (slab_slices), or null.
+// offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att
+// [T, H], qkv [T, 3 H], ffn [T, F], slabs [slices, T, H] fp32 where the down projection is cut into K-slices that the LayerNorm behind it sums (slab_slices), or null.
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,
                     const void* offset, const uintptr_t* layers, void* x_, void* y_, void* att_, void* qkv_, void* ffn_,

@@ -892,7 +892,9 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   // keep some 11 row panels under way on an XCD instead of 4; the panels' second and third reads find them on the chip.  us
   // behind a LayerNorm that wrote A, 4 rows x all columns -> this: (108800, 2304, 768) 439 -> 355, (95000, 2304, 768) 345 ->
   // 295, (80000, 2304, 1024) 368 -> 313, (108800, 3072, 768) 532 -> 473, (108800, 1792, 768) 300 -> 311; below that
-  // (80000, 2304, 768) 235 -> 240.  The GELU epilogue covers it: up of 108800 rows 553 us either way.
+  // (80000, 2304, 768) 235 -> 240.  A last block of one or two columns gains less or nothing, behind an addition that wrote A:
+  // (108800, 2560, 768) 389 -> 368, (108800, 2048, 768) 357 -> 320, (108800, 1792, 768) 291 -> 294.  The GELU epilogue covers
+  // it: up of 108800 rows 553 us either way.
   const bool far_a = K <= 1024 && !b_shuf && !residual && epilogue == G_NONE && (long)M * K * 2 >= (128L << 20);
   // Otherwise groups of 4 tile rows; where there are many columns, even ones of up to 6: the 32 tiles an XCD runs at once are
   // then 6 row panels and 5-6 column panels, the fewest, and no group of one row is left over that reads 32.  us a step of

@@ -518,8 +518,8 @@ int gemm_mid_ok(int M, int N, int K, long lda) {
 }
 
 // Estimated us of a product on `groups` groups.  Its K-steps take 0.7 each, from some 120 working workgroups on 0.5 +
-// 0.00165 a workgroup, or the weights' way from memory (4.5 TB/s), whichever is longer; its ends 5.6 for whole tiles, 8.1 and 1.56 a part where every tile is cut into
-// parts of as many K-steps, 10.5 and 1.56 a part otherwise, and 2.5 for each further tile of a group.  (Fitted to 1,480
+// 0.00165 a workgroup, or the weights' way from memory (4.5 TB/s), whichever is longer; its ends 5.6 for whole tiles, 8.1
+// and 1.56 a part where every tile is cut into parts of as many K-steps, 10.5 and 1.56 a part otherwise, and 2.5 for each further tile of a group.  (Fitted to 1,480
 // launches of 1-32 row tiles, N 256-28,672, K 256-14,336: half of them within 5 %, nine of ten within 16 %.)
 static double mid_us(int M, int N, int K, int groups) {
   const int tm = (M + 127) / 128, tn = N / 256, kt = K / 64;

@@ -638,8 +638,8 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
 // workgroup each, whose share of the operands from past L2 is what takes the time; in slices they are up to two workgroups of
 // 64 x 64 a CU (one and a half where K is above 2048), or one of 128 x 128.  Between those, below 139 tiles of 64 x 64 and
 // with a short K the slabs (8 bytes an element and slice there and back) cost more than that.  us of product and LayerNorm,
-// one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 -> 15.9, (2200, 384, 1536) 14.2 -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200, 768,
-// 3072) 29.4 -> 26.2, (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5 -> 13.9,
+// one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 -> 15.9, (2200, 384, 1536) 14.2
+// -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200, 768, 3072) 29.4 -> 26.2, (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5 -> 13.9,
 // (1500, 384, 1536) 12.0 -> 12.3 in three slices of 512, (4600, 768, 3072) 41.8 -> 48.3, (832, 768, 768) 9.5 -> 10.3.
 // Whole calls of the encoder, weights of three copies in turn: bge-base 800 tokens 703 -> 676, 900 735 -> 708, 1400 964 -> 922,
 // 1650 1091 -> 1021, 2500 1293 -> 1207; MiniLM 1850 275 -> 269, 2650 330 -> 321, 3200 391 -> 368, 5000 493 -> 469; not taken bge-base

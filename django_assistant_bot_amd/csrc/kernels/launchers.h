@@ -69,8 +69,8 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
                     const OutputGate* gate = nullptr);  // gate: D = 128, paged, with sink or slopes, over all keys
 // attention_packed.hip: bidirectional self-attention over packed sequences, heads of 64
 bool flash_packed64_wins(long units, int max_len);
-int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, const void* v_cache, const int* tables, int max_blocks,
-                  int block_size, void* out, long o_tok, long o_head, const int* cu, const int* ctx, int batch, int max_q, int Hq,
+int flash_paged64(const void* q, long q_tok, long q_head, const void* k_cache, const void* v_cache, const int* tables,
+                  int max_blocks, int block_size, void* out, long o_tok, long o_head, const int* cu, const int* ctx, int batch, int max_q, int Hq,
                   int Hkv, float scale, hipStream_t s);
 int flash_packed64(const void* q, long q_tok, long q_head, const void* k, const void* v, long kv_tok, long kv_head, void* out,
                    long o_tok, long o_head, const int* cu, int batch, int max_len, int Hq, int Hkv, float scale, hipStream_t s);
@@ -304,14 +304,14 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
             const void* residual, long ldr, int M, int N, int K, int epilogue, hipStream_t s, int b_shuf = 0,
             int b_group = 1);
 
-// gemm_mid.hip (M = 256..4096: mixed serving steps / single prompts; grouped stream-K over the N x K
-// plane, 128 x 256 tiles, in-launch last-arriver combine; B in the shuffle_weights layout;
-// epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
 // norm_stream.hip: RMSNorm(sum of slabs + residual) . W^T of up to 4 decode rows
 int norm_stream_ok(int M, int N, int K, int SO, int bn);
 int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, const void* gain, void* residual_out, float eps,
                 const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn,
                 hipStream_t s);
+// gemm_mid.hip (M = 256..4096: mixed serving steps / single prompts; grouped stream-K over the N x K
+// plane, 128 x 256 tiles, in-launch combine by the owner; B in the shuffle_weights layout;
+// epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
 int gemm_mid_groups(int M, int N, int K);
 double gemm_mid_us(int M, int N, int K);
 int gemm_mid_ok(int M, int N, int K, long lda);

@@ -4,8 +4,8 @@
 //
 // A decode layer of a few sequences is a chain of launches; the two norms of a layer are one small workgroup a row between
 // two weight streams, 3.2 us each for 40 KB of work, most of it launch, round trip and drain.  Here every workgroup of the
-// consuming projection normalises the rows itself: four waves sum the slabs, add the residual and write the normalised
-// slice of K to LDS (the same roundings as rmsnorm_slab_kernel), while the other waves have their whole weight ring on its
+// consuming projection normalises the rows itself: eight waves sum the slabs, add the residual and write the normalised
+// slice of K to LDS (the same roundings as rmsnorm_slab_kernel), while the other four have their whole weight ring on its
 // way, whose first loads take longer from HBM than the norm.  Every workgroup reads all slabs and the residual from L2 or
 // the Infinity Cache, 40 KB a row and CU; 8 / M waves share a row, so that up to 4 rows come in one round trip.  Workgroup 0
 // writes the new residual.

@@ -225,8 +225,8 @@ __device__ __forceinline__ int bin_shift(uint32_t lo, uint32_t hi) { return max(
 // most).  each(f) hands this thread's entries to f; those of the block differ from each other (ordered bits << 32 | ~place), so
 // the histograms of ever narrower ranges end at the latest with one entry a bin.  Leaves hist cleared.
 template <int CAP, typename F>
-__device__ __forceinline__ unsigned long long bound_of(RankShared<CAP>& sh, unsigned long long lo, unsigned long long hi, uint32_t need,
-                                       uint32_t most, F each) {
+__device__ __forceinline__ unsigned long long bound_of(RankShared<CAP>& sh, unsigned long long lo, unsigned long long hi,
+                                                       uint32_t need, uint32_t most, F each) {
   for (uint32_t above = 0;;) {
     const int shift = max(0, 54 - __clzll((long long)(hi - lo)));  // (hi - lo) >> shift < RK_BINS
     sh.hist[threadIdx.x] = 0;
@@ -272,8 +272,8 @@ __device__ __forceinline__ void sort_desc(unsigned long long* key, int P) {
   __syncthreads();
 }
 
-// sh.key[0 .. c) in any order -> emit(place, entry, id, document) for the `kept` (1 .. c) greatest.  lo, hi: of the entries this thread has
-// written; the caller has cleared hist, rank and n and no barrier is due.
+// sh.key[0 .. c) in any order -> emit(place, entry, id, document) for the `kept` (1 .. c) greatest.  lo, hi: of the entries
+// this thread has written; the caller has cleared hist, rank and n and no barrier is due.
 template <int CAP, typename F>
 __device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uint32_t hi, const int64_t* row_ids,
                           const int64_t* row_docs, F emit) {
@@ -347,15 +347,15 @@ __device__ void rank_list(RankShared<CAP>& sh, int c, int kept, uint32_t lo, uin
 }
 
 // One row's candidates (unordered, cnt[row] of them) -> its k best: score, item id, document id, best first, equal
-// scores in row order (lists above 4096: in the list's, which its appends leave open); -inf / -1 past the last.  status[row] = 1 where the list cannot be trusted: it overflowed,
-// or it holds fewer than k entries although a threshold cut rows off.
+// scores in row order (lists above 4096: in the list's, which its appends leave open); -inf / -1 past the last.
+// status[row] = 1 where the list cannot be trusted: it overflowed, or it holds fewer than k entries although a threshold cut rows off.
 //
 // A search's lists hold 1-2 thousand entries for some 250 hits.  A histogram of 1024 bins between the list's least and
 // greatest score leaves little more than the hits (bins are equal steps of the ordered bits: monotone for any scores),
 // and up to 512 entries are ranked by counting the greater ones: one chain of LDS reads instead of the 66 steps of a
 // bitonic sort of the list.  Where more remain (k above some 400, many near-equal scores) they are sorted, up to 2048, or
-// cut by score and row to as many first.  Lists above 4096 are radix-selected.  With the ids and documents in the same launch 7.9 us for 1,300
-// candidates of one query and 9.8 for 128 queries (sorted whole: 22 and 31; radix select of 16,000 and five
+// cut by score and row to as many first.  Lists above 4096 are radix-selected.  With the ids and documents in the same
+// launch 7.9 us for 1,300 candidates of one query and 9.8 for 128 queries (sorted whole: 22 and 31; radix select of 16,000 and five
 // element-wise launches behind it: 61 and 91).
 __global__ __launch_bounds__(SEL_NT) void rank_hits_kernel(const float* __restrict__ cand_val,
                                                            const int* __restrict__ cand_idx,
@@ -581,13 +581,15 @@ __global__ __launch_bounds__(SEL_NT) void top_hits_kernel(const float* __restric
     each_chosen([&](int i) { take(i, bound); });
     __syncthreads();
     if (sh.n_cand > TH_CAND) {  // to what rank_list ranks by counting, or sorts alone
-      bound = bound_of(sh.list, entry((uint32_t)(bound >> 32), n - 1), top, (uint32_t)k, (uint32_t)(k <= RK_FEW ? RK_FEW : RK_MANY), [&](auto f) __attribute__((always_inline)) {
+      auto each_score = [&](auto f) __attribute__((always_inline)) {
         each_chosen([&](int i) {
           const f32x4 v = *reinterpret_cast<const f32x4*>(s + i);
 #pragma unroll
           for (int e = 0; e < 4; ++e) f(entry(float_key(v[e]), i + e));
         });
-      });
+      };
+      bound = bound_of(sh.list, entry((uint32_t)(bound >> 32), n - 1), top, (uint32_t)k,
+                       (uint32_t)(k <= RK_FEW ? RK_FEW : RK_MANY), each_score);
       if (tid == 0) sh.n_cand = 0;
       lo = ~0u, hi = 0u;
       __syncthreads();

@@ -216,7 +216,8 @@ class LlamaModel(FragmentProjections):
         RAG context lengths: fewer combines, longer streams per workgroup) once the (sequence, kv head) pairs cover
         the 256 CUs, ``part_size`` below that.  us a layer of Llama-3-8B, 512 / 2048 keys: 24 sequences of 300-1700
         tokens 26.7 / 30.1, 32 of them 36.7 / 30.5, 48 of 200-1400 36.9 / 32.8, 128 of 900-1500 121.7 / 99.0.  (The
-        kernel halves the partitions of the smallest batches by itself.)"""
+        kernel halves the partitions of the smallest batches by itself, and lengthens those of up to 256 pairs until each
+        finds a workgroup.)"""
         return max(part_size, self.long_part) if batch * self.hkv >= 256 else part_size
 
     def _all_reduce(self, x):
