@@ -2386,13 +2386,14 @@ int flash_attention(const void* q, long q_stride_tok, long q_stride_head, const 
       else hipLaunchKernelGGL((flash_q64_kernel<false>), gq, dim3(256), 0, s, prm);
       return hipGetLastError();
     }
-    // up to 384 query blocks of at least four a sequence, or 512 of at least eight: the keys of each split over two wave
-    // groups (SPLIT), heaviest blocks first.  us, one block or pair a workgroup -> split, 32 heads: 400 tokens 16.3 -> 15.5, 700 23.6 -> 19.6, 1093 36.0 ->
-    // 26.4, 1500 56.0 -> 38.1, 2000 66.7 -> 57.1, 2 x 600 26.6 -> 24.5, 3 x 500 27.8 -> 27.4, 2 x 900 40.5 -> 37.0, 2 x
-    // 1000 43.3 -> 40.1; not taken 200 11.6 -> 11.9 (the second group's sums cost 1.7), 4 x 300 18.2 -> 23.1, 4 x 480 28.0 ->
-    // 30.7, 3 x 600 29.7 -> 32.0, 4 x 700 44.1 -> 48.7, 16 x 250 32.9 -> 50.8
+    // up to 256 query blocks of at least four a sequence, a workgroup a CU, or 512 of at least eight: the keys of each split over
+    // two wave groups (SPLIT), heaviest blocks first.  us, one block or pair a workgroup -> split, 32 heads: 400 tokens 18.5 -> 18.6,
+    // 500 21.3 -> 20.2, 900 31.5 -> 25.8, 1093 37.6 -> 29.9, 1500 56.9 -> 40.8, 2000 67.6 -> 57.0, 2 x 400 18.3 -> 18.6, 2 x 500 21.6 ->
+    // 20.5, 2 x 900 42.5 -> 39.6, 2 x 1000 43.1 -> 41.4; not taken 200 11.6 -> 11.9 (the second group's sums cost 1.7), 3 x 400 24.6
+    // -> 29.3, 3 x 500 29.3 -> 31.7, 2 x 560 25.9 -> 29.3, 2 x 640 30.8 -> 30.0, 2 x 700 29.9 -> 33.5, 2 x 780 34.4 -> 36.0, 4 x 300
+    // 18.2 -> 23.1, 3 x 600 29.7 -> 32.0, 4 x 700 44.1 -> 48.7, 16 x 250 32.9 -> 50.8 (behind 2000 cached tokens 3 x 400 92.6 -> 87.5)
     const long blocks = (long)g32.x * Hq * batch;
-    if (causal && vpipe && !std::getenv("DAB_FLASH_PAIR") && g32.x >= 4 && blocks <= (g32.x >= 8 ? 512 : 384)) {
+    if (causal && vpipe && !std::getenv("DAB_FLASH_PAIR") && g32.x >= 4 && blocks <= (g32.x >= 8 ? 512 : 256)) {
       prm.lpt = ((long)Hq * batch) % 8 == 0;
       hipLaunchKernelGGL((flash_d128_kernel<true, true, 8, false, false, false, false, false, false, true>), g32, dim3(512), 0, s,
                          prm);

@@ -10,7 +10,7 @@ DEV = "cuda"
 
 
 # odd and even numbers of 64-key tiles, a tile of one key, blocks of one query, a sequence without queries, keys of earlier
-# steps (whole tiles and not), heads that divide by the XCDs and not; the last four are on the other side of the rule
+# steps (whole tiles and not), heads that divide by the XCDs and not; the last five are on the other side of the rule
 @pytest.mark.parametrize("Hq,Hkv,lens,past", [
     (8, 2, [385], 0), (8, 2, [448], 0), (8, 2, [449], 0), (8, 2, [512, 1, 0, 130], 0), (6, 2, [513, 400], 0), (8, 2, [400], 64),
     (8, 2, [641], 333), (3, 1, [1093], 0), (8, 8, [385, 64, 70], 8200), (32, 8, [1093], 0), (32, 8, [2048], 0), (32, 8, [1000, 900], 7),
@@ -49,3 +49,33 @@ def test_keys_in_two_groups(Hq, Hkv, lens, past, rope):
             moved = 2.0 ** -8 * ((qh.abs() @ kh.abs().t().contiguous()) * D ** -0.5).masked_fill(mask, 0).amax(1, keepdim=True)
             bound = 2.0 ** -8 * (most + exp.abs()) + (2 * moved * most if rope else 0.0) + 1e-4
             assert ((out[at, h].double() - exp).abs() <= bound).all()
+
+
+# either side of the rule with 32 heads: a workgroup a CU at most, one and a quarter, one and a half, two with blocks enough
+@pytest.mark.parametrize("lens", [[500], [1093], [2000], [500, 500], [400] * 3, [450] * 3, [560, 560], [700, 700], [780, 780], [900, 900]])
+def test_the_rule_costs_no_more_than_a_block_a_workgroup(lens, monkeypatch):
+    """Keys in two groups for 256 to 384 blocks of four to six a sequence took up to 1.2 times as long as a block a workgroup."""
+    Hq, Hkv, D, bs, B, layers = 32, 8, 128, 64, len(lens), 6
+    n = -(-max(lens) // bs)
+    caches = [torch.randn(2, B * n, Hkv, bs, D, device=DEV).to(torch.bfloat16) for _ in range(layers)]
+    bt = torch.randperm(B * n).view(B, n).to(torch.int32).to(DEV)
+    q = torch.randn(sum(lens), Hq, D, device=DEV).to(torch.bfloat16)
+    cu, ctx = torch.tensor([0, *lens]).cumsum(0).to(torch.int32).to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+
+    def us():
+        best = []
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda.synchronize()
+            a.record()
+            for i in range(24):
+                ops.flash_attention_paged(q, *caches[i % layers], bt, cu, ctx, max(lens), causal=True)
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b) / 24 * 1e3)
+        return min(best)
+    taken = us()
+    monkeypatch.setenv("DAB_FLASH_PAIR", "0")
+    single = us()
+    print(f"{lens}: {taken:.1f} us, a block a workgroup {single:.1f}")
+    assert taken <= 1.06 * single
