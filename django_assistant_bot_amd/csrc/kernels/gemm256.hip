@@ -899,10 +899,9 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   // Otherwise groups of 4 tile rows; where there are many columns, even ones of up to 6: the 32 tiles an XCD runs at once are
   // then 6 row panels and 5-6 column panels, the fewest, and no group of one row is left over that reads 32.  us a step of
   // Llama-3-8B (gate_up, 102-112 columns), 4 rows -> these: 1093 tokens (4 + 1 -> 5) 16889 -> 16660, 3000 36434 -> 36171, 11,000
-  // 124055 -> 122744, 7900 83166 -> 83659; not taken 64 columns (Llama-3.2-1B), 9600 tokens 16477 -> 16476, gate_up of 1500 82.4
-  // -> 86.6.
+  // 124055 -> 122744, 7900 83166 -> 83659; Llama-3.2-1B (64 columns) 9600 16477 -> 16476.
   const int tm = (M + 255) / 256, groups = (tm + 5) / 6;
-  p.gm = far_a ? 8 : N / 256 >= 96 ? (tm + groups - 1) / groups : 4;
+  p.gm = far_a ? 8 : N / 256 >= 64 ? (tm + groups - 1) / groups : 4;
   p.cn = far_a ? 3 : N / 256;
   // persistent: one workgroup (128 KB of LDS) per CU walks a strided tile list
   const int nwg = tiles > cus ? cus : tiles;

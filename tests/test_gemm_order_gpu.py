@@ -33,7 +33,7 @@ def test_every_tile_once(M, N):
 
 # one group of 1 and of 6 tile rows, 4 + 4, 5 + 5, 5 + 5 + 3; more than 256 workgroups and fewer
 @pytest.mark.parametrize("M", [1, 1281, 1793, 2305, 3100])
-@pytest.mark.parametrize("cols", [64, 67, 96, 99])
+@pytest.mark.parametrize("cols", [64, 67])
 def test_even_groups_of_rows(M, cols):
     K, N = 128, 256 * cols
     g = torch.Generator(device=DEV).manual_seed(M + cols)
