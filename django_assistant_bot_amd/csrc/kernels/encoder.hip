@@ -54,7 +54,8 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
 
 // Packed token ids [T] -> hidden states x [T, H].  `layers`: per layer qkv, o, ln1, i, d, ln2 as (weight, bias) or (gain,
 // offset) pairs.  Up to 32 or 64 tokens the attention runs inside the output projection (gemm_attn_ok).  Buffers: x, y, att
-// [T, H], qkv [T, 3 H], ffn [T, F], slabs [slices, T, H] fp32 where the down projection is cut into K-slices that the LayerNorm behind it sums (slab_slices), or null.
+// [T, H], qkv [T, 3 H], ffn [T, F], slabs [slices, T, H] fp32 where the down projection is cut into K-slices that the
+// LayerNorm behind it sums (slab_slices), or null.
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,
                     const void* offset, const uintptr_t* layers, void* x_, void* y_, void* att_, void* qkv_, void* ffn_,
@@ -82,7 +83,9 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     const uintptr_t* w = layers + 12 * l;
     auto W = [&](int i) { return (const void*)w[i]; };
     rc = ln ? norm_projection(ln, W(0), W(1), qkv, 3 * H, 0) : projection(x, W(0), W(1), nullptr, qkv, T, 3 * H, H, 0, s);
-    const bool attn_o = gemm_attn_ok(T, H, D, batch) && !(w[2] % 16 || w[3] % 8);
+    // (33-64 tokens of 768, weights of several copies in turn, us a call apart -> inside: one text of 40 370 -> 360, of 56 379 -> 370,
+    // four of 15 379 -> 377, eight of 8 381 -> 383, twenty of 3 378 -> 384: up to four texts)
+    const bool attn_o = gemm_attn_ok(T, H, D, batch) && (T <= 32 || H <= 384 || batch <= 4) && !(w[2] % 16 || w[3] % 8);
     if (!rc && attn_o) rc = gemm_attn(qkv, cu, batch, D, scale, W(2), W(3), x, y, T, H, s);
     if (!rc && !attn_o)
       rc = flash_attention(qkv, 3 * H, D, qkv + H, qkv + 2 * H, 3 * H, D, nullptr, nullptr, nullptr, 0, 0, att, H, D, cu, cu,
