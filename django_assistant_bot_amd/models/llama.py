@@ -421,13 +421,13 @@ class LlamaModel(FragmentProjections):
         return x, residual
 
     def rope_in_decode(self, T: int, meta: AttnMeta) -> bool:
-        """Whether a decode step rotates its rows and writes them to the cache inside the attention.  Heads of 64 up to 128
-        (sequence, kv head) pairs: beyond, that form's two workgroups a CU lose what the launch saves.  us a layer, apart /
-        inside, 8 key heads: 9 sequences of 300-1700 15.5 / 14.3, 16: 19.1 / 19.2, 24: 20.6 / 20.7, of 900-1500 22.5 / 24.3,
-        48 of 2000-4000 62.5 / 67.7."""
+        """Whether a decode step rotates its rows and writes them to the cache inside the attention.  Heads of 64 up to 256
+        (sequence, kv head) pairs: beyond, that form's two workgroups a CU lose on long contexts what the launch saves.  us a
+        step of Llama-3.2-1B, apart / inside: 24 sequences of 151-574 1054 / 1020, of 900-1500 1155 / 1165, 32 of 900-1500 1210 /
+        1171; 40 of 300-1700 1220 / 1218, 36 of 3000-4000 1729 / 1858."""
         D = self.cfg.head_dim
         return (meta.workspace is not None and ops.decode_rope_ok(T, self.hkv, D, meta.part_size)
-                and (D == 128 or T * self.hkv <= 128))
+                and (D == 128 or T * self.hkv <= 256))
 
     @staticmethod
     def _mixed_attention(q, kv: KVCache, li: int, meta: AttnMeta) -> torch.Tensor:
