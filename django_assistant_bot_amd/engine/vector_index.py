@@ -300,7 +300,7 @@ class VectorIndex:
         refuses the copy that is waited for; it would record the other, whose buffer a replay finds in other hands."""
         if self.device.type == "cuda" and not t.is_cuda and not torch.cuda.is_current_stream_capturing():
             own = t.pin_memory()
-            if own.data_ptr() != t.data_ptr():
+            if own is not t:
                 return own.to(self.device, non_blocking=True)
         return t.to(self.device)
 
