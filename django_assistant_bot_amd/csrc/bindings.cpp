@@ -643,10 +643,9 @@ PYBIND11_MODULE(_native, m) {
   });
   m.def("operand_ptrs", &operand_ptrs);
   m.def("gemm_small_ok", &dab::gemm_small_ok);
-  m.def("slab_slices", [](int M, int N, int K) {
-    int tile;
-    return dab::slab_slices(M, N, K, &tile);
-  });
+  m.def("slab_slices", &dab::slab_slices);
+  m.def("ring_tile", &dab::ring_tile);
+  m.def("ring_wins", &dab::ring_wins);
   m.def("gemm_slab", [](u A, u B, u slabs, int M, int N, int K, u s) {
     check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s)), "gemm_slab");
   });

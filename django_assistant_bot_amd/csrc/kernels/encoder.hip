@@ -9,14 +9,15 @@
 
 namespace dab {
 
-// Which tile of gemm_small a projection with row-major weights takes, -1: the 128 x 128 / 256 x 256 kernels.
+// Which tile of gemm_small a projection with row-major weights takes, -1: the 128 x 128 / 256 x 256 kernels unless ring_wins.
+// 2 to 5 are the barrier-stepped ring, whose tile ring_tile (gemm_small.hip) picks.
 //
 // The smallest tile that still gives each CU about one workgroup: K split over a workgroup's waves up to 256 tiles of
 // 16 x 16, 32 x 16, 32 x 32, 32 x 64, and 64 x 64 where K is long (K of 384 and more: every other kernel sums K in one
-// order, so that results there do not depend on M); then the barrier-stepped ring with 32 x 64 tiles up to 320, 64 x 64
-// up to 1200 (1000 where M is over 3 N: each XCD streams the rows again for every column block; 512 where K is long: a
-// K-tile's chain is paid K / 64 times and the larger tile has fewer workgroups to queue), 128 x 128 up to 256.  Both
-// sides of each line, us (us of the tile before -> of the tile after it): 192 tiles of 16 x 16 at (64, 768, 768) 3.1 /
+// order, so that results there do not depend on M); then the barrier-stepped ring up to 1200 tiles of 64 x 64 (1000
+// where M is over 3 N: each XCD streams the rows again for every column block), with a long K up to 512 of them or 256 of
+// 128 x 128.  Both sides of each line, us (us of the tile before -> of the tile after it; the ring with one tile of 32 x 64, 64 x 64
+// or 128 x 128): 192 tiles of 16 x 16 at (64, 768, 768) 3.1 /
 // 3.4, 288 at (19, 2304, 768) 3.6 / 3.4; 192 of 32 x 16 at (128, 768, 768) 3.4 / 3.8, 288 at (64, 2304, 768) 5.3 / 4.1;
 // 192 of 32 x 32 at (256, 768, 768) 3.9 / 4.6, 288 at (128, 2304, 768) 5.3 / 4.8; 192 of 32 x 64 at (512, 768, 768) 5.1
 // / 5.5, with K 3072 11.4 / 14.7, 288 at (256, 2304, 768) 7.9 / 6.4; 224 of 64 x 64 at (870, 1024, 4096) 17.6 / 20.6,
@@ -43,7 +44,8 @@ int small_tile(int M, int N, int K) {
 // y[M, N] = x[M, K] w[N, K]^T + b (GELU) (+ residual), everything contiguous: ops.gemm_bt's choice of kernel.
 static int projection(const bf16* x, const void* w, const void* b, const bf16* residual, bf16* y, int M, int N, int K, int gelu,
                       hipStream_t s) {
-  const int tile = small_tile(M, N, K);
+  int tile = small_tile(M, N, K);
+  if (tile < 0 && ring_wins(M, N, K, gelu, residual != nullptr)) tile = 3;
   if (tile >= 0 && gemm_small_ok(M, N, K, K, K, N, N) &&
       !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8))
     return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s);
@@ -76,8 +78,7 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s);
     return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s);
   };
-  int tile;
-  const int slices = slabs ? slab_slices(T, H, F, &tile) : 0;
+  const int slices = slabs ? slab_slices(T, H, F) : 0;
   const uintptr_t* ln = nullptr;  // the layer's own norm of y, applied in front of the next projection
   for (int l = 0; l < n_layers && !rc; ++l) {
     const uintptr_t* w = layers + 12 * l;

@@ -12,16 +12,17 @@
 //   * two pieces in flight a wave for the 16-wide tiles, one for the larger ones (the eight waves are 64-128 KB in
 //     flight already; a second piece measured the same and took the second workgroup's LDS).
 //
-// gemm_pipe_kernel above that: tiles of 32 x 64 to 128 x 128 over an LDS ring, one barrier a K-tile and counted
-// waits, so the loads of the next K-tiles stay in flight (gemm.hip drains its queue every K-tile).  Its step of
-// about 0.27 us measured the same with deeper rings (6, 8), with fragments read a K-tile ahead, with K rotated by
-// column block and with other shares of the tiles for each XCD.
+// gemm_ring_kernel above that: tiles of 32 x 64 to 128 x 256 over an LDS ring, one barrier a K-tile and counted waits, so
+// the loads of the next K-tiles stay in flight (gemm.hip drains its queue every K-tile).  A K-tile takes 0.26-0.66 us, with
+// the tile's size, not with what is left of the ring (4 and 6 buffers, fragments read a K-tile ahead and K rotated by column
+// block measured the same), so what counts is how many tiles the busiest CU has and how large they are: ring_tile.
 //
-// us at (M, N, K), cold weights, before -> here (gemm.hip 128 x 128; from M = 1024 gemm256):
+// us at (M, N, K), cold weights: gemm.hip's 128 x 128 (from M = 1024 gemm256) -> tiles of 64 x 64 -> here:
 //     19, 768, 768   11.9 -> 3.0     19, 2304, 768  12.0 -> 3.4     19, 3072, 768  15.9 -> 4.0     19, 768, 3072  44.2 -> 5.2
 //    256, 768, 768   13.9 -> 3.9    256, 2304, 768  14.3 -> 6.4    256, 3072, 768  14.9 -> 8.1    256, 768, 3072  34.8 -> 8.6
-//    870, 768, 768   16.1 -> 6.9    870, 2304, 768  16.8 -> 9.3    870, 3072, 768  20.8 -> 12.7   870, 768, 3072  49.1 -> 15.3
-//   2048, 768, 768   22.9 -> 9.7   2048, 2304, 768  25.4 -> 20.2  2048, 3072, 768  26.1 -> 26.1  2048, 768, 3072  64.6 -> 28.5
+//    930, 768, 768   16.1 -> 7.2 -> 6.5     930, 2304, 768  16.8 -> 11.0 -> 9.5    930, 3072, 768  20.8 -> 12.0 -> 10.6
+//   1700, 768, 768    8.7 -> 8.0           1700, 2304, 768  14.3 -> 11.8          1700, 3072, 768  25.5 (gemm256) -> 16.7
+//   2900, 768, 768   12.7 -> 11.1          2900, 768, 3072 (128 x 128, with the norm behind it) 40.3 -> 30.0
 // Epilogues round as gemm.hip does.
 #include "common.h"
 #include "launchers.h"
@@ -466,45 +467,67 @@ __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAtte
   small_finish<16, 16, LDN, W, false, 1>(p, tail, part, m0, n0);
 }
 
-// BM x BN tiles by 2 x 2 waves over a ring of NS K-tiles (64 wide) in LDS, filled by LDS-DMA NS - 1 tiles ahead with
+// BM x BN tiles by WM x WN waves over a ring of NS K-tiles (64 wide) in LDS, filled by LDS-DMA NS - 1 tiles ahead with
 // counted waits: one barrier a K-tile and no drained queue.  LDS rows of 128 B, 16-B chunk c of row r at
-// c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly).
-template <int BM, int BN, int NS, bool GELU, bool SLAB = false>
-__global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
-  constexpr int MI = BM / 32, NI = BN / 32;           // 16 x 16 tiles of a wave
-  constexpr int PA = BM / 32, PB = BN / 32;           // LDS-DMA instructions of a wave for a K-tile (8 rows each)
-  constexpr int kA = BM * 128, kStage = (BM + BN) * 128, kDma = PA + PB;
+// c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly); a copy is 8 rows, and copy q of a
+// K-tile's A and B rows, one behind the other, is wave q mod the waves'.  Bias and residual are asked for at the start: at
+// the end they were one more round trip (0.2-0.7 us).
+constexpr int ring_occupancy(int rows, int waves, int ns) {  // waves a SIMD that the ring leaves room for
+  const int n = 163840 / (rows * 128 * ns) * waves / 4;
+  return n < 1 ? 1 : n > 8 ? 8 : n;
+}
+
+template <int BM, int BN, int WM, int WN, int NS, bool GELU, bool SLAB = false>
+__global__ __launch_bounds__(64 * WM * WN, ring_occupancy(BM + BN, WM * WN, NS)) void gemm_ring_kernel(SmallParams p) {
+  constexpr int W = WM * WN, MI = BM / (16 * WM), NI = BN / (16 * WN);  // 16 x 16 tiles of a wave
+  constexpr int kA = BM * 128, kStage = (BM + BN) * 128, kDma = (BM + BN) / 8 / W;
+  static_assert((BM + BN) % (8 * W) == 0 && BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "whole copies and tiles a wave");
+  static_assert(NS == 3 || NS == 4, "waits for up to two K-tiles ahead");
   __shared__ __attribute__((aligned(16))) char smem[NS * kStage];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = w >> 1, wn = w & 1;
+  const int wm = w / WN, wn = w % WN;
   // SLAB: the tiles of a K-slice have neighbouring ids, so an XCD reads one or two slices of A and a few columns' weights
-  const int tiles_m = (p.M + BM - 1) / BM, tiles = SLAB ? tiles_m * ((p.N + BN - 1) / BN) : 0, id0 = small_id();
+  const int tiles_m = (p.M + BM - 1) / BM, tiles = SLAB ? tiles_m * ((p.N + BN - 1) / BN) : 1, id0 = small_id();
   const int slice = SLAB ? id0 / tiles : 0, id = id0 - slice * tiles;
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
 
   const __amdgpu_buffer_rsrc_t ra = rows_rsrc(p.A, p.M, p.lda, p.K), rb = rows_rsrc(p.B, p.N, p.ldb, p.K);
-  unsigned va[PA], vb[PB];  // rows past the matrix read the last one
+  unsigned at[kDma];  // rows past the matrix read the last one
 #pragma unroll
-  for (int i = 0; i < PA; ++i) {
-    const int r = (4 * i + w) * 8 + (lane >> 3);
-    va[i] = (unsigned)((min(m0 + r, p.M - 1) * p.lda + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2);
-  }
-#pragma unroll
-  for (int i = 0; i < PB; ++i) {
-    const int r = (4 * i + w) * 8 + (lane >> 3);
-    vb[i] = (unsigned)((min(n0 + r, p.N - 1) * p.ldb + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2);
+  for (int i = 0; i < kDma; ++i) {
+    const int r = 8 * (i * W + w) + (lane >> 3), c = 8 * ((lane & 7) ^ ((r >> 1) & 7));
+    at[i] = (unsigned)((r < BM ? min(m0 + r, p.M - 1) * p.lda + c : min(n0 + r - BM, p.N - 1) * p.ldb + c) * 2);
   }
   auto stage = [&](int buf, int kt) {
     char* dst = smem + buf * kStage + w * 1024;
     const unsigned so = (unsigned)kt * 128u;
 #pragma unroll
-    for (int i = 0; i < PA; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (small_lds*)(dst + i * 4096), 16, (unsigned)va[i], so, 0, 0);
-#pragma unroll
-    for (int i = 0; i < PB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (small_lds*)(dst + kA + i * 4096), 16, (unsigned)vb[i], so, 0, 0);
+    for (int i = 0; i < kDma; ++i) {
+      // (which operand: known here but for the copies of a step that holds rows of both)
+      if (8 * (i * W + W) <= BM || (8 * i * W < BM && 8 * (i * W + w) < BM))
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
+    }
   };
+  const int k0 = SLAB ? p.K / 64 * slice / p.slices : 0, nk = (SLAB ? p.K / 64 * (slice + 1) / p.slices : p.K / 64) - k0;
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+    if (t < nk) stage(t, k0 + t);
+  u32x2 bias[NI], res[NI][MI];
+  if constexpr (!SLAB) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int n = n0 + wn * (BN / WN) + 16 * i + 4 * g;
+      bias[i] = p.bias && n < p.N ? *reinterpret_cast<const u32x2*>(p.bias + n) : u32x2{0u, 0u};
+#pragma unroll
+      for (int j = 0; j < MI; ++j) {
+        const int m = m0 + wm * (BM / WM) + 16 * j + li;
+        res[i][j] = p.residual && n < p.N && m < p.M ? *reinterpret_cast<const u32x2*>(p.residual + (size_t)m * p.ldr + n) : u32x2{0u, 0u};
+      }
+    }
+  }
   const int sw = (li >> 1) & 7;
   int rd[2];
 #pragma unroll
@@ -515,14 +538,9 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int k0 = SLAB ? p.K / 64 * slice / p.slices : 0, nk = (SLAB ? p.K / 64 * (slice + 1) / p.slices : p.K / 64) - k0;
-#pragma unroll
-  for (int t = 0; t < NS - 1; ++t)
-    if (t < nk) stage(t, k0 + t);
   int buf = 0;
   for (int t = 0; t < nk; ++t) {
     const int ahead = min(NS - 2, nk - 1 - t);  // K-tiles after t that may stay in flight
-    static_assert(NS <= 4, "waits for up to two K-tiles ahead");
     if (ahead >= 2) small_wait<2 * kDma>();
     else if (ahead == 1) small_wait<kDma>();
     else small_wait<0>();
@@ -530,8 +548,8 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + NS - 1 < nk) stage(buf == 0 ? NS - 1 : buf - 1, k0 + t + NS - 1);
-    const char* sa = smem + buf * kStage + wm * (BM / 2) * 128;
-    const char* sb = smem + buf * kStage + kA + wn * (BN / 2) * 128;
+    const char* sa = smem + buf * kStage + wm * (BM / WM) * 128;
+    const char* sb = smem + buf * kStage + kA + wn * (BN / WN) * 128;
     bf16x8 af[MI][2], bfr[NI][2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -550,41 +568,101 @@ __global__ __launch_bounds__(256) void gemm_pipe_kernel(SmallParams p) {
     __builtin_amdgcn_s_setprio(0);
     buf = buf == NS - 1 ? 0 : buf + 1;
   }
-  // acc[i][j][r] = C[m0 + wm BM/2 + 16 j + li][n0 + wn BN/2 + 16 i + 4 g + r]
+  // acc[i][j][r] = C[m0 + wm BM / WM + 16 j + li][n0 + wn BN / WN + 16 i + 4 g + r]
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int n = n0 + wn * (BN / 2) + 16 * i + 4 * g;
+    const int n = n0 + wn * (BN / WN) + 16 * i + 4 * g;
     if (n >= p.N) continue;
-    if constexpr (SLAB) {
-#pragma unroll
-      for (int j = 0; j < MI; ++j) {
-        const int m = m0 + wm * (BM / 2) + 16 * j + li;
-        if (m < p.M) *reinterpret_cast<f32x4*>(p.slabs + ((size_t)slice * p.M + m) * p.N + n) = acc[i][j];
-      }
-      continue;
-    }
-    f32x4 b4 = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
-      const u32x2 b = *reinterpret_cast<const u32x2*>(p.bias + n);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) b4[q] = bf2f((uint16_t)(b[q >> 1] >> (16 * (q & 1))));
-    }
 #pragma unroll
     for (int j = 0; j < MI; ++j) {
-      const int m = m0 + wm * (BM / 2) + 16 * j + li;
+      const int m = m0 + wm * (BM / WM) + 16 * j + li;
       if (m >= p.M) continue;
-      f32x4 s = acc[i][j] + b4;
+      if constexpr (SLAB) {
+        *reinterpret_cast<f32x4*>(p.slabs + ((size_t)slice * p.M + m) * p.N + n) = acc[i][j];
+        continue;
+      }
+      f32x4 s = acc[i][j];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[q] += bf2f((uint16_t)(bias[i][q >> 1] >> (16 * (q & 1))));
       if constexpr (GELU) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) s[q] = gelu_erf(s[q]);
       }
       if (p.residual) {
-        const u32x2 b = *reinterpret_cast<const u32x2*>(p.residual + (size_t)m * p.ldr + n);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = bf2f(f2bf(s[q])) + bf2f((uint16_t)(b[q >> 1] >> (16 * (q & 1))));
+        for (int q = 0; q < 4; ++q) s[q] = bf2f(f2bf(s[q])) + bf2f((uint16_t)(res[i][j][q >> 1] >> (16 * (q & 1))));
       }
       *reinterpret_cast<u32x2*>(p.C + (size_t)m * p.ldc + n) = u32x2{pack2bf(s[0], s[1]), pack2bf(s[2], s[3])};
     }
+  }
+}
+
+// The ring's tiles, and what their time was fitted with: us = start + round (rounds - 1) + tile c + K-tiles max(step rounds,
+// share c), c tiles on the busiest of 256 CUs, `fit` of them at a time; a GELU 50 ns more for 1000 elements of a tile.
+struct RingTile {
+  int bm, bn, fit;
+  float start, round, tile, step, share;
+};
+constexpr RingTile kRing[] = {{32, 64, 4, 2.28f, 0.f, 0.46f, 0.209f, 0.132f},    {64, 64, 3, 2.52f, 0.89f, 0.42f, 0.256f, 0.201f},
+                              {96, 64, 2, 3.09f, 2.81f, 0.45f, 0.309f, 0.245f},  {96, 96, 2, 3.46f, 3.76f, 0.91f, 0.381f, 0.289f},
+                              {64, 128, 2, 3.15f, 1.72f, 0.92f, 0.316f, 0.264f}, {64, 192, 1, 3.50f, 2.25f, 1.67f, 0.392f, 0.150f},
+                              {128, 192, 1, 4.69f, 4.32f, 2.92f, 0.578f, 0.150f}, {128, 256, 1, 5.34f, 4.64f, 3.36f, 0.660f, 0.157f}};
+constexpr int kRings = sizeof(kRing) / sizeof(kRing[0]);
+
+static float ring_us(const RingTile& t, int M, int N, int K, int gelu, int slices = 1) {
+  const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * slices;
+  const long c = (tiles + 255) / 256, rounds = (c + t.fit - 1) / t.fit;
+  const float steps = K / 64 / slices, step = t.step * rounds, share = t.share * c;
+  return t.start + t.round * (rounds - 1) + (t.tile + (gelu ? 5e-5f * t.bm * t.bn : 0.f)) * c + steps * (step > share ? step : share);
+}
+
+// The tile of the ring with the least estimate.  All of them sum K in one order: the choice changes no bits.  Fitted to 4,300
+// launches (M 200-6400, the projections of encoders of 384, 768 and 1024): half of the estimates within 5 %, nine of ten
+// within 15 %.  Over those shapes 9 % faster than tiles of 64 x 64 (128 x 128 with a long K) and gemm256 as they were chosen
+// before, up to 69 % ((4000, 1024, 1024) 27.6 -> 16.4 us), 0.95 at worst ((560, 1024, 4096) in three slices 16.2 -> 17.0).  Calls of the
+// encoder: bge-base 24 texts of 8-64 tokens 748 -> 716, 1300 tokens 854 -> 766, 2200 1186 -> 1045, 7000 2509 -> 2027; MiniLM
+// 4000 473 -> 404; bge-large 1000 1907 -> 1719, 5000 5604 -> 4609.
+int ring_tile(int M, int N, int K, int gelu, int slices) {
+  int best = 0;
+  for (int i = 1; i < kRings; ++i)
+    if (ring_us(kRing[i], M, N, K, gelu, slices) < ring_us(kRing[best], M, N, K, gelu, slices)) best = i;
+  return best;
+}
+
+// Whether the ring beats gemm256 (row-major weights), or the 128 x 128 kernel where that does not take the shape, at a size
+// that small_tile leaves to them: by a tenth of their estimate, waves of 256 tiles of 256 x 256, each with its epilogue (and
+// 1.6 times that).  Over 1,113 sizes (24 pairs of N and K, M 400-30,000) 8 % faster than without the ring, 0.91 at worst.
+// us, before -> ring: (6400, 768, 768) 24.3 -> 17.2, (5300, 1152, 384) 15.8 -> 11.2, (17500, 1000, 768) 86 -> 53; the other way
+// (3200, 3072, 768) 26.1 / 28.4, (4600, 2304, 768) 21.9 / 32; wrongly (20000, 1152, 384) 46 / 36, (4000, 2048, 512) 16.9 / 15.3.
+bool ring_wins(int M, int N, int K, int gelu, int residual) {
+  if (M <= 0 || N <= 0 || K < 64) return false;
+  const long waves = ((long)((M + 255) / 256) * ((N + 255) / 256) + 255) / 256;
+  const float us = 2.1f + waves * (0.0146f * K + 7.f + (gelu ? 5.7f : 0.f) + (residual ? 3.9f : 0.f));
+  const float other = gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K) ? us : 1.6f * us;
+  return ring_us(kRing[ring_tile(M, N, K, gelu, 1)], M, N, K, gelu) < 0.9f * other;
+}
+
+template <int I, int WM, int WN, int NS>
+static void ring_launch(const SmallParams& p, int gelu, hipStream_t s) {
+  constexpr RingTile t = kRing[I];
+  const int slices = p.slabs ? p.slices : 1;
+  const dim3 grid(((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * slices), block(64 * WM * WN);
+  if (p.slabs) hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, false, true>), grid, block, 0, s, p);
+  else if (gelu) hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, false>), grid, block, 0, s, p);
+}
+
+// The ring buffers are as many as `fit` tiles of them leave room for.
+static void gemm_ring(const SmallParams& p, int gelu, hipStream_t s) {
+  switch (ring_tile(p.M, p.N, p.K, gelu, p.slabs ? p.slices : 1)) {
+    case 0: return ring_launch<0, 2, 2, 4>(p, gelu, s);
+    case 1: return ring_launch<1, 2, 4, 3>(p, gelu, s);
+    case 2: return ring_launch<2, 2, 2, 3>(p, gelu, s);
+    case 3: return ring_launch<3, 2, 2, 3>(p, gelu, s);
+    case 4: return ring_launch<4, 2, 4, 3>(p, gelu, s);
+    case 5: return ring_launch<5, 2, 4, 4>(p, gelu, s);
+    case 6: return ring_launch<6, 4, 2, 3>(p, gelu, s);
+    default: return ring_launch<7, 4, 4, 3>(p, gelu, s);
   }
 }
 
@@ -609,34 +687,26 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
     else hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, false>), dim3(grid), dim3(64 * W_), 0, s, p);     \
     break;                                                                                                      \
   }
-#define PIPE(T, BM_, BN_, NS_)                                                                                  \
-  case T: {                                                                                                    \
-    const int grid = ((M + BM_ - 1) / BM_) * ((N + BN_ - 1) / BN_);                                            \
-    if (gelu) hipLaunchKernelGGL((gemm_pipe_kernel<BM_, BN_, NS_, true>), dim3(grid), dim3(256), 0, s, p);     \
-    else hipLaunchKernelGGL((gemm_pipe_kernel<BM_, BN_, NS_, false>), dim3(grid), dim3(256), 0, s, p);         \
-    break;                                                                                                     \
-  }
   switch (tile) {
     SMALL(0, 1, 1, 8, 2)
     SMALL(1, 2, 1, 8, 2)
-    PIPE(2, 32, 64, 4)
-    PIPE(3, 64, 64, 3)
-    PIPE(4, 64, 64, 4)
-    PIPE(5, 128, 128, 4)
+    case 2:
+    case 3:
+    case 4:
+    case 5: gemm_ring(p, gelu, s); break;
     SMALL(6, 2, 2, 8, 1)
     SMALL(7, 2, 4, 8, 1)
     SMALL(8, 4, 4, 8, 1)
     default: return hipErrorInvalidValue;
   }
-#undef PIPE
 #undef SMALL
   return hipGetLastError();
 }
 
-// K-slices that a long-K projection in front of a LayerNorm (which sums them: layernorm_slabs) is cut into, 0: none, and its
-// tile (64 or 128 wide).  The widths are those of layernorm_slab_kernel's instances.  Its tiles alone leave CUs idle or one
-// workgroup each, whose share of the operands from past L2 is what takes the time; in slices they are up to two workgroups of
-// 64 x 64 a CU (one and a half where K is above 2048), or one of 128 x 128.  Between those, below 139 tiles of 64 x 64 and
+// K-slices that a long-K projection in front of a LayerNorm (which sums them: layernorm_slabs) is cut into, 0: none.  The
+// widths are those of layernorm_slab_kernel's instances.  Its tiles alone leave CUs idle or one workgroup each, whose share of
+// the operands from past L2 is what takes the time; in slices they are up to two workgroups of 64 x 64 a CU (one and a half
+// where K is above 2048), or one of 128 x 128 (ring_tile then takes the tile of the slices).  Between those, below 139 tiles of 64 x 64 and
 // with a short K the slabs (8 bytes an element and slice there and back) cost more than that.  us of product and LayerNorm,
 // one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 -> 15.9, (2200, 384, 1536) 14.2
 // -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200, 768, 3072) 29.4 -> 26.2, (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5 -> 13.9,
@@ -645,14 +715,12 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
 // 1650 1091 -> 1021, 2500 1293 -> 1207; MiniLM 1850 275 -> 269, 2650 330 -> 321, 3200 391 -> 368, 5000 493 -> 469; not taken bge-base
 // in two slices of 1536, 1000 765 -> 776, 1150 818 -> 832, 1300 847 -> 861 (with the weights on the die 773 -> 751 at 1180), 1300
 // in three of 128 x 128 847 -> 869; bge-large 765 in two of 2048 1757 -> 1788.
-int slab_slices(int M, int N, int K, int* tile) {
+int slab_slices(int M, int N, int K) {
   if (M <= 0 || K < 1536 || K % 64 || (N != 384 && N != 768 && N != 1024)) return 0;
   const long t64 = ((M + 63) / 64) * (long)(N / 64), t128 = ((M + 127) / 128) * (long)(N / 128);
-  *tile = 64;
   if (t64 >= 139 && t64 <= 170 && K >= 3 * 768) return 3;
   if (t64 >= 171 && t64 <= (K <= 2048 ? 256 : 180) && K < 4096) return 2;
   if (t64 <= 256) return 0;
-  *tile = 128;
   if (t128 >= 64 && t128 <= 85) return 3;
   if (t128 >= 96 && t128 <= 128) return 2;
   return 0;
@@ -660,14 +728,11 @@ int slab_slices(int M, int N, int K, int* tile) {
 
 // slabs [slices][M][N] fp32 = the K-slices' sums of A w^T, as slab_slices says
 int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s) {
-  int tile = 0;
-  const int slices = slab_slices(M, N, K, &tile);
+  const int slices = slab_slices(M, N, K);
   if (!slices || !gemm_small_ok(M, N, K, K, K, N, 0)) return hipErrorInvalidValue;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)slabs) % 16) return hipErrorInvalidValue;
   const SmallParams p = {(const bf16*)A, (const bf16*)B, nullptr, nullptr, nullptr, M, N, K, K, K, N, 0, (float*)slabs, slices};
-  const dim3 grid(((M + tile - 1) / tile) * (N / tile) * slices);
-  if (tile == 64) hipLaunchKernelGGL((gemm_pipe_kernel<64, 64, 4, false, true>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((gemm_pipe_kernel<128, 128, 4, false, true>), grid, dim3(256), 0, s, p);
+  gemm_ring(p, 0, s);
   return hipGetLastError();
 }
 

@@ -390,7 +390,9 @@ int gemm_attn_ok(int T, int H, int D, int batch);
 int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
               void* y, int T, int H, hipStream_t s);
 int gemm_ln_ok(int M, int N, int K, int tile);
-int slab_slices(int M, int N, int K, int* tile);
+int slab_slices(int M, int N, int K);
+int ring_tile(int M, int N, int K, int gelu, int slices);
+bool ring_wins(int M, int N, int K, int gelu, int residual);
 int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
             int M, int N, int K, int gelu, int tile, hipStream_t s);
