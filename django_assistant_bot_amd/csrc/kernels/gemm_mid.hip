@@ -113,6 +113,29 @@ __device__ __forceinline__ int grp_owner(int i, int q, int r) {
   return i < big ? i / (q + 1) : r + (i - big) / q;
 }
 
+// Row tile and group of a block, false where it has none: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that
+// whole groups leave over are joined, XCD after XCD, into further groups.
+//   LAST_FIRST: groups of later blocks hold earlier parts of the iteration space.  An owner waits for the groups behind it,
+// whose workgroups so stand in front of its own in the order of placement: the first workgroup of a launch that has not ended
+// waits for nobody, and a launch whose workgroups fill a CU's registers ends however few of them are resident.  Otherwise the
+// groups of an XCD follow each other, and most of their partial tiles are read from its L2 (128-row kernel, LAST_FIRST instead:
+// (384, 4096, 4096) 29.4 -> 33.4 us, (2000, 6144, 4096) 87 -> 98; the 256-row kernel's 8 MB an XCD don't fit: 148 against 150).
+template <bool LAST_FIRST>
+__device__ __forceinline__ bool grp_place(const GMid& p, int bid, int& mt, int& j) {
+  const int x = bid & 7, slot = bid >> 3, whole = 8 * p.gpx;
+  int g = slot / p.tiles_m;
+  mt = slot - g * p.tiles_m;
+  if (g < p.gpx) {
+    j = LAST_FIRST ? p.gn - 1 - (8 * g + x) : x * p.gpx + g;
+    return true;
+  }
+  const int over = p.spx - p.gpx * p.tiles_m, u = x * over + slot - p.gpx * p.tiles_m;
+  g = u / p.tiles_m;
+  mt = u - g * p.tiles_m;
+  j = LAST_FIRST ? p.gn - whole - 1 - g : whole + g;
+  return g < p.gn - whole;
+}
+
 }  // namespace
 
 // BK: K-step width (see MidGeo); DIAG (timing only, benchmarks/gemm_bench.py): 1 = partial tiles
@@ -125,22 +148,13 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   // behind the ring: the count the launch's number comes from
   __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem + 256];
 
-  // ---- which group / row tile this block is: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that whole
-  // groups leave over are joined, XCD after XCD, into further groups
   const int bid = blockIdx.x, tid = threadIdx.x;
-  const int x = bid & 7, slot = bid >> 3;
-  unsigned* const ended = p.ended + 32 * x;
+  unsigned* const ended = p.ended + 32 * (bid & 7);
   auto count_out = [&]() {
     if (tid == 0) __hip_atomic_fetch_add(ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  int g = slot / p.tiles_m, mt = slot - g * p.tiles_m, j = x * p.gpx + g;
-  if (g >= p.gpx) {
-    const int over = p.spx - p.gpx * p.tiles_m, u = x * over + slot - p.gpx * p.tiles_m;
-    g = u / p.tiles_m;
-    mt = u - g * p.tiles_m;
-    j = 8 * p.gpx + g;
-    if (j >= p.gn) return count_out();  // whole workgroup (uniform)
-  }
+  int mt, j;
+  if (!grp_place<false>(p, bid, mt, j)) return count_out();  // whole workgroup (uniform)
   const int start = grp_start(j, p.q, p.r);
   const int end = start + p.q + (j < p.r ? 1 : 0);
   if (end <= start) return count_out();
@@ -499,6 +513,352 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   count_out();
 }
 
+// Tiles of 256 x 256 with the same split of the iteration space (in pairs of K-steps), partial tiles and flags.  What bounds
+// the kernel above is the way of its loads into a CU: 48 KB a K-step (64 B a cycle at best, 43 measured from L2) against 1024
+// cycles of MFMAs; with both operands' addresses held still its K-step takes as long, and weights straight into registers
+// instead of LDS gain nothing.  A tile of 256 rows loads 32 KB for the same MFMAs.  Loop, staging and LDS layout are those of
+// gemm256: two buffers of K-steps, a phase of two quadrants of 128 x 128, pieces of 16 KB restaged one phase after their last
+// read and waited for three phases later.
+namespace {
+constexpr int kWBuf = 65536, kWHalf = 16384;  // a K-step: A0 | A1 | B0 | B1, 128 rows of 128 B each
+constexpr int kWE = 16, kWSlabSt = 32;        // VMEM stores per wave of an epilogue and of a published partial tile
+constexpr int kWSlabFloats = 256 * 256;       // one a workgroup: only the first part of its range can be another's tile
+static_assert(kWSlabFloats == 2 * kSlabFloats, "the partial tiles of both kernels take the same workspace");
+}  // namespace
+
+template <int EPI, bool RES>
+__global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
+  // behind the buffers: the count the launch's number comes from, and whether an owner's waits ended well
+  __shared__ __attribute__((aligned(16))) char smem[2 * kWBuf + 256];
+
+  const int bid = blockIdx.x, tid = threadIdx.x;
+  unsigned* const ended = p.ended + 32 * (bid & 7);
+  auto count_out = [&]() {
+    if (tid == 0) __hip_atomic_fetch_add(ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  int mt, j;
+  if (!grp_place<true>(p, bid, mt, j)) return count_out();
+  const int start = grp_start(j, p.q, p.r);
+  const int end = start + p.q + (j < p.r ? 1 : 0);
+  if (end <= start) return count_out();
+
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w >> 2, wc = w & 3;
+  const int li = lane & 15, gq = lane >> 4;
+  const int m0 = mt * 256;
+  const int kt = p.kt;  // pairs of K-steps per tile
+
+  // ---- LDS-DMA staging, as the kernel above: piece = 128 rows of A (16-B chunk c of row r at c ^ ((r >> 1) & 7), swizzled
+  // at the source) or 8 blocks of 16 weight rows, 2 KB each
+  const int cc = (lane & 7) ^ ((4 * (w & 1) + (lane >> 4)) & 7);
+  const unsigned vA0 = (unsigned)(((8 * w + (lane >> 3)) * p.lda + 8 * cc) * 2), rowsA = (unsigned)(64 * p.lda * 2);
+  const unsigned kblk = (unsigned)(p.K / 32) * 1024u;
+  const bool bgrp = p.bgrp == 8;
+  const unsigned cb = bgrp ? 8192u : 1024u;
+  const unsigned vB0 = (unsigned)(lane * 16) + (unsigned)w * (bgrp ? 1024u : kblk);
+  const long a_rows = min(256, p.M - m0);
+  const __amdgpu_buffer_rsrc_t rA = mk_rsrc(p.A + (size_t)m0 * p.lda, (unsigned)(((a_rows - 1) * p.lda + p.K) * 2));
+  const __amdgpu_buffer_rsrc_t rB = mk_rsrc(p.B, p.b_bytes);
+  auto stage_a = [&](int buf, int half, int ks) {
+    char* dst = smem + buf * kWBuf + half * kWHalf + w * 1024;
+    const unsigned v0 = vA0 + (half ? 2u * rowsA : 0u), v1 = v0 + rowsA, so = (unsigned)ks * 128u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)dst, 16, v0, so, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)(dst + 8192), 16, v1, so, 0, 0);
+  };
+  auto stage_b = [&](int buf, int half, int nt, int ks) {
+    char* dst = smem + buf * kWBuf + (2 + half) * kWHalf + w * 2048;
+    const unsigned v0 = vB0 + (half ? 8u * kblk : 0u), v1 = v0 + cb, so = (unsigned)nt * 16u * kblk + (unsigned)ks * 2u * cb;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)dst, 16, v0, so, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)(dst + 1024), 16, v1, so, 0, 0);
+  };
+
+  // ---- fragment reads
+  // (buffer 1's offsets in registers of their own: past the 64 KB of an instruction's offset hipcc adds each read's anew)
+  int rdA[2][2], rdB[2];
+#pragma unroll
+  for (int buf = 0; buf < 2; ++buf) {
+    rdA[buf][0] = buf * kWBuf + (64 * wr + li) * 128 + 16 * (gq ^ (li >> 1));
+    rdA[buf][1] = buf * kWBuf + (64 * wr + li) * 128 + 16 * ((4 + gq) ^ (li >> 1));
+    rdB[buf] = buf * kWBuf + 2 * kWHalf + wc * 4096 + lane * 16;
+    asm volatile("" : "+v"(rdA[buf][0]), "+v"(rdA[buf][1]), "+v"(rdB[buf]));
+  }
+  bf16x8 af[4][2], bfr[2][2][2];
+  f32x4 acc[2][2][4][2];
+  auto zero_acc = [&]() {
+#pragma unroll
+    for (int e = 0; e < 32; ++e) acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  zero_acc();
+#define WIDE_READ_A(BUF, IH)                                                                  \
+  _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                             \
+    const char* base = smem + (IH) * kWHalf + i * 2048;                                       \
+    af[i][0] = *reinterpret_cast<const bf16x8*>(base + rdA[BUF][0]);                          \
+    af[i][1] = *reinterpret_cast<const bf16x8*>(base + rdA[BUF][1]);                          \
+  }
+#define WIDE_READ_B(BUF)                                                                      \
+  _Pragma("unroll") for (int jh = 0; jh < 2; ++jh)                                            \
+  _Pragma("unroll") for (int jn = 0; jn < 2; ++jn) {                                          \
+    const char* base = smem + jh * kWHalf + jn * 2048 + rdB[BUF];                             \
+    bfr[jh][jn][0] = *reinterpret_cast<const bf16x8*>(base);                                  \
+    bfr[jh][jn][1] = *reinterpret_cast<const bf16x8*>(base + 1024);                           \
+  }
+#define WIDE_MFMA(IH, JH1)                                                                    \
+  __builtin_amdgcn_s_setprio(1);                                                              \
+  _Pragma("unroll") for (int jj = 0; jj < 2; ++jj)                                            \
+  _Pragma("unroll") for (int ks = 0; ks < 2; ++ks)                                            \
+  _Pragma("unroll") for (int i = 0; i < 4; ++i)                                               \
+  _Pragma("unroll") for (int jn = 0; jn < 2; ++jn)                                            \
+    acc[IH][JH1 ^ jj][i][jn] = mfma16(bfr[JH1 ^ jj][jn][ks], af[i][ks], acc[IH][JH1 ^ jj][i][jn]); \
+  __builtin_amdgcn_s_setprio(0);
+
+  int it = start;
+  int nt = start / kt, k0 = start - nt * kt;
+  // the launch's number: see the kernel above
+  if (w == 0)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(mk_rsrc(ended, 4), (lds_void*)(smem + 2 * kWBuf), 4, 0u, 0u, 0, 0);
+  // prologue: K-step 0 complete, A0 / B0 / B1 of K-step 1 in flight
+  stage_a(0, 0, 2 * k0);
+  stage_b(0, 0, nt, 2 * k0);
+  stage_b(0, 1, nt, 2 * k0);
+  stage_a(0, 1, 2 * k0);
+  stage_a(1, 0, 2 * k0 + 1);
+  stage_b(1, 0, nt, 2 * k0 + 1);
+  stage_b(1, 1, nt, 2 * k0 + 1);
+  wait_vmc<8>();
+  mbar();
+  unsigned before;
+  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+               : "=v"(before)
+               : "v"((unsigned)(uintptr_t)(lds_void*)(smem + 2 * kWBuf))
+               : "memory");
+  const int launch = (int)((unsigned)__builtin_amdgcn_readfirstlane((int)before) / (unsigned)p.spx) + 1;
+
+  const __amdgpu_buffer_rsrc_t rS = mk_rsrc(p.slabs, p.slab_bytes);
+  auto slab_off = [&](int jj) { return (unsigned)((mt * p.gn + jj) * kWSlabFloats) * 4u + (unsigned)(tid * 16); };
+  auto flag_of = [&](int jj) { return p.cnt + mt * p.gn + jj; };
+  bool pending = false;  // the first part is stored as a partial tile, its flag not raised yet
+  auto raise_flag = [&]() {  // after every wave's stores retired and a barrier
+    if (tid == 0) __hip_atomic_store(flag_of(j), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    pending = false;
+  };
+  int after_st = 0;  // VMEM stores younger than the copies in flight
+  while (it < end) {
+    const int k1 = min(kt, k0 + (end - it));
+    it += k1 - k0;
+    const bool more = it < end;
+    if (wr == 1) mbar();  // group 1 one barrier behind through the K-loop (ping-pong)
+    for (int k = k0; k < k1; ++k) {
+      const bool last = k == k1 - 1;
+      const bool st = !last || more;
+      const int ks = 2 * k + 1, kn = last ? 0 : 2 * k + 2, nn = last ? nt + 1 : nt;
+      // phase 1
+      WIDE_READ_A(0, 0)
+      WIDE_READ_B(0)
+      stage_a(1, 1, ks);
+      if (after_st == kWSlabSt) wait_vmc<8 + kWSlabSt>();
+      else if (after_st == kWE) wait_vmc<8 + kWE>();
+      else wait_vmc<8>();
+      mread_bar();
+      WIDE_MFMA(0, 0)
+      mbar();
+      // phase 2
+      WIDE_READ_A(0, 1)
+      if (st) {
+        stage_a(0, 0, kn);
+        stage_b(0, 0, nn, kn);
+        stage_b(0, 1, nn, kn);
+        if (after_st == kWSlabSt) wait_vmc<8 + kWSlabSt>();
+        else if (after_st == kWE) wait_vmc<8 + kWE>();
+        else wait_vmc<8>();
+      } else {
+        wait_vmc<0>();
+      }
+      after_st = 0;
+      mread_bar();
+      WIDE_MFMA(1, 1)
+      mbar();
+      // phase 3
+      WIDE_READ_A(1, 0)
+      WIDE_READ_B(1)
+      if (st) {
+        stage_a(0, 1, kn);
+        wait_vmc<8>();
+      }
+      mread_bar();
+      WIDE_MFMA(0, 0)
+      mbar();
+      if (pending) raise_flag();  // both groups are past phase 3's wait, which retired the stores
+      // phase 4
+      WIDE_READ_A(1, 1)
+      if (st) {
+        stage_a(1, 0, kn + 1);
+        stage_b(1, 0, nn, kn + 1);
+        stage_b(1, 1, nn, kn + 1);
+        wait_vmc<8>();
+      }
+      mread_bar();
+      WIDE_MFMA(1, 1)
+      mbar();
+    }
+    if (wr == 0) mbar();  // pairs with group 1's last K-loop barrier
+
+    // ---- end of a part: as in the kernel above
+    const int n0 = nt * 256;
+    bool write = true;
+    if (k0 != 0 || k1 != kt) {
+      const int j_lo = grp_owner(nt * kt, p.q, p.r), j_hi = grp_owner(nt * kt + kt - 1, p.q, p.r);
+      if (j != j_lo) {
+        const unsigned own = slab_off(j);
+#pragma unroll
+        for (int e = 0; e < 32; ++e)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1]), rS, own,
+                                                 (unsigned)(e * 8192), 16);
+        after_st = kWSlabSt;
+        pending = true;
+        if (!more) {  // nothing left to hide the drain behind
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          mbar();
+          raise_flag();
+        }
+        write = false;
+      } else {
+        bool ok = true;
+        for (int jj = j_lo + 1; jj <= j_hi; ++jj) {
+          int* fl = flag_of(jj);
+          if (tid == 0) {
+            long spins = 0;
+            while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != launch) {
+              if (++spins > p.spin_limit) {
+                ok = false;  // a producer never published (cannot happen in a healthy launch)
+                break;
+              }
+              __builtin_amdgcn_s_sleep(2);
+            }
+            if (ok) __hip_atomic_store(fl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          mbar();  // every thread loads only after lane 0 saw the flag
+          const unsigned off = slab_off(jj);
+          u32x4 v[16];  // a window: half of the partial tile
+#pragma unroll
+          for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)(e * 8192), 16);
+#pragma unroll
+          for (int e = 0; e < 32; ++e) {
+            acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] += __builtin_bit_cast(f32x4, v[e & 15]);
+            if (e < 16) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)((16 + e) * 8192), 16);
+          }
+        }
+        // Lane 0 tells the others, by asm statements on the one LDS array: __syncthreads_and brings an object of its own, and
+        // with two of them hipcc waits for every copy in flight ahead of each fragment read
+        const unsigned told = (unsigned)(uintptr_t)(lds_void*)(smem + 2 * kWBuf + 64);
+        if (tid == 0) asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" ::"v"(told), "v"((int)ok) : "memory");
+        mbar();
+        int all;
+        asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(all) : "v"(told) : "memory");
+        if (!__builtin_amdgcn_readfirstlane(all)) {
+          const float nan = __builtin_nanf("");
+#pragma unroll
+          for (int e = 0; e < 32; ++e) acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] = f32x4{nan, nan, nan, nan};
+        }
+      }
+    }
+    if (write) {
+      // ---- epilogue: acc[ih][jh][i][jn][r] = C[m0 + 128 ih + 64 wr + 16 i + li][n0 + 128 jh + 32 wc + 16 jn + 4 gq + r];
+      // exactly kWE stores per wave (rows >= M fall outside the descriptor and are dropped)
+      int e_lane = tid & 63;  // (opaque, so that nothing derived from it stays live across the K-loop)
+      asm volatile("" : "+v"(e_lane));
+      const int e_li = e_lane & 15, e_g = e_lane >> 4;
+      const long c_rows = min(256, p.M - m0);
+      const __amdgpu_buffer_rsrc_t rC = mk_rsrc(p.C + (size_t)m0 * p.ldc, (unsigned)(c_rows * p.ldc * 2));
+      if constexpr (glu8_epilogue(EPI)) {
+        f32x4 bg[2], bu[2];
+#pragma unroll
+        for (int jh = 0; jh < 2; ++jh) {
+          bg[jh] = bu[jh] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if constexpr (RES) {
+            const float* fb = reinterpret_cast<const float*>(p.residual) + (n0 + 128 * jh + 32 * wc) / 2 + 4 * e_g;
+            bg[jh] = *reinterpret_cast<const f32x4*>(fb);
+            bu[jh] = *reinterpret_cast<const f32x4*>(fb + p.N / 2);
+          }
+        }
+        if constexpr (RES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int ih = 0; ih < 2; ++ih)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int jh = 0; jh < 2; ++jh) {
+              const int mr = 128 * ih + 64 * wr + 16 * i + e_li;
+              float o[4];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[ih][jh][i][0][r]),
+                                                                __float_as_uint(acc[ih][jh][i][1][r]), false, false);
+                o[r] = glu_act<glu8_act(EPI)>(__uint_as_float(s[0]) + bg[jh][r]) * (__uint_as_float(s[1]) + bu[jh][r]);
+              }
+              u32x2 v;
+              v[0] = pack2bf(o[0], o[1]);
+              v[1] = pack2bf(o[2], o[3]);
+              const int oc = (n0 + 128 * jh + 32 * wc) / 2 + 4 * e_g;
+              __builtin_amdgcn_raw_buffer_store_b64(v, rC, (unsigned)((mr * p.ldc + oc) * 2), 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+      } else {
+        const int cq = 16 * (e_g & 1) + 8 * (e_g >> 1);
+        const __amdgpu_buffer_rsrc_t rR =
+            mk_rsrc(RES ? p.residual + (size_t)m0 * p.ldr : p.residual, RES ? (unsigned)(c_rows * p.ldr * 2) : 0u);
+#pragma unroll
+        for (int ih = 0; ih < 2; ++ih) {
+          u32x4 rv[4][2];
+          if constexpr (RES) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int jh = 0; jh < 2; ++jh)
+                rv[i][jh] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rR, (unsigned)(((128 * ih + 64 * wr + 16 * i + e_li) * p.ldr + n0 + 128 * jh + 32 * wc + cq) * 2), 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int jh = 0; jh < 2; ++jh) {
+              const int mr = 128 * ih + 64 * wr + 16 * i + e_li;
+              float o[8];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[ih][jh][i][0][r]),
+                                                                __float_as_uint(acc[ih][jh][i][1][r]), false, false);
+                o[r] = __uint_as_float(s[0]);
+                o[4 + r] = __uint_as_float(s[1]);
+              }
+              if constexpr (RES) {
+                const u32x4 rw = rv[i][jh];
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {  // round like a bf16 GEMM output, then the bf16 add (HF)
+                  o[2 * qd] = bf2f(f2bf(o[2 * qd])) + __uint_as_float(rw[qd] << 16);
+                  o[2 * qd + 1] = bf2f(f2bf(o[2 * qd + 1])) + __uint_as_float(rw[qd] & 0xffff0000u);
+                }
+              }
+              u32x4 v;
+#pragma unroll
+              for (int qd = 0; qd < 4; ++qd) v[qd] = pack2bf(o[2 * qd], o[2 * qd + 1]);
+              const int nc = n0 + 128 * jh + 32 * wc + cq;
+              __builtin_amdgcn_raw_buffer_store_b128(v, rC, (unsigned)((mr * p.ldc + nc) * 2), 0, 0);
+            }
+        }
+      }
+      after_st = kWE;
+    }
+    zero_acc();
+    k0 = 0;
+    ++nt;
+  }
+#undef WIDE_READ_A
+#undef WIDE_READ_B
+#undef WIDE_MFMA
+  count_out();
+}
+
 namespace {
 int cu_count() {
   int dev = 0, cus = 256;
@@ -567,11 +927,69 @@ int gemm_mid_groups(int M, int N, int K) {
   return groups;
 }
 
-// Estimated us of the launch, infinite where the kernel does not take M.
-double gemm_mid_us(int M, int N, int K) {
+// Estimated us of a product on `groups` groups of the 256-row kernel.  A pair of K-steps takes 1.84 us, from some 75 working
+// workgroups on 1.62 + 0.003 a workgroup and 0.0048 more for each past 192, or the weights' way from memory; the ends 10.7 for
+// whole tiles and, with partial tiles of 256 KB, 0.043 a workgroup and 2.53 a part besides.  (Fitted to 18,400 launches of M
+// 128-4096 at 15 sizes of N 768-28,672, K 1024-14,336: half of them within 3.4 %, nine of ten within 11 %; the groups taken
+// by it cost 1.1 % more than the best in the mean.)
+static double wide_us(int M, int N, int K, int groups) {
+  const int tm = (M + 255) / 256, tn = N / 256, kt = K / 128;
+  const double iters = (double)tn * kt, q = iters / groups, wgs = (groups < iters ? groups : iters) * tm;
+  const double step = fmax(1.84, 1.62 + 0.003 * wgs) + 0.0048 * fmax(0., wgs - 192.);
+  const double weights = (double)tn * 512 * K / 5.9e6;
+  double ends = 10.7, steps = q * step;
+  if (tn % groups) {
+    const bool equal = groups % tn == 0 && kt % (groups / tn) == 0;
+    const double parts = equal ? (double)(groups / tn) : groups > tn ? ceil(kt / fmax(q, 1.)) : 1.;
+    ends = (equal ? 10.8 : 12.0) + 2.53 * parts + 0.043 * wgs;
+    if (!equal) steps = ceil(q) * step;
+  }
+  if (tn > groups) ends += 7.1 * ((double)tn / groups - 1.);
+  return ends + fmax(steps, weights);
+}
+
+// Groups of the 256-row kernel and the estimate of its time on them; 0 groups where it is not measured (K below 1024) or
+// does not take the sizes.
+static int wide_groups(int M, int N, int K, double* us) {
+  const int spx = cu_count() / 8, tm = (M + 255) / 256, tn = N / 256;
+  *us = __builtin_huge_val();
+  if (M <= 0 || tn <= 0 || K < 1024 || K % 128 || tm > spx) return 0;
+  const int whole = 8 * (spx / tm);
+  int groups = 0;
+  for (int g = 8; g <= whole + 8; g += 8) {
+    const int gn = g <= whole ? g : whole + 8 * (spx % tm) / tm;  // (last: with the groups joined from the slots left over)
+    const double t = wide_us(M, N, K, gn);
+    if (t < *us) {
+      *us = t;
+      groups = gn;
+    }
+  }
+  return groups;
+}
+
+// Which kernel a product takes: the 256-row one where the estimates say 2 % less (taken in 750 of the 2,806 sizes of that
+// sweep, 1.24 times as fast in the mean; slower in 15, by 5.5 % at worst: o of 6144 x 4096 at M 2659.  At any lower estimate:
+// 846, slower in 43, by 8 % at worst).  us, 128 rows -> 256: Llama-3-8B's down at M 1280 144 -> 129, 1500 168 -> 149, 2000 198
+// -> 173, 3000 322 -> 266, gate_up at M 700 184 -> 153, 1500 341 -> 286, Llama-3.2-1B's down at 3400 115 -> 97; but o of
+// Llama-3-8B at M 1093 51 -> 57, qkv at 640 41 -> 55: partial tiles of 256 KB a workgroup are 64 MB to write and read, some 30
+// us of a full launch.
+static int mid_pick(int M, int N, int K, bool* wide, double* us) {
   const int groups = gemm_mid_groups(M, N, K);
-  if (!groups) return M <= 0 || N < 256 ? 0. : __builtin_huge_val();
-  return mid_us(M, N, K, groups);
+  *us = groups ? mid_us(M, N, K, groups) : __builtin_huge_val();
+  double w_us;
+  const int w_groups = groups ? wide_groups(M, N, K, &w_us) : 0;
+  *wide = w_groups && w_us < 0.98 * *us;
+  if (!*wide) return groups;
+  *us = 1.03 * w_us;  // (the other kernels' estimates are some 4 % low where the chip is full)
+  return w_groups;
+}
+
+// Estimated us of the launch, infinite where the kernels do not take M.
+double gemm_mid_us(int M, int N, int K) {
+  bool wide;
+  double us;
+  if (mid_pick(M, N, K, &wide, &us)) return us;
+  return M <= 0 || N < 256 ? 0. : __builtin_huge_val();
 }
 
 // Workspace the launcher needs: partial slabs and behind them the counts of ended workgroups (bytes), and ready flags
@@ -589,7 +1007,7 @@ int gemm_mid_counters(int M, int N) {
 // 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs:
 // gemm_mid_slab_bytes() bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the
 // launch leaves them zero).  spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
-// (BK 64), 32 / 64 force the K-step, + 1000 = DIAG 1 (split tiles not combined: timing only).
+// (by the estimates), 32 / 64 the 128-row kernel with that K-step, 256 the 256-row kernel, + 1000 = DIAG 1 (split tiles not combined: timing only).
 // BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank
 // conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
 int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const void* residual, long ldr, int M, int N,
@@ -601,6 +1019,20 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   if (!slabs || !cnt || slab_bytes < gemm_mid_slab_bytes() || n_cnt < gemm_mid_counters(M, N) ||
       slab_bytes >= (1L << 32))
     return hipErrorInvalidValue;
+  bool wide;
+  double us;
+  int groups = mid_pick(M, N, K, &wide, &us);
+  if (variant == 256) {
+    wide = true;
+    groups = wide_groups(M, N, K, &us);
+  } else if (variant) {
+    wide = false;
+  }
+  if (!groups || (wide && (255L * lda + K) * 2 >= (1L << 31))) {
+    if (variant == 256) return hipErrorInvalidValue;
+    wide = false;
+  }
+  if (!wide) groups = gemm_mid_groups(M, N, K);
   const bool diag = variant >= 1000;
   const int bk = (variant % 1000) == 32 ? 32 : 64;
   GMid p{};
@@ -616,14 +1048,15 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.lda = lda;
   p.ldc = ldc;
   p.ldr = ldr;
-  p.tiles_m = (M + 127) / 128;
+  const int rows = wide ? 256 : 128;
+  p.tiles_m = (M + rows - 1) / rows;
   p.tiles_n = N / 256;
-  p.kt = K / bk;
+  p.kt = K / (wide ? 128 : bk);
   const int grid = cu_count() & ~7;
   p.ended = (unsigned*)((char*)slabs + slabs_end());
   p.spin_limit = spin_limit;
   p.spx = grid / 8;
-  p.gn = gemm_mid_groups(M, N, K);
+  p.gn = groups;
   p.gpx = min(p.spx / p.tiles_m, p.gn / 8);  // (with fewer groups the other slots' workgroups end at once)
   const int iters = p.tiles_n * p.kt;
   p.q = iters / p.gn;
@@ -643,7 +1076,17 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
       MID_LAUNCH(E, R, 32, 0);             \
     }                                      \
   } while (0)
-  if (epilogue == MID_SWIGLU8 && residual) MID_BK(MID_SWIGLU8, true);
+#define WIDE_LAUNCH(E, R) hipLaunchKernelGGL((gemm_wide_kernel<E, R>), dim3(grid), dim3(512), 0, s, p)
+  if (wide) {
+    if (epilogue == MID_SWIGLU8 && residual) WIDE_LAUNCH(MID_SWIGLU8, true);
+    else if (epilogue == MID_GEGLU8 && residual) WIDE_LAUNCH(MID_GEGLU8, true);
+    else if (epilogue == MID_SWIGLU8) WIDE_LAUNCH(MID_SWIGLU8, false);
+    else if (epilogue == MID_GEGLU8) WIDE_LAUNCH(MID_GEGLU8, false);
+    else if (epilogue == MID_REGLU8 && residual) WIDE_LAUNCH(MID_REGLU8, true);
+    else if (epilogue == MID_REGLU8) WIDE_LAUNCH(MID_REGLU8, false);
+    else if (residual) WIDE_LAUNCH(MID_NONE, true);
+    else WIDE_LAUNCH(MID_NONE, false);
+  } else if (epilogue == MID_SWIGLU8 && residual) MID_BK(MID_SWIGLU8, true);
   else if (epilogue == MID_GEGLU8 && residual) MID_BK(MID_GEGLU8, true);
   else if (epilogue == MID_SWIGLU8) MID_BK(MID_SWIGLU8, false);
   else if (epilogue == MID_GEGLU8) MID_BK(MID_GEGLU8, false);
@@ -652,6 +1095,7 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   else if (residual) MID_BK(MID_NONE, true);
   else MID_BK(MID_NONE, false);
 #undef MID_BK
+#undef WIDE_LAUNCH
 #undef MID_LAUNCH
   return hipGetLastError();
 }

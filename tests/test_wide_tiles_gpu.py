@@ -1,0 +1,71 @@
+"""gemm_mid's kernel with tiles of 256 rows (variant 256) against an fp32 product."""
+import pytest
+import torch
+
+from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.ops import kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# one row; full and ragged row tiles; whole tiles, equal parts, parts of unequal length, groups joined over the XCDs, more tiles
+# than groups, groups that take part in three tiles, the largest M
+SHAPES = [(1, 256, 1024), (44, 256, 8192), (256, 2048, 1024), (257, 768, 3072), (1093, 4096, 1024), (1300, 2560, 1152),
+          (2200, 6144, 1024), (700, 28672, 1024), (4096, 2048, 2048)]
+
+
+def _case(M, N, K, group):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    A = torch.randn(M, K + 8, device=DEV, generator=g).to(torch.bfloat16)[:, :K]  # rows with a stride of their own
+    W = (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).to(torch.bfloat16)
+    return A, ops.shuffle_weights(W, group), A.float() @ W.float().t()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("group", [1, 8])
+def test_against_the_product(M, N, K, group):
+    A, B, exp = _case(M, N, K, group)
+    res = torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    first = None
+    for _ in range(3):  # the ready flags are down again after each launch, and the order of the sums is fixed
+        out = kernels.gemm_mid(A, B, variant=256, b_group=group)
+        # one rounding to bf16 (2^-8 of the value); the fp32 sums are far below 1e-4
+        assert ((out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-4).all()
+        first = out if first is None else first
+        assert torch.equal(out, first)
+    out = kernels.gemm_mid(A, B, residual=res, variant=256, b_group=group)
+    assert torch.equal(out, (first.float() + res.float()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("epilogue", kernels.GLU8)
+@pytest.mark.parametrize("bias", [False, True])
+def test_glu(M, N, K, epilogue, bias):
+    A, B, exp = _case(M, N, K, 8)
+    v = exp.view(M, N // 16, 2, 8)
+    gate, up = v[:, :, 0].reshape(M, N // 2), v[:, :, 1].reshape(M, N // 2)
+    b = torch.randn(N, device=DEV) if bias else None
+    if bias:
+        gate, up = gate + b[:N // 2], up + b[N // 2:]
+    act = {ops.EPI_SWIGLU8: torch.nn.functional.silu, ops.EPI_REGLU8: torch.relu}.get(
+        epilogue, lambda t: torch.nn.functional.gelu(t, approximate="tanh"))
+    exp = act(gate) * up
+    out = kernels.gemm_mid(A, B, epilogue=epilogue, variant=256, b_group=8, glu_bias=b)
+    # one rounding to bf16; the sums' 1e-4 of either factor times the other's size, at most 8 or so
+    assert ((out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 512, 4096), (1093, 4096, 1024), (2200, 2560, 1024)])
+def test_a_launch_that_gave_up_leaves_nothing_for_the_next(M, N, K):
+    """Owners that look at a flag once write NaN over their tile; the launches behind take only their own partial tiles."""
+    s = torch.cuda.current_stream().cuda_stream
+    A, B, exp = _case(M, N, K, 1)
+    slabs, cnt = kernels._mid_workspace(A.device, s)
+    for _ in range(3):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        kernels.native().gemm_mid(A.data_ptr(), A.stride(0), B.data_ptr(), out.data_ptr(), N, 0, 0, M, N, K, 0, slabs.data_ptr(),
+                                  slabs.numel() * 4, cnt.data_ptr(), cnt.numel(), s, variant=256, spin_limit=0)
+        near = (out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-4
+        assert (near | out.isnan()).all()
+        for variant in (256, 64, 256):
+            out = kernels.gemm_mid(A, B, variant=variant)
+            assert ((out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-4).all()
