@@ -113,29 +113,6 @@ __device__ __forceinline__ int grp_owner(int i, int q, int r) {
   return i < big ? i / (q + 1) : r + (i - big) / q;
 }
 
-// Row tile and group of a block, false where it has none: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that
-// whole groups leave over are joined, XCD after XCD, into further groups.
-//   LAST_FIRST: groups of later blocks hold earlier parts of the iteration space.  An owner waits for the groups behind it,
-// whose workgroups so stand in front of its own in the order of placement: the first workgroup of a launch that has not ended
-// waits for nobody, and a launch whose workgroups fill a CU's registers ends however few of them are resident.  Otherwise the
-// groups of an XCD follow each other, and most of their partial tiles are read from its L2 (128-row kernel, LAST_FIRST instead:
-// (384, 4096, 4096) 29.4 -> 33.4 us, (2000, 6144, 4096) 87 -> 98; the 256-row kernel's 8 MB an XCD don't fit: 148 against 150).
-template <bool LAST_FIRST>
-__device__ __forceinline__ bool grp_place(const GMid& p, int bid, int& mt, int& j) {
-  const int x = bid & 7, slot = bid >> 3, whole = 8 * p.gpx;
-  int g = slot / p.tiles_m;
-  mt = slot - g * p.tiles_m;
-  if (g < p.gpx) {
-    j = LAST_FIRST ? p.gn - 1 - (8 * g + x) : x * p.gpx + g;
-    return true;
-  }
-  const int over = p.spx - p.gpx * p.tiles_m, u = x * over + slot - p.gpx * p.tiles_m;
-  g = u / p.tiles_m;
-  mt = u - g * p.tiles_m;
-  j = LAST_FIRST ? p.gn - whole - 1 - g : whole + g;
-  return g < p.gn - whole;
-}
-
 }  // namespace
 
 // BK: K-step width (see MidGeo); DIAG (timing only, benchmarks/gemm_bench.py): 1 = partial tiles
@@ -148,13 +125,22 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   // behind the ring: the count the launch's number comes from
   __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem + 256];
 
+  // ---- which group / row tile this block is: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that whole
+  // groups leave over are joined, XCD after XCD, into further groups
   const int bid = blockIdx.x, tid = threadIdx.x;
-  unsigned* const ended = p.ended + 32 * (bid & 7);
+  const int x = bid & 7, slot = bid >> 3;
+  unsigned* const ended = p.ended + 32 * x;
   auto count_out = [&]() {
     if (tid == 0) __hip_atomic_fetch_add(ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  int mt, j;
-  if (!grp_place<false>(p, bid, mt, j)) return count_out();  // whole workgroup (uniform)
+  int g = slot / p.tiles_m, mt = slot - g * p.tiles_m, j = x * p.gpx + g;
+  if (g >= p.gpx) {
+    const int over = p.spx - p.gpx * p.tiles_m, u = x * over + slot - p.gpx * p.tiles_m;
+    g = u / p.tiles_m;
+    mt = u - g * p.tiles_m;
+    j = 8 * p.gpx + g;
+    if (j >= p.gn) return count_out();  // whole workgroup (uniform)
+  }
   const int start = grp_start(j, p.q, p.r);
   const int end = start + p.q + (j < p.r ? 1 : 0);
   if (end <= start) return count_out();
@@ -532,15 +518,21 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   __shared__ __attribute__((aligned(16))) char smem[2 * kWBuf + 256];
 
   const int bid = blockIdx.x, tid = threadIdx.x;
-  unsigned* const ended = p.ended + 32 * (bid & 7);
+  const int x = bid & 7, slot = bid >> 3;
+  unsigned* const ended = p.ended + 32 * x;
   auto count_out = [&]() {
     if (tid == 0) __hip_atomic_fetch_add(ended, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  int mt, j;
-  if (!grp_place<true>(p, bid, mt, j)) return count_out();
+  // Each XCD takes p.tiles_n column tiles of its own, whose parts its groups share: later blocks hold earlier parts.  An owner
+  // waits for groups of its XCD alone, whose workgroups stand in front of its own in the order of placement.  The first
+  // workgroup of an XCD that has not ended so waits for nobody, and the launch ends however few of its workgroups are
+  // resident and whatever other launches hold some XCDs (they fill a CU, and fit beside none).
+  const int g = slot / p.tiles_m, mt = slot - g * p.tiles_m, j = p.gpx - 1 - g;
+  if (j < 0) return count_out();  // whole workgroup (uniform)
   const int start = grp_start(j, p.q, p.r);
   const int end = start + p.q + (j < p.r ? 1 : 0);
   if (end <= start) return count_out();
+  const int nt0 = x * p.tiles_n;
 
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -568,7 +560,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   };
   auto stage_b = [&](int buf, int half, int nt, int ks) {
     char* dst = smem + buf * kWBuf + (2 + half) * kWHalf + w * 2048;
-    const unsigned v0 = vB0 + (half ? 8u * kblk : 0u), v1 = v0 + cb, so = (unsigned)nt * 16u * kblk + (unsigned)ks * 2u * cb;
+    const unsigned v0 = vB0 + (half ? 8u * kblk : 0u), v1 = v0 + cb, so = (unsigned)(nt0 + nt) * 16u * kblk + (unsigned)ks * 2u * cb;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)dst, 16, v0, so, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)(dst + 1024), 16, v1, so, 0, 0);
   };
@@ -635,8 +627,9 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   const int launch = (int)((unsigned)__builtin_amdgcn_readfirstlane((int)before) / (unsigned)p.spx) + 1;
 
   const __amdgpu_buffer_rsrc_t rS = mk_rsrc(p.slabs, p.slab_bytes);
-  auto slab_off = [&](int jj) { return (unsigned)((mt * p.gn + jj) * kWSlabFloats) * 4u + (unsigned)(tid * 16); };
-  auto flag_of = [&](int jj) { return p.cnt + mt * p.gn + jj; };
+  auto block_of = [&](int jj) { return ((p.gpx - 1 - jj) * p.tiles_m + mt) * 8 + x; };
+  auto slab_off = [&](int jj) { return (unsigned)(block_of(jj) * kWSlabFloats) * 4u + (unsigned)(tid * 16); };
+  auto flag_of = [&](int jj) { return p.cnt + block_of(jj); };
   bool pending = false;  // the first part is stored as a partial tile, its flag not raised yet
   auto raise_flag = [&]() {  // after every wave's stores retired and a barrier
     if (tid == 0) __hip_atomic_store(flag_of(j), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -704,7 +697,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
     if (wr == 0) mbar();  // pairs with group 1's last K-loop barrier
 
     // ---- end of a part: as in the kernel above
-    const int n0 = nt * 256;
+    const int n0 = (nt0 + nt) * 256;
     bool write = true;
     if (k0 != 0 || k1 != kt) {
       const int j_lo = grp_owner(nt * kt, p.q, p.r), j_hi = grp_owner(nt * kt + kt - 1, p.q, p.r);
@@ -927,37 +920,36 @@ int gemm_mid_groups(int M, int N, int K) {
   return groups;
 }
 
-// Estimated us of a product on `groups` groups of the 256-row kernel.  A pair of K-steps takes 1.84 us, from some 75 working
-// workgroups on 1.62 + 0.003 a workgroup and 0.0048 more for each past 192, or the weights' way from memory; the ends 10.7 for
-// whole tiles and, with partial tiles of 256 KB, 0.043 a workgroup and 2.53 a part besides.  (Fitted to 18,400 launches of M
-// 128-4096 at 15 sizes of N 768-28,672, K 1024-14,336: half of them within 3.4 %, nine of ten within 11 %; the groups taken
-// by it cost 1.1 % more than the best in the mean.)
+// Estimated us of a product on `groups` groups of the 256-row kernel (all XCDs').  A pair of K-steps takes 1.83 us, from some
+// 70 working workgroups on 1.64 + 0.0027 a workgroup and 0.0048 more for each past 192, or the weights' way from memory; the
+// ends 10.4 for whole tiles and, with partial tiles of 256 KB, 0.027 a workgroup and 2.48 a part besides.  (Fitted to 12,900
+// launches of M 128-4096 at 11 sizes of N 2048-28,672, K 1024-14,336: half of them within 2.7 %, nine of ten within 7.5 %;
+// the groups taken by it cost 0.9 % more than the best in the mean.)
 static double wide_us(int M, int N, int K, int groups) {
   const int tm = (M + 255) / 256, tn = N / 256, kt = K / 128;
   const double iters = (double)tn * kt, q = iters / groups, wgs = (groups < iters ? groups : iters) * tm;
-  const double step = fmax(1.84, 1.62 + 0.003 * wgs) + 0.0048 * fmax(0., wgs - 192.);
-  const double weights = (double)tn * 512 * K / 5.9e6;
-  double ends = 10.7, steps = q * step;
+  const double step = fmax(1.83, 1.64 + 0.0027 * wgs) + 0.0048 * fmax(0., wgs - 192.);
+  const double weights = (double)tn * 512 * K / 5.0e6;
+  double ends = 10.4, steps = q * step;
   if (tn % groups) {
     const bool equal = groups % tn == 0 && kt % (groups / tn) == 0;
     const double parts = equal ? (double)(groups / tn) : groups > tn ? ceil(kt / fmax(q, 1.)) : 1.;
-    ends = (equal ? 10.8 : 12.0) + 2.53 * parts + 0.043 * wgs;
+    ends = (equal ? 11.4 : 12.5) + 2.48 * parts + 0.027 * wgs;
     if (!equal) steps = ceil(q) * step;
   }
-  if (tn > groups) ends += 7.1 * ((double)tn / groups - 1.);
+  if (tn > groups) ends += 7.0 * ((double)tn / groups - 1.);
   return ends + fmax(steps, weights);
 }
 
 // Groups of the 256-row kernel and the estimate of its time on them; 0 groups where it is not measured (K below 1024) or
-// does not take the sizes.
-static int wide_groups(int M, int N, int K, double* us) {
+// does not take the sizes (each XCD as many column tiles).  From three row tiles on: with fewer, weights that take longer from
+// memory than the products are slower ((391, 10240, 8192) 0.81 times as fast), and others gain nothing over gemm256.
+static int wide_groups(int M, int N, int K, int min_tm, double* us) {
   const int spx = cu_count() / 8, tm = (M + 255) / 256, tn = N / 256;
   *us = __builtin_huge_val();
-  if (M <= 0 || tn <= 0 || K < 1024 || K % 128 || tm > spx) return 0;
-  const int whole = 8 * (spx / tm);
+  if (M <= 0 || tn <= 0 || K < 1024 || K % 128 || tn % 8 || tm < min_tm || tm > spx) return 0;
   int groups = 0;
-  for (int g = 8; g <= whole + 8; g += 8) {
-    const int gn = g <= whole ? g : whole + 8 * (spx % tm) / tm;  // (last: with the groups joined from the slots left over)
+  for (int gn = 8; gn <= 8 * (spx / tm); gn += 8) {
     const double t = wide_us(M, N, K, gn);
     if (t < *us) {
       *us = t;
@@ -967,20 +959,20 @@ static int wide_groups(int M, int N, int K, double* us) {
   return groups;
 }
 
-// Which kernel a product takes: the 256-row one where the estimates say 2 % less (taken in 750 of the 2,806 sizes of that
-// sweep, 1.24 times as fast in the mean; slower in 15, by 5.5 % at worst: o of 6144 x 4096 at M 2659.  At any lower estimate:
-// 846, slower in 43, by 8 % at worst).  us, 128 rows -> 256: Llama-3-8B's down at M 1280 144 -> 129, 1500 168 -> 149, 2000 198
-// -> 173, 3000 322 -> 266, gate_up at M 700 184 -> 153, 1500 341 -> 286, Llama-3.2-1B's down at 3400 115 -> 97; but o of
-// Llama-3-8B at M 1093 51 -> 57, qkv at 640 41 -> 55: partial tiles of 256 KB a workgroup are 64 MB to write and read, some 30
-// us of a full launch.
+// Which kernel a product takes: the 256-row one where the estimates say 6.5 % less (798 of the 2,109 sizes of that sweep, 1.21
+// times as fast in the mean, slower in 3, by 0.8 % at worst; at 2 % less 881, slower in 10, and the step of Llama-3-8B at 850
+// tokens, down alone on this kernel, 12,864 -> 12,950).  us, 128 rows -> 256: Llama-3-8B's down at M 1280 144 -> 129,
+// 1500 168 -> 148, 2000 198 -> 172, 3000 322 -> 265, gate_up at M 700 184 -> 155, 1500 341 -> 290, Llama-3.2-1B's down at 3400
+// 115 -> 97; but o of Llama-3-8B at M 1093 51 -> 54, qkv at 640 41 -> 53: partial tiles of 256 KB a workgroup are 64 MB to
+// write and read, some 25 us of a full launch.
 static int mid_pick(int M, int N, int K, bool* wide, double* us) {
   const int groups = gemm_mid_groups(M, N, K);
   *us = groups ? mid_us(M, N, K, groups) : __builtin_huge_val();
   double w_us;
-  const int w_groups = groups ? wide_groups(M, N, K, &w_us) : 0;
-  *wide = w_groups && w_us < 0.98 * *us;
+  const int w_groups = groups ? wide_groups(M, N, K, 3, &w_us) : 0;
+  *wide = w_groups && w_us < 0.935 * *us;
   if (!*wide) return groups;
-  *us = 1.03 * w_us;  // (the other kernels' estimates are some 4 % low where the chip is full)
+  *us = 1.1 * w_us;  // (beside gemm256: the step of Llama-3-8B at 3,000 tokens 34,732 us with it, 35,015 on this)
   return w_groups;
 }
 
@@ -1024,7 +1016,7 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   int groups = mid_pick(M, N, K, &wide, &us);
   if (variant == 256) {
     wide = true;
-    groups = wide_groups(M, N, K, &us);
+    groups = wide_groups(M, N, K, 1, &us);
   } else if (variant) {
     wide = false;
   }
@@ -1057,10 +1049,11 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.spin_limit = spin_limit;
   p.spx = grid / 8;
   p.gn = groups;
+  if (wide) p.tiles_n /= 8;  // an XCD's
   p.gpx = min(p.spx / p.tiles_m, p.gn / 8);  // (with fewer groups the other slots' workgroups end at once)
-  const int iters = p.tiles_n * p.kt;
-  p.q = iters / p.gn;
-  p.r = iters % p.gn;
+  const int iters = p.tiles_n * p.kt, shares = wide ? p.gn / 8 : p.gn;
+  p.q = iters / shares;
+  p.r = iters % shares;
   p.b_bytes = (unsigned)((long)N * K * 2);
   p.slab_bytes = (unsigned)slab_bytes;
   p.bgrp = b_group;

@@ -7,9 +7,9 @@ from django_assistant_bot_amd.ops import kernels
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-# one row; full and ragged row tiles; whole tiles, equal parts, parts of unequal length, groups joined over the XCDs, more tiles
-# than groups, groups that take part in three tiles, the largest M
-SHAPES = [(1, 256, 1024), (44, 256, 8192), (256, 2048, 1024), (257, 768, 3072), (1093, 4096, 1024), (1300, 2560, 1152),
+# one row; full and ragged row tiles; one to fourteen column tiles an XCD: whole ones, equal parts, parts of unequal length, more
+# tiles than groups; an odd number of pairs of K-steps; the largest M
+SHAPES = [(1, 2048, 1024), (44, 2048, 8192), (256, 4096, 1024), (257, 6144, 3072), (1093, 4096, 1024), (1300, 10240, 1152),
           (2200, 6144, 1024), (700, 28672, 1024), (4096, 2048, 2048)]
 
 
@@ -54,7 +54,7 @@ def test_glu(M, N, K, epilogue, bias):
     assert ((out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-3).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 512, 4096), (1093, 4096, 1024), (2200, 2560, 1024)])
+@pytest.mark.parametrize("M,N,K", [(300, 2048, 4096), (1093, 4096, 1024), (2200, 6144, 1024)])
 def test_a_launch_that_gave_up_leaves_nothing_for_the_next(M, N, K):
     """Owners that look at a flag once write NaN over their tile; the launches behind take only their own partial tiles."""
     s = torch.cuda.current_stream().cuda_stream
