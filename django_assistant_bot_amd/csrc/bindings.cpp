@@ -654,10 +654,13 @@ PYBIND11_MODULE(_native, m) {
           "layernorm_slabs");
   });
   m.def("gemm_small", [](u A, long lda, u B, long ldb, u C, long ldc, u bias, u residual, long ldr, int M, int N, int K,
-                         int gelu, int tile, u s) {
-    check(dab::gemm_small(CVP(A), lda, CVP(B), ldb, VP(C), ldc, CVP(bias), CVP(residual), ldr, M, N, K, gelu, tile, ST(s)),
+                         int gelu, int tile, u s, u next, unsigned next_bytes) {
+    check(dab::gemm_small(CVP(A), lda, CVP(B), ldb, VP(C), ldc, CVP(bias), CVP(residual), ldr, M, N, K, gelu, tile, ST(s),
+                          {CVP(next), next_bytes}),
           "gemm_small");
-  });
+  }, py::arg("A"), py::arg("lda"), py::arg("B"), py::arg("ldb"), py::arg("C"), py::arg("ldc"), py::arg("bias"), py::arg("residual"),
+     py::arg("ldr"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("tile"), py::arg("s"),
+     py::arg("next") = 0, py::arg("next_bytes") = 0);
   m.def("norm_stream_ok", [](int M, int N, int K, int SO, int bn) { return dab::norm_stream_ok(M, N, K, SO, bn) != 0; });
   m.def("norm_stream", [](u slabs, int S, int slabs_f32, u residual, u gain, u residual_out, float eps, u W, u out, long ldo,
                           int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn, u s) {
@@ -683,13 +686,21 @@ PYBIND11_MODULE(_native, m) {
                         (float*)out_vals, (int64_t*)out_ids, (int64_t*)out_docs, ST(s)),
           "top_hits");
   });
-  m.def("gemm_attn", [](u qkv, u cu, int batch, int D, float scale, u w, u b, u residual, u y, int T, int H, u s) {
-    check(dab::gemm_attn(CVP(qkv), (const int*)cu, batch, D, scale, CVP(w), CVP(b), CVP(residual), VP(y), T, H, ST(s)), "gemm_attn");
-  });
-  m.def("gemm_ln", [](u x, u gain, u offset, float eps, u normed, u w, u b, u C, int M, int N, int K, int gelu, int tile, u s) {
-    check(dab::gemm_ln(CVP(x), CVP(gain), CVP(offset), eps, VP(normed), CVP(w), CVP(b), VP(C), M, N, K, gelu, tile, ST(s)),
+  m.def("gemm_attn", [](u qkv, u cu, int batch, int D, float scale, u w, u b, u residual, u y, int T, int H, u s, u next,
+                        unsigned next_bytes) {
+    check(dab::gemm_attn(CVP(qkv), (const int*)cu, batch, D, scale, CVP(w), CVP(b), CVP(residual), VP(y), T, H, ST(s),
+                         {CVP(next), next_bytes}),
+          "gemm_attn");
+  }, py::arg("qkv"), py::arg("cu"), py::arg("batch"), py::arg("D"), py::arg("scale"), py::arg("w"), py::arg("b"),
+     py::arg("residual"), py::arg("y"), py::arg("T"), py::arg("H"), py::arg("s"), py::arg("next") = 0, py::arg("next_bytes") = 0);
+  m.def("gemm_ln", [](u x, u gain, u offset, float eps, u normed, u w, u b, u C, int M, int N, int K, int gelu, int tile, u s,
+                      u next, unsigned next_bytes) {
+    check(dab::gemm_ln(CVP(x), CVP(gain), CVP(offset), eps, VP(normed), CVP(w), CVP(b), VP(C), M, N, K, gelu, tile, ST(s),
+                       {CVP(next), next_bytes}),
           "gemm_ln");
-  });
+  }, py::arg("x"), py::arg("gain"), py::arg("offset"), py::arg("eps"), py::arg("normed"), py::arg("w"), py::arg("b"), py::arg("C"),
+     py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("tile"), py::arg("s"), py::arg("next") = 0,
+     py::arg("next_bytes") = 0);
   m.def("unit_rows", [](u x, long ldx, u out, int rows, int cols, u s) {
     check(dab::unit_rows((const float*)x, ldx, VP(out), rows, cols, ST(s)), "unit_rows");
   });

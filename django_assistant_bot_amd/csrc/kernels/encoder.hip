@@ -43,12 +43,12 @@ int small_tile(int M, int N, int K) {
 
 // y[M, N] = x[M, K] w[N, K]^T + b (GELU) (+ residual), everything contiguous: ops.gemm_bt's choice of kernel.
 static int projection(const bf16* x, const void* w, const void* b, const bf16* residual, bf16* y, int M, int N, int K, int gelu,
-                      hipStream_t s) {
+                      hipStream_t s, Upcoming next = {}) {
   int tile = small_tile(M, N, K);
   if (tile < 0 && ring_wins(M, N, K, gelu, residual != nullptr)) tile = 3;
   if (tile >= 0 && gemm_small_ok(M, N, K, K, K, N, N) &&
       !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8))
-    return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s);
+    return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s, next);
   if (gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K))
     return gemm256(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, s, 0, 1);
   return gemm_bt(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, 0, nullptr, nullptr, nullptr, 0, s, 0, 1);
@@ -71,35 +71,38 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
   const float scale = 1.f / sqrtf((float)D);
   // x = LayerNorm(y), then out = x w^T + b: one launch where the projection takes a split-K tile (one or two row tiles, so
   // that a row is normalised by as many workgroups as read it anyway), two where its rows outgrow that
-  auto norm_projection = [&](const uintptr_t* ln, const void* w, const void* b, bf16* out, int N, int gelu) {
+  auto norm_projection = [&](const uintptr_t* ln, const void* w, const void* b, bf16* out, int N, int gelu, Upcoming next) {
     const int tile = small_tile(T, N, H);
     if (gemm_ln_ok(T, N, H, tile) && !(((uintptr_t)w) % 16 || (ln[0] | ln[1] | (uintptr_t)b) % 8))
-      return gemm_ln(y, (const void*)ln[0], (const void*)ln[1], eps, x, w, b, out, T, N, H, gelu, tile, s);
+      return gemm_ln(y, (const void*)ln[0], (const void*)ln[1], eps, x, w, b, out, T, N, H, gelu, tile, s, next);
     const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s);
-    return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s);
+    return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s, next);
   };
   const int slices = slabs ? slab_slices(T, H, F) : 0;
   const uintptr_t* ln = nullptr;  // the layer's own norm of y, applied in front of the next projection
   for (int l = 0; l < n_layers && !rc; ++l) {
     const uintptr_t* w = layers + 12 * l;
     auto W = [&](int i) { return (const void*)w[i]; };
-    rc = ln ? norm_projection(ln, W(0), W(1), qkv, 3 * H, 0) : projection(x, W(0), W(1), nullptr, qkv, T, 3 * H, H, 0, s);
+    auto ahead = [&](const void* m, long n, long k) { return Upcoming{m, (unsigned)(n * k * 2)}; };
+    const Upcoming o = ahead(W(2), H, H), up = ahead(W(6), F, H), down = ahead(W(8), H, F);
+    const Upcoming qkv_next = l + 1 < n_layers ? ahead((const void*)w[12], 3 * H, H) : Upcoming{};
+    rc = ln ? norm_projection(ln, W(0), W(1), qkv, 3 * H, 0, o) : projection(x, W(0), W(1), nullptr, qkv, T, 3 * H, H, 0, s, o);
     // (33-64 tokens of 768, weights of several copies in turn, us a call apart -> inside: one text of 40 370 -> 360, of 56 379 -> 370,
     // four of 15 379 -> 377, eight of 8 381 -> 383, twenty of 3 378 -> 384: up to four texts)
     const bool attn_o = gemm_attn_ok(T, H, D, batch) && (T <= 32 || H <= 384 || batch <= 4) && !(w[2] % 16 || w[3] % 8);
-    if (!rc && attn_o) rc = gemm_attn(qkv, cu, batch, D, scale, W(2), W(3), x, y, T, H, s);
+    if (!rc && attn_o) rc = gemm_attn(qkv, cu, batch, D, scale, W(2), W(3), x, y, T, H, s, up);
     if (!rc && !attn_o)
       rc = flash_attention(qkv, 3 * H, D, qkv + H, qkv + 2 * H, 3 * H, D, nullptr, nullptr, nullptr, 0, 0, att, H, D, cu, cu,
                            nullptr, batch, max_len, heads, heads, D, 0, 0, scale, s);
-    if (!rc && !attn_o) rc = projection(att, W(2), W(3), x, y, T, H, H, 0, s);
-    if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1);
+    if (!rc && !attn_o) rc = projection(att, W(2), W(3), x, y, T, H, H, 0, s, up);
+    if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1, down);
     if (slices && !(w[8] % 16 || (w[9] | w[10] | w[11]) % 4)) {
       if (!rc) rc = gemm_slab(ffn, W(8), slabs, T, H, F, s);
       if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s);
       ln = nullptr;
       continue;
     }
-    if (!rc) rc = projection(ffn, W(8), W(9), x, y, T, H, F, 0, s);
+    if (!rc) rc = projection(ffn, W(8), W(9), x, y, T, H, F, 0, s, qkv_next);
     ln = w + 10;
   }
   if (!rc && ln) rc = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s);

@@ -39,8 +39,10 @@ struct SmallParams {
   const bf16* residual;
   int M, N, K;
   int lda, ldb, ldc, ldr;
+  int work;  // AHEAD: workgroups with a tile; those behind them read the next launch's weights
   float* slabs;  // SLAB: the slices' fp32 sums [slices][M][N] instead of C
   int slices;
+  Upcoming next;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const bf16* base, int rows, int ld, int K) {
@@ -108,9 +110,33 @@ __device__ __forceinline__ void small_finish(const SmallParams& p, const SmallTa
 }
 
 // neighbouring ids on one XCD: the row tiles of a column block read its weights from one L2
-__device__ __forceinline__ int small_id() {
-  const int nwg = gridDim.x, xcd = blockIdx.x % 8, q8 = nwg / 8, r8 = nwg % 8;
+__device__ __forceinline__ int small_id(int nwg) {
+  const int xcd = blockIdx.x % 8, q8 = nwg / 8, r8 = nwg % 8;
   return (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + blockIdx.x / 8;
+}
+
+// Reads ahead the weights of the launch behind this one, by the workgroups behind those with a tile.  A workgroup's XCD is its
+// id % 8 in every launch and an L2 keeps what the launch in front read, so XCD x reads the eighth of the rows whose column
+// blocks small_id gives it: the next launch begins with weights from L2 instead of memory.  (All of them there, the forward
+// of one question would take 249 us instead of 283.)
+__device__ __forceinline__ void read_next(const SmallParams& p) {
+  const int x = blockIdx.x & 7, before = (p.work + 7 - x) >> 3, mine = ((int)gridDim.x + 7 - x) / 8 - before;
+  const unsigned part = p.next.bytes / 8, step = (unsigned)mine * 8192u;  // part: a multiple of 16
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.next.w), (short)0, (int)p.next.bytes, 0x00020000);
+  const unsigned own = (unsigned)((((int)(blockIdx.x >> 3) - before) * 512 + (int)threadIdx.x) * 16);
+  for (unsigned at = own; at < part; at += 8 * step) {
+    u32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_raw_buffer_load_b128(r, min(at + j * step, part - 16), x * part, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" ::"v"(v[j]));
+  }
+}
+
+// The arguments in one round of scalar loads, ahead of the branch on `work` (a second round behind it: 0.15 us a launch)
+__device__ __forceinline__ void small_args(const SmallParams& p) {
+  asm volatile("" ::"s"(p.A), "s"(p.B), "s"(p.C), "s"(p.bias), "s"(p.residual), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.lda), "s"(p.ldb),
+               "s"(p.ldc), "s"(p.ldr), "s"(p.work));
 }
 
 typedef __attribute__((address_space(3))) void small_lds;
@@ -121,8 +147,10 @@ __device__ __forceinline__ void small_wait() {
 }
 
 // K-pieces of 64 go round the W waves: piece w + W j is wave w's, through a ring of D pieces of its own in LDS.
-template <int MT, int NT, int W, int D, bool GELU>
+template <int MT, int NT, int W, int D, bool GELU, bool AHEAD = false>
 __global__ __launch_bounds__(64 * W) void gemm_small_kernel(SmallParams p) {
+  if (AHEAD) small_args(p);
+  if (AHEAD && __builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
   constexpr int BM = 16 * MT, BN = 16 * NT, LDN = BN + 4;  // LDN: fp32 row of a partial tile, off the bank period
   constexpr int kA = BM * 128, kPiece = kA + BN * 128, kDma = 2 * MT + 2 * NT;
   constexpr int kRing = W * D * kPiece, kPart = W * BM * LDN * 4;
@@ -133,7 +161,7 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(SmallParams p) {
   float(*part)[BM * LDN] = reinterpret_cast<float(*)[BM * LDN]>(smem + (kOver ? 0 : kRing));
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tiles_m = (p.M + BM - 1) / BM, id = small_id();
+  const int tiles_m = (p.M + BM - 1) / BM, id = small_id(AHEAD ? p.work : (int)gridDim.x);
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
   const SmallTail<E> tail = small_tail<BM, BN, 64 * W, E>(p, m0, n0);
 
@@ -225,12 +253,15 @@ struct SmallNorm {
 
 template <int MT, int S, bool GELU>
 __global__ __launch_bounds__(512) void gemm_ln_kernel(SmallParams p, SmallNorm nm) {
+  small_args(p);
+  asm volatile("" ::"s"(nm.gain), "s"(nm.offset), "s"(nm.normed), "s"(nm.eps));
+  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
   constexpr int BM = 16 * MT, BN = 16, LDN = BN + 4, W = 8, K = 256 * S, LDA = 2 * K + 16;  // bytes of an LDS row
   __shared__ __attribute__((aligned(16))) float part[W][BM * LDN];
   __shared__ __attribute__((aligned(16))) char rows[BM * LDA];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tiles_m = (p.M + BM - 1) / BM, id = small_id();
+  const int tiles_m = (p.M + BM - 1) / BM, id = small_id(p.work);
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
 
   u32x2 xv[2 * MT][S], gv[S], ov[S];
@@ -337,6 +368,9 @@ struct SmallAttention {
 
 template <int D, int KB>
 __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAttention at) {
+  small_args(p);
+  asm volatile("" ::"s"(at.qkv), "s"(at.cu), "s"(at.batch), "s"(at.scale_log2));
+  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
   constexpr int W = 8, LDN = 20, KT = 2 * KB, ND = D / 32, HP = 64 / D;  // HP: heads of a 64-wide piece
   // a wave's rows of 128 B: 16 of Q, 16 of the weights, 32 KB of K and, once the scores are there, of V
   constexpr int kW = 2048, kKV = 4096, kWave = kKV + KB * 4096;
@@ -345,7 +379,7 @@ __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAtte
   __shared__ __attribute__((aligned(16))) char rows[W * kWave];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tiles_m = (p.M + 15) / 16, id = small_id();
+  const int tiles_m = (p.M + 15) / 16, id = small_id(p.work);
   const int m0 = (id % tiles_m) * 16, n0 = (id / tiles_m) * 16;
   const SmallTail<1> tail = small_tail<16, 16, 64 * W, 1>(p, m0, n0);
   const int H = p.K, last = p.M - 1, ld = 3 * H;
@@ -488,7 +522,7 @@ __global__ __launch_bounds__(64 * WM * WN, ring_occupancy(BM + BN, WM * WN, NS))
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w / WN, wn = w % WN;
   // SLAB: the tiles of a K-slice have neighbouring ids, so an XCD reads one or two slices of A and a few columns' weights
-  const int tiles_m = (p.M + BM - 1) / BM, tiles = SLAB ? tiles_m * ((p.N + BN - 1) / BN) : 1, id0 = small_id();
+  const int tiles_m = (p.M + BM - 1) / BM, tiles = SLAB ? tiles_m * ((p.N + BN - 1) / BN) : 1, id0 = small_id(gridDim.x);
   const int slice = SLAB ? id0 / tiles : 0, id = id0 - slice * tiles;
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
 
@@ -673,8 +707,18 @@ int gemm_small_ok(long M, long N, long K, long lda, long ldb, long ldc, long ldr
          ldc < (1L << 31) && ldr < (1L << 31);
 }
 
+// Workgroups behind `grid` of 512 that read the next launch's weights: as few as do it in 16 loads a thread, on CUs that have no
+// workgroup with a tile.  us a forward of 19 / 6 tokens of bge-base and 19 of bge-large, weights of three copies in turn: without
+// 284 / 259 / 626, 8 loads a thread 267 / 237 / 610, 16 265 / 237 / 600, 24 279 / 276 / 596; up to 320 workgroups 278 / 251 /
+// 664; as 2 to 8 loads a thread of the workgroups with a tile, waited for at their end, 295 / 274 / 650.  40 tokens 360 -> 348.
+static int next_blocks(const Upcoming& next, int grid) {
+  if (!next.w || next.bytes < 128 || next.bytes % 128 || (uintptr_t)next.w % 16) return 0;
+  const int room = (256 - grid) & ~7, want = (int)(((long)next.bytes / 8 + 16 * 8192 - 1) / (16 * 8192) * 8);
+  return room < 8 ? 0 : min(want, room);
+}
+
 int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, const void* residual,
-               long ldr, int M, int N, int K, int gelu, int tile, hipStream_t s) {
+               long ldr, int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next) {
   if (M <= 0 || N <= 0) return 0;
   if (!gemm_small_ok(M, N, K, lda, ldb, ldc, residual ? ldr : 0)) return hipErrorInvalidValue;
   if (((uintptr_t)A | (uintptr_t)B) % 16 || ((uintptr_t)C | (uintptr_t)bias | (uintptr_t)residual) % 8) return hipErrorInvalidValue;
@@ -686,6 +730,15 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
     if (gelu) hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, true>), dim3(grid), dim3(64 * W_), 0, s, p); \
     else hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, false>), dim3(grid), dim3(64 * W_), 0, s, p);     \
     break;                                                                                                      \
+  }
+  if (tile == 0 && !gelu) {
+    SmallParams pn = p;
+    pn.work = ((M + 15) / 16) * ((N + 15) / 16);
+    pn.next = next;
+    if (const int more = next_blocks(next, pn.work)) {
+      hipLaunchKernelGGL((gemm_small_kernel<1, 1, 8, 2, false, true>), dim3(pn.work + more), dim3(512), 0, s, pn);
+      return hipGetLastError();
+    }
   }
   switch (tile) {
     SMALL(0, 1, 1, 8, 2)
@@ -731,7 +784,7 @@ int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hi
   const int slices = slab_slices(M, N, K);
   if (!slices || !gemm_small_ok(M, N, K, K, K, N, 0)) return hipErrorInvalidValue;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)slabs) % 16) return hipErrorInvalidValue;
-  const SmallParams p = {(const bf16*)A, (const bf16*)B, nullptr, nullptr, nullptr, M, N, K, K, K, N, 0, (float*)slabs, slices};
+  const SmallParams p = {(const bf16*)A, (const bf16*)B, nullptr, nullptr, nullptr, M, N, K, K, K, N, 0, 0, (float*)slabs, slices};
   gemm_ring(p, 0, s);
   return hipGetLastError();
 }
@@ -743,13 +796,15 @@ int gemm_ln_ok(int M, int N, int K, int tile) {
 }
 
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
-            int M, int N, int K, int gelu, int tile, hipStream_t s) {
+            int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next) {
   if (!gemm_ln_ok(M, N, K, tile) || normed == x) return hipErrorInvalidValue;
   if (((uintptr_t)w) % 16 || ((uintptr_t)x | (uintptr_t)gain | (uintptr_t)offset | (uintptr_t)normed | (uintptr_t)C | (uintptr_t)b) % 8)
     return hipErrorInvalidValue;
-  const SmallParams p = {(const bf16*)x, (const bf16*)w, (bf16*)C, (const bf16*)b, nullptr, M, N, K, K, K, N, N};
+  SmallParams p = {(const bf16*)x, (const bf16*)w, (bf16*)C, (const bf16*)b, nullptr, M, N, K, K, K, N, N};
   const SmallNorm nm = {(const bf16*)gain, (const bf16*)offset, (bf16*)normed, eps};
-  const int mt = tile + 1, grid = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 15) / 16);
+  const int mt = tile + 1, work = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 15) / 16), grid = work + next_blocks(next, work);
+  p.work = work;
+  p.next = next;
 #define LN_GEMM(MT_, S_)                                                                                               \
   if (mt == MT_ && K == 256 * S_) {                                                                                    \
     if (gelu) hipLaunchKernelGGL((gemm_ln_kernel<MT_, S_, true>), dim3(grid), dim3(512), 0, s, p, nm);                  \
@@ -772,13 +827,15 @@ int gemm_attn_ok(int T, int H, int D, int batch) {
 }
 
 int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
-              void* y, int T, int H, hipStream_t s) {
+              void* y, int T, int H, hipStream_t s, Upcoming next) {
   if (!gemm_attn_ok(T, H, D, batch)) return hipErrorInvalidValue;
   if (((uintptr_t)qkv | (uintptr_t)w) % 16 || ((uintptr_t)b | (uintptr_t)residual | (uintptr_t)y) % 8 || (uintptr_t)cu % 4)
     return hipErrorInvalidValue;
-  const SmallParams p = {nullptr, (const bf16*)w, (bf16*)y, (const bf16*)b, (const bf16*)residual, T, H, H, H, H, H, H};
+  SmallParams p = {nullptr, (const bf16*)w, (bf16*)y, (const bf16*)b, (const bf16*)residual, T, H, H, H, H, H, H};
+  p.work = ((T + 15) / 16) * (H / 16);
+  p.next = next;
   const SmallAttention at = {(const bf16*)qkv, cu, batch, scale * 1.44269504088896340736f};
-  const dim3 grid(((T + 15) / 16) * (H / 16));
+  const dim3 grid(p.work + next_blocks(next, p.work));
   if (D == 64 && T <= 32) hipLaunchKernelGGL((gemm_attn_kernel<64, 1>), grid, dim3(512), 0, s, p, at);
   else if (D == 64) hipLaunchKernelGGL((gemm_attn_kernel<64, 2>), grid, dim3(512), 0, s, p, at);
   else if (T <= 32) hipLaunchKernelGGL((gemm_attn_kernel<32, 1>), grid, dim3(512), 0, s, p, at);

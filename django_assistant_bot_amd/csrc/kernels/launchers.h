@@ -387,17 +387,22 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
 // gemm_small.hip
 int gemm_small_ok(long M, long N, long K, long lda, long ldb, long ldc, long ldr);
 int gemm_attn_ok(int T, int H, int D, int batch);
+// Row-major weights of the launch behind, read ahead by the small kernels (ReadNext in gemm_small.hip)
+struct Upcoming {
+  const void* w;  // null: none
+  unsigned bytes;
+};
 int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
-              void* y, int T, int H, hipStream_t s);
+              void* y, int T, int H, hipStream_t s, Upcoming next = {});
 int gemm_ln_ok(int M, int N, int K, int tile);
 int slab_slices(int M, int N, int K);
 int ring_tile(int M, int N, int K, int gelu, int slices);
 bool ring_wins(int M, int N, int K, int gelu, int residual);
 int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
-            int M, int N, int K, int gelu, int tile, hipStream_t s);
+            int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next = {});
 int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, const void* residual,
-               long ldr, int M, int N, int K, int gelu, int tile, hipStream_t s);
+               long ldr, int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next = {});
 
 // search.hip
 constexpr int kRankMax = 64;  // largest rank rank_value finds
