@@ -75,7 +75,7 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     const int tile = small_tile(T, N, H);
     if (gemm_ln_ok(T, N, H, tile) && !(((uintptr_t)w) % 16 || (ln[0] | ln[1] | (uintptr_t)b) % 8))
       return gemm_ln(y, (const void*)ln[0], (const void*)ln[1], eps, x, w, b, out, T, N, H, gelu, tile, s, next);
-    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s);
+    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s, {w, (unsigned)((long)N * H * 2)});
     return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s, next);
   };
   const int slices = slabs ? slab_slices(T, H, F) : 0;
@@ -98,7 +98,7 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1, down);
     if (slices && !(w[8] % 16 || (w[9] | w[10] | w[11]) % 4)) {
       if (!rc) rc = gemm_slab(ffn, W(8), slabs, T, H, F, s);
-      if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s);
+      if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s, qkv_next);
       ln = nullptr;
       continue;
     }

@@ -115,24 +115,6 @@ __device__ __forceinline__ int small_id(int nwg) {
   return (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + blockIdx.x / 8;
 }
 
-// Reads ahead the weights of the launch behind this one, by the workgroups behind those with a tile.  A workgroup's XCD is its
-// id % 8 in every launch and an L2 keeps what the launch in front read, so XCD x reads the eighth of the rows whose column
-// blocks small_id gives it: the next launch begins with weights from L2 instead of memory.  (All of them there, the forward
-// of one question would take 249 us instead of 283.)
-__device__ __forceinline__ void read_next(const SmallParams& p) {
-  const int x = blockIdx.x & 7, before = (p.work + 7 - x) >> 3, mine = ((int)gridDim.x + 7 - x) / 8 - before;
-  const unsigned part = p.next.bytes / 8, step = (unsigned)mine * 8192u;  // part: a multiple of 16
-  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.next.w), (short)0, (int)p.next.bytes, 0x00020000);
-  const unsigned own = (unsigned)((((int)(blockIdx.x >> 3) - before) * 512 + (int)threadIdx.x) * 16);
-  for (unsigned at = own; at < part; at += 8 * step) {
-    u32x4 v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_raw_buffer_load_b128(r, min(at + j * step, part - 16), x * part, 0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) asm volatile("" ::"v"(v[j]));
-  }
-}
-
 // The arguments in one round of scalar loads, ahead of the branch on `work` (a second round behind it: 0.15 us a launch)
 __device__ __forceinline__ void small_args(const SmallParams& p) {
   asm volatile("" ::"s"(p.A), "s"(p.B), "s"(p.C), "s"(p.bias), "s"(p.residual), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.lda), "s"(p.ldb),
@@ -150,7 +132,7 @@ __device__ __forceinline__ void small_wait() {
 template <int MT, int NT, int W, int D, bool GELU, bool AHEAD = false>
 __global__ __launch_bounds__(64 * W) void gemm_small_kernel(SmallParams p) {
   if (AHEAD) small_args(p);
-  if (AHEAD && __builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
+  if (AHEAD && __builtin_expect((int)blockIdx.x >= p.work, 0)) return read_upcoming<512>(p.next, p.work);
   constexpr int BM = 16 * MT, BN = 16 * NT, LDN = BN + 4;  // LDN: fp32 row of a partial tile, off the bank period
   constexpr int kA = BM * 128, kPiece = kA + BN * 128, kDma = 2 * MT + 2 * NT;
   constexpr int kRing = W * D * kPiece, kPart = W * BM * LDN * 4;
@@ -255,7 +237,7 @@ template <int MT, int S, bool GELU>
 __global__ __launch_bounds__(512) void gemm_ln_kernel(SmallParams p, SmallNorm nm) {
   small_args(p);
   asm volatile("" ::"s"(nm.gain), "s"(nm.offset), "s"(nm.normed), "s"(nm.eps));
-  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
+  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_upcoming<512>(p.next, p.work);
   constexpr int BM = 16 * MT, BN = 16, LDN = BN + 4, W = 8, K = 256 * S, LDA = 2 * K + 16;  // bytes of an LDS row
   __shared__ __attribute__((aligned(16))) float part[W][BM * LDN];
   __shared__ __attribute__((aligned(16))) char rows[BM * LDA];
@@ -370,7 +352,7 @@ template <int D, int KB>
 __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAttention at) {
   small_args(p);
   asm volatile("" ::"s"(at.qkv), "s"(at.cu), "s"(at.batch), "s"(at.scale_log2));
-  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_next(p);
+  if (__builtin_expect((int)blockIdx.x >= p.work, 0)) return read_upcoming<512>(p.next, p.work);
   constexpr int W = 8, LDN = 20, KT = 2 * KB, ND = D / 32, HP = 64 / D;  // HP: heads of a 64-wide piece
   // a wave's rows of 128 B: 16 of Q, 16 of the weights, 32 KB of K and, once the scores are there, of V
   constexpr int kW = 2048, kKV = 4096, kWave = kKV + KB * 4096;

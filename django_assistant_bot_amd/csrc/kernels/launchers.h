@@ -41,10 +41,15 @@ int rmsnorm(void* out, void* res_out, const void* x, const void* res_in, const v
             hipStream_t s);
 int rmsnorm_slabs(void* out, void* res_out, const void* slabs, int S, long slab_stride, const void* res_in,
                   const void* w, int rows, int cols, float eps, hipStream_t s, int slab_bf16 = 0);
+// Row-major weights of the launch behind, read ahead by workgroups behind those at work (common.h read_upcoming)
+struct Upcoming {
+  const void* w;  // null: none
+  unsigned bytes;
+};
 int layernorm_slabs(void* out, const void* slabs, int S, const void* bias, const void* res, const void* gamma,
-                    const void* beta, int rows, int cols, float eps, hipStream_t s);
+                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next = {});
 int layernorm(void* out, const void* x, const void* res_in, const void* gamma, const void* beta, int rows, int cols,
-              float eps, hipStream_t s);
+              float eps, hipStream_t s, Upcoming next = {});
 int bert_embed(void* out, const int* ids, const int* pos_ids, const int* type_ids, const void* word, const void* pos,
                const void* type, const void* gamma, const void* beta, int rows, int cols, float eps, hipStream_t s);
 int embed_gather(void* out, const int* ids, const void* table, int rows, int cols, hipStream_t s);
@@ -387,11 +392,6 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
 // gemm_small.hip
 int gemm_small_ok(long M, long N, long K, long lda, long ldb, long ldc, long ldr);
 int gemm_attn_ok(int T, int H, int D, int batch);
-// Row-major weights of the launch behind, read ahead by the small kernels (ReadNext in gemm_small.hip)
-struct Upcoming {
-  const void* w;  // null: none
-  unsigned bytes;
-};
 int gemm_attn(const void* qkv, const int* cu, int batch, int D, float scale, const void* w, const void* b, const void* residual,
               void* y, int T, int H, hipStream_t s, Upcoming next = {});
 int gemm_ln_ok(int M, int N, int K, int tile);

@@ -222,11 +222,16 @@ __global__ __launch_bounds__(NT) void layernorm_kernel(bf16* __restrict__ out, c
 // LN in the bge encoder (rocprof, profiles/embed_study.md): row-per-workgroup kernel 45.2 us, RPW 1
 // 41.0, RPW 2 34.1 (5.9 TB/s), RPW 4 34.0.  The row-per-workgroup kernel above left a quarter of its 128 lanes
 // idle at 768 columns and waited on two workgroup barriers per row.
-template <int CPL, int RPW>
+template <int CPL, int RPW, bool AHEAD>
 __global__ __launch_bounds__(256) void layernorm_rows_kernel(bf16* __restrict__ out, const bf16* __restrict__ x,
                                                             const bf16* __restrict__ res_in,
                                                             const bf16* __restrict__ gamma,
-                                                            const bf16* __restrict__ beta, int rows, float eps) {
+                                                            const bf16* __restrict__ beta, int rows, float eps, int work,
+                                                            Upcoming next) {
+  if constexpr (AHEAD) {
+    asm volatile("" ::"s"(out), "s"(x), "s"(res_in), "s"(gamma), "s"(beta), "s"(rows), "s"(eps), "s"(work));  // (one round of loads)
+    if (__builtin_expect((int)blockIdx.x >= work, 0)) return read_upcoming<256>(next, work);
+  }
   constexpr int cols = 256 * CPL;
   const int lane = threadIdx.x & 63;
   const size_t row0 = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
@@ -300,11 +305,15 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(bf16* __restrict__ 
 
 // LayerNorm(sum of S fp32 slabs [S][rows][cols] + bias + residual), rounded once; a row a wave, every load in front of the
 // sums (a launch and one round trip bound it; out may be the residual).  3.5-4 us at 832 rows of 768 in 3 slabs.
-template <int CP, int S>
+template <int CP, int S, bool AHEAD>
 __global__ __launch_bounds__(256) void layernorm_slab_kernel(bf16* out, const float* __restrict__ slabs,
                                                              const bf16* __restrict__ bias, const bf16* res,
                                                              const bf16* __restrict__ gamma, const bf16* __restrict__ beta,
-                                                             int rows, float eps) {
+                                                             int rows, float eps, int work, Upcoming next) {
+  if constexpr (AHEAD) {
+    asm volatile("" ::"s"(out), "s"(slabs), "s"(bias), "s"(res), "s"(gamma), "s"(beta), "s"(rows), "s"(eps), "s"(work));
+    if (__builtin_expect((int)blockIdx.x >= work, 0)) return read_upcoming<256>(next, work);
+  }
   constexpr int cols = 128 * CP;
   const int lane = threadIdx.x & 63;
   const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -576,39 +585,56 @@ int rmsnorm_slabs(void* out, void* res_out, const void* slabs, int S, long slab_
   return rmsnorm_slabs_t(out, res_out, (const float*)slabs, S, slab_stride, res_in, w, rows, cols, eps, s);
 }
 
+// Workgroups of 256 behind a LayerNorm's that read the next projection's weights, 8 loads a thread.  us a forward, weights of
+// three copies in turn, without -> with 16 / 8 / 4 loads: bge-base 120 tokens 430 -> 431 / 422 / 423, 240 502 -> 495 / 486 / 486, 816
+// 663 -> 640 / 632 / 634, 1500 854 -> 830 / 824 / 831, 3000 1,227 -> 1,208 / 1,207 / 1,212, 6000 2,008 -> 2,004 / 2,002 / 1,995;
+// bge-large 180 1,108 -> 1,066 / 1,050 / 1,054, 600 1,460 -> 1,421 / 1,432 / 1,434, 1200 2,002 -> 1,959 / 1,957 / 1,969, but 1800 2,245 ->
+// 2,277 / 2,253 / 2,261: more rows need the weights less, and larger ones take longer than the norm.
+static int norm_readers(const Upcoming& next, int rows) {
+  if (!next.w || next.bytes < 128 || next.bytes % 128 || (uintptr_t)next.w % 16 || (double)rows * next.bytes > 14e9) return 0;
+  return (int)(((long)next.bytes / 8 + 8 * 4096 - 1) / (8 * 4096) * 8);
+}
+
 int layernorm(void* out, const void* x, const void* res_in, const void* gamma, const void* beta, int rows, int cols,
-              float eps, hipStream_t s) {
+              float eps, hipStream_t s, Upcoming next) {
   if (rows <= 0) return 0;
   if (cols % 8 || cols > 16384) return hipErrorInvalidValue;
   // encoder widths: one wave per LN_RPW rows, 4 waves per workgroup
   constexpr int LN_RPW = 2;  // 4 measured the same (34.0 us)
-  const dim3 g4((rows + 4 * LN_RPW - 1) / (4 * LN_RPW));
-  if (cols == 768) {
-    hipLaunchKernelGGL((layernorm_rows_kernel<3, LN_RPW>), g4, dim3(256), 0, s, (bf16*)out, (const bf16*)x,
-                       (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps);
-    return hipGetLastError();
+  const int work = (rows + 4 * LN_RPW - 1) / (4 * LN_RPW), more = norm_readers(next, rows);
+#define LN_ROWS(CPL)                                                                                                 \
+  if (cols == 256 * CPL) {                                                                                           \
+    if (more)                                                                                                        \
+      hipLaunchKernelGGL((layernorm_rows_kernel<CPL, LN_RPW, true>), dim3(work + more), dim3(256), 0, s, (bf16*)out, \
+                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+    else                                                                                                             \
+      hipLaunchKernelGGL((layernorm_rows_kernel<CPL, LN_RPW, false>), dim3(work), dim3(256), 0, s, (bf16*)out,       \
+                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+    return hipGetLastError();                                                                                        \
   }
-  if (cols == 1024) {
-    hipLaunchKernelGGL((layernorm_rows_kernel<4, LN_RPW>), g4, dim3(256), 0, s, (bf16*)out, (const bf16*)x,
-                       (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps);
-    return hipGetLastError();
-  }
+  LN_ROWS(3)
+  LN_ROWS(4)
+#undef LN_ROWS
   DAB_ROW_DISPATCH(layernorm_kernel, rows, cols, s, (bf16*)out, (const bf16*)x, (const bf16*)res_in,
                    (const bf16*)gamma, (const bf16*)beta, cols, eps);
   return hipGetLastError();
 }
 
 int layernorm_slabs(void* out, const void* slabs_, int S, const void* bias, const void* res, const void* gamma,
-                    const void* beta, int rows, int cols, float eps, hipStream_t s) {
+                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next) {
   if (rows <= 0) return 0;
   const float* slabs = (const float*)slabs_;
   if ((uintptr_t)slabs % 8 || ((uintptr_t)out | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)gamma | (uintptr_t)beta) % 4)
     return hipErrorInvalidValue;
-  const dim3 grid((rows + 3) / 4);
+  const int work = (rows + 3) / 4, more = norm_readers(next, rows);
 #define LN_SLAB(CP, SS)                                                                                               \
   if (cols == 128 * CP && S == SS) {                                                                                  \
-    hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS>), grid, dim3(256), 0, s, (bf16*)out, slabs, (const bf16*)bias,  \
-                       (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps);                           \
+    if (more)                                                                                                         \
+      hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS, true>), dim3(work + more), dim3(256), 0, s, (bf16*)out, slabs, \
+                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+    else                                                                                                              \
+      hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS, false>), dim3(work), dim3(256), 0, s, (bf16*)out, slabs,       \
+                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
     return hipGetLastError();                                                                                         \
   }
 #define LN_SLABS(CP) LN_SLAB(CP, 2) LN_SLAB(CP, 3)

@@ -55,3 +55,20 @@ def test_attention_and_projection(H, D, lens):
     s = torch.cuda.current_stream().cuda_stream
     _each(lambda w, n: ops.native().gemm_attn(qkv.data_ptr(), cu.data_ptr(), len(lens), D, D ** -0.5, w0.data_ptr(), b.data_ptr(),
                                               r.data_ptr(), out.data_ptr(), T, H, s, next=w, next_bytes=n), out)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 768), (8, 1024), (120, 768), (817, 1024), (3000, 768), (33, 384)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_norm(rows, cols, residual):
+    x, r, g, o, out = _r(rows, cols), _r(rows, cols), _r(cols), _r(cols), torch.empty(rows, cols, dtype=torch.bfloat16, device=DEV)
+    s = torch.cuda.current_stream().cuda_stream
+    _each(lambda w, n: ops.native().layernorm(out.data_ptr(), x.data_ptr(), r.data_ptr() if residual else 0, g.data_ptr(), o.data_ptr(),
+                                              rows, cols, 1e-12, s, next=w, next_bytes=n), out)
+
+
+@pytest.mark.parametrize("rows,cols,S", [(1, 768, 2), (817, 768, 3), (600, 1024, 2), (2200, 384, 3)])
+def test_norm_of_slabs(rows, cols, S):
+    x, r, b, g, o = torch.randn(S, rows, cols, device=DEV), _r(rows, cols), _r(cols), _r(cols), _r(cols)
+    out, s = torch.empty(rows, cols, dtype=torch.bfloat16, device=DEV), torch.cuda.current_stream().cuda_stream
+    _each(lambda w, n: ops.native().layernorm_slabs(out.data_ptr(), x.data_ptr(), S, b.data_ptr(), r.data_ptr(), g.data_ptr(),
+                                                    o.data_ptr(), rows, cols, 1e-12, s, next=w, next_bytes=n), out)
