@@ -692,7 +692,8 @@ int gemm_small_ok(long M, long N, long K, long lda, long ldb, long ldc, long ldr
 // Workgroups behind `grid` of 512 that read the next launch's weights: as few as do it in 16 loads a thread, on CUs that have no
 // workgroup with a tile.  us a forward of 19 / 6 tokens of bge-base and 19 of bge-large, weights of three copies in turn: without
 // 284 / 259 / 626, 8 loads a thread 267 / 237 / 610, 16 265 / 237 / 600, 24 279 / 276 / 596; up to 320 workgroups 278 / 251 /
-// 664; as 2 to 8 loads a thread of the workgroups with a tile, waited for at their end, 295 / 274 / 650.  40 tokens 360 -> 348.
+// 664; as 2 to 8 loads a thread of the workgroups with a tile, waited for at their end, 295 / 274 / 650.  40 tokens 360 -> 347 with the
+// tiles of 16 x 16 alone, 329 with the other split-K tiles; 120 417 -> 402, 240 486 -> 479.
 static int next_blocks(const Upcoming& next, int grid) {
   if (!next.w || next.bytes < 128 || next.bytes % 128 || (uintptr_t)next.w % 16) return 0;
   const int room = (256 - grid) & ~7, want = (int)(((long)next.bytes / 8 + 16 * 8192 - 1) / (16 * 8192) * 8);
@@ -704,23 +705,22 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
   if (M <= 0 || N <= 0) return 0;
   if (!gemm_small_ok(M, N, K, lda, ldb, ldc, residual ? ldr : 0)) return hipErrorInvalidValue;
   if (((uintptr_t)A | (uintptr_t)B) % 16 || ((uintptr_t)C | (uintptr_t)bias | (uintptr_t)residual) % 8) return hipErrorInvalidValue;
-  const SmallParams p = {(const bf16*)A, (const bf16*)B, (bf16*)C, (const bf16*)bias, (const bf16*)residual, M, N, K,
+  SmallParams p = {(const bf16*)A, (const bf16*)B, (bf16*)C, (const bf16*)bias, (const bf16*)residual, M, N, K,
                          (int)lda, (int)ldb, (int)ldc, (int)ldr};
-#define SMALL(T, MT_, NT_, W_, D_)                                                                              \
-  case T: {                                                                                                     \
-    const int grid = ((M + 16 * MT_ - 1) / (16 * MT_)) * ((N + 16 * NT_ - 1) / (16 * NT_));                     \
-    if (gelu) hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, true>), dim3(grid), dim3(64 * W_), 0, s, p); \
-    else hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, false>), dim3(grid), dim3(64 * W_), 0, s, p);     \
-    break;                                                                                                      \
-  }
-  if (tile == 0 && !gelu) {
-    SmallParams pn = p;
-    pn.work = ((M + 15) / 16) * ((N + 15) / 16);
-    pn.next = next;
-    if (const int more = next_blocks(next, pn.work)) {
-      hipLaunchKernelGGL((gemm_small_kernel<1, 1, 8, 2, false, true>), dim3(pn.work + more), dim3(512), 0, s, pn);
-      return hipGetLastError();
-    }
+  p.next = next;
+#define SMALL_AS(MT_, NT_, W_, D_, A_)                                                                                  \
+  do {                                                                                                                \
+    if (gelu) hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, true, A_>), grid, dim3(64 * W_), 0, s, p);       \
+    else hipLaunchKernelGGL((gemm_small_kernel<MT_, NT_, W_, D_, false, A_>), grid, dim3(64 * W_), 0, s, p);           \
+  } while (0)
+#define SMALL(T, MT_, NT_, W_, D_)                                                                                    \
+  case T: {                                                                                                           \
+    p.work = ((M + 16 * MT_ - 1) / (16 * MT_)) * ((N + 16 * NT_ - 1) / (16 * NT_));                                   \
+    const int more = next_blocks(next, p.work);                                                                       \
+    const dim3 grid(p.work + more);                                                                                   \
+    if (more) SMALL_AS(MT_, NT_, W_, D_, true);                                                                       \
+    else SMALL_AS(MT_, NT_, W_, D_, false);                                                                           \
+    break;                                                                                                            \
   }
   switch (tile) {
     SMALL(0, 1, 1, 8, 2)
@@ -735,6 +735,7 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
     default: return hipErrorInvalidValue;
   }
 #undef SMALL
+#undef SMALL_AS
   return hipGetLastError();
 }
 

@@ -29,11 +29,13 @@ def _r(*shape):
 
 # grids that leave room for readers, that are no multiple of 8, and that leave none
 @pytest.mark.parametrize("M,N,K", [(1, 768, 3072), (16, 64, 768), (19, 768, 3072), (19, 1000, 768), (64, 1024, 4096), (33, 1024, 1024)])
-def test_split_tile(M, N, K):
+@pytest.mark.parametrize("tile", [0, 1, 6, 7, 8])
+@pytest.mark.parametrize("gelu", [0, 1])
+def test_split_tile(M, N, K, tile, gelu):
     A, B, b, r, out = _r(M, K), _r(N, K), _r(N), _r(M, N), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
     s = torch.cuda.current_stream().cuda_stream
-    _each(lambda w, n: ops.native().gemm_small(A.data_ptr(), K, B.data_ptr(), K, out.data_ptr(), N, b.data_ptr(), r.data_ptr(), N, M, N,
-                                               K, 0, 0, s, next=w, next_bytes=n), out)
+    _each(lambda w, n: ops.native().gemm_small(A.data_ptr(), K, B.data_ptr(), K, out.data_ptr(), N, b.data_ptr(),
+                                               0 if gelu else r.data_ptr(), N, M, N, K, gelu, tile, s, next=w, next_bytes=n), out)
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (19, 3072, 768), (32, 2304, 768), (40, 1024, 1024), (19, 4096, 1024)])
