@@ -123,11 +123,13 @@ PYBIND11_MODULE(_native, m) {
   m.def("rmsnorm", [](u out, u res_out, u x, u res_in, u w, int rows, int cols, float eps, u s) {
     check(dab::rmsnorm(VP(out), VP(res_out), CVP(x), CVP(res_in), CVP(w), rows, cols, eps, ST(s)), "rmsnorm");
   });
-  m.def("layernorm", [](u out, u x, u res_in, u gamma, u beta, int rows, int cols, float eps, u s, u next, unsigned next_bytes) {
-    check(dab::layernorm(VP(out), CVP(x), CVP(res_in), CVP(gamma), CVP(beta), rows, cols, eps, ST(s), {CVP(next), next_bytes}),
+  m.def("layernorm", [](u out, u x, u res_in, u gamma, u beta, int rows, int cols, float eps, u s, u next, unsigned next_bytes, u then, unsigned then_bytes) {
+    check(dab::layernorm(VP(out), CVP(x), CVP(res_in), CVP(gamma), CVP(beta), rows, cols, eps, ST(s), {CVP(next), next_bytes},
+                         {CVP(then), then_bytes}),
           "layernorm");
   }, py::arg("out"), py::arg("x"), py::arg("res_in"), py::arg("gamma"), py::arg("beta"), py::arg("rows"), py::arg("cols"),
-     py::arg("eps"), py::arg("s"), py::arg("next") = 0, py::arg("next_bytes") = 0);
+     py::arg("eps"), py::arg("s"), py::arg("next") = 0, py::arg("next_bytes") = 0,
+     py::arg("then") = 0, py::arg("then_bytes") = 0);
   m.def("bert_embed", [](u out, u ids, u pos_ids, u type_ids, u word, u pos, u type, u gamma, u beta, int rows, int cols,
                          float eps, u s) {
     check(dab::bert_embed(VP(out), (const int*)ids, (const int*)pos_ids, (const int*)type_ids, CVP(word), CVP(pos),
@@ -652,12 +654,14 @@ PYBIND11_MODULE(_native, m) {
     check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s)), "gemm_slab");
   });
   m.def("layernorm_slabs", [](u out, u slabs, int S, u bias, u res, u gamma, u beta, int rows, int cols, float eps, u s,
-                              u next, unsigned next_bytes) {
+                              u next, unsigned next_bytes, u then, unsigned then_bytes) {
     check(dab::layernorm_slabs(VP(out), CVP(slabs), S, CVP(bias), CVP(res), CVP(gamma), CVP(beta), rows, cols, eps, ST(s),
-                               {CVP(next), next_bytes}),
+                               {CVP(next), next_bytes},
+                         {CVP(then), then_bytes}),
           "layernorm_slabs");
   }, py::arg("out"), py::arg("slabs"), py::arg("S"), py::arg("bias"), py::arg("res"), py::arg("gamma"), py::arg("beta"), py::arg("rows"),
-     py::arg("cols"), py::arg("eps"), py::arg("s"), py::arg("next") = 0, py::arg("next_bytes") = 0);
+     py::arg("cols"), py::arg("eps"), py::arg("s"), py::arg("next") = 0, py::arg("next_bytes") = 0,
+     py::arg("then") = 0, py::arg("then_bytes") = 0);
   m.def("gemm_small", [](u A, long lda, u B, long ldb, u C, long ldc, u bias, u residual, long ldr, int M, int N, int K,
                          int gelu, int tile, u s, u next, unsigned next_bytes) {
     check(dab::gemm_small(CVP(A), lda, CVP(B), ldb, VP(C), ldc, CVP(bias), CVP(residual), ldr, M, N, K, gelu, tile, ST(s),

@@ -69,13 +69,18 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
   bf16 *x = (bf16*)x_, *y = (bf16*)y_, *att = (bf16*)att_, *qkv = (bf16*)qkv_, *ffn = (bf16*)ffn_;
   int rc = bert_embed(x, ids, pos, nullptr, word, pos_table, type, gain, offset, T, H, eps, s);
   const float scale = 1.f / sqrtf((float)D);
+  // The weights that launches read ahead: each the next launch's, a LayerNorm also those of the projection behind the next,
+  // where that one's tiles leave no room for readers.  us a forward, weights of three copies in turn, without the latter -> with:
+  // bge-base 240 tokens 481 -> 468, 816 632 -> 609, 1500 820 -> 798, 3000 1,209 -> 1,210; bge-large 180 1,040 -> 981, 600 1,428 ->
+  // 1,369, 1200 1,937 -> 1,837, 1800 2,239 -> 2,222; where the next launch has readers too 120 405 -> 414.
+  auto reads_next = [](int tile) { return tile >= 0 && !(tile >= 2 && tile <= 5); };
   // x = LayerNorm(y), then out = x w^T + b: one launch where the projection takes a split-K tile (one or two row tiles, so
   // that a row is normalised by as many workgroups as read it anyway), two where its rows outgrow that
   auto norm_projection = [&](const uintptr_t* ln, const void* w, const void* b, bf16* out, int N, int gelu, Upcoming next) {
     const int tile = small_tile(T, N, H);
     if (gemm_ln_ok(T, N, H, tile) && !(((uintptr_t)w) % 16 || (ln[0] | ln[1] | (uintptr_t)b) % 8))
       return gemm_ln(y, (const void*)ln[0], (const void*)ln[1], eps, x, w, b, out, T, N, H, gelu, tile, s, next);
-    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s, {w, (unsigned)((long)N * H * 2)});
+    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s, {w, (unsigned)((long)N * H * 2)}, reads_next(tile) ? Upcoming{} : next);
     return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s, next);
   };
   const int slices = slabs ? slab_slices(T, H, F) : 0;
@@ -86,6 +91,7 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     auto ahead = [&](const void* m, long n, long k) { return Upcoming{m, (unsigned)(n * k * 2)}; };
     const Upcoming o = ahead(W(2), H, H), up = ahead(W(6), F, H), down = ahead(W(8), H, F);
     const Upcoming qkv_next = l + 1 < n_layers ? ahead((const void*)w[12], 3 * H, H) : Upcoming{};
+    const Upcoming o_next = l + 1 < n_layers && !reads_next(small_tile(T, 3 * H, H)) ? ahead((const void*)w[14], H, H) : Upcoming{};
     rc = ln ? norm_projection(ln, W(0), W(1), qkv, 3 * H, 0, o) : projection(x, W(0), W(1), nullptr, qkv, T, 3 * H, H, 0, s, o);
     // (33-64 tokens of 768, weights of several copies in turn, us a call apart -> inside: one text of 40 370 -> 360, of 56 379 -> 370,
     // four of 15 379 -> 377, eight of 8 381 -> 383, twenty of 3 378 -> 384: up to four texts)
@@ -98,7 +104,7 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
     if (!rc) rc = norm_projection(w + 4, W(6), W(7), ffn, F, 1, down);
     if (slices && !(w[8] % 16 || (w[9] | w[10] | w[11]) % 4)) {
       if (!rc) rc = gemm_slab(ffn, W(8), slabs, T, H, F, s);
-      if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s, qkv_next);
+      if (!rc) rc = layernorm_slabs(x, slabs, slices, W(9), x, W(10), W(11), T, H, eps, s, qkv_next, o_next);
       ln = nullptr;
       continue;
     }

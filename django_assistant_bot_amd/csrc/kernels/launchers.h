@@ -47,9 +47,9 @@ struct Upcoming {
   unsigned bytes;
 };
 int layernorm_slabs(void* out, const void* slabs, int S, const void* bias, const void* res, const void* gamma,
-                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next = {});
+                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next = {}, Upcoming then = {});
 int layernorm(void* out, const void* x, const void* res_in, const void* gamma, const void* beta, int rows, int cols,
-              float eps, hipStream_t s, Upcoming next = {});
+              float eps, hipStream_t s, Upcoming next = {}, Upcoming then = {});
 int bert_embed(void* out, const int* ids, const int* pos_ids, const int* type_ids, const void* word, const void* pos,
                const void* type, const void* gamma, const void* beta, int rows, int cols, float eps, hipStream_t s);
 int embed_gather(void* out, const int* ids, const void* table, int rows, int cols, hipStream_t s);

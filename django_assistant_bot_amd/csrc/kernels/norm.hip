@@ -227,10 +227,14 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(bf16* __restrict__ 
                                                             const bf16* __restrict__ res_in,
                                                             const bf16* __restrict__ gamma,
                                                             const bf16* __restrict__ beta, int rows, float eps, int work,
-                                                            Upcoming next) {
+                                                            Upcoming next, Upcoming then) {
   if constexpr (AHEAD) {
     asm volatile("" ::"s"(out), "s"(x), "s"(res_in), "s"(gamma), "s"(beta), "s"(rows), "s"(eps), "s"(work));  // (one round of loads)
-    if (__builtin_expect((int)blockIdx.x >= work, 0)) return read_upcoming<256>(next, work);
+    if (__builtin_expect((int)blockIdx.x >= work, 0)) {
+      read_upcoming<256>(next, work);
+      if (then.bytes) read_upcoming<256>(then, work);
+      return;
+    }
   }
   constexpr int cols = 256 * CPL;
   const int lane = threadIdx.x & 63;
@@ -309,10 +313,14 @@ template <int CP, int S, bool AHEAD>
 __global__ __launch_bounds__(256) void layernorm_slab_kernel(bf16* out, const float* __restrict__ slabs,
                                                              const bf16* __restrict__ bias, const bf16* res,
                                                              const bf16* __restrict__ gamma, const bf16* __restrict__ beta,
-                                                             int rows, float eps, int work, Upcoming next) {
+                                                             int rows, float eps, int work, Upcoming next, Upcoming then) {
   if constexpr (AHEAD) {
     asm volatile("" ::"s"(out), "s"(slabs), "s"(bias), "s"(res), "s"(gamma), "s"(beta), "s"(rows), "s"(eps), "s"(work));
-    if (__builtin_expect((int)blockIdx.x >= work, 0)) return read_upcoming<256>(next, work);
+    if (__builtin_expect((int)blockIdx.x >= work, 0)) {
+      read_upcoming<256>(next, work);
+      if (then.bytes) read_upcoming<256>(then, work);
+      return;
+    }
   }
   constexpr int cols = 128 * CP;
   const int lane = threadIdx.x & 63;
@@ -585,31 +593,33 @@ int rmsnorm_slabs(void* out, void* res_out, const void* slabs, int S, long slab_
   return rmsnorm_slabs_t(out, res_out, (const float*)slabs, S, slab_stride, res_in, w, rows, cols, eps, s);
 }
 
-// Workgroups of 256 behind a LayerNorm's that read the next projection's weights, 8 loads a thread.  us a forward, weights of
+// Workgroups of 256 behind a LayerNorm's that read the next projection's weights (and those of the one behind it: encoder.hip), 8
+// loads of the former a thread.  us a forward, weights of
 // three copies in turn, without -> with 16 / 8 / 4 loads: bge-base 120 tokens 430 -> 431 / 422 / 423, 240 502 -> 495 / 486 / 486, 816
 // 663 -> 640 / 632 / 634, 1500 854 -> 830 / 824 / 831, 3000 1,227 -> 1,208 / 1,207 / 1,212, 6000 2,008 -> 2,004 / 2,002 / 1,995;
 // bge-large 180 1,108 -> 1,066 / 1,050 / 1,054, 600 1,460 -> 1,421 / 1,432 / 1,434, 1200 2,002 -> 1,959 / 1,957 / 1,969, but 1800 2,245 ->
 // 2,277 / 2,253 / 2,261: more rows need the weights less, and larger ones take longer than the norm.
-static int norm_readers(const Upcoming& next, int rows) {
+static int norm_readers(const Upcoming& next, Upcoming& then, int rows) {
+  if (!then.w || then.bytes % 128 || (uintptr_t)then.w % 16) then = {};
   if (!next.w || next.bytes < 128 || next.bytes % 128 || (uintptr_t)next.w % 16 || (double)rows * next.bytes > 14e9) return 0;
   return (int)(((long)next.bytes / 8 + 8 * 4096 - 1) / (8 * 4096) * 8);
 }
 
 int layernorm(void* out, const void* x, const void* res_in, const void* gamma, const void* beta, int rows, int cols,
-              float eps, hipStream_t s, Upcoming next) {
+              float eps, hipStream_t s, Upcoming next, Upcoming then) {
   if (rows <= 0) return 0;
   if (cols % 8 || cols > 16384) return hipErrorInvalidValue;
   // encoder widths: one wave per LN_RPW rows, 4 waves per workgroup
   constexpr int LN_RPW = 2;  // 4 measured the same (34.0 us)
-  const int work = (rows + 4 * LN_RPW - 1) / (4 * LN_RPW), more = norm_readers(next, rows);
+  const int work = (rows + 4 * LN_RPW - 1) / (4 * LN_RPW), more = norm_readers(next, then, rows);
 #define LN_ROWS(CPL)                                                                                                 \
   if (cols == 256 * CPL) {                                                                                           \
     if (more)                                                                                                        \
       hipLaunchKernelGGL((layernorm_rows_kernel<CPL, LN_RPW, true>), dim3(work + more), dim3(256), 0, s, (bf16*)out, \
-                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next, then); \
     else                                                                                                             \
       hipLaunchKernelGGL((layernorm_rows_kernel<CPL, LN_RPW, false>), dim3(work), dim3(256), 0, s, (bf16*)out,       \
-                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+                         (const bf16*)x, (const bf16*)res_in, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next, then); \
     return hipGetLastError();                                                                                        \
   }
   LN_ROWS(3)
@@ -621,20 +631,20 @@ int layernorm(void* out, const void* x, const void* res_in, const void* gamma, c
 }
 
 int layernorm_slabs(void* out, const void* slabs_, int S, const void* bias, const void* res, const void* gamma,
-                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next) {
+                    const void* beta, int rows, int cols, float eps, hipStream_t s, Upcoming next, Upcoming then) {
   if (rows <= 0) return 0;
   const float* slabs = (const float*)slabs_;
   if ((uintptr_t)slabs % 8 || ((uintptr_t)out | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)gamma | (uintptr_t)beta) % 4)
     return hipErrorInvalidValue;
-  const int work = (rows + 3) / 4, more = norm_readers(next, rows);
+  const int work = (rows + 3) / 4, more = norm_readers(next, then, rows);
 #define LN_SLAB(CP, SS)                                                                                               \
   if (cols == 128 * CP && S == SS) {                                                                                  \
     if (more)                                                                                                         \
       hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS, true>), dim3(work + more), dim3(256), 0, s, (bf16*)out, slabs, \
-                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next, then); \
     else                                                                                                              \
       hipLaunchKernelGGL((layernorm_slab_kernel<CP, SS, false>), dim3(work), dim3(256), 0, s, (bf16*)out, slabs,       \
-                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next); \
+                         (const bf16*)bias, (const bf16*)res, (const bf16*)gamma, (const bf16*)beta, rows, eps, work, next, then); \
     return hipGetLastError();                                                                                         \
   }
 #define LN_SLABS(CP) LN_SLAB(CP, 2) LN_SLAB(CP, 3)

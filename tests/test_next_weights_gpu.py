@@ -65,7 +65,7 @@ def test_norm(rows, cols, residual):
     x, r, g, o, out = _r(rows, cols), _r(rows, cols), _r(cols), _r(cols), torch.empty(rows, cols, dtype=torch.bfloat16, device=DEV)
     s = torch.cuda.current_stream().cuda_stream
     _each(lambda w, n: ops.native().layernorm(out.data_ptr(), x.data_ptr(), r.data_ptr() if residual else 0, g.data_ptr(), o.data_ptr(),
-                                              rows, cols, 1e-12, s, next=w, next_bytes=n), out)
+                                              rows, cols, 1e-12, s, next=w, next_bytes=n, then=w, then_bytes=n // 2), out)
 
 
 @pytest.mark.parametrize("rows,cols,S", [(1, 768, 2), (817, 768, 3), (600, 1024, 2), (2200, 384, 3)])
@@ -73,4 +73,4 @@ def test_norm_of_slabs(rows, cols, S):
     x, r, b, g, o = torch.randn(S, rows, cols, device=DEV), _r(rows, cols), _r(cols), _r(cols), _r(cols)
     out, s = torch.empty(rows, cols, dtype=torch.bfloat16, device=DEV), torch.cuda.current_stream().cuda_stream
     _each(lambda w, n: ops.native().layernorm_slabs(out.data_ptr(), x.data_ptr(), S, b.data_ptr(), r.data_ptr(), g.data_ptr(),
-                                                    o.data_ptr(), rows, cols, 1e-12, s, next=w, next_bytes=n), out)
+                                                    o.data_ptr(), rows, cols, 1e-12, s, next=w, next_bytes=n, then=w, then_bytes=n // 2), out)
