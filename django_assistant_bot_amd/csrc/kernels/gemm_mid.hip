@@ -959,21 +959,34 @@ static int wide_groups(int M, int N, int K, int min_tm, double* us) {
   return groups;
 }
 
-// Which kernel a product takes: the 256-row one where the estimates say 6.5 % less (798 of the 2,109 sizes of that sweep, 1.21
-// times as fast in the mean, slower in 3, by 0.8 % at worst; at 2 % less 881, slower in 10, and the step of Llama-3-8B at 850
-// tokens, down alone on this kernel, 12,864 -> 12,950).  us, 128 rows -> 256: Llama-3-8B's down at M 1280 144 -> 129,
-// 1500 168 -> 148, 2000 198 -> 172, 3000 322 -> 265, gate_up at M 700 184 -> 155, 1500 341 -> 290, Llama-3.2-1B's down at 3400
-// 115 -> 97; but o of Llama-3-8B at M 1093 51 -> 54, qkv at 640 41 -> 53: partial tiles of 256 KB a workgroup are 64 MB to
-// write and read, some 25 us of a full launch.
+// Which kernel a product takes: the 256-row one where the estimates say 13 % less (527 of the 1,156 sizes of that sweep with
+// three row tiles and more, 1.26 times as fast in the mean, none slower, the least 1.024; at 6.5 % less 656, 9 of them slower,
+// (1001, 4096, 14336) 0.95).  Between those lines a call has nothing or 1-2 % of it, too little for sums of K in another order:
+// prefill of Llama-3-8B, us of a call, 128 rows -> 256, and the ratio of the estimates of down: 660 tokens 11,902 -> 11,713
+// (0.907), 900 13,256 -> 13,249 and 1,000 13,691 -> 13,738 (0.892), 1,093 16,175 -> 15,940 here and 15,971 -> 15,877 on another
+// card (0.933), 1,350 18,905 -> 18,663 (0.892); below it 1,200 17,210 -> 16,636 (0.825), 1,280 17,578 -> 16,998, 1,500 19,876
+// -> 19,585 (0.821), 1,700 22,519 -> 21,606 (0.782), 2,000 24,336 -> 23,693 (0.806).  us of a launch, 128 rows -> 256:
+// Llama-3-8B's down at M 1500 168 -> 148, 2000 198 -> 172, 3000 322 -> 265, Llama-3.2-1B's down at 3400 115 -> 97; but o of
+// Llama-3-8B at M 1093 51 -> 54, qkv at 640 41 -> 53: partial tiles of 256 KB a workgroup are 64 MB to write and read, some 25
+// us of a full launch.
 static int mid_pick(int M, int N, int K, bool* wide, double* us) {
   const int groups = gemm_mid_groups(M, N, K);
   *us = groups ? mid_us(M, N, K, groups) : __builtin_huge_val();
   double w_us;
   const int w_groups = groups ? wide_groups(M, N, K, 3, &w_us) : 0;
-  *wide = w_groups && w_us < 0.935 * *us;
+  *wide = w_groups && w_us < 0.87 * *us;
   if (!*wide) return groups;
   *us = 1.1 * w_us;  // (beside gemm256: the step of Llama-3-8B at 3,000 tokens 34,732 us with it, 35,015 on this)
   return w_groups;
+}
+
+// Groups on which the 256-row kernel runs a product, 0: it does not; forced: where the rule would leave it to the other one, too.
+int gemm_mid_wide_groups(int M, int N, int K, int forced) {
+  bool wide;
+  double us;
+  if (forced) return wide_groups(M, N, K, 1, &us);
+  const int groups = mid_pick(M, N, K, &wide, &us);
+  return wide ? groups : 0;
 }
 
 // Estimated us of the launch, infinite where the kernels do not take M.

@@ -69,3 +69,12 @@ def test_a_launch_that_gave_up_leaves_nothing_for_the_next(M, N, K):
         for variant in (256, 64, 256):
             out = kernels.gemm_mid(A, B, variant=variant)
             assert ((out.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 4096, 14336), (1000, 4096, 14336), (1093, 4096, 14336), (1200, 4096, 14336), (1700, 4096, 14336)])
+def test_the_kernel_of_128_rows_where_the_estimates_are_near(M, N, K):
+    """Unless its estimate is 13 % less the 256-row kernel is not taken: the sums of K keep their order."""
+    wide = kernels.native().gemm_mid_wide_groups(M, N, K, 0) > 0
+    assert wide == (M >= 1200)
+    A, B, _ = _case(M, N, K, 1)
+    assert torch.equal(kernels.gemm_mid(A, B), kernels.gemm_mid(A, B, variant=256 if wide else 64))
