@@ -1033,7 +1033,9 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   } else if (variant) {
     wide = false;
   }
-  if (!groups || (wide && (255L * lda + K) * 2 >= (1L << 31))) {
+  // (its buffer descriptors span 256 rows of the operands, of C and of the residual in 32 bits)
+  const bool spans = (255L * lda + K) * 2 < (1L << 31) && 512L * ldc < (1L << 32) && (!residual || 512L * ldr < (1L << 32));
+  if (!groups || (wide && !spans)) {
     if (variant == 256) return hipErrorInvalidValue;
     wide = false;
   }

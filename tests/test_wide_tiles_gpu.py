@@ -78,3 +78,22 @@ def test_the_kernel_of_128_rows_where_the_estimates_are_near(M, N, K):
     assert wide == (M >= 1200)
     A, B, _ = _case(M, N, K, 1)
     assert torch.equal(kernels.gemm_mid(A, B), kernels.gemm_mid(A, B, variant=256 if wide else 64))
+
+
+@pytest.mark.parametrize("stride,residual", [(1 << 23, False), (1 << 23, True), ((1 << 23) - 8, False)])
+def test_output_rows_that_lie_far_apart(stride, residual):
+    """256 rows of 2^23 elements are 4 GiB, past a buffer descriptor: the 128-row kernel takes them."""
+    M, N, K = 700, 28672, 4096
+    assert kernels.native().gemm_mid_wide_groups(M, N, K, 0)
+    A, B, exp = _case(M, N, K, 1)
+    out, res = torch.empty(M * stride, dtype=torch.bfloat16, device=DEV).as_strided((M, N), (stride, 1)), None
+    out.fill_(7.0)
+    if residual:
+        res = torch.empty(M * stride, dtype=torch.bfloat16, device=DEV).as_strided((M, N), (stride, 1))
+        res.normal_()
+    got = kernels.gemm_mid(A, B, residual=res, out=out).float()
+    tol = 2.0 ** -8 * exp.abs() + 1e-4  # one rounding to bf16, a second with the residual
+    if residual:
+        exp = exp + res.float()
+        tol = tol + 2.0 ** -8 * exp.abs()
+    assert ((got - exp).abs() <= tol).all()
