@@ -24,17 +24,18 @@
 //   * a tile whose K range spans several groups is combined in-launch by its OWNER, the group
 //     holding the tile's first K-steps: that segment ends the owner's range, so in time it finishes
 //     last.  The other segments store their fp32 partial (write-through sc1 stores, 1 KB per
-//     wave-instruction) and raise a per-slot ready flag two K-steps later, when the pipeline's own
+//     wave-instruction) and count themselves in at the tile two K-steps later, when the pipeline's own
 //     counted wait has retired the stores (no drain); the owner keeps its partial in registers,
-//     waits for each flag (bounded spin), adds the partials with sc1 loads in segment order (no
-//     fence needed: cdna_hip_programming.md section 5 item 2), clears the flags and runs the
-//     epilogue.  A flag holds the
-//     number of the launch that raised it (the workgroups count their ends in the workspace, so a
-//     replayed graph goes on counting): what a launch that gave up left raised, or raised late, means
-//     nothing to the next.  Only owners wait, on producers that never wait, so there is no deadlock (and the
-//     grid is at most one workgroup per CU).  Replaces a last-arriver combine (every segment stored
-//     and drained, then an atomic ticket) that cost 5-9 us per launch on the small projections
-//     (profiles/gemm_mid_r6.md).
+//     waits until all are in, adds the partials with sc1 loads in segment order (no
+//     fence needed: cdna_hip_programming.md section 5 item 2), clears the count and runs the
+//     epilogue;
+//   * no workgroup waits without end.  The parts an owner waits for may stand on any XCD and behind it in the order of
+//     placement, and workgroups of another stream's launch that wait in the same way can hold the CUs they need (16 row
+//     tiles: two launches with half of each XCD's CUs each).  So after some 0.1 ms an owner stores its sum too, counts itself
+//     in and goes on, and the workgroup whose part comes last adds them all, in the same order: the same bits.  One count a
+//     tile instead of a flag a part: 0.98-1.06 times the speed over 136 sizes of Llama-3-8B's and 1B's projections, 1.01 in the mean.
+//     A last-arriver combine for every tile (every segment stored and drained, then an atomic ticket) cost 5-9 us
+//     per launch on the small projections (profiles/gemm_mid_r6.md).
 #include <cmath>
 
 #include "common.h"
@@ -51,8 +52,10 @@ struct GMid {
   const bf16* B;  // shuffle_weights layout, [N][K]
   bf16* C;
   const bf16* residual;   // GLU epilogues with RES: fp32 bias [gate N / 2 | up N / 2] instead
-  float* slabs;  // [tiles_m][gn][2] partial tiles of 128 x 256 fp32 (in accumulator order)
-  int* cnt;      // [tiles_m][gn][2] ready flags of the stored partial tiles (the launch that stored them), zero at rest
+  float* slabs;  // [tiles_m][gn][2] partial tiles of 128 x 256 fp32 (in accumulator order): a range's first part, and the sum
+                 // that an owner handed over
+  int* cnt;      // zero at rest.  128 rows: [8 spx ..) the parts of a divided tile that are in, by its owner, [tiles_m][gn]; 256 rows:
+                 // [.. 8 spx) ready flags (the launch that stored a partial tile)
   unsigned* ended;  // [8][32]: workgroups of an XCD label that ended, over all launches on this workspace, a line each
   long spin_limit;
   int M, N, K;
@@ -122,8 +125,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   using Geo = MidGeo<BK>;
   constexpr int kStage = Geo::kStage, kStages = Geo::kStages, kDist = Geo::kDist, kDma = Geo::kDma;
   constexpr int kA = Geo::kA;
-  // behind the ring: the count the launch's number comes from
-  __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem + 256];
+  __shared__ __attribute__((aligned(16))) char smem[Geo::kSmem];
 
   // ---- which group / row tile this block is: blocks b, b + 8, ... share an XCD label.  The slots of an XCD that whole
   // groups leave over are joined, XCD after XCD, into further groups
@@ -232,13 +234,6 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
       ++s_nt;
     }
   };
-  // The launch's number, the same for all of its workgroups: this one has not ended yet, so its launch has added less
-  // than the label's p.spx workgroups to their count (which may wrap: 2^32 is a multiple of 32).  Wave 0 copies the count
-  // to LDS ahead of the first stage, so that it has landed when that has (a scalar load in front, and one count for all
-  // labels, cost 0.8 to 2 us a launch; the addition behind the prologue instead of at the end 1 to 3 us where a group
-  // takes few K-steps).  The number is read by an asm statement: before an ordinary read hipcc drains the copies in flight.
-  if (w == 0)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(mk_rsrc(ended, 4), (lds_void*)(smem + Geo::kSmem), 4, 0u, 0u, 0, 0);
   // prologue: iterations start .. start + kDist - 1 in flight (buffers 0 ..), the first landed
 #pragma unroll
   for (int d = 0; d < kDist; ++d)
@@ -255,32 +250,51 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
     else wait_vmc<0>();
   }
   mbar();
-  unsigned before;
-  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
-               : "=v"(before)
-               : "v"((unsigned)(uintptr_t)(lds_void*)(smem + Geo::kSmem))
-               : "memory");
-  const int launch = (int)((unsigned)__builtin_amdgcn_readfirstlane((int)before) / (unsigned)p.spx) + 1;
 
   int it = start;
   int b = 0;  // ring buffer of iteration `it`
   // VMEM stores issued since the last phase's wait (younger than the DMA in flight): an epilogue's
   // kE or a published partial's kSlabSt; the next phase's counted wait lets them stay in flight
   int after_st = 0;
-  // a partial tile stored by this workgroup whose ready flag is not raised yet: raised at the
-  // second phase after the stores, when that phase's vmcnt(kDma) has retired them (no drain)
-  int pend_flag = -1, pend_phases = 0;
+  // the tile of a partial stored by this workgroup that is not counted in yet: counted at the second phase after the
+  // stores, when that phase's vmcnt(kDma) has retired them (no drain)
+  int pend = -1, pend_phases = 0;
+  int before = -1;  // lane 0: how many of its tile's parts were in before this workgroup's first one
   const __amdgpu_buffer_rsrc_t rS = mk_rsrc(p.slabs, p.slab_bytes);
   auto slab_off = [&](int jj, int side) { return (unsigned)(((mt * p.gn + jj) * 2 + side) * kSlabFloats) * 4u; };
-  auto flag_of = [&](int jj, int side) { return p.cnt + (mt * p.gn + jj) * 2 + side; };
-  auto raise_flag = [&]() {  // after every wave's stores retired and a barrier
-    if (tid == 0) __hip_atomic_store(p.cnt + pend_flag, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    pend_flag = -1;
+  auto count_in = [&](int at) {  // after every wave's stores retired and a barrier
+    return tid == 0 ? __hip_atomic_fetch_add(p.cnt + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
   };
-  while (it < end) {
-    const int nt = it / kt;
-    const int k0 = it - nt * kt;
-    const int k1 = min(kt, k0 + (end - it));
+  auto publish = [&](int side) {
+    const unsigned own = slab_off(j, side);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][jn]), rS, (unsigned)(tid * 16),
+                                               own + (unsigned)((i * 4 + jn) * 8192), 16);
+  };
+  auto add_partial = [&](int jj, int side) {
+    const unsigned off = slab_off(jj, side);
+    u32x4 v[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn)
+        v[i][jn] = __builtin_amdgcn_raw_buffer_load_b128(rS, (unsigned)(tid * 16), off + (unsigned)((i * 4 + jn) * 8192), 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn) acc[i][jn] += __builtin_bit_cast(f32x4, v[i][jn]);
+  };
+  for (;;) {
+    // behind its range a workgroup whose part of the first tile came last finishes that tile (a round without K-steps)
+    const bool late = it >= end;
+    const int nt = (late ? start : it) / kt;
+    const int j_lo = grp_owner(nt * kt, p.q, p.r), j_hi = grp_owner(nt * kt + kt - 1, p.q, p.r);
+    if (late && (j == j_lo || !__syncthreads_or(before == j_hi - j_lo))) break;
+    const int k0 = late ? 0 : it - nt * kt;
+    const int k1 = late ? 0 : min(kt, k0 + (end - it));
     if (wr == 1) mbar();  // group 1 one barrier behind through the K-loop (ping-pong)
     for (int kk = k0; kk < k1; ++kk, ++it) {
       const char* sb = smem + b * kStage;
@@ -311,7 +325,10 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
       }
       after_st = 0;
       mread_bar();
-      if (pend_flag >= 0 && ++pend_phases >= 2) raise_flag();  // this phase's wait retired the stores
+      if (pend >= 0 && ++pend_phases >= 2) {  // this phase's wait retired the stores
+        before = count_in(pend);
+        pend = -1;
+      }
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -324,85 +341,63 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
       b = b == kStages - 1 ? 0 : b + 1;
     }
     if (wr == 0) mbar();  // pairs with group 1's last K-loop barrier
-    if (pend_flag >= 0) {  // (a one-phase segment followed: drain and raise now)
+    if (pend >= 0) {  // (a one-phase segment followed: drain and count now)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      raise_flag();
+      before = count_in(pend);
+      pend = -1;
     }
 
     // ---- segment end.  A whole tile goes straight to the epilogue.  A split tile's segments are
     // held by groups j_lo .. j_hi in K order; its OWNER is j_lo, whose segment (the tile's first
     // K-steps) ends its own range, so in time it finishes last.  The other segments store their
-    // fp32 partial (sc1, write-through) and raise a per-slot ready flag; the owner never stores its
-    // own, waits for each flag (bounded spin), adds the partials in segment order (its registers
-    // first), clears the flags and runs the epilogue.  Nobody else waits, so the owner's wait
-    // cannot deadlock (and the grid is <= one workgroup per CU anyway).
+    // fp32 partial (sc1, write-through) and count themselves in; the owner waits until all are in
+    // and adds them in segment order, its registers first.  Where they stay out it stores its own as well: of all of
+    // them one counts itself in last, and that workgroup adds them.
     const int n0 = nt * 256;
     bool write = true;
     if (k0 != 0 || k1 != kt) {
-      const int j_lo = grp_owner(nt * kt, p.q, p.r), j_hi = grp_owner(nt * kt + kt - 1, p.q, p.r);
-      const int side = start >= nt * kt ? 0 : 1;
-      if (j != j_lo) {
-        const unsigned own = slab_off(j, side);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int jn = 0; jn < 4; ++jn)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][jn]), rS,
-                                                   own + (unsigned)(((i * 4 + jn) * 512 + tid) * 16), 0, 16);
+      const int at = 8 * p.spx + mt * p.gn + j_lo;  // where the tile's parts are counted
+      if (late) {
+        add_partial(j_lo, 1);
+      } else if (j != j_lo) {
+        publish(0);
         after_st = kSlabSt;
-        if (!DIAG) {  // (DIAG: the owner reads nothing, so no flag may be left raised)
-          pend_flag = (int)(flag_of(j, side) - p.cnt);
+        if (!DIAG) {  // (DIAG: the owner reads nothing, so nothing may be counted)
+          pend = at;
           pend_phases = 0;
           if (it >= end) {  // nothing left to hide the drain behind
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
-            raise_flag();
+            before = count_in(at);
+            pend = -1;
           }
         }
         write = false;
       } else if (DIAG) {
         write = false;
       } else {
-        bool ok = true;
-        for (int jj = j_lo + 1; jj <= j_hi; ++jj) {
-          const int sd = grp_start(jj, p.q, p.r) >= nt * kt ? 0 : 1;
-          int* fl = flag_of(jj, sd);
-          if (tid == 0) {
-            long spins = 0;
-            while (__hip_atomic_load(fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != launch) {
-              if (++spins > p.spin_limit) {
-                ok = false;  // a producer never published (cannot happen in a healthy launch)
-                break;
-              }
-              __builtin_amdgcn_s_sleep(2);
+        bool in = true;
+        if (tid == 0) {
+          long spins = 0;
+          while (__hip_atomic_load(p.cnt + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != j_hi - j_lo) {
+            if (++spins > p.spin_limit) {
+              in = false;
+              break;
             }
-            if (ok) __hip_atomic_store(fl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_sleep(2);
           }
-          __syncthreads();  // every thread loads only after lane 0 saw the flag
-          const unsigned off = slab_off(jj, sd);
-          u32x4 v[4][4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int jn = 0; jn < 4; ++jn)
-              v[i][jn] = __builtin_amdgcn_raw_buffer_load_b128(rS, off + (unsigned)(((i * 4 + jn) * 512 + tid) * 16),
-                                                               0, 16);
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int jn = 0; jn < 4; ++jn) acc[i][jn] += __builtin_bit_cast(f32x4, v[i][jn]);
         }
-        ok = __builtin_amdgcn_readfirstlane((int)ok) != 0 || tid != 0;
-        if (!__syncthreads_and(ok)) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int jn = 0; jn < 4; ++jn) {
-              const float nan = __builtin_nanf("");
-              acc[i][jn] = f32x4{nan, nan, nan, nan};
-            }
+        if (!__syncthreads_and(in)) {  // (every thread loads only after lane 0 saw the count)
+          publish(1);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+          write = __syncthreads_or(count_in(at) == j_hi - j_lo);
         }
+      }
+      if (write) {
+        for (int jj = j_lo + 1; jj <= j_hi; ++jj) add_partial(jj, 0);
+        if (tid == 0) __hip_atomic_store(p.cnt + at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
     if (write) {
@@ -491,6 +486,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
       }
       after_st = kE;
     }
+    if (late) break;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -606,7 +602,12 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
 
   int it = start;
   int nt = start / kt, k0 = start - nt * kt;
-  // the launch's number: see the kernel above
+  // The launch's number, the same for all of its workgroups: this one has not ended yet, so its launch has added less
+  // than the label's p.spx workgroups to their count (which may wrap: 2^32 is a multiple of 32; the 128-row kernel counts its
+  // own there too).  What a launch that gave up left raised, or raised late, so means nothing to the next.  Wave 0 copies the count
+  // to LDS ahead of the first stage, so that it has landed when that has (in the 128-row kernel a scalar load in front, and one
+  // count for all labels, cost 0.8 to 2 us a launch; the addition behind the prologue instead of at the end 1 to 3 us where a
+  // group takes few K-steps).  The number is read by an asm statement: before an ordinary read hipcc drains the copies in flight.
   if (w == 0)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(mk_rsrc(ended, 4), (lds_void*)(smem + 2 * kWBuf), 4, 0u, 0u, 0, 0);
   // prologue: K-step 0 complete, A0 / B0 / B1 of K-step 1 in flight
@@ -963,8 +964,8 @@ static int wide_groups(int M, int N, int K, int min_tm, double* us) {
 // three row tiles and more, 1.26 times as fast in the mean, none slower, the least 1.024; at 6.5 % less 656, 9 of them slower,
 // (1001, 4096, 14336) 0.95).  Between those lines a call has nothing or 1-2 % of it, too little for sums of K in another order:
 // prefill of Llama-3-8B, us of a call, 128 rows -> 256, and the ratio of the estimates of down: 660 tokens 11,902 -> 11,713
-// (0.907), 900 13,256 -> 13,249 and 1,000 13,691 -> 13,738 (0.892), 1,093 16,175 -> 15,940 here and 15,971 -> 15,877 on another
-// card (0.933), 1,350 18,905 -> 18,663 (0.892); below it 1,200 17,210 -> 16,636 (0.825), 1,280 17,578 -> 16,998, 1,500 19,876
+// (0.907), 900 13,256 -> 13,249 and 1,000 13,691 -> 13,738 (0.892), 1,093 16,175 -> 15,940, 15,942 -> 15,562 and 15,971 -> 15,877 on other
+// cards (0.933), 1,350 18,905 -> 18,663 (0.892); below it 1,200 17,210 -> 16,636 (0.825), 1,280 17,578 -> 16,998, 1,500 19,876
 // -> 19,585 (0.821), 1,700 22,519 -> 21,606 (0.782), 2,000 24,336 -> 23,693 (0.806).  us of a launch, 128 rows -> 256:
 // Llama-3-8B's down at M 1500 168 -> 148, 2000 198 -> 172, 3000 322 -> 265, Llama-3.2-1B's down at 3400 115 -> 97; but o of
 // Llama-3-8B at M 1093 51 -> 54, qkv at 640 41 -> 53: partial tiles of 256 KB a workgroup are 64 MB to write and read, some 25
@@ -998,10 +999,10 @@ double gemm_mid_us(int M, int N, int K) {
 }
 
 // Workspace the launcher needs: partial slabs and behind them the counts of ended workgroups (bytes), and ready flags
-// (ints).
+// and counts (ints).
 static long slabs_end() { return (long)cu_count() * 2 * kSlabFloats * 4; }
 long gemm_mid_slab_bytes() { return slabs_end() + 8 * 128; }
-// ready flags of the partial tiles: two per (row tile, group) <= two per workgroup
+// ready flags of the 256-row kernel's workgroups, and behind them the 128-row kernel's counts, one per (row tile, group)
 int gemm_mid_counters(int M, int N) {
   (void)M;
   (void)N;
@@ -1011,7 +1012,8 @@ int gemm_mid_counters(int M, int N) {
 // epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over
 // 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs:
 // gemm_mid_slab_bytes() bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the
-// launch leaves them zero).  spin_limit: looks at a flag before an owner gives up and writes NaN.  variant (A/B harness only): 0 default
+// launch leaves them zero).  spin_limit: looks at a count before an owner hands its tile over (256 rows: at a flag, before it gives up
+// and writes NaN), -1: the kernel's own.  variant (A/B harness only): 0 default
 // (by the estimates), 32 / 64 the 128-row kernel with that K-step, 256 the 256-row kernel, + 1000 = DIAG 1 (split tiles not combined: timing only).
 // BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank
 // conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
@@ -1061,7 +1063,7 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.kt = K / (wide ? 128 : bk);
   const int grid = cu_count() & ~7;
   p.ended = (unsigned*)((char*)slabs + slabs_end());
-  p.spin_limit = spin_limit;
+  p.spin_limit = spin_limit >= 0 ? spin_limit : wide ? 1L << 22 : 128;
   p.spx = grid / 8;
   p.gn = groups;
   if (wide) p.tiles_n /= 8;  // an XCD's

@@ -678,8 +678,8 @@ _MID_WS: dict = {}
 
 
 def _mid_workspace(device: torch.device, s: int):
-    """Partial-tile slabs + ready flags of ``gemm_mid``, one set per (device, stream): two streams
-    running the kernel at once must not share them.  The flags are zero at rest (every launch leaves
+    """Partial-tile slabs, ready flags and counts of ``gemm_mid``, one set per (device, stream): two streams
+    running the kernel at once must not share them.  Flags and counts are zero at rest (every launch leaves
     them zero); the slabs' last 1024 bytes count the workgroups that ended."""
     key = (device.index, s)
     ws = _MID_WS.get(key)

@@ -79,3 +79,63 @@ def test_replays_go_on_counting():
             eager = ops.kernels.gemm_mid(a2, b2)
             s.synchronize()
             assert all(_close(o, exp).all() for o in outs) and _close(eager, exp2).all()
+
+
+# tiles in equal parts, of unequal length, in groups joined over the XCDs, parts of one K-step; with parts in front of others of
+# their group's range and without
+HANDED = [(300, 512, 4096), (44, 256, 8192), (384, 4096, 4096), (4096, 256, 4096), (300, 6144, 4096), (2000, 6144, 4096),
+          (1093, 4096, 14336), (1400, 6144, 1024), (2200, 2560, 1024), (1500, 5120, 128)]
+
+
+def _run(A, B, out, spin_limit, s, res=None, epilogue=0, group=1):
+    slabs, cnt = kernels._mid_workspace(A.device, s.cuda_stream)
+    (M, K), N = A.shape, B.shape[0]
+    kernels.native().gemm_mid(A.data_ptr(), K, B.data_ptr(), out.data_ptr(), out.stride(0), 0 if res is None else res.data_ptr(),
+                              N, M, N, K, epilogue, slabs.data_ptr(), slabs.numel() * 4, cnt.data_ptr(), cnt.numel(),
+                              s.cuda_stream, variant=64, b_group=group, spin_limit=spin_limit)
+    return cnt
+
+
+@pytest.mark.parametrize("M,N,K", HANDED)
+@pytest.mark.parametrize("kind", ["plain", "residual", "glu"])
+@pytest.mark.parametrize("busy", [False, True])
+def test_owners_that_do_not_wait_hand_their_tiles_over(M, N, K, kind, busy):
+    """An owner whose other parts are not in on the first look stores its own, and the last one in finishes the tile: the bits of a
+    launch that waits, and no count left.  Busy: a product on another stream holds CUs, so workgroups are placed unevenly."""
+    A, B, _ = _case(M, N, K, 1)
+    group, epilogue, width = (8, ops.EPI_SWIGLU8, N // 2) if kind == "glu" else (1, 0, N)
+    res = torch.randn(M, N, device=DEV).to(torch.bfloat16) if kind == "residual" else None
+    s, other = torch.cuda.current_stream(), torch.cuda.Stream()
+    exp = torch.empty(M, width, dtype=torch.bfloat16, device=DEV)
+    _run(A, B, exp, 1 << 22, s, res, epilogue, group)
+    X = torch.randn(2000, 2048, device=DEV).to(torch.bfloat16)
+    Y = ops.shuffle_weights(torch.randn(4096, 2048, device=DEV).to(torch.bfloat16))
+    other.wait_stream(s)
+    for _ in range(8):
+        out = torch.full_like(exp, 7.0)
+        if busy:
+            with torch.cuda.stream(other):
+                for _ in range(4):
+                    ops.kernels.gemm256(X, Y, shuffled=True)
+        cnt = _run(A, B, out, 0, s, res, epilogue, group)
+        assert torch.equal(out, exp) and exp.isfinite().all()
+        assert not cnt.any()
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,N,K", [(2000, 6144, 4096), (1093, 4096, 14336), (300, 6144, 4096)])
+def test_two_streams(M, N, K):
+    """Launches of two streams whose owners wait for workgroups that the other launch keeps from being placed."""
+    A, B, _ = _case(M, N, K, 2)
+    exp = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    _run(A, B, exp, 1 << 22, torch.cuda.current_stream())
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [[torch.empty_like(exp) for _ in range(20)] for _ in streams]
+    for s in streams:
+        kernels._mid_workspace(A.device, s.cuda_stream)
+    torch.cuda.synchronize()
+    for pair in zip(*outs):
+        for s, out in zip(streams, pair):
+            _run(A, B, out, -1, s)
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, exp) for each in outs for out in each)
