@@ -619,7 +619,7 @@ struct RingTile {
   int bm, bn, fit;
   float start, round, tile, step, share;
 };
-constexpr RingTile kRing[] = {{32, 64, 4, 2.28f, 0.f, 0.46f, 0.209f, 0.132f},    {64, 64, 3, 2.52f, 0.89f, 0.42f, 0.256f, 0.201f},
+constexpr RingTile kRing[] = {{32, 64, 3, 2.28f, 0.f, 0.46f, 0.209f, 0.132f},    {64, 64, 3, 2.52f, 0.89f, 0.42f, 0.256f, 0.201f},
                               {96, 64, 2, 3.09f, 2.81f, 0.45f, 0.309f, 0.245f},  {96, 96, 2, 3.46f, 3.76f, 0.91f, 0.381f, 0.289f},
                               {64, 128, 2, 3.15f, 1.72f, 0.92f, 0.316f, 0.264f}, {64, 192, 1, 3.50f, 2.25f, 1.67f, 0.392f, 0.150f},
                               {128, 192, 1, 4.69f, 4.32f, 2.92f, 0.578f, 0.150f}, {128, 256, 1, 5.34f, 4.64f, 3.36f, 0.660f, 0.157f}};
@@ -661,6 +661,7 @@ bool ring_wins(int M, int N, int K, int gelu, int residual) {
 template <int I, int WM, int WN, int NS>
 static void ring_launch(const SmallParams& p, int gelu, hipStream_t s) {
   constexpr RingTile t = kRing[I];
+  static_assert(t.fit == 163840 / ((t.bm + t.bn) * 128 * NS), "as many tiles at a time as a CU's LDS has rings for");
   const int slices = p.slabs ? p.slices : 1;
   const dim3 grid(((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * slices), block(64 * WM * WN);
   if (p.slabs) hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, false, true>), grid, block, 0, s, p);
@@ -668,7 +669,6 @@ static void ring_launch(const SmallParams& p, int gelu, hipStream_t s) {
   else hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, false>), grid, block, 0, s, p);
 }
 
-// The ring buffers are as many as `fit` tiles of them leave room for.
 static void gemm_ring(const SmallParams& p, int gelu, hipStream_t s) {
   switch (ring_tile(p.M, p.N, p.K, gelu, p.slabs ? p.slices : 1)) {
     case 0: return ring_launch<0, 2, 2, 4>(p, gelu, s);
