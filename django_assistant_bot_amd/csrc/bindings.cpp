@@ -635,6 +635,7 @@ PYBIND11_MODULE(_native, m) {
   });
 
   m.def("small_tile", &dab::small_tile);
+  m.attr("RING_TILE") = dab::kRingTile;
   m.def("encoder_forward", [](u ids, u pos, u cu, int T, int batch, int max_len, int H, int heads, int F, float eps, u word,
                               u pos_table, u type, u gain, u offset, const std::vector<u>& layers, u x, u y, u att, u qkv,
                               u ffn, u slabs, u s) {

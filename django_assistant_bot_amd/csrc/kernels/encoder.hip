@@ -9,23 +9,22 @@
 
 namespace dab {
 
-// Which tile of gemm_small a projection with row-major weights takes, -1: the 128 x 128 / 256 x 256 kernels unless ring_wins.
-// 2 to 5 are the barrier-stepped ring, whose tile ring_tile (gemm_small.hip) picks.
+// Which kernel of gemm_small a projection with row-major weights takes: 0, 1, 6, 7, 8 a tile of the split-K kernel, kRingTile
+// (3) the barrier-stepped ring, whose tile ring_tile (gemm_small.hip) picks, -1 the 128 x 128 / 256 x 256 kernels unless ring_wins.
 //
 // The smallest tile that still gives each CU about one workgroup: K split over a workgroup's waves up to 256 tiles of
 // 16 x 16, 32 x 16, 32 x 32, 32 x 64, and 64 x 64 where K is long (K of 384 and more: every other kernel sums K in one
-// order, so that results there do not depend on M); then the barrier-stepped ring up to 1200 tiles of 64 x 64 (1000
-// where M is over 3 N: each XCD streams the rows again for every column block), with a long K up to 512 of them or 256 of
-// 128 x 128.  Both sides of each line, us (us of the tile before -> of the tile after it; the ring with one tile of 32 x 64, 64 x 64
-// or 128 x 128): 192 tiles of 16 x 16 at (64, 768, 768) 3.1 /
+// order, so that results there do not depend on M); then the ring, up to 1200 tiles of 64 x 64 (1000 where M is over 3 N: each
+// XCD streams the rows again for every column block), with a long K up to 256 of 128 x 128.  Both sides of each line, us (us of the
+// tile before -> of the tile after it): 192 tiles of 16 x 16 at (64, 768, 768) 3.1 /
 // 3.4, 288 at (19, 2304, 768) 3.6 / 3.4; 192 of 32 x 16 at (128, 768, 768) 3.4 / 3.8, 288 at (64, 2304, 768) 5.3 / 4.1;
 // 192 of 32 x 32 at (256, 768, 768) 3.9 / 4.6, 288 at (128, 2304, 768) 5.3 / 4.8; 192 of 32 x 64 at (512, 768, 768) 5.1
-// / 5.5, with K 3072 11.4 / 14.7, 288 at (256, 2304, 768) 7.9 / 6.4; 224 of 64 x 64 at (870, 1024, 4096) 17.6 / 20.6,
-// 288 at (1500, 768, 3072) 26.5 / 19.6, but with the short K 168 at (870, 768, 768) 7.0 / 6.7; 288 of the ring's 32 x
-// 64 at (256, 2304, 768) 6.4 / 6.8, 384 at (256, 3072, 768) 8.1 / 7.3; 1152 of its 64 x 64 at (2048, 2304, 768) 20.2 /
-// 25.4 (gemm256), 1692 at (3000, 2304, 768) 29.3 / 26.7, 1008 at (5333, 768, 768) 18.0 / 18.4, 1104 at (5866, 768, 768)
-// 20.3 / 18.5, at (4400, 1024, 1024) 23.9 / 22.0; with K 3072 288 at (1500, 768, 3072) 19.8 / 36.0, 564 at (3000, 768,
-// 3072) 43.0 / 36.1; 192 of 128 x 128 at (4096, 768, 3072) 37.7 / 64.4 (gemm256), 282 at (6000, 768, 3072) 71.3 / 64.0.
+// / 5.5 (ring of 64 x 64, as below), with K 3072 11.4 / 14.7, 288 at (256, 2304, 768) 7.9 / 6.4; 224 of 64 x 64 at (870, 1024,
+// 4096) 17.6 / 20.6, 288 at (1500, 768, 3072) 26.5 / 19.6, but with the short K 168 at (870, 768, 768) 7.0 / 6.7.  The ring's end
+// was measured when it had no tiles but 64 x 64 and, with a long K, 128 x 128: ring / gemm256 with 1152 tiles at (2048, 2304, 768)
+// 20.2 / 25.4, 1692 at (3000, 2304, 768) 29.3 / 26.7, 1008 at (5333, 768, 768) 18.0 / 18.4, 1104 at (5866, 768, 768) 20.3 / 18.5, at (4400,
+// 1024, 1024) 23.9 / 22.0; 192 of 128 x 128 at (4096, 768, 3072) 37.7 / 64.4, 282 at (6000, 768, 3072) 71.3 / 64.0.  The tiles that it
+// has now only make it faster: up to there it is taken without a look at the estimates, behind them where ring_wins says so.
 int small_tile(int M, int N, int K) {
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (K >= 384) {
@@ -35,17 +34,15 @@ int small_tile(int M, int N, int K) {
     if (tiles(32, 64) <= 256) return 7;
     if (K > 1024 && tiles(64, 64) <= 256) return 8;
   }
-  if (tiles(32, 64) <= 320) return 2;
-  if (K <= 1024) return tiles(64, 64) <= (M > 3L * N ? 1000 : 1200) ? 3 : -1;
-  if (tiles(64, 64) <= 512) return 4;
-  return tiles(128, 128) <= 256 ? 5 : -1;
+  const bool ring = K <= 1024 ? tiles(64, 64) <= (M > 3L * N ? 1000 : 1200) : tiles(128, 128) <= 256;
+  return ring ? kRingTile : -1;
 }
 
 // y[M, N] = x[M, K] w[N, K]^T + b (GELU) (+ residual), everything contiguous: ops.gemm_bt's choice of kernel.
 static int projection(const bf16* x, const void* w, const void* b, const bf16* residual, bf16* y, int M, int N, int K, int gelu,
                       hipStream_t s, Upcoming next = {}) {
   int tile = small_tile(M, N, K);
-  if (tile < 0 && ring_wins(M, N, K, gelu, residual != nullptr)) tile = 3;
+  if (tile < 0 && ring_wins(M, N, K, gelu, residual != nullptr)) tile = kRingTile;
   if (tile >= 0 && gemm_small_ok(M, N, K, K, K, N, N) &&
       !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8))
     return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s, next);
@@ -73,14 +70,15 @@ int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int ba
   // where that one's tiles leave no room for readers.  us a forward, weights of three copies in turn, without the latter -> with:
   // bge-base 240 tokens 481 -> 468, 816 632 -> 609, 1500 820 -> 798, 3000 1,209 -> 1,210; bge-large 180 1,040 -> 981, 600 1,428 ->
   // 1,369, 1200 1,937 -> 1,837, 1800 2,239 -> 2,222; where the next launch has readers too 120 405 -> 414.
-  auto reads_next = [](int tile) { return tile >= 0 && !(tile >= 2 && tile <= 5); };
+  auto reads_next = [](int tile) { return tile >= 0 && tile != kRingTile; };
   // x = LayerNorm(y), then out = x w^T + b: one launch where the projection takes a split-K tile (one or two row tiles, so
   // that a row is normalised by as many workgroups as read it anyway), two where its rows outgrow that
   auto norm_projection = [&](const uintptr_t* ln, const void* w, const void* b, bf16* out, int N, int gelu, Upcoming next) {
     const int tile = small_tile(T, N, H);
     if (gemm_ln_ok(T, N, H, tile) && !(((uintptr_t)w) % 16 || (ln[0] | ln[1] | (uintptr_t)b) % 8))
       return gemm_ln(y, (const void*)ln[0], (const void*)ln[1], eps, x, w, b, out, T, N, H, gelu, tile, s, next);
-    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s, {w, (unsigned)((long)N * H * 2)}, reads_next(tile) ? Upcoming{} : next);
+    const int e = layernorm(x, y, nullptr, (const void*)ln[0], (const void*)ln[1], T, H, eps, s, {w, (unsigned)((long)N * H * 2)},
+                            reads_next(tile) ? Upcoming{} : next);
     return e ? e : projection(x, w, b, nullptr, out, T, N, H, gelu, s, next);
   };
   const int slices = slabs ? slab_slices(T, H, F) : 0;

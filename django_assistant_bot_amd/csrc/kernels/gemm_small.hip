@@ -732,10 +732,7 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
   switch (tile) {
     SMALL(0, 1, 1, 8, 2)
     SMALL(1, 2, 1, 8, 2)
-    case 2:
-    case 3:
-    case 4:
-    case 5: gemm_ring(p, gelu, s); break;
+    case kRingTile: gemm_ring(p, gelu, s); break;
     SMALL(6, 2, 2, 8, 1)
     SMALL(7, 2, 4, 8, 1)
     SMALL(8, 4, 4, 8, 1)

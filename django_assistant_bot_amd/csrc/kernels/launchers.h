@@ -384,6 +384,7 @@ int topk_rows_2stage(const float* scores, long ld, int rows, int n, int k, float
                      int64_t index_base, int64_t* out_idx64, void* workspace, size_t workspace_bytes, hipStream_t s);
 
 // encoder.hip
+constexpr int kRingTile = 3;  // small_tile: the ring of gemm_small.hip
 int small_tile(int M, int N, int K);
 int encoder_forward(const int* ids, const int* pos, const int* cu, int T, int batch, int max_len, int H, int heads, int F,
                     int n_layers, float eps, const void* word, const void* pos_table, const void* type, const void* gain,

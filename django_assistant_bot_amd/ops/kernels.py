@@ -563,7 +563,7 @@ def _gemm_small_into(A, B, out, bias, residual, epilogue) -> bool:
     tile = small_tile(M, N, K) if M and N else -1
     ldr = residual.stride(0) if residual is not None else 0
     if tile < 0 and native().ring_wins(M, N, K, int(epilogue == EPI_GELU), int(residual is not None)):
-        tile = 3
+        tile = native().RING_TILE
     if (tile < 0 or not native().gemm_small_ok(M, N, K, A.stride(0), B.stride(0), out.stride(0), ldr)
             or (ptr(A) | ptr(B)) % 16 or (ptr(out) | ptr(bias) | ptr(residual)) % 8):
         return False
