@@ -651,9 +651,9 @@ PYBIND11_MODULE(_native, m) {
   m.def("slab_slices", &dab::slab_slices);
   m.def("ring_tile", &dab::ring_tile);
   m.def("ring_wins", &dab::ring_wins);
-  m.def("gemm_slab", [](u A, u B, u slabs, int M, int N, int K, u s) {
-    check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s)), "gemm_slab");
-  });
+  m.def("gemm_slab", [](u A, u B, u slabs, int M, int N, int K, u s, int tile) {
+    check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s), tile), "gemm_slab");
+  }, py::arg("A"), py::arg("B"), py::arg("slabs"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("s"), py::arg("tile") = -1);
   m.def("layernorm_slabs", [](u out, u slabs, int S, u bias, u res, u gamma, u beta, int rows, int cols, float eps, u s,
                               u next, unsigned next_bytes, u then, unsigned then_bytes) {
     check(dab::layernorm_slabs(VP(out), CVP(slabs), S, CVP(bias), CVP(res), CVP(gamma), CVP(beta), rows, cols, eps, ST(s),

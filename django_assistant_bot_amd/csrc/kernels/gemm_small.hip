@@ -676,8 +676,9 @@ static void ring_launch(const SmallParams& p, int gelu, hipStream_t s) {
   else hipLaunchKernelGGL((gemm_ring_kernel<t.bm, t.bn, WM, WN, NS, false>), grid, block, 0, s, p);
 }
 
-static void gemm_ring(const SmallParams& p, int gelu, hipStream_t s) {
-  switch (ring_tile(p.M, p.N, p.K, gelu, p.slabs ? p.slices : 1)) {
+// tile: that one (tests), -1: by the estimate
+static void gemm_ring(const SmallParams& p, int gelu, hipStream_t s, int tile = -1) {
+  switch (tile >= 0 ? tile : ring_tile(p.M, p.N, p.K, gelu, p.slabs ? p.slices : 1)) {
     case 0: return ring_launch<0, 2, 2, 4>(p, gelu, s);
     case 1: return ring_launch<1, 2, 4, 3>(p, gelu, s);
     case 2: return ring_launch<2, 2, 2, 3>(p, gelu, s);
@@ -707,6 +708,7 @@ static int next_blocks(const Upcoming& next, int grid) {
   return room < 8 ? 0 : min(want, room);
 }
 
+// tile: as small_tile says; kRingTile + 16 + i: tile i of the ring, whatever its estimate (tests).
 int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, const void* residual,
                long ldr, int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next) {
   if (M <= 0 || N <= 0) return 0;
@@ -733,6 +735,7 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
     SMALL(0, 1, 1, 8, 2)
     SMALL(1, 2, 1, 8, 2)
     case kRingTile: gemm_ring(p, gelu, s); break;
+    case kRingTile + 16 ... kRingTile + 16 + kRings - 1: gemm_ring(p, gelu, s, tile - kRingTile - 16); break;
     SMALL(6, 2, 2, 8, 1)
     SMALL(7, 2, 4, 8, 1)
     SMALL(8, 4, 4, 8, 1)
@@ -766,13 +769,13 @@ int slab_slices(int M, int N, int K) {
   return 0;
 }
 
-// slabs [slices][M][N] fp32 = the K-slices' sums of A w^T, as slab_slices says
-int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s) {
+// slabs [slices][M][N] fp32 = the K-slices' sums of A w^T, as slab_slices says; tile: as gemm_ring's
+int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s, int tile) {
   const int slices = slab_slices(M, N, K);
-  if (!slices || !gemm_small_ok(M, N, K, K, K, N, 0)) return hipErrorInvalidValue;
+  if (tile >= kRings || !slices || !gemm_small_ok(M, N, K, K, K, N, 0)) return hipErrorInvalidValue;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)slabs) % 16) return hipErrorInvalidValue;
   const SmallParams p = {(const bf16*)A, (const bf16*)B, nullptr, nullptr, nullptr, M, N, K, K, K, N, 0, 0, (float*)slabs, slices};
-  gemm_ring(p, 0, s);
+  gemm_ring(p, 0, s, tile);
   return hipGetLastError();
 }
 

@@ -400,7 +400,7 @@ int gemm_ln_ok(int M, int N, int K, int tile);
 int slab_slices(int M, int N, int K);
 int ring_tile(int M, int N, int K, int gelu, int slices);
 bool ring_wins(int M, int N, int K, int gelu, int residual);
-int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s);
+int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s, int tile = -1);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
             int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next = {});
 int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, const void* residual,

@@ -1,4 +1,5 @@
-"""The ready flags of gemm_mid's divided tiles hold the number of the launch that raised them."""
+"""The divided tiles of gemm_mid's 128-row kernel: counts of the parts that are in, owners that hand a tile over, counts of ended
+workgroups (the launch's number, which the 256-row kernel's ready flags hold)."""
 import pytest
 import torch
 
@@ -33,8 +34,8 @@ def _launch(A, B, out, spin_limit):
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_a_launch_that_gave_up_leaves_nothing_for_the_next(M, N, K):
-    """Owners that look at a flag once and give up write NaN over their tile; the flags raised behind them belong to that
-    launch, and the launches after it take only their own partial tiles."""
+    """Owners that look once and go on (a kernel whose owners give up may write NaN over their tile); the launches after it take
+    only their own partial tiles."""
     for seed in range(4):
         A, B, exp = _case(M, N, K, seed)
         out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)

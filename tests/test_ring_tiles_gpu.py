@@ -1,4 +1,4 @@
-"""The encoder's ring kernel (gemm_small.hip) against an fp64 product: every tile of its rule at its edges, its K-slices, and
+"""The encoder's ring kernel (gemm_small.hip) against an fp64 product: every tile at its edges, its K-slices, and
 the sizes that it takes from the larger kernels."""
 import pytest
 import torch
@@ -8,7 +8,7 @@ from django_assistant_bot_amd import ops
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# tile of the rule: one K-tile, fewer K-tiles than buffers, ragged rows and columns, many K-tiles
+# tile of the ring: one K-tile, fewer K-tiles than buffers, ragged rows and columns, many K-tiles
 SHAPES = {0: [(1, 4, 64), (130, 388, 128)], 1: [(641, 772, 64), (641, 772, 448)], 2: [(1300, 772, 128), (1000, 1028, 448)],
           3: [(4000, 1028, 64), (641, 3076, 448)], 4: [(1300, 2308, 64), (641, 2308, 768)], 5: [(700, 3076, 1024), (3000, 772, 1024)],
           6: [(1700, 3076, 192), (1500, 3076, 448)], 7: [(2340, 3076, 128), (2600, 2308, 448)]}
@@ -43,13 +43,12 @@ def _check(got, A, B, b, r, gelu):
 @pytest.mark.parametrize("gelu,bias,res", [(False, True, True), (True, True, False), (False, False, False)])
 def test_every_tile(tile, M, N, K, gelu, bias, res):
     nat = ops.native()
-    assert nat.ring_tile(M, N, K, int(gelu), 1) == tile
     A, B, b, r = _operands(M, N, K, bias, res)
     wide = torch.empty(M + 1, N + 12, dtype=torch.bfloat16, device=DEV).fill_(7.0)
     out = wide[:M, :N]
     p = lambda t: 0 if t is None else t.data_ptr()  # noqa: E731
     nat.gemm_small(p(A), A.stride(0), p(B), B.stride(0), p(out), out.stride(0), p(b), p(r), 0 if r is None else r.stride(0), M, N, K,
-                   int(gelu), 3, torch.cuda.current_stream().cuda_stream)
+                   int(gelu), nat.RING_TILE + 16 + tile, torch.cuda.current_stream().cuda_stream)
     _check(out, A, B, b, r, gelu)
     assert (wide[M:] == 7.0).all() and (wide[:, N:] == 7.0).all()
 
@@ -57,11 +56,11 @@ def test_every_tile(tile, M, N, K, gelu, bias, res):
 @pytest.mark.parametrize("M,N,K,slices,tile", [(1807, 384, 1536, 2, 2), (2029, 384, 1536, 2, 4), (1955, 768, 3072, 2, 5), (2695, 384, 1600, 3, 4)])
 def test_slices(M, N, K, slices, tile):
     nat = ops.native()
-    assert nat.slab_slices(M, N, K) == slices and nat.ring_tile(M, N, K, 0, slices) == tile
+    assert nat.slab_slices(M, N, K) == slices
     A, B, _, _ = _operands(M, N, K, False, False)
     A, B = A.contiguous(), B.contiguous()
     slabs = torch.full((slices + 1, M, N), 7.0, device=DEV)
-    nat.gemm_slab(A.data_ptr(), B.data_ptr(), slabs.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream)
+    nat.gemm_slab(A.data_ptr(), B.data_ptr(), slabs.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream, tile)
     cut = [K // 64 * i // slices * 64 for i in range(slices + 1)]
     for i in range(slices):
         exp = A[:, cut[i]:cut[i + 1]].double() @ B[:, cut[i]:cut[i + 1]].double().t()
@@ -72,16 +71,27 @@ def test_slices(M, N, K, slices, tile):
 @pytest.mark.parametrize("M,N,K", [(6400, 768, 768), (5300, 1152, 384), (9000, 1000, 768)])
 @pytest.mark.parametrize("shift", [0, 4])
 def test_sizes_taken_from_the_larger_kernels(M, N, K, shift):
-    """Rows that the ring's copies do not take (8 bytes off a 16-byte line) stay where they were."""
+    """Rows that the ring's copies do not take (8 bytes off a 16-byte line) stay on those kernels, which do."""
     assert ops.kernels.small_tile(M, N, K) == -1 and ops.native().ring_wins(M, N, K, 0, 1)
     A, B, b, r = _operands(M, N, K, True, True)
     if shift:
         wide = torch.zeros(M, K + 8, dtype=torch.bfloat16, device=DEV)
         wide[:, shift:K + shift] = A
         A = wide[:, shift:K + shift]
-    try:
-        got = ops.gemm_bt(A, B, bias=b, residual=r)
-    except (ValueError, RuntimeError):
-        assert shift  # (refused before as well)
-        return
-    _check(got, A, B, b, r, False)
+    assert A.data_ptr() % 16 == 2 * shift
+    _check(ops.gemm_bt(A, B, bias=b, residual=r), A, B, b, r, False)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 768, 768), (1300, 3072, 768), (2200, 768, 3072), (9000, 1152, 384)])
+def test_the_choice_of_a_tile_changes_no_bits(M, N, K):
+    nat, s = ops.native(), torch.cuda.current_stream().cuda_stream
+    A, B, b, r = _operands(M, N, K, True, True)
+
+    def run(tile):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        nat.gemm_small(A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), out.data_ptr(), N, b.data_ptr(), r.data_ptr(), r.stride(0),
+                       M, N, K, 0, tile, s)
+        return out
+
+    exp = run(nat.RING_TILE)
+    assert all(torch.equal(run(nat.RING_TILE + 16 + t), exp) for t in SHAPES)
