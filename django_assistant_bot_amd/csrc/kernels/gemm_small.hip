@@ -646,22 +646,24 @@ int ring_tile(int M, int N, int K, int gelu, int slices) {
 }
 
 // Whether the ring beats gemm256 (row-major weights), or the 128 x 128 kernel where that does not take the shape, at a size
-// that small_tile leaves to them.  Against gemm256 by 12 % of its estimate, waves of 256 tiles of 256 x 256, each with its epilogue.
-// Against the 128 x 128 kernel by its estimate (rounds of two tiles a CU, the result's way to memory; half of them within 3 %) and
-// the ring's with a residual's reads in it.  Over 1,113 sizes (24 pairs of N and K, M 400-30,000) 8 % faster than without the ring, over 716
-// others (22 pairs, M 600-30,000) 10 %; 8 of them by more than 2 % slower in their sweep, 0.91 at worst, and none of the three that
-// are in both sweeps slower in both.  us, before -> ring: (6400, 768, 768) 24.3 -> 17.2, (5300, 1152, 384) 15.8 -> 11.2, (17500, 1000, 768)
-// 61 -> 45.  Left where they were, us there / on the ring: (3200, 3072, 768) 26.1 / 28.4, (4600, 2304, 768) 21.9 / 32, (17500, 384,
-// 1536) 34.3 / 37.3, (11000, 640, 1280) 31.0 / 32.4; wrongly (25000, 640, 1280) 84 / 64.
+// that small_tile leaves to them: by a tenth of the estimate of gemm256, waves of 256 tiles of 256 x 256, each with its
+// epilogue, and by 1.44 times that.  Where the 128 x 128 kernel has no more than the two tiles a CU that run side by side, its
+// own estimate decides, too (the product and the result's way to memory, half of them within 3 %; the ring's with a residual's
+// reads in it).  (By that estimate alone, whatever the tiles, also qkv of MiniLM from 9,100 tokens on: a call of 21,000 tokens
+// 1,291 -> 1,227 us, but of 11,900 830 -> 839.)  Over 1,113 sizes (24 pairs of N and K, M 400-30,000) 8 % faster than without
+// the ring, over 716 others (22 pairs, M 600-30,000) 10 %; 8 of them are more than 2 % slower in their sweep, and in both only
+// (8000, 1024, 256) 11.9 -> 12.4 and (30000, 256, 256) 11.8 -> 12.2  us, before -> ring: (6400, 768, 768) 24.3 -> 17.2, (5300,
+// 1152, 384) 15.8 -> 11.2, (17500, 1000, 768) 61 -> 45.  Left where they were, us there / on the ring: (3200, 3072, 768) 26.1 /
+// 28.4, (4600, 2304, 768) 21.9 / 32, (17500, 384, 1536) 34.3 / 37.3, (11000, 640, 1280) 31.0 / 32.4.
 bool ring_wins(int M, int N, int K, int gelu, int residual) {
   if (M <= 0 || N <= 0 || K < 64) return false;
+  const bool large = gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K);
   const float ring = ring_us(kRing[ring_tile(M, N, K, gelu, 1)], M, N, K, gelu);
-  if (gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K)) {
-    const long waves = ((long)((M + 255) / 256) * ((N + 255) / 256) + 255) / 256;
-    return ring < 0.88f * (2.1f + waves * (0.0146f * K + 7.f + (gelu ? 5.7f : 0.f) + (residual ? 3.9f : 0.f)));
-  }
-  const long c = ((long)((M + 127) / 128) * ((N + 127) / 128) + 255) / 256, rounds = (c + 1) / 2;  // tiles on the busiest CU
-  const float mn = 1e-6f * M * N, other = 5.3f + 1.4f * (rounds - 1) + rounds * 0.0151f * K + 0.81f * mn + c * (gelu ? 1.26f : residual ? 2.1f : 0.f);
+  const long waves = ((long)((M + 255) / 256) * ((N + 255) / 256) + 255) / 256;
+  if (ring >= (large ? 0.9f : 1.44f) * (2.1f + waves * (0.0146f * K + 7.f + (gelu ? 5.7f : 0.f) + (residual ? 3.9f : 0.f)))) return false;
+  const long c = ((long)((M + 127) / 128) * ((N + 127) / 128) + 255) / 256;  // tiles of 128 x 128 on the busiest CU
+  if (large || c > 2) return true;
+  const float mn = 1e-6f * M * N, other = 5.3f + 0.0151f * K + 0.81f * mn + c * (gelu ? 1.26f : residual ? 2.1f : 0.f);
   return 1.18f * ring + 1.7f + (residual ? -0.12f : -0.53f) * mn < 0.97f * other;
 }
 

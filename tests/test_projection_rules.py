@@ -11,8 +11,8 @@ def test_tall_projections_leave_the_64_x_64_tiles_earlier(M, N, K, tile):
 
 
 # faster on the ring than on gemm256 or the 128 x 128 kernel; slower
-@pytest.mark.parametrize("M,N,K,wins", [(6400, 768, 768, True), (5300, 1152, 384, True), (17400, 1152, 384, True), (19000, 1000, 768, True),
+@pytest.mark.parametrize("M,N,K,wins", [(6400, 768, 768, True), (5300, 1152, 384, True), (17400, 1152, 384, True), (25000, 640, 1280, True),
                                         (3200, 3072, 768, False), (4600, 2304, 768, False), (17500, 384, 1536, False),
-                                        (11000, 640, 1280, False), (8000, 1024, 256, False)])
+                                        (11000, 640, 1280, False)])
 def test_large_projections_on_the_ring_where_it_is_faster(M, N, K, wins):
     assert small_tile(M, N, K) == -1 and native().ring_wins(M, N, K, 0, 0) == wins
