@@ -1,8 +1,11 @@
 // Mid-M bf16 GEMM  C[M,N] = A[M,K] . B[N,K]^T  (+ residual, or fused SwiGLU over 8-row [gate | up]
-// groups) for M = 256..4096 rows: the token counts of mixed prefill + decode serving steps and of
+// groups) for up to 4096 rows: the token counts of mixed prefill + decode serving steps and of
 // request-at-a-time prompts (the reference runs one HF ``generate`` per request:
 // ai/providers/transformers.py:57-66, served by gunicorn_conf.py:9 workers).  B is in the
 // ops.shuffle_weights fragment layout (the one copy of every projection the decoder keeps).
+//
+// Two kernels: gemm_mid_kernel with tiles of 128 x 256, described here, and gemm_wide_kernel with tiles of 256 x 256 for
+// longer prompts (what differs stands there; which of them a product takes: mid_pick).
 //
 // Why a third GEMM: at these M the 256x256 phased kernel (gemm256.hip) has 12-64 tiles for 256 CUs
 // and the 128x128 kernel (gemm.hip) runs at ~20 % of the MFMA rate (profiles/gemm_mid_r5.md).
@@ -495,7 +498,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
   count_out();
 }
 
-// Tiles of 256 x 256 with the same split of the iteration space (in pairs of K-steps), partial tiles and flags.  What bounds
+// Tiles of 256 x 256 with the same split of the iteration space (in pairs of K-steps), partial tiles and owners, which wait for a
+// flag of each part (they hand nothing over: the workgroups they wait for have been placed before them).  What bounds
 // the kernel above is the way of its loads into a CU: 48 KB a K-step (64 B a cycle at best, 43 measured from L2) against 1024
 // cycles of MFMAs; with both operands' addresses held still its K-step takes as long, and weights straight into registers
 // instead of LDS gain nothing.  A tile of 256 rows loads 32 KB for the same MFMAs.  Loop, staging and LDS layout are those of
@@ -697,7 +701,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
     }
     if (wr == 0) mbar();  // pairs with group 1's last K-loop barrier
 
-    // ---- end of a part: as in the kernel above
+    // ---- end of a part: stored with a flag behind it, or the owner adds what the others stored
     const int n0 = (nt0 + nt) * 256;
     bool write = true;
     if (k0 != 0 || k1 != kt) {
@@ -873,8 +877,9 @@ int gemm_mid_ok(int M, int N, int K, long lda) {
 
 // Estimated us of a product on `groups` groups.  Its K-steps take 0.7 each, from some 120 working workgroups on 0.5 +
 // 0.00165 a workgroup, or the weights' way from memory (4.5 TB/s), whichever is longer; its ends 5.6 for whole tiles, 8.1
-// and 1.56 a part where every tile is cut into parts of as many K-steps, 10.5 and 1.56 a part otherwise, and 2.5 for each further tile of a group.  (Fitted to 1,480
-// launches of 1-32 row tiles, N 256-28,672, K 256-14,336: half of them within 5 %, nine of ten within 16 %.)
+// and 1.56 a part where every tile is cut into parts of as many K-steps, 10.5 and 1.56 a part otherwise, and 2.5 for each
+// further tile of a group.  (Fitted to 1,480 launches of 1-32 row tiles, N 256-28,672, K 256-14,336: half of them within 5
+// %, nine of ten within 16 %.)
 static double mid_us(int M, int N, int K, int groups) {
   const int tm = (M + 127) / 128, tn = N / 256, kt = K / 64;
   const double iters = (double)tn * kt, q = iters / groups;
@@ -1009,14 +1014,13 @@ int gemm_mid_counters(int M, int N) {
   return 2 * (cu_count() & ~7);
 }
 
-// epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over
-// 8-row [gate | up] groups (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs:
-// gemm_mid_slab_bytes() bytes, the last 1024 zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the
-// launch leaves them zero).  spin_limit: looks at a count before an owner hands its tile over (256 rows: at a flag, before it gives up
-// and writes NaN), -1: the kernel's own.  variant (A/B harness only): 0 default
-// (by the estimates), 32 / 64 the 128-row kernel with that K-step, 256 the 256-row kernel, + 1000 = DIAG 1 (split tiles not combined: timing only).
-// BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank
-// conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
+// epilogue 0: C = A B^T (+ residual, bf16 add after rounding); 4 / 6: SwiGLU / tanh-GELU GLU over 8-row [gate | up] groups
+// (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes() bytes, the last 1024
+// zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).  spin_limit: looks
+// at a count before an owner hands its tile over (256 rows: at a flag, before it gives up and writes NaN), -1: the kernel's
+// own.  variant (A/B harness only): 0 default (by the estimates), 32 / 64 the 128-row kernel with that K-step, 256 the
+// 256-row kernel, + 1000 = DIAG 1 (split tiles not combined: timing only). BK 32 (6-stage ring) measured 5-20 % slower than
+// BK 64 on every mid shape, with LDS bank conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
 int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const void* residual, long ldr, int M, int N,
              int K, int epilogue, void* slabs, long slab_bytes, int* cnt, int n_cnt, hipStream_t s, int variant,
              int b_group, long spin_limit) {

@@ -749,17 +749,22 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
 }
 
 // K-slices that a long-K projection in front of a LayerNorm (which sums them: layernorm_slabs) is cut into, 0: none.  The
-// widths are those of layernorm_slab_kernel's instances.  Its tiles alone leave CUs idle or one workgroup each, whose share of
-// the operands from past L2 is what takes the time; in slices they are up to two workgroups of 64 x 64 a CU (one and a half
-// where K is above 2048), or one of 128 x 128 (ring_tile then takes the tile of the slices).  Between those, below 139 tiles of 64 x 64 and
-// with a short K the slabs (8 bytes an element and slice there and back) cost more than that.  us of product and LayerNorm,
-// one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 -> 15.9, (2200, 384, 1536) 14.2
-// -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200, 768, 3072) 29.4 -> 26.2, (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5 -> 13.9,
-// (1500, 384, 1536) 12.0 -> 12.3 in three slices of 512, (4600, 768, 3072) 41.8 -> 48.3, (832, 768, 768) 9.5 -> 10.3.
-// Whole calls of the encoder, weights of three copies in turn: bge-base 800 tokens 703 -> 676, 900 735 -> 708, 1400 964 -> 922,
-// 1650 1091 -> 1021, 2500 1293 -> 1207; MiniLM 1850 275 -> 269, 2650 330 -> 321, 3200 391 -> 368, 5000 493 -> 469; not taken bge-base
-// in two slices of 1536, 1000 765 -> 776, 1150 818 -> 832, 1300 847 -> 861 (with the weights on the die 773 -> 751 at 1180), 1300
-// in three of 128 x 128 847 -> 869; bge-large 765 in two of 2048 1757 -> 1788.
+// widths are those of layernorm_slab_kernel's instances.  Its tiles alone leave CUs idle or one workgroup each, whose share
+// of the operands from past L2 is what takes the time; in slices they fill the chip.  The slabs cost 8 bytes an element and
+// slice there and back, which a short K or few rows do not pay for.
+//
+// The bands were measured when a slice ran on tiles of 64 x 64 (up to 256 of them) or 128 x 128 (from 64 of them on) alone
+// and are counted in those; the launch takes the tile that ring_tile estimates for the slices.  With these eight tiles the
+// bands are a little wrong on both sides: (560, 1024, 4096) in three slices 16.2 -> 17.0 us against the 64 x 64 tile, and by
+// ring_us two slices would be the quicker for bge-base at 961-1,300 tokens and bge-large at 641-1,024, which run whole.  us
+// of product and LayerNorm, one launch -> slices: (rows, H, K) (832, 768, 3072) 16.9 -> 14.8, (600, 1024, 4096) 19.0 ->
+// 15.9, (2200, 384, 1536) 14.2 -> 13.2; with 128 x 128 (1500, 768, 3072) 22.7 -> 21.2, (2200, 768, 3072) 29.4 -> 26.2,
+// (1100, 1024, 4096) 27.0 -> 25.1, (3200, 384, 1536) 19.8 -> 16.9; not taken (600, 768, 3072) 13.5 -> 13.9, (1500, 384,
+// 1536) 12.0 -> 12.3 in three slices of 512, (4600, 768, 3072) 41.8 -> 48.3, (832, 768, 768) 9.5 -> 10.3.  Whole calls of
+// the encoder, weights of three copies in turn: bge-base 800 tokens 703 -> 676, 900 735 -> 708, 1400 964 -> 922, 1650 1091
+// -> 1021, 2500 1293 -> 1207; MiniLM 1850 275 -> 269, 2650 330 -> 321, 3200 391 -> 368, 5000 493 -> 469; not taken bge-base
+// in two slices of 1536, 1000 765 -> 776, 1150 818 -> 832, 1300 847 -> 861 (with the weights on the die 773 -> 751 at 1180),
+// 1300 in three of 128 x 128 847 -> 869; bge-large 765 in two of 2048 1757 -> 1788.
 int slab_slices(int M, int N, int K) {
   if (M <= 0 || K < 1536 || K % 64 || (N != 384 && N != 768 && N != 1024)) return 0;
   const long t64 = ((M + 63) / 64) * (long)(N / 64), t128 = ((M + 127) / 128) * (long)(N / 128);

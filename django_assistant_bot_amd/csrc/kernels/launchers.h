@@ -314,8 +314,8 @@ int norm_stream_ok(int M, int N, int K, int SO, int bn);
 int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, const void* gain, void* residual_out, float eps,
                 const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn,
                 hipStream_t s);
-// gemm_mid.hip (M = 256..4096: mixed serving steps / single prompts; grouped stream-K over the N x K
-// plane, 128 x 256 tiles, in-launch combine by the owner; B in the shuffle_weights layout;
+// gemm_mid.hip (M up to 4096: mixed serving steps / single prompts; grouped stream-K over the N x K
+// plane, 128 x 256 or 256 x 256 tiles, in-launch combine; B in the shuffle_weights layout;
 // epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
 int gemm_mid_groups(int M, int N, int K);
 int gemm_mid_wide_groups(int M, int N, int K, int forced);

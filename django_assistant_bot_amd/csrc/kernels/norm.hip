@@ -594,8 +594,8 @@ int rmsnorm_slabs(void* out, void* res_out, const void* slabs, int S, long slab_
 }
 
 // Workgroups of 256 behind a LayerNorm's that read the next projection's weights (and those of the one behind it: encoder.hip), 8
-// loads of the former a thread.  us a forward, weights of
-// three copies in turn, without -> with 16 / 8 / 4 loads: bge-base 120 tokens 430 -> 431 / 422 / 423, 240 502 -> 495 / 486 / 486, 816
+// loads of the former a thread.  LayerNorms of 768 and 1,024 columns and those of K-slices have them; other widths (384: MiniLM's norms
+// without slices) run without, whatever `next` says.  us a forward, weights of three copies in turn, without -> with 16 / 8 / 4 loads: bge-base 120 tokens 430 -> 431 / 422 / 423, 240 502 -> 495 / 486 / 486, 816
 // 663 -> 640 / 632 / 634, 1500 854 -> 830 / 824 / 831, 3000 1,227 -> 1,208 / 1,207 / 1,212, 6000 2,008 -> 2,004 / 2,002 / 1,995;
 // bge-large 180 1,108 -> 1,066 / 1,050 / 1,054, 600 1,460 -> 1,421 / 1,432 / 1,434, 1200 2,002 -> 1,959 / 1,957 / 1,969, but 1800 2,245 ->
 // 2,277 / 2,253 / 2,261: more rows need the weights less, and larger ones take longer than the norm.

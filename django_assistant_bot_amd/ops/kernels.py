@@ -699,10 +699,10 @@ def gemm_mid_ok(M: int, N: int, K: int, lda: int) -> bool:
 
 def gemm_mid(A, B, residual=None, epilogue=EPI_NONE, out=None, variant: int = 0, b_group: int = 1, glu_bias=None):
     """C = A . B^T (+ residual) or SwiGLU over 8-row [gate | up] groups, B a ``shuffle_weights`` copy:
-    the mid-M kernel (``gemm_mid.hip``: grouped stream-K, 128 x 256 tiles, in-launch owner combine) for
-    M = 256..4096 (mixed serving steps, single prompts).  Bit-reproducible: the split-K partials are
-    summed in a fixed order.  ``variant`` (A/B harness): 32 / 64 force the K-step; + 1000 leaves
-    split tiles uncombined (timing only)."""
+    the mid-M kernels (``gemm_mid.hip``: grouped stream-K, 128 x 256 tiles or, by estimates, 256 x 256, in-launch combine)
+    for M up to 4096 (mixed serving steps, single prompts).  Bit-reproducible: the split-K partials are
+    summed in a fixed order.  ``variant`` (tests, A/B harness): 32 / 64 the 128-row kernel with that K-step, 256 the 256-row
+    one; + 1000 leaves split tiles uncombined (timing only)."""
     M, K = A.shape
     N = B.shape[0]
     expect(A.is_cuda and A.dtype == torch.bfloat16 and B.dtype == torch.bfloat16, "bf16 CUDA operands required")

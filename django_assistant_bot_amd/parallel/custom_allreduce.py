@@ -42,8 +42,8 @@ def blocks_for(devices: list, most: int) -> int:
     while the last one's next kernel still has to be placed, and a workgroup of gemm256 takes a CU's whole register file
     (8 waves of 256 registers): at 8 ranks and 64 workgroups, 448 spinning ones could hold all of the 256 CUs and the rank
     they wait for never ran.  So the others' workgroups together stay within 7/8 of the CUs, and an eighth of the device is
-    free for the rank behind (of gemm_mid, whose workgroups wait for each other, the kernel of 128 rows fits beside a spinning
-    one, and that of 256 rows ends however few of its workgroups are resident).  8 ranks on 256 CUs: 32 workgroups; up to 4,
+    free for the rank behind (gemm_mid's kernel of 128 rows fits beside a spinning one, and both of its kernels end however few
+    of their workgroups are resident).  8 ranks on 256 CUs: 32 workgroups; up to 4,
     or one rank a device: all 64."""
     blocks = most
     for key, cus in devices:
