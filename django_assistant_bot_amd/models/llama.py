@@ -252,7 +252,7 @@ class LlamaModel(FragmentProjections):
                     and self.tp_size == 1)
         sk = (meta.decode and T <= self.STREAM_MAX_M or small_pf) and x.is_cuda
         if sk and not meta.decode and T > 128:
-            sk = self.SLABS_F32
+            sk = False if self._frag_serves(T) else self.SLABS_F32
         if sk and meta.decode and T <= self.SMALL_FUSED_MAX_M and self.small_norm_fused and self.fold_norms and self.tp_size == 1:
             h = x  # the residual stream itself: no RMSNorm launches (``_layer_small``)
             for li, L in enumerate(self.layers):
@@ -339,6 +339,18 @@ class LlamaModel(FragmentProjections):
             x = ops.slab_reduce(x)
         return self._all_reduce(x)
 
+    def _frag_serves(self, T: int) -> bool:
+        """Whether qkv, o and down of a step of ``T`` tokens are of the sizes that ``gemm_frag`` was measured at: past 128 tokens
+        its tiles beat the streamed projections (us a layer of qkv, o and down with their norms at T 200: Llama-3-8B 91 -> 75, 1B
+        43 -> 38)."""
+        L = self.layers[0]
+        return all(ops.native().frag_us(T, w.shape[0], w.shape[1], 1) < float("inf") for w in (L.qkv_w, L.o_w, L.down_w))
+
+    def _slab_proj(self, x, w, name: str):
+        """fp32 slabs of a prefill projection where summing them in the norm behind it is the quicker, else None."""
+        s = ops.frag_slices(x.shape[0], w.shape[0], w.shape[1]) if self.frag and w.shape[0] % 256 == 0 else 0
+        return ops.gemm_frag(x, w, slices=s, b_group=self.proj_group.get(name, 1)) if s else None
+
     def _layer(self, li: int, L: DecoderLayer, x, residual, meta: AttnMeta, kv: KVCache, sk: bool):
         """One decoder layer: (layer input, residual stream) -> (next layer input, residual stream)."""
         cfg, D, T = self.cfg, self.cfg.head_dim, meta.positions.numel()  # x may be [S, T, H] split-K slabs
@@ -393,9 +405,13 @@ class LlamaModel(FragmentProjections):
         epi = ops.EPI_SWIGLU8 if (self.interleaved_mlp and a.is_cuda) else ops.EPI_NONE
         both = None
         if fuse:
-            residual = ops.gemm_bt(a.view(T, self.hq * D), L.o_w, residual=residual, shuffled=self.frag,
-                                   b_group=self.proj_group.get("o", 1))
-            h, _ = ops.rmsnorm(residual, L.mlp_norm, cfg.eps)
+            a = a.view(T, self.hq * D)
+            o = self._slab_proj(a, L.o_w, "o")
+            if o is None:
+                residual = ops.gemm_bt(a, L.o_w, residual=residual, shuffled=self.frag, b_group=self.proj_group.get("o", 1))
+                h, _ = ops.rmsnorm(residual, L.mlp_norm, cfg.eps)
+            else:
+                h, residual = ops.rmsnorm(o, L.mlp_norm, cfg.eps, residual=residual)
         elif sk and self.tp_size > 1:
             # TP decode: the o partial (split-K slabs) meets its all-reduce inside the MLP norm's launch
             o = self._tp_partial(self._proj(a.view(T, self.hq * D), L.o_w, sk, True, name="o"), cfg.hidden)
@@ -413,8 +429,10 @@ class LlamaModel(FragmentProjections):
             if h.is_cuda and epi == ops.EPI_NONE:
                 act = ops.silu_mul(act)
         if fuse:
-            return None, ops.gemm_bt(act, L.down_w, residual=residual, shuffled=self.frag,
-                                     b_group=self.proj_group.get("down", 1))
+            x = self._slab_proj(act, L.down_w, "down")
+            if x is not None:  # summed by the norm in front of the next layer (or the final one)
+                return x, residual
+            return None, ops.gemm_bt(act, L.down_w, residual=residual, shuffled=self.frag, b_group=self.proj_group.get("down", 1))
         if sk and self.tp_size > 1:  # reduced inside the next layer's (or the final) norm launch
             return self._tp_partial(self._proj(act, L.down_w, sk, True, name="down"), cfg.hidden), residual
         x = self._all_reduce(self._proj(act, L.down_w, sk, slabs_ok, name="down"))

@@ -489,9 +489,38 @@ def _mid_us(M: int, tiles_n: int, K: int) -> float:
 
 
 @functools.lru_cache(maxsize=4096)
-def frag_plan(M: int, N: int, K: int, cols: bool = True):
+def _frag_plan(M: int, N: int, K: int, cols: bool, frag: bool):
+    """``frag_plan`` and the estimate of its time."""
+    tm, tn = -(-M // 256), N // 256
+    one = {"256": _g256_us(tm * tn, K), "mid": _mid_us(M, tn, K)}
+    if use_gemm_mid(M, N, K, K):
+        best = "mid"
+    elif use_gemm256(M, N, K, K, K):
+        best = "256"
+    else:
+        return None, float("inf")
+    other = "256" if best == "mid" else "mid"
+    if one[other] < 0.985 * one[best]:
+        best = other
+    plan, took, least = ((best, M, N), None), one[best], 0.95 * one[best]
+    for waves in range(1, tm * tn // 256 + 1):
+        n1, m1 = waves * 256 // tm, waves * 256 // tn
+        if cols and 0 < n1 < tn:
+            us = _g256_us(tm * n1, K) + _mid_us(M, tn - n1, K)
+            if us < least:
+                plan, took, least = (("256", M, 256 * n1), ("mid", M, N - 256 * n1)), us, us
+        if 0 < m1 < tm:
+            us = _g256_us(m1 * tn, K) + _mid_us(M - 256 * m1, tn, K)
+            if us < least:
+                plan, took, least = (("256", 256 * m1, N), ("mid", M - 256 * m1, N)), us, us
+    us = native().frag_us(M, N, K, 1) if frag else float("inf")
+    return ((("frag", M, N), None), us) if us < 0.93 * took else (plan, took)
+
+
+def frag_plan(M: int, N: int, K: int, cols: bool = True, frag: bool = True):
     """How a projection with fragment-layout weights that both gemm256 and gemm_mid take is run: (first kernel, its
-    rows, its columns) and the same of what remains (or None).  ``cols``: its columns may be divided.
+    rows, its columns) and the same of what remains (or None).  ``cols``: its columns may be divided; ``frag``: gemm_frag takes
+    its operands.
 
     gemm256 alone pays a whole wave of 256 tiles for the last few (Llama-3-8B gate_up at M = 1093: 560 tiles, 235 us
     where two waves take 157), gemm_mid runs at about half its rate but divides evenly.  So the whole waves go to
@@ -504,30 +533,60 @@ def frag_plan(M: int, N: int, K: int, cols: bool = True):
     Outside that range the estimates only have to order the two kernels: over 24 shapes with N and K of 256..28,672 and M 1
     ..16,000 the plan differs from the old bounds 196 times and is 0.97..2.05 times as fast, median 1.53: few tiles of a
     short K are the quicker on gemm256 ((44, 512, 4096) 114 -> 62 us, (256, 4096, 512) 22.9 -> 14.6); the worst are (257,
-    8192, 1024) 21.3 -> 22.0 and (1093, 4096, 1024) 22.4 -> 23.1."""
-    tm, tn = -(-M // 256), N // 256
-    one = {"256": _g256_us(tm * tn, K), "mid": _mid_us(M, tn, K)}
-    if use_gemm_mid(M, N, K, K):
-        best = "mid"
-    elif use_gemm256(M, N, K, K, K):
-        best = "256"
-    else:
-        return None
-    other = "256" if best == "mid" else "mid"
-    if one[other] < 0.985 * one[best]:
-        best = other
-    plan, least = ((best, M, N), None), 0.95 * one[best]
-    for waves in range(1, tm * tn // 256 + 1):
-        n1, m1 = waves * 256 // tm, waves * 256 // tn
-        if cols and 0 < n1 < tn:
-            us = _g256_us(tm * n1, K) + _mid_us(M, tn - n1, K)
-            if us < least:
-                plan, least = (("256", M, 256 * n1), ("mid", M, N - 256 * n1)), us
-        if 0 < m1 < tm:
-            us = _g256_us(m1 * tn, K) + _mid_us(M - 256 * m1, tn, K)
-            if us < least:
-                plan, least = (("256", 256 * m1, N), ("mid", M - 256 * m1, N)), us
-    return plan
+    8192, 1024) 21.3 -> 22.0 and (1093, 4096, 1024) 22.4 -> 23.1.
+
+    gemm_frag, whole, where its estimate is 7 % below: over M 96..2300 at 19 pairs of N 1024..28,672 and K 1024..14,336 that
+    is 236 of 414 sizes, 1.64 times as fast in the mean, none slower (at 4 % below two of 271 are 7-9 % slower)."""
+    return _frag_plan(M, N, K, cols, frag)[0]
+
+
+@functools.lru_cache(maxsize=4096)
+def frag_slices(M: int, N: int, K: int) -> int:
+    """K-slices that ``gemm_frag`` leaves as fp32 slabs to the norm behind a projection with a residual, 0: the whole product
+    is the quicker.  The norm reads them at some 4.5 TB/s.  us of product and norm, whole on the quickest kernel -> in slices:
+    (260, 2048, 8192) 33.5 -> 23.8, (515, 2048, 8192) 39.8 -> 35.6, (140, 4096, 14336) 57 -> 39.7, (260, 4096, 14336) 62.6 ->
+    55.4; (1093, 2048, 8192) 57.4 -> 53.1."""
+    whole = _frag_plan(M, N, K, True, True)[1]
+    best, least = 0, 0.95 * whole
+    for s in (2, 3, 4, 6, 8):
+        us = native().frag_us(M, N, K, s) + 0.7 + 4 * s * M * N / 4.5e6 if K // 64 >= 4 * s else float("inf")
+        if us < least:
+            best, least = s, us
+    return best
+
+
+def gemm_frag(A, B, residual=None, epilogue=EPI_NONE, out=None, b_group: int = 1, glu_bias=None, slices: int = 0, tile: int = -1):
+    """C = A . B^T (+ residual) or a GLU over 8-row [gate | up] groups, B a ``shuffle_weights`` copy, on tiles of 32 x 64 to 128 x
+    256 (``gemm_frag.hip``).  ``slices`` S > 0: the K-slices' sums as fp32 slabs [S, M, N] for ``rmsnorm``.  ``tile`` (tests): that
+    one instead of the one with the least estimate."""
+    M, K = A.shape
+    N = B.shape[0]
+    expect(A.is_cuda and A.dtype == torch.bfloat16 and B.dtype == torch.bfloat16, "bf16 CUDA operands required")
+    expect(A.stride(-1) == 1 and B.is_contiguous() and B.shape[1] == K, "A K-contiguous, B a contiguous [N, K] copy")
+    expect(native().gemm_frag_ok(M, N, K, A.stride(0)), "gemm_frag: N % 32, K % 64, 16-B rows")
+    expect(epilogue in (EPI_NONE, *GLU8) and b_group in (1, 8), "gemm_frag epilogues: none (+residual) or an 8-row-group GLU")
+    n_out = N // 2 if epilogue in GLU8 else N
+    if residual is not None:
+        expect(epilogue == EPI_NONE and not slices and residual.dtype == torch.bfloat16 and residual.stride(-1) == 1
+               and tuple(residual.shape) == (M, N), "residual must be bf16 [M, N]")
+    _glu_bias(glu_bias, epilogue, N)
+    if slices:
+        expect(out is None and epilogue == EPI_NONE and 0 < slices <= K // 64, "slabs: a plain product, K-slices of whole K-tiles")
+        slabs = torch.empty((slices, M, N), dtype=torch.float32, device=A.device)
+    elif out is None:
+        out = torch.empty((M, n_out), dtype=torch.bfloat16, device=A.device)
+    expect(out is None or (out.dtype == torch.bfloat16 and out.stride(-1) == 1 and tuple(out.shape) == (M, n_out)), "bad output")
+    native().gemm_frag(ptr(A), A.stride(0), ptr(B), ptr(out), out.stride(0) if out is not None else 0, ptr(residual),
+                       residual.stride(0) if residual is not None else 0, ptr(glu_bias), ptr(slabs) if slices else 0, int(slices),
+                       M, N, K, int(epilogue), int(b_group), int(tile), stream(A))
+    return slabs if slices else out
+
+
+def _frag_takes(A, B, out, residual, glu_bias) -> bool:
+    """Whether ``gemm_frag`` takes a projection's operands (the kernels beside it take any alignment)."""
+    return (native().gemm_frag_ok(A.shape[0], B.shape[0], A.shape[1], A.stride(0)) and out.stride(0) % 8 == 0
+            and (residual is None or residual.stride(0) % 8 == 0)
+            and (ptr(A) | ptr(B) | ptr(out) | ptr(residual) | ptr(glu_bias)) % 16 == 0)
 
 
 def _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias):
@@ -542,7 +601,9 @@ def _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias):
         a, b = A[m:m + rows], B[n:n + cols]
         o = out[m:m + rows, n // per:(n + cols) // per]
         r = None if residual is None else residual[m:m + rows, n:n + cols]
-        if kind == "mid":
+        if kind == "frag":
+            gemm_frag(a, b, residual=r, epilogue=epilogue, out=o, b_group=b_group, glu_bias=glu_bias)
+        elif kind == "mid":
             gemm_mid(a, b, residual=r, epilogue=epilogue, out=o, b_group=b_group, glu_bias=glu_bias)
         else:
             _gemm256_into(a, b, o, glu_bias, r, epilogue, True, b_group)
@@ -629,8 +690,9 @@ def gemm_bt(A, B, bias=None, residual=None, epilogue=EPI_NONE, out_f32=False, ro
     plain = not out_f32 and row_group is None and q_group is None and allow is None
     if plain and shuffled and N == B.shape[0] and bias is None and epilogue in (EPI_NONE, *GLU8) and N % 256 == 0:
         lda = A.stride(0)
-        plan = frag_plan(M, N, K, glu_bias is None) if M >= GEMM_MID_MIN_M and native().gemm256_ok(M, N, K, lda, K) else None
-        if plan is not None and all(q is None or q[0] == "256" or gemm_mid_ok(q[1], q[2], K, lda) for q in plan):
+        plan = (frag_plan(M, N, K, glu_bias is None, _frag_takes(A, B, out, residual, glu_bias))
+                if M >= GEMM_MID_MIN_M and native().gemm256_ok(M, N, K, lda, K) else None)
+        if plan is not None and all(q is None or q[0] != "mid" or gemm_mid_ok(q[1], q[2], K, lda) for q in plan):
             return _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias)
         if use_gemm_mid(M, N, K, A.stride(0)):
             return gemm_mid(A, B, residual=residual, epilogue=epilogue, out=out, b_group=b_group, glu_bias=glu_bias)

@@ -1,0 +1,27 @@
+"""Which prefill projections gemm_frag takes, and in how many K-slices."""
+import pytest
+
+from django_assistant_bot_amd.ops.kernels import frag_plan, frag_slices, native
+
+
+# faster there by measurement; slower, or outside what was measured (rows, N, K)
+@pytest.mark.parametrize("M,N,K,takes", [(260, 2048, 2048, True), (515, 3072, 2048, True), (260, 6144, 4096, True), (1093, 2048, 2048, True),
+                                         (140, 28672, 4096, True), (1093, 28672, 4096, False), (1093, 4096, 14336, False),
+                                         (700, 10240, 8192, False), (2300, 4096, 4096, False), (64, 2048, 2048, False),
+                                         (300, 768, 2048, False), (300, 2048, 512, False), (5000, 2048, 2048, False)])
+def test_plan(M, N, K, takes):
+    assert (frag_plan(M, N, K)[0][0] == "frag") == takes
+    assert frag_plan(M, N, K, True, False)[0][0] != "frag"
+
+
+def test_slices():
+    assert frag_slices(260, 2048, 8192) > 1 and frag_slices(140, 4096, 14336) > 1
+    assert frag_slices(1093, 4096, 14336) == frag_slices(400, 2048, 2048) == frag_slices(3000, 4096, 4096) == 0
+    for M, N, K in ((140, 1024, 1024), (260, 2048, 8192), (515, 2048, 8192), (260, 4096, 14336)):
+        s = frag_slices(M, N, K)
+        assert s == 0 or K // 64 >= 4 * s
+
+
+@pytest.mark.parametrize("slices", [0, 17])
+def test_estimate_of_no_product(slices):
+    assert native().frag_us(300, 2048, 1024, slices) == float("inf")
