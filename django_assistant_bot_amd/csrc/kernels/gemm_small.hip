@@ -24,6 +24,8 @@
 //   1700, 768, 768    8.7 -> 8.0           1700, 2304, 768  14.3 -> 11.8          1700, 3072, 768  25.5 (gemm256) -> 16.7
 //   2900, 768, 768   12.7 -> 11.1          2900, 768, 3072 (128 x 128, with the norm behind it) 40.3 -> 30.0
 // Epilogues round as gemm.hip does.
+#include <type_traits>
+
 #include "common.h"
 #include "launchers.h"
 
@@ -486,8 +488,10 @@ __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAtte
 // BM x BN tiles by WM x WN waves over a ring of NS K-tiles (64 wide) in LDS, filled by LDS-DMA NS - 1 tiles ahead with
 // counted waits: one barrier a K-tile and no drained queue.  LDS rows of 128 B, 16-B chunk c of row r at
 // c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly); a copy is 8 rows, and copy q of a
-// K-tile's A and B rows, one behind the other, is wave q mod the waves'.  Bias and residual are asked for at the start: at
-// the end they were one more round trip (0.2-0.7 us).
+// K-tile's A and B rows, one behind the other, is wave q mod the waves'.  The copies go out one at a time between the products:
+// all in front of the fragment reads, they hold the waves up until the last is accepted, which is as long as the products take
+// (24 texts of 8-64 tokens 616 -> 581 us, 10 of 200 876 -> 841; fragments read a K-tile ahead besides: the same).  Bias and
+// residual are asked for at the start: at the end they were one more round trip (0.2-0.7 us).
 constexpr int ring_occupancy(int rows, int waves, int ns) {  // waves a SIMD that the ring leaves room for
   const int n = 163840 / (rows * 128 * ns) * waves / 4;
   return n < 1 ? 1 : n > 8 ? 8 : n;
@@ -515,17 +519,16 @@ __global__ __launch_bounds__(64 * WM * WN, ring_occupancy(BM + BN, WM * WN, NS))
     const int r = 8 * (i * W + w) + (lane >> 3), c = 8 * ((lane & 7) ^ ((r >> 1) & 7));
     at[i] = (unsigned)((r < BM ? min(m0 + r, p.M - 1) * p.lda + c : min(n0 + r - BM, p.N - 1) * p.ldb + c) * 2);
   }
+  auto copy = [&](int i, char* dst, unsigned so) __attribute__((always_inline)) {
+    // (which operand: known here but for the copies of a step that holds rows of both)
+    if (8 * (i * W + W) <= BM || (8 * i * W < BM && 8 * (i * W + w) < BM))
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
+  };
   auto stage = [&](int buf, int kt) {
-    char* dst = smem + buf * kStage + w * 1024;
-    const unsigned so = (unsigned)kt * 128u;
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) {
-      // (which operand: known here but for the copies of a step that holds rows of both)
-      if (8 * (i * W + W) <= BM || (8 * i * W < BM && 8 * (i * W + w) < BM))
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
-      else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (small_lds*)(dst + i * W * 1024), 16, (unsigned)at[i], so, 0, 0);
-    }
+    for (int i = 0; i < kDma; ++i) copy(i, smem + buf * kStage + w * 1024, (unsigned)kt * 128u);
   };
   const int k0 = SLAB ? p.K / 64 * slice / p.slices : 0, nk = (SLAB ? p.K / 64 * (slice + 1) / p.slices : p.K / 64) - k0;
 #pragma unroll
@@ -555,15 +558,17 @@ __global__ __launch_bounds__(64 * WM * WN, ring_occupancy(BM + BN, WM * WN, NS))
 #pragma unroll
     for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   int buf = 0;
-  for (int t = 0; t < nk; ++t) {
-    const int ahead = min(NS - 2, nk - 1 - t);  // K-tiles after t that may stay in flight
+  auto step = [&](int t, auto more) __attribute__((always_inline)) {
+    constexpr bool kMore = decltype(more)::value;  // a K-tile is left to be copied
+    const int ahead = kMore ? NS - 2 : min(NS - 2, nk - 1 - t);  // K-tiles after t that may stay in flight
     if (ahead >= 2) small_wait<2 * kDma>();
     else if (ahead == 1) small_wait<kDma>();
     else small_wait<0>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last K-tile's reads: its buffer is filled next
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + NS - 1 < nk) stage(buf == 0 ? NS - 1 : buf - 1, k0 + t + NS - 1);
+    char* const dst = smem + (buf == 0 ? NS - 1 : buf - 1) * kStage + w * 1024;
+    const unsigned so = (unsigned)(k0 + t + NS - 1) * 128u;
     const char* sa = smem + buf * kStage + wm * (BM / WM) * 128;
     const char* sb = smem + buf * kStage + kA + wn * (BN / WN) * 128;
     bf16x8 af[MI][2], bfr[NI][2];
@@ -575,15 +580,27 @@ __global__ __launch_bounds__(64 * WM * WN, ring_occupancy(BM + BN, WM * WN, NS))
       for (int i = 0; i < NI; ++i) bfr[i][ks] = *reinterpret_cast<const bf16x8*>(sb + i * 2048 + rd[ks]);
     }
     __builtin_amdgcn_s_setprio(1);
+    constexpr int kMul = 2 * NI * MI;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+    for (int x = 0; x < kMul; ++x) {
+      if constexpr (kMore) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < MI; ++j) acc[i][j] = mfma16(bfr[i][ks], af[j][ks], acc[i][j]);
+        for (int c = 0; c < kDma; ++c)
+          if (c * kMul / kDma == x) {
+            __builtin_amdgcn_sched_barrier(0);
+            copy(c, dst, so);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      const int ks = x / (NI * MI), i = x / MI % NI, j = x % MI;
+      acc[i][j] = mfma16(bfr[i][ks], af[j][ks], acc[i][j]);
+    }
     __builtin_amdgcn_s_setprio(0);
     buf = buf == NS - 1 ? 0 : buf + 1;
-  }
+  };
+  int t = 0;
+  for (; t + NS - 1 < nk; ++t) step(t, std::true_type());
+  for (; t < nk; ++t) step(t, std::false_type());
   // acc[i][j][r] = C[m0 + wm BM / WM + 16 j + li][n0 + wn BN / WN + 16 i + 4 g + r]
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
