@@ -691,6 +691,7 @@ PYBIND11_MODULE(_native, m) {
   });
   m.def("gemm_mid_groups", &dab::gemm_mid_groups);
   m.def("gemm_mid_wide_groups", &dab::gemm_mid_wide_groups);
+  m.def("gemm_mid_192_us", &dab::gemm_mid_192_us);
   m.def("gemm_mid_us", &dab::gemm_mid_us);
   m.def("gemm256_wins", &dab::gemm256_wins);
   m.attr("GEMM256_FILL") = dab::kGemm256Fill;

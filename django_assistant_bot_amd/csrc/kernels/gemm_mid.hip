@@ -4,8 +4,8 @@
 // ai/providers/transformers.py:57-66, served by gunicorn_conf.py:9 workers).  B is in the
 // ops.shuffle_weights fragment layout (the one copy of every projection the decoder keeps).
 //
-// Two kernels: gemm_mid_kernel with tiles of 128 x 256, described here, and gemm_wide_kernel with tiles of 256 x 256 for
-// longer prompts (what differs stands there; which of them a product takes: mid_pick).
+// Two kernels: gemm_mid_kernel with tiles of 128 x 256, described here, and gemm_wide_kernel with tiles of 256 or 192 x 256 for
+// longer prompts (what differs stands there; which of them a product takes: mid_pick, and the caller for 192 rows).
 //
 // Why a third GEMM: at these M the 256x256 phased kernel (gemm256.hip) has 12-64 tiles for 256 CUs
 // and the 128x128 kernel (gemm.hip) runs at ~20 % of the MFMA rate (profiles/gemm_mid_r5.md).
@@ -506,14 +506,21 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GMid p) {
 // gemm256: two buffers of K-steps, a phase of two quadrants of 128 x 128, pieces of 16 KB restaged one phase after their last
 // read and waited for three phases later.
 namespace {
-constexpr int kWBuf = 65536, kWHalf = 16384;  // a K-step: A0 | A1 | B0 | B1, 128 rows of 128 B each
-constexpr int kWE = 16, kWSlabSt = 32;        // VMEM stores per wave of an epilogue and of a published partial tile
-constexpr int kWSlabFloats = 256 * 256;       // one a workgroup: only the first part of its range can be another's tile
+constexpr int kWHalf = 16384;                // a K-step: A0 | A1 | B0 | B1, 128 rows of 128 B each (A1: the tile's rows past 128)
+constexpr int kWSlabFloats = 256 * 256;      // one a workgroup: only the first part of its range can be another's tile
 static_assert(kWSlabFloats == 2 * kSlabFloats, "the partial tiles of both kernels take the same workspace");
 }  // namespace
 
-template <int EPI, bool RES>
+// ROWS 256, or 192 (the second half of A is 64 rows, its phases of half the products) where that leaves fewer rows past the
+// prompt's end: a pair of K-steps 1.45-2.2 us against 1.83-2.7, partial tiles of 192 KB.  us of a call of Llama-3-8B without -> with
+// it: 560 tokens 10,220 -> 9,789, 1,093 15,949 -> 15,754, 1,300 18,085 -> 17,349; Llama-3.2-1B, 1,300 3,709 -> 3,483.
+template <int EPI, bool RES, int ROWS>
 __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
+  static_assert(ROWS == 256 || ROWS == 192, "a second half of 128 or 64 rows");
+  constexpr int H2 = ROWS - 128, I2 = H2 / 32;               // rows of the second half, 16-row blocks of a wave in it
+  constexpr int kWBuf = 3 * kWHalf + H2 * 128;
+  constexpr int NE = 16 + 4 * I2, kWSlabSt = NE, kWE = NE / 2;  // accumulators; VMEM stores per wave of a published partial tile, of an epilogue
+  constexpr int kFly = 6 + H2 / 64;                          // copies that a phase's wait leaves in flight
   // behind the buffers: the count the launch's number comes from, and whether an owner's waits ended well
   __shared__ __attribute__((aligned(16))) char smem[2 * kWBuf + 256];
 
@@ -538,7 +545,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = w >> 2, wc = w & 3;
   const int li = lane & 15, gq = lane >> 4;
-  const int m0 = mt * 256;
+  const int m0 = mt * ROWS;
   const int kt = p.kt;  // pairs of K-steps per tile
 
   // ---- LDS-DMA staging, as the kernel above: piece = 128 rows of A (16-B chunk c of row r at c ^ ((r >> 1) & 7), swizzled
@@ -549,17 +556,17 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   const bool bgrp = p.bgrp == 8;
   const unsigned cb = bgrp ? 8192u : 1024u;
   const unsigned vB0 = (unsigned)(lane * 16) + (unsigned)w * (bgrp ? 1024u : kblk);
-  const long a_rows = min(256, p.M - m0);
+  const long a_rows = min(ROWS, p.M - m0);
   const __amdgpu_buffer_rsrc_t rA = mk_rsrc(p.A + (size_t)m0 * p.lda, (unsigned)(((a_rows - 1) * p.lda + p.K) * 2));
   const __amdgpu_buffer_rsrc_t rB = mk_rsrc(p.B, p.b_bytes);
   auto stage_a = [&](int buf, int half, int ks) {
     char* dst = smem + buf * kWBuf + half * kWHalf + w * 1024;
     const unsigned v0 = vA0 + (half ? 2u * rowsA : 0u), v1 = v0 + rowsA, so = (unsigned)ks * 128u;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)dst, 16, v0, so, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)(dst + 8192), 16, v1, so, 0, 0);
+    if (half == 0 || H2 == 128) __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)(dst + 8192), 16, v1, so, 0, 0);
   };
   auto stage_b = [&](int buf, int half, int nt, int ks) {
-    char* dst = smem + buf * kWBuf + (2 + half) * kWHalf + w * 2048;
+    char* dst = smem + buf * kWBuf + (1 + half) * kWHalf + H2 * 128 + w * 2048;
     const unsigned v0 = vB0 + (half ? 8u * kblk : 0u), v1 = v0 + cb, so = (unsigned)(nt0 + nt) * 16u * kblk + (unsigned)ks * 2u * cb;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)dst, 16, v0, so, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void*)(dst + 1024), 16, v1, so, 0, 0);
@@ -572,19 +579,22 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   for (int buf = 0; buf < 2; ++buf) {
     rdA[buf][0] = buf * kWBuf + (64 * wr + li) * 128 + 16 * (gq ^ (li >> 1));
     rdA[buf][1] = buf * kWBuf + (64 * wr + li) * 128 + 16 * ((4 + gq) ^ (li >> 1));
-    rdB[buf] = buf * kWBuf + 2 * kWHalf + wc * 4096 + lane * 16;
+    rdB[buf] = buf * kWBuf + kWHalf + H2 * 128 + wc * 4096 + lane * 16;
     asm volatile("" : "+v"(rdA[buf][0]), "+v"(rdA[buf][1]), "+v"(rdB[buf]));
   }
+  const int second = kWHalf - (64 - H2 / 2) * 128 * wr;  // from a wave's rows in the first half to those in the second
   bf16x8 af[4][2], bfr[2][2][2];
-  f32x4 acc[2][2][4][2];
+  f32x4 acc[2][2][4][2];  // (192 rows: [1][..] of two row blocks)
+#define WIDE_ACC(E) \
+  acc[(E) >> 4][(E) < 16 ? ((E) >> 3) & 1 : ((E)-16) / (2 * I2)][(E) < 16 ? ((E) >> 1) & 3 : ((E)-16) / 2 % I2][(E)&1]
   auto zero_acc = [&]() {
 #pragma unroll
-    for (int e = 0; e < 32; ++e) acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < NE; ++e) WIDE_ACC(e) = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   zero_acc();
 #define WIDE_READ_A(BUF, IH)                                                                  \
-  _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                             \
-    const char* base = smem + (IH) * kWHalf + i * 2048;                                       \
+  _Pragma("unroll") for (int i = 0; i < ((IH) ? I2 : 4); ++i) {                               \
+    const char* base = smem + ((IH) ? second : 0) + i * 2048;                                 \
     af[i][0] = *reinterpret_cast<const bf16x8*>(base + rdA[BUF][0]);                          \
     af[i][1] = *reinterpret_cast<const bf16x8*>(base + rdA[BUF][1]);                          \
   }
@@ -599,7 +609,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   __builtin_amdgcn_s_setprio(1);                                                              \
   _Pragma("unroll") for (int jj = 0; jj < 2; ++jj)                                            \
   _Pragma("unroll") for (int ks = 0; ks < 2; ++ks)                                            \
-  _Pragma("unroll") for (int i = 0; i < 4; ++i)                                               \
+  _Pragma("unroll") for (int i = 0; i < ((IH) ? I2 : 4); ++i)                                 \
   _Pragma("unroll") for (int jn = 0; jn < 2; ++jn)                                            \
     acc[IH][JH1 ^ jj][i][jn] = mfma16(bfr[JH1 ^ jj][jn][ks], af[i][ks], acc[IH][JH1 ^ jj][i][jn]); \
   __builtin_amdgcn_s_setprio(0);
@@ -622,7 +632,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
   stage_a(1, 0, 2 * k0 + 1);
   stage_b(1, 0, nt, 2 * k0 + 1);
   stage_b(1, 1, nt, 2 * k0 + 1);
-  wait_vmc<8>();
+  wait_vmc<kFly>();
   mbar();
   unsigned before;
   asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
@@ -654,9 +664,9 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
       WIDE_READ_A(0, 0)
       WIDE_READ_B(0)
       stage_a(1, 1, ks);
-      if (after_st == kWSlabSt) wait_vmc<8 + kWSlabSt>();
-      else if (after_st == kWE) wait_vmc<8 + kWE>();
-      else wait_vmc<8>();
+      if (after_st == kWSlabSt) wait_vmc<kFly + kWSlabSt>();
+      else if (after_st == kWE) wait_vmc<kFly + kWE>();
+      else wait_vmc<kFly>();
       mread_bar();
       WIDE_MFMA(0, 0)
       mbar();
@@ -666,9 +676,9 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
         stage_a(0, 0, kn);
         stage_b(0, 0, nn, kn);
         stage_b(0, 1, nn, kn);
-        if (after_st == kWSlabSt) wait_vmc<8 + kWSlabSt>();
-        else if (after_st == kWE) wait_vmc<8 + kWE>();
-        else wait_vmc<8>();
+        if (after_st == kWSlabSt) wait_vmc<kFly + kWSlabSt>();
+        else if (after_st == kWE) wait_vmc<kFly + kWE>();
+        else wait_vmc<kFly>();
       } else {
         wait_vmc<0>();
       }
@@ -681,7 +691,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
       WIDE_READ_B(1)
       if (st) {
         stage_a(0, 1, kn);
-        wait_vmc<8>();
+        wait_vmc<kFly>();
       }
       mread_bar();
       WIDE_MFMA(0, 0)
@@ -693,7 +703,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
         stage_a(1, 0, kn + 1);
         stage_b(1, 0, nn, kn + 1);
         stage_b(1, 1, nn, kn + 1);
-        wait_vmc<8>();
+        wait_vmc<kFly>();
       }
       mread_bar();
       WIDE_MFMA(1, 1)
@@ -709,9 +719,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
       if (j != j_lo) {
         const unsigned own = slab_off(j);
 #pragma unroll
-        for (int e = 0; e < 32; ++e)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1]), rS, own,
-                                                 (unsigned)(e * 8192), 16);
+        for (int e = 0; e < NE; ++e)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, WIDE_ACC(e)), rS, own, (unsigned)(e * 8192), 16);
         after_st = kWSlabSt;
         pending = true;
         if (!more) {  // nothing left to hide the drain behind
@@ -737,13 +746,13 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
           }
           mbar();  // every thread loads only after lane 0 saw the flag
           const unsigned off = slab_off(jj);
-          u32x4 v[16];  // a window: half of the partial tile
+          u32x4 v[NE / 2];  // a window: half of the partial tile
 #pragma unroll
-          for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)(e * 8192), 16);
+          for (int e = 0; e < NE / 2; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)(e * 8192), 16);
 #pragma unroll
-          for (int e = 0; e < 32; ++e) {
-            acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] += __builtin_bit_cast(f32x4, v[e & 15]);
-            if (e < 16) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)((16 + e) * 8192), 16);
+          for (int e = 0; e < NE; ++e) {
+            WIDE_ACC(e) += __builtin_bit_cast(f32x4, v[e % (NE / 2)]);
+            if (e < NE / 2) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rS, off, (unsigned)((NE / 2 + e) * 8192), 16);
           }
         }
         // Lane 0 tells the others, by asm statements on the one LDS array: __syncthreads_and brings an object of its own, and
@@ -756,17 +765,17 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
         if (!__builtin_amdgcn_readfirstlane(all)) {
           const float nan = __builtin_nanf("");
 #pragma unroll
-          for (int e = 0; e < 32; ++e) acc[e >> 4][(e >> 3) & 1][(e >> 1) & 3][e & 1] = f32x4{nan, nan, nan, nan};
+          for (int e = 0; e < NE; ++e) WIDE_ACC(e) = f32x4{nan, nan, nan, nan};
         }
       }
     }
     if (write) {
-      // ---- epilogue: acc[ih][jh][i][jn][r] = C[m0 + 128 ih + 64 wr + 16 i + li][n0 + 128 jh + 32 wc + 16 jn + 4 gq + r];
+      // ---- epilogue: acc[ih][jh][i][jn][r] = C[m0 + 128 ih + (64 or H2 / 2) wr + 16 i + li][n0 + 128 jh + 32 wc + 16 jn + 4 gq + r];
       // exactly kWE stores per wave (rows >= M fall outside the descriptor and are dropped)
       int e_lane = tid & 63;  // (opaque, so that nothing derived from it stays live across the K-loop)
       asm volatile("" : "+v"(e_lane));
       const int e_li = e_lane & 15, e_g = e_lane >> 4;
-      const long c_rows = min(256, p.M - m0);
+      const long c_rows = min(ROWS, p.M - m0);
       const __amdgpu_buffer_rsrc_t rC = mk_rsrc(p.C + (size_t)m0 * p.ldc, (unsigned)(c_rows * p.ldc * 2));
       if constexpr (glu8_epilogue(EPI)) {
         f32x4 bg[2], bu[2];
@@ -783,10 +792,10 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
 #pragma unroll
         for (int ih = 0; ih < 2; ++ih)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < (ih ? I2 : 4); ++i)
 #pragma unroll
             for (int jh = 0; jh < 2; ++jh) {
-              const int mr = 128 * ih + 64 * wr + 16 * i + e_li;
+              const int mr = 128 * ih + (ih ? H2 / 2 : 64) * wr + 16 * i + e_li;
               float o[4];
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
@@ -810,17 +819,17 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
           u32x4 rv[4][2];
           if constexpr (RES) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < (ih ? I2 : 4); ++i)
 #pragma unroll
               for (int jh = 0; jh < 2; ++jh)
                 rv[i][jh] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rR, (unsigned)(((128 * ih + 64 * wr + 16 * i + e_li) * p.ldr + n0 + 128 * jh + 32 * wc + cq) * 2), 0, 0);
+                    rR, (unsigned)(((128 * ih + (ih ? H2 / 2 : 64) * wr + 16 * i + e_li) * p.ldr + n0 + 128 * jh + 32 * wc + cq) * 2), 0, 0);
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < (ih ? I2 : 4); ++i)
 #pragma unroll
             for (int jh = 0; jh < 2; ++jh) {
-              const int mr = 128 * ih + 64 * wr + 16 * i + e_li;
+              const int mr = 128 * ih + (ih ? H2 / 2 : 64) * wr + 16 * i + e_li;
               float o[8];
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
@@ -851,6 +860,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GMid p) {
     k0 = 0;
     ++nt;
   }
+#undef WIDE_ACC
 #undef WIDE_READ_A
 #undef WIDE_READ_B
 #undef WIDE_MFMA
@@ -926,37 +936,45 @@ int gemm_mid_groups(int M, int N, int K) {
   return groups;
 }
 
-// Estimated us of a product on `groups` groups of the 256-row kernel (all XCDs').  A pair of K-steps takes 1.83 us, from some
-// 70 working workgroups on 1.64 + 0.0027 a workgroup and 0.0048 more for each past 192, or the weights' way from memory; the
-// ends 10.4 for whole tiles and, with partial tiles of 256 KB, 0.027 a workgroup and 2.48 a part besides.  (Fitted to 12,900
-// launches of M 128-4096 at 11 sizes of N 2048-28,672, K 1024-14,336: half of them within 2.7 %, nine of ten within 7.5 %;
-// the groups taken by it cost 0.9 % more than the best in the mean.)
-static double wide_us(int M, int N, int K, int groups) {
-  const int tm = (M + 255) / 256, tn = N / 256, kt = K / 128;
+// Estimated us of a product on `groups` groups of the kernel with tiles of 256 or 192 rows (all XCDs').  A pair of K-steps takes
+// 1.83 us, from some 70 working workgroups on 1.64 + 0.0027 a workgroup and 0.0048 more for each past 192, or the weights' way
+// from memory; the ends 10.4 for whole tiles and, with partial tiles of 256 KB, 0.027 a workgroup and 2.48 a part besides.
+// (256 rows: fitted to 12,900 launches of M 128-4096 at 11 sizes of N 2048-28,672, K 1024-14,336: half of them within 2.7 %,
+// nine of ten within 7.5 %; the groups taken by it cost 0.9 % more than the best in the mean.  192 rows: to 520 launches of M
+// 400-3700 at nine of those sizes, on another card: 3.2 and 8.2 %, the groups 0.6 %.)
+struct WideTime {
+  double step, base, per, over, whole, equal, uneven, part, wgs, further;
+};
+constexpr WideTime kWide256 = {1.83, 1.64, 0.0027, 0.0048, 10.4, 11.4, 12.5, 2.48, 0.027, 7.0};
+constexpr WideTime kWide192 = {1.445, 1.586, 0.0022, 0.0041, 7.2, 6.4, 5.9, 2.16, 0.039, 5.2};
+
+static double wide_us(int M, int N, int K, int groups, int rows) {
+  const WideTime& f = rows == 192 ? kWide192 : kWide256;
+  const int tm = (M + rows - 1) / rows, tn = N / 256, kt = K / 128;
   const double iters = (double)tn * kt, q = iters / groups, wgs = (groups < iters ? groups : iters) * tm;
-  const double step = fmax(1.83, 1.64 + 0.0027 * wgs) + 0.0048 * fmax(0., wgs - 192.);
+  const double step = fmax(f.step, f.base + f.per * wgs) + f.over * fmax(0., wgs - 192.);
   const double weights = (double)tn * 512 * K / 5.0e6;
-  double ends = 10.4, steps = q * step;
+  double ends = f.whole, steps = q * step;
   if (tn % groups) {
     const bool equal = groups % tn == 0 && kt % (groups / tn) == 0;
     const double parts = equal ? (double)(groups / tn) : groups > tn ? ceil(kt / fmax(q, 1.)) : 1.;
-    ends = (equal ? 11.4 : 12.5) + 2.48 * parts + 0.027 * wgs;
+    ends = (equal ? f.equal : f.uneven) + f.part * parts + f.wgs * wgs;
     if (!equal) steps = ceil(q) * step;
   }
-  if (tn > groups) ends += 7.0 * ((double)tn / groups - 1.);
+  if (tn > groups) ends += f.further * ((double)tn / groups - 1.);
   return ends + fmax(steps, weights);
 }
 
-// Groups of the 256-row kernel and the estimate of its time on them; 0 groups where it is not measured (K below 1024) or
+// Groups of that kernel and the estimate of its time on them; 0 groups where it is not measured (K below 1024) or
 // does not take the sizes (each XCD as many column tiles).  From three row tiles on: with fewer, weights that take longer from
 // memory than the products are slower ((391, 10240, 8192) 0.81 times as fast), and others gain nothing over gemm256.
-static int wide_groups(int M, int N, int K, int min_tm, double* us) {
-  const int spx = cu_count() / 8, tm = (M + 255) / 256, tn = N / 256;
+static int wide_groups(int M, int N, int K, int min_tm, int rows, double* us) {
+  const int spx = cu_count() / 8, tm = (M + rows - 1) / rows, tn = N / 256;
   *us = __builtin_huge_val();
   if (M <= 0 || tn <= 0 || K < 1024 || K % 128 || tn % 8 || tm < min_tm || tm > spx) return 0;
   int groups = 0;
   for (int gn = 8; gn <= 8 * (spx / tm); gn += 8) {
-    const double t = wide_us(M, N, K, gn);
+    const double t = wide_us(M, N, K, gn, rows);
     if (t < *us) {
       *us = t;
       groups = gn;
@@ -979,7 +997,7 @@ static int mid_pick(int M, int N, int K, bool* wide, double* us) {
   const int groups = gemm_mid_groups(M, N, K);
   *us = groups ? mid_us(M, N, K, groups) : __builtin_huge_val();
   double w_us;
-  const int w_groups = groups ? wide_groups(M, N, K, 3, &w_us) : 0;
+  const int w_groups = groups ? wide_groups(M, N, K, 3, 256, &w_us) : 0;
   *wide = w_groups && w_us < 0.87 * *us;
   if (!*wide) return groups;
   *us = 1.1 * w_us;  // (beside gemm256: the step of Llama-3-8B at 3,000 tokens 34,732 us with it, 35,015 on this)
@@ -990,7 +1008,7 @@ static int mid_pick(int M, int N, int K, bool* wide, double* us) {
 int gemm_mid_wide_groups(int M, int N, int K, int forced) {
   bool wide;
   double us;
-  if (forced) return wide_groups(M, N, K, 1, &us);
+  if (forced) return wide_groups(M, N, K, 1, 256, &us);
   const int groups = mid_pick(M, N, K, &wide, &us);
   return wide ? groups : 0;
 }
@@ -1001,6 +1019,13 @@ double gemm_mid_us(int M, int N, int K) {
   double us;
   if (mid_pick(M, N, K, &wide, &us)) return us;
   return M <= 0 || N < 256 ? 0. : __builtin_huge_val();
+}
+
+// ... of the kernel with tiles of 192 rows, which the caller asks for by the variant of that name: in front of the other two
+// where fewer rows of its tiles lie past the prompt's end.
+double gemm_mid_192_us(int M, int N, int K) {
+  double us;
+  return gemm_mid_groups(M, N, K) && wide_groups(M, N, K, 3, 192, &us) ? us : __builtin_huge_val();
 }
 
 // Workspace the launcher needs: partial slabs and behind them the counts of ended workgroups (bytes), and ready flags
@@ -1018,9 +1043,10 @@ int gemm_mid_counters(int M, int N) {
 // (C has N / 2 columns; residual: null, or their fp32 bias [gate | up]).  slabs: gemm_mid_slab_bytes() bytes, the last 1024
 // zero on first use; cnt: >= gemm_mid_counters() ints, zero on first use (the launch leaves them zero).  spin_limit: looks
 // at a count before an owner hands its tile over (256 rows: at a flag, before it gives up and writes NaN), -1: the kernel's
-// own.  variant (A/B harness only): 0 default (by the estimates), 32 / 64 the 128-row kernel with that K-step, 256 the
-// 256-row kernel, + 1000 = DIAG 1 (split tiles not combined: timing only). BK 32 (6-stage ring) measured 5-20 % slower than
-// BK 64 on every mid shape, with LDS bank conflicts on its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
+// own.  variant: 0 default (by the estimates), 192 tiles of 192 rows (as the 128-row kernel where those do not take the sizes);
+// A/B harness only: 32 / 64 the 128-row kernel with that K-step, 256 the 256-row kernel, + 1000 = DIAG 1 (split tiles not
+// combined: timing only). BK 32 (6-stage ring) measured 5-20 % slower than BK 64 on every mid shape, with LDS bank conflicts on
+// its 64-B A rows (profiles/gemm_mid_r6.md): kept as an A/B arm only.
 int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const void* residual, long ldr, int M, int N,
              int K, int epilogue, void* slabs, long slab_bytes, int* cnt, int n_cnt, hipStream_t s, int variant,
              int b_group, long spin_limit) {
@@ -1033,9 +1059,9 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   bool wide;
   double us;
   int groups = mid_pick(M, N, K, &wide, &us);
-  if (variant == 256) {
+  if (variant == 256 || variant == 192) {
     wide = true;
-    groups = wide_groups(M, N, K, 1, &us);
+    groups = wide_groups(M, N, K, 1, variant, &us);
   } else if (variant) {
     wide = false;
   }
@@ -1045,6 +1071,7 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
     if (variant == 256) return hipErrorInvalidValue;
     wide = false;
   }
+  const int rows = !wide ? 128 : variant == 192 ? 192 : 256;
   if (!wide) groups = gemm_mid_groups(M, N, K);
   const bool diag = variant >= 1000;
   const int bk = (variant % 1000) == 32 ? 32 : 64;
@@ -1061,7 +1088,6 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
   p.lda = lda;
   p.ldc = ldc;
   p.ldr = ldr;
-  const int rows = wide ? 256 : 128;
   p.tiles_m = (M + rows - 1) / rows;
   p.tiles_n = N / 256;
   p.kt = K / (wide ? 128 : bk);
@@ -1090,7 +1116,11 @@ int gemm_mid(const void* A, long lda, const void* B, void* C, long ldc, const vo
       MID_LAUNCH(E, R, 32, 0);             \
     }                                      \
   } while (0)
-#define WIDE_LAUNCH(E, R) hipLaunchKernelGGL((gemm_wide_kernel<E, R>), dim3(grid), dim3(512), 0, s, p)
+#define WIDE_LAUNCH(E, R)                                                                            \
+  do {                                                                                               \
+    if (rows == 192) hipLaunchKernelGGL((gemm_wide_kernel<E, R, 192>), dim3(grid), dim3(512), 0, s, p); \
+    else hipLaunchKernelGGL((gemm_wide_kernel<E, R, 256>), dim3(grid), dim3(512), 0, s, p);            \
+  } while (0)
   if (wide) {
     if (epilogue == MID_SWIGLU8 && residual) WIDE_LAUNCH(MID_SWIGLU8, true);
     else if (epilogue == MID_GEGLU8 && residual) WIDE_LAUNCH(MID_GEGLU8, true);

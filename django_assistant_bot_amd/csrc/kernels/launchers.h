@@ -319,6 +319,7 @@ int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, c
 // epilogue 0 none (+ residual) or 4 SwiGLU over 8-row [gate | up] groups)
 int gemm_mid_groups(int M, int N, int K);
 int gemm_mid_wide_groups(int M, int N, int K, int forced);
+double gemm_mid_192_us(int M, int N, int K);
 double gemm_mid_us(int M, int N, int K);
 int gemm_mid_ok(int M, int N, int K, long lda);
 long gemm_mid_slab_bytes();

@@ -25,3 +25,10 @@ def test_slices():
 @pytest.mark.parametrize("slices", [0, 17])
 def test_estimate_of_no_product(slices):
     assert native().frag_us(300, 2048, 1024, slices) == float("inf")
+
+
+# tiles of 192 rows where they leave fewer rows past the prompt's end; else 128 or 256
+@pytest.mark.parametrize("M,N,K,kind", [(768, 4096, 14336, "192"), (1300, 6144, 4096, "192"), (2300, 4096, 4096, "192"), (560, 16384, 2048, "192"),
+                                        (400, 4096, 14336, "mid"), (1900, 4096, 14336, "mid"), (1093, 6144, 4096, "mid"), (700, 2304, 2048, "mid")])
+def test_rows_of_a_tile(M, N, K, kind):
+    assert frag_plan(M, N, K, True, False)[0][0] == kind
