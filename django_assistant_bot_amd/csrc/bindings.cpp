@@ -724,9 +724,13 @@ PYBIND11_MODULE(_native, m) {
   }, py::arg("x"), py::arg("gain"), py::arg("offset"), py::arg("eps"), py::arg("normed"), py::arg("w"), py::arg("b"), py::arg("C"),
      py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("tile"), py::arg("s"), py::arg("next") = 0,
      py::arg("next_bytes") = 0);
-  m.def("unit_rows", [](u x, long ldx, u out, int rows, int cols, u s) {
-    check(dab::unit_rows((const float*)x, ldx, VP(out), rows, cols, ST(s)), "unit_rows");
-  });
+  m.attr("HOST_VALUES") = dab::kHostValues;
+  m.def("unit_rows", [](u x, long ldx, u out, int rows, int cols, u s, u groups, int n_groups, u groups_out, u clear, long words) {
+    check(dab::unit_rows((const float*)x, ldx, VP(out), rows, cols, ST(s), (const int*)groups, n_groups, (int*)groups_out,
+                         (uint32_t*)clear, words),
+          "unit_rows");
+  }, py::arg("x"), py::arg("ldx"), py::arg("out"), py::arg("rows"), py::arg("cols"), py::arg("s"), py::arg("groups") = 0,
+     py::arg("n_groups") = 0, py::arg("groups_out") = 0, py::arg("clear") = 0, py::arg("words") = 0L);
   m.def("rank_value", [](u scores, long ld, int rows, int n, int r, float slack, u thr, u cnt, u s) {
     check(dab::rank_value((const float*)scores, ld, rows, n, r, slack, (float*)thr, (int*)cnt, ST(s)), "rank_value");
   });
@@ -747,11 +751,12 @@ PYBIND11_MODULE(_native, m) {
                           (uint32_t*)mask, words, queries, longest, ST(s)),
           "allow_bits");
   });
-  m.def("doc_lt_bits", [](u docs, u limit, int n, u mask, int words, int queries, int intersect, u s) {
-    check(dab::doc_lt_bits((const int64_t*)docs, (const int64_t*)limit, n, (uint32_t*)mask, words, queries, intersect,
+  m.def("doc_lt_bits", [](u docs, u limit, int n, u mask, int words, int queries, int intersect, u s, int host) {
+    check(dab::doc_lt_bits((const int64_t*)docs, (const int64_t*)limit, n, (uint32_t*)mask, words, queries, intersect, host,
                            ST(s)),
           "doc_lt_bits");
-  });
+  }, py::arg("docs"), py::arg("limit"), py::arg("n"), py::arg("mask"), py::arg("words"), py::arg("queries"), py::arg("intersect"),
+     py::arg("s"), py::arg("host") = 0);
   m.def("gather_rows", [](u src, u rows, u out, int n, int K, u s) {
     check(dab::gather_rows(CVP(src), (const int64_t*)rows, VP(out), n, K, ST(s)), "gather_rows");
   });

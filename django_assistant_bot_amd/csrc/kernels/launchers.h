@@ -416,7 +416,9 @@ int gemm_small(const void* A, long lda, const void* B, long ldb, void* C, long l
 
 // search.hip
 constexpr int kRankMax = 64;  // largest rank rank_value finds
-int unit_rows(const float* x, long ldx, void* out, int rows, int cols, hipStream_t s);
+constexpr int kHostValues = 128;  // groups or document bounds of a search that go into a launch's arguments
+int unit_rows(const float* x, long ldx, void* out, int rows, int cols, hipStream_t s, const int* groups = nullptr, int n_groups = 0,
+              int* groups_out = nullptr, uint32_t* clear = nullptr, long words = 0);
 int rank_value(const float* scores, long ld, int rows, int n, int r, float slack, float* thr, int* cnt, hipStream_t s);
 int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const float* thr, int cap, int rows, int k,
               const int64_t* row_ids, const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs,
@@ -425,7 +427,7 @@ int top_hits(const float* scores, int rows, int n, const void* parts, int ldp, i
              const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs, hipStream_t s);
 int allow_bits(const int64_t* ids, const int64_t* off, const int64_t* keys, const int64_t* rows, int n_keys,
                uint32_t* mask, int words, int queries, int longest, hipStream_t s);
-int doc_lt_bits(const int64_t* docs, const int64_t* limit, int n, uint32_t* mask, int words, int queries, int intersect,
+int doc_lt_bits(const int64_t* docs, const int64_t* limit, int n, uint32_t* mask, int words, int queries, int intersect, int host,
                 hipStream_t s);
 int gather_rows(const void* src, const int64_t* rows, void* out, int n, int K, hipStream_t s);
 int hit_ids(const float* vals, const int* rows, const int64_t* row_ids, const int64_t* row_docs, int64_t* ids,

@@ -205,9 +205,9 @@ class VectorIndex:
         packed = packed - (packed >= (1 << 31)).to(torch.int64) * (1 << 32)
         return packed.to(torch.int32).contiguous()
 
-    def allow_mask(self, allowed) -> torch.Tensor:
+    def allow_mask(self, allowed, mask=None) -> torch.Tensor:
         """Per-query allowed item ids (sets, lists or int arrays) -> int32 bitmask [q, ceil(n/32)] over
-        rows, built on the device (no per-id Python loop)."""
+        rows, built on the device (no per-id Python loop).  ``mask``: one of zeros to set the bits of."""
         words = (self.n + 31) // 32
         lists = [np.fromiter(ids, dtype=np.int64) if isinstance(ids, (set, frozenset)) else
                  np.asarray(ids, dtype=np.int64).reshape(-1) for ids in allowed]
@@ -220,7 +220,7 @@ class VectorIndex:
             np.cumsum(lens, out=flat[1:len(lists) + 1])
             np.concatenate(lists, out=flat[len(lists) + 1:])
             dev = host.to(self.device, non_blocking=True)
-            return ops.allow_bits(dev[len(lists) + 1:], dev[:len(lists) + 1], max(lens), *self._live_ids(), words)
+            return ops.allow_bits(dev[len(lists) + 1:], dev[:len(lists) + 1], max(lens), *self._live_ids(), words, mask)
         m = torch.zeros((len(allowed), words * 32), dtype=torch.bool, device=self.device)
         for qi, ids in enumerate(lists):
             rows = self.rows_of(ids)
@@ -273,10 +273,11 @@ class VectorIndex:
         if mask is not None and mask.shape[0] != len(limits):
             return mask & self.doc_lt_mask(limits)
         words = (self.n + 31) // 32
-        lim = self._there(torch.as_tensor(np.asarray(limits, dtype=np.int64)))
+        lim = torch.as_tensor(np.asarray(limits, dtype=np.int64))
+        lim = lim.contiguous() if self._by_value(lim) else self._there(lim)
         if self.device.type == "cuda" and lim.dim() == 1 and self.n and 0 < len(lim) <= 65535:
             return ops.doc_lt_bits(self.row_docs[: self.n], lim, mask)
-        lim = lim[:, None]
+        lim = lim.to(self.device)[:, None]
         m = torch.zeros((len(limits), words * 32), dtype=torch.bool, device=self.device)
         m[:, : self.n] = self.row_docs[None, : self.n] < lim
         m = self._pack_rows(m)
@@ -304,11 +305,33 @@ class VectorIndex:
                 return own.to(self.device, non_blocking=True)
         return t.to(self.device)
 
+    def _by_value(self, t: torch.Tensor) -> bool:
+        """Whether a small tensor can go into the arguments of the launch that reads it: of the host, a row of up to
+        ``HOST_VALUES``.  (Not while a stream is captured: ``_there``.  A pinned one may be the target of a copy that the
+        stream has yet to make: it is read in the stream's order.)"""
+        return (self.device.type == "cuda" and not t.is_cuda and t.dim() == 1 and t.numel() <= ops.native().HOST_VALUES
+                and not t.is_pinned() and not torch.cuda.is_current_stream_capturing())
+
+    def _unit(self, queries, q_groups, clear=None):
+        """(unit queries, their groups) on the device; ``clear``: a mask to be zeroed."""
+        x = torch.as_tensor(queries).to(self.device, torch.float32)
+        if q_groups is None and clear is None:
+            return ops.unit_rows(x, self.dtype), None
+        groups = None if q_groups is None else torch.as_tensor(q_groups, dtype=torch.int32)
+        if not (x.is_cuda and self.dtype == torch.bfloat16 and len(x)):
+            if clear is not None:
+                clear.zero_()
+            return ops.unit_rows(x, self.dtype), None if groups is None else self._there(groups)
+        q, there = ops.unit_queries(x, groups.contiguous() if groups is not None and self._by_value(groups) else None, clear)
+        return q, self._there(groups) if there is None and groups is not None else there
+
     def _query(self, queries, q_groups, allowed, doc_lt):
         """(unit queries, their groups, row mask, rows in whole fours) on the device."""
-        q = ops.unit_rows(torch.as_tensor(queries).to(self.device, torch.float32), self.dtype)
-        qg = None if q_groups is None else self._there(torch.as_tensor(q_groups, dtype=torch.int32))
-        allow = None if allowed is None else self.allow_mask(allowed)
+        mask, allowed = None, None if allowed is None else list(allowed)
+        if allowed and self.device.type == "cuda" and len(allowed) <= 65535:
+            mask = torch.empty((len(allowed), (self.n + 31) // 32), dtype=torch.int32, device=self.device)
+        q, qg = self._unit(queries, q_groups, mask)
+        allow = None if allowed is None else self.allow_mask(allowed, mask)
         if doc_lt is not None:
             allow = self.doc_lt_mask(doc_lt, allow)
         return q, qg, allow, (max(self.n, 4) + 3) // 4 * 4
@@ -381,8 +404,7 @@ class VectorIndex:
         query, and the list is ranked.  The threshold is the ``_sample_rank``-th best score of a strided row sample.
         It is exact whenever the list holds k rows (or the threshold cut nothing off), which the ranking kernel
         reports per query: one host read at the end, and the rare query that fails it takes ``_safe_search``."""
-        q = ops.unit_rows(torch.as_tensor(queries).to(self.device, torch.float32), self.dtype)
-        qg = None if q_groups is None else self._there(torch.as_tensor(q_groups, dtype=torch.int32))
+        q, qg = self._unit(queries, q_groups)
         n4 = (self.n + 3) // 4 * 4
         ns = (self.n // self.sample_stride) // 4 * 4
         if ns < k:  # (``_safe_search`` needs k rows in the sample)

@@ -1270,6 +1270,25 @@ def unit_rows(x, dtype=torch.bfloat16):
     return out
 
 
+def unit_queries(x, groups=None, clear=None):
+    """``unit_rows`` of a search's queries on the GPU and what else it begins with, in one launch: ``groups``, int32 of the host and
+    at most ``HOST_VALUES``, on the device (-> second result, else None); ``clear``, a contiguous int32 tensor, zeroed."""
+    expect(x.is_cuda and x.dtype == torch.float32 and x.dim() == 2, "unit_rows: fp32 [rows, cols]")
+    x = x if x.stride(1) == 1 else x.contiguous()
+    out = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+    n, there = 0, None
+    if groups is not None:
+        n = groups.numel()
+        expect(not groups.is_cuda and groups.dtype == torch.int32 and groups.dim() == 1 and groups.is_contiguous()
+               and n <= native().HOST_VALUES and x.shape[0], "unit_queries: a few int32 groups of the host, for queries")
+        there = torch.empty(n, dtype=torch.int32, device=x.device)
+    if clear is not None:
+        expect(clear.device == x.device and clear.dtype == torch.int32 and clear.is_contiguous() and x.shape[0], "unit_queries: int32 words")
+    native().unit_rows(ptr(x), x.stride(0), ptr(out), x.shape[0], x.shape[1], stream(x), ptr(groups), n, ptr(there), ptr(clear),
+                       0 if clear is None else clear.numel())
+    return out, there
+
+
 RANK_MAX = 64  # largest rank of ``rank_value``
 
 
@@ -1319,28 +1338,32 @@ def hit_ids(vals, rows, row_ids, row_docs):
     return ids, docs
 
 
-def allow_bits(ids, offsets, longest: int, keys, rows, words: int):
+def allow_bits(ids, offsets, longest: int, keys, rows, words: int, mask=None):
     """int32 bitmask [q, words] of the rows whose item id is in list q of ``ids`` (int64, list q = ids[offsets[q] :
-    offsets[q + 1]], none longer than ``longest``); ``keys`` sorted int64 ids of the live rows, ``rows`` int64 their rows."""
+    offsets[q + 1]], none longer than ``longest``); ``keys`` sorted int64 ids of the live rows, ``rows`` int64 their rows.
+    ``mask``: one of zeros, whose bits are set."""
     for t in (ids, offsets, keys, rows):
         expect(t.is_cuda and t.dtype == torch.int64 and t.is_contiguous(), "allow_bits: contiguous CUDA int64 tensors")
     q = offsets.numel() - 1
     expect(q >= 1 and keys.numel() == rows.numel(), "allow_bits: offsets of every list, one row per key")
-    mask = torch.zeros((q, words), dtype=torch.int32, device=ids.device)
+    if mask is None:
+        mask = torch.zeros((q, words), dtype=torch.int32, device=ids.device)
+    expect(mask.dtype == torch.int32 and tuple(mask.shape) == (q, words) and mask.is_contiguous() and mask.is_cuda, "mask shape")
     native().allow_bits(ptr(ids), ptr(offsets), ptr(keys), ptr(rows), keys.numel(), ptr(mask), int(words), q, int(longest),
                         stream(ids))
     return mask
 
 
 def doc_lt_bits(docs, limits, mask=None):
-    """int32 bitmask [q, ceil(n / 32)] of the rows with docs[r] < limits[q] (int64); ``mask``: intersected in place."""
-    expect(docs.is_cuda and docs.dtype == torch.int64 and limits.dtype == torch.int64 and docs.is_contiguous()
-           and limits.is_contiguous() and limits.is_cuda, "doc_lt_bits: contiguous CUDA int64 tensors")
+    """int32 bitmask [q, ceil(n / 32)] of the rows with docs[r] < limits[q] (int64, on the device, or up to ``HOST_VALUES`` of
+    the host); ``mask``: intersected in place."""
     n, q = docs.numel(), limits.numel()
+    expect(docs.is_cuda and docs.dtype == torch.int64 and limits.dtype == torch.int64 and docs.is_contiguous()
+           and limits.is_contiguous() and (limits.is_cuda or q <= native().HOST_VALUES), "doc_lt_bits: contiguous int64 tensors")
     words = (n + 31) // 32
     out = torch.empty((q, words), dtype=torch.int32, device=docs.device) if mask is None else mask
     expect(out.dtype == torch.int32 and tuple(out.shape) == (q, words) and out.is_contiguous(), "mask shape")
-    native().doc_lt_bits(ptr(docs), ptr(limits), n, ptr(out), words, q, int(mask is not None), stream(docs))
+    native().doc_lt_bits(ptr(docs), ptr(limits), n, ptr(out), words, q, int(mask is not None), stream(docs), int(not limits.is_cuda))
     return out
 
 

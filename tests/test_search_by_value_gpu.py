@@ -1,0 +1,90 @@
+"""A search's small host tensors in its launches' arguments (search.hip) against the same from tensors of the device."""
+import numpy as np
+import pytest
+import torch
+
+from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.engine.vector_index import VectorIndex
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# groups around a wave and at the most that a launch takes; words around a thread's four and a workgroup's 1024
+@pytest.mark.parametrize("rows,groups,words", [(1, 1, 0), (1, 0, 1), (3, 64, 3), (3, 65, 5), (128, 128, 1023), (2, 128, 1024), (130, 0, 1025),
+                                               (2, 2, 70_001)])
+def test_unit_queries_writes_groups_and_clears(rows, groups, words):
+    g = torch.Generator(device=DEV).manual_seed(rows + words)
+    x = torch.randn(rows, 768, device=DEV, generator=g)
+    host = torch.randint(-2 ** 31, 2 ** 31 - 1, (groups,), dtype=torch.int64).to(torch.int32) if groups else None
+    room = torch.full((words + 64,), -1, dtype=torch.int32, device=DEV)
+    q, there = ops.unit_queries(x, host, room[:words] if words else None)
+    assert torch.equal(q, ops.unit_rows(x)) and not room[:words].any() and (room[words:] == -1).all()
+    assert there is None if host is None else torch.equal(there.cpu(), host)
+
+
+def test_unit_queries_takes_no_more_values_than_fit():
+    x = torch.zeros(2, 64, device=DEV)
+    for bad in (torch.zeros(129, dtype=torch.int32), torch.zeros(2, dtype=torch.int64), torch.zeros(2, dtype=torch.int32, device=DEV)):
+        with pytest.raises(ValueError):
+            ops.unit_queries(x, bad)
+
+
+@pytest.mark.parametrize("n", [1, 32, 255, 257, 70_001])
+@pytest.mark.parametrize("queries", [1, 128, 129])
+def test_limits_of_the_host(n, queries):
+    docs = torch.arange(n, device=DEV) // 3 - 5
+    limits = torch.randint(-6, n // 3 + 2, (queries,))
+    limits[0] = -2 ** 63
+    limits[-1] = 2 ** 63 - 1
+    start = torch.randint(-2 ** 31, 2 ** 31, (queries, (n + 31) // 32), device=DEV).to(torch.int32)
+    for mask in (None, start):
+        exp = ops.doc_lt_bits(docs, limits.to(DEV), None if mask is None else mask.clone())
+        if queries > ops.native().HOST_VALUES:
+            with pytest.raises(ValueError):
+                ops.doc_lt_bits(docs, limits, None if mask is None else mask.clone())
+        else:
+            assert torch.equal(ops.doc_lt_bits(docs, limits, None if mask is None else mask.clone()), exp)
+
+
+# queries around what the arguments hold, of an index that selects (20,000 rows)
+@pytest.mark.parametrize("queries", [1, 128, 129])
+@pytest.mark.parametrize("form", ["list", "host", "strided", "pinned", "device"])
+def test_filters_of_any_form(queries, form):
+    n = 20_000
+    idx = VectorIndex(256, DEV, capacity=n)
+    g = torch.Generator(device=DEV).manual_seed(queries)
+    idx.add(np.arange(n), torch.randn(n, 256, device=DEV, generator=g), doc_ids=np.arange(n) // 4, groups=np.arange(n) % 3)
+    q = torch.randn(queries, 256, device=DEV, generator=g)
+    groups, limits = torch.arange(queries, dtype=torch.int32) % 4 - 1, 100 + 37 * torch.arange(queries)
+    allowed = [np.arange(i % 7, n, 2 + i % 5) for i in range(queries)]
+    s = idx.scores(q, groups.to(DEV))
+    lists = torch.zeros(queries, n, dtype=torch.bool, device=DEV)
+    for i, ids in enumerate(allowed):
+        lists[i, torch.from_numpy(ids).to(DEV)] = True
+    below = torch.arange(n, device=DEV)[None] // 4 < limits.to(DEV)[:, None]
+
+    def of(t):
+        return {"list": t.tolist(), "host": t, "strided": t.repeat_interleave(2)[::2], "pinned": t.pin_memory(),
+                "device": t.to(DEV) if t.dtype == torch.int32 else t}[form]
+    for kw, live in ((dict(), torch.ones_like(lists)), (dict(allowed=iter(allowed)), lists), (dict(doc_lt=of(limits)), below),
+                     (dict(allowed=tuple(allowed), doc_lt=of(limits)), lists & below)):
+        vals, ids, docs = idx.search(q, 30, q_groups=of(groups), **kw)
+        exp = s.masked_fill(~live, float("-inf"))
+        top = exp.topk(30, dim=1).values
+        hit = ~torch.isinf(top)
+        assert torch.equal(~torch.isinf(vals), hit) and torch.equal(ids >= 0, hit)
+        assert ((vals - top)[hit].abs() <= 256 * 2.0 ** -22).all()  # two fp32 sums of 256 products of unit vectors
+        at = exp.gather(1, ids.clamp(min=0))
+        assert ((vals - at)[hit].abs() <= 256 * 2.0 ** -22).all() and torch.equal(docs[hit], ids[hit] // 4)
+
+
+def test_empty_lists_allow_nothing():
+    idx = VectorIndex(256, DEV, capacity=64)
+    idx.add(np.arange(50), torch.randn(50, 256, device=DEV))
+    q = torch.randn(2, 256, device=DEV)
+    for allowed in ([[], []], [np.empty(0, np.int64), {99}], [[], [7]]):
+        vals, ids, docs = idx.search(q, 5, allowed=allowed)
+        assert ids[0].eq(-1).all() and ids[1].tolist() == ([7] if allowed[1] == [7] else [-1]) + [-1] * 4
+    idx.remove(np.arange(50))
+    assert idx.search(q, 5, allowed=[[1], [2]])[1].eq(-1).all()
