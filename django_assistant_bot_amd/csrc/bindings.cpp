@@ -725,6 +725,19 @@ PYBIND11_MODULE(_native, m) {
      py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("tile"), py::arg("s"), py::arg("next") = 0,
      py::arg("next_bytes") = 0);
   m.attr("HOST_VALUES") = dab::kHostValues;
+  m.def("search_space", [](int queries, int cols, int n, int n_groups, int masked) {
+    return dab::search_space(queries, cols, n, n_groups, masked).bytes;
+  });
+  m.def("selected_search", [](u x, long ldx, int queries, int cols, u vecs, int rows, int n, u row_group, u row_ids, u row_docs,
+                              u host_groups, int n_groups, int lists, u ids, u offsets, u keys, u key_rows, int n_keys,
+                              int longest, u limits, int k, u space, long space_bytes, u vals, u out_ids, u out_docs, u s) {
+    using I = const int64_t*;
+    const dab::SearchCall c = {(const float*)x, ldx, queries, cols, CVP(vecs), rows, n, (const int*)row_group, (I)row_ids, (I)row_docs,
+                               (const int*)host_groups, n_groups, lists, (I)ids, (I)offsets, (I)keys, (I)key_rows,
+                               n_keys, longest, (I)limits, k, VP(space), space_bytes, (float*)vals, (int64_t*)out_ids,
+                               (int64_t*)out_docs};
+    check(dab::selected_search(c, ST(s)), "selected_search");
+  });
   m.def("unit_rows", [](u x, long ldx, u out, int rows, int cols, u s, u groups, int n_groups, u groups_out, u clear, long words) {
     check(dab::unit_rows((const float*)x, ldx, VP(out), rows, cols, ST(s), (const int*)groups, n_groups, (int*)groups_out,
                          (uint32_t*)clear, words),

@@ -419,6 +419,31 @@ constexpr int kRankMax = 64;  // largest rank rank_value finds
 constexpr int kHostValues = 128;  // groups or document bounds of a search that go into a launch's arguments
 int unit_rows(const float* x, long ldx, void* out, int rows, int cols, hipStream_t s, const int* groups = nullptr, int n_groups = 0,
               int* groups_out = nullptr, uint32_t* clear = nullptr, long words = 0);
+struct SearchSpace {  // bytes into a search's workspace, and their sum; words of a query's mask, of its maxima
+  long unit, groups, mask, scores, parts, bytes;
+  int words, ldp;
+};
+SearchSpace search_space(int queries, int cols, int n, int n_groups, int masked);
+struct SearchCall {
+  const float* x;  // [queries][cols], rows ldx apart
+  long ldx;
+  int queries, cols;
+  const void* vecs;  // shuffle_weights layout
+  int rows, n;       // in use; the same in whole fours
+  const int* row_group;
+  const int64_t *row_ids, *row_docs;
+  const int* host_groups;  // of the queries (or null)
+  int n_groups, lists;     // lists: there are allow-lists, as allow_bits takes them (ids and keys may be null: none)
+  const int64_t *ids, *offsets, *keys, *key_rows;
+  int n_keys, longest;
+  const int64_t* limits;  // document bounds of the host, one a query (or null)
+  int k;
+  void* space;
+  long space_bytes;
+  float* vals;
+  int64_t *out_ids, *out_docs;
+};
+int selected_search(const SearchCall& c, hipStream_t s);
 int rank_value(const float* scores, long ld, int rows, int n, int r, float slack, float* thr, int* cnt, hipStream_t s);
 int rank_hits(const float* cand_val, const int* cand_idx, const int* cnt, const float* thr, int cap, int rows, int k,
               const int64_t* row_ids, const int64_t* row_docs, float* out_vals, int64_t* out_ids, int64_t* out_docs,

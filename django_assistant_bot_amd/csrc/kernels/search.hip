@@ -730,6 +730,54 @@ int doc_lt_bits(const int64_t* docs, const int64_t* limit, int n, uint32_t* mask
   return doc_lt_launch(docs, values, n, mask, words, queries, intersect, s);
 }
 
+// Everything a search that selects from its scores launches, in one call: unit queries (with the groups and the cleared mask),
+// the masks' bits, scores and maxima, selection.  Up to some 30k rows a search is bound by its host time, and a third of that
+// were the calls from Python with their checks and buffers: 1 query in 5,000 rows of a group 35 -> 25 us, document bounds of
+// 16 in 20k rows 40 -> 27, lists of 16 in 3,000 rows 62 -> 50, of 4 in 60k rows 67 with 46 instead of 66 of the host.
+//
+// One workspace, in pieces of 256 bytes: unit queries, groups, mask, scores, maxima.
+SearchSpace search_space(int queries, int cols, int n, int n_groups, int masked) {
+  SearchSpace w = {};
+  const auto piece = [&](long bytes) {
+    const long at = w.bytes;
+    w.bytes += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  w.ldp = ((n + 15) / 16 + 3) / 4 * 4;
+  w.words = (n + 31) / 32;
+  w.unit = piece((long)queries * cols * 2);
+  w.groups = piece((long)n_groups * 4);
+  w.mask = piece(masked ? (long)queries * w.words * 4 : 0);
+  w.scores = piece((long)queries * n * 4);
+  w.parts = piece((long)queries * w.ldp * 4);
+  return w;
+}
+
+int selected_search(const SearchCall& c, hipStream_t s) {
+  if (c.queries <= 0 || c.k <= 0 || c.k > c.n || c.rows <= 0 || c.rows > c.n || c.n % 4) return hipErrorInvalidValue;
+  if (c.host_groups && (c.n_groups < c.queries || c.n_groups > kHostValues)) return hipErrorInvalidValue;
+  if (c.limits && c.queries > kHostValues) return hipErrorInvalidValue;
+  const bool masked = c.lists || c.limits;
+  const SearchSpace w = search_space(c.queries, c.cols, c.n, c.host_groups ? c.n_groups : 0, masked);
+  if (c.space_bytes < w.bytes) return hipErrorInvalidValue;
+  char* const base = (char*)c.space;
+  uint32_t* const mask = masked ? (uint32_t*)(base + w.mask) : nullptr;
+  int* const groups = c.host_groups ? (int*)(base + w.groups) : nullptr;
+  const int words = (c.rows + 31) / 32;  // (of the rows rounded up to fours: as many)
+  if (words != w.words) return hipErrorInvalidValue;
+  int rc = unit_rows(c.x, c.ldx, base + w.unit, c.queries, c.cols, s, c.host_groups, c.host_groups ? c.n_groups : 0, groups,
+                     c.lists ? mask : nullptr, c.lists ? (long)c.queries * words : 0);
+  if (!rc && c.lists) rc = allow_bits(c.ids, c.offsets, c.keys, c.key_rows, c.n_keys, mask, words, c.queries, c.longest, s);
+  if (!rc && c.limits) rc = doc_lt_bits(c.row_docs, c.limits, c.rows, mask, words, c.queries, c.lists, 1, s);
+  if (!rc)
+    rc = index_scan_scores_shuf(base + w.unit, c.cols, c.vecs, c.queries, c.n, c.cols, c.row_group, groups, mask, (float*)(base + w.scores),
+                                base + w.parts, w.ldp, s);
+  if (!rc)
+    rc = top_hits((const float*)(base + w.scores), c.queries, c.n, base + w.parts, w.ldp, c.k, c.row_ids, c.row_docs, c.vals, c.out_ids,
+                  c.out_docs, s);
+  return rc;
+}
+
 // Rows first, first + step, ... of a matrix in the shuffle_weights layout, row-major (the search's row sample, rows of
 // a snapshot): a thread a 16-B piece, piece (c, g) of row r at [r / 16][c][g][r % 16].
 __global__ __launch_bounds__(256) void gather_rows_kernel(const u32x4* __restrict__ src, const int64_t* __restrict__ rows,

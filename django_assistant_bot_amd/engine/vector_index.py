@@ -21,6 +21,8 @@ the next update.
 """
 from __future__ import annotations
 
+from itertools import accumulate
+
 import numpy as np
 import torch
 import torch.nn.functional as F
@@ -205,22 +207,29 @@ class VectorIndex:
         packed = packed - (packed >= (1 << 31)).to(torch.int64) * (1 << 32)
         return packed.to(torch.int32).contiguous()
 
+    @staticmethod
+    def _id_lists(allowed) -> list:
+        return [np.fromiter(ids, dtype=np.int64) if isinstance(ids, (set, frozenset)) else
+                np.asarray(ids, dtype=np.int64).reshape(-1) for ids in allowed]
+
+    def _lists_there(self, lists):
+        """(ids, offsets, longest list, keys, rows) as ``ops.allow_bits`` takes them: one copy, the lists behind their offsets;
+        the ids are looked up on the device."""
+        lens = [len(x) for x in lists]
+        host = torch.empty(len(lists) + 1 + sum(lens), dtype=torch.int64, pin_memory=True)
+        flat = host.numpy()
+        flat[:len(lists) + 1] = list(accumulate(lens, initial=0))
+        np.concatenate(lists, out=flat[len(lists) + 1:])
+        dev = host.to(self.device, non_blocking=True)
+        return dev[len(lists) + 1:], dev[:len(lists) + 1], max(lens), *self._live_ids()
+
     def allow_mask(self, allowed, mask=None) -> torch.Tensor:
         """Per-query allowed item ids (sets, lists or int arrays) -> int32 bitmask [q, ceil(n/32)] over
         rows, built on the device (no per-id Python loop).  ``mask``: one of zeros to set the bits of."""
         words = (self.n + 31) // 32
-        lists = [np.fromiter(ids, dtype=np.int64) if isinstance(ids, (set, frozenset)) else
-                 np.asarray(ids, dtype=np.int64).reshape(-1) for ids in allowed]
+        lists = self._id_lists(allowed)
         if self.device.type == "cuda" and 0 < len(lists) <= 65535:
-            # one copy: the lists behind their offsets; the ids are looked up on the device
-            lens = [len(x) for x in lists]
-            host = torch.empty(len(lists) + 1 + sum(lens), dtype=torch.int64, pin_memory=True)
-            flat = host.numpy()
-            flat[0] = 0
-            np.cumsum(lens, out=flat[1:len(lists) + 1])
-            np.concatenate(lists, out=flat[len(lists) + 1:])
-            dev = host.to(self.device, non_blocking=True)
-            return ops.allow_bits(dev[len(lists) + 1:], dev[:len(lists) + 1], max(lens), *self._live_ids(), words, mask)
+            return ops.allow_bits(*self._lists_there(lists), words, mask)
         m = torch.zeros((len(allowed), words * 32), dtype=torch.bool, device=self.device)
         for qi, ids in enumerate(lists):
             rows = self.rows_of(ids)
@@ -377,10 +386,22 @@ class VectorIndex:
 
     def _selected_search(self, queries, k: int, q_groups, allowed, doc_lt):
         """Exact top-k in three launches and without a host read: unit queries, scores with the greatest of every 16 rows,
-        selection.  (The bound below which parts are not looked into is the k-th greatest of those maxima.)"""
-        q, qg, allow, n = self._query(queries, q_groups, allowed, doc_lt)
-        scores, parts = ops.scores_and_parts(q, self.vecs, n, self.row_group[:n], qg, allow)
+        selection.  (The bound below which parts are not looked into is the k-th greatest of those maxima.)  The usual filters
+        and those launches are one call; others take a call for each."""
+        rows, nq = self.n, queries.shape[0]
+        n = (max(rows, 4) + 3) // 4 * 4
+        groups = None if q_groups is None else torch.as_tensor(q_groups, dtype=torch.int32)
+        allowed = None if allowed is None else list(allowed)
+        limits = None if doc_lt is None else torch.as_tensor(np.asarray(doc_lt, dtype=np.int64))
         self.stats["selected_searches"] = self.stats.get("selected_searches", 0) + 1
+        if ((groups is None or self._by_value(groups)) and (allowed is None or len(allowed) == nq <= 65535)
+                and (limits is None or limits.numel() == nq and self._by_value(limits))):
+            lists = None if allowed is None else self._lists_there(self._id_lists(allowed))
+            return ops.selected_search(queries.to(self.device, torch.float32), self.vecs, rows, self.row_group, self.row_ids,
+                                       self.row_docs, min(k, n, 1024), None if groups is None else groups.contiguous(), lists,
+                                       None if limits is None else limits.contiguous())
+        q, qg, allow, n = self._query(queries, groups, allowed, limits)
+        scores, parts = ops.scores_and_parts(q, self.vecs, n, self.row_group[:n], qg, allow)
         return ops.top_hits(scores, parts, min(k, n, 1024), self.row_ids, self.row_docs)
 
     def _sample_rank(self, k: int) -> int:

@@ -926,6 +926,38 @@ def top_hits(scores, parts, k: int, row_ids, row_docs):
     return vals, ids, docs
 
 
+def selected_search(x, vecs, rows: int, row_group, row_ids, row_docs, k: int, groups=None, lists=None, limits=None):
+    """``top_hits`` of ``scores_and_parts`` of the unit rows of ``x`` (fp32 [q, K]) over the first ``rows`` rows of ``vecs``, in one
+    call.  ``groups``: up to ``HOST_VALUES`` int32 of the host; ``lists``: (ids, offsets, longest, keys, rows) of
+    ``allow_bits``, a list a query; ``limits``: int64 of the host, a bound on a row's document id a query."""
+    M, K = x.shape
+    n = (max(rows, 4) + 3) // 4 * 4
+    nat = native()
+    expect(x.is_cuda and x.dtype == torch.float32 and vecs.dtype == torch.bfloat16 and vecs.is_contiguous() and vecs.shape[1] == K
+           and vecs.shape[0] % 16 == 0 and vecs.shape[0] >= -(-n // 128) * 128, "selected_search: fp32 [q, K] and a shuffled copy [R, K]")
+    expect(scan_scores_ok(M, n, K) and 1 <= k <= min(n, 1024) and row_group.data_ptr() % 16 == 0
+           and min(row_group.numel(), row_ids.numel(), row_docs.numel()) >= n, "selected_search: the scan's shapes, rows' groups and ids")
+    expect(groups is None or (not groups.is_cuda and groups.dtype == torch.int32 and groups.dim() == 1 and groups.is_contiguous()
+                              and groups.numel() >= M), "q_group shorter than M")
+    ids, offsets, longest, keys, key_rows = lists if lists is not None else (None, None, 0, None, None)
+    for t in (ids, offsets, keys, key_rows) if lists is not None else ():
+        expect(t.is_cuda and t.dtype == torch.int64 and t.is_contiguous(), "allow lists: contiguous CUDA int64 tensors")
+    expect(lists is None or (offsets.numel() == M + 1 and keys.numel() == key_rows.numel()), "allow lists: one a query")
+    expect(limits is None or (not limits.is_cuda and limits.dtype == torch.int64 and limits.is_contiguous() and limits.shape == (M,)),
+           "limits: int64 of the host, one a query")
+    x = x if x.stride(1) == 1 else x.contiguous()
+    n_groups = 0 if groups is None else groups.numel()
+    nb = nat.search_space(M, K, n, n_groups, int(lists is not None or limits is not None))
+    space = torch.empty(nb, dtype=torch.uint8, device=x.device)
+    vals = torch.empty((M, k), dtype=torch.float32, device=x.device)
+    out_ids, out_docs = (torch.empty((M, k), dtype=torch.int64, device=x.device) for _ in range(2))
+    nat.selected_search(x.data_ptr(), x.stride(0), M, K, vecs.data_ptr(), rows, n, row_group.data_ptr(), row_ids.data_ptr(),
+                        row_docs.data_ptr(), ptr(groups), n_groups, int(lists is not None), ptr(ids), ptr(offsets), ptr(keys),
+                        ptr(key_rows), 0 if keys is None else keys.numel(), int(longest), ptr(limits), int(k), space.data_ptr(), nb,
+                        vals.data_ptr(), out_ids.data_ptr(), out_docs.data_ptr(), stream(x))
+    return vals, out_ids, out_docs
+
+
 def shuffled_scan_ok(M: int, K: int) -> bool:
     """Query counts / widths ``score_candidates_shuffled`` serves."""
     return M >= 1 and K % 128 == 0

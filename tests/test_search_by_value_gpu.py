@@ -88,3 +88,43 @@ def test_empty_lists_allow_nothing():
         assert ids[0].eq(-1).all() and ids[1].tolist() == ([7] if allowed[1] == [7] else [-1]) + [-1] * 4
     idx.remove(np.arange(50))
     assert idx.search(q, 5, allowed=[[1], [2]])[1].eq(-1).all()
+
+
+# rows that are no whole fours and around a mask's words; queries around a fragment and the most that the scan takes
+@pytest.mark.parametrize("dim,queries", [(256, 1), (256, 256), (512, 17), (768, 128), (1024, 2)])
+@pytest.mark.parametrize("rows", [1, 5, 31, 33, 8190, 20_003])
+def test_one_call_is_its_launches(rows, dim, queries):
+    n, k = (max(rows, 4) + 3) // 4 * 4, min(max(rows // 3, 1), 60)
+    g = torch.Generator(device=DEV).manual_seed(rows + dim)
+    frag = ops.shuffle_weights(ops.unit_rows(torch.randn(-(-n // 128) * 128, dim, device=DEV, generator=g)))
+    group, docs = (torch.arange(n, device=DEV) % 3).to(torch.int32), torch.arange(n, device=DEV) // 4
+    group[rows:] = -1
+    ids = torch.randperm(n, device=DEV, generator=g) + 9
+    keys, order = ids[:rows].sort()
+    x = torch.randn(queries, dim + 8, device=DEV, generator=g)[:, 8:]
+    few = queries <= ops.native().HOST_VALUES
+    groups = (torch.arange(queries) % 4 - 1).to(torch.int32) if few else None
+    limits = torch.randint(0, rows // 4 + 2, (queries,)) if few else None
+    lens = torch.randint(0, rows + 1, (queries,))
+    off = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).to(DEV)
+    flat = ids[torch.randint(0, n, (int(off[-1]),), device=DEV)]
+    words = (rows + 31) // 32
+    for gq, lists, lim in ((None, None, None), (groups, None, None), (None, True, None), (None, None, limits), (groups, True, limits)):
+        lists = lists and (flat, off, int(lens.max()), keys, order)
+        allow = None if lists is None else ops.allow_bits(*lists, words)
+        if lim is not None:
+            allow = ops.doc_lt_bits(docs[:rows], lim.to(DEV), allow)
+        s, p = ops.scores_and_parts(ops.unit_rows(x), frag, n, group, None if gq is None else gq.to(DEV), allow)
+        for got, exp in zip(ops.selected_search(x, frag, rows, group, ids, docs, k, gq, lists, lim), ops.top_hits(s, p, k, ids, docs)):
+            assert torch.equal(got, exp)
+
+
+def test_one_call_refuses_what_its_launches_do():
+    frag, x = torch.zeros(128, 256, dtype=torch.bfloat16, device=DEV), torch.zeros(2, 256, device=DEV)
+    group, ids = torch.zeros(8, dtype=torch.int32, device=DEV), torch.zeros(8, dtype=torch.int64, device=DEV)
+    i64 = torch.zeros(1, dtype=torch.int64)
+    for bad in (dict(x=x[:, :128]), dict(x=x.to(torch.bfloat16)), dict(rows=9), dict(k=0), dict(k=9), dict(groups=group.cpu()[:1]),
+                dict(groups=torch.zeros(2, dtype=torch.int64)), dict(limits=i64), dict(limits=i64.to(DEV)), dict(rows=129),
+                dict(lists=(i64.to(DEV), i64.to(DEV), 1, i64.to(DEV), i64.to(DEV))), dict(lists=(i64, ids[:3], 1, ids, ids))):
+        with pytest.raises(ValueError):
+            ops.selected_search(**{**dict(x=x, vecs=frag, rows=8, row_group=group, row_ids=ids, row_docs=ids, k=4), **bad})
