@@ -138,6 +138,10 @@ class VectorIndex:
                     rows[i] = self.n + j
                     self._row_of[idl[i]] = self.n + j
                 self.n += len(fresh)
+            last = dict(zip(rows.tolist(), range(n)))
+            if len(last) < n:  # an id of the index named twice: its later vector (writes to one row in one launch have no order)
+                at = np.sort(np.fromiter(last.values(), dtype=np.int64, count=len(last)))
+                rows, ids, docs, grp, v = rows[at], ids[at], docs[at], grp[at], v[torch.from_numpy(at).to(self.device)]
         pin = self.device.type == "cuda"
 
         def dev(a):
