@@ -58,20 +58,25 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return v;
 }
 
-// Exact-erf GELU, 0.5 x (1 + erf(x / sqrt 2)), without the library erff (a long piecewise routine
-// that, in a GEMM epilogue, costs more VALU time than the tile's bf16 stores): erfc by Abramowitz &
-// Stegun 7.1.26 (|error| <= 1.5e-7 in erf), one v_rcp + one v_exp + 7 FMAs.  For x < 0 the result is
-// 0.5 x erfc(|x| / sqrt 2) directly (no cancellation), for x >= 0 it is x - 0.5 x erfc(x / sqrt 2).
+// Exact-erf GELU as max(x, 0) - |x| Phi(-|x|), Phi(-a) = erfc(a / sqrt 2) / 2 = 2^P(a): P a polynomial of degree 10, fitted
+// (weighted least squares, reweighted towards the greatest error) to log2 Phi(-a) for a up to 13, where Phi leaves fp32; beyond
+// that P only falls.  Against 64 bits: 2.5e-7 at most for |x| <= 8 and, for negative x, relative errors below half of those of Abramowitz &
+// Stegun 7.1.26, which stood here before (3.3e-7 at most), at almost every x and nowhere above.  13 instructions, of which v_exp
+// takes four turns, instead of 17 with v_exp and v_rcp: the epilogue of a 256 x 256 tile is bound by them
+// (400 chunks of 32-512 tokens, bge-base, 23,542 -> 23,188 us a call; 31,900 tokens 6,690 -> 6,576).
 __device__ __forceinline__ float gelu_erf(float x) {
-  const float z = fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.f));
-  float q = fmaf(1.061405429f, t, -1.453152027f);
-  q = fmaf(q, t, 1.421413741f);
-  q = fmaf(q, t, -0.284496736f);
-  q = fmaf(q, t, 0.254829592f);
-  q *= t;
-  const float c = 0.5f * x * q * __builtin_amdgcn_exp2f(z * z * -1.4426950408889634f);  // 0.5 x erfc(z)
-  return x >= 0.f ? x - c : c;
+  const float a = fabsf(x);
+  float q = fmaf(-2.5495212607751228e-09f, a, 1.2625694978396496e-07f);
+  q = fmaf(q, a, -2.490008455424686e-06f);
+  q = fmaf(q, a, 2.3970595066202804e-05f);
+  q = fmaf(q, a, -9.180279448628426e-05f);
+  q = fmaf(q, a, -0.0003955680876970291f);
+  q = fmaf(q, a, 0.007427059579640627f);
+  q = fmaf(q, a, -0.05275694653391838f);
+  q = fmaf(q, a, -0.45912280678749084f);
+  q = fmaf(q, a, -1.1511143445968628f);
+  q = fmaf(q, a, -1.f);
+  return fmaf(-a, __builtin_amdgcn_exp2f(q), fmaxf(x, 0.f));
 }
 
 // SiLU x / (1 + e^-x) with one v_rcp_f32 instead of the IEEE division (a ~10-instruction
