@@ -662,6 +662,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("slab_slices", &dab::slab_slices);
   m.def("ring_tile", &dab::ring_tile);
   m.def("ring_wins", &dab::ring_wins);
+  m.def("gemm256_rows", &dab::gemm256_rows);
   m.def("gemm_slab", [](u A, u B, u slabs, int M, int N, int K, u s, int tile) {
     check(dab::gemm_slab(CVP(A), CVP(B), VP(slabs), M, N, K, ST(s), tile), "gemm_slab");
   }, py::arg("A"), py::arg("B"), py::arg("slabs"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("s"), py::arg("tile") = -1);

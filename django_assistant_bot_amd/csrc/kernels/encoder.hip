@@ -43,11 +43,16 @@ static int projection(const bf16* x, const void* w, const void* b, const bf16* r
                       hipStream_t s, Upcoming next = {}) {
   int tile = small_tile(M, N, K);
   if (tile < 0 && ring_wins(M, N, K, gelu, residual != nullptr)) tile = kRingTile;
-  if (tile >= 0 && gemm_small_ok(M, N, K, K, K, N, N) &&
-      !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8))
-    return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s, next);
-  if (gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K))
-    return gemm256(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, s, 0, 1);
+  const bool small = gemm_small_ok(M, N, K, K, K, N, N) &&
+                     !(((uintptr_t)x | (uintptr_t)w) % 16 || ((uintptr_t)y | (uintptr_t)b | (uintptr_t)residual) % 8);
+  if (tile >= 0 && small) return gemm_small(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, tile, s, next);
+  if (gemm256_wins(M, N) && gemm256_ok(M, N, K, K, K)) {
+    const int rows = small ? gemm256_rows(M, N, K, gelu, residual != nullptr) : M;
+    const int rc = gemm256(x, K, w, K, y, N, b, residual, N, rows, N, K, gelu, s, 0, 1);
+    if (rc || rows == M) return rc;
+    const long o = (long)rows * N;
+    return gemm_small(x + (long)rows * K, K, w, K, y + o, N, b, residual ? residual + o : nullptr, N, M - rows, N, K, gelu, kRingTile, s);
+  }
   return gemm_bt(x, K, w, K, y, N, b, residual, N, M, N, K, gelu, 0, nullptr, nullptr, nullptr, 0, s, 0, 1);
 }
 

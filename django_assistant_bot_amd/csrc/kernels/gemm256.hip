@@ -895,7 +895,7 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   // (80000, 2304, 768) 235 -> 240.  A last block of one or two columns gains less or nothing, behind an addition that wrote A:
   // (108800, 2560, 768) 389 -> 368, (108800, 2048, 768) 357 -> 320, (108800, 1792, 768) 291 -> 294.  The GELU epilogue covers
   // it: up of 108800 rows 553 us either way.
-  const bool far_a = K <= 1024 && !b_shuf && !residual && epilogue == G_NONE && (long)M * K * 2 >= (128L << 20);
+  const bool far_a = !b_shuf && !residual && epilogue == G_NONE && gemm256_far_a(M, K);
   // Otherwise groups of 4 tile rows; where there are many columns, even ones of up to 6: the 32 tiles an XCD runs at once are
   // then 6 row panels and 5-6 column panels, the fewest, and no group of one row is left over that reads 32.  us a step of
   // Llama-3-8B (gate_up, 102-112 columns), 4 rows -> these: 1093 tokens (4 + 1 -> 5) 16889 -> 16660, 3000 36434 -> 36171, 11,000

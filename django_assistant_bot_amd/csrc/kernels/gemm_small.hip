@@ -684,6 +684,23 @@ bool ring_wins(int M, int N, int K, int gelu, int residual) {
   return 1.18f * ring + 1.7f + (residual ? -0.12f : -0.53f) * mn < 0.97f * other;
 }
 
+// Rows of a projection that go to gemm256, all or whole waves of 256 tiles: the few rows behind those, for which a last wave
+// would run as long as a full one, go to the ring, where its estimate and 4 us are under 0.85 of that wave's.  The sums of K have one
+// order in both: no bits change.  Past twelve waves nothing is gained: the power limit holds the clock, and the workgroups have
+// drifted apart until the last wave.  Over 422 sizes (the projections of encoders of 384, 768 and 1024, M 5,000-112,000) it takes
+// 247, 1.11 times as fast in the mean, two of them 0.98.  us, gemm256 -> with the ring: (24291, 768, 3072) 139 -> 111, (70055, 768,
+// 3072) 313 -> 296, (10885, 3072, 768) GELU 72 -> 58, (29177, 2304, 768) 109 -> 100; left whole (98339, 3072, 768) GELU 513 / 518,
+// (12292, 2304, 768) 47 / 60.
+int gemm256_rows(int M, int N, int K, int gelu, int residual) {
+  if (M <= 0 || N < 256 || N % 256 || K < 64 || (gelu && residual)) return M;
+  const long tn = N / 256, waves = ((M + 255) / 256) * tn / 256;
+  const int rows = (int)(waves * 256 / tn * 256);
+  if (waves < 1 || waves > 12 || rows <= 0 || rows >= M) return M;
+  if (!gelu && !residual && gemm256_far_a(M, K) && !gemm256_far_a(rows, K)) return M;  // (its tile order is worth more)
+  const float ring = ring_us(kRing[ring_tile(M - rows, N, K, gelu, 1)], M - rows, N, K, gelu);
+  return ring + 4.f < 0.85f * (0.0146f * K + 7.f + (gelu ? 5.7f : 0.f) + (residual ? 3.9f : 0.f)) ? rows : M;
+}
+
 template <int I, int WM, int WN, int NS>
 static void ring_launch(const SmallParams& p, int gelu, hipStream_t s) {
   constexpr RingTile t = kRing[I];

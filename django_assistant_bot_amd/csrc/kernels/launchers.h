@@ -293,6 +293,8 @@ int gemm_grouped(const void* A, long lda, const void* B, void* C, long ldc, int 
 // 2 SwiGLU on [gate 16 | up 16]-interleaved weight rows; bias / residual optional)
 constexpr int kGemm256Fill = 192;  // 256 x 256 tiles that keep a shape on gemm256 below 1024 rows
 bool gemm256_wins(int M, int N);
+// A of a short K that has left the Infinity Cache when the projection starts (gemm256: its tile order)
+inline bool gemm256_far_a(long M, int K) { return K <= 1024 && M * K * 2 >= (128L << 20); }
 int gemm256_ok(int M, int N, int K, long lda, long ldb);
 int gemm256_candidates(const void* A, long lda, const void* B, long ldb, int M, int N, int K, const int* row_group,
                        const int* q_group, const float* thr, int* cnt, float* cand_val, int* cand_idx, int cap,
@@ -408,6 +410,7 @@ int gemm_ln_ok(int M, int N, int K, int tile);
 int slab_slices(int M, int N, int K);
 int ring_tile(int M, int N, int K, int gelu, int slices);
 bool ring_wins(int M, int N, int K, int gelu, int residual);
+int gemm256_rows(int M, int N, int K, int gelu, int residual);
 int gemm_slab(const void* A, const void* B, void* slabs, int M, int N, int K, hipStream_t s, int tile = -1);
 int gemm_ln(const void* x, const void* gain, const void* offset, float eps, void* normed, const void* w, const void* b, void* C,
             int M, int N, int K, int gelu, int tile, hipStream_t s, Upcoming next = {});

@@ -629,19 +629,25 @@ def small_tile(M: int, N: int, K: int) -> int:
     return native().small_tile(M, N, K)
 
 
-def _gemm_small_into(A, B, out, bias, residual, epilogue) -> bool:
-    """Runs a projection on ``gemm_small`` where it is the faster kernel and takes the operands; else False."""
+def _gemm_small_takes(A, B, out, bias, residual) -> bool:
+    ldr = residual.stride(0) if residual is not None else 0
+    return bool(native().gemm_small_ok(A.shape[0], B.shape[0], A.shape[1], A.stride(0), B.stride(0), out.stride(0), ldr)
+                and not ((ptr(A) | ptr(B)) % 16 or (ptr(out) | ptr(bias) | ptr(residual)) % 8))
+
+
+def _gemm_small_into(A, B, out, bias, residual, epilogue, tile: int | None = None) -> bool:
+    """Runs a projection on ``gemm_small`` where it is the faster kernel (or on its given tile) and takes the operands; else
+    False."""
     M, K = A.shape
     N = B.shape[0]
-    tile = small_tile(M, N, K) if M and N else -1
-    ldr = residual.stride(0) if residual is not None else 0
-    if tile < 0 and native().ring_wins(M, N, K, int(epilogue == EPI_GELU), int(residual is not None)):
-        tile = native().RING_TILE
-    if (tile < 0 or not native().gemm_small_ok(M, N, K, A.stride(0), B.stride(0), out.stride(0), ldr)
-            or (ptr(A) | ptr(B)) % 16 or (ptr(out) | ptr(bias) | ptr(residual)) % 8):
+    if tile is None:
+        tile = small_tile(M, N, K) if M and N else -1
+        if tile < 0 and native().ring_wins(M, N, K, int(epilogue == EPI_GELU), int(residual is not None)):
+            tile = native().RING_TILE
+    if tile < 0 or not _gemm_small_takes(A, B, out, bias, residual):
         return False
-    native().gemm_small(ptr(A), A.stride(0), ptr(B), B.stride(0), ptr(out), out.stride(0), ptr(bias), ptr(residual), ldr,
-                        M, N, K, int(epilogue == EPI_GELU), tile, stream(A))
+    native().gemm_small(ptr(A), A.stride(0), ptr(B), B.stride(0), ptr(out), out.stride(0), ptr(bias), ptr(residual),
+                        residual.stride(0) if residual is not None else 0, M, N, K, int(epilogue == EPI_GELU), tile, stream(A))
     return True
 
 
@@ -712,7 +718,14 @@ def gemm_bt(A, B, bias=None, residual=None, epilogue=EPI_NONE, out_f32=False, ro
         return out
     if (epilogue in (EPI_NONE, EPI_GELU, EPI_SWIGLU, *GLU8) and plain and (not shuffled or N == B.shape[0])
             and use_gemm256(M, N, K, A.stride(0), B.stride(0))):
-        return _gemm256_into(A, B, out, bias if glu_bias is None else glu_bias, residual, epilogue, shuffled, b_group)
+        rows = M
+        if not shuffled and epilogue in (EPI_NONE, EPI_GELU) and _gemm_small_takes(A, B, out, bias, residual):
+            rows = native().gemm256_rows(M, N, K, int(epilogue == EPI_GELU), int(residual is not None))
+        _gemm256_into(A[:rows], B, out[:rows], bias if glu_bias is None else glu_bias, None if residual is None else residual[:rows],
+                      epilogue, shuffled, b_group)
+        if rows < M:
+            _gemm_small_into(A[rows:], B, out[rows:], bias, None if residual is None else residual[rows:], epilogue, native().RING_TILE)
+        return out
     native().gemm_bt(ptr(A), A.stride(0), ptr(B), B.stride(0), ptr(out), out.stride(0),
                      ptr(bias if glu_bias is None else glu_bias), ptr(residual),
                      residual.stride(0) if residual is not None else 0, M, N, K, int(epilogue), int(out_f32),
