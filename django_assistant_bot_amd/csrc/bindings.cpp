@@ -683,6 +683,16 @@ PYBIND11_MODULE(_native, m) {
   }, py::arg("A"), py::arg("lda"), py::arg("B"), py::arg("ldb"), py::arg("C"), py::arg("ldc"), py::arg("bias"), py::arg("residual"),
      py::arg("ldr"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("gelu"), py::arg("tile"), py::arg("s"),
      py::arg("next") = 0, py::arg("next_bytes") = 0);
+  m.def("rows_stream_ok", [](int M, int N, int K, long ldx, int w_group) { return dab::rows_stream_ok(M, N, K, ldx, w_group) != 0; });
+  m.def("rows_stream", [](u X, long ldx, u W, u residual, u out, int M, int N, int K, int w_group, u s, int tile) {
+    check(dab::rows_stream(CVP(X), ldx, CVP(W), CVP(residual), VP(out), M, N, K, w_group, ST(s), tile), "rows_stream");
+  }, py::arg("X"), py::arg("ldx"), py::arg("W"), py::arg("residual"), py::arg("out"), py::arg("M"), py::arg("N"), py::arg("K"),
+     py::arg("w_group"), py::arg("s"), py::arg("tile") = -1);
+  m.def("norm_rows_ok", [](int M, int N, int K, int SO, int bn) { return dab::norm_rows_ok(M, N, K, SO, bn) != 0; });
+  m.def("norm_rows", [](u x, u gain, float eps, u W, u out, long ldo, int M, int N, int K, int SO, int out_f32, int glu, int w_group,
+                        int bn, u s) {
+    check(dab::norm_rows(CVP(x), CVP(gain), eps, CVP(W), VP(out), ldo, M, N, K, SO, out_f32, glu, w_group, bn, ST(s)), "norm_rows");
+  });
   m.def("norm_stream_ok", [](int M, int N, int K, int SO, int bn) { return dab::norm_stream_ok(M, N, K, SO, bn) != 0; });
   m.def("norm_stream", [](u slabs, int S, int slabs_f32, u residual, u gain, u residual_out, float eps, u W, u out, long ldo,
                           int M, int N, int K, int SO, int out_f32, int glu, int w_group, int bn, u s) {

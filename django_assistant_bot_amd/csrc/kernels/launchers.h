@@ -311,6 +311,14 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
             const void* residual, long ldr, int M, int N, int K, int epilogue, hipStream_t s, int b_shuf = 0,
             int b_group = 1);
 
+// rows_stream.hip: X . W^T + residual of up to 8 decode rows, K whole in a workgroup
+int rows_stream_ok(int M, int N, int K, long ldx, int w_group);
+int rows_stream(const void* X, long ldx, const void* W, const void* residual, void* out, int M, int N, int K, int w_group,
+                hipStream_t s, int tile = -1);
+// norm_stream.hip: RMSNorm(rows) . W^T of up to 8 decode rows
+int norm_rows_ok(int M, int N, int K, int SO, int bn);
+int norm_rows(const void* x, const void* gain, float eps, const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32,
+              int glu, int w_group, int bn, hipStream_t s);
 // norm_stream.hip: RMSNorm(sum of slabs + residual) . W^T of up to 4 decode rows
 int norm_stream_ok(int M, int N, int K, int SO, int bn);
 int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, const void* gain, void* residual_out, float eps,

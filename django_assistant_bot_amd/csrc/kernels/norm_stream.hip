@@ -1,5 +1,5 @@
 // Decode projections of a few rows with the RMS norm in front of them:  C[M, N] = RMSNorm(x + residual) . W[N, K]^T, the
-// norm's input being the split-K slabs of the projection before it (or plain rows).  M <= 4, weights in the shuffle_weights
+// norm's input being the split-K slabs of the projection before it (or plain rows).  M <= 4 (complete rows: 8), weights in the shuffle_weights
 // layout, K <= 4096, M K_slice <= 32768.
 //
 // A decode layer of a few sequences is a chain of launches; the two norms of a layer are one small workgroup a row between
@@ -12,7 +12,9 @@
 //
 // us, norm launch and stream_gemm -> here, 4 slabs of K 4096 / 8 of K 2048: (1, 6144, 4096) 14.1 -> 12.0, 4 rows 14.6 ->
 // 12.9; gated (1, 28672, 4096) 43.0 -> 40.1, 4 rows 43.8 -> 41.8; (1, 3072, 2048) 7.9 -> 6.3, 4 rows 8.2 -> 7.0; gated (1,
-// 16384, 2048) 16.9 -> 15.5, 4 rows 16.9 -> 16.3.  5-8 rows, a wave each: (5, 3072, 2048) 8.2 -> 9.5, not taken.
+// 16384, 2048) 16.9 -> 15.5, 4 rows 16.9 -> 16.3.  5-8 rows, a wave each: (5, 3072, 2048) 8.2 -> 9.5, not taken of slabs.
+// Complete rows (norm_rows; rows_stream.hip leaves them), up to 8, are one read each: 6 rows, norm launch and stream_gemm ->
+// here, gated (28672, 4096) 42.4 -> 37.5, (6144, 4096) 16.4 -> 12.2, gated (16384, 2048) 18.5 -> 15.0, (3072, 2048) 10.5 -> 5.9.
 //
 // Weights: wave w of the tile's NWC compute waves holds RT 16-row blocks; a chunk is 32 k of them, 1 KB a block, MFMA A
 // fragments straight to registers through a ring of DEP chunks (128 KB in flight a CU).  The rows are the B operand, in
@@ -70,54 +72,77 @@ __global__ __launch_bounds__(64 * (NWC + kNormWaves), 1) void norm_stream_kernel
     const bool mine = nw / WPR < p.M;
     int iv[VPL];
     bool ok[VPL];
-    u32x4 gain[VPL], r[VPL], h[VPL];  // h: the row (with the residual), bf16
-    float v[VPL][8];
+    u32x4 gain[VPL], h[VPL];  // h: the row (with the residual), bf16
+    float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       const int i = (nw % WPR + k * WPR) * 64 + lane;
       ok[k] = mine && i < nvec;
       iv[k] = min(i, nvec - 1);
-      if (p.residual) r[k] = reinterpret_cast<const u32x4*>(p.residual + (size_t)m * p.K)[iv[k]];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
     }
-    const ST* base = (const ST*)p.slabs + (size_t)m * p.K;
-    for (int s0 = 0; s0 < p.S; s0 += U) {
-      SlabVec8<ST> a[VPL][U];
+    if constexpr (U == 0) {
 #pragma unroll
-      for (int k = 0; k < VPL; ++k)
+      for (int k = 0; k < VPL; ++k) h[k] = reinterpret_cast<const u32x4*>((const bf16*)p.slabs + (size_t)m * p.K)[iv[k]];
 #pragma unroll
-        for (int u = 0; u < U; ++u) a[k][u].load(base + (size_t)min(s0 + u, p.S - 1) * p.slab_stride + (size_t)iv[k] * 8);
-      if (s0 == 0) {
-#pragma unroll
-        for (int k = 0; k < VPL; ++k) gain[k] = reinterpret_cast<const u32x4*>(p.gain)[iv[k]];
-        __builtin_amdgcn_sched_barrier(0);
-        // the weights' loads start behind these: queued behind 128 KB of them the rows came 1.5 us later
-        __builtin_amdgcn_s_barrier();
-      }
+      for (int k = 0; k < VPL; ++k) gain[k] = reinterpret_cast<const u32x4*>(p.gain)[iv[k]];
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();  // (the weights' loads start behind these, as below)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (s0 + u < p.S) {  // uniform
-#pragma unroll
-          for (int k = 0; k < VPL; ++k) a[k][u].add_to(v[k]);
-        }
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int k = 0; k < VPL; ++k) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[k][j] = bf2f(f2bf(v[k][j]));
-      if (p.residual) {
+      for (int k = 0; k < VPL; ++k) {
         float f[8];
-        unpack8(r[k], f);
+        unpack8(h[k], f);
+        if (ok[k]) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[k][j] = bf2f(f2bf(v[k][j] + f[j]));
+          for (int j = 0; j < 8; ++j) ss += f[j] * f[j];
+        }
       }
-      h[k] = pack8(v[k]);
-      if (ok[k]) {
+    } else {
+      u32x4 r[VPL];
+      float v[VPL][8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss += v[k][j] * v[k][j];
+      for (int k = 0; k < VPL; ++k) {
+        if (p.residual) r[k] = reinterpret_cast<const u32x4*>(p.residual + (size_t)m * p.K)[iv[k]];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
+      }
+      const ST* base = (const ST*)p.slabs + (size_t)m * p.K;
+      for (int s0 = 0; s0 < p.S; s0 += U) {
+        SlabVec8<ST> a[VPL][U];
+#pragma unroll
+        for (int k = 0; k < VPL; ++k)
+#pragma unroll
+          for (int u = 0; u < U; ++u) a[k][u].load(base + (size_t)min(s0 + u, p.S - 1) * p.slab_stride + (size_t)iv[k] * 8);
+        if (s0 == 0) {
+#pragma unroll
+          for (int k = 0; k < VPL; ++k) gain[k] = reinterpret_cast<const u32x4*>(p.gain)[iv[k]];
+          __builtin_amdgcn_sched_barrier(0);
+          // the weights' loads start behind these: queued behind 128 KB of them the rows came 1.5 us later
+          __builtin_amdgcn_s_barrier();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (s0 + u < p.S) {  // uniform
+#pragma unroll
+            for (int k = 0; k < VPL; ++k) a[k][u].add_to(v[k]);
+          }
+      }
+#pragma unroll
+      for (int k = 0; k < VPL; ++k) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[k][j] = bf2f(f2bf(v[k][j]));
+        if (p.residual) {
+          float f[8];
+          unpack8(r[k], f);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[k][j] = bf2f(f2bf(v[k][j] + f[j]));
+        }
+        h[k] = pack8(v[k]);
+        if (ok[k]) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss += v[k][j] * v[k][j];
+        }
       }
     }
     ss = wave_sum_valu(ss);
@@ -275,6 +300,36 @@ int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, c
 #undef NS_TILE
 #undef NS_ROWS
 #undef NS_LAUNCH
+  return hipGetLastError();
+}
+
+// ... of up to 8 complete rows (no slabs, no residual); with more than 4 a norm wave each.  Slices of whole eights of 16-B
+// pieces, in which the rows are permuted.
+int norm_rows_ok(int M, int N, int K, int SO, int bn) {
+  return M >= 1 && M <= kNormWaves && norm_stream_ok(1, N, K, SO, bn) && K / SO % 64 == 0 && (long)M * (K / SO) * 2 <= kNormX &&
+         (long)SO * M * N * 4 < (1L << 31);
+}
+
+int norm_rows(const void* x, const void* gain, float eps, const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32,
+              int glu, int w_group, int bn, hipStream_t s) {
+  if (!norm_rows_ok(M, N, K, SO, bn) || (glu && SO > 1) || ldo % 4) return hipErrorInvalidValue;
+  if (w_group < 1 || N % (16 * w_group)) return hipErrorInvalidValue;
+  const NormStream p = {x, 1, (long)M * K, nullptr, (const bf16*)gain, nullptr, eps, (const bf16*)W,
+                        out, ldo, M, N, K, SO, K / SO, glu, out_f32, w_group};
+  const dim3 grid(N / bn * SO), block(64 * (4 + kNormWaves));
+#define NS_ROWS(WPR)                                                                                                          \
+  do {                                                                                                                        \
+    constexpr int few = (4 + WPR - 1) / WPR, more = 8 / WPR;                                                                  \
+    if (K <= 2048 && bn == 64) hipLaunchKernelGGL((norm_stream_kernel<1, 4, 32, WPR, few, 0, bf16>), grid, block, 0, s, p);   \
+    else if (K <= 2048) hipLaunchKernelGGL((norm_stream_kernel<2, 4, 16, WPR, few, 0, bf16>), grid, block, 0, s, p);          \
+    else if (bn == 64) hipLaunchKernelGGL((norm_stream_kernel<1, 4, 32, WPR, more, 0, bf16>), grid, block, 0, s, p);          \
+    else hipLaunchKernelGGL((norm_stream_kernel<2, 4, 16, WPR, more, 0, bf16>), grid, block, 0, s, p);                        \
+  } while (0)
+  if (M == 1) NS_ROWS(8);
+  else if (M == 2) NS_ROWS(4);
+  else if (M <= 4) NS_ROWS(2);
+  else NS_ROWS(1);
+#undef NS_ROWS
   return hipGetLastError();
 }
 

@@ -57,6 +57,7 @@ class LlamaModel(FragmentProjections):
     VOCAB_PAD = 384
     PREFILL_STREAM_MAX_M = 256
     NORM_STREAM_MAX_M = 4  # rows up to which the norms run inside the projections behind them (0: off)
+    ROWS_MAX_M = 8  # sequences up to which a decode step's o and down leave the residual stream complete, where the model's sizes allow (0: off)
 
     def __init__(self, cfg: DecoderConfig, weights: dict, device, tp_group=None, tp_size: int = 1,
                  interleaved_mlp: bool = False, fragment_layout: bool = True, consume: bool = False,
@@ -130,6 +131,7 @@ class LlamaModel(FragmentProjections):
         if small_norm_fused is not None:
             self.small_norm_fused = bool(small_norm_fused)
         self.fold_norms = self.frag and self.small_norm_fused
+        self._rows_of: dict[int, bool] = {}
         self.layers = []
         for i in range(cfg.layers):
             an = take(f"l{i}.attn_norm").to(self.device)
@@ -351,6 +353,18 @@ class LlamaModel(FragmentProjections):
         s = ops.frag_slices(x.shape[0], w.shape[0], w.shape[1]) if self.frag and w.shape[0] % 256 == 0 else 0
         return ops.gemm_frag(x, w, slices=s, b_group=self.proj_group.get(name, 1)) if s else None
 
+    def _rows(self, L: DecoderLayer, T: int) -> bool:
+        """Whether a decode step of ``T`` sequences keeps the residual stream complete between its projections: o and down over
+        the whole K (``ops.rows_stream``), the norms inside qkv and gate_up.  Up to 4 rows those summed slabs before, from 5 on norm
+        launches did.  us a step, slabs -> complete: Llama-3-8B 1 sequence of 1150 tokens 3028 -> 2917, 4 of 300-1700 3425 -> 3252, 6 of
+        200-900 3407 -> 3100, 8 of 300-1700 3602 -> 3376; Llama-3.2-1B 1 of 500 833 -> 781, 6 of 200-900 926 -> 815, 8 960 -> 856."""
+        if not (T <= self.ROWS_MAX_M and self.tp_size == 1 and self.interleaved_mlp):
+            return False
+        serves = self._rows_of.get(T)  # (the layers' shapes are one)
+        if serves is None:
+            serves = self._rows_of[T] = self._rows_serve(T, L.qkv_w, L.o_w, L.gate_up_w, L.down_w)
+        return serves
+
     def _layer(self, li: int, L: DecoderLayer, x, residual, meta: AttnMeta, kv: KVCache, sk: bool):
         """One decoder layer: (layer input, residual stream) -> (next layer input, residual stream)."""
         cfg, D, T = self.cfg, self.cfg.head_dim, meta.positions.numel()  # x may be [S, T, H] split-K slabs
@@ -359,9 +373,13 @@ class LlamaModel(FragmentProjections):
         # like the separate bf16 add), so the RMSNorms read and write one tensor instead of two each;
         # x is None then: the residual stream already holds the layer input
         fuse = not sk and self.tp_size == 1 and (x if x is not None else residual).is_cuda
+        rows = sk and meta.decode and self._rows(L, T)
         few = sk and self.tp_size == 1 and T <= self.NORM_STREAM_MAX_M
-        both = self._norm_proj(x, L.attn_norm, cfg.eps, residual, L.qkv_w, "qkv") if few else None
-        if both is not None:
+        both = self._norm_proj(x, L.attn_norm, cfg.eps, residual, L.qkv_w, "qkv") if few and not rows else None
+        if rows:
+            residual = x if x is not None else residual
+            qkv = self._rows_proj(residual, L.attn_norm, cfg.eps, L.qkv_w, "qkv")
+        elif both is not None:
             qkv, residual = both
         else:
             if x is None:
@@ -381,12 +399,12 @@ class LlamaModel(FragmentProjections):
             q = qkv[:, :self.hq * D].view(T, self.hq, D)
             a = ops.flash_attention_paged(q, kv.k[li], kv.v[li], meta.block_tables, meta.cu_q, meta.ctx_lens,
                                           meta.max_q, causal=True, rope=(meta.positions, self.cos_sin))
-            return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D)
+            return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D, rows)
         if meta.decode and qkv.is_cuda and qkv.dtype in (torch.float32, torch.bfloat16) and self.rope_in_decode(T, meta):
             a = ops.paged_decode_rope(qkv, meta.positions, self.cos_sin, kv.k[li], kv.v[li], meta.slots, self.hq,
                                       meta.block_tables, meta.ctx_lens, meta.part_size, meta.workspace, order=meta.order,
                                       warm=self._warm(L, T, qkv))
-            return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D)
+            return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D, rows)
         q = ops.rope_kv_write(qkv, meta.positions, self.cos_sin, kv.k[li], kv.v[li], meta.slots, self.hq, self.hkv, D)
         if meta.decode:
             a = ops.paged_decode(q, kv.k[li], kv.v[li], meta.block_tables, meta.ctx_lens, meta.part_size,
@@ -396,14 +414,18 @@ class LlamaModel(FragmentProjections):
         else:
             a = ops.flash_attention_paged(q, kv.k[li], kv.v[li], meta.block_tables, meta.cu_q, meta.ctx_lens,
                                           meta.max_q, causal=True)
-        return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D)
+        return self._layer_tail(L, a, residual, sk, fuse, slabs_ok, T, D, rows)
 
-    def _layer_tail(self, L, a, residual, sk, fuse, slabs_ok, T, D):
+    def _layer_tail(self, L, a, residual, sk, fuse, slabs_ok, T, D, rows=False):
         """o projection, MLP norm, gate_up (+SwiGLU), down: -> (next layer input, residual stream)."""
         cfg = self.cfg
         # SwiGLU in the GEMM epilogue (8-row [gate | up] groups) on the GPU
         epi = ops.EPI_SWIGLU8 if (self.interleaved_mlp and a.is_cuda) else ops.EPI_NONE
         both = None
+        if rows:
+            residual = ops.rows_stream(a.view(T, self.hq * D), L.o_w, residual, self.proj_group.get("o", 1))
+            act = self._rows_proj(residual, L.mlp_norm, cfg.eps, L.gate_up_w, "gate_up", epi)
+            return None, ops.rows_stream(act, L.down_w, residual, self.proj_group.get("down", 1))
         if fuse:
             a = a.view(T, self.hq * D)
             o = self._slab_proj(a, L.o_w, "o")

@@ -140,7 +140,7 @@ class FragmentProjections:
     def _norm_proj(self, x, gain, eps: float, residual, w, name: str, epilogue=ops.EPI_NONE):
         """RMSNorm(x + residual) and the projection behind it in one launch for a few decode rows (``ops.norm_stream``, TP 1,
         fragment layout) -> (product, slabs where a consumer sums them; new residual), or None where that is not taken: up to
-        4 rows, projections that split as ``stream_gemm`` does on 64 weight rows a workgroup, gated ones unsplit on 128 (us,
+        4 rows whose model ``_rows_serve`` leaves out, projections that split as ``stream_gemm`` does on 64 weight rows a workgroup, gated ones unsplit on 128 (us,
         4 rows of gated (28672, 4096) / (16384, 2048): 41.8 / 16.3 on 128, 43.7 / 18.5 on 64).  ``residual`` None: the first layer's
         input is the residual stream."""
         M, K, N, grp = x.shape[-2], x.shape[-1], w.shape[0], self.proj_group.get(name, 1)
@@ -151,6 +151,23 @@ class FragmentProjections:
         sd = torch.bfloat16 if self.slab_bf16 else torch.float32
         y, new = ops.norm_stream(x, gain, eps, residual, w, splits=s, bn=bn, epilogue=epilogue, slab_dtype=sd, w_group=grp)
         return y, (x if residual is None else new)
+
+    def _rows_proj(self, x, gain, eps: float, w, name: str, epilogue=ops.EPI_NONE):
+        """``_norm_proj`` of up to 8 rows that are complete (the residual stream itself, as ``ops.rows_stream`` leaves it)."""
+        gated = epilogue != ops.EPI_NONE
+        bn, s = (128, 1) if gated else (64, self._stream_splits(w.shape[0], w.shape[1], 64))
+        return ops.norm_rows(x, gain, eps, w, splits=s, bn=bn, epilogue=epilogue, w_group=self.proj_group.get(name, 1),
+                             slab_dtype=torch.bfloat16 if self.slab_bf16 else torch.float32)
+
+    def _rows_serve(self, T: int, qkv, o, gate_up, down) -> bool:
+        """Whether a layer's projections of ``T`` rows all take ``_rows_proj`` and ``ops.rows_stream``."""
+        nat, group = ops.native(), lambda name: self.proj_group.get(name, 1)
+
+        def normed(w, name, bn, s):
+            return w.shape[0] % (16 * group(name)) == 0 and nat.norm_rows_ok(T, *w.shape, s, bn)
+
+        return (self.frag and normed(qkv, "qkv", 64, self._stream_splits(*qkv.shape, 64)) and normed(gate_up, "gate_up", 128, 1)
+                and all(nat.rows_stream_ok(T, *w.shape, w.shape[1], group(name)) for w, name in ((o, "o"), (down, "down"))))
 
     def _stream_or_tile(self, x, w, dec: bool, allow_slabs: bool, name: str, epilogue, grp: int, out=None, glu_bias=None):
         """``out`` / ``glu_bias``: of a gated epilogue (a view to write, fp32 [gate | up])."""

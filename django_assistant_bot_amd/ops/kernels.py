@@ -1132,6 +1132,38 @@ def norm_stream(x, gain, eps, residual, w, splits=1, bn=64, epilogue=EPI_NONE, s
     return out, new
 
 
+def norm_rows(x, gain, eps, w, splits=1, bn=64, epilogue=EPI_NONE, slab_dtype=torch.float32, w_group: int = 1):
+    """``norm_stream`` of up to 8 complete rows (bf16 [M, K], no slabs, no residual) -> product."""
+    (M, K), N = x.shape, w.shape[0]
+    expect(x.is_cuda, "norm_rows: rows on the GPU")
+    expect_bf16_contig(x, gain, w)
+    same_device(x, gain, w)
+    expect(gain.numel() == K and w.shape[1] == K and native().norm_rows_ok(M, N, K, splits, bn), "norm_rows: shapes")
+    expect(epilogue == EPI_NONE or (epilogue == EPI_SWIGLU8 and splits == 1), "norm_rows: slabs, rows or SwiGLU of 8-row groups")
+    expect(N % (16 * w_group) == 0 and slab_dtype in (torch.float32, torch.bfloat16), "whole groups; fp32 or bf16 slabs")
+    if splits > 1:
+        out = torch.empty((splits, M, N), dtype=slab_dtype, device=x.device)
+    else:
+        out = torch.empty((M, N // 2 if epilogue else N), dtype=torch.bfloat16, device=x.device)
+    native().norm_rows(ptr(x), ptr(gain), float(eps), ptr(w), ptr(out), out.shape[-1], M, N, K, splits, int(slab_dtype == torch.float32),
+                       int(epilogue != EPI_NONE), int(w_group), int(bn), stream(x))
+    return out
+
+
+def rows_stream(x, w, residual, w_group: int = 1, tile: int = -1):
+    """x w^T (rounded to bf16) + residual of up to 8 decode rows, w a ``shuffle_weights`` copy (rows_stream.hip).  ``tile`` (tests):
+    that form of the kernel."""
+    (M, K), N = x.shape, w.shape[0]
+    expect(x.is_cuda and x.dtype == torch.bfloat16 and x.stride(1) == 1, "rows_stream: bf16 rows on the GPU")
+    expect_bf16_contig(w, residual)
+    same_device(x, w, residual)
+    expect(w.shape[1] == K and tuple(residual.shape) == (M, N), "rows_stream: shapes")
+    expect(native().rows_stream_ok(M, N, K, x.stride(0), w_group), "rows_stream: up to 8 rows, whole groups, K % 64")
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    native().rows_stream(ptr(x), x.stride(0), ptr(w), ptr(residual), ptr(out), M, N, K, int(w_group), stream(x), int(tile))
+    return out
+
+
 def slab_reduce(slabs, residual=None, out=None):
     """fp32 / bf16 slabs [S, M, N] -> bf16 [M, N] (fp32 sum rounded to bf16, then + residual)."""
     if not slabs.is_cuda:

@@ -1,0 +1,108 @@
+"""Decode rows kept complete: projections over the whole K with the residual (rows_stream.hip), and the norm of such
+rows inside the projection behind (norm_stream.hip), against fp64 products and the norm kernel."""
+import dataclasses
+
+import pytest
+import torch
+
+from django_assistant_bot_amd import ops
+from django_assistant_bot_amd.models import AttnMeta, LlamaModel, decoder_config, random_decoder_weights
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rand(seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+
+
+# fewer pairs of chunks than waves, as many as a ring, more and not in whole turns; one block of weight rows and groups of 8
+@pytest.mark.parametrize("N,K,grp", [(16, 256, 1), (48, 320, 1), (128, 4096, 8), (64, 4160, 1), (2048, 2048, 1), (128, 14336, 8)])
+@pytest.mark.parametrize("M", [1, 2, 5, 8])
+@pytest.mark.parametrize("pad,tile", [(0, -1), (8, 0), (0, 1), (8, 2)])
+def test_rows_stream(N, K, grp, M, pad, tile):
+    rand = _rand(N + K + M)
+    x = rand(M, K + pad).to(torch.bfloat16)[:, :K]
+    W, res = (rand(N, K) * K ** -0.5).to(torch.bfloat16), rand(M, N).to(torch.bfloat16)
+    y = ops.rows_stream(x, ops.shuffle_weights(W, grp), res, grp, tile)
+    exp = x.double() @ W.double().t()
+    # roundings to bf16 of the product and of the sum (2^-8 of each); fp32 sums of K products of size about K^-1/2
+    tol = 2.0 ** -8 * exp.abs() + 1e-4
+    exp = exp + res.double()
+    assert ((y.double() - exp).abs() <= tol + 2.0 ** -8 * exp.abs()).all()
+
+
+def test_nothing_of_the_rows_behind_reaches_a_result():
+    x = torch.full((6, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+    x[:, :320] = 1.0  # chunks behind K: the same buffer, as the rows of a wider tensor
+    W = torch.ones(32, 320, dtype=torch.bfloat16, device=DEV)
+    y = ops.rows_stream(x[:, :320], ops.shuffle_weights(W), torch.zeros(6, 32, dtype=torch.bfloat16, device=DEV))
+    assert (y == 320.0).all()
+
+
+@pytest.mark.parametrize("N,K,splits,bn,grp", [(64, 256, 1, 64, 1), (128, 512, 8, 64, 8), (256, 2048, 4, 128, 8), (128, 2560, 1, 128, 1),
+                                               (640, 4096, 2, 64, 1), (256, 4096, 1, 128, 8)])
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 7, 8])
+def test_norm_rows(N, K, splits, bn, grp, M):
+    rand = _rand(N + K + M)
+    x, gain = rand(M, K).to(torch.bfloat16), (1 + 0.1 * rand(K)).to(torch.bfloat16)
+    W = (rand(N, K) * K ** -0.5).to(torch.bfloat16)
+    frag = ops.shuffle_weights(W, grp)
+    h, _ = ops.rmsnorm(x, gain, 1e-5)
+    exp = h.double() @ W.double().t()
+    # the row's length is summed in another order: 2^-8 of the product's terms in the root of their squares, and the rounding
+    # of what is stored
+    tol = 2.0 ** -8 * ((h.double() ** 2) @ (W.double() ** 2).t()).sqrt() + 1e-5
+    for sd in (torch.float32, torch.bfloat16):
+        y = ops.norm_rows(x, gain, 1e-5, frag, splits=splits, bn=bn, slab_dtype=sd, w_group=grp)
+        part = y.double() if splits > 1 else y.double()[None]
+        store = 0 if splits > 1 and sd == torch.float32 else 2.0 ** -8 * part.abs().sum(0)
+        assert ((part.sum(0) - exp).abs() <= tol + store).all()
+    if splits == 1:
+        y = ops.norm_rows(x, gain, 1e-5, frag, bn=bn, epilogue=ops.EPI_SWIGLU8, w_group=grp)
+        v, t = exp.view(M, N // 16, 2, 8), tol.view(M, N // 16, 2, 8)
+        gate, up, tg, tu = (z.reshape(M, -1) for z in (v[:, :, 0], v[:, :, 1], t[:, :, 0], t[:, :, 1]))
+        act = torch.nn.functional.silu(gate) * up
+        assert ((y.double() - act).abs() <= 2.0 ** -8 * act.abs() + 1.1 * tg * up.abs() + (gate.abs() + tg) * tu + 1e-5).all()
+
+
+def test_what_is_refused():
+    nat = ops.native()
+    for M, K, splits, bn in ((0, 2048, 1, 64), (9, 2048, 1, 64), (8, 4096 + 64, 1, 64), (6, 288, 1, 64), (6, 2048, 3, 64), (6, 2048, 1, 96)):
+        assert not nat.norm_rows_ok(M, 192, K, splits, bn)
+    for M, N, K, ldx, grp in ((9, 64, 512, 512, 1), (5, 64, 128, 128, 1), (5, 64, 544, 544, 1), (5, 72, 512, 512, 1), (5, 64, 512, 516, 1),
+                              (5, 64, 512, 512, 8)):
+        assert not nat.rows_stream_ok(M, N, K, ldx, grp)
+
+
+@pytest.mark.parametrize("B", [1, 4, 5, 8, 9])
+def test_decode_steps(B, monkeypatch):
+    """A model whose layers are of the sizes: against the steps that sum slabs, and the fp32 reference."""
+    cfg = dataclasses.replace(decoder_config("tiny-llama"), hidden=1024, intermediate=2048, heads=16, kv_heads=8, layers=2)
+    w32 = random_decoder_weights(cfg, dtype=torch.float32, seed=5, interleave_mlp=True)
+    model = LlamaModel(cfg, {k: v.to(torch.bfloat16) for k, v in w32.items()}, DEV, interleaved_mlp=True)
+    ref = LlamaModel(cfg, {k: v.bfloat16().float() for k, v in w32.items()}, "cpu", interleaved_mlp=True)
+    bs, g = 64, torch.Generator().manual_seed(B)
+    ids = torch.randint(0, cfg.vocab_size, (B,), generator=g, dtype=torch.int32)
+    ctx = torch.randint(1, 4 * bs, (B,), generator=g, dtype=torch.int32)
+    tables = torch.arange(4 * B, dtype=torch.int32).view(B, 4)
+    pos = ctx - 1
+    slots = tables[torch.arange(B), (pos // bs).long()].long() * bs + pos % bs
+    old = torch.randn(cfg.layers, 4 * B, cfg.kv_heads, bs, cfg.head_dim, generator=g).bfloat16()
+
+    def step(m, dev, dtype):
+        kv = m.make_cache(4 * B, bs)
+        kv.k.copy_(old.to(dtype)), kv.v.copy_(old.flip(1).to(dtype))
+        ws = dict(workspace=m.make_workspace(B, 4 * bs, 512), part_size=512, max_len=4 * bs) if dev == DEV else {}
+        meta = AttnMeta(decode=True, positions=pos.to(dev), slots=slots.to(dev), block_tables=tables.to(dev), ctx_lens=ctx.to(dev), **ws)
+        return m.forward(ids.to(dev), meta, kv).float().cpu()
+
+    calls, orig = [], ops.rows_stream
+    monkeypatch.setattr(ops, "rows_stream", lambda *a: calls.append(1) or orig(*a))
+    got = step(model, DEV, torch.bfloat16)
+    assert len(calls) == (2 * cfg.layers if B <= 8 else 0)
+    monkeypatch.setattr(LlamaModel, "ROWS_MAX_M", 0)
+    torch.testing.assert_close(got, step(model, DEV, torch.bfloat16), atol=6e-2, rtol=5e-2)
+    assert len(calls) == (2 * cfg.layers if B <= 8 else 0)
+    assert (got - step(ref, "cpu", torch.float32)).abs().max().item() < 0.15
