@@ -57,6 +57,7 @@ struct G256 {
   long lda, ldb, ldc, ldr;
   int gm;  // tile rows per group of the grouped tile order
   int cn;  // tile columns per block of it
+  int tail;  // tile columns that the last row of tiles has (the others: all)
   int rows_b;  // SHUF: rows of the B copy (>= N)
   int bgrp;    // SHUF: row blocks per group of the B copy, 1 or 8 (shuffle_weights(w, 8))
   // G_CAND (index threshold search, see gemm.hip EPI_CANDIDATES): filtered scores >= thr[m] are
@@ -132,6 +133,17 @@ __device__ __forceinline__ void tile_of(int sid, int tiles_m, int tiles_n, int G
   n0 = (first_n + inner / gsz) << 8;
 }
 
+// ... of all rows of tiles over the first `tail` columns, and behind them of all but the last row over the others
+__device__ __forceinline__ void tile_of(int sid, int tiles_m, int tiles_n, int tail, int GM, int CN, int& m0, int& n0) {
+  const int first = tiles_m * tail;
+  if (sid < first) {
+    tile_of(sid, tiles_m, tail, GM, CN, m0, n0);
+  } else {
+    tile_of(sid - first, tiles_m - 1, tiles_n - tail, GM, CN, m0, n0);
+    n0 += tail << 8;
+  }
+}
+
 template <int EPI, bool BIAS, bool RES, bool SHUF = false, bool STAMP = false, int SAUX = 0>
 __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
   __shared__ __attribute__((aligned(16))) char smem[2 * kBuf + (EPI == G_CAND ? kCandExtra : 0)];
@@ -144,7 +156,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
   // workgroups of chunk x take ids cstart + l, cstart + l + nper, ... -> at any time the ~32
   // workgroups of one XCD run consecutive (grouped) tiles that share A / B panels in its L2.
   const int tiles_m = (p.M + 255) >> 8, tiles_n = EPI == G_CAND ? (p.N + 255) >> 8 : p.N >> 8;
-  const int nwg = tiles_m * tiles_n;
+  const int tail = EPI == G_CAND ? tiles_n : p.tail;
+  const int nwg = (tiles_m - 1) * tiles_n + tail;
   const int G = gridDim.x, bid = blockIdx.x;
   const int x = bid & 7, l = bid >> 3;
   const int nper = (G >> 3) + (x < (G & 7) ? 1 : 0);
@@ -154,7 +167,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
   int sid = cstart + l;
   if (sid >= cend) return;  // whole workgroup: uniform
   int m0, n0;
-  tile_of(sid, tiles_m, tiles_n, p.gm, p.cn, m0, n0);
+  tile_of(sid, tiles_m, tiles_n, tail, p.gm, p.cn, m0, n0);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -351,7 +364,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(G256 p) {
     const int nsid = sid + nper;
     const bool more = nsid < cend;
     int nm0 = m0, nn0 = n0;
-    if (more) tile_of(nsid, tiles_m, tiles_n, p.gm, p.cn, nm0, nn0);
+    if (more) tile_of(nsid, tiles_m, tiles_n, tail, p.gm, p.cn, nm0, nn0);
     const __amdgpu_buffer_rsrc_t nA = rsrc_a(nm0), nB = rsrc_b(nn0);
     // G_CAND: a tile whose rows 128-255 are all past M (97-128 queries, or the last row tile of a
     // larger batch) skips their MFMAs (the accumulators stay zero; their thresholds are +inf).
@@ -741,7 +754,7 @@ int gemm256_candidates(const void* A, long lda, const void* B, long ldb, int M, 
   p.lda = lda;
   p.ldb = ldb;
   p.gm = 4;
-  p.cn = (N + 255) / 256;
+  p.cn = p.tail = (N + 255) / 256;
   p.row_group = row_group;
   p.q_group = q_group;
   p.thr = thr;
@@ -775,7 +788,7 @@ int gemm256_candidates_stamped(const void* A, long lda, const void* B, int M, in
   p.lda = lda;
   p.ldb = K;
   p.gm = 4;
-  p.cn = (N + 255) / 256;
+  p.cn = p.tail = (N + 255) / 256;
   p.thr = thr;
   p.cnt = cnt;
   p.cand_val = cand_val;
@@ -814,7 +827,7 @@ int gemm256_stamped(const void* A, long lda, const void* B, void* C, const void*
   p.ldr = N;
   p.rows_b = N;
   p.gm = 4;
-  p.cn = (N + 255) / 256;
+  p.cn = p.tail = (N + 255) / 256;
   p.stamps = (u32x4*)stamps;
   p.stamp_tiles = stamp_tiles;
   int dev = 0, cus = 256;
@@ -862,9 +875,11 @@ bool gemm256_wins(int M, int N) {
 
 // b_shuf: B is in the shuffle_weights layout (ldb == K).  Epilogues: 0 none, 1 GELU, 2 SwiGLU over
 // 16-row [gate | up] groups, 4 / 6 SwiGLU / tanh-GELU GLU over 8-row groups (bias: fp32 [gate | up]); bias / residual optional.
+// tail > 0: the last row of tiles (of several) over its first `tail` columns of 256 only, the rest of it is not written.
 int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,
             const void* residual, long ldr, int M, int N, int K, int epilogue, hipStream_t s, int b_shuf,
-            int b_group) {
+            int b_group, int tail) {
+  if (tail < 0 || (tail && (tail > N / 256 || M <= 256))) return hipErrorInvalidValue;
   if (!gemm256_ok(M, N, K, lda, ldb)) return hipErrorInvalidValue;
   if (b_group != 1 && !(b_group == 8 && b_shuf)) return hipErrorInvalidValue;  // (N % 256: whole groups)
   if ((epilogue == G_SWIGLU || glu8_epilogue(epilogue)) && residual) return hipErrorInvalidValue;
@@ -886,7 +901,8 @@ int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc,
   p.bgrp = b_group;
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int tiles = ((M + 255) / 256) * (N / 256);
+  p.tail = tail ? tail : N / 256;
+  const int tiles = ((M + 255) / 256 - 1) * (N / 256) + p.tail;
   // Tile order.  Short K: A of half the Infinity Cache (256 MB) and more has left it when the projection starts, since its producer
   // moved as much again, and with a short K every K-tile is a first touch from HBM.  Blocks of 3 columns, 8 tile rows each,
   // keep some 11 row panels under way on an XCD instead of 4; the panels' second and third reads find them on the chip.  us

@@ -309,7 +309,7 @@ int gemm256_stamped(const void* A, long lda, const void* B, void* C, const void*
                     int N, int K, int epilogue, int b_shuf, void* stamps, int stamp_tiles, hipStream_t s, int store_aux);
 int gemm256(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,
             const void* residual, long ldr, int M, int N, int K, int epilogue, hipStream_t s, int b_shuf = 0,
-            int b_group = 1);
+            int b_group = 1, int tail = 0);
 
 // rows_stream.hip: X . W^T + residual of up to 8 decode rows, K whole in a workgroup
 int rows_stream_ok(int M, int N, int K, long ldx, int w_group);

@@ -526,7 +526,14 @@ def _frag_plan(M: int, N: int, K: int, cols: bool, frag: bool):
             if us < least:
                 plan, took, least = (("256", 256 * m1, N), (kind, M - 256 * m1, N)), us, us
     us = native().frag_us(M, N, K, 1) if frag else float("inf")
-    return ((("frag", M, N), None), us) if us < 0.93 * took else (plan, took)
+    if us < 0.93 * took:
+        return (("frag", M, N), None), us
+    if frag and plan[1] is not None:  # the same division with gemm_frag behind the waves
+        kind, m, n = plan[1]
+        mid, us = _mid(m, n // 256, K)[0], native().frag_us(max(m, 65), n, K, 1)
+        if us < 0.93 * mid:
+            return (plan[0], ("frag", m, n)), took - mid + us
+    return plan, took
 
 
 def frag_plan(M: int, N: int, K: int, cols: bool = True, frag: bool = True):
@@ -548,8 +555,37 @@ def frag_plan(M: int, N: int, K: int, cols: bool = True, frag: bool = True):
     8192, 1024) 21.3 -> 22.0 and (1093, 4096, 1024) 22.4 -> 23.1.
 
     gemm_frag, whole, where its estimate is 7 % below: over M 96..2300 at 19 pairs of N 1024..28,672 and K 1024..14,336 that
-    is 236 of 414 sizes, 1.64 times as fast in the mean, none slower (at 4 % below two of 271 are 7-9 % slower)."""
+    is 236 of 414 sizes, 1.64 times as fast in the mean, none slower (at 4 % below two of 271 are 7-9 % slower).  Behind whole
+    waves of gemm256 in gemm_mid's place by the same line, where the product is divided without it, too (a call of Llama-3.2-1B,
+    1,200 tokens 3,451 -> 3,391, 2,300 4,980 -> 4,870; where it alone makes the division pay, 1,300 tokens 3,497 -> 3,659)."""
     return _frag_plan(M, N, K, cols, frag)[0]
+
+
+@functools.lru_cache(maxsize=4096)
+def corner_plan(M: int, N: int, K: int):
+    """(tile columns of 256 that gemm256 takes of the prompt's last rows, the estimate), or (0, None): all it takes of a product
+    are whole waves of tiles, and gemm_frag what is left of the last row of them, where that is 1.5 % quicker by the estimates than
+    ``frag_plan``.  The last rows are up to 256, often few; a tile of them takes as long as any.  us: (1093, 28672, 4096) GLU 234 ->
+    219, (1600, 28672, 4096) 306 -> 285, (3333, 28672, 4096) 599 -> 552, (2760, 6144, 4096) 116 -> 104; a call of Llama-3-8B, 1,093
+    tokens 15,890 -> 15,700, 1,600 21,214 -> 20,604, 2,400 27,957 -> 27,536, 3,332 38,536 -> 37,416; as before (0.997-1.003) at
+    1,000, 4,000 and 7,900.  Left: (640, 28672, 4096), 80 of 336 tiles, alone 145 -> 135, but a call 10,775 -> 10,878."""
+    tm, tn = -(-M // 256), N // 256
+    waves = tm * tn // 256
+    left = tm * tn - 256 * waves
+    if tm < 2 or not waves or not 0 < left < tn or not native().gemm256_ok(M, N, K, K, K):
+        return 0, None
+    # (its weights, which gemm256 has read already, come from memory again, and slower than a projection's: 3.5 TB/s in calls)
+    us = _g256_us(256 * waves, K) + max(native().frag_us(max(M - 256 * (tm - 1), 65), 256 * left, K, 1), 3 + 512 * left * K / 3.5e6)
+    return (tn - left, us) if us < 0.985 * _frag_plan(M, N, K, True, True)[1] else (0, None)
+
+
+def _run_corner(tail: int, A, B, out, residual, epilogue, b_group):
+    """gemm256's whole waves and gemm_frag's corner behind them (``corner_plan``)."""
+    m, n = (A.shape[0] - 1) // 256 * 256, 256 * tail
+    _gemm256_into(A, B, out, None, residual, epilogue, True, b_group, tail)
+    gemm_frag(A[m:], B[n:], residual=None if residual is None else residual[m:, n:], epilogue=epilogue,
+              out=out[m:, n // (2 if epilogue in GLU8 else 1):], b_group=b_group)
+    return out
 
 
 @functools.lru_cache(maxsize=4096)
@@ -558,7 +594,7 @@ def frag_slices(M: int, N: int, K: int) -> int:
     is the quicker.  The norm reads them at some 4.5 TB/s.  us of product and norm, whole on the quickest kernel -> in slices:
     (260, 2048, 8192) 33.5 -> 23.8, (515, 2048, 8192) 39.8 -> 35.6, (140, 4096, 14336) 57 -> 39.7, (260, 4096, 14336) 62.6 ->
     55.4; (1093, 2048, 8192) 57.4 -> 53.1."""
-    whole = _frag_plan(M, N, K, True, True)[1]
+    whole = corner_plan(M, N, K)[1] or _frag_plan(M, N, K, True, True)[1]
     best, least = 0, 0.95 * whole
     for s in (2, 3, 4, 6, 8):
         us = native().frag_us(M, N, K, s) + 0.7 + 4 * s * M * N / 4.5e6 if K // 64 >= 4 * s else float("inf")
@@ -708,7 +744,12 @@ def gemm_bt(A, B, bias=None, residual=None, epilogue=EPI_NONE, out_f32=False, ro
     plain = not out_f32 and row_group is None and q_group is None and allow is None
     if plain and shuffled and N == B.shape[0] and bias is None and epilogue in (EPI_NONE, *GLU8) and N % 256 == 0:
         lda = A.stride(0)
-        plan = (frag_plan(M, N, K, glu_bias is None, _frag_takes(A, B, out, residual, glu_bias))
+        frag = _frag_takes(A, B, out, residual, glu_bias)
+        if frag and glu_bias is None and M > 256 and native().gemm256_ok(M, N, K, lda, K):
+            tail = corner_plan(M, N, K)[0]
+            if tail:
+                return _run_corner(tail, A, B, out, residual, epilogue, b_group)
+        plan = (frag_plan(M, N, K, glu_bias is None, frag)
                 if M >= GEMM_MID_MIN_M and native().gemm256_ok(M, N, K, lda, K) else None)
         if plan is not None and all(q is None or q[0] not in ("mid", "192") or gemm_mid_ok(q[1], q[2], K, lda) for q in plan):
             return _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias)
@@ -740,11 +781,12 @@ def _glu_bias(glu_bias, epilogue, N: int) -> None:
                "glu_bias: fp32 [gate | up] of a GLU8 epilogue")
 
 
-def _gemm256_into(A, B, out, bias, residual, epilogue, shuffled, b_group=1):
+def _gemm256_into(A, B, out, bias, residual, epilogue, shuffled, b_group=1, tail: int = 0):
+    """``tail`` > 0: the last 256 rows' tiles over so many columns of 256 only."""
     M, K = A.shape
     native().gemm256(ptr(A), A.stride(0), ptr(B), B.stride(0), ptr(out), out.stride(0), ptr(bias), ptr(residual),
                      residual.stride(0) if residual is not None else 0, M, B.shape[0], K, int(epilogue), stream(A),
-                     int(shuffled), int(b_group))
+                     int(shuffled), int(b_group), int(tail))
     return out
 
 
