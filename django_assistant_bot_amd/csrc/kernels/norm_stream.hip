@@ -14,7 +14,7 @@
 // 12.9; gated (1, 28672, 4096) 43.0 -> 40.1, 4 rows 43.8 -> 41.8; (1, 3072, 2048) 7.9 -> 6.3, 4 rows 8.2 -> 7.0; gated (1,
 // 16384, 2048) 16.9 -> 15.5, 4 rows 16.9 -> 16.3.  5-8 rows, a wave each: (5, 3072, 2048) 8.2 -> 9.5, not taken of slabs.
 // Complete rows (norm_rows; rows_stream.hip leaves them), up to 8, are one read each: 6 rows, norm launch and stream_gemm ->
-// here, gated (28672, 4096) 42.4 -> 37.5, (6144, 4096) 16.4 -> 12.2, gated (16384, 2048) 18.5 -> 15.0, (3072, 2048) 10.5 -> 5.9.
+// here, gated (28672, 4096) 42.4 -> 36.3, (6144, 4096) 16.4 -> 10.6, gated (16384, 2048) 18.5 -> 14.2, (3072, 2048) 10.5 -> 4.4.
 //
 // Weights: wave w of the tile's NWC compute waves holds RT 16-row blocks; a chunk is 32 k of them, 1 KB a block, MFMA A
 // fragments straight to registers through a ring of DEP chunks (128 KB in flight a CU).  The rows are the B operand, in
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(64 * (NWC + kNormWaves), 1) void norm_stream_kernel
     for (int a = 0; a < RT; ++a) acc[a][j & 1] = mfma16(wr[j][a], x, acc[a][j & 1]);
   };
   int c0 = 0;
-  for (; c0 + DEP <= nch; c0 += DEP) {
+  for (; c0 + DEP < nch; c0 += DEP) {
 #pragma unroll
     for (int j = 0; j < DEP; ++j) {
       step(j, c0 + j);
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(64 * (NWC + kNormWaves), 1) void norm_stream_kernel
     }
   }
 #pragma unroll
-  for (int j = 0; j < DEP - 1; ++j)
+  for (int j = 0; j < DEP; ++j)
     if (c0 + j < nch) step(j, c0 + j);
 
   // acc[a]: weight rows 16 (RT w + a) + 4 g + r of column (row of X) li
@@ -304,10 +304,15 @@ int norm_stream(const void* slabs, int S, int slabs_f32, const void* residual, c
 }
 
 // ... of up to 8 complete rows (no slabs, no residual); with more than 4 a norm wave each.  Slices of whole eights of 16-B
-// pieces, in which the rows are permuted.
+// pieces, in which the rows are permuted.  bn: 48, 64 or 128 weight rows a workgroup, a compute wave for 16.
+//
+// With the rows read once the ring need not cover the norm's reads of slabs, and short ones are quicker; 48 rows find 256 CUs
+// work where 64 find 192.  us, 6 rows, 4 waves with rings of 32 or, gated, 16 chunks of two blocks -> rings of 8: (6144, 4096) in
+// two slices 12.3 -> 11.4 on 64 rows, 10.7 on 48, (3072, 2048) in four 5.9 -> 5.0, 4.4; gated (28672, 4096) 37.3 -> 36.4, (16384,
+// 2048) 15.0 -> 14.4 (one row 15.7 -> 13.7).  Gated on 64 rows 41.2 and 16.3.
 int norm_rows_ok(int M, int N, int K, int SO, int bn) {
-  return M >= 1 && M <= kNormWaves && norm_stream_ok(1, N, K, SO, bn) && K / SO % 64 == 0 && (long)M * (K / SO) * 2 <= kNormX &&
-         (long)SO * M * N * 4 < (1L << 31);
+  return M >= 1 && M <= kNormWaves && (bn == 48 || bn == 64 || bn == 128) && N > 0 && N % bn == 0 && K >= 256 && K <= 4096 && SO >= 1 &&
+         K % (64 * SO) == 0 && (long)M * (K / SO) * 2 <= kNormX && (long)SO * M * N * 4 < (1L << 31) && (long)N * K * 2 < (1L << 31);
 }
 
 int norm_rows(const void* x, const void* gain, float eps, const void* W, void* out, long ldo, int M, int N, int K, int SO, int out_f32,
@@ -316,20 +321,26 @@ int norm_rows(const void* x, const void* gain, float eps, const void* W, void* o
   if (w_group < 1 || N % (16 * w_group)) return hipErrorInvalidValue;
   const NormStream p = {x, 1, (long)M * K, nullptr, (const bf16*)gain, nullptr, eps, (const bf16*)W,
                         out, ldo, M, N, K, SO, K / SO, glu, out_f32, w_group};
-  const dim3 grid(N / bn * SO), block(64 * (4 + kNormWaves));
-#define NS_ROWS(WPR)                                                                                                          \
-  do {                                                                                                                        \
-    constexpr int few = (4 + WPR - 1) / WPR, more = 8 / WPR;                                                                  \
-    if (K <= 2048 && bn == 64) hipLaunchKernelGGL((norm_stream_kernel<1, 4, 32, WPR, few, 0, bf16>), grid, block, 0, s, p);   \
-    else if (K <= 2048) hipLaunchKernelGGL((norm_stream_kernel<2, 4, 16, WPR, few, 0, bf16>), grid, block, 0, s, p);          \
-    else if (bn == 64) hipLaunchKernelGGL((norm_stream_kernel<1, 4, 32, WPR, more, 0, bf16>), grid, block, 0, s, p);          \
-    else hipLaunchKernelGGL((norm_stream_kernel<2, 4, 16, WPR, more, 0, bf16>), grid, block, 0, s, p);                        \
+  const dim3 grid(N / bn * SO);
+#define NS_LAUNCH(NWC, WPR)                                                                                        \
+  do {                                                                                                             \
+    constexpr int few = (4 + WPR - 1) / WPR, more = 8 / WPR;                                                       \
+    const dim3 block(64 * (NWC + kNormWaves));                                                                     \
+    if (K <= 2048) hipLaunchKernelGGL((norm_stream_kernel<1, NWC, 8, WPR, few, 0, bf16>), grid, block, 0, s, p);   \
+    else hipLaunchKernelGGL((norm_stream_kernel<1, NWC, 8, WPR, more, 0, bf16>), grid, block, 0, s, p);            \
+  } while (0)
+#define NS_ROWS(WPR)                       \
+  do {                                     \
+    if (bn == 48) NS_LAUNCH(3, WPR);       \
+    else if (bn == 64) NS_LAUNCH(4, WPR);  \
+    else NS_LAUNCH(8, WPR);                \
   } while (0)
   if (M == 1) NS_ROWS(8);
   else if (M == 2) NS_ROWS(4);
   else if (M <= 4) NS_ROWS(2);
   else NS_ROWS(1);
 #undef NS_ROWS
+#undef NS_LAUNCH
   return hipGetLastError();
 }
 

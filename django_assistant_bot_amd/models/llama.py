@@ -356,8 +356,8 @@ class LlamaModel(FragmentProjections):
     def _rows(self, L: DecoderLayer, T: int) -> bool:
         """Whether a decode step of ``T`` sequences keeps the residual stream complete between its projections: o and down over
         the whole K (``ops.rows_stream``), the norms inside qkv and gate_up.  Up to 4 rows those summed slabs before, from 5 on norm
-        launches did.  us a step, slabs -> complete: Llama-3-8B 1 sequence of 1150 tokens 3028 -> 2917, 4 of 300-1700 3425 -> 3252, 6 of
-        200-900 3407 -> 3100, 8 of 300-1700 3602 -> 3376; Llama-3.2-1B 1 of 500 833 -> 781, 6 of 200-900 926 -> 815, 8 960 -> 856."""
+        launches did.  us a step, slabs -> complete: Llama-3-8B 1 sequence of 1150 tokens 3010 -> 2844, 4 of 300-1700 3370 -> 3168, 6 of
+        200-900 3465 -> 3137, 8 of 300-1700 3612 -> 3291; Llama-3.2-1B 1 of 500 848 -> 778, 6 of 200-900 943 -> 817, 8 976 -> 877."""
         if not (T <= self.ROWS_MAX_M and self.tp_size == 1 and self.interleaved_mlp):
             return False
         serves = self._rows_of.get(T)  # (the layers' shapes are one)

@@ -152,10 +152,14 @@ class FragmentProjections:
         y, new = ops.norm_stream(x, gain, eps, residual, w, splits=s, bn=bn, epilogue=epilogue, slab_dtype=sd, w_group=grp)
         return y, (x if residual is None else new)
 
+    def _rows_tile(self, w, gated: bool) -> tuple[int, int]:
+        """(weight rows a workgroup, K-slices) of ``ops.norm_rows``."""
+        bn = 128 if gated else 48 if w.shape[0] % 48 == 0 else 64
+        return bn, 1 if gated else self._stream_splits(*w.shape, bn)
+
     def _rows_proj(self, x, gain, eps: float, w, name: str, epilogue=ops.EPI_NONE):
         """``_norm_proj`` of up to 8 rows that are complete (the residual stream itself, as ``ops.rows_stream`` leaves it)."""
-        gated = epilogue != ops.EPI_NONE
-        bn, s = (128, 1) if gated else (64, self._stream_splits(w.shape[0], w.shape[1], 64))
+        bn, s = self._rows_tile(w, epilogue != ops.EPI_NONE)
         return ops.norm_rows(x, gain, eps, w, splits=s, bn=bn, epilogue=epilogue, w_group=self.proj_group.get(name, 1),
                              slab_dtype=torch.bfloat16 if self.slab_bf16 else torch.float32)
 
@@ -163,10 +167,11 @@ class FragmentProjections:
         """Whether a layer's projections of ``T`` rows all take ``_rows_proj`` and ``ops.rows_stream``."""
         nat, group = ops.native(), lambda name: self.proj_group.get(name, 1)
 
-        def normed(w, name, bn, s):
+        def normed(w, name, gated):
+            bn, s = self._rows_tile(w, gated)
             return w.shape[0] % (16 * group(name)) == 0 and nat.norm_rows_ok(T, *w.shape, s, bn)
 
-        return (self.frag and normed(qkv, "qkv", 64, self._stream_splits(*qkv.shape, 64)) and normed(gate_up, "gate_up", 128, 1)
+        return (self.frag and normed(qkv, "qkv", False) and normed(gate_up, "gate_up", True)
                 and all(nat.rows_stream_ok(T, *w.shape, w.shape[1], group(name)) for w, name in ((o, "o"), (down, "down"))))
 
     def _stream_or_tile(self, x, w, dec: bool, allow_slabs: bool, name: str, epilogue, grp: int, out=None, glu_bias=None):

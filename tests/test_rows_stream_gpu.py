@@ -42,7 +42,8 @@ def test_nothing_of_the_rows_behind_reaches_a_result():
 
 
 @pytest.mark.parametrize("N,K,splits,bn,grp", [(64, 256, 1, 64, 1), (128, 512, 8, 64, 8), (256, 2048, 4, 128, 8), (128, 2560, 1, 128, 1),
-                                               (640, 4096, 2, 64, 1), (256, 4096, 1, 128, 8)])
+                                               (640, 4096, 2, 64, 1), (256, 4096, 1, 128, 8), (48, 256, 1, 48, 1), (384, 2112, 1, 48, 8),
+                                               (96, 4096, 8, 48, 1)])
 @pytest.mark.parametrize("M", [1, 2, 3, 5, 7, 8])
 def test_norm_rows(N, K, splits, bn, grp, M):
     rand = _rand(N + K + M)
