@@ -452,8 +452,8 @@ static constexpr StreamCfg kStreamCfgs[] = {
     {8, 2, 2, 4, 4, 2, true},   // 9: = 2, shuffled weights
     {8, 2, 1, 4, 3, 4, true},   // 10: = 5, shuffled weights
     {8, 2, 2, 3, 6, 1, true},   // 11: M<=128 BN 64, 6-stage ring, shuffled
-    {4, 2, 2, 4, 4, 4, true},   // 12: = 7, shuffled weights
-    {4, 2, 1, 4, 4, 2, true},   // 13: = 8, shuffled weights
+    {4, 2, 2, 4, 3, 4, true},   // 12: = 7, shuffled weights, 3-stage weight ring
+    {4, 2, 1, 4, 3, 2, true},   // 13: = 8, shuffled weights, 3-stage weight ring
     {8, 2, 1, 4, 4, 4, true},   // 14: M<=128 BN 128, 4-stage ring, 4 loaders, shuffled
     {8, 2, 1, 4, 4, 2, true},   // 15: M<=128 BN 128, 4-stage ring, 2 loaders, shuffled
     {4, 2, 1, 4, 6, 4, true},   // 16: M<=64  BN 128, 6-stage ring, 4 loaders, shuffled
@@ -461,7 +461,7 @@ static constexpr StreamCfg kStreamCfgs[] = {
     {8, 2, 1, 4, 3, 4, true, 2},  // 18: = 10 without MFMA             (ablation, wrong results)
     {8, 2, 1, 4, 3, 4, true, 3},  // 19: = 10 weight stream only       (ablation, wrong results)
     // whole-chip tilings at M <= 128: BN = 16 x compute waves (one 16-row tile per wave)
-    {8, 1, 1, 4, 4, 2, true, 0, 7},  // 20: BN 112, 7 compute + 2 loader waves (gate_up 28672 -> 256 WGs)
+    {8, 1, 1, 4, 3, 2, true, 0, 7},  // 20: BN 112, 7 compute + 2 loader waves (gate_up 28672 -> 256 WGs)
     {8, 1, 1, 4, 4, 2, true, 0, 6},  // 21: BN 96, 6 + 2 waves (qkv 6144 x S4 -> 256 WGs)
     {8, 1, 1, 3, 6, 1, true, 0, 7},  // 22: = 20, 1 loader wave, 6-stage weight ring
     {8, 1, 1, 3, 6, 2, true, 0, 6},  // 23: = 21, 6-stage weight ring
@@ -476,8 +476,8 @@ static constexpr StreamCfg kStreamCfgs[] = {
     {8, 2, 1, 4, 2, 2, true, 0, 6},  // 29: = 28 with a 2-stage weight ring
     // M <= 16 (interactive decode, batch 1-16): one 16-row X tile per stage, a quarter of cfg 13's X
     // staging and MFMAs
-    {1, 2, 1, 4, 4, 2, true},  // 30: BN 128, 2 loaders
-    {2, 2, 1, 4, 4, 2, true},  // 31: M <= 32, BN 128, 2 loaders
+    {1, 2, 1, 4, 3, 2, true},  // 30: BN 128, 2 loaders
+    {2, 2, 1, 4, 3, 2, true},  // 31: M <= 32, BN 128, 2 loaders
     // M <= 16, whole-K producers of the residual stream (o / down with the residual add, no split-K
     // slabs, so the consumer can normalise X itself): 16 / 32 weight rows per workgroup, an 8-stage
     // weight ring per compute wave
@@ -498,12 +498,24 @@ static constexpr StreamCfg kStreamCfgs[] = {
     {8, 1, 1, 4, 6, 2, true, 0, 7},  // 41: 6-stage weight ring
     {8, 1, 1, 3, 8, 1, true, 0, 7},  // 42: 8-stage weight ring, 1 loader wave
     // M <= 16 / 32 with 64 weight rows: the small projections fill the chip with half the K-slices (half the slabs for
-    // their consumers), unsplit ones below 192 tiles of 128 with all of its CUs.  us, BN 128 -> 64 at M 6: (4096, 4096) 9.7
+    // their consumers), unsplit ones below 192 tiles of 128 with all of its CUs.  us, BN 128 -> 64 at M 6 (both with longer weight rings): (4096, 4096) 9.7
     // -> 9.0, (6144, 4096) 11.7 -> 11.4, gated (16384, 2048) 15.5 -> 13.4, (2048, 2048) 5.4 -> 4.7, (2048, 8192) 9.7 -> 8.8;
     // not gated (28672, 4096), 224 tiles of 128: 36.8 -> 38.9.  (BN 96 and 112, 256 workgroups of 6 and 7 waves: slower.)
-    {1, 1, 1, 4, 8, 2, true, 0, 4},  // 43: M <= 16
-    {2, 1, 1, 4, 8, 2, true, 0, 4},  // 44: M <= 32
+    {1, 1, 1, 4, 3, 2, true, 0, 4},  // 43: M <= 16
+    {2, 1, 1, 4, 3, 2, true, 0, 4},  // 44: M <= 32
+    // The weight rings of 12, 13, 20, 30, 31, 43 and 44 are as short as they can be: what is in flight ahead of the first stage
+    // delays it, and the stages that a ring asks for past the slice's end (the last one again) are traffic of the same CU,
+    // with 8 of 16 a third of it.  us of 8 stages (43, 44) or 4 -> 3: 6 rows (6144, 4096) 11.5 -> 10.2, (4096, 4096) 8.9 ->
+    // 7.6, (4096, 14336) 20.5 -> 19.8, gated (28672, 4096) 37.6 -> 36.4; 32 rows (6144, 4096) 12.3 -> 11.2, (4096, 4096) 9.5 ->
+    // 7.9, (4096, 14336) 21.3 -> 20.4, (2048, 8192) 9.6 -> 7.9, gated (28672, 4096) 38.7 -> 37.7, (16384, 2048) 14.4 -> 12.7; 64 rows
+    // (4096, 14336) 22.6 -> 22.0, LM head (128256, 4096) 197 -> 192; 128 rows gated (28672, 4096) 49.4 -> 48.5 (at 65-128 rows the
+    // others' 2 stages of 128 rows gain and lose: (4096, 4096) 12.0 -> 11.5, (3072, 2048) 7.9 -> 8.5).  Two stages are as good up
+    // to 32 rows but for an LM head (31: 177 -> 190).
+    // An LM head of many tiles on 43 keeps 8: (128256, 4096) 161 -> 166 with 3.
+    {1, 1, 1, 4, 8, 2, true, 0, 4},  // 45: 43's tile where the workgroups are many
+    {4, 2, 2, 4, 4, 4, true},        // 46: 12's, for candidates
 };
+constexpr int kStreamMany = 45, kStreamManyFor = 43;  // from 512 workgroups on
 constexpr int kNumStreamCfgs = sizeof(kStreamCfgs) / sizeof(kStreamCfgs[0]);
 
 template <int C>
@@ -584,7 +596,7 @@ int stream_gemm(const void* X, long ldx, const void* W, long ldw, void* out, lon
   if (p.wgrp > 1 && (!kStreamCfgs[cfg].shuf || N % (16 * p.wgrp) || (long)N * K * 2 >= (1L << 31)))
     return hipErrorInvalidValue;
   if (p.norm && (residual || K % 8 || M > stream_gemm_max_m(cfg))) return hipErrorInvalidValue;
-  launch_any(cfg, p, s, nt_weights != 0);
+  launch_any(cfg == kStreamManyFor && (long)N / bn * S >= 512 ? kStreamMany : cfg, p, s, nt_weights != 0);
   return hipGetLastError();
 }
 
@@ -634,9 +646,9 @@ static int stream_candidates_launch(bool shuf, const void* X, long ldx, const vo
                                     const int* row_group, const int* q_group, const float* thr, int* cnt,
                                     float* cand_val, int* cand_idx, int cap, hipStream_t s) {
   constexpr int KS = 128;
-  // M <= 64, BN 64, 4 loader waves: row-major rows (cfg 7) or a shuffle_weights copy (cfg 12);
+  // M <= 64, BN 64, 4 loader waves: row-major rows (cfg 7) or a shuffle_weights copy (cfg 46);
   // M <= 128 (shuffled copy only): BN 128 (cfg 10, the decode GEMM's)
-  const int CFG = shuf ? (M > 64 ? 10 : 12) : 7;
+  const int CFG = shuf ? (M > 64 ? 10 : 46) : 7;
   if (M <= 0 || N <= 0) return 0;
   if (M > stream_gemm_max_m(CFG) || K % KS || ldx % 8 || ldw % 8 || cap <= 0) return hipErrorInvalidValue;
   if ((long)stream_gemm_bn(CFG) * ldw * 2 >= (1L << 31)) return hipErrorInvalidValue;
@@ -661,8 +673,8 @@ static int stream_candidates_launch(bool shuf, const void* X, long ldx, const vo
   p.cap = cap;
   if (CFG == 10)
     launch_cfg<10>(p, s, true);
-  else if (CFG == 12)
-    launch_cfg<12>(p, s, true);
+  else if (CFG == 46)
+    launch_cfg<46>(p, s, true);
   else
     launch_cfg<7>(p, s, true);
   return hipGetLastError();

@@ -28,7 +28,8 @@ class FragmentProjections:
     # stream_gemm.hip configurations (shuffled weights): BN 128 rows per workgroup at M <= 64 (13)
     # and M <= 128 (10).  Whole-chip tilings at M 65..128: gate_up's 28672 rows / 112 make exactly
     # 256 workgroups where BN 128 left 32 of the 256 CUs idle (cfg 20: 54.9 -> 51.5 us cold); the LM
-    # head uses 192-row tiles (cfg 28: 2/3 of the X staging per weight byte, 228.7 -> 221.3 us).
+    # head uses 192-row tiles (cfg 28: 2/3 of the X staging per weight byte, 228.7 -> 221.3 us; 29, its shorter ring: 96 rows of
+    # (128256, 4096) 213.7 -> 211.0, of (128256, 2048) 114.3 -> 111.6, 128 rows 221.7 -> 220.9 and 119.3 -> 115.8).
     # qkv at 96 rows x 4 K-slices (cfg 21) measured slower than BN 128 x 4 (17.1 vs 15.8 us).
     # Decode batches of 129..256 rows: 64-row tiles, 2 k-groups x 4 row groups (cfg 27; M = 256:
     # qkv 27.4 / o 18.6 / gate_up 98.7 / down 49.2 us against 32.4 / 25.8 / 104 / 55 for two
@@ -37,7 +38,7 @@ class FragmentProjections:
     STREAM_NARROW = {30: 43, 31: 44, 13: 12}
     STREAM_GATE_NARROW = 9
     STREAM_CFG_M16, STREAM_CFG_M32, STREAM_CFG_M64, STREAM_CFG_M128, STREAM_CFG_M256 = 30, 31, 13, 10, 27
-    STREAM_WIDE = {"gate_up": 20, "lm_head": 28}
+    STREAM_WIDE = {"gate_up": 20, "lm_head": 29}
     STREAM_MAX_M = ops.STREAM_MAX_M
     PREFILL_STREAM_MAX_M = 128  # prefill steps of at most this many tokens stream too (0: off)
 
