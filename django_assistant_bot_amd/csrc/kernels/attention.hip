@@ -2187,6 +2187,11 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
       return gt;
     };
     const size_t hq0 = (size_t)b * p.Hq + hk * G;
+    // The partial sums of the key head's group, with heads of 128 16 bytes at a time (as four dwords each a step of Llama-3-8B
+    // takes 2837 instead of 2814 us at one sequence, 3610 instead of 3585 at 12; heads of 64 gain at 20 sequences and lose at 6).
+    auto parts_of = [&]() __attribute__((always_inline)) {
+      return __builtin_amdgcn_make_buffer_rsrc(p.part_o + hq0 * p.max_parts * D, 0, G * p.max_parts * D * 4, 0x00020000);
+    };
     for (int e = tid; e < G * (D / 4); e += 256) {
       const int qh = e / (D / 4), d = 4 * (e % (D / 4));
       const f32x4 gate = direct ? gate4(qh, d) : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -2207,9 +2212,12 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
         const size_t pi = (hq0 + qh) * p.max_parts + part;
         // write-through (sc1) stores: visible to the combining workgroup on any XCD without a
         // release fence (cdna_hip_programming.md Guideline 16, R1)
+        if constexpr (D == 128)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O), parts_of(), ((qh * p.max_parts + part) * D + d) * 4, 0, 16);
+        else
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          __hip_atomic_store(p.part_o + pi * D + d + j, O[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int j = 0; j < 4; ++j)
+            __hip_atomic_store(p.part_o + pi * D + d + j, O[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (d == 0) {
           __hip_atomic_store(p.part_m + pi, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_store(p.part_l + pi, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2235,6 +2243,7 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
       if (*last_flag) {
         auto ld = [](const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
         constexpr int NPF = kCombine;
+        const auto parts = parts_of();
         for (int e = tid; e < G * (D / 4); e += 256) {
           const int qh = e / (D / 4), d = 4 * (e % (D / 4));
           const f32x4 gate = gate4(qh, d);
@@ -2246,11 +2255,15 @@ __global__ __launch_bounds__(256, NSLOT == 1 ? 2 : 1) void paged_decode_kernel(D
             f32x4 po[NPF];
 #pragma unroll
             for (int i = 0; i < NPF; ++i) {
-              const size_t pi = base + min(i0 + i, np - 1);
-              pm[i] = ld(p.part_m + pi);
-              pl[i] = ld(p.part_l + pi);
+              const int at = min(i0 + i, np - 1);
+              pm[i] = ld(p.part_m + base + at);
+              pl[i] = ld(p.part_l + base + at);
+              if constexpr (D == 128)
+                po[i] = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(parts, ((qh * p.max_parts + at) * D + d) * 4, 0, 16));
+              else
 #pragma unroll
-              for (int j = 0; j < 4; ++j) po[i][j] = ld(p.part_o + pi * D + d + j);
+                for (int j = 0; j < 4; ++j) po[i][j] = ld(p.part_o + (base + at) * D + d + j);
             }
             float M2 = M;
 #pragma unroll
