@@ -100,19 +100,26 @@ class VectorIndex:
 
     def add(self, ids, vectors, doc_ids=None, groups=None) -> None:
         """Upsert rows.  ids: int64 [n]; vectors [n, dim] (any float dtype / device); doc_ids int64 [n]
-        (document each row belongs to); groups int32 [n] (e.g. bot id; must be >= 0)."""
+        (document each row belongs to); groups int32 [n] (e.g. bot id; must be >= 0), or one value for all rows.  What is
+        refused leaves the index as it was."""
         ids = np.asarray(ids, dtype=np.int64).reshape(-1)
         n = len(ids)
         if n == 0:
             return
         v = torch.as_tensor(vectors).to(self.device, torch.float32).reshape(n, self.dim)
         v = F.normalize(v, dim=-1).to(self.dtype)
-        docs = np.full(n, -1, dtype=np.int64) if doc_ids is None else np.asarray(doc_ids, dtype=np.int64)
-        grp = np.zeros(n, dtype=np.int32) if groups is None else np.asarray(groups, dtype=np.int32)
+
+        def per_row(a):
+            if a.ndim > 1 and a.size == a.shape[-1]:
+                a = a.reshape(-1)
+            return a if a.shape == (n,) else np.broadcast_to(a, (n,)).copy()
+        docs = per_row(np.asarray(-1 if doc_ids is None else doc_ids, dtype=np.int64))
+        grp = per_row(np.asarray(0 if groups is None else groups, dtype=np.int32))
         if (grp < 0).any():
             raise ValueError("groups must be >= 0 (negative marks deleted rows)")
         idl = ids.tolist()
-        if len(set(idl)) == n and not (self._row_of.keys() & set(idl)):
+        distinct = set(idl)
+        if len(distinct) == n and not (self._row_of.keys() & distinct):
             # bulk insert of new ids (ingest): C-speed bookkeeping, contiguous rows
             if self.n + n > self._cap:
                 self._grow(max(self.n + n, 2 * self._cap))
@@ -138,7 +145,7 @@ class VectorIndex:
                     rows[i] = self.n + j
                     self._row_of[idl[i]] = self.n + j
                 self.n += len(fresh)
-            last = dict(zip(rows.tolist(), range(n)))
+            last = dict(zip(rows.tolist(), range(n))) if len(distinct) < n else rows
             if len(last) < n:  # an id of the index named twice: its later vector (writes to one row in one launch have no order)
                 at = np.sort(np.fromiter(last.values(), dtype=np.int64, count=len(last)))
                 rows, ids, docs, grp, v = rows[at], ids[at], docs[at], grp[at], v[torch.from_numpy(at).to(self.device)]

@@ -24,6 +24,35 @@ def _check(device, dim, monkeypatch):
     assert ids.tolist() == [[7]]
 
 
+# ids of the index and new ones, with and without an id that is named twice
+@pytest.mark.parametrize("ids", [[1, 3, 1], [3, 4, 3], [1, 3, 4], [3, 4, 5]])
+@pytest.mark.parametrize("name", ["doc_ids", "groups"])
+def test_one_value_for_all_rows(ids, name):
+    for one in (5, [5], np.array([[5]])):
+        idx = VectorIndex(32, "cpu", capacity=4)
+        idx.add([1, 2], torch.eye(32)[:2])
+        idx.add(ids, torch.eye(32)[2:5], **{name: one})
+        kept = idx.row_docs if name == "doc_ids" else idx.row_group
+        for i, item in enumerate(ids):
+            row = int(idx.rows_of([item])[0])
+            assert int(kept[row]) == 5
+            if item not in ids[i + 1:]:
+                assert torch.equal(idx.rows_data([row])[0].float(), torch.eye(32)[2 + i])
+        assert len(idx) == 2 + len(set(ids) - {1, 2})
+
+
+@pytest.mark.parametrize("ids", [[1, 3, 1], [3, 4, 3], [1, 3, 4], [3, 4, 5]])
+@pytest.mark.parametrize("name", ["doc_ids", "groups"])
+@pytest.mark.parametrize("bad", [[1, 2], [1, 2, 3, 4], [[1], [2], [3]]])
+def test_what_is_refused_changes_nothing(ids, name, bad):
+    idx = VectorIndex(32, "cpu", capacity=4)
+    idx.add([1, 2], torch.eye(32)[:2], doc_ids=7)
+    with pytest.raises((ValueError, RuntimeError)):
+        idx.add(ids, torch.eye(32)[2:5], **{name: bad})
+    assert len(idx) == idx.n == 2 and idx.search(torch.eye(32)[1], 2)[1].tolist() == [[2, 1]]
+    assert idx.row_docs[:2].tolist() == [7, 7] and torch.equal(idx.rows_data([0, 1]).float(), torch.eye(32)[:2])
+
+
 def test_a_row_is_written_once(monkeypatch):
     _check("cpu", 32, monkeypatch)
 
