@@ -990,13 +990,18 @@ def selected_search(x, vecs, rows: int, row_group, row_ids, row_docs, k: int, gr
     nat = native()
     expect(x.is_cuda and x.dtype == torch.float32 and vecs.dtype == torch.bfloat16 and vecs.is_contiguous() and vecs.shape[1] == K
            and vecs.shape[0] % 16 == 0 and vecs.shape[0] >= -(-n // 128) * 128, "selected_search: fp32 [q, K] and a shuffled copy [R, K]")
+    there, i64 = x.get_device(), torch.int64
+    expect(vecs.get_device() == there and row_group.get_device() == there and row_group.dtype == torch.int32 and row_group.is_contiguous()
+           and row_ids.get_device() == there and row_ids.dtype == i64 and row_ids.is_contiguous()
+           and row_docs.get_device() == there and row_docs.dtype == i64 and row_docs.is_contiguous(),
+           "selected_search: contiguous int32 groups, int64 row ids and documents, on the queries' device")
     expect(scan_scores_ok(M, n, K) and 1 <= k <= min(n, 1024) and row_group.data_ptr() % 16 == 0
            and min(row_group.numel(), row_ids.numel(), row_docs.numel()) >= n, "selected_search: the scan's shapes, rows' groups and ids")
     expect(groups is None or (not groups.is_cuda and groups.dtype == torch.int32 and groups.dim() == 1 and groups.is_contiguous()
                               and groups.numel() >= M), "q_group shorter than M")
     ids, offsets, longest, keys, key_rows = lists if lists is not None else (None, None, 0, None, None)
     for t in (ids, offsets, keys, key_rows) if lists is not None else ():
-        expect(t.is_cuda and t.dtype == torch.int64 and t.is_contiguous(), "allow lists: contiguous CUDA int64 tensors")
+        expect(t.get_device() == there and t.dtype == i64 and t.is_contiguous(), "allow lists: contiguous CUDA int64 tensors")
     expect(lists is None or (offsets.numel() == M + 1 and keys.numel() == key_rows.numel()), "allow lists: one a query")
     expect(limits is None or (not limits.is_cuda and limits.dtype == torch.int64 and limits.is_contiguous() and limits.shape == (M,)),
            "limits: int64 of the host, one a query")

@@ -119,6 +119,19 @@ def test_one_call_is_its_launches(rows, dim, queries):
             assert torch.equal(got, exp)
 
 
+def test_one_call_refuses_rows_that_its_launches_would_not_take():
+    frag, x = torch.zeros(128, 256, dtype=torch.bfloat16, device=DEV), torch.zeros(2, 256, device=DEV)
+    group, ids = torch.zeros(8, dtype=torch.int32, device=DEV), torch.zeros(8, dtype=torch.int64, device=DEV)
+    wide = torch.zeros(8, 2, dtype=torch.int64, device=DEV)[:, 0]
+    two = torch.zeros(3, dtype=torch.int64, device=DEV)
+    for bad in (dict(row_group=ids), dict(row_group=wide.to(torch.int32).repeat_interleave(2)[::2]), dict(row_group=group.float()),
+                dict(row_group=group.cpu()), dict(row_ids=group), dict(row_ids=wide), dict(row_ids=ids.cpu()), dict(row_docs=group),
+                dict(row_docs=wide), dict(row_docs=ids.double()), dict(row_docs=ids.cpu()), dict(vecs=frag.cpu()),
+                dict(lists=(ids, two, 1, ids, ids.cpu())), dict(lists=(ids.cpu(), two, 1, ids, ids)), dict(lists=(ids, two, 1, ids, group))):
+        with pytest.raises((ValueError, TypeError)):
+            ops.selected_search(**{**dict(x=x, vecs=frag, rows=8, row_group=group, row_ids=ids, row_docs=ids, k=4), **bad})
+
+
 def test_one_call_refuses_what_its_launches_do():
     frag, x = torch.zeros(128, 256, dtype=torch.bfloat16, device=DEV), torch.zeros(2, 256, device=DEV)
     group, ids = torch.zeros(8, dtype=torch.int32, device=DEV), torch.zeros(8, dtype=torch.int64, device=DEV)
