@@ -342,11 +342,13 @@ class LlamaModel(FragmentProjections):
         return self._all_reduce(x)
 
     def _frag_serves(self, T: int) -> bool:
-        """Whether qkv, o and down of a step of ``T`` tokens are of the sizes that ``gemm_frag`` was measured at: past 128 tokens
-        its tiles beat the streamed projections (us a layer of qkv, o and down with their norms at T 200: Llama-3-8B 91 -> 75, 1B
-        43 -> 38)."""
+        """Whether qkv, o and down of a step of ``T`` tokens are of the sizes that ``gemm_frag`` was measured at, and of whole 256
+        weight rows, as ``gemm_bt`` gives it: past 128 tokens its tiles beat the streamed projections (us a layer of qkv, o and
+        down with their norms at T 200: Llama-3-8B 91 -> 75, 1B 43 -> 38).  Other rows would fall to the 128 x 128 kernel (a layer of
+        hidden 1920, qkv of 3200 rows, at T 129 streamed 97, there 168; hidden 2176 126, 192)."""
         L = self.layers[0]
-        return all(ops.native().frag_us(T, w.shape[0], w.shape[1], 1) < float("inf") for w in (L.qkv_w, L.o_w, L.down_w))
+        return all(w.shape[0] % 256 == 0 and ops.native().frag_us(T, w.shape[0], w.shape[1], 1) < float("inf")
+                   for w in (L.qkv_w, L.o_w, L.down_w))
 
     def _slab_proj(self, x, w, name: str):
         """fp32 slabs of a prefill projection where summing them in the norm behind it is the quicker, else None."""

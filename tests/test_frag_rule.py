@@ -1,6 +1,10 @@
 """Which prefill projections gemm_frag takes, and in how many K-slices."""
-import pytest
+from types import SimpleNamespace
 
+import pytest
+import torch
+
+from django_assistant_bot_amd.models import LlamaModel
 from django_assistant_bot_amd.ops.kernels import frag_plan, frag_slices, native
 
 
@@ -32,3 +36,13 @@ def test_estimate_of_no_product(slices):
                                         (400, 4096, 14336, "mid"), (1900, 4096, 14336, "mid"), (1093, 6144, 4096, "mid"), (700, 2304, 2048, "mid")])
 def test_rows_of_a_tile(M, N, K, kind):
     assert frag_plan(M, N, K, True, False)[0][0] == kind
+
+
+# a step's projections leave the stream only for sizes that gemm_bt gives to gemm_frag: whole 256 weight rows (qkv, hidden, MLP)
+@pytest.mark.parametrize("qkv,hidden,mlp,serves", [(6144, 4096, 14336, True), (3072, 2048, 8192, True), (3200, 1920, 5120, False), (6528, 2176, 5888, False),
+                                                   (3200, 2048, 8192, False), (3072, 1920, 8192, False), (1152, 896, 4864, False)])
+def test_steps_that_are_not_streamed(qkv, hidden, mlp, serves):
+    layer = SimpleNamespace(**{n: torch.empty(s, device="meta") for n, s in (("qkv_w", (qkv, hidden)), ("o_w", (hidden, hidden)), ("down_w", (hidden, mlp)))})
+    model = SimpleNamespace(layers=[layer])
+    for T in (129, 200, 256):
+        assert LlamaModel._frag_serves(model, T) == serves
