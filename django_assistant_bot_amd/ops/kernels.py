@@ -603,15 +603,31 @@ def frag_slices(M: int, N: int, K: int) -> int:
     return best
 
 
-def gemm_frag(A, B, residual=None, epilogue=EPI_NONE, out=None, b_group: int = 1, glu_bias=None, slices: int = 0, tile: int = -1):
+@functools.lru_cache(maxsize=4096)
+def _frag_ok(M: int, N: int, K: int, lda: int) -> bool:
+    return native().gemm_frag_ok(M, N, K, lda)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm256_ok(M: int, N: int, K: int, lda: int) -> bool:
+    """Whether gemm256 takes a projection with fragment-layout weights."""
+    return bool(native().gemm256_ok(M, N, K, lda, K))
+
+
+def gemm_frag(A, B, residual=None, epilogue=EPI_NONE, out=None, b_group: int = 1, glu_bias=None, slices: int = 0, tile: int = -1,
+              checked: bool = False):
     """C = A . B^T (+ residual) or a GLU over 8-row [gate | up] groups, B a ``shuffle_weights`` copy, on tiles of 32 x 64 to 128 x
     256 (``gemm_frag.hip``).  ``slices`` S > 0: the K-slices' sums as fp32 slabs [S, M, N] for ``rmsnorm``.  ``tile`` (tests): that
-    one instead of the one with the least estimate."""
+    one instead of the one with the least estimate.  ``checked``: the operands and ``out`` have passed ``gemm_bt``'s checks."""
     M, K = A.shape
     N = B.shape[0]
+    if checked:
+        native().gemm_frag(ptr(A), A.stride(0), ptr(B), ptr(out), out.stride(0), ptr(residual),
+                           residual.stride(0) if residual is not None else 0, ptr(glu_bias), 0, 0, M, N, K, epilogue, b_group, tile, stream(A))
+        return out
     expect(A.is_cuda and A.dtype == torch.bfloat16 and B.dtype == torch.bfloat16, "bf16 CUDA operands required")
     expect(A.stride(-1) == 1 and B.is_contiguous() and B.shape[1] == K, "A K-contiguous, B a contiguous [N, K] copy")
-    expect(native().gemm_frag_ok(M, N, K, A.stride(0)), "gemm_frag: N % 32, K % 64, 16-B rows")
+    expect(_frag_ok(M, N, K, A.stride(0)), "gemm_frag: N % 32, K % 64, 16-B rows")
     expect(epilogue in (EPI_NONE, *GLU8) and b_group in (1, 8), "gemm_frag epilogues: none (+residual) or an 8-row-group GLU")
     n_out = N // 2 if epilogue in GLU8 else N
     if residual is not None:
@@ -632,13 +648,13 @@ def gemm_frag(A, B, residual=None, epilogue=EPI_NONE, out=None, b_group: int = 1
 
 def _frag_takes(A, B, out, residual, glu_bias) -> bool:
     """Whether ``gemm_frag`` takes a projection's operands (the kernels beside it take any alignment)."""
-    return (native().gemm_frag_ok(A.shape[0], B.shape[0], A.shape[1], A.stride(0)) and out.stride(0) % 8 == 0
+    return (_frag_ok(A.shape[0], B.shape[0], A.shape[1], A.stride(0)) and out.stride(0) % 8 == 0
             and (residual is None or residual.stride(0) % 8 == 0)
             and (ptr(A) | ptr(B) | ptr(out) | ptr(residual) | ptr(glu_bias)) % 16 == 0)
 
 
 def _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias):
-    """Runs the parts of a ``frag_plan`` (views of the operands: a part starts at a whole tile)."""
+    """Runs the parts of a ``frag_plan``: the whole product, or views of the operands (a part starts at a whole tile)."""
     M, N = A.shape[0], B.shape[0]
     m = n = 0
     per = 2 if epilogue in GLU8 else 1  # weight rows per output column
@@ -646,11 +662,13 @@ def _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias):
         if part is None:
             continue
         kind, rows, cols = part
-        a, b = A[m:m + rows], B[n:n + cols]
-        o = out[m:m + rows, n // per:(n + cols) // per]
-        r = None if residual is None else residual[m:m + rows, n:n + cols]
+        a, b, o, r = A, B, out, residual
+        if rows < M or cols < N:
+            a, b = A[m:m + rows], B[n:n + cols]
+            o = out[m:m + rows, n // per:(n + cols) // per]
+            r = None if residual is None else residual[m:m + rows, n:n + cols]
         if kind == "frag":
-            gemm_frag(a, b, residual=r, epilogue=epilogue, out=o, b_group=b_group, glu_bias=glu_bias)
+            gemm_frag(a, b, residual=r, epilogue=epilogue, out=o, b_group=b_group, glu_bias=glu_bias, checked=True)
         elif kind != "256":
             gemm_mid(a, b, residual=r, epilogue=epilogue, out=o, variant=192 if kind == "192" else 0, b_group=b_group, glu_bias=glu_bias)
         else:
@@ -745,12 +763,12 @@ def gemm_bt(A, B, bias=None, residual=None, epilogue=EPI_NONE, out_f32=False, ro
     if plain and shuffled and N == B.shape[0] and bias is None and epilogue in (EPI_NONE, *GLU8) and N % 256 == 0:
         lda = A.stride(0)
         frag = _frag_takes(A, B, out, residual, glu_bias)
-        if frag and glu_bias is None and M > 256 and native().gemm256_ok(M, N, K, lda, K):
+        if frag and glu_bias is None and M > 256 and _gemm256_ok(M, N, K, lda):
             tail = corner_plan(M, N, K)[0]
             if tail:
                 return _run_corner(tail, A, B, out, residual, epilogue, b_group)
         plan = (frag_plan(M, N, K, glu_bias is None, frag)
-                if M >= GEMM_MID_MIN_M and native().gemm256_ok(M, N, K, lda, K) else None)
+                if M >= GEMM_MID_MIN_M and _gemm256_ok(M, N, K, lda) else None)
         if plan is not None and all(q is None or q[0] not in ("mid", "192") or gemm_mid_ok(q[1], q[2], K, lda) for q in plan):
             return _run_frag_plan(plan, A, B, out, residual, epilogue, b_group, glu_bias)
         if use_gemm_mid(M, N, K, A.stride(0)):

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from django_assistant_bot_amd.models import LlamaModel
+from django_assistant_bot_amd.ops import kernels
 from django_assistant_bot_amd.ops.kernels import frag_plan, frag_slices, native
 
 
@@ -46,3 +47,20 @@ def test_steps_that_are_not_streamed(qkv, hidden, mlp, serves):
     model = SimpleNamespace(layers=[layer])
     for T in (129, 200, 256):
         assert LlamaModel._frag_serves(model, T) == serves
+
+
+# a whole product runs on the operands themselves (views of them are host time that short prompts wait for), parts on theirs
+def test_parts_of_a_plan(monkeypatch):
+    calls = []
+    monkeypatch.setattr(kernels, "gemm_frag", lambda a, b, **kw: calls.append((a, b, kw["out"], kw["residual"])))
+    monkeypatch.setattr(kernels, "_gemm256_into", lambda a, b, o, bias, r, *rest: calls.append((a, b, o, r)))
+    A, B, out, r = torch.zeros(600, 64), torch.zeros(512, 64), torch.zeros(600, 512), torch.zeros(600, 512)
+    kernels._run_frag_plan((("frag", 600, 512), None), A, B, out, r, kernels.EPI_NONE, 1, None)
+    assert all(x is y for x, y in zip(calls.pop(), (A, B, out, r)))
+    for plan, cut in (((("256", 512, 512), ("frag", 88, 512)), (512, 0)), ((("256", 600, 256), ("frag", 600, 256)), (0, 256))):
+        kernels._run_frag_plan(plan, A, B, out, r, kernels.EPI_NONE, 1, None)
+        m, n = cut
+        for got, (rows, cols) in zip(calls, ((slice(0, m or 600), slice(0, n or 512)), (slice(m, 600), slice(n, 512)))):
+            for x, y in zip(got, (A[rows], B[cols], out[rows, cols], r[rows, cols])):
+                assert x.data_ptr() == y.data_ptr() and x.shape == y.shape and x.stride() == y.stride()
+        del calls[:]
