@@ -591,10 +591,13 @@ def _run_corner(tail: int, A, B, out, residual, epilogue, b_group):
 @functools.lru_cache(maxsize=4096)
 def frag_slices(M: int, N: int, K: int) -> int:
     """K-slices that ``gemm_frag`` leaves as fp32 slabs to the norm behind a projection with a residual, 0: the whole product
-    is the quicker.  The norm reads them at some 4.5 TB/s.  us of product and norm, whole on the quickest kernel -> in slices:
+    is the quicker, or its time not known (K an odd multiple of 64 of several thousand rows, the 128 x 128 kernel's: (3500, 4096,
+    1600) with the norm 68 whole, 97 in slices).  The norm reads them at some 4.5 TB/s.  us of product and norm, whole on the quickest kernel -> in slices:
     (260, 2048, 8192) 33.5 -> 23.8, (515, 2048, 8192) 39.8 -> 35.6, (140, 4096, 14336) 57 -> 39.7, (260, 4096, 14336) 62.6 ->
     55.4; (1093, 2048, 8192) 57.4 -> 53.1."""
     whole = corner_plan(M, N, K)[1] or _frag_plan(M, N, K, True, True)[1]
+    if whole == float("inf"):
+        return 0
     best, least = 0, 0.95 * whole
     for s in (2, 3, 4, 6, 8):
         us = native().frag_us(M, N, K, s) + 0.7 + 4 * s * M * N / 4.5e6 if K // 64 >= 4 * s else float("inf")

@@ -22,6 +22,8 @@ def test_plan(M, N, K, takes):
 def test_slices():
     assert frag_slices(260, 2048, 8192) > 1 and frag_slices(140, 4096, 14336) > 1
     assert frag_slices(1093, 4096, 14336) == frag_slices(400, 2048, 2048) == frag_slices(3000, 4096, 4096) == 0
+    for M, N, K in ((3000, 4096, 6848), (3300, 4096, 6848), (2048, 6144, 1088), (3500, 4096, 1600)):  # no estimate of the whole product
+        assert frag_plan(M, N, K) is None and frag_slices(M, N, K) == 0
     for M, N, K in ((140, 1024, 1024), (260, 2048, 8192), (515, 2048, 8192), (260, 4096, 14336)):
         s = frag_slices(M, N, K)
         assert s == 0 or K // 64 >= 4 * s
