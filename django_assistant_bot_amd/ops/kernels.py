@@ -786,7 +786,8 @@ def gemm_bt(A, B, bias=None, residual=None, epilogue=EPI_NONE, out_f32=False, ro
         _gemm256_into(A[:rows], B, out[:rows], bias if glu_bias is None else glu_bias, None if residual is None else residual[:rows],
                       epilogue, shuffled, b_group)
         if rows < M:
-            _gemm_small_into(A[rows:], B, out[rows:], bias, None if residual is None else residual[rows:], epilogue, native().RING_TILE)
+            took = _gemm_small_into(A[rows:], B, out[rows:], bias, None if residual is None else residual[rows:], epilogue, native().RING_TILE)
+            expect(took, "gemm_bt: the rows behind the waves")  # (what it takes of all rows it takes of the last)
         return out
     native().gemm_bt(ptr(A), A.stride(0), ptr(B), B.stride(0), ptr(out), out.stride(0),
                      ptr(bias if glu_bias is None else glu_bias), ptr(residual),

@@ -70,6 +70,16 @@ def test_rows_behind_the_waves(N, K, gelu, res, more, bias):
 
 
 @pytest.mark.gpu
+def test_rows_that_the_ring_refuses_are_not_left_out(monkeypatch):
+    M, N, K = 256 // 3 * 256 + 1, 768, 768
+    assert _rows(M, N, K, False, False) == M - 1
+    A, B = (torch.zeros(n, K, dtype=torch.bfloat16, device=DEV) for n in (M, N))
+    monkeypatch.setattr(kernels, "_gemm_small_into", lambda *a: False)
+    with pytest.raises(ValueError):
+        ops.gemm_bt(A, B)
+
+
+@pytest.mark.gpu
 def test_the_encoders_projections_take_the_same_rows(monkeypatch):
     cfg = EncoderConfig("t", vocab_size=500, hidden=768, layers=1, heads=12, intermediate=3072)
     model = BertEncoder(cfg, random_encoder_weights(cfg, DEV, seed=1), DEV)
