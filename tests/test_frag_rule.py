@@ -66,3 +66,19 @@ def test_parts_of_a_plan(monkeypatch):
             for x, y in zip(got, (A[rows], B[cols], out[rows, cols], r[rows, cols])):
                 assert x.data_ptr() == y.data_ptr() and x.shape == y.shape and x.stride() == y.stride()
         del calls[:]
+
+
+# with gemm_frag behind the waves, too, the parts are the product
+def test_plans_with_gemm_frag_behind_the_waves():
+    seen = 0
+    for M in (641, 700, 1100, 1200, 1280, 2420, 3100, 3500, 4097, 4200, 5000, 5500, 5900):
+        for N, K in ((2048, 2048), (4096, 4096), (6144, 4096), (8192, 2048), (16384, 2048), (28672, 4096)):
+            for cols in (True, False):
+                plan = frag_plan(M, N, K, cols)
+                if plan is None or plan[1] is None or plan[1][0] != "frag":
+                    continue
+                (_, m, n), (_, m2, n2) = plan
+                assert (m == m2 == M and n + n2 == N and cols) or (n == n2 == N and m + m2 == M)
+                assert n % 256 == 0 and (m == M or m % 256 == 0)
+                seen += 1
+    assert seen > 10

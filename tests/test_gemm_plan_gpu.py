@@ -84,3 +84,35 @@ def test_mid_groups_joined_over_xcds(M, N, K, glu):
     for _ in range(3):  # the counts are zero again after each launch
         out = ops.kernels.gemm_mid(A, B, residual=res, epilogue=epi, b_group=8 if glu else 1, variant=64)
         assert ((out.float() - exp).abs() <= tol).all()
+
+
+# gemm_frag behind gemm256's whole waves: columns divided, rows divided, a single row, a gate's half columns and its bias
+@pytest.mark.parametrize("M,N,K,kind,rows", [(700, 28672, 4096, "glu", False), (3500, 6144, 4096, "plain", False), (3500, 6144, 4096, "residual", False),
+                                             (3100, 6144, 4096, "plain", True), (3100, 6144, 4096, "residual", True), (4097, 4096, 4096, "residual", True),
+                                             (1200, 16384, 2048, "glu", True), (1200, 16384, 2048, "glu_bias", True)])
+def test_gemm_frag_behind_the_waves(M, N, K, kind, rows):
+    glu = kind.startswith("glu")
+    first, rest = frag_plan(M, N, K, kind != "glu_bias")
+    assert rest[0] == "frag" and (rest[2] == N) == rows and ops.kernels.corner_plan(M, N, K)[0] == 0
+    grp, n_out = (8, N // 2) if glu else (1, N)
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    A = torch.randn(M, K + 8, device=DEV, generator=g).to(torch.bfloat16)[:, :K]
+    B = (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).to(torch.bfloat16)
+    r = torch.randn(M, N + 16, device=DEV, generator=g).to(torch.bfloat16)[:, :N] if kind == "residual" else None
+    gb = torch.randn(N, device=DEV, generator=g) if kind == "glu_bias" else None
+    wide = torch.full((M + 1, n_out + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    got = ops.gemm_bt(A, ops.shuffle_weights(B, grp), residual=r, shuffled=True, b_group=grp, glu_bias=gb, out=wide[:M, :n_out],
+                      epilogue=ops.EPI_SWIGLU8 if glu else ops.EPI_NONE).double()
+    assert (wide[M:] == 7.0).all() and (wide[:, n_out:] == 7.0).all()
+    exp = A.double() @ B.double().t()
+    if glu:
+        v = exp.view(M, N // 16, 2, 8)
+        if gb is not None:
+            v = v + gb.double().view(2, N // 16, 8).transpose(0, 1)
+        exp = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    # as ``test_planned_projection``; the gate's and the up projection's 1e-4 multiply the other's size, up to 8 or so
+    tol = 2.0 ** -8 * exp.abs() + (1e-3 if glu else 1e-4)
+    if r is not None:
+        exp = exp + r.double()
+        tol = tol + 2.0 ** -8 * exp.abs()
+    assert ((got - exp).abs() <= tol).all()

@@ -44,3 +44,25 @@ def test_where_they_are_chosen():
     for M in (65, 128):
         assert p._stream_cfg("qkv", M, 4096) == 10 and p._stream_cfg("gate_up", M, 16384) == 9
         assert p._stream_cfg("gate_up", M, 28672) == 20
+
+
+# 512 workgroups of 64 rows and more run with the ring of 8 stages (45): K of one stage, one more than the ring, several rings; K-slices
+# that make the workgroups many; and that form asked for, at few
+@pytest.mark.parametrize("M", [1, 15, 16])
+@pytest.mark.parametrize("N,K,S,glu", [(32768, 128, 1, False), (32768, 1152, 1, False), (33024, 4096, 1, False), (8192, 2048, 4, False),
+                                       (32768, 1152, 1, True), (64, 128, 1, False), (192, 1152, 9, False), (256, 2304, 1, True)])
+def test_many_workgroups(M, N, K, S, glu):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).to(torch.bfloat16)
+    exp, grp = x.double() @ w.double().t(), 8 if glu else 1
+    B = ops.shuffle_weights(w, grp)
+    kw = dict(epilogue=ops.EPI_SWIGLU8, w_group=grp) if glu else dict(splits=S)
+    y = ops.stream_gemm(x, B, nt=True, cfg=45, **kw)
+    if glu:
+        v = exp.view(M, N // 16, 2, 8)
+        exp = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    got = y.double().sum(0) if S > 1 else y.double()
+    # rounded to bf16 (2^-8) unless in fp32 slabs; fp32 sums of K products of size about K^-1/2
+    assert got.shape == exp.shape and ((got - exp).abs() <= (0 if S > 1 else 2.0 ** -8) * exp.abs() + 1e-4).all()
+    assert torch.equal(ops.stream_gemm(x, B, nt=True, cfg=43, **kw), y)  # rings of 3 and 8 stages: one order of the sums
