@@ -505,7 +505,6 @@ PYBIND11_MODULE(_native, m) {
      py::arg("residual"), py::arg("ldr"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("epilogue"),
      py::arg("out_f32"), py::arg("row_group"), py::arg("q_group"), py::arg("allow"), py::arg("allow_words"),
      py::arg("s"), py::arg("b_rows") = 0, py::arg("b_group") = 1);
-  m.def("frag_tile", &dab::frag_tile);
   m.def("frag_us", &dab::frag_us);
   m.def("gemm_frag_ok", [](long M, long N, long K, long lda) { return dab::gemm_frag_ok(M, N, K, lda) != 0; });
   m.def("gemm_frag", [](u A, long lda, u B, u C, long ldc, u residual, long ldr, u glu_bias, u slabs, int slices, int M, int N,

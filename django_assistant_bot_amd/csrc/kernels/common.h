@@ -60,9 +60,10 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
 
 // Exact-erf GELU as max(x, 0) - |x| Phi(-|x|), Phi(-a) = erfc(a / sqrt 2) / 2 = 2^P(a): P a polynomial of degree 10, fitted
 // (weighted least squares, reweighted towards the greatest error) to log2 Phi(-a) for a up to 13, where Phi leaves fp32; beyond
-// that P only falls.  Against 64 bits: 2.5e-7 at most for |x| <= 8 and, for negative x, relative errors below half of those of Abramowitz &
-// Stegun 7.1.26, which stood here before (3.3e-7 at most), at almost every x and nowhere above.  13 instructions, of which v_exp
-// takes four turns, instead of 17 with v_exp and v_rcp: the epilogue of a 256 x 256 tile is bound by them
+// that P only falls.  Against 64 bits: 2.5e-7 at most for |x| <= 8, where Abramowitz & Stegun 7.1.26, which stood here before, has
+// 3.3e-7.  For negative x the greatest relative error of every interval is lower than its (0-1 4e-7 for 7e-7, 1-2 1.8e-6 for 3.4e-6,
+// 2-3 1.0e-5 for 5.3e-5, 3-5 7e-4 for 1.6e-3, 5-8 0.0042 for 0.0103), though not that of every x: 40 % of the x above -1 and a
+// tenth of those from -3 to -1 had a smaller one.  13 instructions, of which v_exp takes four turns, instead of 17 with v_exp and v_rcp: the epilogue of a 256 x 256 tile is bound by them
 // (400 chunks of 32-512 tokens, bge-base, 23,542 -> 23,188 us a call; 31,900 tokens 6,690 -> 6,576).
 __device__ __forceinline__ float gelu_erf(float x) {
   const float a = fabsf(x);

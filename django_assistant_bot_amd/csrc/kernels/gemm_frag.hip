@@ -15,8 +15,10 @@
 //   * The copies of a later K-tile go out one at a time between the products: all of them in front hold the waves up until
 //     the last is accepted (192 x 128: 0.65 -> 0.57 us a K-tile, 128 x 256 0.80 -> 0.77).
 //
-// us, cold weights, gemm_mid / gemm256 -> here: (260, 2048, 2048) 20.3 -> 10.0, (515, 3072, 2048) 22.3 -> 13.5, (260, 6144,
-// 4096) 32 -> 25.5, (600, 4096, 4096) 38 -> 33, (1093, 4096, 4096) 50.7 -> 44.5, (140, 28672, 4096) GLU 70 -> 53.
+// us, cold weights, gemm_mid / gemm256 -> here: (260, 2048, 2048) 19.4 -> 9.7, (515, 3072, 2048) 22.2 -> 13.6, (260, 6144,
+// 4096) 35 -> 26, (800, 6144, 4096) 55 -> 48, (140, 28672, 4096) GLU 75 -> 60; with a residual (300, 4096, 4096) 29 -> 21, (1200, 4096,
+// 4096) 57 -> 47.  Launches alone are quicker here, too, where the estimates, which know no epilogue, lie within the plan's 7 % and
+// gemm_mid keeps the product: (600, 4096, 4096) with a residual 37.6 / 34.7, (1093, 4096, 4096) 51 / 45, (1093, 6144, 4096) 62.5 / 58.
 #include <cmath>
 #include <type_traits>
 
@@ -282,7 +284,7 @@ float frag_tile_us(const FragTile& t, int M, int N, int K, int slices) {
 }  // namespace
 
 // The tile with the least estimate for a product in so many K-slices (1: whole).
-int frag_tile(int M, int N, int K, int slices) {
+static int frag_tile(int M, int N, int K, int slices) {
   int best = 0;
   for (int i = 1; i < kFrags; ++i)
     if (frag_tile_us(kFrag[i], M, N, K, slices) < frag_tile_us(kFrag[best], M, N, K, slices)) best = i;

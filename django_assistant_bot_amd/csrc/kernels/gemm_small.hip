@@ -490,7 +490,7 @@ __global__ __launch_bounds__(512) void gemm_attn_kernel(SmallParams p, SmallAtte
 // c ^ ((r >> 1) & 7) (the swizzle goes on the source address, LDS-DMA writes lane-linearly); a copy is 8 rows, and copy q of a
 // K-tile's A and B rows, one behind the other, is wave q mod the waves'.  The copies go out one at a time between the products:
 // all in front of the fragment reads, they hold the waves up until the last is accepted, which is as long as the products take
-// (24 texts of 8-64 tokens 616 -> 581 us, 10 of 200 876 -> 841; fragments read a K-tile ahead besides: the same).  Bias and
+// (24 texts of 8-64 tokens 628 -> 596 us, 10 of 200 920 -> 908; fragments read a K-tile ahead besides: the same).  Bias and
 // residual are asked for at the start: at the end they were one more round trip (0.2-0.7 us).
 constexpr int ring_occupancy(int rows, int waves, int ns) {  // waves a SIMD that the ring leaves room for
   const int n = 163840 / (rows * 128 * ns) * waves / 4;
@@ -655,6 +655,10 @@ static float ring_us(const RingTile& t, int M, int N, int K, int gelu, int slice
 // before, up to 69 % ((4000, 1024, 1024) 27.6 -> 16.4 us), 0.95 at worst ((560, 1024, 4096) in three slices 16.2 -> 17.0).  Calls of the
 // encoder: bge-base 24 texts of 8-64 tokens 748 -> 716, 1300 tokens 854 -> 766, 2200 1186 -> 1045, 7000 2509 -> 2027; MiniLM
 // 4000 473 -> 404; bge-large 1000 1907 -> 1719, 5000 5604 -> 4609.
+// (All of that with the copies of a K-tile in front of its products and the former GELU.  As both are now the estimates are 7 % too long
+// in the middle, 15 % too short to 25 % too long for eight of ten of 60 sizes, and the tile taken by them is 2 % slower than the
+// best in the mean; the most (3100, 768, 768) 12.5 us on 96 x 64, 9.6 on 64 x 192, and (6000, 768, 3072) 48 on 96 x 96, 37 on 128 x
+// 192.)
 int ring_tile(int M, int N, int K, int gelu, int slices) {
   int best = 0;
   for (int i = 1; i < kRings; ++i)

@@ -395,7 +395,6 @@ int topk_rows_2stage(const float* scores, long ld, int rows, int n, int k, float
                      int64_t index_base, int64_t* out_idx64, void* workspace, size_t workspace_bytes, hipStream_t s);
 
 // gemm_frag.hip (M up to some 2000: tiles of 32 x 64 to 128 x 256 on fragment-layout weights)
-int frag_tile(int M, int N, int K, int slices);
 double frag_us(int M, int N, int K, int slices);
 int gemm_frag_ok(long M, long N, long K, long lda);
 int gemm_frag(const void* A, long lda, const void* B, void* C, long ldc, const void* residual, long ldr, const void* glu_bias,

@@ -498,12 +498,12 @@ static constexpr StreamCfg kStreamCfgs[] = {
     {8, 1, 1, 4, 6, 2, true, 0, 7},  // 41: 6-stage weight ring
     {8, 1, 1, 3, 8, 1, true, 0, 7},  // 42: 8-stage weight ring, 1 loader wave
     // M <= 16 / 32 with 64 weight rows: the small projections fill the chip with half the K-slices (half the slabs for
-    // their consumers), unsplit ones below 192 tiles of 128 with all of its CUs.  us, BN 128 -> 64 at M 6 (both with longer weight rings): (4096, 4096) 9.7
-    // -> 9.0, (6144, 4096) 11.7 -> 11.4, gated (16384, 2048) 15.5 -> 13.4, (2048, 2048) 5.4 -> 4.7, (2048, 8192) 9.7 -> 8.8;
-    // not gated (28672, 4096), 224 tiles of 128: 36.8 -> 38.9.  (BN 96 and 112, 256 workgroups of 6 and 7 waves: slower.)
+    // their consumers), unsplit ones below 192 tiles of 128 with all of its CUs.  us, BN 128 -> 64 at M 6: (4096, 4096) 9.0
+    // -> 7.8, (6144, 4096) 11.5 -> 11.2, gated (16384, 2048) 16.5 -> 13.3, (2048, 2048) 5.1 -> 4.1, (2048, 8192) 9.2 -> 7.7;
+    // not gated (22016, 4096), 172 tiles of 128: 34.0 -> 37.4.  (BN 96 and 112, 256 workgroups of 6 and 7 waves: slower.)
     {1, 1, 1, 4, 3, 2, true, 0, 4},  // 43: M <= 16
     {2, 1, 1, 4, 3, 2, true, 0, 4},  // 44: M <= 32
-    // The weight rings of 12, 13, 20, 30, 31, 43 and 44 are as short as they can be: what is in flight ahead of the first stage
+    // The weight rings of 12, 13, 20, 30, 31, 43 and 44 have three stages: what is in flight ahead of the first stage
     // delays it, and the stages that a ring asks for past the slice's end (the last one again) are traffic of the same CU,
     // with 8 of 16 a third of it.  us of 8 stages (43, 44) or 4 -> 3: 6 rows (6144, 4096) 11.5 -> 10.2, (4096, 4096) 8.9 ->
     // 7.6, (4096, 14336) 20.5 -> 19.8, gated (28672, 4096) 37.6 -> 36.4; 32 rows (6144, 4096) 12.3 -> 11.2, (4096, 4096) 9.5 ->
@@ -511,7 +511,8 @@ static constexpr StreamCfg kStreamCfgs[] = {
     // (4096, 14336) 22.6 -> 22.0, LM head (128256, 4096) 197 -> 192; 128 rows gated (28672, 4096) 49.4 -> 48.5 (at 65-128 rows the
     // others' 2 stages of 128 rows gain and lose: (4096, 4096) 12.0 -> 11.5, (3072, 2048) 7.9 -> 8.5).  Two stages are as good up
     // to 32 rows but for an LM head (31: 177 -> 190).
-    // An LM head of many tiles on 43 keeps 8: (128256, 4096) 161 -> 166 with 3.
+    // An LM head of many tiles on 43 keeps 8: (128256, 4096) 161 -> 166 with 3.  Up to 508 workgroups 3 are the quicker: 8 -> 3 stages
+    // (32512, 4096) 46.7 -> 44.5, (24576, 4096) 40 -> 37.5, (32512, 2048) 26.4 -> 23.8, (8192, 4096) in two slices 14.2 -> 13.1.
     {1, 1, 1, 4, 8, 2, true, 0, 4},  // 45: 43's tile where the workgroups are many
     {4, 2, 2, 4, 4, 4, true},        // 46: 12's, for candidates
 };

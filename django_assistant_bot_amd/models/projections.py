@@ -47,10 +47,11 @@ class FragmentProjections:
         workgroup, or where they need half the K-slices, so that the workgroups stay as many; but with few K-slices each
         of them then walks so long a K that the wider tile's smaller share of X counts.
 
-        Time with 64 rows / with 128, M 1 .. 64: as many K-slices, 8-256 workgroups 0.6-1.0, 264-320 of them 1.1-1.4 (gate_up
-        of 22016 x 4096 at 6 rows 30.5 / 37 us, at 100 42 / 57; qkv of 1280 x 8192 8.0 / 9.3); half the K-slices, K / slices up to
-        2048 0.85-1.0; from 3584 on at 33-64 rows 1.0-1.13 (8192 x 28672 at 64 76 / 83 us), from 7168 on at 17-32 rows
-        1.0-1.06, up to 16 rows 0.97-1.03.  An LM head of 1002 tiles up to 16 rows: K 4096 0.98, K 2048 1.0-1.03; above 1.02."""
+        Time with 64 rows / with 128, M 1 .. 64: as many K-slices, up to 256 workgroups 0.60-0.88, 264-320 of them 1.02-1.16, more
+        1.0-1.18 (gate_up of 22016 x 4096 at 6 rows 37.4 / 34.0 us, at 100 58 / 44; qkv of 1280 x 8192 7.5 / 7.2); half the
+        K-slices, K / slices up to 2048 0.69-1.02, but 6144 x 4096 at 33-64 rows 1.07 (15.5 / 14.5 us); from 3584 on at 33-64 rows
+        0.96-1.09 (8192 x 28672 at 64 83 / 76 us), from 7168 on at 17-32 rows 0.99-1.0, up to 16 rows 0.99-1.0.  An LM head of 1002
+        tiles up to 16 rows: K 4096 0.98-1.02, K 2048 1.05-1.07; above 1.0-1.06."""
         tiles = N // 128
         if tiles >= 768:
             return M <= 16 and not 0 < K < 4096
@@ -141,7 +142,7 @@ class FragmentProjections:
     def _norm_proj(self, x, gain, eps: float, residual, w, name: str, epilogue=ops.EPI_NONE):
         """RMSNorm(x + residual) and the projection behind it in one launch for a few decode rows (``ops.norm_stream``, TP 1,
         fragment layout) -> (product, slabs where a consumer sums them; new residual), or None where that is not taken: up to
-        4 rows whose model ``_rows_serve`` leaves out, projections that split as ``stream_gemm`` does on 64 weight rows a workgroup, gated ones unsplit on 128 (us,
+        4 rows whose model ``_rows_serve`` leaves out (gate and up rows not interleaved, above all), projections that split as ``stream_gemm`` does on 64 weight rows a workgroup, gated ones unsplit on 128 (us,
         4 rows of gated (28672, 4096) / (16384, 2048): 41.8 / 16.3 on 128, 43.7 / 18.5 on 64).  ``residual`` None: the first layer's
         input is the residual stream."""
         M, K, N, grp = x.shape[-2], x.shape[-1], w.shape[0], self.proj_group.get(name, 1)
